@@ -1,36 +1,27 @@
-// C[M,N] = A[M,K] * W[N,K]^T for any sizes and for fp32 or bf16 operands, accumulated in true fp32 with
-// plain FMAs in ascending k (no matrix-core shortcuts): the 32-bit path of every linear layer, and the
-// fallback for shapes the MFMA kernels refuse. One output element's sum never depends on M or on the
-// other rows of the batch.
+// C[M,N] = A[M,K] * W[N,K]^T for any sizes and for fp32 or bf16 operands (widened), every sum in true fp32: the 32-bit path
+// of every linear layer, and the fallback for shapes the bf16 matrix-core kernels refuse.
+//
+// The products run on the matrix cores' fp32 form, v_mfma_f32_16x16x4_f32, which rounds after every multiply-add and
+// takes its four k in ascending order: an output is the same bits as one accumulator walked with fmaf from k = 0 to
+// K - 1 (compared bit for bit on the GPU, also for sums that end in denormals). So an output never depends on M, on the
+// other rows of the batch or on which of the two kernels below computed it, and K is never cut. The vector units, which
+// this project builds without their packed fp32 forms, reach half the matrix cores' fp32 rate.
+//
+// Fragments: lane l of the MFMA holds row l % 16 at k = 4 s + l / 16 of step s. Memory holds a row's k side by side, so 16
+// bytes of a lane (k = 4 q .. 4 q + 3, q = l / 16) are one step's values of four lane groups, and a lane wants one value of
+// four steps: a transposition of 4 x 4 over the lane groups, done as the operands are written to LDS.
 //
 // Epilogues: 0 store (fp32 or bf16), 1 add into an fp32 matrix (the residual stream), 2 gated:
 // out = gate(A*Wg^T, A*Wu^T) (the gate functions of common.h) with two weight matrices sharing the A tile.
 #include "common.h"
 
-#define GBN 64
-#define GBK 32
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-// rows x GBK k of a row-major matrix into dst[k][row]; thread i: row i / (GBK / 4) (+ a round's rows), four k
-template <typename T, int ROWS>
-__device__ __forceinline__ void load_tile(const T* __restrict__ base, int ld, int row0, int nrows, int k0, int K,
-                                          float (*dst)[ROWS + 4]) {
-  constexpr int TPR = GBK / 4;  // threads per row
-  const int kq = (threadIdx.x % TPR) * 4;
-#pragma unroll
-  for (int r0 = 0; r0 < ROWS; r0 += 256 / TPR) {
-    const int r = r0 + (threadIdx.x / TPR);
-    const int row = row0 + r;
-    const T* p = base + (size_t)row * ld + k0 + kq;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float v = 0.f;
-      if (row < nrows && k0 + kq + j < K) v = ldf(p, j);
-      dst[kq + j][r] = v;
-    }
-  }
+__device__ __forceinline__ floatx4 mfma_f32(float w, float a, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(w, a, c, 0, 0, 0);
 }
 
-// bias, gate and store of one output: the same arithmetic in both kernels of this file
+// bias, gate and store of one output
 template <bool GATED>
 __device__ __forceinline__ void finish_output(float v, float up, int m, int n, const void* __restrict__ bias, int bias_dtype,
                                               void* __restrict__ out, int out_dtype, int ldo, int epilogue, GateSpec gs) {
@@ -49,161 +40,343 @@ __device__ __forceinline__ void finish_output(float v, float up, int m, int n, c
   }
 }
 
-// TM rows by 4 columns of outputs per thread: a tile of 16 TM rows by 64 columns. With TM = 8 a k step is 32
-// multiply-adds for 12 values read from LDS, which the vector units, not LDS, then bound; TM = 4 for few rows, where a
-// tile of 128 would be mostly empty.
-template <typename TA, typename TW, bool GATED, int TM>
-__global__ __launch_bounds__(256) void gemm_generic_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W,
-                                                           const TW* __restrict__ W2, const void* __restrict__ bias,
-                                                           int bias_dtype, void* __restrict__ out, int out_dtype,
-                                                           int ldo, int M, int N, int K, int epilogue, GateSpec gs) {
-  constexpr int GBM = 16 * TM;
-  __shared__ float As[GBK][GBM + 4];
-  __shared__ float Ws[GBK][GBN + 4];
-  __shared__ float Us[GATED ? GBK : 1][GBN + 4];
-  const int tx = threadIdx.x & 15;
-  const int ty = threadIdx.x >> 4;
-  const int m0 = blockIdx.y * GBM;
-  const int n0 = blockIdx.x * GBN;
-  float acc[TM][4] = {};
-  float acc2[TM][4] = {};
-  for (int k0 = 0; k0 < K; k0 += GBK) {
-    load_tile<TA, GBM>(A, lda, m0, M, k0, K, As);
-    load_tile<TW, GBN>(W, K, n0, N, k0, K, Ws);
-    if (GATED) load_tile<TW, GBN>(W2, K, n0, N, k0, K, Us);
-    __syncthreads();
+// four neighbouring outputs of one row: as finish_output, with one access where all four exist and lie on a boundary
+template <bool GATED>
+__device__ __forceinline__ void finish_four(floatx4 v, floatx4 u, int m, int n, int N, const void* __restrict__ bias, int bias_dtype,
+                                            void* __restrict__ out, int out_dtype, int ldo, int epilogue, GateSpec gs) {
+  if (n + 3 < N && out_dtype == JLLM_F32 && (ldo & 3) == 0 && (((uintptr_t)out) & 15) == 0) {
 #pragma unroll
-    for (int kk = 0; kk < GBK; ++kk) {
-      float a[TM], w[4], u[4];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) a[i] = As[kk][ty * TM + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = Ws[kk][tx * 4 + j];
-      if (GATED) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) u[j] = Us[kk][tx * 4 + j];
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
-          if (GATED) acc2[i][j] = fmaf(a[i], u[j], acc2[i][j]);
-        }
+    for (int c = 0; c < 4; ++c) {
+      if (bias) v[c] += (bias_dtype == JLLM_BF16) ? ldf((const bf16_t*)bias, n + c) : ldf((const float*)bias, n + c);
+      if (GATED) v[c] = gated<false>(v[c], u[c], gs);
     }
-    __syncthreads();
+    floatx4* o = (floatx4*)((float*)out + (size_t)m * ldo + n);
+    if (epilogue == 1) {
+      const floatx4 cur = *o;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[c] = cur[c] + v[c];
+    }
+    *o = v;
+    return;
   }
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = m0 + ty * TM + i;
-    if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n >= N) continue;
-      finish_output<GATED>(acc[i][j], acc2[i][j], m, n, bias, bias_dtype, out, out_dtype, ldo, epilogue, gs);
-    }
-  }
+  for (int c = 0; c < 4; ++c)
+    if (n + c < N) finish_output<GATED>(v[c], u[c], m, n + c, bias, bias_dtype, out, out_dtype, ldo, epilogue, gs);
 }
 
-// The same sums for up to 16 rows (decode steps of the 32-bit path), where a 64 x 64 tile would leave most of the
-// GPU idle: one accumulator per output, ascending k, fmaf, as above, so an output has the same bits whichever of the
-// two kernels computed it. A workgroup owns 32 weight rows and all the activation rows: thread (r, q) has weight row r
-// and activation rows q and q + 8. K advances in turns of 64 through two LDS buffers: the workgroup fetches the turn's
-// 32 x 64 weights with every 16 lanes reading 256 contiguous bytes of a row (whole cache lines; a thread walking
-// along a row of its own reads 16 bytes of 64 different lines per load instruction, and the loads of such a kernel took
-// 3 us a turn), and the activations, which lanes share. A K that is not a multiple of 64 ends in a turn filled up with
-// zeros, which add nothing.
-#define GR_ROWS 32   // weight rows per workgroup
-#define GR_K 64      // k per turn
-#define GR_WLD 65    // row stride of the weights in LDS: the lanes of a wave read one column of 32 rows
-#define GR_ALD 68    // of the activations: rows q and q + 1 in different banks
+// four consecutive elements of a row as floats. WIDE: k and K are multiples of four and the row starts on a boundary of
+// four elements; else element by element. Beyond K: zeros, which add nothing to a sum (in both operands, so that an
+// infinity in the other one is not multiplied by them).
+__device__ __forceinline__ floatx4 widen(floatx4 v) { return v; }
+__device__ __forceinline__ floatx4 widen(uint2 t) {
+  return floatx4{__uint_as_float(t.x << 16), __uint_as_float(t.x & 0xffff0000u), __uint_as_float(t.y << 16), __uint_as_float(t.y & 0xffff0000u)};
+}
+template <typename T>
+struct Four;  // four elements as they lie in memory
+template <>
+struct Four<float> {
+  typedef floatx4 type;
+};
+template <>
+struct Four<bf16_t> {
+  typedef uint2 type;
+};
+template <typename T, bool WIDE>
+__device__ __forceinline__ floatx4 load4k(const T* __restrict__ row, int k, int K) {
+  if (WIDE) {
+    const floatx4 v = widen(*(const typename Four<T>::type*)(row + (k < K ? k : 0)));
+    return k < K ? v : floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  floatx4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (k + j < K) v[j] = ldf(row, k + j);
+  return v;
+}
+// a piece of a stage in registers: four elements as they lie in memory, or, where rows cannot be read four at a time, as floats
+template <typename T, bool WIDE>
+struct Piece {
+  typedef typename Four<T>::type type;
+  static __device__ __forceinline__ type load(const T* __restrict__ row, int k, int K) { return *(const type*)(row + (k < K ? k : 0)); }
+  static __device__ __forceinline__ floatx4 value(type v, bool in) { return in ? widen(v) : floatx4{0.f, 0.f, 0.f, 0.f}; }
+};
+template <typename T>
+struct Piece<T, false> {
+  typedef floatx4 type;
+  static __device__ __forceinline__ type load(const T* __restrict__ row, int k, int K) { return load4k<T, false>(row, k, K); }
+  static __device__ __forceinline__ floatx4 value(type v, bool) { return v; }
+};
 
-template <typename TA, typename TW, bool GATED>
-__global__ __launch_bounds__(256) void gemm_rows_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W,
-                                                        const TW* __restrict__ W2, const void* __restrict__ bias,
-                                                        int bias_dtype, void* __restrict__ out, int out_dtype, int ldo,
-                                                        int M, int N, int K, int epilogue, GateSpec gs) {
-  __shared__ float ws[2][GATED ? 2 : 1][GR_ROWS][GR_WLD];
-  __shared__ float as[2][16][GR_ALD];
-  const int r = threadIdx.x & (GR_ROWS - 1), q = threadIdx.x / GR_ROWS;  // q = 0 .. 7
-  const int n0 = blockIdx.x * GR_ROWS;
-  // staging: element e = threadIdx.x + 256 i of the 32 x 64 tile is (row e / 64, k e % 64): a wave reads one row's 256
-  // bytes; of the 16 x 64 activations likewise
-  struct Staged {
-    float w[8], u[GATED ? 8 : 1], a[4];
+// Many rows: a workgroup of WM x WN waves owns a tile of 16 WM FM rows by 16 WN FN outputs, a wave FM x FN accumulators of
+// 16 x 16. Eight waves (two on every SIMD) where the tile has work for them: a wave alone on its SIMD multiplies nothing
+// while it reads and writes LDS.
+// K advances in stages of BK through two LDS buffers, the operands of the next two stages on their way into registers while
+// one is multiplied. LDS holds blocks of 16 rows x 16 k in the order the lanes read them (lane l's 16 bytes: its row at
+// k = q, 4 + q, 8 + q, 12 + q), so a fragment read is 1 KB side by side and the four 4-byte writes of a thread's 16
+// bytes go to neighbouring words across the wave.
+template <typename TA, typename TW, bool GATED, int WM, int WN, int FM, int FN, int BK, bool WIDE>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_f32_tile_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W,
+                                                            const TW* __restrict__ W2, const void* __restrict__ bias,
+                                                            int bias_dtype, void* __restrict__ out, int out_dtype, int ldo,
+                                                            int M, int N, int K, int epilogue, GateSpec gs) {
+  constexpr int TM = WM * FM * 16, TN = WN * FN * 16, NW = GATED ? 2 : 1, TH = WM * WN * 64;
+  constexpr int ROWS = TM + NW * TN, CH = BK / 16, QPR = BK / 4;  // rows staged, 16-k chunks and 16-byte pieces per row
+  constexpr int UA = TM * QPR / TH, UW = NW * TN * QPR / TH;      // pieces per thread and stage
+  static_assert(TM * QPR % TH == 0 && TN * QPR % TH == 0, "whole pieces of one operand per thread");
+  extern __shared__ __align__(16) float lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
+  // a stage's pieces on their way: as memory holds them (widened, and zeroed beyond K, when they are written to LDS), so
+  // that nothing waits for a load before its stage
+  struct Set {
+    typename Piece<TA, WIDE>::type a[UA];
+    typename Piece<TW, WIDE>::type w[UW];
   };
-  auto fetch = [&](Staged& st, int k0) {
+  const int pr = tid / QPR, pk = (tid % QPR) * 4;  // this thread's row (+ TH / QPR per piece) and place in a stage's k
+  auto fetch = [&](Set& st, int k0) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int e = threadIdx.x + 256 * i;
-      const int row = min(n0 + e / GR_K, N - 1), k = k0 + e % GR_K;
-      st.w[i] = k < K ? ldf(W + (size_t)row * K, k) : 0.f;
-      if (GATED) st.u[i] = k < K ? ldf(W2 + (size_t)row * K, k) : 0.f;
+    for (int i = 0; i < UA; ++i)
+      st.a[i] = Piece<TA, WIDE>::load(A + (size_t)min(m0 + pr + i * (TH / QPR), M - 1) * lda, k0 + pk, K);
+#pragma unroll
+    for (int i = 0; i < UW; ++i) {  // which weight a piece belongs to is the same for all threads
+      const int r = pr + (i % (UW / NW)) * (TH / QPR);
+      st.w[i] = Piece<TW, WIDE>::load((i < UW / NW ? W : W2) + (size_t)min(n0 + r, N - 1) * K, k0 + pk, K);
     }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto put = [&](const Set& st, int buf, int k0) {
+    const bool in = k0 + pk < K;
+    float* base = lds + buf * ROWS * BK + (pk >> 4) * 256;
+    const int turn = (pk >> 4) * (64 / CH);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int e = threadIdx.x + 256 * i;
-      const int m = e / GR_K, k = k0 + e % GR_K;
-      st.a[i] = (m < M && k < K) ? ldf(A + (size_t)m * lda, k) : 0.f;
+    for (int i = 0; i < UA + UW; ++i) {
+      const floatx4 v = i < UA ? Piece<TA, WIDE>::value(st.a[i < UA ? i : 0], in) : Piece<TW, WIDE>::value(st.w[i < UA ? 0 : i - UA], in);
+      const int r = pr + i * (TH / QPR);
+      float* dst = base + (r >> 4) * CH * 256 + (((r & 15) * 4 + ((pk >> 2) & 3)) ^ turn);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dst[j * 64] = v[j];
     }
   };
-  auto put = [&](const Staged& st, int buf) {
+  floatx4 acc[NW][FM][FN];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int e = threadIdx.x + 256 * i;
-      ws[buf][0][e / GR_K][e % GR_K] = st.w[i];
-      if (GATED) ws[buf][GATED ? 1 : 0][e / GR_K][e % GR_K] = st.u[i];
-    }
+  for (int w = 0; w < NW; ++w)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int e = threadIdx.x + 256 * i;
-      as[buf][e / GR_K][e % GR_K] = st.a[i];
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[w][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int buf) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const float* at = lds + buf * ROWS * BK + ((lane * 4) ^ (c * (64 / CH)));
+      floatx4 a[FM], w[NW][FN];
+#pragma unroll
+      for (int i = 0; i < FM; ++i) a[i] = *(const floatx4*)(at + ((wm * FM + i) * CH + c) * 256);
+#pragma unroll
+      for (int z = 0; z < NW; ++z)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) w[z][j] = *(const floatx4*)(at + ((WM * FM + (z * WN + wn) * FN + j) * CH + c) * 256);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)  // k = 16 c + 4 q .. + 3
+#pragma unroll
+        for (int z = 0; z < NW; ++z)
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[z][i][j] = mfma_f32(w[z][j][q], a[i][q], acc[z][i][j]);
     }
   };
-  float acc[2] = {0.f, 0.f}, acc2[2] = {0.f, 0.f};
-  const int turns = (K + GR_K - 1) / GR_K;
-  Staged st;
-  fetch(st, 0);
-  put(st, 0);
+  const int stages = (K + BK - 1) / BK;
+  Set s0, s1;
+  fetch(s0, 0);
+  fetch(s1, BK);
+  put(s0, 0, 0);
   __syncthreads();
-  for (int turn = 0; turn < turns; ++turn) {
-    const int buf = turn & 1;
-    if (turn + 1 < turns) fetch(st, (turn + 1) * GR_K);
-#pragma unroll 8
-    for (int k = 0; k < GR_K; ++k) {
-      const float wv = ws[buf][0][r][k];
-      const float uv = GATED ? ws[buf][GATED ? 1 : 0][r][k] : 0.f;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const float av = as[buf][q + 8 * i][k];
-        acc[i] = fmaf(av, wv, acc[i]);
-        if (GATED) acc2[i] = fmaf(av, uv, acc2[i]);
-      }
-    }
-    if (turn + 1 < turns) put(st, buf ^ 1);
+  for (int s = 0; s < stages; s += 2) {
+    fetch(s0, (s + 2) * BK);  // beyond the end: some place inside the rows, never multiplied
+    multiply(0);
+    put(s1, 1, (s + 1) * BK);
+    __syncthreads();
+    if (s + 1 >= stages) break;
+    fetch(s1, (s + 3) * BK);
+    multiply(1);
+    put(s0, 0, (s + 2) * BK);
     __syncthreads();
   }
-  const int n = n0 + r;
-  if (n >= N) return;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-    if (q + 8 * i < M) finish_output<GATED>(acc[i], acc2[i], q + 8 * i, n, bias, bias_dtype, out, out_dtype, ldo, epilogue, gs);
+  for (int i = 0; i < FM; ++i) {
+    const int m = m0 + (wm * FM + i) * 16 + (lane & 15);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int n = n0 + (wn * FN + j) * 16 + (lane >> 4) * 4;
+      if (m < M) finish_four<GATED>(acc[0][i][j], acc[NW - 1][i][j], m, n, N, bias, bias_dtype, out, out_dtype, ldo, epilogue, gs);
+    }
+  }
 }
 
-template <typename TA, typename TW>
-static void launch_rows(const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype, void* out,
-                        int out_dtype, int ldo, int M, int N, int K, int epilogue, GateSpec gs, hipStream_t stream) {
-  dim3 grid((N + GR_ROWS - 1) / GR_ROWS);
-  if (W2)
-    gemm_rows_kernel<TA, TW, true><<<grid, 256, 0, stream>>>((const TA*)A, lda, (const TW*)W, (const TW*)W2, bias,
-                                                             bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs);
-  else
-    gemm_rows_kernel<TA, TW, false><<<grid, 256, 0, stream>>>((const TA*)A, lda, (const TW*)W, nullptr, bias,
-                                                              bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs);
+// Up to 16 rows (decode steps of the 32-bit path). An output's chain is 8 cycles per k (a 16 x 16 x 4 product takes 32), so
+// a product of few weight rows is bound by that chain (3,072 k: 11 us) as long as nothing else stands in it: a workgroup
+// owns 16 weight rows and all activation rows, one wave (two with the gated epilogue, one per weight matrix) does nothing
+// but read fragments from LDS and multiply, and three others keep two turns of 16 CH k on their way from memory (1 KB of
+// weights per instruction: 16 rows x 64 bytes) and write the turn that arrived to LDS, transposed, in the half that is
+// not being multiplied. One wave that loads, transposes with lane swaps (v_permlane16/32_swap) and multiplies took twice
+// the chain.
+template <typename TA, typename TW, bool GATED, bool WIDE>
+__global__ __launch_bounds__(GATED ? 320 : 256) void gemm_f32_rows_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W,
+                                                                        const TW* __restrict__ W2, const void* __restrict__ bias,
+                                                                        int bias_dtype, void* __restrict__ out, int out_dtype,
+                                                                        int ldo, int M, int N, int K, int epilogue, GateSpec gs) {
+  constexpr int NC = GATED ? 2 : 1, CPP = GATED ? 3 : 4, CH = 3 * CPP;  // multiplying waves; chunks of 16 k per loading wave, per turn
+  __shared__ __align__(16) float lds[2][CH][NC + 1][256];             // a chunk's activations, then its weights
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * 16;
+  const int r = lane & 15, quad = lane >> 4;
+  const int turns = (K + CH * 16 - 1) / (CH * 16);
+  if (wave >= NC) {
+    const int c0 = (wave - NC) * CPP;
+    const TA* arow = A + (size_t)min(r, M - 1) * lda;
+    const TW* wrow = W + (size_t)min(n0 + r, N - 1) * K;
+    const TW* urow = GATED ? W2 + (size_t)min(n0 + r, N - 1) * K : wrow;
+    struct Set {
+      typename Piece<TA, WIDE>::type a[CPP];
+      typename Piece<TW, WIDE>::type w[CPP * NC];
+    };
+    auto fetch = [&](Set& st, int t) {  // beyond the end: some place inside the rows, never multiplied
+#pragma unroll
+      for (int c = 0; c < CPP; ++c) {
+        const int k = (t * CH + c0 + c) * 16 + quad * 4;
+        st.w[c] = Piece<TW, WIDE>::load(wrow, k, K);
+        if (GATED) st.w[CPP * (NC - 1) + c] = Piece<TW, WIDE>::load(urow, k, K);
+        st.a[c] = Piece<TA, WIDE>::load(arow, k, K);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto put = [&](const Set& st, int t) {
+#pragma unroll
+      for (int c = 0; c < CPP; ++c) {
+        const bool in = (t * CH + c0 + c) * 16 + quad * 4 < K;
+#pragma unroll
+        for (int z = 0; z <= NC; ++z) {
+          const floatx4 v = z == 0 ? Piece<TA, WIDE>::value(st.a[c], in) : Piece<TW, WIDE>::value(st.w[(z ? z - 1 : 0) * CPP + c], in);
+          float* dst = &lds[t & 1][c0 + c][z][r * 4 + quad];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) dst[j * 64] = v[j];  // k = 4 quad + j: step `quad` of lane group j
+        }
+      }
+    };
+    Set s0, s1;
+    fetch(s0, 0);
+    fetch(s1, 1);
+    put(s0, 0);
+    __syncthreads();
+    for (int t = 0; t < turns; t += 2) {
+      fetch(s0, t + 2);
+      put(s1, t + 1);
+      __syncthreads();
+      if (t + 1 >= turns) break;
+      fetch(s1, t + 3);
+      put(s0, t + 2);
+      __syncthreads();
+    }
+    if (GATED) __syncthreads();
+    return;
+  }
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+  for (int t = 0; t < turns; ++t) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const floatx4 a = *(const floatx4*)&lds[t & 1][c][0][lane * 4], w = *(const floatx4*)&lds[t & 1][c][1 + wave][lane * 4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc = mfma_f32(w[q], a[q], acc);
+    }
+    __syncthreads();
+  }
+  floatx4 up = acc;
+  if (GATED) {
+    floatx4* meet = (floatx4*)&lds[0][0][0][0];  // the last turn has been read
+    if (wave) meet[lane] = acc;
+    __syncthreads();
+    if (wave) return;
+    up = meet[lane];
+  }
+  const int n = n0 + quad * 4;
+  if (r < M) finish_four<GATED>(acc, up, r, n, N, bias, bias_dtype, out, out_dtype, ldo, epilogue, gs);
 }
 
 #define GEMM_ROWS_MAX 16
+
+// Measured (fp32 operands, one product alone, against the vector-unit kernels that stood here): 2,048 x 4,096 x 4,096 1,029 ->
+// 590 us (117 TFLOP/s; a library product reaches 154), 847 rows of N = 1,024 and K = 2,048 337 -> 51, K = 3,072 503 -> 73,
+// 40 rows of the same 168 -> 20; up to 16 rows: N = 1,024 at K = 2,048 / 3,072 40 / 59 -> 12.5 / 17 us, N = 4,096 at K =
+// 12,288 229 -> 71, the head of 151,936 x 1,024 218 -> 182 (3.4 TB/s).
+//
+// The tile is the one with the smallest estimated time: rounds of workgroups (one per compute unit) times the tile's
+// products, the smaller tiles a little dearer for their share of loads. K cannot be cut (one accumulator per output), so
+// where large tiles leave compute units idle only smaller ones fill them.
+struct F32Tile {
+  int rows, cols;  // of the output
+};
+static int f32_tile(long M, long N, bool is_gated) {
+  static const double price[3] = {1.0, 1.1, 1.4};  // 128 x 128, 64 x 64, 32 x 32 (gated: half the columns of the first two)
+  const F32Tile plain[3] = {{128, 128}, {64, 64}, {32, 32}}, pairs[3] = {{128, 64}, {64, 32}, {32, 32}};
+  int cus = jllm_compute_units();
+  if (cus <= 0) cus = 256;
+  int best = 0;
+  double least = 0.0;
+  for (int i = 0; i < 3; ++i) {
+    const F32Tile t = is_gated ? pairs[i] : plain[i];
+    const long rows = (M + t.rows - 1) / t.rows, groups = rows * ((N + t.cols - 1) / t.cols);
+    const double cost = (double)((groups + cus - 1) / cus) * t.rows * t.cols * price[i];
+    if (i == 0 || (cost < least && rows <= 65535)) best = i, least = cost;
+  }
+  return best;
+}
+
+extern "C" int jllm_f32_tile(int M, int N, int is_gated) { return f32_tile(M, N, is_gated != 0); }
+
+struct F32Args {
+  const void *A, *W, *W2, *bias;
+  void* out;
+  int lda, bias_dtype, out_dtype, ldo, M, N, K, epilogue;
+  GateSpec gs;
+};
+
+template <typename TA, typename TW, bool GATED, int WM, int WN, int FM, int FN, int BK, bool WIDE>
+static int launch_f32_tile(const F32Args& g, hipStream_t stream) {
+  constexpr int TM = WM * FM * 16, TN = WN * FN * 16;
+  constexpr size_t smem = (size_t)2 * (TM + (GATED ? 2 : 1) * TN) * BK * sizeof(float);
+  static_assert(smem <= 65536, "no LDS beyond what a launch gets unasked");
+  dim3 grid((g.N + TN - 1) / TN, (g.M + TM - 1) / TM);
+  if (grid.y > 65535) JLLM_FAIL("gemm: M=%d is too large for this kernel", g.M);
+  gemm_f32_tile_kernel<TA, TW, GATED, WM, WN, FM, FN, BK, WIDE><<<grid, WM * WN * 64, smem, stream>>>(
+      (const TA*)g.A, g.lda, (const TW*)g.W, (const TW*)g.W2, g.bias, g.bias_dtype, g.out, g.out_dtype, g.ldo, g.M, g.N, g.K, g.epilogue, g.gs);
+  return 0;
+}
+
+template <typename TA, typename TW, bool WIDE>
+static int launch_f32(const F32Args& g, hipStream_t stream) {
+  if (g.M <= GEMM_ROWS_MAX) {
+    dim3 grid((g.N + 15) / 16);
+    if (g.W2)
+      gemm_f32_rows_kernel<TA, TW, true, WIDE><<<grid, 320, 0, stream>>>((const TA*)g.A, g.lda, (const TW*)g.W, (const TW*)g.W2, g.bias,
+                                                                         g.bias_dtype, g.out, g.out_dtype, g.ldo, g.M, g.N, g.K, g.epilogue, g.gs);
+    else
+      gemm_f32_rows_kernel<TA, TW, false, WIDE><<<grid, 256, 0, stream>>>((const TA*)g.A, g.lda, (const TW*)g.W, nullptr, g.bias,
+                                                                         g.bias_dtype, g.out, g.out_dtype, g.ldo, g.M, g.N, g.K, g.epilogue, g.gs);
+    return 0;
+  }
+  const int tile = f32_tile(g.M, g.N, g.W2 != nullptr);
+  if (g.W2)
+    return tile == 0   ? launch_f32_tile<TA, TW, true, 2, 4, 4, 1, 32, WIDE>(g, stream)
+           : tile == 1 ? launch_f32_tile<TA, TW, true, 4, 2, 1, 1, 64, WIDE>(g, stream)
+                       : launch_f32_tile<TA, TW, true, 2, 2, 1, 1, 64, WIDE>(g, stream);
+  return tile == 0   ? launch_f32_tile<TA, TW, false, 2, 4, 4, 2, 32, WIDE>(g, stream)
+         : tile == 1 ? launch_f32_tile<TA, TW, false, 2, 4, 2, 1, 64, WIDE>(g, stream)
+                     : launch_f32_tile<TA, TW, false, 2, 2, 1, 1, 128, WIDE>(g, stream);
+}
 
 extern "C" int jllm_gemm_generic(const void* A, int a_dtype, int lda, const void* W, const void* W2, int w_dtype,
                                  const void* bias, int bias_dtype, void* out, int out_dtype, int ldo, int M, int N,
@@ -215,34 +388,15 @@ extern "C" int jllm_gemm_generic(const void* A, int a_dtype, int lda, const void
   if (epilogue < 0 || epilogue > 2) JLLM_FAIL("gemm: epilogue %d", epilogue);
   if ((epilogue == 2) != (W2 != nullptr)) JLLM_FAIL("gemm: the gated epilogue needs exactly two weight matrices");
   if (epilogue == 1 && out_dtype != JLLM_F32) JLLM_FAIL("gemm: the accumulate epilogue adds into fp32");
-  if (M <= GEMM_ROWS_MAX) {
-    JLLM_DISPATCH_1(a_dtype, TA, {
-      JLLM_DISPATCH_1(w_dtype, TW, {
-        launch_rows<TA, TW>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, stream);
-      })
-    })
-    JLLM_CHECK_LAUNCH("gemm_rows");
-    return 0;
-  }
-  const bool tall = M > 64;  // tiles of 128 rows
-  dim3 grid((N + GBN - 1) / GBN, tall ? (M + 127) / 128 : (M + 63) / 64);
-  if (grid.y > 65535) JLLM_FAIL("gemm: M=%d is too large for this kernel", M);
+  const F32Args g = {A, W, W2, bias, out, lda, bias_dtype, out_dtype, ldo, M, N, K, epilogue, gs};
+  // 16 bytes (fp32) or 8 bytes (bf16) at a time where every row of both operands starts on such a boundary and ends on one
+  const size_t abytes = a_dtype == JLLM_F32 ? 16 : 8, wbytes = w_dtype == JLLM_F32 ? 16 : 8;
+  const bool wide = (K & 3) == 0 && (lda & 3) == 0 && (uintptr_t)A % abytes == 0 && (uintptr_t)W % wbytes == 0 && (uintptr_t)W2 % wbytes == 0;
+  int rc = 0;
   JLLM_DISPATCH_1(a_dtype, TA, {
-    JLLM_DISPATCH_1(w_dtype, TW, {
-      if (W2 && tall)
-        gemm_generic_kernel<TA, TW, true, 8><<<grid, 256, 0, stream>>>((const TA*)A, lda, (const TW*)W, (const TW*)W2, bias,
-                                                                        bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs);
-      else if (W2)
-        gemm_generic_kernel<TA, TW, true, 4><<<grid, 256, 0, stream>>>((const TA*)A, lda, (const TW*)W, (const TW*)W2, bias,
-                                                                        bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs);
-      else if (tall)
-        gemm_generic_kernel<TA, TW, false, 8><<<grid, 256, 0, stream>>>((const TA*)A, lda, (const TW*)W, nullptr, bias,
-                                                                         bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs);
-      else
-        gemm_generic_kernel<TA, TW, false, 4><<<grid, 256, 0, stream>>>((const TA*)A, lda, (const TW*)W, nullptr, bias,
-                                                                         bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs);
-    })
+    JLLM_DISPATCH_1(w_dtype, TW, { rc = wide ? launch_f32<TA, TW, true>(g, stream) : launch_f32<TA, TW, false>(g, stream); })
   })
+  if (rc != 0) return rc;
   JLLM_CHECK_LAUNCH("gemm_generic");
   return 0;
 }

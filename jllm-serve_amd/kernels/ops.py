@@ -435,7 +435,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, w2: Optional[torch.Tensor] = None,
     EPI_STORE writes ``out_dtype``; EPI_ADD adds into the fp32 ``out`` (the residual stream); EPI_GATED
     writes gate(a @ w.T, a @ w2.T) with the gate function of code ``gate`` (``GATE_FUNCTIONS``; 0 = SiLU times the
     second product) and its parameter ``gate_limit`` where it has one.
-    ``exact`` forces the plain-FMA fp32-accumulation kernel. ``a`` may be a ``NormedRows``.
+    ``exact`` forces the true fp32 kernel (chains of multiply-adds in ascending k). ``a`` may be a ``NormedRows``.
     """
     normed = None
     if isinstance(a, NormedRows):
@@ -710,7 +710,7 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0) -> bool:
     """The bf16 matrix-core kernels: a weight-streaming one for up to 16 rows, another for up to 64; for many rows
     the two-group kernel with 256 x 256 tiles where enough of them fill the GPU (`_pingpong_plan`), else the other
     tiled kernel (with K cut over several workgroups when the output has few tiles). Each declines shapes it does
-    not take; then the plain-FMA kernel runs."""
+    not take; then the fp32 kernel runs."""
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         return False
     M, K = a.shape

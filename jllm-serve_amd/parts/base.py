@@ -59,7 +59,7 @@ class BuildContext:
     dtype: torch.dtype  # activations and cache: torch.float32 or torch.bfloat16
     device: torch.device
     max_positions: int  # longest sequence the engine will hold
-    exact: bool = False  # float32 runs: plain-FMA kernels only
+    exact: bool = False  # float32 runs: kernels whose sums are chains of fp32 multiply-adds only
 
 
 class Part:

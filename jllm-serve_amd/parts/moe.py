@@ -178,7 +178,7 @@ class RoutedMoe(Part):
     def _run(self, xb, residual, step, overwrite):
         s, exact = self.spec, self.build.exact
         T = xb.shape[0]
-        # fp32 logits: plain FMAs for an fp32 router, the matrix cores' exact products for a bf16 one
+        # fp32 logits: the fp32 kernel for an fp32 router, the matrix cores' exact products for a bf16 one
         zz = ops.gemm(xb, self.w_router, bias=self.b_router, out_dtype=torch.float32, exact=self.w_router.dtype == torch.float32)
         z = zz[:, :s.experts]
         shared_rows = self.shared.output(xb, step) if self.shared is not None else None

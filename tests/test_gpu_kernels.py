@@ -268,6 +268,32 @@ def test_gemm_rows_do_not_depend_on_the_batch(ops):
     assert torch.allclose(few, many, rtol=1e-4, atol=1e-4) and torch.allclose(few, some, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (3, 100, 203), (16, 49, 772), (17, 33, 100), (65, 130, 192), (33, 1030, 36),
+                                   (700, 1100, 68), (2041, 4090, 40)])
+@pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16])
+def test_float32_products_are_one_chain_of_multiply_adds(ops, M, N, K, wdt):
+    """Every tile of the 32-bit products, at its edges: an output has the bits of one fp32 accumulator that takes its
+    multiply-adds in ascending k. Operands of 12 (8) bits: a product and an accumulator then add without rounding in
+    float64 (2^-44 .. 2^6), so the chain is restated there with one rounding to fp32 per step, exactly. The gated form
+    gives, in any batch, the bits it gives its rows in batches of 16."""
+    assert [ops.library().jllm_f32_tile(m, n, 0) for m, n in ((33, 1030), (700, 1100), (2041, 4090))] == [2, 1, 0]
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M + N + K)
+
+    def short(*shape):
+        return ((torch.randn(*shape, device=DEV, generator=gen) * 512).round() / 512).to(wdt).float()
+
+    a, w, w2 = short(M, K), short(N, K), short(N, K)
+    want = torch.zeros(M, N, device=DEV)
+    for k in range(K):
+        want = (want.double() + a[:, k:k + 1].double() * w[:, k].double()).float()
+    assert torch.equal(ops.gemm(a, w.to(wdt), exact=True), want)
+    gated = ops.gemm(a, w.to(wdt), w2=w2.to(wdt), epilogue=ops.EPI_GATED, exact=True)
+    for at in range(0, M, max(16, M // 4)):
+        few = ops.gemm(a[at:at + 16].contiguous(), w.to(wdt), w2=w2.to(wdt), epilogue=ops.EPI_GATED, exact=True)
+        assert torch.equal(few, gated[at:at + 16])
+
+
 def test_gemm_refuses_bad_arguments(ops):
     a = torch.randn(4, 32, device=DEV)
     w = torch.randn(8, 31, device=DEV)
