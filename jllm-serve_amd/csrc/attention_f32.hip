@@ -1,0 +1,406 @@
+// Causal grouped-query attention over a paged cache, fp32, head size 128: the two kernels that the 32-bit path takes at
+// the head size of its models. A row's result has the same bits from either of them and from the general kernel
+// (attention_generic.hip), whatever the step's other rows are: the walk over the keys (64-key blocks aligned to absolute
+// positions, wave w of four takes the blocks c with c % 4 == w), the order of every sum (dot products in ascending dims, the
+// block's probabilities over a tree of lanes 32, 16, .. 1 apart, weighted sums in ascending keys, the waves' results
+// in the order of the waves) and what is one multiply-add are the general kernel's. Cache layout and table as there.
+//
+//  * single rows (decode steps): a workgroup per row and up to four heads of a kv head, a lane per key. The general kernel
+//    waits for a handful of 16-byte loads at a time (two blocks of 64 keys took 50 us); here a lane requests its whole
+//    key row at once, and a block's values in four groups of 16 keys, each on its way while the one before is used.
+//  * many rows (portions): a workgroup takes 16 query vectors (rows of one request x the heads of a kv head), so a key is
+//    read once for all of them instead of once per row, and both products run on the matrix cores' fp32 form, whose sums
+//    are chains of multiply-adds in ascending order (see gemm_generic.hip).
+#include <math.h>
+
+#include "common.h"
+
+#define AF_HD 128
+#define AF_WAVES 4
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+struct AttF32 {
+  const float* q;
+  float* out;
+  const float *k, *v;
+  const int *table, *row_req, *positions;
+  int ldq, ldo, max_blocks, n_tokens, H, Hkv, page_size, window;
+  float scale;
+};
+
+// where position j of the request with this table row lies, in rows of AF_HD
+__device__ __forceinline__ int cache_row(const AttF32& A, const int* __restrict__ tbl, int kvh, int j) {
+  return (tbl[j / A.page_size] * A.Hkv + kvh) * A.page_size + j % A.page_size;
+}
+
+// ---------------------------------------------------------------------------------------------- single rows
+
+template <int GC>
+__global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_rows_kernel(AttF32 A) {
+  __shared__ __align__(16) float qs[GC][AF_HD];
+  __shared__ float mg[AF_WAVES][GC][2 + AF_HD];  // every wave's maximum, sum and weighted sums
+  const int t = blockIdx.x, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int G = A.H / A.Hkv, chunks = (G + GC - 1) / GC;
+  const int kvh = blockIdx.y / chunks;
+  const int h0 = kvh * G + (blockIdx.y % chunks) * GC;
+  const int gn = min(GC, kvh * G + G - h0);  // a spare place does the last head again and is not stored
+  const int pos = A.positions[t];
+  const int* tbl = A.table + (size_t)A.row_req[t] * A.max_blocks;
+  const int first = A.window > 0 ? max(0, pos + 1 - A.window) : 0;
+  const int b_first = first >> 6;
+  int blk = b_first + ((wave - b_first) & (AF_WAVES - 1));
+  // every lane names a key inside the row's range: those beyond it repeat the nearest one with probability 0
+  auto row_of = [&](int b) { return cache_row(A, tbl, kvh, min(max(b * 64 + lane, first), pos)); };
+  int row = row_of(blk);
+  for (int i = threadIdx.x; i < GC * AF_HD; i += 64 * AF_WAVES)
+    qs[i / AF_HD][i % AF_HD] = A.q[(size_t)t * A.ldq + (size_t)(h0 + min(i / AF_HD, gn - 1)) * AF_HD + i % AF_HD];
+  __syncthreads();
+  float acc[GC][2], m[GC], l[GC];
+#pragma unroll
+  for (int g = 0; g < GC; ++g) m[g] = -INFINITY, l[g] = 0.f, acc[g][0] = acc[g][1] = 0.f;
+  for (; blk * 64 <= pos; blk += AF_WAVES) {
+    const int c0 = blk * 64, kj = c0 + lane;
+    const bool valid = kj >= first && kj <= pos;
+    const floatx4* kr = (const floatx4*)(A.k + (size_t)row * AF_HD);
+    floatx4 kv[AF_HD / 4];
+#pragma unroll
+    for (int i = 0; i < AF_HD / 4; ++i) kv[i] = kr[i];
+    __builtin_amdgcn_sched_barrier(0);
+    auto fetch = [&](float (&vv)[16][2], int jb) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const float* vr = A.v + (size_t)__builtin_amdgcn_readlane(row, jb + u) * AF_HD;
+        vv[u][0] = vr[lane];
+        vv[u][1] = vr[lane + 64];
+      }
+    };
+    float d[GC], p[GC];
+#pragma unroll
+    for (int g = 0; g < GC; ++g) d[g] = 0.f;
+#pragma unroll
+    for (int i0 = 0; i0 < AF_HD / 4; i0 += 4) {  // (four at a time: the queries' LDS reads would take all registers)
+#pragma unroll
+      for (int i = i0; i < i0 + 4; ++i)
+#pragma unroll
+        for (int g = 0; g < GC; ++g) {
+          const floatx4 qv = *(const floatx4*)&qs[g][4 * i];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) d[g] = fmaf(qv[e], kv[i][e], d[g]);
+        }
+#pragma unroll
+      for (int g = 0; g < GC; ++g) asm volatile("" : "+v"(d[g]));  // (nor does the chain sink below to where its sum is used)
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    float va[16][2], vb[16][2];
+    fetch(va, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < GC; ++g) {
+#pragma clang fp contract(off)
+      const float s = valid ? d[g] * A.scale : -INFINITY;
+      const float m_new = fmaxf(m[g], wave_max(s));
+      p[g] = valid ? expf(s - m_new) : 0.f;
+      const float alpha = expf(m[g] - m_new);
+      l[g] = fmaf(l[g], alpha, wave_sum(p[g]));
+      acc[g][0] *= alpha;
+      acc[g][1] *= alpha;
+      m[g] = m_new;
+    }
+    const int j0 = max(0, first - c0), j1 = min(63, pos - c0);
+    auto use = [&](const float (&vv)[16][2], int jb) {
+#pragma unroll
+      for (int u4 = 0; u4 < 16; u4 += 4) {
+        if (jb + u4 + 3 < j0 || jb + u4 > j1) continue;  // (in fours, as the general kernel: p = 0 of a key outside is multiplied)
+#pragma unroll
+        for (int u = u4; u < u4 + 4; ++u)
+#pragma unroll
+          for (int g = 0; g < GC; ++g) {
+            const float pj = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p[g]), jb + u));
+            acc[g][0] = fmaf(pj, vv[u][0], acc[g][0]);
+            acc[g][1] = fmaf(pj, vv[u][1], acc[g][1]);
+          }
+      }
+    };
+    fetch(vb, 16);
+    __builtin_amdgcn_sched_barrier(0);
+    use(va, 0);
+    fetch(va, 32);
+    __builtin_amdgcn_sched_barrier(0);
+    use(vb, 16);
+    fetch(vb, 48);
+    const int next = blk + AF_WAVES;
+    if (next * 64 <= pos) row = row_of(next);
+    __builtin_amdgcn_sched_barrier(0);
+    use(va, 32);
+    use(vb, 48);
+  }
+#pragma unroll
+  for (int g = 0; g < GC; ++g) {
+    if (lane == 0) mg[wave][g][0] = m[g], mg[wave][g][1] = l[g];
+    mg[wave][g][2 + lane] = acc[g][0];
+    mg[wave][g][2 + lane + 64] = acc[g][1];
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < gn * AF_HD; i += 64 * AF_WAVES) {
+    const int g = i / AF_HD, dim = i % AF_HD;
+    float mm = mg[0][g][0], ll = mg[0][g][1], x = mg[0][g][2 + dim];
+#pragma unroll
+    for (int w = 1; w < AF_WAVES; ++w) {
+#pragma clang fp contract(off)
+      const float om = mg[w][g][0], ol = mg[w][g][1];
+      if (ol == 0.f) continue;  // that wave had no key
+      const float m_new = fmaxf(mm, om);
+      const float ca = expf(mm - m_new), cb = expf(om - m_new);
+      ll = fmaf(ll, ca, ol * cb);
+      x = fmaf(x, ca, mg[w][g][2 + dim] * cb);
+      mm = m_new;
+    }
+    A.out[(size_t)t * A.ldo + (size_t)(h0 + g) * AF_HD + dim] = x * (1.0f / ll);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------- many rows
+
+// lane group q (of 16 lanes) holds x[j] = X[q][j]; afterwards x[s] = X[s][q]. v_permlane32_swap exchanges the upper half of
+// its first register with the lower half of its second, v_permlane16_swap the odd groups with the even ones.
+__device__ __forceinline__ floatx4 lanes_transposed(floatx4 x) {
+  auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[0]), __float_as_uint(x[2]), false, false);
+  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[1]), __float_as_uint(x[3]), false, false);
+  auto lo = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  auto hi = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return floatx4{__uint_as_float(lo[0]), __uint_as_float(lo[1]), __uint_as_float(hi[0]), __uint_as_float(hi[1])};
+}
+
+__device__ __forceinline__ floatx4 mfma_f32(float a, float b, floatx4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// Column c of a wave's products is query vector c: row c / G of the tile, head c % G of the kv head; lane l holds column
+// l % 16. Scores: D[key][c] += K[key][dims] q[c][dims], four tiles of 16 keys, 32 steps of four dims each; lane l then has
+// keys 16 t + 4 (l / 16) + i. Weighted sums: D[dim][c] += V^T[dim][key] p[c][key]; a lane's 16 bytes of V are four
+// neighbouring dims of one key, which go to four tiles (a tile's row r is dim 4 r + j of its 64 dims), so V needs no
+// transposition; keys and probabilities are transposed over the lane groups in registers. A tile whose rows belong to
+// several requests is walked once per request.
+__global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_tiles_kernel(AttF32 A, int rows) {
+  __shared__ __align__(16) float mg[AF_WAVES][16][4 + AF_HD];  // every wave's maximum, sum (and two spare places), weighted sums
+  const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int G = A.H / A.Hkv, kvh = blockIdx.y;
+  const int t0 = blockIdx.x * rows, n = min(rows, A.n_tokens - t0);
+  const int ri = col / G;             // this lane's row of the tile ...
+  const int head = kvh * G + col % G;  // ... and head
+  floatx4 qf[AF_HD / 16];             // the lane's query vector at dims 16 c + 4 s + quad
+  {
+    const floatx4* qr = (const floatx4*)(A.q + (size_t)(t0 + min(ri, n - 1)) * A.ldq + (size_t)head * AF_HD);
+#pragma unroll
+    for (int c = 0; c < AF_HD / 16; ++c) qf[c] = qr[4 * c + quad];
+#pragma unroll
+    for (int c = 0; c < AF_HD / 16; ++c) qf[c] = lanes_transposed(qf[c]);
+  }
+  for (int i0 = 0; i0 < n;) {  // the rows of one request
+    const int req = A.row_req[t0 + i0];
+    int i1 = i0, low = 0x7fffffff, high = -1, last_first = 0, low_pos = 0x7fffffff;
+    for (; i1 < n && A.row_req[t0 + i1] == req; ++i1) {
+      const int p = A.positions[t0 + i1], f = A.window > 0 ? max(0, p + 1 - A.window) : 0;
+      low = min(low, f), high = max(high, p), last_first = max(last_first, f), low_pos = min(low_pos, p);
+    }
+    const int* tbl = A.table + (size_t)req * A.max_blocks;
+    const bool mine = ri >= i0 && ri < i1;
+    const int pos = mine ? A.positions[t0 + ri] : -1;  // a lane of other rows sees no key
+    const int first = mine && A.window > 0 ? max(0, pos + 1 - A.window) : 0;
+    floatx4 acc[2][4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[h][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    const int b_first = low >> 6;
+    for (int blk = b_first + ((wave - b_first) & (AF_WAVES - 1)); blk * 64 <= high; blk += AF_WAVES) {
+      const int c0 = blk * 64;
+      const int row = cache_row(A, tbl, kvh, min(max(c0 + lane, low), high));  // key c0 + lane, or the nearest that some row sees
+      floatx4 s[4];
+      floatx4 kf[4][AF_HD / 16];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const floatx4* kr = (const floatx4*)(A.k + (size_t)__shfl(row, 16 * t + col, 64) * AF_HD);
+#pragma unroll
+        for (int c = 0; c < AF_HD / 16; ++c) kf[t][c] = kr[4 * c + quad];
+        s[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < 4; t += 2) {
+#pragma unroll
+        for (int c = 0; c < AF_HD / 16; ++c) {
+          const floatx4 ka = lanes_transposed(kf[t][c]), kb = lanes_transposed(kf[t + 1][c]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            s[t] = mfma_f32(ka[e], qf[c][e], s[t]);
+            s[t + 1] = mfma_f32(kb[e], qf[c][e], s[t + 1]);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // values of 16 keys (t): lane's key 16 t + 4 u + quad, dims 64 h + 4 col .. + 3
+      auto fetch = [&](floatx4 (&vv)[4][2], int t) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const float* vr = A.v + (size_t)__shfl(row, 16 * t + 4 * u + quad, 64) * AF_HD + 4 * col;
+          vv[u][0] = *(const floatx4*)vr;
+          vv[u][1] = *(const floatx4*)(vr + 64);
+        }
+      };
+      floatx4 va[4][2], vb[4][2];
+      fetch(va, 0);
+      fetch(vb, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      const bool any = c0 <= pos && c0 + 63 >= first;  // this lane's row sees a key of the block
+      float m_new, alpha;
+      {
+#pragma clang fp contract(off)
+        float top = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int key = c0 + 16 * t + 4 * quad + i;
+            s[t][i] = key >= first && key <= pos ? s[t][i] * A.scale : -INFINITY;
+            top = fmaxf(top, s[t][i]);
+          }
+        top = fmaxf(top, __shfl_xor(top, 16, 64));
+        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        m_new = any ? fmaxf(m, top) : m;
+        alpha = any ? expf(m - m_new) : 1.f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[t][i] = s[t][i] == -INFINITY ? 0.f : expf(s[t][i] - m_new);
+        // the sum over the block's 64 keys, key k with k ^ 32 first, then k ^ 16, .. k ^ 1
+        float x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          x[i] = (s[0][i] + s[2][i]) + (s[1][i] + s[3][i]);
+          x[i] += __shfl_xor(x[i], 32, 64);
+          x[i] += __shfl_xor(x[i], 16, 64);
+        }
+        l = fmaf(l, alpha, (x[0] + x[2]) + (x[1] + x[3]));
+        m = m_new;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[h][j][i] *= alpha;
+      }
+      // a key that some of the rows do not see is multiplied by 0 for them, which an infinite value would not survive
+      const bool partial = c0 < last_first || c0 + 63 > low_pos;
+      auto use = [&](const floatx4 (&vv)[4][2], int t) {
+        const floatx4 pt = lanes_transposed(s[t]);  // pt[u]: key 16 t + 4 u + quad
+        if (partial) {
+          bool odd = false;
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) odd = odd || !(fabsf(vv[u][h][j]) < INFINITY);
+          if (__ballot(odd)) {  // (rare) key by key, for the rows that see it
+#pragma unroll 1
+            for (int k = 0; k < 16; ++k) {
+              const int key = c0 + 16 * t + k;
+              const float pk = k < 8 ? (k < 4 ? pt[0] : pt[1]) : (k < 12 ? pt[2] : pt[3]);
+              const float pe = __shfl(pk, col + 16 * (k & 3), 64);
+              const float* vr = A.v + (size_t)__shfl(row, 16 * t + k, 64) * AF_HD;
+#pragma unroll
+              for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                  for (int i = 0; i < 4; ++i)
+                    if (key >= first && key <= pos) acc[h][j][i] = fmaf(pe, vr[64 * h + 4 * (4 * quad + i) + j], acc[h][j][i]);
+            }
+            return;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[h][j] = mfma_f32(vv[u][h][j], pt[u], acc[h][j]);
+      };
+      use(va, 0);
+      fetch(va, 2);
+      __builtin_amdgcn_sched_barrier(0);
+      use(vb, 1);
+      fetch(vb, 3);
+      __builtin_amdgcn_sched_barrier(0);
+      use(va, 2);
+      use(vb, 3);
+    }
+    if (quad == 0) mg[wave][col][0] = m, mg[wave][col][1] = l;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)  // dims 64 h + 4 (4 quad + i) .. + 3 lie in the four tiles
+        *(floatx4*)&mg[wave][col][4 + 64 * h + 16 * quad + 4 * i] = floatx4{acc[h][0][i], acc[h][1][i], acc[h][2][i], acc[h][3][i]};
+    __syncthreads();
+    {
+      const int c = threadIdx.x >> 4, r = c / G, d0 = (threadIdx.x & 15) * 8;
+      if (r >= i0 && r < i1) {
+        float mm = mg[0][c][0], ll = mg[0][c][1], x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = mg[0][c][4 + d0 + i];
+#pragma unroll
+        for (int w = 1; w < AF_WAVES; ++w) {
+#pragma clang fp contract(off)
+          const float om = mg[w][c][0], ol = mg[w][c][1];
+          if (ol == 0.f) continue;
+          const float m_new = fmaxf(mm, om);
+          const float ca = expf(mm - m_new), cb = expf(om - m_new);
+          ll = fmaf(ll, ca, ol * cb);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[i] = fmaf(x[i], ca, mg[w][c][4 + d0 + i] * cb);
+          mm = m_new;
+        }
+        const float inv = 1.0f / ll;
+        float* o = A.out + (size_t)(t0 + r) * A.ldo + (size_t)(kvh * G + c % G) * AF_HD + d0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = x[i] * inv;
+      }
+    }
+    __syncthreads();
+    i0 = i1;
+  }
+}
+
+// fp32, head size 128, 16-byte aligned rows; returns 1 for what it leaves to the general kernel. `n_requests` bounds
+// row_req. Which kernel: a tile holds 16 / G rows of one request, and reads their keys once; where the rows are spread
+// over as many requests (steps of single tokens) there is nothing to share and a workgroup per row has more waves.
+extern "C" int jllm_paged_attention_f32(const void* q, int ldq, void* out, int ldo, const void* kcache, const void* vcache,
+                                        const int* block_table, int max_blocks, const int* row_req, const int* positions,
+                                        int n_tokens, int n_requests, int H, int Hkv, int hd, int page_size, int window,
+                                        float scale, hipStream_t stream) {
+  if (n_tokens <= 0) return 0;
+  if (hd != AF_HD || H <= 0 || Hkv <= 0 || H % Hkv != 0 || page_size <= 0 || max_blocks <= 0 || window < 0 || n_requests <= 0) return 1;
+  if (ldq < H * hd || ldo < H * hd || (ldq & 3) || H > 65535) return 1;
+  if (((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache) & 15) return 1;
+  const AttF32 A = {(const float*)q, (float*)out, (const float*)kcache, (const float*)vcache, block_table, row_req, positions,
+                    ldq, ldo, max_blocks, n_tokens, H, Hkv, page_size, window, scale};
+  const int G = H / Hkv;
+  if (G <= 8 && n_tokens >= 4 * n_requests) {
+    const int rows = 16 / G;
+    attention_f32_tiles_kernel<<<dim3((n_tokens + rows - 1) / rows, Hkv), 64 * AF_WAVES, 0, stream>>>(A, rows);
+  } else {  // heads share a workgroup where the step still has two workgroups for every compute unit, as in the general kernel
+    int cus = jllm_compute_units();
+    if (cus <= 0) cus = 256;
+    if (G >= 3 && (long)n_tokens * Hkv * ((G + 3) / 4) >= 2L * cus)
+      attention_f32_rows_kernel<4><<<dim3(n_tokens, Hkv * ((G + 3) / 4)), 64 * AF_WAVES, 0, stream>>>(A);
+    else if (G >= 2 && (long)n_tokens * Hkv * ((G + 1) / 2) >= 2L * cus)
+      attention_f32_rows_kernel<2><<<dim3(n_tokens, Hkv * ((G + 1) / 2)), 64 * AF_WAVES, 0, stream>>>(A);
+    else
+      attention_f32_rows_kernel<1><<<dim3(n_tokens, H), 64 * AF_WAVES, 0, stream>>>(A);
+  }
+  JLLM_CHECK_LAUNCH("paged_attention_f32");
+  return 0;
+}

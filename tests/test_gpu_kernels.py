@@ -510,6 +510,38 @@ ATT_CASES = [  # H, Hkv, hd, page, window
 ]
 
 
+@pytest.mark.parametrize("H,Hkv,page,window", [(16, 8, 16, 0), (4, 4, 4, 70), (8, 2, 16, 100), (10, 2, 32, 0), (24, 3, 16, 300), (17, 1, 16, 0)])
+def test_float32_attention_gives_the_general_kernels_bits(ops, H, Hkv, page, window):
+    """Head size 128 in fp32: single rows and tiles of rows (requests that end inside a tile, one-row requests between
+    portions, heads that fill 16 columns or leave some empty, more than 8 heads to a kv head) against the general kernel,
+    bit for bit. One value is infinite: the rows in front of it must not feel it."""
+    lens = [1, 200, 37, 64, 5, 333, 1]
+    kc, vc, table, _, _ = make_cache(len(lens), lens, Hkv, 128, page, torch.float32, seed=H)
+    vc[int(table[5, 100 // page]), 0, 100 % page, 77] = float("inf")
+    g = torch.Generator().manual_seed(2)
+    news = [1, 130, 37, 3, 1, 333, 1]  # the last rows of every request
+    row_req = torch.tensor([r for r, n in enumerate(news) for _ in range(n)], dtype=torch.int32, device=DEV)
+    positions = torch.tensor([p for c, n in zip(lens, news) for p in range(c - n, c)], dtype=torch.int32, device=DEV)
+    q = (torch.randn(len(positions), H * 128, generator=g) * 1.5).to(DEV)
+    zeros = torch.zeros(H, device=DEV)  # a bias of nothing: only the general kernel takes one
+
+    def attend(rows, slopes=None):
+        return ops.paged_attention(q[rows].contiguous(), kc, vc, table, row_req[rows].contiguous(), positions[rows].contiguous(), H,
+                                   Hkv, 128, window, 128 ** -0.5, exact=True, slopes=slopes)
+
+    every = torch.arange(len(positions), device=DEV)
+    want = attend(every, zeros)
+    ops.reset_stats()
+    forms = [(every, attend(every))] + [(every[a:a + n], attend(every[a:a + n])) for a, n in ((0, 7), (60, 20), (200, 27), (len(every) - 1, 1))]
+    assert ops.stats()["ran"] == {"jllm_paged_attention_f32": 5}
+    for rows, got in forms:
+        ref = want[rows]
+        fine = torch.isfinite(ref)  # (a row that does see the infinite value: infinite or NaN)
+        assert torch.equal(torch.isfinite(got), fine) and torch.equal(got[fine], ref[fine])
+    seen = (row_req == 5) & (positions >= 100) & ((positions < 100 + window) if window else True)
+    assert bool(torch.isfinite(want[~seen]).all()) and not bool(torch.isfinite(want[seen]).all())
+
+
 @pytest.mark.parametrize("H,Hkv,hd,window", [(12, 3, 32, 0), (10, 2, 48, 70), (6, 3, 64, 0), (8, 8, 16, 0)])
 def test_general_attention_gives_a_row_the_same_bits_in_any_step(ops, H, Hkv, hd, window):
     """The general kernel (the 32-bit path) takes up to four query heads of a kv head in one workgroup when the step
