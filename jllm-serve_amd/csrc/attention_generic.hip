@@ -205,9 +205,15 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void paged_attention_generic_kernel
   }
 }
 
+// attention_f32.hip; returns 1 for what it leaves to the kernel above
+extern "C" int jllm_attention_f32(const void* q, int ldq, void* out, int ldo, const void* kcache, const void* vcache, const int* block_table,
+                                  int max_blocks, const int* row_req, const int* positions, int n_tokens, int n_requests, int H,
+                                  int Hkv, int hd, int page_size, int window, float scale, hipStream_t stream);
+
+// `n_requests`: rows of the block table
 extern "C" int jllm_paged_attention_generic(const void* q, int ldq, void* out, int ldo, int dtype, const void* kcache,
                                             const void* vcache, const int* block_table, int max_blocks,
-                                            const int* row_req, const int* positions, int n_tokens, int H, int Hkv,
+                                            const int* row_req, const int* positions, int n_tokens, int n_requests, int H, int Hkv,
                                             int hd, int page_size, int window, float scale, const float* slopes,
                                             hipStream_t stream) {
   if (n_tokens <= 0) return 0;
@@ -217,6 +223,11 @@ extern "C" int jllm_paged_attention_generic(const void* q, int ldq, void* out, i
   if (ldq < H * hd || ldo < H * hd) JLLM_FAIL("attention: row strides %d/%d < %d", ldq, ldo, H * hd);
   if (window < 0) JLLM_FAIL("attention: window %d", window);
   if (H > 65535) JLLM_FAIL("attention: too many heads");
+  if (dtype == JLLM_F32 && !slopes) {  // the same bits, faster, at the head size of the 32-bit path's models
+    const int rc = jllm_attention_f32(q, ldq, out, ldo, kcache, vcache, block_table, max_blocks, row_req, positions, n_tokens,
+                                      n_requests, H, Hkv, hd, page_size, window, scale, stream);
+    if (rc <= 0) return rc;
+  }
   // up to four heads of a kv head per workgroup where the accumulators fit in registers (head sizes up to 256) and
   // the step still has two workgroups for every compute unit (a head's result is the same bits either way)
   const int G = H / Hkv;

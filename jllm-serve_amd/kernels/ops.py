@@ -62,8 +62,7 @@ def _declare(lib) -> None:
         "jllm_rmsnorm": [_P, _P, _I, _I, _P, _I, _F, _P, _I, _I, _P],
         "jllm_gemm_generic": [_P, _I, _I, _P, _P, _I, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _P],
         "jllm_qk_norm_rope_store": [_P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _F, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P],
-        "jllm_paged_attention_generic": [_P, _I, _P, _I, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P],
-        "jllm_paged_attention_f32": [_P, _I, _P, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P],
+        "jllm_paged_attention_generic": [_P, _I, _P, _I, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P, _P],
         "jllm_argmax": [_P, _I, _I, _I, _P, _P, _P],
         "jllm_sample": [_P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P],
         "jllm_adjust_logits": [_P, _I, _P, _P, _I, _F, _F, _F, _P, _P, _I, _P],
@@ -805,16 +804,11 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                                                                       positions, heads, kv_heads, head_dim, window,
                                                                       scale, meta):
         return out
-    if q.dtype == torch.float32 and slopes is None and _try(
-            "jllm_paged_attention_f32", _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_cache), _ptr(v_cache),
-            _ptr(block_table), block_table.shape[1], _ptr(row_req), _ptr(positions), T, block_table.shape[0], heads, kv_heads,
-            head_dim, k_cache.shape[2], int(window), float(scale), _stream()):
-        return out  # the same bits as the general kernel's
     if not exact and slopes is None:
         _count("general", "jllm_paged_attention_generic")
     _call("jllm_paged_attention_generic", _ptr(q), q.stride(0), _ptr(out), out.stride(0), _code(q.dtype), _ptr(k_cache),
-          _ptr(v_cache), _ptr(block_table), block_table.shape[1], _ptr(row_req), _ptr(positions), T, heads, kv_heads,
-          head_dim, k_cache.shape[2], int(window), float(scale), _ptr(slopes), _stream())
+          _ptr(v_cache), _ptr(block_table), block_table.shape[1], _ptr(row_req), _ptr(positions), T, block_table.shape[0],
+          heads, kv_heads, head_dim, k_cache.shape[2], int(window), float(scale), _ptr(slopes), _stream())
     return out
 
 

@@ -531,9 +531,7 @@ def test_float32_attention_gives_the_general_kernels_bits(ops, H, Hkv, page, win
 
     every = torch.arange(len(positions), device=DEV)
     want = attend(every, zeros)
-    ops.reset_stats()
     forms = [(every, attend(every))] + [(every[a:a + n], attend(every[a:a + n])) for a, n in ((0, 7), (60, 20), (200, 27), (len(every) - 1, 1))]
-    assert ops.stats()["ran"] == {"jllm_paged_attention_f32": 5}
     for rows, got in forms:
         ref = want[rows]
         fine = torch.isfinite(ref)  # (a row that does see the infinite value: infinite or NaN)
