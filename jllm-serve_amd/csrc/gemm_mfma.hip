@@ -1,8 +1,8 @@
 // out[M,N] = A[M,K] * W[N,K]^T for many rows (prompt portions): bf16 operands staged through LDS, fp32
-// accumulation on the matrix cores (v_mfma_f32_32x32x16_bf16).
+// accumulation on the matrix cores (v_mfma_f32_16x16x32_bf16, as in gemm_pingpong.hip, whose outputs have the same bits).
 //
 // Two tile shapes. The small one: 4 waves in a 2 x 2 arrangement over a 128 x 128 output tile, each wave owning
-// 64 x 64 = four 32 x 32 accumulators; two such workgroups share a compute unit. The large one, for products
+// 64 x 64 outputs; two such workgroups share a compute unit. The large one, for products
 // with many tiles: 8 waves in a 2 x 4 arrangement over 256 x 256, each wave owning 128 x 64 (fewer LDS bytes per
 // multiply). K advances in steps of 64 through two LDS buffers: while the waves multiply out of
 // one, the 16-byte global loads of the next step are already in registers and are stored into the other.
@@ -23,7 +23,7 @@
 #define TPCS (TBK / 8)  // 16-byte pieces per tile row
 #define TLD (TBK + 8)   // LDS row stride in elements
 
-// WGM x WGN waves, each with FM x FN accumulators of 32 x 32 (FN = 2 for the gated epilogue: gate and up)
+// WGM x WGN waves, each with 32 FM x 32 FN outputs (FN = 2 for the gated epilogue: gate and up)
 template <bool GATED, int WGM, int WGN, int FM, int FN, bool DEEP>
 __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
@@ -84,13 +84,12 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
   const int nk_per = (nk_all + gridDim.z - 1) / gridDim.z;
   const int kt0 = blockIdx.z * nk_per;
   const int nk = max(0, min(nk_all, kt0 + nk_per) - kt0);
-  floatx16 acc[FM][FN];
+  constexpr int RM = 2 * FM, CN = 2 * FN;  // a wave's blocks of 16 rows and of 16 columns
+  floatx4 acc[RM][CN];
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+  for (int i = 0; i < RM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    for (int j = 0; j < CN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int j = 0; j < PA; ++j) aptr[j] += (size_t)kt0 * TBK;
 #pragma unroll
@@ -110,38 +109,39 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
 #pragma unroll
     for (int j = 0; j < PB; ++j) *(u32x4*)(Bs + (size_t)buf * TBN * TLD + (size_t)(lrow + TRSTEP * j) * TLD + lpc * 8) = r.b[j];
   };
-  const int fr = lane & 31;        // fragment row / column
-  const int fk = (lane >> 5) * 8;  // fragment k offset
+  const int fr = lane & 15;        // fragment row / column
+  const int fk = (lane >> 4) * 8;  // fragment k offset
   auto multiply = [&](int cur) {
-    const bf16_t* Ac = As + (size_t)cur * TBM * TLD + (size_t)(wm * FM * 32 + fr) * TLD + fk;
-    const bf16_t* Bc = Bs + (size_t)cur * TBN * TLD + (size_t)(wn * FN * 32 + fr) * TLD + fk;
+    const bf16_t* Ac = As + (size_t)cur * TBM * TLD + (size_t)(wm * RM * 16 + fr) * TLD + fk;
+    const bf16_t* Bc = Bs + (size_t)cur * TBN * TLD + (size_t)(wn * CN * 16 + fr) * TLD + fk;
     // the weight fragment goes in as the first operand: the accumulator then holds the tile transposed (rows =
     // output columns), so a lane owns four consecutive output columns of one row and stores them at once
-    constexpr int KS = DEEP ? 2 : TBK / 16;  // k16 steps whose fragments are in registers together
+    constexpr int KS = FM > 2 ? 1 : TBK / 32;  // k32 steps whose fragments are in registers together
 #pragma unroll
-    for (int k0 = 0; k0 < TBK / 16; k0 += KS) {
-      u32x4 af[KS][FM], bf[KS][FN];
+    for (int k0 = 0; k0 < TBK / 32; k0 += KS) {
+      u32x4 af[KS][RM], bf[KS][CN];
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i) af[ks][i] = *(const u32x4*)(Ac + i * 32 * TLD + (k0 + ks) * 16);
+        for (int j = 0; j < CN; ++j) bf[ks][j] = *(const u32x4*)(Bc + j * 16 * TLD + (k0 + ks) * 32);
 #pragma unroll
-        for (int j = 0; j < FN; ++j) bf[ks][j] = *(const u32x4*)(Bc + j * 32 * TLD + (k0 + ks) * 16);
+        for (int i = 0; i < RM; ++i) af[ks][i] = *(const u32x4*)(Ac + i * 16 * TLD + (k0 + ks) * 32);
       }
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+        for (int i = 0; i < RM; ++i)
 #pragma unroll
-          for (int j = 0; j < FN; ++j) acc[i][j] = mfma32(bf[ks][j], af[ks][i], acc[i][j]);
+          for (int j = 0; j < CN; ++j) acc[i][j] = mfma16(bf[ks][j], af[ks][i], acc[i][j]);
       }
-      // the order of issue: the LDS reads of step ks + 1 go out before the multiplies of step ks
-      __builtin_amdgcn_sched_group_barrier(0x100, FM + FN, 0);
+      // the order of issue: what the first two rows of multiplies need, then a read behind every two multiplies
+      __builtin_amdgcn_sched_group_barrier(0x100, CN + 2, 0);
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        if (ks + 1 < KS) __builtin_amdgcn_sched_group_barrier(0x100, FM + FN, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, FM * FN, 0);
+      for (int r = CN + 2; r < KS * (RM + CN); ++r) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
+      __builtin_amdgcn_sched_group_barrier(0x008, KS * RM * CN - 2 * (KS * (RM + CN) - CN - 2), 0);
     }
   };
   if (nk > 0) {
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
       }
     }
   }
-  tile_epilogue<GATED, FM, FN, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
+  tile_epilogue<GATED, RM, CN, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
                                          (int)blockIdx.z, (int)gridDim.z);
 }
 

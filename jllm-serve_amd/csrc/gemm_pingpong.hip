@@ -1,21 +1,24 @@
-// out[M,N] = A[M,K] * W[N,K]^T for many rows, bf16 on the matrix cores (v_mfma_f32_32x32x16_bf16), built so that the
+// out[M,N] = A[M,K] * W[N,K]^T for many rows, bf16 on the matrix cores (v_mfma_f32_16x16x32_bf16), built so that the
 // matrix cores of a compute unit never wait for operands:
 //
-//  * A workgroup of 8 waves (2 x 4) owns a 256 x 256 output tile (a wave 128 x 64: FM = 4 by FN = 2 accumulators of
-//    32 x 32). K advances in stages of 32 through a ring of NS stages in LDS.
+//  * A workgroup of 8 waves (2 x 4) owns a 256 x 256 output tile (a wave 128 x 64: 8 by 4 accumulators of 16 x 16). K
+//    advances in stages of 32 through a ring of NS stages in LDS. (The 16 x 16 x 32 form rather than 32 x 32 x 16: the
+//    full chip is bound by its power, and a multiply-add of the smaller form reads and writes half as many accumulator
+//    bytes. MFMAs alone on random operands run at 2.04 PFLOP/s against 1.85; this kernel with either form: 2,048 rows of
+//    the 8B shape's gate/up 340 -> 329 us, qkv 109 -> 103, down 201 -> 188, 8,192^3 923 -> 866 (1.27 PFLOP/s).)
 //  * Global -> LDS without registers: global_load_lds_dwordx4 writes 16 bytes per lane straight into LDS, 1 KB
 //    (16 tile rows of 64 bytes) per instruction, NS - 1 stages ahead of the multiplies. A lane's place in LDS is
 //    fixed by its number, so the bank swizzle is applied on the global side: the lane that fills slot s of row r
 //    fetches the row's 16-byte piece s ^ f(r).
 //  * The waves form two groups, one wave of each on every SIMD, that run half a stage apart: while one group
-//    multiplies (16 MFMAs from registers, nothing else), the other reads the next stage's fragments from LDS and
+//    multiplies (32 MFMAs from registers, nothing else), the other reads the next stage's fragments from LDS and
 //    issues its share of the global loads; a workgroup barrier after every phase keeps them apart. A SIMD's matrix
 //    core so always has a wave with all operands in registers.
 //
 // Phases are the times between two workgroup barriers. In phase 2t group 0 is in its memory phase of stage t (it reads
-// the stage's second half of fragments from LDS and issues the loads of stage t + NS - 1) while group 1 multiplies
-// stage t - 1 and, between the multiplies, reads the first half of stage t's fragments; in phase 2t + 1 the groups
-// have swapped (group 0 multiplies stage t and reads the first half of stage t + 1). So stage s is read from phase
+// the second half of the stage's row fragments from LDS and issues the loads of stage t + NS - 1) while group 1 multiplies
+// stage t - 1 and, between the multiplies, reads the rest of stage t's fragments; in phase 2t + 1 the groups
+// have swapped (group 0 multiplies stage t and reads the first fragments of stage t + 1). So stage s is read from phase
 // 2s - 1 on and must have landed when that phase starts: before the barrier in front of it every wave waits until
 // its own loads of stages <= s are complete (loads complete in order; group 0 has issued two stages beyond s by
 // then, group 1 one). The loads of stage t + NS - 1 go to the slot of stage t - 1, whose last reader (group 1, second
@@ -30,6 +33,7 @@
 #define PP_BK 32
 #define PP_ROW_BYTES (PP_BK * 2)  // a tile row in LDS: 64 bytes = 4 pieces of 16
 #define PP_WAVES 8
+#define PP_MUL 3  // multiplies between two LDS reads of the multiply phase
 
 // The piece of row r that lies in slot s is s ^ pp_swz(r): 16 lanes that read the same piece of 16 consecutive rows,
 // and 8 lanes of 8 rows, then cover every bank once, whichever of the two the LDS takes per pass.
@@ -43,8 +47,8 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
     const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N, int K,
     int epilogue, GateSpec gs, float* __restrict__ partial) {
-  constexpr int WGM = 2, WGN = 4, FN = 2;
-  constexpr int TBM = WGM * FM * 32, TBN = WGN * FN * 32;
+  constexpr int WGM = 2, WGN = 4, RM = 2 * FM, CN = 4;  // a wave's blocks of 16 rows and of 16 columns
+  constexpr int TBM = WGM * RM * 16, TBN = WGN * CN * 16;
   constexpr int STAGE = (TBM + TBN) * PP_ROW_BYTES;
   constexpr int LA = TBM / 16 / PP_WAVES, LB = TBN / 16 / PP_WAVES;  // load instructions per wave and stage
   constexpr int LPW = LA + LB;
@@ -107,23 +111,16 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
     }
   };
 
-  // ---- LDS side: fragment (row block i, k16 step ks): row = block * 32 + lane % 32, piece = 2 ks + lane / 32
-  const int fr = lane & 31, half = lane >> 5;
-  int aoff[2], boff[2];
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    const int ra = wm * FM * 32 + fr, rb = wn * FN * 32 + fr;  // + 32 i leaves pp_swz unchanged
-    aoff[ks] = ra * PP_ROW_BYTES + (((2 * ks + half) ^ pp_swz(ra)) * 16);
-    boff[ks] = TBM * PP_ROW_BYTES + rb * PP_ROW_BYTES + (((2 * ks + half) ^ pp_swz(rb)) * 16);
-  }
+  // ---- LDS side: fragment of a block of 16 rows: row = block * 16 + lane % 16, piece = lane / 16 (16 bytes: 8 of the stage's k)
+  const int ra = wm * RM * 16 + (lane & 15), rb = wn * CN * 16 + (lane & 15);  // + 16 i leaves pp_swz unchanged
+  const int aoff = ra * PP_ROW_BYTES + (((lane >> 4) ^ pp_swz(ra)) * 16);
+  const int boff = TBM * PP_ROW_BYTES + rb * PP_ROW_BYTES + (((lane >> 4) ^ pp_swz(rb)) * 16);
 
-  floatx16 acc[FM][FN];
+  floatx4 acc[RM][CN];
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+  for (int i = 0; i < RM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    for (int j = 0; j < CN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   // ---- prologue: NS - 1 stages on their way, stages 0 and 1 landed
 #pragma unroll
@@ -137,22 +134,27 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
-  // fragments: f0 = the k16 step 0 of the stage being multiplied, f1 = its step 1, fn = step 0 of the next stage (read
-  // during the multiplies); the loop is unrolled by two so that f0 and fn swap names instead of being copied
-  u32x4 a0[FM], b0[FN], a1[FM], b1[FN], an[FM], bn[FN];
-  auto read = [&](int t, int ks, u32x4 (&af)[FM], u32x4 (&bf)[FN]) {
-    const unsigned char* st = smem + (t % NS) * STAGE;
+  // fragments of a stage: the weights' and the first half of the rows' (read during the multiplies of the stage before), the
+  // second half of the rows' (read in the memory phase); the loop is unrolled by two so that a stage's and the next
+  // one's swap names instead of being copied
+  constexpr int RH = RM / 2;
+  u32x4 a0[RH], b0[CN], a1[RH], an[RH], bn[CN];
+  auto read_rows = [&](int t, int half, u32x4 (&af)[RH]) {
+    const unsigned char* st = smem + (t % NS) * STAGE + aoff + half * RH * 16 * PP_ROW_BYTES;
 #pragma unroll
-    for (int i = 0; i < FM; ++i) af[i] = *(const u32x4*)(st + aoff[ks] + i * 32 * PP_ROW_BYTES);
-#pragma unroll
-    for (int j = 0; j < FN; ++j) bf[j] = *(const u32x4*)(st + boff[ks] + j * 32 * PP_ROW_BYTES);
+    for (int i = 0; i < RH; ++i) af[i] = *(const u32x4*)(st + i * 16 * PP_ROW_BYTES);
   };
-  // one stage of one group. Memory phase: the second half of the stage's fragments, then the global loads (a compute
+  auto read_cols = [&](int t, u32x4 (&bf)[CN]) {
+    const unsigned char* st = smem + (t % NS) * STAGE + boff;
+#pragma unroll
+    for (int j = 0; j < CN; ++j) bf[j] = *(const u32x4*)(st + j * 16 * PP_ROW_BYTES);
+  };
+  // one stage of one group. Memory phase: the second half of the rows' fragments, then the global loads (a compute
   // unit's load pipe takes about 40 cycles per load instruction and a wave waits at the issue while it is busy, so
-  // the LDS reads go first). Multiply phase: 16 MFMAs with the reads of the next stage's first fragments between them.
-  auto stage = [&](int t, u32x4 (&fa0)[FM], u32x4 (&fb0)[FN], u32x4 (&na0)[FM], u32x4 (&nb0)[FN]) {
+  // the LDS reads go first). Multiply phase: 32 MFMAs with the reads of the next stage's first fragments between them.
+  auto stage = [&](int t, u32x4 (&fa0)[RH], u32x4 (&fb0)[CN], u32x4 (&na0)[RH], u32x4 (&nb0)[CN]) {
     const bool more = t + NS - 1 < nk;
-    read(t, 1, a1, b1);
+    read_rows(t, 1, a1);
     __builtin_amdgcn_sched_barrier(0);
     if (more) issue(t + NS - 1);
     // own loads of stage t + 1 must have landed before the barrier that lets group 0 read it during its multiplies:
@@ -168,22 +170,23 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    read(t + 1, 0, na0, nb0);  // beyond the last stage: some slot's bytes, never multiplied
+    read_cols(t + 1, nb0);  // beyond the last stage: some slot's bytes, never multiplied
+    read_rows(t + 1, 0, na0);
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < RH; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j) acc[i][j] = mfma32(fb0[j], fa0[i], acc[i][j]);
+      for (int j = 0; j < CN; ++j) acc[i][j] = mfma16(fb0[j], fa0[i], acc[i][j]);
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < RH; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j) acc[i][j] = mfma32(b1[j], a1[i], acc[i][j]);
-    // order of issue: two multiplies, then one LDS read, ...; the rest of the multiplies
+      for (int j = 0; j < CN; ++j) acc[RH + i][j] = mfma16(fb0[j], a1[i], acc[RH + i][j]);
+    // order of issue: PP_MUL multiplies, then one LDS read, ...; the rest of the multiplies
 #pragma unroll
-    for (int r = 0; r < FM + FN; ++r) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+    for (int r = 0; r < RH + CN; ++r) {
+      __builtin_amdgcn_sched_group_barrier(0x008, PP_MUL, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, 2 * FM * FN - 2 * (FM + FN), 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, RM * CN - PP_MUL * (RH + CN), 0);
     if (group == 1) {  // has issued up to stage t + 3; stage t + 2 must have landed (group 0 reads it after the next barrier but one)
       if (more) {
         PP_VMCNT(1 * LPW);
@@ -195,7 +198,10 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   };
-  if (nk > 0) read(0, 0, a0, b0);
+  if (nk > 0) {
+    read_cols(0, b0);
+    read_rows(0, 0, a0);
+  }
   if (group == 1) {  // half a stage behind
     PP_LGKMCNT0();
     __builtin_amdgcn_s_barrier();
@@ -209,7 +215,7 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   }
-  tile_epilogue<GATED, FM, FN, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
+  tile_epilogue<GATED, RM, CN, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
                                          (int)blockIdx.z, (int)gridDim.z);
 }
 
