@@ -158,6 +158,38 @@ def _attend_plain(qa, rows, R, window, scale, sink, q_pos):
     return torch.einsum("thj,jr->thr", e / den, rows[:, :R])
 
 
+@pytest.mark.parametrize("N,K", [(16, 8), (20, 72), (33 * 4, 520), (48, 1096), (36, 2048), (64, 2128)])
+def test_grouped_products_of_few_rows(N, K):
+    """The experts' products for few rows per expert at the ends of K (whole turns of 512 of a workgroup, parts of one,
+    single pieces of 8) and of N, gated and plain, every row map, against float64: sums of K products of bf16 numbers in
+    fp32 (an error of K 2^-24 of the sum of magnitudes at most), rounded once where the output is bf16."""
+    from jllm_serve_amd.kernels import ops
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(N + K)
+    E, top, T = 5, 2, 23
+    w, w2 = (torch.randn(E, N, K, device="cuda", generator=gen).bfloat16() for _ in range(2))
+    table = torch.rand(T, E, device="cuda", generator=gen).argsort(dim=1)[:, :top].to(torch.int32).contiguous()
+    table[:20] = torch.tensor([3, 1], dtype=torch.int32, device="cuda")  # an expert with more rows than one tile holds
+    routing = ops.moe_route(None, table, E)
+    experts = table.long().reshape(-1)
+    x = torch.randn(T, K, device="cuda", generator=gen).bfloat16()
+    rows = x.double().repeat_interleave(top, dim=0)
+    y, u = (torch.einsum("ak,ank->an", rows, t.double()[experts]) for t in (w, w2))
+    room = K * 2.0 ** -24 * torch.einsum("ak,ank->an", rows.abs(), w.double()[experts].abs())
+    place = routing.place_of.long()
+    out = torch.full((T * top, N), float("nan"), device="cuda")
+    ops.moe_gemm(x, w, routing, out=out, in_map=1, out_map=0)
+    assert bool(((out[place].double() - y).abs() <= room + 1e-30).all())
+    by_assignment = torch.full_like(out, float("nan"))
+    ops.moe_gemm(x, w, routing, out=by_assignment, in_map=1, out_map=1)
+    assert torch.equal(by_assignment, out[place])
+    h = torch.full((T * top, N), float("nan"), device="cuda", dtype=torch.bfloat16)
+    ops.moe_gemm(x, w, routing, w2=w2, out=h, in_map=1, out_map=0)
+    want = y * torch.sigmoid(y) * u
+    scale = (y.abs() + 1.0) * (u.abs() + 1.0) * (1.0 + room.max())
+    assert bool(((h[place].double() - want).abs() <= 2.0 ** -8 * want.abs() + 4.0 * room.max() * scale + 2.0 ** -20 * scale).all())
+
+
 @pytest.mark.parametrize("dtype, fast", [("float32", False), ("bfloat16", True), ("bfloat16", False)])
 @pytest.mark.parametrize("H, R, Dr, page", [(4, 32, 16, 8), (5, 48, 8, 16), (16, 64, 32, 32), (40, 16, 16, 4), (3, 24, 6, 8)])
 def test_attention_kernels_on_crafted_keys(dtype, fast, H, R, Dr, page):
