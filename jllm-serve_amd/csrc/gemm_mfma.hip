@@ -24,12 +24,21 @@
 #define TLD (TBK + 8)   // LDS row stride in elements
 
 // WGM x WGN waves, each with 32 FM x 32 FN outputs (FN = 2 for the gated epilogue: gate and up)
-template <bool GATED, int WGM, int WGN, int FM, int FN, bool DEEP>
+// What the per-head form (HEADS) takes beside the operands: head h = blockIdx.z multiplies the rows at A + h * a_stride with
+// its own weights (W [heads][N][K]) and writes bf16 at out + h * o_stride, times sigmoid(gate[row][h * N + column]) where a
+// gate is given.
+struct HeadsArgs {
+  int a_stride, o_stride;
+  const bf16_t* gate;
+  int ld_gate;
+};
+
+template <bool GATED, int WGM, int WGN, int FM, int FN, bool DEEP, bool HEADS = false>
 __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
     const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N, int K,
     int epilogue, GateSpec gs, float* __restrict__ partial, const int* __restrict__ groups, const int* __restrict__ row_map,
-    int row_div) {
+    int row_div, HeadsArgs ha) {
   static_assert(FN == 2, "a wave's columns are two 32-wide accumulators (gate and up with the gated epilogue)");
   constexpr int NT = WGM * WGN * 64;
   constexpr int TBM = WGM * FM * 32, TBN = WGN * FN * 32;
@@ -53,6 +62,10 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
     const size_t at = (size_t)groups[3 * blockIdx.y] * N * K;
     W += at;
     if (GATED) W2 += at;
+  }
+  if (HEADS) {
+    A += (size_t)blockIdx.z * ha.a_stride;
+    W += (size_t)blockIdx.z * N * K;
   }
   const int n0 = blockIdx.x * (GATED ? TBN / 2 : TBN);  // output columns covered by this workgroup start here
   // global -> register staging: piece c = tid + NT j: row c / TPCS, 16 bytes number c % TPCS
@@ -81,8 +94,8 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
   }
   // gridDim.z > 1: this workgroup multiplies only its share of K and leaves an fp32 partial tile
   const int nk_all = K / TBK;
-  const int nk_per = (nk_all + gridDim.z - 1) / gridDim.z;
-  const int kt0 = blockIdx.z * nk_per;
+  const int nk_per = HEADS ? nk_all : (nk_all + gridDim.z - 1) / gridDim.z;
+  const int kt0 = HEADS ? 0 : blockIdx.z * nk_per;
   const int nk = max(0, min(nk_all, kt0 + nk_per) - kt0);
   constexpr int RM = 2 * FM, CN = 2 * FN;  // a wave's blocks of 16 rows and of 16 columns
   floatx4 acc[RM][CN];
@@ -183,6 +196,29 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
       }
     }
   }
+  if (HEADS) {
+    bf16_t* o = (bf16_t*)out + (size_t)blockIdx.z * ha.o_stride;
+#pragma unroll
+    for (int i = 0; i < RM; ++i) {
+      const int m = m0 + (wm * RM + i) * 16 + (lane & 15);
+      if (m >= M) continue;
+#pragma unroll
+      for (int j = 0; j < CN; ++j) {
+        const int n = n0 + (wn * CN + j) * 16 + (lane >> 4) * 4;
+        if (n >= N) continue;  // N is a multiple of four
+        floatx4 v = acc[i][j];
+        if (ha.gate) {
+          const u32x2 g = *(const u32x2*)(ha.gate + (size_t)m * ha.ld_gate + (size_t)blockIdx.z * N + n);
+          const float gv[4] = {__uint_as_float(g[0] << 16), __uint_as_float(g[0] & 0xffff0000u), __uint_as_float(g[1] << 16),
+                               __uint_as_float(g[1] & 0xffff0000u)};
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] = v[c] / (1.0f + __expf(-gv[c]));
+        }
+        *(u32x2*)(o + (size_t)m * ldo + n) = u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+      }
+    }
+    return;
+  }
   tile_epilogue<GATED, RM, CN, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
                                          (int)blockIdx.z, (int)gridDim.z);
 }
@@ -265,10 +301,10 @@ static int launch_tiled(const void* A, int lda, const void* W, const void* W2, c
   }
   if (W2)
     gemm_mfma_kernel<true, WGM, WGN, FM, FN, DEEP><<<grid, WGM * WGN * 64, smem, stream>>>(
-        (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, nullptr, nullptr, 1);
+        (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, nullptr, nullptr, 1, HeadsArgs{});
   else
     gemm_mfma_kernel<false, WGM, WGN, FM, FN, DEEP><<<grid, WGM * WGN * 64, smem, stream>>>(
-        (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, nullptr, nullptr, 1);
+        (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, nullptr, nullptr, 1, HeadsArgs{});
   return 0;
 }
 
@@ -338,10 +374,32 @@ extern "C" int jllm_gemm_mfma_grouped_bf16(const void* A, int lda, const void* W
   }
   if (W2)
     gemm_mfma_kernel<true, 2, 2, 2, 2, false><<<grid, 256, smem, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, nullptr, 0, out,
-                                                                           out_dtype, ldo, M, N, K, epilogue, gs, nullptr, tiles, row_map, row_div);
+                                                                           out_dtype, ldo, M, N, K, epilogue, gs, nullptr, tiles, row_map, row_div, HeadsArgs{});
   else
     gemm_mfma_kernel<false, 2, 2, 2, 2, false><<<grid, 256, smem, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, nullptr, nullptr, 0, out, out_dtype,
-                                                                            ldo, M, N, K, epilogue, gs, nullptr, tiles, row_map, row_div);
+                                                                            ldo, M, N, K, epilogue, gs, nullptr, tiles, row_map, row_div, HeadsArgs{});
   JLLM_CHECK_LAUNCH("gemm_mfma_grouped");
+  return 0;
+}
+
+// The per-head products of latent attention for many rows (latent_heads.hip, which checks the arguments): K a multiple of
+// 64, N of 4. Through LDS in tiles of 128 x 128 a row's and a weight's loads are shared by a workgroup; read straight
+// from memory by every wave (64 x 64 outputs each) 2,500 rows of 16 heads took 95 us at 512 x 128 and 47 at 128 x 512.
+int jllm_gemm_mfma_heads(const void* in, int ld_in, int in_hstride, const void* W, void* out, int ld_out, int out_hstride, int M,
+                         int H, int N, int K, const void* gate, int ld_gate, hipStream_t stream) {
+  constexpr int TB = 128;
+  const size_t smem = (size_t)2 * (TB + TB) * TLD * sizeof(bf16_t);
+  static bool configured = false;
+  if (!configured) {
+    if (hipFuncSetAttribute((const void*)gemm_mfma_kernel<false, 2, 2, 2, 2, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+      JLLM_FAIL("gemm_mfma_heads: cannot reserve %zu bytes of LDS", smem);
+    configured = true;
+  }
+  dim3 grid((N + TB - 1) / TB, (M + TB - 1) / TB, H);
+  if (grid.y > 65535) return 1;
+  gemm_mfma_kernel<false, 2, 2, 2, 2, false, true><<<grid, 256, smem, stream>>>(
+      (const bf16_t*)in, ld_in, (const bf16_t*)W, nullptr, nullptr, 0, out, JLLM_BF16, ld_out, M, N, K, 0, GateSpec{}, nullptr, nullptr, nullptr, 1,
+      HeadsArgs{in_hstride, out_hstride, (const bf16_t*)gate, ld_gate});
+  JLLM_CHECK_LAUNCH("gemm_mfma_heads");
   return 0;
 }

@@ -11,10 +11,12 @@
 
 #define LHM_WAVES 4
 
-// RB = 1 (up to 16 rows: a decode step): the four waves of a workgroup take four blocks of 64 outputs of the same 16
-// rows. RB = 4: a wave takes 64 rows by 64 outputs (a weight fragment meets four activation fragments), the four waves
-// four such row blocks.
-template <int RB>
+// RB = 1 (up to 16 rows: a decode step): the four waves of a workgroup take four blocks of 16 outputs of the same 16
+// rows, and request 512 k of weights and activations before the first multiply (with 64 outputs per wave and a few
+// steps ahead, W_uv of 16 heads of 128 x 512 was a chain of four memory latencies: 11.7 us). RB = 4: a wave takes 64 rows by
+// 64 outputs (a weight fragment meets four activation fragments), the four waves four such row blocks.
+// AHEAD: steps of 32 k whose operands are requested together
+template <int RB, int AHEAD>
 __global__ __launch_bounds__(LHM_WAVES * 64) void latent_heads_mfma_kernel(
     const bf16_t* __restrict__ in, int ld_in, int in_hstride, const bf16_t* __restrict__ W, bf16_t* __restrict__ out,
     int ld_out, int out_hstride, int M, int N, int K, int mode, int tail, int rot_dims,
@@ -44,39 +46,45 @@ __global__ __launch_bounds__(LHM_WAVES * 64) void latent_heads_mfma_kernel(
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int sub = lane & 15, q4 = lane >> 4;
   const int t0 = RB == 1 ? m0 : m0 + wave * 64;
-  const int n0 = RB == 1 ? (blockIdx.y * LHM_WAVES + wave) * 64 : blockIdx.y * 64;
+  constexpr int NB = RB == 1 ? 1 : 4;    // blocks of 16 outputs of a wave
+  const int n0 = RB == 1 ? (blockIdx.y * LHM_WAVES + wave) * 16 : blockIdx.y * 64;
   if (t0 >= M || n0 >= N) return;
   const bf16_t* xrow[RB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) xrow[rb] = a + (size_t)min(t0 + 16 * rb + sub, M - 1) * ld_in + 8 * q4;
   const bf16_t* w = W + (size_t)h * N * K + 8 * q4;
-  floatx4 acc[RB][4];
+  floatx4 acc[RB][NB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[rb][b] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    const bool in_k = k0 + 8 * q4 < K;
-    u32x4 xf[RB], wf[4];
+    for (int b = 0; b < NB; ++b) acc[rb][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < K; k0 += 32 * AHEAD) {
+    u32x4 xf[AHEAD][RB], wf[AHEAD][NB];
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) xf[rb] = in_k ? *(const u32x4*)(xrow[rb] + k0) : u32x4{0u, 0u, 0u, 0u};
+    for (int u = 0; u < AHEAD; ++u) {  // (places beyond K and N are read inside the rows; those beyond K count as zeros)
+      const int k = k0 + 32 * u + 8 * q4 < K ? k0 + 32 * u : 0;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int n = n0 + 16 * b + sub;
-      wf[b] = (in_k && n < N) ? *(const u32x4*)(w + (size_t)n * K + k0) : u32x4{0u, 0u, 0u, 0u};
+      for (int rb = 0; rb < RB; ++rb) xf[u][rb] = *(const u32x4*)(xrow[rb] + (k + 8 * q4 < K ? k : -8 * q4));
+#pragma unroll
+      for (int b = 0; b < NB; ++b) wf[u][b] = *(const u32x4*)(w + (size_t)min(n0 + 16 * b + sub, N - 1) * K + (k + 8 * q4 < K ? k : -8 * q4));
     }
+    if (RB == 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
+    for (int u = 0; u < AHEAD; ++u) {
+      const bool in_k = k0 + 32 * u + 8 * q4 < K;
+      const u32x4 none = {0u, 0u, 0u, 0u};
 #pragma unroll
-      for (int b = 0; b < 4; ++b) acc[rb][b] = mfma16(wf[b], xf[rb], acc[rb][b]);
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[rb][b] = mfma16(in_k ? wf[u][b] : none, in_k ? xf[u][rb] : none, acc[rb][b]);
+    }
   }
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     const int t = t0 + 16 * rb + sub;
     if (t >= M) continue;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
+    for (int b = 0; b < NB; ++b) {
       const int n = n0 + 16 * b + 4 * q4;  // this lane's four outputs n .. n + 3 of row t
       if (n >= N) continue;
       float v[4] = {acc[rb][b][0], acc[rb][b][1], acc[rb][b][2], acc[rb][b][3]};
@@ -92,6 +100,10 @@ __global__ __launch_bounds__(LHM_WAVES * 64) void latent_heads_mfma_kernel(
   }
 }
 
+// the products of many rows in tiles through LDS (gemm_mfma.hip); returns 1 when it declines
+int jllm_gemm_mfma_heads(const void* in, int ld_in, int in_hstride, const void* W, void* out, int ld_out, int out_hstride, int M,
+                         int H, int N, int K, const void* gate, int ld_gate, hipStream_t stream);
+
 // returns 0 when it ran, 1 when the shape is not one it takes, -1 on errors
 extern "C" int jllm_latent_heads_bf16(const void* in, int ld_in, int in_hstride, const void* W, void* out, int ld_out,
                                       int out_hstride, int M, int H, int N, int K, int mode, int tail, int rot_dims,
@@ -106,20 +118,31 @@ extern "C" int jllm_latent_heads_bf16(const void* in, int ld_in, int in_hstride,
   if (mode == 1 && ((ld_gate & 3) || ((uintptr_t)gate & 7) || !gate)) return 1;
   if (mode == 0 && tail > 0 && (!positions || (rot_dims && (!cos_t || !sin_t)))) JLLM_FAIL("latent_heads: the rotated tail needs positions and tables");
   const bool few = M <= 16;
-  const int n_blocks = few ? (N + LHM_WAVES * 64 - 1) / (LHM_WAVES * 64) : (N + 63) / 64;
-  const int rows = few ? 16 : LHM_WAVES * 64;
+  // Tiles of 128 rows (the same bits: one accumulator per output, K in steps of 32); the rotated tail then is the only column
+  // of workgroups of the kernel above, a launch of its own. 16 heads of 512 x 128 with a tail: 70 rows 11 us in one
+  // launch, 13 in two, 100 rows 14.1 / 13.8, 300 38 / 14, 2,556 76 / 34; of 128 x 512 without one: 70 rows 14.8 / 13.8,
+  // 2,556 41 / 21.
+  const bool tiled = M > (mode == 0 && tail > 0 ? 96 : 64) && (K & 63) == 0;
+  if (tiled) {
+    const int rc = jllm_gemm_mfma_heads(in, ld_in, in_hstride, W, out, ld_out, out_hstride, M, H, N, K, mode == 1 ? gate : nullptr, ld_gate, stream);
+    if (rc != 0) return rc;
+    if (mode == 1 || tail <= 0) return 0;
+  }
+  const int n_blocks = tiled ? 0 : (N + 63) / 64;
+  const int rows = few || tiled ? 16 : LHM_WAVES * 64;  // (the tail alone: a few elements per thread)
   dim3 grid((M + rows - 1) / rows, n_blocks + ((mode == 0 && tail > 0) ? 1 : 0), H);
   if (grid.y > 65535) return 1;
-  if (few)
-    latent_heads_mfma_kernel<1><<<grid, LHM_WAVES * 64, 0, stream>>>((const bf16_t*)in, ld_in, in_hstride, (const bf16_t*)W,
-                                                                    (bf16_t*)out, ld_out, out_hstride, M, N, K, mode,
-                                                                    mode == 0 ? tail : 0, rot_dims, positions, cos_t, sin_t,
-                                                                    (const bf16_t*)gate, ld_gate, n_blocks);
+#define LHM_LAUNCH(RB, AHEAD)                                                                                                   \
+  latent_heads_mfma_kernel<RB, AHEAD><<<grid, LHM_WAVES * 64, 0, stream>>>(                                                      \
+      (const bf16_t*)in, ld_in, in_hstride, (const bf16_t*)W, (bf16_t*)out, ld_out, out_hstride, M, N, K, mode, mode == 0 ? tail : 0, \
+      rot_dims, positions, cos_t, sin_t, (const bf16_t*)gate, ld_gate, n_blocks)
+  if (!few && !tiled)
+    LHM_LAUNCH(4, 4);
+  else if (K <= 128 || tiled)  // (steps beyond K are multiplied as zeros: no branch stands between a load and the next one)
+    LHM_LAUNCH(1, 4);
   else
-    latent_heads_mfma_kernel<4><<<grid, LHM_WAVES * 64, 0, stream>>>((const bf16_t*)in, ld_in, in_hstride, (const bf16_t*)W,
-                                                                    (bf16_t*)out, ld_out, out_hstride, M, N, K, mode,
-                                                                    mode == 0 ? tail : 0, rot_dims, positions, cos_t, sin_t,
-                                                                    (const bf16_t*)gate, ld_gate, n_blocks);
+    LHM_LAUNCH(1, 16);
+#undef LHM_LAUNCH
   JLLM_CHECK_LAUNCH("latent_heads_bf16");
   return 0;
 }

@@ -158,6 +158,45 @@ def _attend_plain(qa, rows, R, window, scale, sink, q_pos):
     return torch.einsum("thj,jr->thr", e / den, rows[:, :R])
 
 
+@pytest.mark.parametrize("N,K,tail,gated", [(512, 128, 64, False), (128, 512, 0, True), (36, 64, 24, False), (132, 192, 0, True),
+                                            (20, 40, 8, False)])
+def test_heads_products_at_every_row_count(N, K, tail, gated):
+    """The per-head products where their kernel changes (up to 16 rows, up to 64 or 96, tiles of 128 rows beyond) and at odd
+    sizes: against float64, and a row's bits are those it has in any other batch."""
+    from jllm_serve_amd.kernels import ops
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(N + K)
+    H, M = 3, 261
+    x = torch.randn(M, H * (K + tail), device="cuda", generator=gen).bfloat16()
+    w = (torch.randn(H, N, K, device="cuda", generator=gen) * K ** -0.5).bfloat16()
+    gate = torch.randn(M, H * N, device="cuda", generator=gen).bfloat16() if gated else None
+    positions = torch.arange(5, 5 + M, dtype=torch.int32, device="cuda")
+    rot = tail // 8 * 8
+    angle = torch.rand(M + 5, rot // 2, device="cuda", generator=gen) * 6.0
+    cos, sin = torch.cos(angle), torch.sin(angle)
+
+    def heads(n):
+        return ops.latent_heads(x[:n].contiguous(), w, tail=tail, rot_dims=rot, positions=positions[:n].contiguous(),
+                                cos=cos if tail else None, sin=sin if tail else None, gate=gate[:n].contiguous() if gated else None)
+
+    whole = heads(M)
+    for n in (1, 16, 17, 64, 65, 96, 97, 128, 129):
+        assert torch.equal(heads(n), whole[:n]), n
+    rows = x.double().view(M, H, K + tail)
+    want = torch.einsum("mhk,hnk->mhn", rows[..., :K], w.double())
+    if gated:
+        want = want * torch.sigmoid(gate.double().view(M, H, N))
+    got = whole.double().view(M, H, N + tail)
+    room = 2.0 ** -8 * want.abs() + (K * 2.0 ** -24) * torch.einsum("mhk,hnk->mhn", rows[..., :K].abs(), w.double().abs())
+    assert bool(((got[..., :N] - want).abs() <= room).all())
+    if tail:
+        c, s = cos.double()[positions.long()][:, None], sin.double()[positions.long()][:, None]
+        t = rows[..., K:]
+        a, b = t[..., :rot // 2], t[..., rot // 2:rot]
+        turned = torch.cat([a * c - b * s, b * c + a * s, t[..., rot:]], dim=-1)
+        assert bool(((got[..., N:] - turned).abs() <= 2.0 ** -8 * turned.abs() + 2.0 ** -22 * (a.abs().max() + b.abs().max())).all())
+
+
 @pytest.mark.parametrize("N,K", [(16, 8), (20, 72), (33 * 4, 520), (48, 1096), (36, 2048), (64, 2128)])
 def test_grouped_products_of_few_rows(N, K):
     """The experts' products for few rows per expert at the ends of K (whole turns of 512 of a workgroup, parts of one,
