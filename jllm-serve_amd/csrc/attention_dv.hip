@@ -494,56 +494,67 @@ extern "C" int jllm_heads_finish(const void* att, int lda, int att_dtype, int n_
 // matrix-core attention kernel leaves them (attention_dv_mfma.hip). Lane z holds range z's maximum and sum, so the
 // ranges' weights are known after two wave reductions; merging here saves the launch of a merge kernel.
 template <typename TG, typename TW, typename TO>
-__global__ __launch_bounds__(64) void heads_finish_split_kernel(const float* __restrict__ partial, int splits, int maps,
-                                                                int dv, float lambda, int normed, float eps, float norm_mul,
-                                                                const TW* __restrict__ gain, const TG* __restrict__ gate,
-                                                                int ldg, int gate_fn, float out_mul, TO* __restrict__ out,
-                                                                int ldo, int gate_per_head, const float* __restrict__ sinks) {
-  const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
-  float o[4] = {0.f, 0.f, 0.f, 0.f};  // dv <= 256
-  for (int m = 0; m < maps; ++m) {
-    const float* pr = partial + (((size_t)t * gridDim.y + h) * maps + m) * splits * (dv + 2);
-    const float mz = lane < splits ? pr[(size_t)lane * (dv + 2) + dv] : -INFINITY;
-    const float lz = lane < splits ? pr[(size_t)lane * (dv + 2) + dv + 1] : 0.f;
-    const float mx = wave_max(mz);
-    const float wz = mz == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mz - mx);
+__global__ __launch_bounds__(256) void heads_finish_split_kernel(const float* __restrict__ partial, int splits, int maps,
+                                                                 int dv, float lambda, int normed, float eps, float norm_mul,
+                                                                 const TW* __restrict__ gain, const TG* __restrict__ gate,
+                                                                 int ldg, int gate_fn, float out_mul, TO* __restrict__ out,
+                                                                 int ldo, int gate_per_head, const float* __restrict__ sinks) {
+  __shared__ float sums[4];
+  const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, j = threadIdx.x;  // a thread owns one dim (dv <= 256)
+  const int jc = min(j, dv - 1);
+  // everything that does not hang on another load is asked for first: the ranges' maxima and sums (lane z holds range
+  // z's), the first eight ranges' values of both maps, the gate and the gain
+  const float* pr[2];
+  float mz[2], lz[2], v[2][8];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    pr[m] = partial + (((size_t)t * gridDim.y + h) * maps + min(m, maps - 1)) * splits * (dv + 2);
+    const size_t at = (size_t)min(lane, splits - 1) * (dv + 2) + dv;
+    mz[m] = pr[m][at];
+    lz[m] = pr[m][at + 1];
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int z = 0; z < 8; ++z) v[m][z] = pr[m][(size_t)min(z, splits - 1) * (dv + 2) + jc];
+  const float g = gate ? ldf(gate + (size_t)t * ldg, gate_per_head ? (size_t)h : (size_t)h * dv + jc) : 0.f;
+  const float w_gain = gain ? ldf(gain, jc) : 1.0f;
+  float o = 0.f;
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    if (m >= maps) break;
+    const float pm = lane < splits ? mz[m] : -INFINITY;
+    const float mx = wave_max(pm);
+    const float wz = pm == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(pm - mx);
     // a sink is one more term of the denominator: exp(sink) on the scale of the ranges' common maximum
     const float sink_term = sinks ? __builtin_amdgcn_exp2f(sinks[h] * 1.4426950408889634f - mx) : 0.f;
-    const float inv = 1.0f / (wave_sum(lz * wz) + sink_term);
+    const float inv = 1.0f / (wave_sum(lane < splits ? lz[m] * wz : 0.f) + sink_term);
+    float acc = 0.f;
+    for (int z0 = 0; z0 < splits; z0 += 8) {
+      if (z0 > 0) {
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int j = lane + 64 * jj;
-      if (j >= dv) continue;
-      float acc = 0.f;
-#pragma unroll 4
-      for (int z = 0; z < splits; ++z) {
-        const float w = __shfl(wz, z, 64);
-        const float v = pr[(size_t)z * (dv + 2) + j];
-        acc = w != 0.f ? fmaf(v, w, acc) : acc;  // a range without keys left its sums unwritten
+        for (int z = 0; z < 8; ++z) v[m][z] = pr[m][(size_t)min(z0 + z, splits - 1) * (dv + 2) + jc];
       }
-      o[jj] = m == 0 ? acc * inv : o[jj] - lambda * (acc * inv);
+#pragma unroll
+      for (int z = 0; z < 8; ++z) {
+        const float w = z0 + z < splits ? __shfl(wz, z0 + z, 64) : 0.f;
+        acc = w != 0.f ? fmaf(v[m][z], w, acc) : acc;  // a range without keys left its sums unwritten
+      }
     }
+    o = m == 0 ? acc * inv : o - lambda * (acc * inv);
   }
-  float ss = 0.f;
+  float r = 1.0f;
   if (normed) {
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj)
-      if (lane + 64 * jj < dv) ss = fmaf(o[jj], o[jj], ss);
-    ss = wave_sum(ss);
+    const float ss = wave_sum(j < dv ? o * o : 0.f);
+    if (lane == 0) sums[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    r = norm_scale((sums[0] + sums[1]) + (sums[2] + sums[3]), dv, eps) * norm_mul;
   }
-  const float r = normed ? norm_scale(ss, dv, eps) * norm_mul : 1.0f;
-#pragma unroll
-  for (int jj = 0; jj < 4; ++jj) {
-    const int j = lane + 64 * jj;
-    if (j >= dv) continue;
-    float v = o[jj] * r;
-    if (gain) v *= ldf(gain, j);
-    if (gate) {
-      const float z = ldf(gate + (size_t)t * ldg, gate_per_head ? (size_t)h : (size_t)h * dv + j);
-      v *= (gate_fn == 1 ? z : 1.0f) / (1.0f + expf(-z));
-    }
-    stf(out + (size_t)t * ldo, (size_t)h * dv + j, v * out_mul);
-  }
+  if (j >= dv) return;
+  float x = o * r;
+  if (gain) x *= w_gain;
+  if (gate) x *= (gate_fn == 1 ? g : 1.0f) / (1.0f + expf(-g));
+  stf(out + (size_t)t * ldo, (size_t)h * dv + j, x * out_mul);
 }
 
 extern "C" int jllm_heads_finish_split(const float* partial, int splits, int n_tokens, int heads, int maps, int dv, float lambda,
@@ -560,7 +571,7 @@ extern "C" int jllm_heads_finish_split(const float* partial, int splits, int n_t
   JLLM_DISPATCH_1(gate_dtype, TG, {
     JLLM_DISPATCH_1(gain_dtype, TW, {
       JLLM_DISPATCH_1(out_dtype, TO, {
-        heads_finish_split_kernel<TG, TW, TO><<<grid, 64, 0, stream>>>(partial, splits, maps, dv, lambda, normed, eps, norm_mul,
+        heads_finish_split_kernel<TG, TW, TO><<<grid, 256, 0, stream>>>(partial, splits, maps, dv, lambda, normed, eps, norm_mul,
                                                                       (const TW*)gain, (const TG*)gate, ldg, gate_fn, out_mul,
                                                                       (TO*)out, ldo, gate_per_head, sinks);
       })

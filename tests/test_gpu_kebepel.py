@@ -63,6 +63,34 @@ def act_type(dtype):
 # ------------------------------------------------------------------------------------------------ mechanisms alone
 
 
+@pytest.mark.parametrize("channels,biased", [(8, False), (520, True), (2056, False)])
+def test_convolution_of_many_rows(channels, biased):
+    """The convolution's kernel for many bf16 rows (eight rows and eight channels per thread): requests of one to seventy rows
+    that begin and end anywhere in a group of eight, channels that do not fill a workgroup, inputs from the states in front
+    of a request's first rows; against float64, rounded once, and the states that it leaves."""
+    from jllm_serve_amd.kernels import ops
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(channels)
+    rows = [1, 2, 3, 70, 5, 1, 64, 13]
+    n = sum(rows)
+    x = torch.randn(n, channels + 8, device="cuda", generator=gen).bfloat16()[:, :channels]
+    taps = torch.randn(channels, 4, device="cuda", generator=gen).bfloat16()
+    bias = torch.randn(channels, device="cuda", generator=gen).bfloat16() if biased else None
+    state = torch.randn(len(rows) + 2, 3, channels, device="cuda", generator=gen)
+    slots = torch.tensor([4, 1, 0, 7, 2, 9, 5, 3], dtype=torch.int32, device="cuda")
+    row_req = torch.tensor([r for r, k in enumerate(rows) for _ in range(k)], dtype=torch.int32, device="cuda")
+    before = state.clone()
+    y = ops.short_conv(x, taps, state, row_req, slots, len(rows), bias=bias)
+    at = 0
+    for r, k in enumerate(rows):
+        seen = torch.cat([before[slots[r]].double(), x[at:at + k].double()])
+        z = sum(seen[j:j + k] * taps[:, j].double() for j in range(4)) + (bias.double() if biased else 0.0)
+        want = z * torch.sigmoid(z)
+        assert bool(((y[at:at + k].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()), r
+        assert torch.equal(state[slots[r]], seen[-3:].float()), r
+        at += k
+
+
 @pytest.mark.parametrize("width", [70, 256, 1100, 5000])
 def test_layer_norm_seam(width):
     """The seam kernel's three parts alone and together, one and two branches, fp32 and bf16 operands, a row list."""
