@@ -24,6 +24,10 @@
 // then, group 1 one). The loads of stage t + NS - 1 go to the slot of stage t - 1, whose last reader (group 1, second
 // half, phase 2t - 1) has waited for its LDS reads before the barrier that ends that phase.
 //
+// A second tile has 192 rows (a wave 96 x 64): it moves a sixth more bytes per multiply and reaches about 0.86 of the rate
+// of the 256-row tile (a full chip's stage 0.69 us for 0.75 of the multiplies of one of 0.81 us), but 900 rows of the 8B
+// shape's gate/up are 480 tiles in two rounds of 256 compute units instead of 384 in two: 196 -> 177 us.
+//
 // Epilogues as in the other tiled kernel (gemm_epilogue.h). Needs K % 32 == 0 and at least NS - 1 stages, 16-byte
 // aligned rows; any M and N (rows beyond the end are read as the last row and never stored).
 #include "common.h"
@@ -50,9 +54,11 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
   constexpr int WGM = 2, WGN = 4, RM = 2 * FM, CN = 4;  // a wave's blocks of 16 rows and of 16 columns
   constexpr int TBM = WGM * RM * 16, TBN = WGN * CN * 16;
   constexpr int STAGE = (TBM + TBN) * PP_ROW_BYTES;
-  constexpr int LA = TBM / 16 / PP_WAVES, LB = TBN / 16 / PP_WAVES;  // load instructions per wave and stage
-  constexpr int LPW = LA + LB;
-  static_assert(LA >= 1 && LB >= 1, "every wave loads rows of both operands");
+  // load instructions (16 rows each) per wave and stage. Tiles of 192 rows are twelve chunks of A: two for each wave of the
+  // first group, one for each of the second's.
+  constexpr int LA = (TBM / 16 + PP_WAVES - 1) / PP_WAVES, LB = TBN / 16 / PP_WAVES, LA1 = TBM / 16 * 2 / PP_WAVES - LA;
+  constexpr int L0 = LA + LB, L1 = LA1 + LB;
+  static_assert(LA1 >= 1 && LB >= 1 && (LA + LA1) * PP_WAVES / 2 == TBM / 16, "every wave loads rows of both operands");
   extern __shared__ __align__(1024) unsigned char smem[];
   const int tid = threadIdx.x;
   // the wave's number is the same in all its lanes: said so, its group, its part of the tile and the places in LDS it
@@ -71,16 +77,17 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
   // scalar base (the operand's start plus the stage's place in K, advanced by scalar arithmetic) plus a 32-bit byte
   // offset per lane that never changes (row and piece), so a stage's loads cost no vector instruction.
   const int lrow = lane >> 2, lslot = lane & 3;
-  uint32_t goff[LPW];              // this lane's byte offset from the operand's start (rows x row length < 4 GB: checked on the host)
-  const unsigned char* gbase[LPW];  // the operand's start at this workgroup's first K step (the same in all lanes)
-  uint32_t ldst[LPW];              // LDS byte address of the chunk inside stage 0 (the same in all lanes)
+  uint32_t goff[L0];               // this lane's byte offset from the operand's start (rows x row length < 4 GB: checked on the host)
+  const unsigned char* gbase[L0];  // the operand's start at this workgroup's first K step (the same in all lanes)
+  uint32_t ldst[L0];               // LDS byte address of the chunk inside stage 0 (the same in all lanes)
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
 #pragma unroll
   for (int c = 0; c < LA; ++c) {
-    const int r = (wave * LA + c) * 16 + lrow;
+    const int chunk = LA == LA1 || group == 0 ? wave * LA + c : PP_WAVES / 2 * LA + (wave - PP_WAVES / 2) * LA1;  // (the second group's c = LA1 .. is never asked for)
+    const int r = chunk * 16 + lrow;
     goff[c] = (uint32_t)min(m0 + r, M - 1) * (uint32_t)lda * 2u + (uint32_t)((lslot ^ pp_swz(r)) * 16);
     gbase[c] = (const unsigned char*)A + (size_t)kt0 * PP_ROW_BYTES;
-    ldst[c] = lds0 + (wave * LA + c) * 16 * PP_ROW_BYTES;
+    ldst[c] = lds0 + chunk * 16 * PP_ROW_BYTES;
   }
 #pragma unroll
   for (int c = 0; c < LB; ++c) {
@@ -102,7 +109,8 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
     const uint32_t slot = (uint32_t)(t % NS) * STAGE;
     const size_t kbytes = (size_t)t * PP_ROW_BYTES;
 #pragma unroll
-    for (int c = 0; c < LPW; ++c) {
+    for (int c = 0; c < L0; ++c) {
+      if (c >= LA1 && c < LA && group != 0) continue;
       // the instruction itself: m0 holds the LDS address of the wave's 1 KB, lane l's 16 bytes land at m0 + 16 l
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                    :
@@ -126,10 +134,12 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s)
     if (s < nk) issue(s);
-  if (nk >= NS - 1) {
-    PP_VMCNT((NS - 3) * LPW);
-  } else {
+  if (nk < NS - 1) {
     PP_VMCNT(0);
+  } else if (group == 0) {
+    PP_VMCNT((NS - 3) * L0);
+  } else {
+    PP_VMCNT((NS - 3) * L1);
   }
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_barrier();
@@ -161,7 +171,7 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
     // group 0 is here (it has issued up to stage t + 3), group 1 at the end of its multiplies of stage t - 1
     if (group == 0) {
       if (more) {
-        PP_VMCNT(2 * LPW);
+        PP_VMCNT(2 * L0);
       } else {
         PP_VMCNT(0);
       }
@@ -189,7 +199,7 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
     __builtin_amdgcn_sched_group_barrier(0x008, RM * CN - PP_MUL * (RH + CN), 0);
     if (group == 1) {  // has issued up to stage t + 3; stage t + 2 must have landed (group 0 reads it after the next barrier but one)
       if (more) {
-        PP_VMCNT(1 * LPW);
+        PP_VMCNT(1 * L1);
       } else {
         PP_VMCNT(0);
       }
@@ -223,7 +233,7 @@ template <int FM, int NS>
 static int launch_pingpong(const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype,
                            void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue, GateSpec gs, int splits,
                            float* partial, hipStream_t stream) {
-  constexpr int TBM = 2 * FM * 32, TBN = 256;
+  constexpr int TBM = 4 * FM * 16, TBN = 256;
   const int cols = W2 ? TBN / 2 : TBN;
   dim3 grid((N + cols - 1) / cols, (M + TBM - 1) / TBM, splits);
   if (grid.y > 65535) return 1;
@@ -244,7 +254,7 @@ static int launch_pingpong(const void* A, int lda, const void* W, const void* W2
   return 0;
 }
 
-// `tile_rows`: 256 (rows of the output tile; 256 columns, 128 outputs with the gated epilogue).
+// `tile_rows`: 256 or 192 (rows of the output tile; 256 columns, 128 outputs with the gated epilogue).
 // `splits` > 1 cuts K over gridDim.z (not with the gated epilogue): `partial` then holds splits * M * N floats, summed
 // in ascending order of the split by the other tiled kernel's reduction. Returns 0 when it ran, 1 when the shape is not one it takes, -1 on errors.
 extern "C" int jllm_gemm_pingpong_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias,
@@ -265,8 +275,10 @@ extern "C" int jllm_gemm_pingpong_bf16(const void* A, int lda, const void* W, co
   int rc;
   if (tile_rows == 256)
     rc = launch_pingpong<4, 4>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, splits, partial, stream);
+  else if (tile_rows == 192)
+    rc = launch_pingpong<3, 4>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, splits, partial, stream);
   else
-    JLLM_FAIL("gemm_pingpong: tile of %d rows (256 is built)", tile_rows);
+    JLLM_FAIL("gemm_pingpong: tile of %d rows (256 and 192 are built)", tile_rows);
   if (rc != 0) return rc;
   JLLM_CHECK_LAUNCH("gemm_pingpong");
   if (splits > 1) return jllm_splitk_reduce(partial, splits, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, stream);

@@ -597,6 +597,72 @@ def _pingpong_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int]:
     return plan
 
 
+# Estimated times of the tiled products for the choice of `_tiled_plan`, in microseconds. A step's time grows with the compute
+# units at work (they share the memory and the chip's power): "lone" for a few, "full" for all.
+SMALL_DEEP_STEP_US = (0.665, 0.092)   # 64 of K on 128 x 128 tiles, a workgroup per compute unit at most: lone, + for all
+SMALL_STEP_US = (0.629, 1.125)        # the same, two workgroups to a compute unit: a round of few, a full one
+SMALL_ROUND_US = 1.2                  # what a round of workgroups costs beside its steps
+LARGE_STEP_US = {256: (0.576, 0.808), 192: (0.45, 0.687)}  # 32 of K on tiles of 256 or 192 rows by 256 columns: lone, full
+LARGE_ROUND_US = 2.33
+CUT_US = (2.2, 1.255e-6)              # a cut of K: the reduction's launch, and per element of a partial result
+
+
+def _small_us(M: int, N: int, K: int, gated: bool, splits: int) -> float:
+    """The small tile (128 x 128; 128 x 64 outputs of the gated product): one workgroup per compute unit with two K steps
+    requested ahead, or rounds of two per compute unit."""
+    cus = compute_units()
+    groups = -(-N // (64 if gated else 128)) * -(-M // 128) * splits
+    steps = K / 64 / splits
+    if groups <= cus:
+        t = steps * (SMALL_DEEP_STEP_US[0] + SMALL_DEEP_STEP_US[1] * groups / cus)
+    else:
+        lone, full = SMALL_STEP_US
+        rounds, last = divmod(groups, 2 * cus)
+        t = rounds * (steps * full + SMALL_ROUND_US)
+        if last:
+            t += steps * (lone + (full - lone) * last / (2 * cus)) + SMALL_ROUND_US
+    return t + (CUT_US[0] + CUT_US[1] * M * N * splits if splits > 1 else 0.0)
+
+
+def _large_us(M: int, N: int, K: int, gated: bool, rows: int, cut: int) -> float:
+    """The two-group kernel: rounds of one workgroup per compute unit."""
+    cus = compute_units()
+    lone, full = LARGE_STEP_US[rows]
+    steps = K / 32 / cut
+    rounds, last = divmod(-(-N // (128 if gated else 256)) * -(-M // rows) * cut, cus)
+    t = rounds * (steps * full + LARGE_ROUND_US)
+    if last:
+        t += steps * (lone + (full - lone) * last / cus) + LARGE_ROUND_US
+    return t + (CUT_US[0] + CUT_US[1] * M * N * cut if cut > 1 else 0.0)
+
+
+@functools.lru_cache(maxsize=8192)
+def _tiled_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int]:
+    """(rows of the two-group kernel's tile or 0 for the small tile, ways K is cut): what `_pingpong_plan` and `_k_splits`
+    choose between 256 rows and the small tile, or tiles of 192 rows where these are estimated to be faster. A tile of
+    192 rows moves a sixth more bytes per multiply, but its rounds and its empty rows fall differently.
+
+    The constants were fitted to the times, inside a graph, of every choice for 252 products (ten row counts from 100 to
+    4,614 on the products of six shapes). Inside whole prompt passes, which run hotter: 900 rows of the 8B shape 17.3 -> 16.5
+    ms, 3,000 of the 4B shape 27.6 -> 27.0, prompts of 7,777 rows of the 14B shape 129.7 -> 127.6, 1,100 of the 1.7B shape
+    6.51 -> 6.48. Not taken: cuts of K where 192 leaves no fewer empty rows than 256 (631 rows of the 8B shape: the o and
+    down products 6 % faster alone, the pass 1 % slower: what binds there is the chip's power), and the small tile's count
+    of cuts by the same estimate (up to a third faster alone, nothing or 1 % slower inside a pass)."""
+    rows, cut = _pingpong_plan(M, N, K, gated)
+    if K % 64 == 0:
+        cut = cut if rows else _k_splits(M, N, K, gated)
+        least = _large_us(M, N, K, gated, rows, cut) if rows else _small_us(M, N, K, gated, cut)
+        if K >= 128 and (gated or M >= PINGPONG_MIN_ROWS):
+            fewer = -(-M // 192) * 192 < -(-M // 256) * 256
+            for c in (1, 2, 4):
+                if c > 1 and (gated or not fewer or (K // 32) % c or K // c < PINGPONG_SPLIT_MIN_K):
+                    continue
+                t = _large_us(M, N, K, gated, 192, c)
+                if t < least:
+                    least, rows, cut = t, 192, c
+    return rows, cut
+
+
 STREAM_MAX_ROWS = 64   # up to here the second weight-streaming kernel (activations through LDS)
 
 
@@ -708,8 +774,8 @@ def _few_rows_prefer_stream(N: int, K: int, gated: bool) -> bool:
 
 def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0) -> bool:
     """The bf16 matrix-core kernels: a weight-streaming one for up to 16 rows, another for up to 64; for many rows
-    the two-group kernel with 256 x 256 tiles where enough of them fill the GPU (`_pingpong_plan`), else the other
-    tiled kernel (with K cut over several workgroups when the output has few tiles). Each declines shapes it does
+    the two-group kernel with tiles of 256 or 192 rows by 256 columns or the small tile, either with K cut over several
+    workgroups when the output has few tiles (`_tiled_plan`). Each declines shapes it does
     not take; then the fp32 kernel runs."""
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         return False
@@ -726,7 +792,7 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0) -> bool:
             if parts > 1 else None
         if _try("jllm_gemm_stream_bf16", *head, parts, _ptr(partial), _stream()):
             return True
-    tile_rows, cut = _pingpong_plan(M, N, K, w2 is not None)
+    tile_rows, cut = _tiled_plan(M, N, K, w2 is not None)
     if tile_rows:
         partial = torch.empty((cut * M * N,), dtype=torch.float32, device=a.device) if cut > 1 else None
         if _try("jllm_gemm_pingpong_bf16", *head, tile_rows, cut, _ptr(partial), _stream()):

@@ -166,6 +166,31 @@ def test_gemm_two_group_kernel(ops, M, N, K, plan):
     assert ops.stats()["ran"].get("jllm_gemm_pingpong_bf16") >= 3 and not ops.stats()["general"], ops.stats()
 
 
+@pytest.mark.parametrize("M,N,K,cut", [(193, 520, 160, 1), (600, 2500, 128, 1), (575, 1300, 2048, 2), (577, 700, 4224, 4)])
+def test_gemm_two_group_kernel_with_tiles_of_192_rows(ops, monkeypatch, M, N, K, cut):
+    """The 192-row tile (waves of one group load four chunks of a stage, the other's three) against the 256-row tile, bit
+    for bit: one row beyond a tile and one short of it, K from four stages on and cut in two and four, every epilogue."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M + K)
+    a = torch.randn(M, K, device=DEV, generator=gen).bfloat16()
+    w, w2 = ((torch.randn(N, K, device=DEV, generator=gen) * K ** -0.5).bfloat16() for _ in range(2))
+    bias = torch.randn(N, device=DEV, generator=gen)
+
+    def outputs(rows):
+        monkeypatch.setattr(ops, "_tiled_plan", lambda m, n, k, gated: (rows, 1 if gated else cut))
+        ops.reset_stats()
+        res = torch.ones(M, N, device=DEV)
+        ops.gemm(a, w, bias=bias, out=res, epilogue=ops.EPI_ADD)
+        got = [res, ops.gemm(a, w, out_dtype=torch.float32), ops.gemm(a, w, bias=bias), ops.gemm(a, w, w2=w2, epilogue=ops.EPI_GATED)]
+        assert ops.stats()["ran"] == {"jllm_gemm_pingpong_bf16": 4}
+        return got
+
+    tall, got = outputs(256), outputs(192)
+    assert all(torch.equal(x, y) for x, y in zip(got, tall))
+    ref = a.double() @ w.double().T  # fp32 sums of K rounded products: K 2^-24 of the sum of magnitudes at most
+    assert bool(((got[1].double() - ref).abs() <= K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
+
+
 @pytest.mark.parametrize("M,N,K,N2", [(1, 128, 256, 48), (5, 4096, 384, 4112), (8, 640, 4096, 304), (16, 304, 128, 16), (13, 5120, 1024, 640),
                                       (40, 1024, 1024, 512), (64, 2048, 2048, 768), (17, 1024, 4096, 256),
                                       # few rows, N / 16 just above the compute units: 20 weight rows per workgroup
