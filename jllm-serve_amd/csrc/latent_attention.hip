@@ -1,25 +1,22 @@
-// Latent attention on the matrix cores, bf16: portions of prompts and single decoded rows through one kernel.
+// Latent attention on the matrix cores, bf16: one kernel for single decoded rows, one for portions of prompts.
 //
 // All heads of a row attend over the same cached rows (Dk = R + Dr numbers per position, the first R of which are also
-// the values), so the query vectors of many heads and rows share every key they read. A workgroup takes 64 query
-// vectors of one run of rows of one request (HB heads x 64 / HB consecutive rows). It has eight waves: waves w and w + 4
-// own the same 16 query vectors and both compute their scores and softmax, but each keeps only one half of the latent's
-// accumulators (a 512-wide latent is 128 registers per lane; one wave holding all of it and its queries left no
-// registers to have LDS reads in flight, and timestamps showed every fragment read's latency standing in front of its
-// product: 2,900 cycles for the 18 score products of 16 keys). The workgroup
-// walks the keys its rows can see in blocks of 64 aligned to absolute positions, and stages each block once in LDS as
+// the values), so the query vectors of many heads (and rows) share every key they read. A workgroup takes up to 64 query
+// vectors. It walks the keys they can see in blocks of 64 aligned to absolute positions, and stages each block once in LDS as
 // it lies in the cache (two buffers take turns: the next block travels while this one is multiplied). Per 16 keys a wave computes
 //   S^T = K . Q^T   (MFMA 16x16x32; K fragments from LDS, Q^T in registers): a lane then holds four keys' scores of
 //                   ONE query vector, so masks (causal and window, per query vector), maximum and sum need only two
 //                   shuffles over the lane groups;
-//   O^T += V^T . P^T (MFMA 16x16x16): those probabilities, packed to bf16, already are the B operand, and V^T is read
-//                   from the staged block with the transposing LDS load.
+//   O^T += V^T . P^T: those probabilities, packed to bf16, are the B operand, and V^T is read from the staged block
+//                   with the transposing LDS load.
 // The running maximum moves only when it grows by more than 8 (probabilities stay below e^8, exact in fp32 sums).
 // exp(sink) of the query vector's head joins the denominator at the end. Scores, softmax and sums are fp32.
 //
 // The runs come from the step's plan: (request, first row, rows <= 16, -) per tile; positions are read per row.
 //
-// Steps of single rows (decoding) with few workgroups cut every row's keys into absolute ranges of `split` keys over
+// Single rows: eight waves, of which w and w + 4 own the same 16 query vectors (heads) and both compute their scores and
+// softmax, but each keeps only one half of the latent's accumulators (a 512-wide latent is 128 registers per lane).
+// Steps with few workgroups cut every row's keys into absolute ranges of `split` keys over
 // gridDim.z: a workgroup then leaves maximum, sum and unnormalised sums per query vector, and a second kernel merges
 // the ranges in ascending order, adds the sink and normalises.
 #include <math.h>
@@ -31,6 +28,8 @@
 #define LM_QW 4  // waves with query vectors of their own; waves 4..7 repeat them for the other half of the latent
 #define LM_KEYS 64
 #define LM_TILE_ROWS 16
+#define LM_AHEAD 3
+#define LM_PS (LM_KEYS + 8)  // elements between two query vectors' probabilities
 
 __device__ __forceinline__ float lm_exp_diff(float a, float b) { return a == -INFINITY ? 0.f : __expf(a - b); }
 
@@ -40,21 +39,15 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
     const bf16_t* __restrict__ qa, int ldq, bf16_t* __restrict__ out, int ldo, const bf16_t* __restrict__ cache,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ tiles,
     const int* __restrict__ positions, int H, int R, int Dk, int page_size, int window, float scale,
-    const float* __restrict__ sink, int HB, int n_hb, int LD, int split, float* __restrict__ part) {
+    const float* __restrict__ sink, int HB, int LD, int split, float* __restrict__ part) {
   extern __shared__ __align__(16) unsigned char lm_smem[];
   bf16_t* Ks = (bf16_t*)lm_smem;  // [2][LM_KEYS][LD]
   const int tile = blockIdx.x;
-  const int req = tiles[4 * tile], row0 = tiles[4 * tile + 1], rows = tiles[4 * tile + 2];
-  const int RW = 64 / HB;
-  const int rg = blockIdx.y / n_hb, hb = blockIdx.y % n_hb;
-  const int r_lo = rg * RW;
-  if (r_lo >= rows) return;
-  const int r_hi = min(rows, r_lo + RW) - 1;
-  const int p_lo = positions[row0 + r_lo];
-  const int p_hi = p_lo + (r_hi - r_lo);
-  int kb = window > 0 ? max(0, p_lo + 1 - window) : 0;
-  int ke = p_hi;
-  if (split > 0) {  // single rows: this workgroup's range of the row's keys
+  const int req = tiles[4 * tile], row = tiles[4 * tile + 1];
+  const int hb = blockIdx.y;
+  int ke = positions[row];
+  int kb = window > 0 ? max(0, ke + 1 - window) : 0;
+  if (split > 0) {  // this workgroup's range of the row's keys
     const int s0 = kb / split + (int)blockIdx.z;
     kb = max(kb, s0 * split);
     ke = min(ke, s0 * split + split - 1);
@@ -62,20 +55,14 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
   }
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = lane & 15, q4 = lane >> 4;
-  // A single row of at most 16 heads is 16 query vectors, one wave's worth: then all four waves take the same query
-  // vectors and every fourth group of 16 keys each, and merge at the end in the order of the waves.
-  const bool kpar = r_hi == r_lo && HB <= 16;
+  // At most 16 heads are 16 query vectors, one wave's worth: then all four waves take the same query vectors and
+  // every fourth group of 16 keys each, and merge at the end in the order of the waves.
+  const bool kpar = HB <= 16;
   const int qwave = wave & (LM_QW - 1), rhalf = wave / LM_QW;
   const int v = kpar ? sub : qwave * 16 + sub;
-  const int my_r = r_lo + v / HB, my_h = hb * HB + v % HB;
-  const bool live = my_r <= r_hi && my_h < H;
-  const int my_pos = p_lo + v / HB;
-  const int my_first = window > 0 ? max(0, my_pos + 1 - window) : 0;
-  // the keys this wave's rows can see (a wave without a live query vector only helps to load)
-  const int wr_lo = kpar ? r_lo : r_lo + (qwave * 16) / HB, wr_hi = kpar ? r_lo : min(r_hi, r_lo + (qwave * 16 + 15) / HB);
-  const bool wave_live = wr_lo <= r_hi;
-  const int w_lo = window > 0 ? max(0, p_lo + (wr_lo - r_lo) + 1 - window) : 0;
-  const int w_hi = p_lo + (wr_hi - r_lo);  // (with a split the loop's own bounds narrow these further)
+  const int my_h = hb * HB + v;
+  const bool live = v < HB && my_h < H;
+  const bool wave_live = kpar || qwave * 16 < HB;  // (a wave without a live query vector only helps to load)
   const int dks = (Dk + 31) >> 5, r16 = R >> 4;
   constexpr int RTH = (RT + 1) / 2;  // accumulators of one wave: its half of the latent's 16-dim blocks
   const int j_lo = rhalf ? (r16 + 1) / 2 : 0, nj = rhalf ? r16 - (r16 + 1) / 2 : (r16 + 1) / 2;
@@ -84,7 +71,7 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
 
   u32x4 qf[DKS];
   {
-    const bf16_t* qrow = qa + (size_t)(row0 + min(my_r, r_hi)) * ldq + (size_t)min(my_h, H - 1) * Dk;
+    const bf16_t* qrow = qa + (size_t)row * ldq + (size_t)min(my_h, H - 1) * Dk;
 #pragma unroll
     for (int j = 0; j < DKS; ++j) {
       const int d = 32 * j + 8 * q4;
@@ -129,7 +116,7 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
 #pragma unroll 1
       for (int st = 0; st < LM_KEYS / 16; ++st) {
         const int k0 = c0 + st * 16;
-        if (k0 + 15 < w_lo || k0 > w_hi) continue;  // none of these keys is seen by a row of this wave
+        if (k0 + 15 < kb || k0 > ke) continue;  // none of these keys is this workgroup's
         if (kpar && st != qwave) continue;           // another wave's keys
         floatx4 sc = floatx4{0.f, 0.f, 0.f, 0.f}, sc2 = floatx4{0.f, 0.f, 0.f, 0.f};  // two chains of dependent MFMAs
         const bf16_t* krow = Kb + (st * 16 + sub) * LD + 8 * q4;
@@ -144,7 +131,7 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int key = k0 + 4 * q4 + i;
-          z[i] = (live && key >= my_first && key <= my_pos && key >= kb && key <= ke) ? sc[i] * scale : -INFINITY;
+          z[i] = (live && key >= kb && key <= ke) ? sc[i] * scale : -INFINITY;
           mx = fmaxf(mx, z[i]);
         }
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -208,7 +195,7 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
   }
   if (!live) return;
   if (split > 0) {
-    float* dst = part + (((size_t)(row0 + my_r) * H + my_h) * gridDim.z + blockIdx.z) * (R + 4);  // R sums, maximum, sum
+    float* dst = part + (((size_t)row * H + my_h) * gridDim.z + blockIdx.z) * (R + 4);  // R sums, maximum, sum
     if (q4 == 0 && rhalf == 0) dst[R] = m1, dst[R + 1] = l1;
 #pragma unroll
     for (int j = 0; j < RTH; ++j)
@@ -223,11 +210,209 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
     l1 = l1 * ca + __expf(sk - mn);
   }
   const float inv = ca / l1;
-  bf16_t* o = out + (size_t)(row0 + my_r) * ldo + (size_t)my_h * R + 4 * q4;
+  bf16_t* o = out + (size_t)row * ldo + (size_t)my_h * R + 4 * q4;
 #pragma unroll
   for (int j = 0; j < RTH; ++j)
     if (j < nj)
       *(u32x2*)(o + 16 * (j_lo + j)) = u32x2{pack_bf16(acc[j][0] * inv, acc[j][1] * inv), pack_bf16(acc[j][2] * inv, acc[j][3] * inv)};
+}
+
+// Runs of several rows (portions of prompts). A workgroup takes 64 query vectors of one run (HB heads x 64 / HB rows) and
+// walks the keys they can see in blocks of 64 as the kernel above, but no product is computed twice: wave w computes the
+// scores of 16 query vectors (w % 4) with 32 of a block's keys (w / 4), its queries in registers; the waves agree on the
+// block's maxima over LDS, leave their probabilities there as bf16, and wave w then sums all 64 query vectors' values over
+// an eighth of the latent. A V^T fragment so serves four products and only the scores' K fragments one. What bounds
+// it are those: 288 KB of LDS reads a block of 64 keys of 576 entries. Two barriers a block: the scores of a block
+// follow the sums of the one before without one. Nothing in the loops is conditional on sizes (a conditional step waits for
+// its own LDS reads): rows are staged with zeros up to DKS steps of 32. 16 heads, 512 + 64 entries, against the kernel above
+// for single rows, which took these runs too and computed every score twice: prompts of 300 to 1,211 rows (3,611 in all)
+// 325 -> 133 us, 4,096 rows 1,204 -> 472, 487 rows 74 -> 33, six of 20 rows and ten single rows of 1,500 to 1,950 keys
+// 108 -> 80. A key's probability lies where the value product's lane wants it (keys
+// 4 g .. and 16 + 4 g .. of 32 together, the order in which two transposing loads deliver V^T).
+template <int NJ, int DKS>  // NJ: 16-dim blocks of the latent per wave at most (8 NJ >= R / 16); DKS as above
+__global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_rows_kernel(
+    const bf16_t* __restrict__ qa, int ldq, bf16_t* __restrict__ out, int ldo, const bf16_t* __restrict__ cache,
+    const int* __restrict__ block_table, int max_blocks, const int* __restrict__ tiles, const int* __restrict__ positions,
+    int H, int R, int Dk, int page_size, int window, float scale, const float* __restrict__ sink, int HB, int n_hb) {
+  constexpr int LD = DKS * 32 + 16;          // elements between two keys' rows in LDS (16 mod 64: see the launch)
+  extern __shared__ __align__(16) unsigned char lm_smem[];
+  bf16_t* Ks = (bf16_t*)lm_smem;             // [2][LM_KEYS][LD]
+  bf16_t* Ps = Ks + (size_t)2 * LM_KEYS * LD;  // [64 query vectors][LM_PS]: a block's probabilities
+  float* mxs = (float*)(Ps + 64 * LM_PS);    // [2][64]: the block's maximum over either half of its keys; at the end the sums
+  float* als = mxs + 128;                    // [64]: the factor of what was summed before; at the end of everything
+  const int tile = blockIdx.x;
+  const int req = tiles[4 * tile], row0 = tiles[4 * tile + 1], rows = tiles[4 * tile + 2];
+  const int RW = 64 / HB;
+  const int hb = blockIdx.y % n_hb, r_lo = blockIdx.y / n_hb * RW;
+  if (r_lo >= rows) return;
+  const int r_hi = min(rows, r_lo + RW) - 1;
+  const int p_lo = positions[row0 + r_lo];
+  const int kb = window > 0 ? max(0, p_lo + 1 - window) : 0, ke = p_lo + (r_hi - r_lo);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sub = lane & 15, q4 = lane >> 4;
+  const int qs = wave & 3, kh = wave >> 2;
+  const int v = qs * 16 + sub;  // this lane's query vector of the scores
+  const int my_r = r_lo + v / HB, my_h = hb * HB + v % HB;
+  const bool live = my_r <= r_hi && my_h < H;
+  const int my_pos = p_lo + v / HB;
+  const int my_first = window > 0 ? max(0, my_pos + 1 - window) : 0;
+  const int n_q = min(4, ((r_hi - r_lo + 1) * HB + 15) >> 4);  // groups of 16 query vectors with a row
+  const int j_lo = wave * NJ, nj = min(NJ, (R >> 4) - j_lo);
+  const int psh = __builtin_ctz(page_size);
+  const int* tbl = block_table + (size_t)req * max_blocks;
+
+  u32x4 qf[DKS];
+  {
+    const bf16_t* qrow = qa + (size_t)(row0 + min(my_r, r_hi)) * ldq + (size_t)min(my_h, H - 1) * Dk;
+#pragma unroll
+    for (int j = 0; j < DKS; ++j) {
+      const int d = 32 * j + 8 * q4;
+      qf[j] = (live && d < Dk) ? *(const u32x4*)(qrow + d) : u32x4{0u, 0u, 0u, 0u};
+    }
+  }
+  floatx4 acc[4][NJ];
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[q][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  float m1 = -INFINITY, l1 = 0.f;
+  // keys travel as above (eight threads to a key row, the next block's in registers while this one is multiplied); a
+  // block's page is looked up a block before its rows are requested
+  constexpr int CPT = (DKS + 1) / 2;
+  uint4 staged[CPT];
+  const int srow = threadIdx.x >> 3, scol = (threadIdx.x & 7) * 8;
+  const int blk_last = ke >> 6;
+  int blk = kb >> 6;
+  auto key_of = [&](int b) { return min(max(b * LM_KEYS + srow, kb), ke); };  // (a key outside the range is masked and reads one inside it)
+  int page = tbl[key_of(blk) >> psh];
+  auto fetch = [&](int b) {
+    const bf16_t* src = cache + ((((size_t)page) << psh) + (key_of(b) & (page_size - 1))) * Dk;
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) staged[i] = *(const uint4*)(src + (scol + 64 * i < Dk ? scol + 64 * i : 0));
+    page = tbl[key_of(b + 1) >> psh];
+  };
+  auto put = [&](bf16_t* buf) {
+    bf16_t* dst = buf + srow * LD + scol;
+#pragma unroll
+    for (int i = 0; i < CPT; ++i)
+      *(uint4*)(dst + 64 * i) = scol + 64 * i < Dk ? staged[i] : uint4{0u, 0u, 0u, 0u};
+  };
+  fetch(blk);
+  put(Ks);
+  __syncthreads();
+  for (int cur = 0; blk <= blk_last; ++blk, cur ^= 1) {
+    const bf16_t* Kb = Ks + (size_t)cur * LM_KEYS * LD;
+    if (blk < blk_last) fetch(blk + 1);
+    float z[8];
+    if (qs < n_q) {
+      floatx4 sc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+      const bf16_t* krow = Kb + (kh * 32 + sub) * LD + 8 * q4;
+      u32x4 kf[LM_AHEAD + 1][2];
+#pragma unroll
+      for (int j = 0; j < DKS + LM_AHEAD; ++j) {  // fragments LM_AHEAD steps ahead of the multiplies, no more: registers
+        u32x4* slot = kf[j % (LM_AHEAD + 1)];
+        if (j < DKS) slot[0] = *(const u32x4*)(krow + 32 * j), slot[1] = *(const u32x4*)(krow + 16 * LD + 32 * j);
+        if (j >= LM_AHEAD) {
+          const int m = j - LM_AHEAD;
+          sc[0] = mfma16(kf[m % (LM_AHEAD + 1)][0], qf[m], sc[0]);
+          sc[1] = mfma16(kf[m % (LM_AHEAD + 1)][1], qf[m], sc[1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int key = blk * LM_KEYS + kh * 32 + (i >> 2) * 16 + 4 * q4 + (i & 3);
+        z[i] = (live && key >= my_first && key <= my_pos) ? sc[i >> 2][i & 3] * scale : -INFINITY;
+        mx = fmaxf(mx, z[i]);
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      if (q4 == 0) mxs[kh * 64 + v] = mx;
+    }
+    __syncthreads();  // the maxima are there, and everyone is done with the last block's probabilities and keys
+    if (blk < blk_last) put(Ks + (size_t)(cur ^ 1) * LM_KEYS * LD);
+    if (qs < n_q) {
+      const float mx = fmaxf(mxs[v], mxs[64 + v]);
+      float alpha = 1.0f;
+      if (mx > m1 + 8.0f) {  // also the first visible key (m1 = -inf)
+        alpha = lm_exp_diff(m1, mx);
+        l1 *= alpha;
+        m1 = mx;
+      }
+      if (kh == 0 && q4 == 0) als[v] = alpha;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        z[i] = lm_exp_diff(z[i], m1);
+        l1 += z[i];
+      }
+      *(u32x4*)(Ps + v * LM_PS + kh * 32 + 8 * q4) =
+          u32x4{pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3]), pack_bf16(z[4], z[5]), pack_bf16(z[6], z[7])};
+    }
+    __syncthreads();  // the probabilities and the next block's keys are there
+    float al[4];
+    bool moved = false;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {  // (groups without a row carry what nobody stores)
+      al[q] = als[q * 16 + sub];
+      moved = moved || al[q] != 1.0f;
+    }
+    if (__any(moved)) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[q][j] *= al[q];
+    }
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const bf16_t* v_tr = Kb + (half * 32 + 4 * q4 + (sub >> 2)) * LD + 4 * (sub & 3) + 16 * j_lo;
+      const bf16_t* prow = Ps + sub * LM_PS + half * 32 + 8 * q4;
+      u32x4 vf[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const u32x2 a = lds_read_tr16(v_tr + 16 * j), b = lds_read_tr16(v_tr + 16 * LD + 16 * j);
+        vf[j] = u32x4{a[0], a[1], b[0], b[1]};
+      }
+      const u32x4 p0 = *(const u32x4*)prow;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[0][j] = mfma16(vf[j], p0, acc[0][j]);
+      if (n_q > 1) {
+#pragma unroll
+        for (int q = 1; q < 4; ++q) {
+          const u32x4 pf = *(const u32x4*)(prow + q * 16 * LM_PS);
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) acc[q][j] = mfma16(vf[j], pf, acc[q][j]);
+        }
+      }
+    }
+  }
+  l1 += __shfl_xor(l1, 16, 64);
+  l1 += __shfl_xor(l1, 32, 64);
+  if (q4 == 0 && kh == 1) mxs[v] = l1;
+  __syncthreads();  // (also: everyone has read the last block's factors)
+  if (q4 == 0 && kh == 0 && live) {
+    l1 += mxs[v];
+    float ca = 1.0f;
+    if (sink) {
+      const float sk = sink[my_h];
+      const float mn = fmaxf(m1, sk);
+      ca = lm_exp_diff(m1, mn);
+      l1 = l1 * ca + __expf(sk - mn);
+    }
+    als[v] = ca / l1;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int u = q * 16 + sub, row = r_lo + u / HB, h = hb * HB + u % HB;
+    if (row > r_hi || h >= H) continue;
+    const float inv = als[u];
+    bf16_t* o = out + (size_t)(row0 + row) * ldo + (size_t)h * R + 16 * j_lo + 4 * q4;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      if (j < nj)
+        *(u32x2*)(o + 16 * j) = u32x2{pack_bf16(acc[q][j][0] * inv, acc[q][j][1] * inv), pack_bf16(acc[q][j][2] * inv, acc[q][j][3] * inv)};
+  }
 }
 
 // merges the key ranges of one (row, head); four waves per (row, head), a thread owns dims tid and tid + 256. Lane z of
@@ -273,7 +458,7 @@ __global__ __launch_bounds__(256) void latent_attention_merge_kernel(const float
 template <int RT, int DKS>
 static int lm_launch(dim3 grid, size_t smem, hipStream_t stream, const void* qa, int ldq, void* out, int ldo, const void* cache,
                      const int* block_table, int max_blocks, const int* tiles, const int* positions, int H, int R, int Dk,
-                     int page_size, int window, float scale, const float* sink, int HB, int n_hb, int LD, int split, float* part) {
+                     int page_size, int window, float scale, const float* sink, int HB, int LD, int split, float* part) {
   static size_t reserved = 0;
   if (smem > 48 * 1024 && smem > reserved) {
     if (hipFuncSetAttribute((const void*)latent_attention_mfma_kernel<RT, DKS>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -283,7 +468,25 @@ static int lm_launch(dim3 grid, size_t smem, hipStream_t stream, const void* qa,
   }
   latent_attention_mfma_kernel<RT, DKS><<<grid, LM_WAVES * 64, smem, stream>>>(
       (const bf16_t*)qa, ldq, (bf16_t*)out, ldo, (const bf16_t*)cache, block_table, max_blocks, tiles, positions, H, R, Dk,
-      page_size, window, scale, sink, HB, n_hb, LD, split, part);
+      page_size, window, scale, sink, HB, LD, split, part);
+  return 0;
+}
+
+template <int NJ, int DKS>
+static int lm_launch_rows(dim3 grid, hipStream_t stream, const void* qa, int ldq, void* out, int ldo, const void* cache,
+                          const int* block_table, int max_blocks, const int* tiles, const int* positions, int H, int R, int Dk,
+                          int page_size, int window, float scale, const float* sink, int HB, int n_hb) {
+  static size_t reserved = 0;
+  const size_t smem = ((size_t)2 * LM_KEYS * (DKS * 32 + 16) + 64 * LM_PS) * sizeof(bf16_t) + 192 * sizeof(float);
+  if (smem > 48 * 1024 && smem > reserved) {
+    if (hipFuncSetAttribute((const void*)latent_attention_rows_kernel<NJ, DKS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)smem) != hipSuccess)
+      JLLM_FAIL("latent_attention: cannot reserve %zu bytes of LDS", smem);
+    reserved = smem;
+  }
+  latent_attention_rows_kernel<NJ, DKS><<<grid, LM_WAVES * 64, smem, stream>>>(
+      (const bf16_t*)qa, ldq, (bf16_t*)out, ldo, (const bf16_t*)cache, block_table, max_blocks, tiles, positions, H, R, Dk,
+      page_size, window, scale, sink, HB, n_hb);
   return 0;
 }
 
@@ -310,17 +513,22 @@ extern "C" int jllm_latent_attention_bf16(const void* qa, int ldq, void* out, in
   int LD = dkp + 16;
   while ((LD & 63) != 16) LD += 8;
   const size_t smem = (size_t)2 * LM_KEYS * LD * sizeof(bf16_t);  // two buffers that take turns
-  // `split` > 0: every tile is a single row (the caller's promise), whose keys are cut into absolute ranges of `split`
+  // `split` < 0: runs of up to tile_rows rows. Otherwise every tile is a single row (the caller's promise); > 0: whose keys are cut into absolute ranges of `split`
   // keys over n_z workgroups; `part` holds rows x H x n_z x (R + 4) floats
   if (split > 0 && ((split & 63) || n_z < 1 || n_z > 64 || !part)) JLLM_FAIL("latent_attention: ranges of %d keys over %d workgroups", split, n_z);
-  dim3 grid(n_tiles, n_hb * (split > 0 ? 1 : n_rg), split > 0 ? n_z : 1);
+  dim3 grid(n_tiles, n_hb * (split < 0 ? n_rg : 1), split > 0 ? n_z : 1);
   int rc;
-  if (R <= 64 && dkp <= 128)
-    rc = lm_launch<4, 4>(grid, smem, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, n_hb, LD, split, part);
+  if (split < 0 && dkp > 576) JLLM_FAIL("latent_attention: cannot reserve %zu bytes of LDS", smem);  // (more than 160 KB)
+  if (split < 0)
+    rc = R <= 128 && dkp <= 256
+             ? lm_launch_rows<1, 8>(grid, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, n_hb)
+             : lm_launch_rows<4, 18>(grid, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, n_hb);
+  else if (R <= 64 && dkp <= 128)
+    rc = lm_launch<4, 4>(grid, smem, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, LD, split, part);
   else if (R <= 128 && dkp <= 256)
-    rc = lm_launch<8, 8>(grid, smem, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, n_hb, LD, split, part);
+    rc = lm_launch<8, 8>(grid, smem, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, LD, split, part);
   else
-    rc = lm_launch<32, 20>(grid, smem, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, n_hb, LD, split, part);
+    rc = lm_launch<32, 20>(grid, smem, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, LD, split, part);
   if (rc != 0) return rc;
   JLLM_CHECK_LAUNCH("latent_attention");
   if (split > 0) {

@@ -1142,7 +1142,7 @@ def _fast_latent_attention(qa, out, cache, block_table, row_req, positions, head
     if qa.dtype != torch.bfloat16 or meta is None or meta.get("tiles_dev") is None:
         return False
     n_tiles = int(meta["n_tiles"])
-    split, n_z, part = 0, 1, None
+    split, n_z, part = -1, 1, None  # runs of several rows
     if meta.get("single_rows") and n_tiles == qa.shape[0]:
         split, n_z = _latent_split(n_tiles, heads, int(window), int(meta.get("max_context", 0)))
         if split:

@@ -301,6 +301,49 @@ def test_attention_kernels_on_crafted_keys(dtype, fast, H, R, Dr, page):
             assert (no_sink - want).abs().max() > 0.3
 
 
+@pytest.mark.parametrize("H, R, Dk, window", [(16, 512, 576, 0), (16, 512, 576, 130), (3, 144, 168, 70), (40, 496, 520, 0), (7, 128, 256, 64)])
+def test_latent_attention_of_runs_of_rows(H, R, Dk, window):
+    """Portions of prompts in runs of 1 to 16 rows that begin at any position (keys end one below, at and one beyond a
+    block of 64; a single row beside them), rows whose entries are no multiple of 32 or 64, latents whose last waves have no
+    part; every sum from the definition in 64 bits."""
+    from jllm_serve_amd.kernels import ops
+    g = torch.Generator().manual_seed(R + H + window)
+    page, spans = 16, [(0, 33), (58, 6), (63, 1), (64, 1), (200, 63), (257, 1)]  # (first position, rows) of each request
+    width = 24
+    n_req = len(spans)
+    cache = torch.full((n_req * width, page, Dk), float("nan"), dtype=torch.bfloat16)
+    table = torch.randperm(n_req * width, generator=g).to(torch.int32).view(n_req, width)
+    sink = torch.randn(H, generator=g)
+    rows, runs, pos, req, want, room = [], [], [], [], [], []
+    scale = 1.5 * Dk ** -0.5
+    for r, (p0, n) in enumerate(spans):
+        keys = torch.randn(p0 + n, Dk, generator=g).bfloat16()
+        for k in range(0, p0 + n, page):
+            part = keys[k:k + page]
+            cache[int(table[r, k // page]), :len(part)] = part
+        q = torch.randn(n, H, Dk, generator=g).bfloat16()
+        runs += [(r, len(pos) + i, min(16, n - i), p0 + i) for i in range(0, n, 16)]
+        rows.append(q)
+        at = torch.arange(p0, p0 + n)
+        pos += at.tolist()
+        req += [r] * n
+        z = torch.einsum("nhd,kd->nhk", q.double(), keys.double()) * scale
+        key = torch.arange(p0 + n)
+        seen = (key <= at[:, None]) & ((key > at[:, None] - window) if window else torch.ones_like(key, dtype=torch.bool))
+        z = z.masked_fill(~seen[:, None], -torch.inf)
+        p = torch.softmax(torch.cat([z, sink.double().expand(n, H)[..., None]], dim=2), dim=2)[..., :-1]
+        want.append(p @ keys[:, :R].double())
+        # a score: Dk products' fp32 sum, in any order, and its part in exp; the probabilities and the result as bf16
+        size = torch.einsum("nhd,kd->nhk", q.double().abs(), keys.double().abs()).amax(dim=2, keepdim=True) * scale
+        room.append((2.0 ** -9 + 2.0 * Dk * 2.0 ** -24 * size + 2.0 ** -18) * (p @ keys[:, :R].double().abs()) + 2.0 ** -8 * want[-1].abs())
+    meta = {"tiles_dev": torch.tensor(runs, dtype=torch.int32).flatten().to(DEV), "n_tiles": len(runs)}
+    ops.reset_stats()
+    got = ops.latent_attention(torch.cat(rows).view(-1, H * Dk).to(DEV), cache.to(DEV), table.to(DEV), torch.tensor(req, dtype=torch.int32, device=DEV),
+                               torch.tensor(pos, dtype=torch.int32, device=DEV), H, R, window, scale, sink.to(DEV), meta=meta)
+    assert ops.stats()["ran"] == {"jllm_latent_attention_bf16": 1}
+    assert bool(((got.view(-1, H, R).double().cpu() - torch.cat(want)).abs() <= torch.cat(room)).all())
+
+
 # ------------------------------------------------------------------------------------------------ replays
 
 
