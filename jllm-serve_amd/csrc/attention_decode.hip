@@ -15,7 +15,8 @@
 // The fused form does the whole attention of a decode step in one launch: it takes the projection output
 // qkv[t] = [q | k | v] as it comes from the product, normalises and rotates q in registers (every workgroup for
 // its own heads), lets the workgroup of a row's last split normalise, rotate and store the new key and copy the
-// new value into their page before the keys are read. The splits are merged by the same second kernel. (Merging
+// new value into their page before the keys are read (the matrix-core kernel for head_dim 128: keeps them in LDS as well
+// and never waits for the store). The splits are merged by the same second kernel. (Merging
 // them in the first kernel, by the workgroup that finishes last, was measured: the device-wide fences it needs
 // cost far more than the launch it saves.)
 //
@@ -466,6 +467,12 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(G
 // receives column i % 4 of rows i / 4 + 4 e: lane r names key 4 (l/16) + r / 4, dims 4 (r % 4) .. + 4, and lane i
 // receives dim i of the group's four keys). One running maximum per head serves all four key groups of a wave; it
 // moves only when a turn's maximum exceeds it by more than 2^8, so the accumulators are rarely rescaled.
+//
+// A step of few rows is one chain of latencies: position and table, then the first keys beside q, then the products. So
+// position, request and slot are asked for together, the first keys straight through the table before q is prepared
+// (instead of behind the barrier that shares table and q), the new key is another wave's work than q, and its readers
+// take it from LDS. Whole steps, before and after: 300 keys of the 0.6B shape 1,106 -> 1,101 us, 4 x 4B at long contexts
+// 3,614 -> 3,573, 64 x 8B 6,519 -> 6,404.
 template <int G, bool FUSED>
 __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, 3))) void decode_attention_mfma_kernel(
     const bf16_t* q, int ldq, const bf16_t* kc, const bf16_t* vc, const int* __restrict__ block_table, int max_blocks,
@@ -479,10 +486,14 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
   __shared__ __align__(16) unsigned char pool[VS_BYTES > MRG_BYTES ? VS_BYTES : MRG_BYTES];
   float (*mrg)[64][34] = (float (*)[64][34])pool;
   __shared__ __align__(16) bf16_t qs[G][hd];  // fused form: q after norm and rotation, to be read as the B operand
+  __shared__ __align__(16) bf16_t new_kv[2][hd];  // fused form: the new token's key and value
   const int t = blockIdx.x;
   const int kvh = blockIdx.y;
   const int s = blockIdx.z;
-  const int pos = positions[t];
+  // requested together; the compiler would otherwise ask for what follows the return only behind it
+  const int pos = positions[t], req = row_req[t];
+  const int slot = FUSED && fu.write_kv ? fu.slots[t] : -1;
+  asm volatile("" ::"s"(pos), "s"(req), "s"(slot));
   const int first = window > 0 ? max(0, pos + 1 - window) : 0;
   const int s_lo = first / split, s_hi = pos / split;
   if (s < s_lo || s > s_hi) return;
@@ -492,19 +503,71 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
   const int wave = threadIdx.x >> 6;
   const int sub = lane & 15, q4 = lane >> 4;
   const int H = Hkv * G;
-  const int* tbl = block_table + (size_t)row_req[t] * max_blocks;
+  const int* tbl = block_table + (size_t)req * max_blocks;
   const int psh = __builtin_ctz(page_size);  // pages hold a power of two of positions: shifts, not divisions
   const int b0 = kb >> psh;
   const int nb = (ke >> psh) - b0 + 1;
   for (int i = threadIdx.x; i < nb; i += DA_WAVES * 64) tb[i] = tbl[b0 + i];
+  // a turn: keys k0 .. k0 + 15 of this wave. K for the scores: key k0 + sub, dims 32 j + 8 q4; V for the sums: key
+  // k0 + 4 q4 + u, dims 8 sub. The next turn's are requested before this turn's are used.
+  struct Turn {
+    u32x4 k[4];
+    uint4 v[4];
+  };
+  const bool one_page = page_size >= 4 && (kb & 3) == 0;
+  // keys beyond the end of the range are read as the last key of the range (a valid one): no branches and nothing to
+  // clear; their scores are masked below and their probabilities are zero
+  auto fetch = [&](int k0, Turn& tn, auto page_of) {
+    const int kk = min(k0 + sub, ke);
+    {
+      const int page = page_of(kk);
+      const bf16_t* kp = kc + ((((size_t)page * Hkv + kvh) << psh) + (kk & (page_size - 1))) * hd + q4 * 8;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) tn.k[j] = *(const u32x4*)(kp + j * 32);
+    }
+    if (one_page) {  // the lane's four keys start at a multiple of four and pages hold at least four: one table entry
+      const int kv0 = k0 + 4 * q4;
+      const int page = page_of(min(kv0, ke));
+      const bf16_t* vp = vc + (((size_t)page * Hkv + kvh) << psh) * hd + sub * 8;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) tn.v[u] = *(const uint4*)(vp + (size_t)(min(kv0 + u, ke) & (page_size - 1)) * hd);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int kv = min(k0 + 4 * q4 + u, ke);
+        const int page = page_of(kv);
+        tn.v[u] = *(const uint4*)(vc + ((((size_t)page * Hkv + kvh) << psh) + (kv & (page_size - 1))) * hd + sub * 8);
+      }
+    }
+  };
+  auto from_table = [&](int key) { return tbl[key >> psh]; };
+  auto from_copy = [&](int key) { return tb[(key >> psh) - b0]; };
+  // The token that is only now stored is the range's last key (and stands in for those beyond). Whatever lay in its place is
+  // read with the others, before q is prepared, and replaced here by what wave 1 left in LDS.
+  const bool has_new = slot >= 0 && s == s_hi;
+  auto with_new = [&](int k0, Turn& tn) {
+    if (!has_new || k0 + 15 < ke) return;
+    if (k0 + sub >= ke) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) tn.k[j] = *(const u32x4*)(&new_kv[0][j * 32 + q4 * 8]);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (k0 + 4 * q4 + u >= ke) tn.v[u] = *(const uint4*)(&new_kv[1][sub * 8]);
+  };
+  const int k_first = kb + wave * 16;
+  Turn ta, tb2;
+  fetch(k_first, ta, from_table);
   const bf16_t* qrow = q + (size_t)t * ldq + (size_t)kvh * G * hd;
   u32x4 qf[4];  // B operand: head `sub`, dims 32 j + 8 q4 .. + 8
   if (FUSED) {
-    // wave 0 prepares q: lane group q4 takes heads q4, q4 + 4, ..; norm and rotation in the 8-dims-per-lane layout
+    // wave 0 prepares q: lane group q4 takes heads q4, q4 + 4, ..; norm and rotation in the 8-dims-per-lane layout. Wave 1 of
+    // the last split prepares the new key meanwhile.
     const bool rotate = fu.cos_t != nullptr;
-    if (wave == 0) {
+    const bool stores = wave == 1 && has_new;
+    if (wave == 0 || stores) {
       LaneAngles an;
-      float gq8[8];
+      float gain[8];
       const int d0 = sub * 8, half = fu.rot >> 1;
       an.low = rotate && d0 < half;
       an.high = rotate && d0 >= half && d0 < fu.rot;
@@ -514,35 +577,33 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
         load8(fu.cos_t, JLLM_F32, at, an.c);
         load8(fu.sin_t, JLLM_F32, at, an.s);
       }
-      if (fu.gq) load8(fu.gq, fu.gain_dtype, d0, gq8);
+      if (wave == 0) {
+        if (fu.gq) load8(fu.gq, fu.gain_dtype, d0, gain);
 #pragma unroll
-      for (int g0 = 0; g0 < G; g0 += 4) {
-        const int g = g0 + q4;
-        uint4 v = uint4{0u, 0u, 0u, 0u};
-        if (g < G) v = *(const uint4*)(qrow + (size_t)g * hd + d0);
-        float x[8];
-        unpack8(v, x);
-        norm_rope8<LPK>(x, gq8, fu.gq != nullptr, an, rotate, fu.eps, hd, true);
-        if (g < G) *(uint4*)(&qs[g][d0]) = uint4{pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
-      }
-      if (fu.write_kv && s == s_hi && q4 == 0) {
-        // the new token's key and value go into their page before anyone reads the keys of this split
-        const int slot = fu.slots[t];
-        if (slot >= 0) {
-          const int page = slot >> psh;
-          const size_t dst = ((((size_t)page * Hkv + kvh) << psh) + (slot & (page_size - 1))) * hd + d0;
-          const bf16_t* kin = q + (size_t)t * ldq + (size_t)(H + kvh) * hd + d0;
-          const uint4 kv_ = *(const uint4*)kin;
-          const uint4 vv = *(const uint4*)(kin + (size_t)Hkv * hd);
-          float gk8[8];
-          if (fu.gk) load8(fu.gk, fu.gain_dtype, d0, gk8);
+        for (int g0 = 0; g0 < G; g0 += 4) {
+          const int g = g0 + q4;
+          uint4 v = uint4{0u, 0u, 0u, 0u};
+          if (g < G) v = *(const uint4*)(qrow + (size_t)g * hd + d0);
           float x[8];
-          unpack8(kv_, x);
-          norm_rope8<LPK>(x, gk8, fu.gk != nullptr, an, rotate, fu.eps, hd, true);
-          *(uint4*)(fu.kc_w + dst) = uint4{pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
-          *(uint4*)(fu.vc_w + dst) = vv;
+          unpack8(v, x);
+          norm_rope8<LPK>(x, gain, fu.gq != nullptr, an, rotate, fu.eps, hd, true);
+          if (g < G) *(uint4*)(&qs[g][d0]) = uint4{pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
         }
-        __threadfence_block();
+      } else if (q4 == 0) {
+        const int page = slot >> psh;
+        const size_t dst = ((((size_t)page * Hkv + kvh) << psh) + (slot & (page_size - 1))) * hd + d0;
+        const bf16_t* kin = q + (size_t)t * ldq + (size_t)(H + kvh) * hd + d0;
+        const uint4 kv_ = *(const uint4*)kin;
+        const uint4 vv = *(const uint4*)(kin + (size_t)Hkv * hd);
+        if (fu.gk) load8(fu.gk, fu.gain_dtype, d0, gain);
+        float x[8];
+        unpack8(kv_, x);
+        norm_rope8<LPK>(x, gain, fu.gk != nullptr, an, rotate, fu.eps, hd, true);
+        const uint4 kn = uint4{pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
+        *(uint4*)(&new_kv[0][d0]) = kn;
+        *(uint4*)(&new_kv[1][d0]) = vv;
+        *(uint4*)(fu.kc_w + dst) = kn;
+        *(uint4*)(fu.vc_w + dst) = vv;
       }
     }
   } else {
@@ -562,39 +623,6 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
     for (int j = 0; j < 4; ++j)
       qf[j] = sub < G ? *(const u32x4*)(&qs[sub < G ? sub : 0][j * 32 + q4 * 8]) : u32x4{0u, 0u, 0u, 0u};
   }
-  // a turn: keys k0 .. k0 + 15 of this wave. K for the scores: key k0 + sub, dims 32 j + 8 q4; V for the sums: key
-  // k0 + 4 q4 + u, dims 8 sub. The next turn's are requested before this turn's are used.
-  struct Turn {
-    u32x4 k[4];
-    uint4 v[4];
-  };
-  const bool one_page = page_size >= 4 && (kb & 3) == 0;
-  // keys beyond the end of the range are read as the last key of the range (a valid one): no branches and nothing to
-  // clear; their scores are masked below and their probabilities are zero
-  auto fetch = [&](int k0, Turn& tn) {
-    const int kk = min(k0 + sub, ke);
-    {
-      const int page = tb[(kk >> psh) - b0];
-      const bf16_t* kp = kc + ((((size_t)page * Hkv + kvh) << psh) + (kk & (page_size - 1))) * hd + q4 * 8;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) tn.k[j] = *(const u32x4*)(kp + j * 32);
-    }
-    if (one_page) {  // the lane's four keys start at a multiple of four and pages hold at least four: one table entry
-      const int kv0 = k0 + 4 * q4;
-      const int page = tb[(min(kv0, ke) >> psh) - b0];
-      const bf16_t* vp = vc + (((size_t)page * Hkv + kvh) << psh) * hd + sub * 8;
-#pragma unroll
-      for (int u = 0; u < 4; ++u) tn.v[u] = *(const uint4*)(vp + (size_t)(min(kv0 + u, ke) & (page_size - 1)) * hd);
-    } else {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int kv = min(k0 + 4 * q4 + u, ke);
-        const int page = tb[(kv >> psh) - b0];
-        tn.v[u] = *(const uint4*)(vc + ((((size_t)page * Hkv + kvh) << psh) + (kv & (page_size - 1))) * hd + sub * 8);
-      }
-    }
-  };
-  const int k_first = kb + wave * 16;
   auto turn = [&](int k0, const Turn& tn) {
     floatx4 sc = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -630,13 +658,13 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
     for (int j = 0; j < 8; ++j) acc[j] = mfma16k16(lds_read_tr16(v_tr + 16 * j), pb, acc[j]);
   };
   // two sets of registers take turns: while one turn is computed the next one's keys and values arrive in the other
-  Turn ta, tb2;
-  fetch(k_first, ta);
   for (int k0 = k_first; k0 <= ke; k0 += 2 * DA_WAVES * 16) {
-    fetch(k0 + DA_WAVES * 16, tb2);
+    fetch(k0 + DA_WAVES * 16, tb2, from_copy);
+    with_new(k0, ta);
     turn(k0, ta);
     if (k0 + DA_WAVES * 16 > ke) break;
-    fetch(k0 + 2 * DA_WAVES * 16, ta);
+    fetch(k0 + 2 * DA_WAVES * 16, ta, from_copy);
+    with_new(k0 + DA_WAVES * 16, tb2);
     turn(k0 + DA_WAVES * 16, tb2);
   }
   // the sum over the four key groups; then the waves merge, in order, through LDS
