@@ -468,11 +468,11 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(G
 // receives dim i of the group's four keys). One running maximum per head serves all four key groups of a wave; it
 // moves only when a turn's maximum exceeds it by more than 2^8, so the accumulators are rarely rescaled.
 //
-// A step of few rows is one chain of latencies: position and table, then the first keys beside q, then the products. So
-// position, request and slot are asked for together, the first keys straight through the table before q is prepared
-// (instead of behind the barrier that shares table and q), the new key is another wave's work than q, and its readers
-// take it from LDS. Whole steps, before and after: 300 keys of the 0.6B shape 1,106 -> 1,101 us, 4 x 4B at long contexts
-// 3,614 -> 3,573, 64 x 8B 6,519 -> 6,404.
+// A step of few rows is one chain of latencies: position and table, then q and the new key, then the first keys, then the
+// products. So position, request and slot are asked for together, the new key is another wave's work than q, and its
+// readers take it from LDS, so that nobody waits for its store. Whole steps, before and after: 300 keys of
+// the 0.6B shape 1,106 -> 1,089 us, one request of 2,048 keys (8B) 3,566 -> 3,535, 64 x 8B 6,536 -> 6,461.
+// The first keys straight through the table, before q is prepared, were slower (300 keys of the 0.6B shape 1,089 -> 1,104).
 template <int G, bool FUSED>
 __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, 3))) void decode_attention_mfma_kernel(
     const bf16_t* q, int ldq, const bf16_t* kc, const bf16_t* vc, const int* __restrict__ block_table, int max_blocks,
@@ -517,17 +517,17 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
   const bool one_page = page_size >= 4 && (kb & 3) == 0;
   // keys beyond the end of the range are read as the last key of the range (a valid one): no branches and nothing to
   // clear; their scores are masked below and their probabilities are zero
-  auto fetch = [&](int k0, Turn& tn, auto page_of) {
+  auto fetch = [&](int k0, Turn& tn) {
     const int kk = min(k0 + sub, ke);
     {
-      const int page = page_of(kk);
+      const int page = tb[(kk >> psh) - b0];
       const bf16_t* kp = kc + ((((size_t)page * Hkv + kvh) << psh) + (kk & (page_size - 1))) * hd + q4 * 8;
 #pragma unroll
       for (int j = 0; j < 4; ++j) tn.k[j] = *(const u32x4*)(kp + j * 32);
     }
     if (one_page) {  // the lane's four keys start at a multiple of four and pages hold at least four: one table entry
       const int kv0 = k0 + 4 * q4;
-      const int page = page_of(min(kv0, ke));
+      const int page = tb[(min(kv0, ke) >> psh) - b0];
       const bf16_t* vp = vc + (((size_t)page * Hkv + kvh) << psh) * hd + sub * 8;
 #pragma unroll
       for (int u = 0; u < 4; ++u) tn.v[u] = *(const uint4*)(vp + (size_t)(min(kv0 + u, ke) & (page_size - 1)) * hd);
@@ -535,15 +535,13 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int kv = min(k0 + 4 * q4 + u, ke);
-        const int page = page_of(kv);
+        const int page = tb[(kv >> psh) - b0];
         tn.v[u] = *(const uint4*)(vc + ((((size_t)page * Hkv + kvh) << psh) + (kv & (page_size - 1))) * hd + sub * 8);
       }
     }
   };
-  auto from_table = [&](int key) { return tbl[key >> psh]; };
-  auto from_copy = [&](int key) { return tb[(key >> psh) - b0]; };
-  // The token that is only now stored is the range's last key (and stands in for those beyond). Whatever lay in its place is
-  // read with the others, before q is prepared, and replaced here by what wave 1 left in LDS.
+  // The token that is only now stored is the range's last key (and stands in for those beyond). Whatever lies in its place is
+  // read with the others and replaced here by what wave 1 left in LDS.
   const bool has_new = slot >= 0 && s == s_hi;
   auto with_new = [&](int k0, Turn& tn) {
     if (!has_new || k0 + 15 < ke) return;
@@ -557,7 +555,6 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
   };
   const int k_first = kb + wave * 16;
   Turn ta, tb2;
-  fetch(k_first, ta, from_table);
   const bf16_t* qrow = q + (size_t)t * ldq + (size_t)kvh * G * hd;
   u32x4 qf[4];  // B operand: head `sub`, dims 32 j + 8 q4 .. + 8
   if (FUSED) {
@@ -618,6 +615,7 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
   bf16_t* vw = (bf16_t*)pool + wave * 16 * VLD;
   const bf16_t* v_tr = vw + (4 * q4 + (sub >> 2)) * VLD + 4 * (sub & 3);  // what this lane names in a transposing load
   __syncthreads();
+  fetch(k_first, ta);
   if (FUSED) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -659,11 +657,11 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
   };
   // two sets of registers take turns: while one turn is computed the next one's keys and values arrive in the other
   for (int k0 = k_first; k0 <= ke; k0 += 2 * DA_WAVES * 16) {
-    fetch(k0 + DA_WAVES * 16, tb2, from_copy);
+    fetch(k0 + DA_WAVES * 16, tb2);
     with_new(k0, ta);
     turn(k0, ta);
     if (k0 + DA_WAVES * 16 > ke) break;
-    fetch(k0 + 2 * DA_WAVES * 16, ta, from_copy);
+    fetch(k0 + 2 * DA_WAVES * 16, ta);
     with_new(k0 + DA_WAVES * 16, tb2);
     turn(k0 + DA_WAVES * 16, tb2);
   }
