@@ -499,7 +499,7 @@ __global__ __launch_bounds__(256) void heads_finish_split_kernel(const float* __
                                                                  const TW* __restrict__ gain, const TG* __restrict__ gate,
                                                                  int ldg, int gate_fn, float out_mul, TO* __restrict__ out,
                                                                  int ldo, int gate_per_head, const float* __restrict__ sinks) {
-  __shared__ float sums[4];
+  __shared__ float of_dim[256];
   const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, j = threadIdx.x;  // a thread owns one dim (dv <= 256)
   const int jc = min(j, dv - 1);
   // everything that does not hang on another load is asked for first: the ranges' maxima and sums (lane z holds range
@@ -545,10 +545,14 @@ __global__ __launch_bounds__(256) void heads_finish_split_kernel(const float* __
   }
   float r = 1.0f;
   if (normed) {
-    const float ss = wave_sum(j < dv ? o * o : 0.f);
-    if (lane == 0) sums[threadIdx.x >> 6] = ss;
+    // every wave sums the squares in the order of the kernel for merged heads (a lane's dims 64 apart, then the lanes): a
+    // head's norm has the same bits from either
+    of_dim[j] = j < dv ? o : 0.f;
     __syncthreads();
-    r = norm_scale((sums[0] + sums[1]) + (sums[2] + sums[3]), dv, eps) * norm_mul;
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ss = fmaf(of_dim[lane + 64 * i], of_dim[lane + 64 * i], ss);
+    r = norm_scale(wave_sum(ss), dv, eps) * norm_mul;
   }
   if (j >= dv) return;
   float x = o * r;

@@ -268,6 +268,28 @@ def test_attention_kernel_on_crafted_keys(dtype, maps, softcap):
             assert torch.allclose(merged_late, merged_first, atol=1e-5, rtol=1e-5)
 
 
+@pytest.mark.parametrize("dv,splits,maps", [(256, 9, 2), (128, 3, 2), (70, 12, 1), (200, 64, 2), (5, 2, 1)])
+def test_heads_norm_has_the_same_bits_over_key_ranges(dv, splits, maps):
+    """The kernel that merges key ranges and finishes the heads against the one for merged heads, bit for bit: the first
+    without a norm leaves the heads that the second then norms."""
+    from jllm_serve_amd.kernels import ops
+    g = torch.Generator().manual_seed(dv)
+    T, H = 37, 5
+    part = torch.randn(T, H * maps, splits, dv + 2, generator=g)
+    part[..., dv] = torch.randn(T, H * maps, splits, generator=g) * 4  # maxima as exponents of two
+    part[..., dv + 1] = torch.rand(T, H * maps, splits, generator=g) * 30 + 1
+    part[::3, :, 1:, dv] = -float("inf")  # ranges without keys: their sums were never written
+    part[::3, :, 1:, :dv] = float("nan")
+    heads = ops.SplitHeads(part.to(DEV).flatten(), splits, T, H * maps, dv)
+    gain = (torch.randn(dv, generator=g) * 0.1 + 1).to(DEV)
+    gate = torch.randn(T, H * dv, generator=g).to(DEV)
+    kw = dict(normed=True, eps=1e-5, norm_mul=0.7, gain=gain, gate=gate)
+    at_once = ops.heads_finish(heads, H, maps, dv, torch.float32, lam=0.3, **kw)
+    merged = ops.heads_finish(heads, H, maps, dv, torch.float32, lam=0.3)
+    assert bool(torch.isfinite(merged).all())
+    assert torch.equal(at_once, ops.heads_finish(merged, H, 1, dv, torch.float32, **kw))
+
+
 def test_qkv_prepare_options():
     """Whole-projection norm, pair rotation over a part of the head, the query temperature at its steps, and the
     store into shuffled pages, each alone and together; rows without a place store nothing."""
