@@ -4,24 +4,25 @@
 // gemm_mfma.hip, which shares its operands through LDS.)
 //
 // What counts is how many bytes are on their way. A workgroup owns 32 weight rows of a tile's expert (16 outputs of the
-// gated product: gate and up) and cuts K among its eight waves, 64 k (a whole 128-byte line of every row) at a time, so
-// for K = 2,048 all of a wave's 16 KB of weights are requested at once; the waves' sums (MFMA 16x16x32, weight rows as the
-// first operand, the tile's activation rows, gathered by the tile's row list, as the second) meet in LDS and are added in the
-// order of the waves. With a wave per 64 outputs that walked K by itself, two steps ahead, gate/up of 20 experts of
-// 1,024 x 2,048 took 50 us (3.3 TB/s) and down 26.
+// gated product: gate and up) and cuts K among its eight waves, 256 k each in turn (four waves where K is no longer than
+// theirs), so for K = 2,048 all of its weights are requested at once. The sums (MFMA 16x16x32, weight rows as the first
+// operand, the tile's activation rows, gathered by the tile's row list, as the second) go from wave to wave through LDS:
+// one accumulator per output takes its k in ascending order, as in the grouped form, so that a row's outputs have the same
+// bits however many rows its experts get. Gate/up of 14 experts of 1,024 x 2,048 25 us, down 13; with a wave per 64
+// outputs that walked K by itself, two steps ahead, 46 and 19; with a sum per wave, added at the end, 24 and 13 in other bits.
 #include "common.h"
 #include "mfma.h"
 
-#define MM_WAVES 8
-#define MM_K (MM_WAVES * 64)  // k per turn of the workgroup
-#define MM_AHEAD 4            // turns whose loads are out together
+#define MM_STEPS 8  // steps of 32 k whose operands a wave holds
 
-template <bool GATED>
-__global__ __launch_bounds__(MM_WAVES * 64, 4) void moe_gemm_mfma_kernel(
+template <bool GATED, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 4) void moe_gemm_mfma_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
     void* __restrict__ out, int out_dtype, int ldo, int N, int K, const int* __restrict__ sorted,
     const int* __restrict__ tiles, int top, int in_map, int out_map, float weight, GateSpec gs) {
-  __shared__ floatx4 red[MM_WAVES][2][64];
+  constexpr int TURN = WAVES * MM_STEPS * 32;  // k per turn of the workgroup
+  __shared__ floatx4 sums[2][64];
+  __shared__ int asgs[16];  // the rows' assignments, for the stores (a register less while the operands are held)
   const int tile = blockIdx.y;
   const int rows = tiles[3 * tile + 2];
   if (rows == 0) return;
@@ -30,62 +31,72 @@ __global__ __launch_bounds__(MM_WAVES * 64, 4) void moe_gemm_mfma_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = lane & 15, q4 = lane >> 4;
   const int n0 = blockIdx.x * (GATED ? 16 : 32);
-  const int place = first + min(sub, rows - 1);
-  const int asg = sorted[place];
-  const bf16_t* xrow = A + (size_t)(in_map ? asg / top : place) * lda;
+  const bf16_t* xrow;
+  {
+    const int place = first + min(sub, rows - 1), asg = sorted[place];
+    if (threadIdx.x < 16) asgs[sub] = asg;
+    xrow = A + (size_t)(in_map ? asg / top : place) * lda;
+  }
   // the two blocks of 16 weight rows: gate and up of the same outputs, or 32 neighbouring outputs (beyond N: the last row)
   const bf16_t* w0 = W + ((size_t)e * N + min(n0 + sub, N - 1)) * K;
   const bf16_t* w1 = GATED ? W2 + ((size_t)e * N + min(n0 + sub, N - 1)) * K : W + ((size_t)e * N + min(n0 + 16 + sub, N - 1)) * K;
-  floatx4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
-  int k0 = wave * 64 + 8 * q4;  // this lane's first k; a turn holds two steps of 32
-  for (; k0 - 8 * q4 + (MM_AHEAD - 1) * MM_K + 64 <= K; k0 += MM_AHEAD * MM_K) {
-    u32x4 x[2 * MM_AHEAD], a[2 * MM_AHEAD], b[2 * MM_AHEAD];
+  u32x4 x[MM_STEPS], a[MM_STEPS], b[MM_STEPS];
+  auto fetch = [&](int k0) {  // this wave's share of a turn; places beyond K are read at the row's start
+    const bf16_t *p0 = w0 + k0 + 8 * q4, *p1 = w1 + k0 + 8 * q4, *px = xrow + k0 + 8 * q4;
+    if (k0 + MM_STEPS * 32 <= K) {
 #pragma unroll
-    for (int i = 0; i < 2 * MM_AHEAD; ++i) {
-      const int k = k0 + (i >> 1) * MM_K + (i & 1) * 32;
-      a[i] = *(const u32x4*)(w0 + k);
-      b[i] = *(const u32x4*)(w1 + k);
-      x[i] = *(const u32x4*)(xrow + k);
+      for (int i = 0; i < MM_STEPS; ++i) {
+        a[i] = *(const u32x4*)(p0 + 32 * i);
+        b[i] = *(const u32x4*)(p1 + 32 * i);
+        x[i] = *(const u32x4*)(px + 32 * i);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < MM_STEPS; ++i) {
+        const int by = k0 + 32 * i + 8 * q4 < K ? 32 * i : -(k0 + 8 * q4);
+        a[i] = *(const u32x4*)(p0 + by);
+        b[i] = *(const u32x4*)(p1 + by);
+        x[i] = *(const u32x4*)(px + by);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
+  };
+  int k0 = wave * MM_STEPS * 32;
+  if (k0 < K) fetch(k0);
+  for (int turn = 0; turn < K; turn += TURN) {
+    const int waves = min(WAVES, (K - turn + MM_STEPS * 32 - 1) / (MM_STEPS * 32));  // that have k in this turn
+    for (int w = 0; w < waves; ++w) {
+      if (w == wave) {
+        floatx4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
+        if (k0 > 0) acc0 = sums[0][lane], acc1 = sums[1][lane];
+        if (k0 + MM_STEPS * 32 <= K) {
 #pragma unroll
-    for (int i = 0; i < 2 * MM_AHEAD; ++i) {
-      acc0 = mfma16(a[i], x[i], acc0);
-      acc1 = mfma16(b[i], x[i], acc1);
+          for (int i = 0; i < MM_STEPS; ++i) {
+            acc0 = mfma16(a[i], x[i], acc0);
+            acc1 = mfma16(b[i], x[i], acc1);
+          }
+        } else {  // the end of K: what was read beyond it counts as zeros
+#pragma unroll
+          for (int i = 0; i < MM_STEPS; ++i) {
+            const bool in = k0 + 32 * i + 8 * q4 < K;
+            const u32x4 none = {0u, 0u, 0u, 0u};
+            acc0 = mfma16(in ? a[i] : none, in ? x[i] : none, acc0);
+            acc1 = mfma16(in ? b[i] : none, in ? x[i] : none, acc1);
+          }
+        }
+        sums[0][lane] = acc0;
+        sums[1][lane] = acc1;
+        k0 += TURN;
+        if (k0 < K) fetch(k0);
+      }
+      __syncthreads();
     }
   }
-  {  // what is left of the wave's K: places beyond the end are read inside the row and multiplied as zeros
-    u32x4 x[2 * MM_AHEAD], a[2 * MM_AHEAD], b[2 * MM_AHEAD];
-#pragma unroll
-    for (int i = 0; i < 2 * MM_AHEAD; ++i) {
-      const int k = k0 + (i >> 1) * MM_K + (i & 1) * 32;
-      if (k - 8 * q4 >= K) continue;  // (the same in all lanes)
-      const int at = k < K ? k : 0;
-      a[i] = *(const u32x4*)(w0 + at);
-      b[i] = *(const u32x4*)(w1 + at);
-      x[i] = *(const u32x4*)(xrow + at);
-    }
-#pragma unroll
-    for (int i = 0; i < 2 * MM_AHEAD; ++i) {
-      const int k = k0 + (i >> 1) * MM_K + (i & 1) * 32;
-      if (k - 8 * q4 >= K) continue;
-      const u32x4 none = {0u, 0u, 0u, 0u};
-      acc0 = mfma16(k < K ? a[i] : none, k < K ? x[i] : none, acc0);
-      acc1 = mfma16(k < K ? b[i] : none, k < K ? x[i] : none, acc1);
-    }
-  }
-  red[wave][0][lane] = acc0;
-  red[wave][1][lane] = acc1;
-  __syncthreads();
   if (wave >= (GATED ? 1 : 2)) return;
-  floatx4 s0 = red[0][wave][lane], s1 = red[0][1][lane];
-#pragma unroll
-  for (int w = 1; w < MM_WAVES; ++w) {
-    s0 += red[w][wave][lane];
-    if (GATED) s1 += red[w][1][lane];
-  }
+  const floatx4 s0 = sums[wave][lane], s1 = sums[1][lane];
   const int n = n0 + 16 * wave + 4 * q4;
   if (sub >= rows || n >= N) return;
+  const int place = first + sub, asg = asgs[sub];
   const size_t orow = out_map == 0 ? (size_t)place : out_map == 1 ? (size_t)asg : (size_t)(asg / top);
   float v[4];
 #pragma unroll
@@ -122,13 +133,21 @@ extern "C" int jllm_moe_gemm_bf16(const void* A, int a_dtype, int lda, const voi
   if (((uintptr_t)out & need) || (ldo & 3)) return 1;
   const int per_group = W2 ? 16 : 32;
   dim3 grid((N + per_group - 1) / per_group, max_tiles);
-#define MM_LAUNCH(GATED)                                                                                                    \
-  moe_gemm_mfma_kernel<GATED><<<grid, MM_WAVES * 64, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, out, \
-                                                                  out_dtype, ldo, N, K, sorted, tiles, top, in_map, out_map, weight, gs)
-  if (W2)
-    MM_LAUNCH(true);
-  else
-    MM_LAUNCH(false);
+#define MM_LAUNCH(GATED, WAVES)                                                                                             \
+  moe_gemm_mfma_kernel<GATED, WAVES><<<grid, WAVES * 64, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, out, \
+                                                                      out_dtype, ldo, N, K, sorted, tiles, top, in_map, out_map, weight, gs)
+  const bool four = K <= 4 * MM_STEPS * 32;  // more waves would have no k
+  if (W2) {
+    if (four)
+      MM_LAUNCH(true, 4);
+    else
+      MM_LAUNCH(true, 8);
+  } else {
+    if (four)
+      MM_LAUNCH(false, 4);
+    else
+      MM_LAUNCH(false, 8);
+  }
 #undef MM_LAUNCH
   JLLM_CHECK_LAUNCH("moe_gemm_bf16");
   return 0;

@@ -229,6 +229,31 @@ def test_grouped_products_of_few_rows(N, K):
     assert bool(((h[place].double() - want).abs() <= 2.0 ** -8 * want.abs() + 4.0 * room.max() * scale + 2.0 ** -20 * scale).all())
 
 
+@pytest.mark.parametrize("N,K", [(48, 64), (20, 320), (132, 1024), (36, 1088), (64, 2048), (40, 2368), (16, 4160)])
+def test_experts_rows_have_the_same_bits_in_few_and_in_many(N, K):
+    """A row's outputs from the tiles of 16 rows (K over the waves of a workgroup, whole turns and parts of one) and from the
+    tiles of 128, bit for bit, plain and gated."""
+    from jllm_serve_amd.kernels import ops
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(N + K)
+    E, top, T = 3, 2, 130
+    w, w2 = (torch.randn(E, N, K, device="cuda", generator=gen).bfloat16() for _ in range(2))
+    table = torch.rand(T, E, device="cuda", generator=gen).argsort(dim=1)[:, :top].to(torch.int32).contiguous()
+    x = (torch.randn(T, K, device="cuda", generator=gen) * K ** -0.5).bfloat16()
+    got = []
+    for many in (False, True):
+        routing = ops.moe_route(None, table, E, many_ok=many)
+        assert routing.many == many
+        place = routing.place_of.long()
+        plain = torch.full((T * top, N), float("nan"), device="cuda")
+        ops.moe_gemm(x, w, routing, out=plain, in_map=1, out_map=0)
+        pairs = torch.full((T * top, N), float("nan"), device="cuda")
+        ops.moe_gemm(x, w, routing, w2=w2, out=pairs, in_map=1, out_map=0)
+        got.append((plain[place], pairs[place]))
+    assert bool(torch.isfinite(got[0][0]).all())
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("dtype, fast", [("float32", False), ("bfloat16", True), ("bfloat16", False)])
 @pytest.mark.parametrize("H, R, Dr, page", [(4, 32, 16, 8), (5, 48, 8, 16), (16, 64, 32, 32), (40, 16, 16, 4), (3, 24, 6, 8)])
 def test_attention_kernels_on_crafted_keys(dtype, fast, H, R, Dr, page):
