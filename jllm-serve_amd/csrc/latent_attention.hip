@@ -28,7 +28,7 @@
 #define LM_QW 4  // waves with query vectors of their own; waves 4..7 repeat them for the other half of the latent
 #define LM_KEYS 64
 #define LM_TILE_ROWS 16
-#define LM_AHEAD 3
+#define LM_AHEAD 4  // fragments of keys requested ahead of the multiplies
 #define LM_PS (LM_KEYS + 8)  // elements between two query vectors' probabilities
 
 __device__ __forceinline__ float lm_exp_diff(float a, float b) { return a == -INFINITY ? 0.f : __expf(a - b); }
@@ -224,11 +224,18 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
 // an eighth of the latent. A V^T fragment so serves four products and only the scores' K fragments one. What bounds
 // it are those: 288 KB of LDS reads a block of 64 keys of 576 entries. Two barriers a block: the scores of a block
 // follow the sums of the one before without one. Nothing in the loops is conditional on sizes (a conditional step waits for
-// its own LDS reads): rows are staged with zeros up to DKS steps of 32. 16 heads, 512 + 64 entries, against the kernel above
-// for single rows, which took these runs too and computed every score twice: prompts of 300 to 1,211 rows (3,611 in all)
-// 325 -> 133 us, 4,096 rows 1,204 -> 472, 487 rows 74 -> 33, six of 20 rows and ten single rows of 1,500 to 1,950 keys
-// 108 -> 80. A key's probability lies where the value product's lane wants it (keys
-// 4 g .. and 16 + 4 g .. of 32 together, the order in which two transposing loads deliver V^T).
+// its own LDS reads): rows are staged with zeros up to DKS steps of 32.
+//
+// A row has the bits that the kernel above gives it: scores in two chains, the running maximum and the denominator
+// moved 16 keys at a time (the waves of a block's first 32 keys hand the denominators to those of the second), 32 keys of
+// values in one product (the matrix core adds the first 16 and then the others, as two products of 16 do), a row
+// alone with at most 16 heads in four sums, one for every fourth 16 keys. A key that a row does not see is multiplied by
+// 0, which an infinite value would not survive: a result that is no finite number is computed again from its own keys.
+//
+// 16 heads, 512 + 64 entries, against the kernel above, which took these runs too and computed every score twice: prompts
+// of 300 to 1,211 rows (3,611 in all) 400 -> 186 us, 487 rows 73 -> 36, six of 20 rows and ten single rows of 1,500 to 1,950
+// keys 152 -> 98, 2,048 rows with a window of 512 165 -> 88. With scores in one chain and maxima moved 64 keys at a time,
+// in other bits, 168, 32, 78 and 78.
 template <int NJ, int DKS>  // NJ: 16-dim blocks of the latent per wave at most (8 NJ >= R / 16); DKS as above
 __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_rows_kernel(
     const bf16_t* __restrict__ qa, int ldq, bf16_t* __restrict__ out, int ldo, const bf16_t* __restrict__ cache,
@@ -238,8 +245,9 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_rows_kernel(
   extern __shared__ __align__(16) unsigned char lm_smem[];
   bf16_t* Ks = (bf16_t*)lm_smem;             // [2][LM_KEYS][LD]
   bf16_t* Ps = Ks + (size_t)2 * LM_KEYS * LD;  // [64 query vectors][LM_PS]: a block's probabilities
-  float* mxs = (float*)(Ps + 64 * LM_PS);    // [2][64]: the block's maximum over either half of its keys; at the end the sums
-  float* als = mxs + 128;                    // [64]: the factor of what was summed before; at the end of everything
+  float* mxs = (float*)(Ps + 64 * LM_PS);    // [4][64]: the maxima over the block's four 16 keys; at the end the results' factors
+  floatx4* als = (floatx4*)(mxs + 256);      // [64]: the factors of what was summed before each of them
+  float* den = (float*)(als + 64);           // [4][64]: a lane's part of its denominator, between the waves of a block's halves
   const int tile = blockIdx.x;
   const int req = tiles[4 * tile], row0 = tiles[4 * tile + 1], rows = tiles[4 * tile + 2];
   const int RW = 64 / HB;
@@ -251,12 +259,14 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_rows_kernel(
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = lane & 15, q4 = lane >> 4;
   const int qs = wave & 3, kh = wave >> 2;
+  const bool alone = r_hi == r_lo && HB <= 16;  // the four groups of 16 query vectors are the same ones over every fourth 16 keys
   const int v = qs * 16 + sub;  // this lane's query vector of the scores
-  const int my_r = r_lo + v / HB, my_h = hb * HB + v % HB;
+  const int my_r = r_lo + (alone ? sub : v) / HB, my_h = hb * HB + (alone ? sub : v) % HB;
   const bool live = my_r <= r_hi && my_h < H;
-  const int my_pos = p_lo + v / HB;
-  const int my_first = window > 0 ? max(0, my_pos + 1 - window) : 0;
-  const int n_q = min(4, ((r_hi - r_lo + 1) * HB + 15) >> 4);  // groups of 16 query vectors with a row
+  const int my_pos = p_lo + (my_r - r_lo);
+  const int my_first = !live ? 0x7fffffff : window > 0 ? max(0, my_pos + 1 - window) : 0;  // (dead: sees no key)
+  const int n_q = alone ? 4 : min(4, ((r_hi - r_lo + 1) * HB + 15) >> 4);  // groups of 16 query vectors with a row
+  const int last_first = window > 0 ? max(0, ke + 1 - window) : 0;         // from here on to p_lo all rows see a key
   const int j_lo = wave * NJ, nj = min(NJ, (R >> 4) - j_lo);
   const int psh = __builtin_ctz(page_size);
   const int* tbl = block_table + (size_t)req * max_blocks;
@@ -276,6 +286,7 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_rows_kernel(
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[q][j] = floatx4{0.f, 0.f, 0.f, 0.f};
   float m1 = -INFINITY, l1 = 0.f;
+  if (threadIdx.x < 64) als[threadIdx.x] = floatx4{1.f, 1.f, 1.f, 1.f};  // (of groups without a row they stay so)
   // keys travel as above (eight threads to a key row, the next block's in registers while this one is multiplied); a
   // block's page is looked up a block before its rows are requested
   constexpr int CPT = (DKS + 1) / 2;
@@ -287,131 +298,229 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_rows_kernel(
   int page = tbl[key_of(blk) >> psh];
   auto fetch = [&](int b) {
     const bf16_t* src = cache + ((((size_t)page) << psh) + (key_of(b) & (page_size - 1))) * Dk;
+    int left = Dk - scol;
+    asm volatile("" : "+v"(left));
 #pragma unroll
-    for (int i = 0; i < CPT; ++i) staged[i] = *(const uint4*)(src + (scol + 64 * i < Dk ? scol + 64 * i : 0));
+    for (int i = 0; i < CPT; ++i) staged[i] = *(const uint4*)(src + (64 * i < left ? scol + 64 * i : 0));
     page = tbl[key_of(b + 1) >> psh];
   };
   auto put = [&](bf16_t* buf) {
     bf16_t* dst = buf + srow * LD + scol;
+    int left = Dk - scol;  // (compared per block: the nine results would be held over the loop)
+    asm volatile("" : "+v"(left));
 #pragma unroll
     for (int i = 0; i < CPT; ++i)
-      *(uint4*)(dst + 64 * i) = scol + 64 * i < Dk ? staged[i] : uint4{0u, 0u, 0u, 0u};
+      *(uint4*)(dst + 64 * i) = 64 * i < left ? staged[i] : uint4{0u, 0u, 0u, 0u};
   };
   fetch(blk);
   put(Ks);
   __syncthreads();
   for (int cur = 0; blk <= blk_last; ++blk, cur ^= 1) {
+    const int c0 = blk * LM_KEYS;
     const bf16_t* Kb = Ks + (size_t)cur * LM_KEYS * LD;
     if (blk < blk_last) fetch(blk + 1);
     float z[8];
     if (qs < n_q) {
-      floatx4 sc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
-      const bf16_t* krow = Kb + (kh * 32 + sub) * LD + 8 * q4;
-      u32x4 kf[LM_AHEAD + 1][2];
+      floatx4 sc[2][2];  // two chains for each of the wave's two 16 keys
 #pragma unroll
-      for (int j = 0; j < DKS + LM_AHEAD; ++j) {  // fragments LM_AHEAD steps ahead of the multiplies, no more: registers
-        u32x4* slot = kf[j % (LM_AHEAD + 1)];
-        if (j < DKS) slot[0] = *(const u32x4*)(krow + 32 * j), slot[1] = *(const u32x4*)(krow + 16 * LD + 32 * j);
+      for (int i = 0; i < 4; ++i) sc[i >> 1][i & 1] = floatx4{0.f, 0.f, 0.f, 0.f};
+      const bf16_t* krow = Kb + (kh * 32 + sub) * LD + 8 * q4;
+      u32x4 kf[LM_AHEAD + 1];
+#pragma unroll
+      for (int j = 0; j < 2 * DKS + LM_AHEAD; ++j) {  // fragments LM_AHEAD steps ahead of the multiplies, no more: registers
+        if (j < 2 * DKS) kf[j % (LM_AHEAD + 1)] = *(const u32x4*)(krow + j / DKS * 16 * LD + 32 * (j % DKS));
         if (j >= LM_AHEAD) {
-          const int m = j - LM_AHEAD;
-          sc[0] = mfma16(kf[m % (LM_AHEAD + 1)][0], qf[m], sc[0]);
-          sc[1] = mfma16(kf[m % (LM_AHEAD + 1)][1], qf[m], sc[1]);
+          const int m = j - LM_AHEAD, d = m % DKS;
+          sc[m / DKS][d & 1] = mfma16(kf[m % (LM_AHEAD + 1)], qf[d], sc[m / DKS][d & 1]);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      float mx = -INFINITY;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int key = blk * LM_KEYS + kh * 32 + (i >> 2) * 16 + 4 * q4 + (i & 3);
-        z[i] = (live && key >= my_first && key <= my_pos) ? sc[i >> 2][i & 3] * scale : -INFINITY;
-        mx = fmaxf(mx, z[i]);
+      for (int g = 0; g < 2; ++g) {
+        const floatx4 s = sc[g][0] + sc[g][1];
+        const bool mine = !alone || 2 * kh + g == qs;
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = c0 + kh * 32 + g * 16 + 4 * q4 + i;
+          z[4 * g + i] = (mine && key >= my_first && key <= my_pos) ? s[i] * scale : -INFINITY;
+          mx = fmaxf(mx, z[4 * g + i]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        if (q4 == 0) mxs[(2 * kh + g) * 64 + v] = mx;
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      if (q4 == 0) mxs[kh * 64 + v] = mx;
     }
     __syncthreads();  // the maxima are there, and everyone is done with the last block's probabilities and keys
     if (blk < blk_last) put(Ks + (size_t)(cur ^ 1) * LM_KEYS * LD);
+    float al[4];
     if (qs < n_q) {
-      const float mx = fmaxf(mxs[v], mxs[64 + v]);
-      float alpha = 1.0f;
-      if (mx > m1 + 8.0f) {  // also the first visible key (m1 = -inf)
-        alpha = lm_exp_diff(m1, mx);
-        l1 *= alpha;
-        m1 = mx;
-      }
-      if (kh == 0 && q4 == 0) als[v] = alpha;
+      float m[4];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        z[i] = lm_exp_diff(z[i], m1);
-        l1 += z[i];
+      for (int g = 0; g < 4; ++g) {
+        const float mx = mxs[g * 64 + v];
+        al[g] = 1.0f;
+        if (mx > m1 + 8.0f) {  // also the first visible key (m1 = -inf: nothing was summed yet)
+          al[g] = m1 == -INFINITY ? 1.0f : __expf(m1 - mx);
+          m1 = mx;
+        }
+        m[g] = m1;
       }
-      *(u32x4*)(Ps + v * LM_PS + kh * 32 + 8 * q4) =
-          u32x4{pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3]), pack_bf16(z[4], z[5]), pack_bf16(z[6], z[7])};
+      if (kh == 0 && q4 == 0) als[v] = floatx4{al[0], al[1], al[2], al[3]};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) z[i] = lm_exp_diff(z[i], kh ? m[2 + (i >> 2)] : m[i >> 2]);
+      if (kh == 0) {
+        if (blk > (kb >> 6)) l1 = den[qs * 64 + lane];
+        l1 *= al[0];
+        l1 += z[0], l1 += z[1], l1 += z[2], l1 += z[3];
+        l1 *= al[1];
+        l1 += z[4], l1 += z[5], l1 += z[6], l1 += z[7];
+        den[qs * 64 + lane] = l1;
+      }
+      bf16_t* p = Ps + v * LM_PS + kh * 32 + 4 * q4;
+      *(u32x2*)p = u32x2{pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3])};
+      *(u32x2*)(p + 16) = u32x2{pack_bf16(z[4], z[5]), pack_bf16(z[6], z[7])};
     }
     __syncthreads();  // the probabilities and the next block's keys are there
-    float al[4];
-    bool moved = false;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {  // (groups without a row carry what nobody stores)
-      al[q] = als[q * 16 + sub];
-      moved = moved || al[q] != 1.0f;
+    if (kh == 1 && qs < n_q) {
+      l1 = den[qs * 64 + lane];
+      const floatx4 f = als[v];
+      l1 *= f[2];
+      l1 += z[0], l1 += z[1], l1 += z[2], l1 += z[3];
+      l1 *= f[3];
+      l1 += z[4], l1 += z[5], l1 += z[6], l1 += z[7];
+      den[qs * 64 + lane] = l1;
     }
-    if (__any(moved)) {
+    const floatx4 moved = als[lane];  // lane u: of query vector u; the waves come to the same answer
+    int starts = 0;                   // the groups of 16 keys in front of which some maximum moved
+    if (__any(moved[0] != 1.0f || moved[1] != 1.0f || moved[2] != 1.0f || moved[3] != 1.0f)) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[q][j] *= al[q];
+      for (int g = 0; g < 4; ++g) starts |= __any(moved[g] != 1.0f) ? 1 << g : 0;
     }
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const bf16_t* v_tr = Kb + (half * 32 + 4 * q4 + (sub >> 2)) * LD + 4 * (sub & 3) + 16 * j_lo;
-      const bf16_t* prow = Ps + sub * LM_PS + half * 32 + 8 * q4;
-      u32x4 vf[NJ];
+    const bf16_t* v_tr = Kb + (8 * q4 + (sub >> 2)) * LD + 4 * (sub & 3) + 16 * j_lo;
+    const bf16_t* prow = Ps + sub * LM_PS + 8 * q4;
+    auto values = [&](u32x4 (&vf)[NJ], int half) {
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const u32x2 a = lds_read_tr16(v_tr + 16 * j), b = lds_read_tr16(v_tr + 16 * LD + 16 * j);
+        const u32x2 a = lds_read_tr16(v_tr + half * 32 * LD + 16 * j), b = lds_read_tr16(v_tr + (half * 32 + 4) * LD + 16 * j);
         vf[j] = u32x4{a[0], a[1], b[0], b[1]};
       }
-      const u32x4 p0 = *(const u32x4*)prow;
+    };
+    // the whole block at once or, where a maximum moved inside it (rare), the keys up to there first: the others'
+    // probabilities count as zeros
+#pragma unroll 1
+    for (int g = 0, next; g < 4; g = next) {
+      next = __builtin_ctz((starts >> (g + 1) << (g + 1)) | 16);
+      uint32_t keep[2] = {~0u, ~0u};
+      if (starts) {
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[0][j] = mfma16(vf[j], p0, acc[0][j]);
-      if (n_q > 1) {
+        for (int q = 0; q < 4; ++q) {
+          const float a = ((const float*)als)[(q * 16 + sub) * 4 + g];
 #pragma unroll
-        for (int q = 1; q < 4; ++q) {
-          const u32x4 pf = *(const u32x4*)(prow + q * 16 * LM_PS);
+          for (int j = 0; j < NJ; ++j) acc[q][j] *= a;
+        }
 #pragma unroll
-          for (int j = 0; j < NJ; ++j) acc[q][j] = mfma16(vf[j], pf, acc[q][j]);
+        for (int half = 0; half < 2; ++half) keep[half] = 2 * half + (q4 >> 1) >= g && 2 * half + (q4 >> 1) < next ? ~0u : 0u;
+      }
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        u32x4 vf[NJ];
+        values(vf, half);
+        const u32x4 p0 = *(const u32x4*)(prow + half * 32) & keep[half];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[0][j] = mfma16(vf[j], p0, acc[0][j]);
+        if (n_q > 1) {
+#pragma unroll
+          for (int q = 1; q < 4; ++q) {
+            const u32x4 pf = *(const u32x4*)(prow + q * 16 * LM_PS + half * 32) & keep[half];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[q][j] = mfma16(vf[j], pf, acc[q][j]);
+          }
         }
       }
     }
   }
+  // the denominators lie with the waves of the blocks' second halves
   l1 += __shfl_xor(l1, 16, 64);
   l1 += __shfl_xor(l1, 32, 64);
-  if (q4 == 0 && kh == 1) mxs[v] = l1;
-  __syncthreads();  // (also: everyone has read the last block's factors)
-  if (q4 == 0 && kh == 0 && live) {
-    l1 += mxs[v];
+  auto factor = [&](float m, float l, int h) {
     float ca = 1.0f;
     if (sink) {
-      const float sk = sink[my_h];
-      const float mn = fmaxf(m1, sk);
-      ca = lm_exp_diff(m1, mn);
-      l1 = l1 * ca + __expf(sk - mn);
+      const float sk = sink[h];
+      const float mn = fmaxf(m, sk);
+      ca = lm_exp_diff(m, mn);
+      l = l * ca + __expf(sk - mn);
     }
-    als[v] = ca / l1;
+    return ca / l;
+  };
+  if (kh == 1 && q4 == 0) {
+    if (alone)
+      mxs[v] = m1, mxs[64 + v] = l1;
+    else if (live)
+      mxs[v] = factor(m1, l1, my_h);
   }
   __syncthreads();
+  // one query vector's sums over this wave's part of the latent, key by key
+  auto again = [&](int r, int h) {
+    const bf16_t* qrow = qa + (size_t)(row0 + r) * ldq + (size_t)h * Dk;
+    const int pos = p_lo + (r - r_lo), first = window > 0 ? max(0, pos + 1 - window) : 0;
+    const int dim = 16 * j_lo + lane;
+    float m = -INFINITY, l = 0.f, o = 0.f;
+    for (int k0 = first; k0 <= pos; k0 += 64) {
+      const int key = min(k0 + lane, pos);
+      const int at = (tbl[key >> psh] << psh) + (key & (page_size - 1));
+      float d = 0.f;
+      for (int i = 0; i < Dk; ++i) d = fmaf(ldf(qrow, i), ldf(cache + (size_t)at * Dk, i), d);
+      const float z1 = k0 + lane <= pos ? d * scale : -INFINITY;
+      const float mn = fmaxf(m, wave_max(z1)), a = lm_exp_diff(m, mn);
+      const float p = lm_exp_diff(z1, mn);
+      l = l * a + wave_sum(p);
+      o *= a;
+      m = mn;
+      for (int k = 0; k < 64 && k0 + k <= pos; ++k) {
+        const bf16_t* row = cache + (size_t)__shfl(at, k, 64) * Dk;
+        o = fmaf(__shfl(p, k, 64), lane < 16 * nj ? ldf(row, dim) : 0.f, o);
+      }
+    }
+    if (lane < 16 * nj) stf(out + (size_t)(row0 + r) * ldo, (size_t)h * R + dim, o * factor(m, l, h));
+  };
+  if (alone) {  // the four sums, in order
+    float m = mxs[sub], l = mxs[64 + sub];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+      const float om = mxs[16 * w + sub], ol = mxs[64 + 16 * w + sub];
+      const float mn = fmaxf(m, om);
+      const float a = lm_exp_diff(m, mn), b = lm_exp_diff(om, mn);
+      l = l * a + ol * b;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[0][j][i] = acc[0][j][i] * a + acc[w][j][i] * b;
+      m = mn;
+    }
+    if (sub < HB && hb * HB + sub < H) mxs[128 + sub] = factor(m, l, hb * HB + sub);  // (every wave and lane group the same)
+  }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int u = q * 16 + sub, row = r_lo + u / HB, h = hb * HB + u % HB;
-    if (row > r_hi || h >= H) continue;
-    const float inv = als[u];
+    const bool stored = (alone ? u < HB : row <= r_hi) && h < H;
+    const float inv = mxs[alone ? 128 + sub : u];
     bf16_t* o = out + (size_t)(row0 + row) * ldo + (size_t)h * R + 16 * j_lo + 4 * q4;
+    bool odd = false;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
-      if (j < nj)
-        *(u32x2*)(o + 16 * j) = u32x2{pack_bf16(acc[q][j][0] * inv, acc[q][j][1] * inv), pack_bf16(acc[q][j][2] * inv, acc[q][j][3] * inv)};
+      if (stored && j < nj) {
+        const floatx4 x = acc[q][j] * inv;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) odd = odd || !(fabsf(x[i]) < INFINITY);
+        *(u32x2*)(o + 16 * j) = u32x2{pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3])};
+      }
+    const uint64_t lanes = __ballot(odd);
+    uint32_t again_for = (uint32_t)(lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffffu;
+    for (; again_for; again_for &= again_for - 1) {
+      const int w = q * 16 + __builtin_ctz(again_for);
+      again(r_lo + w / HB, hb * HB + w % HB);
+    }
   }
 }
 
@@ -477,7 +586,7 @@ static int lm_launch_rows(dim3 grid, hipStream_t stream, const void* qa, int ldq
                           const int* block_table, int max_blocks, const int* tiles, const int* positions, int H, int R, int Dk,
                           int page_size, int window, float scale, const float* sink, int HB, int n_hb) {
   static size_t reserved = 0;
-  const size_t smem = ((size_t)2 * LM_KEYS * (DKS * 32 + 16) + 64 * LM_PS) * sizeof(bf16_t) + 192 * sizeof(float);
+  const size_t smem = ((size_t)2 * LM_KEYS * (DKS * 32 + 16) + 64 * LM_PS) * sizeof(bf16_t) + 768 * sizeof(float);
   if (smem > 48 * 1024 && smem > reserved) {
     if (hipFuncSetAttribute((const void*)latent_attention_rows_kernel<NJ, DKS>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)smem) != hipSuccess)

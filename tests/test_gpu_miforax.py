@@ -369,6 +369,75 @@ def test_latent_attention_of_runs_of_rows(H, R, Dk, window):
     assert bool(((got.view(-1, H, R).double().cpu() - torch.cat(want)).abs() <= torch.cat(room)).all())
 
 
+@pytest.mark.parametrize("H, R, Dk, window, single_runs", [(40, 512, 576, 0, False), (40, 144, 168, 90, False), (17, 128, 256, 33, False),
+                                                           (16, 512, 576, 0, True), (16, 512, 576, 70, True), (3, 96, 128, 0, True)])
+def test_latent_attention_gives_a_row_the_same_bits_in_runs_and_alone(H, R, Dk, window, single_runs):
+    """A row's result as a single row of its step and in a run of a portion, bit for bit: with more than 16 heads in runs of up
+    to 16 rows; with up to 16, where a row alone keeps four sums, in runs of one row. Keys grow along the context, so that
+    the running maxima move in every place of a block, and one request has equal keys."""
+    from jllm_serve_amd.kernels import ops
+    g = torch.Generator().manual_seed(H + Dk + window)
+    page, spans = 16, [(0, 100), (58, 6), (63, 1), (100, 130), (250, 5), (0, 1)]
+    width = 16
+    cache = torch.randn(len(spans) * width, page, Dk, generator=g)
+    table = torch.randperm(len(spans) * width, generator=g).to(torch.int32).view(len(spans), width)
+    for r in range(len(spans)):
+        cache[table[r].long()] *= (torch.arange(width * page).view(width, page, 1) / 60.0) if r != 3 else 1.0
+    cache = cache.bfloat16().to(DEV)
+    pos = [p for p0, n in spans for p in range(p0, p0 + n)]
+    req = [r for r, (p0, n) in enumerate(spans) for _ in range(n)]
+    q = (torch.randn(len(pos), H * Dk, generator=g) * 2).bfloat16().to(DEV)
+    sink = torch.randn(H, generator=g).to(DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    rows = [(req[i], i, 1, pos[i]) for i in range(len(pos))]
+    runs, at = rows, 0
+    if not single_runs:
+        runs = []
+        for r, (p0, n) in enumerate(spans):
+            runs += [(r, at + i, min(16, n - i), p0 + i) for i in range(0, n, 16)]
+            at += n
+
+    def attend(tiles, **facts):
+        return ops.latent_attention(q, cache, table.to(DEV), i32(req), i32(pos), H, R, window, Dk ** -0.5, sink,
+                                    meta={"tiles_dev": i32(tiles).flatten(), "n_tiles": len(tiles), **facts})
+
+    assert ops._latent_split(len(rows), H, window, 255) == (0, 1)
+    alone = attend(rows, single_rows=True, max_context=255)
+    assert bool(torch.isfinite(alone).all())
+    assert torch.equal(attend(runs), alone)
+
+
+@pytest.mark.parametrize("H", [3, 16, 40])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_latent_attention_of_runs_keeps_infinities_with_the_rows_that_see_them(H, bad):
+    """A cached entry that is no finite number, behind some of a run's rows and out of the window of others: only the rows
+    that see it may feel it, and those do."""
+    from jllm_serve_amd.kernels import ops
+    g = torch.Generator().manual_seed(H)
+    R, Dk, page, n, window = 64, 96, 16, 150, 40
+    cache = torch.randn(16, page, Dk, generator=g).bfloat16()
+    table = torch.randperm(16, generator=g).to(torch.int32).view(1, 16)
+    at = torch.arange(n)
+    q = torch.randn(n, H, Dk, generator=g).bfloat16()
+    keys = cache[table[0].long()].view(-1, Dk)[:n].double()
+    runs = [(0, i, min(16, n - i), i) for i in range(0, n, 16)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    for place in (1, 35, 63, 70, 149):
+        spoiled = cache.clone()
+        spoiled[int(table[0, place // page]), place % page, 5] = bad
+        got = ops.latent_attention(q.view(n, -1).to(DEV), spoiled.to(DEV), table.to(DEV), torch.zeros(n, dtype=torch.int32, device=DEV),
+                                   i32(at.tolist()), H, R, window, Dk ** -0.5, None,
+                                   meta={"tiles_dev": i32(runs).flatten(), "n_tiles": len(runs)}).cpu().double().view(n, H, R)
+        z = torch.matmul(q.double(), keys.T) * Dk ** -0.5
+        z = z.masked_fill(((at[None] > at[:, None]) | (at[None] <= at[:, None] - window))[:, None], -torch.inf)
+        p = torch.softmax(z, dim=2)
+        want = torch.matmul(p, keys[:, :R])
+        room = (2.0 ** -8 + 2.0 ** -18) * torch.matmul(p, keys[:, :R].abs()) + 2.0 ** -8 * want.abs()
+        sees = (at >= place) & (at < place + window)
+        assert bool(((got - want).abs() <= room)[~sees].all()), place
+        assert not bool(torch.isfinite(got[sees]).all(dim=2).any()), place
+
+
 # ------------------------------------------------------------------------------------------------ replays
 
 
