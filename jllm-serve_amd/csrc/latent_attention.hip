@@ -608,7 +608,7 @@ extern "C" int jllm_latent_attention_bf16(const void* qa, int ldq, void* out, in
   if (n_tiles <= 0) return 0;
   if (tile_rows != LM_TILE_ROWS) JLLM_FAIL("latent_attention: runs of %d rows, this kernel takes %d", tile_rows, LM_TILE_ROWS);
   if (H <= 0 || R <= 0 || Dk < R || window < 0 || page_size <= 0 || max_blocks <= 0) JLLM_FAIL("latent_attention: H %d R %d Dk %d window %d", H, R, Dk, window);
-  if ((R & 15) || (Dk & 7) || R > 512 || Dk > 640 || (page_size & (page_size - 1))) return 1;
+  if ((R & 15) || (Dk & 7) || R > 512 || Dk > 576 || (page_size & (page_size - 1))) return 1;  // (longer rows: two blocks of keys exceed the LDS)
   if (((uintptr_t)qa & 15) || ((uintptr_t)cache & 15) || ((uintptr_t)out & 7) || (ldq & 7) || (ldo & 3)) return 1;
   if (ldq < H * Dk || ldo < H * R) JLLM_FAIL("latent_attention: row strides %d/%d", ldq, ldo);
   int HB = 1;
@@ -627,7 +627,6 @@ extern "C" int jllm_latent_attention_bf16(const void* qa, int ldq, void* out, in
   if (split > 0 && ((split & 63) || n_z < 1 || n_z > 64 || !part)) JLLM_FAIL("latent_attention: ranges of %d keys over %d workgroups", split, n_z);
   dim3 grid(n_tiles, n_hb * (split < 0 ? n_rg : 1), split > 0 ? n_z : 1);
   int rc;
-  if (split < 0 && dkp > 576) JLLM_FAIL("latent_attention: cannot reserve %zu bytes of LDS", smem);  // (more than 160 KB)
   if (split < 0)
     rc = R <= 128 && dkp <= 256
              ? lm_launch_rows<1, 8>(grid, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, n_hb)
@@ -637,7 +636,7 @@ extern "C" int jllm_latent_attention_bf16(const void* qa, int ldq, void* out, in
   else if (R <= 128 && dkp <= 256)
     rc = lm_launch<8, 8>(grid, smem, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, LD, split, part);
   else
-    rc = lm_launch<32, 20>(grid, smem, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, LD, split, part);
+    rc = lm_launch<32, 18>(grid, smem, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, LD, split, part);
   if (rc != 0) return rc;
   JLLM_CHECK_LAUNCH("latent_attention");
   if (split > 0) {

@@ -438,6 +438,31 @@ def test_latent_attention_of_runs_keeps_infinities_with_the_rows_that_see_them(H
         assert not bool(torch.isfinite(got[sees]).all(dim=2).any()), place
 
 
+@pytest.mark.parametrize("Dk", [576, 584, 640])
+def test_latent_rows_too_long_for_the_matrix_core_kernel_take_the_general_one(Dk):
+    """Cached rows at the longest that the matrix-core kernel takes and beyond, as a run of a portion and as single rows."""
+    from jllm_serve_amd.kernels import ops
+    g = torch.Generator().manual_seed(Dk)
+    H, R, page, n = 5, 512, 16, 40
+    cache = torch.randn(4, page, Dk, generator=g).bfloat16()
+    q = torch.randn(n, H, Dk, generator=g).bfloat16()
+    table = torch.tensor([[2, 0, 3, 1]], dtype=torch.int32)
+    keys = cache[table[0].long()].view(-1, Dk)[:n].double()
+    at = torch.arange(n)
+    z = (torch.matmul(q.double(), keys.T) * Dk ** -0.5).masked_fill((at[None] > at[:, None])[:, None], -torch.inf)
+    p = torch.softmax(z, dim=2)
+    want, room = torch.matmul(p, keys[:, :R]), 2.0 ** -8 * torch.matmul(p, keys[:, :R].abs())
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    runs, rows = [(0, i, min(16, n - i), i) for i in range(0, n, 16)], [(0, i, 1, i) for i in range(n)]
+    for tiles, facts in ((runs, {}), (rows, {"single_rows": True, "max_context": n})):
+        ops.reset_stats()
+        got = ops.latent_attention(q.view(n, -1).to(DEV), cache.to(DEV), table.to(DEV), torch.zeros(n, dtype=torch.int32, device=DEV), i32(at.tolist()),
+                                   H, R, 0, Dk ** -0.5, None, meta={"tiles_dev": i32(tiles).flatten(), "n_tiles": len(tiles), **facts})
+        stats = ops.stats()
+        assert bool(stats["general"]) == (Dk > 576) and bool(stats["ran"]) == (Dk <= 576), stats
+        assert bool(((got.view(n, H, R).double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + room).all())
+
+
 # ------------------------------------------------------------------------------------------------ replays
 
 
