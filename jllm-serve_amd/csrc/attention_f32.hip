@@ -180,34 +180,79 @@ __device__ __forceinline__ floatx4 mfma_f32(float a, float b, floatx4 c) { retur
 // l % 16. Scores: D[key][c] += K[key][dims] q[c][dims], four tiles of 16 keys, 32 steps of four dims each; lane l then has
 // keys 16 t + 4 (l / 16) + i. Weighted sums: D[dim][c] += V^T[dim][key] p[c][key]; a lane's 16 bytes of V are four
 // neighbouring dims of one key, which go to four tiles (a tile's row r is dim 4 r + j of its 64 dims), so V needs no
-// transposition; keys and probabilities are transposed over the lane groups in registers. A tile whose rows belong to
-// several requests is walked once per request.
-__global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_tiles_kernel(AttF32 A, int rows) {
+// transposition; keys and probabilities are transposed over the lane groups in registers.
+//
+// A workgroup takes the rows that a tile begins with, as many as are one request's. What else lies in the tile is the work of
+// the first `spread` workgroups (SPREAD: where there are several requests), one for each request: it looks for the places
+// inside tiles where its request's rows begin. A workgroup that walked all of its tile's requests in turn made the step
+// wait for it: 20 rows of a prompt and five single rows of up to 400 keys 71 us, here 24 (the general kernel: 41); 32 single rows of
+// 1,000 to 2,860 keys behind 2,000 rows of a prompt 1,050, here 355 (1,770); 64 requests of 32 rows, where there is nothing
+// to find, 52, here 58 (195).
+template <bool SPREAD>
+__global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_tiles_kernel(AttF32 A, int rows, int spread) {
   __shared__ __align__(16) float mg[AF_WAVES][16][4 + AF_HD];  // every wave's maximum, sum (and two spare places), weighted sums
+  __shared__ int found[AF_WAVES];
   const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = A.H / A.Hkv, kvh = blockIdx.y;
-  const int t0 = blockIdx.x * rows, n = min(rows, A.n_tokens - t0);
-  const int ri = col / G;             // this lane's row of the tile ...
-  const int head = kvh * G + col % G;  // ... and head
-  floatx4 qf[AF_HD / 16];             // the lane's query vector at dims 16 c + 4 s + quad
-  {
-    const floatx4* qr = (const floatx4*)(A.q + (size_t)(t0 + min(ri, n - 1)) * A.ldq + (size_t)head * AF_HD);
+  const bool inner = SPREAD && (int)blockIdx.x < spread;
+  int t0 = inner ? 0 : ((int)blockIdx.x - (SPREAD ? spread : 0)) * rows;
+  for (;; ++t0) {
+    if (__builtin_expect(inner, 0)) {  // the next row inside a tile with which rows of this request begin
+      int at = 0x7fffffff;
+      for (; t0 < A.n_tokens; t0 += 8 * 64 * AF_WAVES) {
+        int before[8], here[8];
 #pragma unroll
-    for (int c = 0; c < AF_HD / 16; ++c) qf[c] = qr[4 * c + quad];
+        for (int u = 0; u < 8; ++u) {
+          const int t = min(t0 + u * 64 * AF_WAVES + (int)threadIdx.x, A.n_tokens - 1);
+          before[u] = A.row_req[max(t - 1, 0)], here[u] = A.row_req[t];
+        }
+#pragma unroll
+        for (int u = 7; u >= 0; --u) {
+          const int t = t0 + u * 64 * AF_WAVES + (int)threadIdx.x;
+          if (t < A.n_tokens && here[u] == (int)blockIdx.x && before[u] != here[u] && t % rows != 0) at = t;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) at = min(at, __shfl_xor(at, o, 64));
+        if (lane == 0) found[wave] = at;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < AF_WAVES; ++w) at = min(at, found[w]);
+        at = __builtin_amdgcn_readfirstlane(at);
+        __syncthreads();
+        if (at != 0x7fffffff) break;
+      }
+      if (at == 0x7fffffff) return;
+      t0 = at;
+    }
+    const int end = min(inner ? rows - t0 % rows : rows, A.n_tokens - t0);  // rows of the tile from here on
+    const int ri = min(col / G, end - 1);  // this lane's row of those taken ...
+    const int head = kvh * G + col % G;     // ... and head
+    floatx4 qf[AF_HD / 16];                // the lane's query vector at dims 16 c + 4 s + quad
+    {
+      const floatx4* qr = (const floatx4*)(A.q + (size_t)(t0 + ri) * A.ldq + (size_t)head * AF_HD);
+#pragma unroll
+      for (int c = 0; c < AF_HD / 16; ++c) qf[c] = qr[4 * c + quad];
+    }
+    // lane i of every 16 looks at row i: how many belong to the first one's request, and which keys they see
+    const int ti = t0 + min(col, end - 1), req_i = A.row_req[ti], pos_i = A.positions[ti];
+    const int req = __builtin_amdgcn_readfirstlane(req_i);
+    const int n = min(end, __builtin_ctz(~((uint32_t)__ballot(req_i == req) & 0xffffu)));
+    const int first_i = A.window > 0 ? max(0, pos_i + 1 - A.window) : 0;
+    int low = col < n ? first_i : 0x7fffffff, low_pos = col < n ? pos_i : 0x7fffffff;
+    int high = col < n ? pos_i : -1, last_first = col < n ? first_i : 0;
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) {
+      low = min(low, __shfl_xor(low, o, 64)), low_pos = min(low_pos, __shfl_xor(low_pos, o, 64));
+      high = max(high, __shfl_xor(high, o, 64)), last_first = max(last_first, __shfl_xor(last_first, o, 64));
+    }
+    low = __builtin_amdgcn_readfirstlane(low), low_pos = __builtin_amdgcn_readfirstlane(low_pos);
+    high = __builtin_amdgcn_readfirstlane(high), last_first = __builtin_amdgcn_readfirstlane(last_first);
 #pragma unroll
     for (int c = 0; c < AF_HD / 16; ++c) qf[c] = lanes_transposed(qf[c]);
-  }
-  for (int i0 = 0; i0 < n;) {  // the rows of one request
-    const int req = A.row_req[t0 + i0];
-    int i1 = i0, low = 0x7fffffff, high = -1, last_first = 0, low_pos = 0x7fffffff;
-    for (; i1 < n && A.row_req[t0 + i1] == req; ++i1) {
-      const int p = A.positions[t0 + i1], f = A.window > 0 ? max(0, p + 1 - A.window) : 0;
-      low = min(low, f), high = max(high, p), last_first = max(last_first, f), low_pos = min(low_pos, p);
-    }
     const int* tbl = A.table + (size_t)req * A.max_blocks;
-    const bool mine = ri >= i0 && ri < i1;
-    const int pos = mine ? A.positions[t0 + ri] : -1;  // a lane of other rows sees no key
+    const bool mine = col / G < n;
+    const int pos = mine ? A.positions[t0 + ri] : -1;  // a lane without a row sees no key
     const int first = mine && A.window > 0 ? max(0, pos + 1 - A.window) : 0;
     floatx4 acc[2][4];
 #pragma unroll
@@ -348,7 +393,7 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_tiles_kernel(A
     __syncthreads();
     {
       const int c = threadIdx.x >> 4, r = c / G, d0 = (threadIdx.x & 15) * 8;
-      if (r >= i0 && r < i1) {
+      if (r < n) {
         float mm = mg[0][c][0], ll = mg[0][c][1], x[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) x[i] = mg[0][c][4 + d0 + i];
@@ -370,8 +415,8 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_tiles_kernel(A
         for (int i = 0; i < 8; ++i) o[i] = x[i] * inv;
       }
     }
+    if (!inner) return;
     __syncthreads();
-    i0 = i1;
   }
 }
 
@@ -390,7 +435,11 @@ extern "C" int jllm_attention_f32(const void* q, int ldq, void* out, int ldo, co
   const int G = H / Hkv;
   if (G <= 8 && n_tokens >= 4 * n_requests) {
     const int rows = 16 / G;
-    attention_f32_tiles_kernel<<<dim3((n_tokens + rows - 1) / rows, Hkv), 64 * AF_WAVES, 0, stream>>>(A, rows);
+    const int tiles = (n_tokens + rows - 1) / rows;
+    if (n_requests > 1)
+      attention_f32_tiles_kernel<true><<<dim3(tiles + n_requests, Hkv), 64 * AF_WAVES, 0, stream>>>(A, rows, n_requests);
+    else
+      attention_f32_tiles_kernel<false><<<dim3(tiles, Hkv), 64 * AF_WAVES, 0, stream>>>(A, rows, 0);
   } else {  // heads share a workgroup where the step still has two workgroups for every compute unit, as in the general kernel
     int cus = jllm_compute_units();
     if (cus <= 0) cus = 256;

@@ -565,6 +565,29 @@ def test_float32_attention_gives_the_general_kernels_bits(ops, H, Hkv, page, win
     assert bool(torch.isfinite(want[~seen]).all()) and not bool(torch.isfinite(want[seen]).all())
 
 
+@pytest.mark.parametrize("H,Hkv,n_req,n,shuffled", [(16, 8, 64, 64, False),  # two heads to a workgroup of a row
+                                                    (12, 4, 70, 70, False),  # the same with three heads of a kv head
+                                                    (16, 8, 6, 25, False),   # single rows behind a portion, inside its last tile
+                                                    (8, 8, 5, 300, True), (24, 3, 40, 1300, True)])  # requests in no order
+def test_float32_attention_of_rows_in_any_order_gives_the_general_kernels_bits(ops, H, Hkv, n_req, n, shuffled):
+    """Head size 128 in fp32 where a tile's rows belong to several requests, whose rows may lie anywhere in the step, and
+    single rows of many requests, against the general kernel, bit for bit."""
+    g = torch.Generator().manual_seed(n)
+    lens = [int(x) for x in torch.randint(1, 200, (n_req,), generator=g)]
+    kc, vc, table, _, _ = make_cache(n_req, lens, Hkv, 128, 16, torch.float32, seed=n)
+    if shuffled:
+        req = torch.randint(0, n_req, (n,), generator=g)
+    else:
+        req = torch.cat([torch.zeros(n - n_req, dtype=torch.int64), torch.arange(n_req)])
+    pos = (torch.rand(n, generator=g) * torch.tensor(lens)[req]).long()
+    q = torch.randn(n, H * 128, generator=g).to(DEV)
+
+    def attend(slopes=None):
+        return ops.paged_attention(q, kc, vc, table, req.int().to(DEV), pos.int().to(DEV), H, Hkv, 128, 0, 128 ** -0.5, exact=True, slopes=slopes)
+
+    assert torch.equal(attend(), attend(torch.zeros(H, device=DEV)))
+
+
 @pytest.mark.parametrize("H,Hkv,hd,window", [(12, 3, 32, 0), (10, 2, 48, 70), (6, 3, 64, 0), (8, 8, 16, 0)])
 def test_general_attention_gives_a_row_the_same_bits_in_any_step(ops, H, Hkv, hd, window):
     """The general kernel (the 32-bit path) takes up to four query heads of a kv head in one workgroup when the step
