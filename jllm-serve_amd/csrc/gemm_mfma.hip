@@ -1,8 +1,12 @@
 // out[M,N] = A[M,K] * W[N,K]^T for many rows (prompt portions): bf16 operands staged through LDS, fp32
-// accumulation on the matrix cores (v_mfma_f32_16x16x32_bf16, as in gemm_pingpong.hip, whose outputs have the same bits).
+// accumulation on the matrix cores (v_mfma_f32_32x32x16_bf16). Two of its products give the bits of one of
+// v_mfma_f32_16x16x32_bf16, which gemm_pingpong.hip uses, so both kernels give the same outputs. That form saves power
+// where the whole chip multiplies, but reads twice the fragments out of LDS, which is what binds here: with it 400 rows of 9,728
+// x 2,560 took 55.6 us instead of 51.3, 193 rows of the gated 2,560 x 9,728 52.7 instead of 49.3, 300 rows of 12,288 x 4,096
+// 68.0 instead of 63.6, and whole prompts of 129 rows of the 4B shape 5.64 ms instead of 5.52.
 //
 // Two tile shapes. The small one: 4 waves in a 2 x 2 arrangement over a 128 x 128 output tile, each wave owning
-// 64 x 64 outputs; two such workgroups share a compute unit. The large one, for products
+// 64 x 64 = four 32 x 32 accumulators; two such workgroups share a compute unit. The large one, for products
 // with many tiles: 8 waves in a 2 x 4 arrangement over 256 x 256, each wave owning 128 x 64 (fewer LDS bytes per
 // multiply). K advances in steps of 64 through two LDS buffers: while the waves multiply out of
 // one, the 16-byte global loads of the next step are already in registers and are stored into the other.
@@ -23,7 +27,6 @@
 #define TPCS (TBK / 8)  // 16-byte pieces per tile row
 #define TLD (TBK + 8)   // LDS row stride in elements
 
-// WGM x WGN waves, each with 32 FM x 32 FN outputs (FN = 2 for the gated epilogue: gate and up)
 // What the per-head form (HEADS) takes beside the operands: head h = blockIdx.z multiplies the rows at A + h * a_stride with
 // its own weights (W [heads][N][K]) and writes bf16 at out + h * o_stride, times sigmoid(gate[row][h * N + column]) where a
 // gate is given.
@@ -33,6 +36,7 @@ struct HeadsArgs {
   int ld_gate;
 };
 
+// WGM x WGN waves, each with FM x FN accumulators of 32 x 32 (FN = 2 for the gated epilogue: gate and up)
 template <bool GATED, int WGM, int WGN, int FM, int FN, bool DEEP, bool HEADS = false>
 __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
@@ -97,12 +101,13 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
   const int nk_per = HEADS ? nk_all : (nk_all + gridDim.z - 1) / gridDim.z;
   const int kt0 = HEADS ? 0 : blockIdx.z * nk_per;
   const int nk = max(0, min(nk_all, kt0 + nk_per) - kt0);
-  constexpr int RM = 2 * FM, CN = 2 * FN;  // a wave's blocks of 16 rows and of 16 columns
-  floatx4 acc[RM][CN];
+  floatx16 acc[FM][FN];
 #pragma unroll
-  for (int i = 0; i < RM; ++i)
+  for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < CN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 #pragma unroll
   for (int j = 0; j < PA; ++j) aptr[j] += (size_t)kt0 * TBK;
 #pragma unroll
@@ -122,39 +127,38 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
 #pragma unroll
     for (int j = 0; j < PB; ++j) *(u32x4*)(Bs + (size_t)buf * TBN * TLD + (size_t)(lrow + TRSTEP * j) * TLD + lpc * 8) = r.b[j];
   };
-  const int fr = lane & 15;        // fragment row / column
-  const int fk = (lane >> 4) * 8;  // fragment k offset
+  const int fr = lane & 31;        // fragment row / column
+  const int fk = (lane >> 5) * 8;  // fragment k offset
   auto multiply = [&](int cur) {
-    const bf16_t* Ac = As + (size_t)cur * TBM * TLD + (size_t)(wm * RM * 16 + fr) * TLD + fk;
-    const bf16_t* Bc = Bs + (size_t)cur * TBN * TLD + (size_t)(wn * CN * 16 + fr) * TLD + fk;
+    const bf16_t* Ac = As + (size_t)cur * TBM * TLD + (size_t)(wm * FM * 32 + fr) * TLD + fk;
+    const bf16_t* Bc = Bs + (size_t)cur * TBN * TLD + (size_t)(wn * FN * 32 + fr) * TLD + fk;
     // the weight fragment goes in as the first operand: the accumulator then holds the tile transposed (rows =
     // output columns), so a lane owns four consecutive output columns of one row and stores them at once
-    constexpr int KS = FM > 2 ? 1 : TBK / 32;  // k32 steps whose fragments are in registers together
+    constexpr int KS = DEEP ? 2 : TBK / 16;  // k16 steps whose fragments are in registers together
 #pragma unroll
-    for (int k0 = 0; k0 < TBK / 32; k0 += KS) {
-      u32x4 af[KS][RM], bf[KS][CN];
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-        for (int j = 0; j < CN; ++j) bf[ks][j] = *(const u32x4*)(Bc + j * 16 * TLD + (k0 + ks) * 32);
-#pragma unroll
-        for (int i = 0; i < RM; ++i) af[ks][i] = *(const u32x4*)(Ac + i * 16 * TLD + (k0 + ks) * 32);
-      }
+    for (int k0 = 0; k0 < TBK / 16; k0 += KS) {
+      u32x4 af[KS][FM], bf[KS][FN];
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
-        for (int i = 0; i < RM; ++i)
+        for (int i = 0; i < FM; ++i) af[ks][i] = *(const u32x4*)(Ac + i * 32 * TLD + (k0 + ks) * 16);
 #pragma unroll
-          for (int j = 0; j < CN; ++j) acc[i][j] = mfma16(bf[ks][j], af[ks][i], acc[i][j]);
+        for (int j = 0; j < FN; ++j) bf[ks][j] = *(const u32x4*)(Bc + j * 32 * TLD + (k0 + ks) * 16);
       }
-      // the order of issue: what the first two rows of multiplies need, then a read behind every two multiplies
-      __builtin_amdgcn_sched_group_barrier(0x100, CN + 2, 0);
 #pragma unroll
-      for (int r = CN + 2; r < KS * (RM + CN); ++r) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[i][j] = mfma32(bf[ks][j], af[ks][i], acc[i][j]);
       }
-      __builtin_amdgcn_sched_group_barrier(0x008, KS * RM * CN - 2 * (KS * (RM + CN) - CN - 2), 0);
+      // the order of issue: the LDS reads of step ks + 1 go out before the multiplies of step ks
+      __builtin_amdgcn_sched_group_barrier(0x100, FM + FN, 0);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        if (ks + 1 < KS) __builtin_amdgcn_sched_group_barrier(0x100, FM + FN, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, FM * FN, 0);
+      }
     }
   };
   if (nk > 0) {
@@ -196,17 +200,25 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
       }
     }
   }
+  constexpr int CN = 4 * FN;  // a lane's runs of four columns per row block
+  floatx4 runs[FM][CN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < CN; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) runs[i][j][c] = acc[i][j / 4][4 * (j % 4) + c];
   if (HEADS) {
     bf16_t* o = (bf16_t*)out + (size_t)blockIdx.z * ha.o_stride;
 #pragma unroll
-    for (int i = 0; i < RM; ++i) {
-      const int m = m0 + (wm * RM + i) * 16 + (lane & 15);
+    for (int i = 0; i < FM; ++i) {
+      const int m = m0 + (wm * FM + i) * 32 + (lane & 31);
       if (m >= M) continue;
 #pragma unroll
       for (int j = 0; j < CN; ++j) {
-        const int n = n0 + (wn * CN + j) * 16 + (lane >> 4) * 4;
+        const int n = n0 + (wn * CN + j) * 8 + (lane >> 5) * 4;
         if (n >= N) continue;  // N is a multiple of four
-        floatx4 v = acc[i][j];
+        floatx4 v = runs[i][j];
         if (ha.gate) {
           const u32x2 g = *(const u32x2*)(ha.gate + (size_t)m * ha.ld_gate + (size_t)blockIdx.z * N + n);
           const float gv[4] = {__uint_as_float(g[0] << 16), __uint_as_float(g[0] & 0xffff0000u), __uint_as_float(g[1] << 16),
@@ -219,8 +231,8 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
     }
     return;
   }
-  tile_epilogue<GATED, RM, CN, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
-                                         (int)blockIdx.z, (int)gridDim.z);
+  tile_epilogue<GATED, 32, FM, CN, TBM, TBN>(runs, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
+                                             (int)blockIdx.z, (int)gridDim.z);
 }
 
 // sums the K-split partials in ascending order of the split and applies bias and epilogue; V outputs per thread

@@ -225,7 +225,7 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   }
-  tile_epilogue<GATED, RM, CN, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
+  tile_epilogue<GATED, 16, RM, CN, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
                                          (int)blockIdx.z, (int)gridDim.z);
 }
 

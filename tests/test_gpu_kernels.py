@@ -191,6 +191,27 @@ def test_gemm_two_group_kernel_with_tiles_of_192_rows(ops, monkeypatch, M, N, K,
     assert bool(((got[1].double() - ref).abs() <= K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 520, 128), (130, 516, 192), (256, 1024, 256), (385, 131, 576)])
+def test_the_small_tile_gives_the_bits_of_the_two_group_kernel(ops, monkeypatch, M, N, K):
+    """The small tile's accumulators lie otherwise over the lanes (32 x 32) than the two-group kernel's (16 x 16): every
+    epilogue at whole tiles, at edges and at rows that cannot be stored eight at a time, bit for bit."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M + N)
+    a = torch.randn(M, K, device=DEV, generator=gen).bfloat16()
+    w, w2 = ((torch.randn(N, K, device=DEV, generator=gen) * K ** -0.5).bfloat16() for _ in range(2))
+    bias = torch.randn(N, device=DEV, generator=gen)
+    got = []
+    for rows, kernel in ((256, "jllm_gemm_pingpong_bf16"), (0, "jllm_gemm_mfma_bf16")):
+        monkeypatch.setattr(ops, "_tiled_plan", lambda m, n, k, gated, rows=rows: (rows, 1))
+        monkeypatch.setattr(ops, "_k_splits", lambda m, n, k, gated: 1)
+        ops.reset_stats()
+        res = torch.ones(M, N, device=DEV)
+        ops.gemm(a, w, bias=bias, out=res, epilogue=ops.EPI_ADD)
+        got.append([res, ops.gemm(a, w, out_dtype=torch.float32), ops.gemm(a, w, bias=bias), ops.gemm(a, w, w2=w2, epilogue=ops.EPI_GATED)])
+        assert ops.stats()["ran"] == {kernel: 4}
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+
+
 @pytest.mark.parametrize("M,N,K,N2", [(1, 128, 256, 48), (5, 4096, 384, 4112), (8, 640, 4096, 304), (16, 304, 128, 16), (13, 5120, 1024, 640),
                                       (40, 1024, 1024, 512), (64, 2048, 2048, 768), (17, 1024, 4096, 256),
                                       # few rows, N / 16 just above the compute units: 20 weight rows per workgroup
