@@ -268,7 +268,7 @@ def test_attention_kernel_on_crafted_keys(dtype, maps, softcap):
             assert torch.allclose(merged_late, merged_first, atol=1e-5, rtol=1e-5)
 
 
-@pytest.mark.parametrize("dv,splits,maps", [(256, 9, 2), (128, 3, 2), (70, 12, 1), (200, 64, 2), (5, 2, 1)])
+@pytest.mark.parametrize("dv,splits,maps", [(256, 9, 2), (128, 3, 2), (70, 12, 1), (200, 64, 2), (5, 2, 1), (64, 4, 1), (96, 2, 2)])
 def test_heads_norm_has_the_same_bits_over_key_ranges(dv, splits, maps):
     """The kernel that merges key ranges and finishes the heads against the one for merged heads, bit for bit: the first
     without a norm leaves the heads that the second then norms."""
