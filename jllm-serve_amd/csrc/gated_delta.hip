@@ -147,8 +147,11 @@ extern "C" int jllm_short_conv(const void* x, int ldx, void* y, int ldy, int dty
   if (channels <= 0 || taps < 1 || taps > CONV_MAX_TAPS) JLLM_FAIL("short_conv: %d channels, %d taps (1..%d taps are taken)", channels, taps, CONV_MAX_TAPS);
   if (ldx < channels || ldy < channels || n_requests <= 0 || n_requests > n_rows) JLLM_FAIL("short_conv: rows %d/%d of %d channels, %d requests in %d rows", ldx, ldy, channels, n_requests, n_rows);
   const int cb = (channels + 255) / 256;
-  // eight rows by eight channels per thread where the rows are many and start on 16 bytes
-  const bool rows_form = dtype == JLLM_BF16 && taps == 4 && n_rows >= 64 && (channels & 7) == 0 && (ldx & 7) == 0 && (ldy & 7) == 0 &&
+  // Eight rows by eight channels per thread where the rows start on 16 bytes and there are enough of them: a thread then is a
+  // chain of about 14 us, however few there are, and the kernel of a thread per output is faster below some 2.3 million
+  // outputs (4,096 channels: 64 rows 6.6 / 14.7 us, 400 13.2 / 15.5, 600 16.9 / 16.1, 1,000 32 / 17; 8,192: 200 13.1 / 15.5, 300 17.3 /
+  // 16.0; 1,032: 1,000 11.1 / 15.3, 4,000 34 / 18)
+  const bool rows_form = dtype == JLLM_BF16 && taps == 4 && (long)n_rows * channels >= 2300000 && (channels & 7) == 0 && (ldx & 7) == 0 && (ldy & 7) == 0 &&
                          (((uintptr_t)x | (uintptr_t)y) & 15) == 0;
   JLLM_DISPATCH_1(dtype, T, {
     JLLM_DISPATCH_1(w_dtype, TW, {

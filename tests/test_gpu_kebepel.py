@@ -63,21 +63,22 @@ def act_type(dtype):
 # ------------------------------------------------------------------------------------------------ mechanisms alone
 
 
-@pytest.mark.parametrize("channels,biased", [(8, False), (520, True), (2056, False)])
-def test_convolution_of_many_rows(channels, biased):
-    """The convolution's kernel for many bf16 rows (eight rows and eight channels per thread): requests of one to seventy rows
-    that begin and end anywhere in a group of eight, channels that do not fill a workgroup, inputs from the states in front
-    of a request's first rows; against float64, rounded once, and the states that it leaves."""
+@pytest.mark.parametrize("channels,biased,times", [(104, False, 140), (520, True, 28), (2056, False, 8), (8, False, 1), (2056, True, 1)])
+def test_convolution_of_many_rows(channels, biased, times):
+    """The convolution's kernel for many bf16 rows (eight rows and eight channels per thread, from 2.3 million outputs on) and
+    the one for fewer: requests of one to seventy rows that begin and end anywhere in a group of eight, channels that do not
+    fill a workgroup, inputs from the states in front of a request's first rows; against float64, rounded once, and the
+    states that it leaves."""
     from jllm_serve_amd.kernels import ops
     gen = torch.Generator(device="cuda")
     gen.manual_seed(channels)
-    rows = [1, 2, 3, 70, 5, 1, 64, 13]
+    rows = [1, 2, 3, 70, 5, 1, 64, 13] * times
     n = sum(rows)
     x = torch.randn(n, channels + 8, device="cuda", generator=gen).bfloat16()[:, :channels]
     taps = torch.randn(channels, 4, device="cuda", generator=gen).bfloat16()
     bias = torch.randn(channels, device="cuda", generator=gen).bfloat16() if biased else None
     state = torch.randn(len(rows) + 2, 3, channels, device="cuda", generator=gen)
-    slots = torch.tensor([4, 1, 0, 7, 2, 9, 5, 3], dtype=torch.int32, device="cuda")
+    slots = torch.randperm(len(rows) + 2, device="cuda", generator=gen)[:len(rows)].to(torch.int32)
     row_req = torch.tensor([r for r, k in enumerate(rows) for _ in range(k)], dtype=torch.int32, device="cuda")
     before = state.clone()
     y = ops.short_conv(x, taps, state, row_req, slots, len(rows), bias=bias)
