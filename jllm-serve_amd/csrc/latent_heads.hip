@@ -136,10 +136,20 @@ extern "C" int jllm_latent_heads_bf16(const void* in, int ld_in, int in_hstride,
   latent_heads_mfma_kernel<RB, AHEAD><<<grid, LHM_WAVES * 64, 0, stream>>>(                                                      \
       (const bf16_t*)in, ld_in, in_hstride, (const bf16_t*)W, (bf16_t*)out, ld_out, out_hstride, M, N, K, mode, mode == 0 ? tail : 0, \
       rot_dims, positions, cos_t, sin_t, (const bf16_t*)gate, ld_gate, n_blocks)
-  if (!few && !tiled)
-    LHM_LAUNCH(4, 4);
-  else if (K <= 128 || tiled)  // (steps beyond K are multiplied as zeros: no branch stands between a load and the next one)
+  // steps beyond K are read again from the row's start and multiplied as zeros (no branch stands between a load and the next
+  // one), so the steps requested together are such that few are beyond it
+  const int steps = (K + 31) / 32;
+  if (!few && !tiled) {
+    if (steps % 4 == 1 || steps % 4 == 2)
+      LHM_LAUNCH(4, 2);
+    else
+      LHM_LAUNCH(4, 4);
+  } else if (steps <= 4 || tiled)
     LHM_LAUNCH(1, 4);
+  else if (steps <= 6)
+    LHM_LAUNCH(1, 6);
+  else if (steps <= 8)
+    LHM_LAUNCH(1, 8);
   else
     LHM_LAUNCH(1, 16);
 #undef LHM_LAUNCH

@@ -159,7 +159,7 @@ def _attend_plain(qa, rows, R, window, scale, sink, q_pos):
 
 
 @pytest.mark.parametrize("N,K,tail,gated", [(512, 128, 64, False), (128, 512, 0, True), (36, 64, 24, False), (132, 192, 0, True),
-                                            (20, 40, 8, False)])
+                                            (20, 40, 8, False), (100, 256, 0, True), (68, 320, 16, False)])
 def test_heads_products_at_every_row_count(N, K, tail, gated):
     """The per-head products where their kernel changes (up to 16 rows, up to 64 or 96, tiles of 128 rows beyond) and at odd
     sizes: against float64, and a row's bits are those it has in any other batch."""
