@@ -4,8 +4,8 @@
 // gemm_mfma.hip, which shares its operands through LDS.)
 //
 // What counts is how many bytes are on their way. A workgroup owns 32 weight rows of a tile's expert (16 outputs of the
-// gated product: gate and up) and cuts K among its eight waves, 256 k each in turn (four waves where K is no longer than
-// theirs), so for K = 2,048 all of its weights are requested at once. The sums (MFMA 16x16x32, weight rows as the first
+// gated product: gate and up) and cuts K among its eight waves, 256 k each in turn (four waves or two where K is no
+// longer than theirs), so for K = 2,048 all of its weights are requested at once. The sums (MFMA 16x16x32, weight rows as the first
 // operand, the tile's activation rows, gathered by the tile's row list, as the second) go from wave to wave through LDS:
 // one accumulator per output takes its k in ascending order, as in the grouped form, so that a row's outputs have the same
 // bits however many rows its experts get. Gate/up of 14 experts of 1,024 x 2,048 25 us, down 13; with a wave per 64
@@ -136,18 +136,19 @@ extern "C" int jllm_moe_gemm_bf16(const void* A, int a_dtype, int lda, const voi
 #define MM_LAUNCH(GATED, WAVES)                                                                                             \
   moe_gemm_mfma_kernel<GATED, WAVES><<<grid, WAVES * 64, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, out, \
                                                                       out_dtype, ldo, N, K, sorted, tiles, top, in_map, out_map, weight, gs)
-  const bool four = K <= 4 * MM_STEPS * 32;  // more waves would have no k
-  if (W2) {
-    if (four)
-      MM_LAUNCH(true, 4);
-    else
-      MM_LAUNCH(true, 8);
+#define MM_WAVES_OF(GATED)           \
+  if (K <= 2 * MM_STEPS * 32)        \
+    MM_LAUNCH(GATED, 2);             \
+  else if (K <= 4 * MM_STEPS * 32)   \
+    MM_LAUNCH(GATED, 4);             \
+  else                               \
+    MM_LAUNCH(GATED, 8);
+  if (W2) {  // (no more waves than have k)
+    MM_WAVES_OF(true)
   } else {
-    if (four)
-      MM_LAUNCH(false, 4);
-    else
-      MM_LAUNCH(false, 8);
+    MM_WAVES_OF(false)
   }
+#undef MM_WAVES_OF
 #undef MM_LAUNCH
   JLLM_CHECK_LAUNCH("moe_gemm_bf16");
   return 0;
