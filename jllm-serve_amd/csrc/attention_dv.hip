@@ -496,8 +496,8 @@ extern "C" int jllm_heads_finish(const void* att, int lda, int att_dtype, int n_
 //
 // A thread owns one dim, a workgroup as many waves as the dims need. MAPS and AT (ranges whose values are requested
 // together: no fewer than there are, up to eight) are what a call has, so that a step of many rows and few ranges asks for
-// nothing twice: 200 rows of 32 heads of 128 in two ranges 7.2 us, with eight
-// ranges of two maps and four waves always 13.4 (a wave per head 7.2; one row of 16 heads of 256 in nine ranges 4.7, so 16.2).
+// nothing twice. One row of 16 heads of 256 (two maps) in nine ranges 4.7 us, 200 rows of 32 heads of 128 in two ranges 7.2;
+// with a wave per head that loads a range at a time 16.2 and 7.2, with four waves, eight ranges and two maps always 4.7 and 13.4.
 template <typename TG, typename TW, typename TO, int MAPS, int AT>
 __global__ __launch_bounds__(256) void heads_finish_split_kernel(const float* __restrict__ partial, int splits,
                                                                  int dv, float lambda, int normed, float eps, float norm_mul,

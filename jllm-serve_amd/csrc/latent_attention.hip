@@ -628,7 +628,12 @@ extern "C" int jllm_latent_attention_bf16(const void* qa, int ldq, void* out, in
   dim3 grid(n_tiles, n_hb * (split < 0 ? n_rg : 1), split > 0 ? n_z : 1);
   int rc;
   if (split < 0)
-    rc = R <= 128 && dkp <= 256
+    // The smallest instance that holds the sizes; what it pads is multiplied as zeros. 2,048 rows, against the kernel for
+    // single rows, which took these runs too: 4 heads of 64 + 32 entries 90 -> 60 us (padded to 256 entries 67), 8 of 128 + 64
+    // 123 -> 70, 3 of 144 + 24 (padded to 512 + 64) 173 -> 101, 16 of 256 + 64 364 -> 189.
+    rc = R <= 128 && dkp <= 128
+             ? lm_launch_rows<1, 4>(grid, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, n_hb)
+         : R <= 128 && dkp <= 256
              ? lm_launch_rows<1, 8>(grid, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, n_hb)
              : lm_launch_rows<4, 18>(grid, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, n_hb);
   else if (R <= 64 && dkp <= 128)

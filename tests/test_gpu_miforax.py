@@ -326,7 +326,8 @@ def test_attention_kernels_on_crafted_keys(dtype, fast, H, R, Dr, page):
             assert (no_sink - want).abs().max() > 0.3
 
 
-@pytest.mark.parametrize("H, R, Dk, window", [(16, 512, 576, 0), (16, 512, 576, 130), (3, 144, 168, 70), (40, 496, 520, 0), (7, 128, 256, 64)])
+@pytest.mark.parametrize("H, R, Dk, window", [(16, 512, 576, 0), (16, 512, 576, 130), (3, 144, 168, 70), (40, 496, 520, 0), (7, 128, 256, 64), (6, 80, 104, 50),
+                                              (2, 128, 128, 0)])
 def test_latent_attention_of_runs_of_rows(H, R, Dk, window):
     """Portions of prompts in runs of 1 to 16 rows that begin at any position (keys end one below, at and one beyond a
     block of 64; a single row beside them), rows whose entries are no multiple of 32 or 64, latents whose last waves have no
@@ -370,7 +371,7 @@ def test_latent_attention_of_runs_of_rows(H, R, Dk, window):
 
 
 @pytest.mark.parametrize("H, R, Dk, window, single_runs", [(40, 512, 576, 0, False), (40, 144, 168, 90, False), (17, 128, 256, 33, False),
-                                                           (16, 512, 576, 0, True), (16, 512, 576, 70, True), (3, 96, 128, 0, True)])
+                                                           (16, 512, 576, 0, True), (16, 512, 576, 70, True), (3, 96, 128, 0, True), (20, 64, 96, 0, False)])
 def test_latent_attention_gives_a_row_the_same_bits_in_runs_and_alone(H, R, Dk, window, single_runs):
     """A row's result as a single row of its step and in a run of a portion, bit for bit: with more than 16 heads in runs of up
     to 16 rows; with up to 16, where a row alone keeps four sums, in runs of one row. Keys grow along the context, so that
