@@ -136,12 +136,13 @@ def test_gemm_large_tile(ops):
 @pytest.mark.parametrize("M,N,K,plan", [(1500, 8200, 160, (256, 1)), (2048, 6144, 1024, (256, 1)), (300, 25000, 128, (256, 1)),
                                         (520, 16400, 4096, (256, 1)), (2000, 4096, 8192, (256, 2)), (1024, 6140, 8256, (256, 2)),
                                         (1000, 4100, 8192, (256, 2)), (640, 4100, 8192, (256, 4)), (1024, 6144, 4096, (256, 2))])
-def test_gemm_two_group_kernel(ops, M, N, K, plan):
-    """The tiled kernel whose waves take turns at the matrix cores (direct-to-LDS loads, a ring of stages): every
-    epilogue, with a bias, partial tiles in both directions, K from four stages to many, inputs and
+def test_gemm_two_group_kernel(ops, monkeypatch, M, N, K, plan):
+    """The tiled kernel whose waves take turns at the matrix cores (direct-to-LDS loads, a ring of stages) with its tile of 256
+    rows, whatever the choice between tiles makes of these sizes: every epilogue, with a bias, partial tiles in both directions, K from four stages to many, inputs and
     outputs whose rows are not contiguous, K cut in two or four with partial sums (also an odd number of stages per half);
     against float64."""
     assert ops._pingpong_plan(M, N, K, False) == plan
+    monkeypatch.setattr(ops, "_tiled_plan", lambda m, n, k, gated: (256, 1) if gated else plan)
     torch.manual_seed(M + N + K)
     a = torch.randn(M, K, device=DEV).bfloat16()
     w = (torch.randn(N, K, device=DEV) / math.sqrt(K)).bfloat16()
@@ -319,8 +320,9 @@ def test_gemm_rows_do_not_depend_on_the_batch(ops):
 @pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16])
 def test_float32_products_are_one_chain_of_multiply_adds(ops, M, N, K, wdt):
     """Every tile of the 32-bit products, at its edges: an output has the bits of one fp32 accumulator that takes its
-    multiply-adds in ascending k. Operands of 12 (8) bits: a product and an accumulator then add without rounding in
-    float64 (2^-44 .. 2^6), so the chain is restated there with one rounding to fp32 per step, exactly. The gated form
+    terms in ascending k. Operands of 12 (8) bits: a product and an accumulator then add without rounding in
+    float64 (2^-44 .. 2^6), so the chain is restated there with one rounding to fp32 per step, exactly. (Products of so few
+    bits are exact in fp32: that they are not rounded by themselves is the next test's.) The gated form
     gives, in any batch, the bits it gives its rows in batches of 16."""
     assert [ops.library().jllm_f32_tile(m, n, 0) for m, n in ((33, 1030), (700, 1100), (2041, 4090))] == [2, 1, 0]
     gen = torch.Generator(device=DEV)
@@ -338,6 +340,27 @@ def test_float32_products_are_one_chain_of_multiply_adds(ops, M, N, K, wdt):
     for at in range(0, M, max(16, M // 4)):
         few = ops.gemm(a[at:at + 16].contiguous(), w.to(wdt), w2=w2.to(wdt), epilogue=ops.EPI_GATED, exact=True)
         assert torch.equal(few, gated[at:at + 16])
+
+
+@pytest.mark.parametrize("M,N,K,exponent", [(3, 17, 67, 0), (16, 20, 200, -70), (20, 33, 70, 0), (40, 35, 68, -71), (130, 40, 36, -70)])
+def test_float32_products_round_once_per_multiply_add(ops, M, N, K, exponent):
+    """The 32-bit products on operands of 24 bits, whose products a multiply-add must not round, against the C library's
+    fmaf in ascending k, bit for bit; with magnitudes around 2^-70 products and sums are denormal."""
+    import ctypes
+    libm = ctypes.CDLL("libm.so.6")
+    libm.fmaf.restype, libm.fmaf.argtypes = ctypes.c_float, [ctypes.c_float] * 3
+    g = torch.Generator().manual_seed(M + N)
+    a, w = (torch.randn(n, K, generator=g) * 2.0 ** exponent for n in (M, N))
+    want = torch.zeros(M, N)
+    for m, row in enumerate(a.tolist()):
+        for n, col in enumerate(w.tolist()):
+            x = 0.0
+            for p, q in zip(row, col):
+                x = libm.fmaf(p, q, x)
+            want[m, n] = x
+    if exponent:
+        assert bool(((want != 0) & (want.abs() < 2.0 ** -126)).any())
+    assert torch.equal(ops.gemm(a.to(DEV), w.to(DEV), exact=True).cpu(), want)
 
 
 def test_gemm_refuses_bad_arguments(ops):

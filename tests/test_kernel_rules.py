@@ -92,6 +92,35 @@ def test_plan_of_the_two_group_kernel():
     assert ops._pingpong_plan(2048, 8192, 1024 + 32, False)[1] == 1, "a cut needs K % 64 == 0 and long ranges"
 
 
+def test_plan_of_the_tiled_products():
+    """The plan that the dispatch asks for: a tile that a kernel has (192 or 256 rows, or none), K cut only where every
+    workgroup keeps a long range of whole stages and never for the gated product, few rows and shapes that the two-group
+    kernel cannot take with the small tile, whose cuts are the small tile's own, tiles of 192 rows with K cut only where they
+    leave fewer empty rows than 256; for the models' products and for odd sizes."""
+    shapes = [s for group in SHAPES.values() for s in group]
+    shapes += [(n, k, gated) for n in (8, 100, 131, 1000, 4100, 25000) for k in (32, 64, 96, 128, 160, 192, 1056, 4096, 8256, 17408)
+               for gated in (False, True)]
+    taken = set()
+    for n, k, gated in shapes:
+        for rows in (65, 90, 128, 129, 192, 193, 256, 257, 300, 385, 577, 700, 1000, 1025, 1536, 2049, 3333, 4614, 8192, 16384):
+            tile, cut = ops._tiled_plan(rows, n, k, gated)
+            where = (rows, n, k, gated, tile, cut)
+            assert tile in (0, 192, 256), where
+            assert not gated or cut == 1, where
+            if tile == 0:
+                assert cut == (ops._k_splits(rows, n, k, gated) if k % 64 == 0 else 1), where
+                continue
+            assert k % 32 == 0 and k >= 128 and cut in (1, 2, 4) and (gated or rows >= ops.PINGPONG_MIN_ROWS), where
+            if cut > 1:
+                assert k % 64 == 0 and (k // 32) % cut == 0 and k // cut >= ops.PINGPONG_SPLIT_MIN_K, where
+            if tile == 192:
+                assert k % 64 == 0 and (cut == 1 or -(-rows // 192) * 192 < -(-rows // 256) * 256), where
+            else:
+                assert (tile, cut) == ops._pingpong_plan(rows, n, k, gated), where
+            taken.add((tile, cut))
+    assert {(192, 1), (192, 2), (192, 4), (256, 1), (256, 2), (256, 4)} <= taken, taken
+
+
 def test_the_attention_plan_says_whether_the_runs_of_a_step_differ_much_in_keys():
     """One prompt from its start has runs of 128 to 2,048 keys (the portion kernel then cuts every run's keys over two
     groups of waves); a portion deep inside a long request, or several of them, has runs of about the same length."""
