@@ -605,6 +605,7 @@ SMALL_ROUND_US = 1.2                  # what a round of workgroups costs beside 
 LARGE_STEP_US = {256: (0.576, 0.808), 192: (0.45, 0.687)}  # 32 of K on tiles of 256 or 192 rows by 256 columns: lone, full
 LARGE_ROUND_US = 2.33
 CUT_US = (2.2, 1.255e-6)              # a cut of K: the reduction's launch, and per element of a partial result
+GATED_192_AT_MOST = 0.97              # of the other choice's estimate, for the gated product
 
 
 def _small_us(M: int, N: int, K: int, gated: bool, splits: int) -> float:
@@ -643,19 +644,34 @@ def _tiled_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int]:
     192 rows moves a sixth more bytes per multiply, but its rounds and its empty rows fall differently.
 
     The constants were fitted to the times, inside a graph, of every choice for 252 products (ten row counts from 100 to
-    4,614 on the products of six shapes). Inside whole prompt passes, which run hotter: 900 rows of the 8B shape 17.3 -> 16.5
-    ms, 3,000 of the 4B shape 27.6 -> 27.0, prompts of 7,777 rows of the 14B shape 129.7 -> 127.6, 1,100 of the 1.7B shape
-    6.51 -> 6.48. Not taken: cuts of K where 192 leaves no fewer empty rows than 256 (631 rows of the 8B shape: the o and
+    4,614 on the products of six shapes). On 216 products at nine other row counts (150 to 3,500) the choice is 0.2 % behind
+    the best on average, within 5 % in 213 and 14 % behind at worst (14B gate/up at 350 rows); without tiles of 192 rows 4.2 %
+    on average, within 5 % in 155. Inside whole prompt passes, which run hotter: 900 rows of the 8B shape 17.3 -> 16.5 ms,
+    1,300 23.8 -> 22.1, 3,000 of the 4B shape 27.6 -> 27.0, prompts of 4,614 rows of the 14B shape 131.5 -> 125.6. Not
+    taken: cuts of K where 192 leaves no fewer empty rows than 256 (631 rows of the 8B shape: the o and
     down products 6 % faster alone, the pass 1 % slower: what binds there is the chip's power), and the small tile's count
-    of cuts by the same estimate (up to a third faster alone, nothing or 1 % slower inside a pass)."""
+    of cuts by the same estimate (up to a third faster alone, nothing or 1 % slower inside a pass).
+
+    Two places where whole passes disagree with the estimate, so that 256 rows stay. A near tie of the gated product, over many
+    rounds: 1,800 rows of the 32B shape 138.4 ms with tiles of 192 rows there, 132.3 with 256, 2,850 of the 14B shape 82.3 /
+    80.3. And one round over a short K where the last tile of 256 rows is nearly empty (what it repeats costs it little) and
+    that of 192 is not: qkv at 1,300 rows of the 4B shape 14.76 / 14.53 ms, at 2,080 of the 0.6B 5.58 / 5.48, at 2,850 6.92 /
+    6.82; a step of 32 rows through all others up to 3,000 found 192 up to 8 % of the pass ahead, as they are at such row
+    counts too from K = 4,096 on (1,318 rows of the 8B shape 23.6 / 23.7)."""
     rows, cut = _pingpong_plan(M, N, K, gated)
     if K % 64 == 0:
         cut = cut if rows else _k_splits(M, N, K, gated)
         least = _large_us(M, N, K, gated, rows, cut) if rows else _small_us(M, N, K, gated, cut)
+        if gated:
+            least *= GATED_192_AT_MOST
         if K >= 128 and (gated or M >= PINGPONG_MIN_ROWS):
             fewer = -(-M // 192) * 192 < -(-M // 256) * 256
+            full = -(-M // 192) > -(-M // 256) and 0 < M % 256 <= 64 and (M % 192 == 0 or M % 192 > 96)
+            one_round = -(-N // (128 if gated else 256)) * -(-M // 192) <= compute_units()
             for c in (1, 2, 4):
                 if c > 1 and (gated or not fewer or (K // 32) % c or K // c < PINGPONG_SPLIT_MIN_K):
+                    continue
+                if c == 1 and rows and one_round and K < 4096 and full:
                     continue
                 t = _large_us(M, N, K, gated, 192, c)
                 if t < least:

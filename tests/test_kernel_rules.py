@@ -96,13 +96,16 @@ def test_plan_of_the_tiled_products():
     """The plan that the dispatch asks for: a tile that a kernel has (192 or 256 rows, or none), K cut only where every
     workgroup keeps a long range of whole stages and never for the gated product, few rows and shapes that the two-group
     kernel cannot take with the small tile, whose cuts are the small tile's own, tiles of 192 rows with K cut only where they
-    leave fewer empty rows than 256; for the models' products and for odd sizes."""
-    shapes = [s for group in SHAPES.values() for s in group]
+    leave fewer empty rows than 256, never for a near tie of the gated product, nor in one round over a short K where they
+    have no empty rows to save; for the models' products and for odd sizes."""
+    cus = ops.compute_units()
+    shapes = [s for group in SHAPES.values() for s in group] + [(4096, 1024, False), (3072, 1024, True), (6144, 2560, False)]
     shapes += [(n, k, gated) for n in (8, 100, 131, 1000, 4100, 25000) for k in (32, 64, 96, 128, 160, 192, 1056, 4096, 8256, 17408)
                for gated in (False, True)]
     taken = set()
     for n, k, gated in shapes:
-        for rows in (65, 90, 128, 129, 192, 193, 256, 257, 300, 385, 577, 700, 1000, 1025, 1536, 2049, 3333, 4614, 8192, 16384):
+        for rows in (65, 90, 128, 129, 192, 193, 256, 257, 300, 385, 577, 700, 1000, 1025, 1318, 1536, 1800, 2049,
+                     2096, 2850, 3333, 4614, 8192, 16384):
             tile, cut = ops._tiled_plan(rows, n, k, gated)
             where = (rows, n, k, gated, tile, cut)
             assert tile in (0, 192, 256), where
@@ -115,6 +118,11 @@ def test_plan_of_the_tiled_products():
                 assert k % 64 == 0 and (k // 32) % cut == 0 and k // cut >= ops.PINGPONG_SPLIT_MIN_K, where
             if tile == 192:
                 assert k % 64 == 0 and (cut == 1 or -(-rows // 192) * 192 < -(-rows // 256) * 256), where
+                t = lambda r: ops._large_us(rows, n, k, gated, r, 1)
+                assert not gated or ops._pingpong_plan(rows, n, k, gated)[0] == 0 or t(192) < 0.98 * t(256), where
+                tiles = -(-n // (128 if gated else 256)) * -(-rows // 192)
+                if rows in (1318, 2096, 2850) and k < 4096 and cut == 1:  # just above whole tiles of 256, just below of 192
+                    assert tiles > cus or ops._pingpong_plan(rows, n, k, gated)[0] == 0, where
             else:
                 assert (tile, cut) == ops._pingpong_plan(rows, n, k, gated), where
             taken.add((tile, cut))
