@@ -471,8 +471,10 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(G
 // A step of few rows is one chain of latencies: position and table, then q and the new key, then the first keys, then the
 // products. So position, request and slot are asked for together, the new key is another wave's work than q, and its
 // readers take it from LDS, so that nobody waits for its store. Whole steps, before and after: 300 keys of
-// the 0.6B shape 1,106 -> 1,089 us, one request of 2,048 keys (8B) 3,566 -> 3,535, 64 x 8B 6,536 -> 6,461.
-// The first keys straight through the table, before q is prepared, were slower (300 keys of the 0.6B shape 1,089 -> 1,104).
+// the 0.6B shape 1,106 -> 1,089 to 1,096 us, one request of 2,048 keys (8B) 3,562 -> 3,544; eight of 900 to 2,500 keys (8B, 20.1
+// / 20.4 us a layer), 64 of up to 1,000 and four of 6,100 to 8,000 (4B) as before, within what two runs of one side differ (0.7
+// to 1.6 %). The first keys straight through the table, before q is prepared, were slower (300 keys of the 0.6B shape 1,089
+// -> 1,104).
 template <int G, bool FUSED>
 __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, 3))) void decode_attention_mfma_kernel(
     const bf16_t* q, int ldq, const bf16_t* kc, const bf16_t* vc, const int* __restrict__ block_table, int max_blocks,

@@ -396,7 +396,8 @@ extern "C" int jllm_gemm_mfma_grouped_bf16(const void* A, int lda, const void* W
 
 // The per-head products of latent attention for many rows (latent_heads.hip, which checks the arguments): K a multiple of
 // 64, N of 4. Through LDS in tiles of 128 x 128 a row's and a weight's loads are shared by a workgroup; read straight
-// from memory by every wave (64 x 64 outputs each) 2,500 rows of 16 heads took 95 us at 512 x 128 and 47 at 128 x 512.
+// from memory by every wave (64 x 64 outputs each) 2,556 rows of 16 heads took 76 us at 512 x 128 with a rotated tail and 41
+// at 128 x 512 with a gate, here (the tail a launch of its own) 35 and 21.
 int jllm_gemm_mfma_heads(const void* in, int ld_in, int in_hstride, const void* W, void* out, int ld_out, int out_hstride, int M,
                          int H, int N, int K, const void* gate, int ld_gate, hipStream_t stream) {
   constexpr int TB = 128;

@@ -120,7 +120,7 @@ extern "C" int jllm_latent_heads_bf16(const void* in, int ld_in, int in_hstride,
   const bool few = M <= 16;
   // Tiles of 128 rows (the same bits: one accumulator per output, K in steps of 32); the rotated tail then is the only column
   // of workgroups of the kernel above, a launch of its own. 16 heads of 512 x 128 with a tail: 70 rows 11 us in one
-  // launch, 13 in two, 100 rows 14.1 / 13.8, 300 38 / 14, 2,556 76 / 34; of 128 x 512 without one: 70 rows 14.8 / 13.8,
+  // launch, 13 in two, 100 rows 14.1 / 13.8, 300 38 / 14, 2,556 76 / 35; of 128 x 512 without one: 70 rows 14.8 / 13.8,
   // 2,556 41 / 21.
   const bool tiled = M > (mode == 0 && tail > 0 ? 96 : 64) && (K & 63) == 0;
   if (tiled) {

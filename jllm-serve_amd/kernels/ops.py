@@ -1153,8 +1153,8 @@ LATENT_TILE_ROWS = 16  # rows of one request per run of the step's plan (parts/l
 
 
 def _fast_latent_attention(qa, out, cache, block_table, row_req, positions, heads, kv_rank, window, scale, sink, meta) -> bool:
-    """The bf16 matrix-core kernel, for portions and single rows alike; it needs the step's runs of rows (``meta``:
-    ``tiles_dev``, ``n_tiles``) and declines sizes it does not take."""
+    """The bf16 matrix-core kernels: one for runs of several rows, one for single rows (whose keys may be cut into ranges);
+    they need the step's runs of rows (``meta``: ``tiles_dev``, ``n_tiles``) and decline sizes that they do not take."""
     if qa.dtype != torch.bfloat16 or meta is None or meta.get("tiles_dev") is None:
         return False
     n_tiles = int(meta["n_tiles"])
