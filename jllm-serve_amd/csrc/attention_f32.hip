@@ -421,8 +421,14 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_tiles_kernel(A
 }
 
 // fp32, head size 128, 16-byte aligned rows; returns 1 for what it leaves to the general kernel. `n_requests` bounds
-// row_req. Which kernel: a tile holds 16 / G rows of one request, and reads their keys once; where the rows are spread
-// over as many requests (steps of single tokens) there is nothing to share and a workgroup per row has more waves.
+// row_req, the block table's width the keys. Which kernel: a tile holds 16 / G rows of one request, and reads their keys
+// once; where the rows are spread over as many requests (steps of single tokens) there is nothing to share and a workgroup
+// per row has more waves. A portion of few rows goes row by row too: a tile's chain is about 12 us for the first 64 keys, a
+// row's 5.5, as long as its workgroups (row x head) are one per compute unit, a few where the keys are few. 16 heads over
+// 8, rows / tiles (the general kernel): 4 rows of a new prompt 5.5 / 11.7 us (6.8), 20 rows 5.9 / 12.1 (10.2), 64 rows 8.4 /
+// 12.3, 96 rows 16.0 / 13.1; 20 rows behind 200 keys 13.2 / 15.1, 40 rows 17.6 / 15.3; 16 rows behind 1,000 keys 31.6 / 39.6,
+// 20 rows 46.7 / 41.6. Up to 16 keys the general kernel lies between: 64 rows of eight new prompts, 24 heads over 3, 9.8 us,
+// 11.8 by rows, 12.5 by tiles.
 extern "C" int jllm_attention_f32(const void* q, int ldq, void* out, int ldo, const void* kcache, const void* vcache, const int* block_table,
                                   int max_blocks, const int* row_req, const int* positions, int n_tokens, int n_requests, int H,
                                   int Hkv, int hd, int page_size, int window, float scale, hipStream_t stream) {
@@ -433,7 +439,13 @@ extern "C" int jllm_attention_f32(const void* q, int ldq, void* out, int ldo, co
   const AttF32 A = {(const float*)q, (float*)out, (const float*)kcache, (const float*)vcache, block_table, row_req, positions,
                     ldq, ldo, max_blocks, n_tokens, H, Hkv, page_size, window, scale};
   const int G = H / Hkv;
-  if (G <= 8 && n_tokens >= 4 * n_requests) {
+  int cus = jllm_compute_units();
+  if (cus <= 0) cus = 256;
+  const long keys = (long)max_blocks * page_size;  // no row sees more
+  const long pairs = (long)n_tokens * H;
+  const bool few = pairs <= (long)cus * (keys <= 64 ? 5 : keys <= 256 ? 2 : 1);
+  if (G <= 8 && n_tokens >= 4 * n_requests && !few) {
+    if (keys <= 16 && pairs <= 6L * cus) return 1;
     const int rows = 16 / G;
     const int tiles = (n_tokens + rows - 1) / rows;
     if (n_requests > 1)
@@ -441,11 +453,9 @@ extern "C" int jllm_attention_f32(const void* q, int ldq, void* out, int ldo, co
     else
       attention_f32_tiles_kernel<false><<<dim3(tiles, Hkv), 64 * AF_WAVES, 0, stream>>>(A, rows, 0);
   } else {  // heads share a workgroup where the step still has two workgroups for every compute unit, as in the general kernel
-    int cus = jllm_compute_units();
-    if (cus <= 0) cus = 256;
     if (G >= 3 && (long)n_tokens * Hkv * ((G + 3) / 4) >= 2L * cus)
       attention_f32_rows_kernel<4><<<dim3(n_tokens, Hkv * ((G + 3) / 4)), 64 * AF_WAVES, 0, stream>>>(A);
-    else if (G >= 2 && (long)n_tokens * Hkv * ((G + 1) / 2) >= 2L * cus)
+    else if (G >= 2 && (G <= 4 || keys > 64) && (long)n_tokens * Hkv * ((G + 1) / 2) >= 2L * cus)
       attention_f32_rows_kernel<2><<<dim3(n_tokens, Hkv * ((G + 1) / 2)), 64 * AF_WAVES, 0, stream>>>(A);
     else
       attention_f32_rows_kernel<1><<<dim3(n_tokens, H), 64 * AF_WAVES, 0, stream>>>(A);

@@ -611,7 +611,8 @@ def test_float32_attention_gives_the_general_kernels_bits(ops, H, Hkv, page, win
 
 @pytest.mark.parametrize("H,Hkv,n_req,n,shuffled", [(16, 8, 64, 64, False),  # two heads to a workgroup of a row
                                                     (12, 4, 70, 70, False),  # the same with three heads of a kv head
-                                                    (16, 8, 6, 25, False),   # single rows behind a portion, inside its last tile
+                                                    (16, 8, 6, 25, False),   # a portion of few rows, row by row
+                                                    (16, 8, 6, 41, False),   # single rows behind a portion, inside its last tile
                                                     (8, 8, 5, 300, True), (24, 3, 40, 1300, True)])  # requests in no order
 def test_float32_attention_of_rows_in_any_order_gives_the_general_kernels_bits(ops, H, Hkv, n_req, n, shuffled):
     """Head size 128 in fp32 where a tile's rows belong to several requests, whose rows may lie anywhere in the step, and
