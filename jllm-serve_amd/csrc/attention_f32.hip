@@ -187,7 +187,9 @@ __device__ __forceinline__ floatx4 mfma_f32(float a, float b, floatx4 c) { retur
 // inside tiles where its request's rows begin. A workgroup that walked all of its tile's requests in turn made the step
 // wait for it: 20 rows of a prompt and five single rows of up to 400 keys 71 us, here 24 (the general kernel: 41); 32 single rows of
 // 1,000 to 2,860 keys behind 2,000 rows of a prompt 1,050, here 355 (1,770); 64 requests of 32 rows, where there is nothing
-// to find, 52, here 58 (195).
+// to find, 52, here 58 (195), eight of 32 rows behind 500 keys 37, here 47 (152): the workgroups that find nothing stand in front
+// of tiles. (All of them in front of all tiles, or behind them where all are resident: these two 129 instead of 134 and 37, but
+// single rows behind portions 2 to 6 % slower.)
 template <bool SPREAD>
 __global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_tiles_kernel(AttF32 A, int rows, int spread) {
   __shared__ __align__(16) float mg[AF_WAVES][16][4 + AF_HD];  // every wave's maximum, sum (and two spare places), weighted sums
