@@ -233,8 +233,8 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
 // 0, which an infinite value would not survive: a result that is no finite number is computed again from its own keys.
 //
 // 16 heads, 512 + 64 entries, against the kernel above, which took these runs too and computed every score twice: prompts
-// of 300 to 1,211 rows (3,611 in all) 400 -> 186 us, 487 rows 73 -> 36, six of 20 rows and ten single rows of 1,500 to 1,950
-// keys 152 -> 98, 2,048 rows with a window of 512 165 -> 88. With scores in one chain and maxima moved 64 keys at a time,
+// of 300 to 1,211 rows (3,611 in all) 400 -> 186 us, 487 rows 73 -> 36, a portion of 30 rows and three single rows of 1,500 keys
+// 85 -> 73, 2,048 rows with a window of 512 165 -> 88. With scores in one chain and maxima moved 64 keys at a time,
 // in other bits, 168, 32, 78 and 78.
 template <int NJ, int DKS>  // NJ: 16-dim blocks of the latent per wave at most (8 NJ >= R / 16); DKS as above
 __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_rows_kernel(
@@ -320,7 +320,39 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_rows_kernel(
     const bf16_t* Kb = Ks + (size_t)cur * LM_KEYS * LD;
     if (blk < blk_last) fetch(blk + 1);
     float z[8];
-    if (qs < n_q) {
+    if (alone) {  // the waves of one half of the block have nothing to do, the others one 16 keys
+#pragma unroll
+      for (int i = 0; i < 8; ++i) z[i] = -INFINITY;
+      float mx = -INFINITY;
+      if (kh == qs >> 1) {
+        floatx4 sc[2];
+        sc[0] = sc[1] = floatx4{0.f, 0.f, 0.f, 0.f};
+        const bf16_t* krow = Kb + (qs * 16 + sub) * LD + 8 * q4;
+        u32x4 kf[LM_AHEAD + 1];
+#pragma unroll
+        for (int j = 0; j < DKS + LM_AHEAD; ++j) {
+          if (j < DKS) kf[j % (LM_AHEAD + 1)] = *(const u32x4*)(krow + 32 * j);
+          if (j >= LM_AHEAD) sc[(j - LM_AHEAD) & 1] = mfma16(kf[(j - LM_AHEAD) % (LM_AHEAD + 1)], qf[j - LM_AHEAD], sc[(j - LM_AHEAD) & 1]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        const floatx4 s = sc[0] + sc[1];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = c0 + qs * 16 + 4 * q4 + i;
+          const float x = (key >= my_first && key <= my_pos) ? s[i] * scale : -INFINITY;
+          if (qs & 1)
+            z[4 + i] = x;
+          else
+            z[i] = x;
+          mx = fmaxf(mx, x);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      }
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+        if (q4 == 0) mxs[(2 * kh + g) * 64 + v] = 2 * kh + g == qs ? mx : -INFINITY;
+    } else if (qs < n_q) {
       floatx4 sc[2][2];  // two chains for each of the wave's two 16 keys
 #pragma unroll
       for (int i = 0; i < 4; ++i) sc[i >> 1][i & 1] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -338,12 +370,11 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_rows_kernel(
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
         const floatx4 s = sc[g][0] + sc[g][1];
-        const bool mine = !alone || 2 * kh + g == qs;
         float mx = -INFINITY;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int key = c0 + kh * 32 + g * 16 + 4 * q4 + i;
-          z[4 * g + i] = (mine && key >= my_first && key <= my_pos) ? s[i] * scale : -INFINITY;
+          z[4 * g + i] = (key >= my_first && key <= my_pos) ? s[i] * scale : -INFINITY;
           mx = fmaxf(mx, z[4 * g + i]);
         }
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -630,7 +661,10 @@ extern "C" int jllm_latent_attention_bf16(const void* qa, int ldq, void* out, in
   if (split < 0)
     // The smallest instance that holds the sizes; what it pads is multiplied as zeros. 2,048 rows, against the kernel for
     // single rows, which took these runs too: 4 heads of 64 + 32 entries 90 -> 60 us (padded to 256 entries 67), 8 of 128 + 64
-    // 123 -> 70, 3 of 144 + 24 (padded to 512 + 64) 173 -> 101, 16 of 256 + 64 364 -> 189.
+    // 123 -> 70, 3 of 144 + 24 (padded to 512 + 64) 173 -> 101, 16 of 256 + 64 364 -> 189. What that kernel did faster are rows
+    // alone and a few rows of a new prompt where latents are short and heads few: 30 rows and three single rows of 1,500 keys with
+    // 4 heads of 64 + 32 30 -> 44, 3 of 144 + 24 61 -> 70, 8 of 256 + 64 69 -> 71, 16 of 512 + 64 85 -> 73; 20 rows 5.0 -> 6.1,
+    // 7.8 -> 8.7, 9.9 -> 10.3, 15.6 -> 13.8.
     rc = R <= 128 && dkp <= 128
              ? lm_launch_rows<1, 4>(grid, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, n_hb)
          : R <= 128 && dkp <= 256
