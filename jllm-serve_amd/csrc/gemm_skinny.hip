@@ -1,32 +1,51 @@
-// out[M,N] = A[M,K] * W[N,K]^T for few rows (decode steps): bf16 operands, fp32 accumulation on the matrix
-// cores, bound by streaming W from HBM once.
+// out[M,N] = A[M,K] * W[N,K]^T for up to 16 rows (decode steps): bf16 operands, fp32 accumulation on the matrix cores
+// (16x16x32), bound by streaming W from HBM once.
 //
-// One workgroup of 8 (or 4) waves owns 16 weight rows (16 outputs per activation row). The K dimension is cut in
-// blocks of 128; wave w takes blocks w, w+8, ...: per block each lane issues 4 loads of 16 bytes of its weight
-// row (lane l, load j: row l%16, k = block*128 + j*32 + (l/16)*8 .. +8), so every load instruction covers whole
-// 64-byte pieces of 16 rows (no sector is fetched for a quarter of its bytes) and a block is 16 rows x 256
-// contiguous bytes; each load feeds one MFMA (16x16x32) per 16 activation rows. The two operands use the same k assignment, which
-// is all a dot product needs. The 8 partial tiles are summed through LDS in wave order, so a result does not
-// depend on M or on the other rows. Epilogues: store, add into the fp32 residual, gated (two weights).
+// A workgroup of 8 (or 4) waves owns `rows` weight rows (up to 32, 16 with the gated epilogue) and cuts K, in blocks of
+// 64, among its waves: wave w takes blocks w, w + WAVES, ... Both operands of a block go straight from memory into a ring
+// of S blocks in LDS that belongs to the wave alone (global_load_lds_dwordx4, 1 KB per instruction: 8 rows of 128 bytes),
+// S - 1 blocks ahead of the multiplies; nothing but the wave's own counter of loads in flight stands between a load and its
+// use, so there is no barrier before the end. A lane's place in LDS is fixed by its number, so the bank swizzle is
+// applied on the global side: the lane that fills slot s of row r fetches the row's 16-byte piece s ^ sk_swz(r).
+//
+// Why not from memory into the registers that feed the matrix cores, as this kernel used to: such a load takes 64 bytes of
+// each of 16 rows, and a compute unit's load pipe then passes 25 bytes a clock (6.6 TB/s of the whole chip with everything in
+// L2, against 10 for 8 rows of 128 bytes), which the activations, once per workgroup and as many as the weights at 16 rows,
+// had to share. In LDS the activations of up to 8 rows cost half as much, and K blocks of 64 keep the waves even.
+// Inside a graph, before / now, in us at 1, 8 and 16 rows: 8B shape qkv 14.0 15.7 16.0 / 12.4 13.0 13.4, o 8.7 9.8 11.3 / 8.6
+// 9.0 9.6, gate/up 39.6 41.9 45.7 / 37.6 39.0 39.5, down 21.0 25.0 30.4 / 19.9 20.6 22.5; 32B down 51.2 58.6 68.4 / 47.3 48.8
+// 50.8; 0.6B o 4.7 5.8 6.4 / 4.1 4.5 4.8, down 7.4 9.0 10.4 / 5.0 5.6 6.3; slower: 1.7B qkv at one row 6.0 / 6.7.
+// What a large copy reaches (6.2 TB/s) would take 8.1, 5.4, 32.5 and 16.2 us of the 8B shape's four: what is left is the
+// launch, the first bytes' latency and the sum over the waves, about 4 us each. Measured and not taken: three blocks in
+// flight instead of up to six (8B gate/up at one row 37.9 -> 38.2), a contiguous range of K per wave (42.2).
+//
+// The WAVES partial tiles are summed through LDS in wave order, and how K is cut depends on nothing but K and N: a row's
+// result depends neither on M nor on the rows beside it.
+//
+// How many weight rows a workgroup owns (`rows`) is the caller's choice: as many as let N / rows workgroups fill the
+// compute units evenly. Rows beyond those (a load covers eight) are the last row again and never stored.
 //
 // An RMSNorm between two such products costs no launch of its own. The product that adds into the residual
 // ("emit") also leaves, for the norm that follows, the new residual values times that norm's gain as bf16
-// [M, N] and the sum of their squares over its 16 columns as partial[m][block]. The product that consumes the
+// [M, N] and the sum of their squares over its columns as partial[m][block]. The product that consumes the
 // norm ("normed") takes those bf16 rows as its input and multiplies its sums by rsqrt(sum of the partials / K +
 // eps) at the end: sum_k W[n,k] (x[k] g[k]) s = the product over the normalised row. The partials are summed in
 // an order that depends on nothing but their count.
 //
-// Needs K % 128 == 0, N % 16 == 0, M <= 64, 16-byte aligned rows; the caller falls back otherwise.
+// Needs K % 128 == 0, N % 16 == 0, M <= 16, 16-byte aligned rows; the caller falls back otherwise.
 #include "common.h"
 #include "mfma.h"
 
+#define SK_BLOCK 64                    // k per block
+#define SK_ROW_BYTES (SK_BLOCK * 2)    // a row of a block in LDS: 128 bytes = 8 pieces of 16
 
 // what the two norm-carrying forms need beyond the plain product
 struct SkinnyNorm {
   bf16_t* emit_rows;          // emit: [M, N] bf16, (residual after the add) * emit_gain
   const void* emit_gain;      // [N]
   int emit_gain_dtype;
-  float* emit_partial;        // [M][N / 16]
+  float* emit_partial;        // [M][emit_parts]: a sum per workgroup, zeros behind them
+  int emit_parts;
   const float* norm_partial;  // normed: [M][norm_parts] sums of squares of the input rows
   int norm_parts;
   float norm_eps;
@@ -42,267 +61,206 @@ __device__ __forceinline__ float row16_sum(float d) {
   return d;
 }
 
-// TWO: the workgroup owns 16 + rows2 weight rows (rows2 = 1 .. 16), the second tile in the place the up weight
-// has with the gated epilogue: the activations are read once for both, and N / 24 (or N / 20, N / 28) workgroups may
-// fill the compute units where N / 16 leaves some of them with one workgroup more. Store and accumulate epilogues,
-// the norm forms included: the squares of the second tile's columns go into the workgroup's one partial sum, and the
-// places of the [M][N / 16] partial sums that no workgroup owns are set to zero.
-template <int MT, bool GATED, int SK_WAVES, bool TWO = false>
-__global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(
+// The piece of row r in slot s is s ^ sk_swz(r): 16 lanes that read one piece of 16 rows cover the 64 banks once, and so do 8
+// lanes of 8 rows half of them.
+__device__ __forceinline__ int sk_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+
+template <int N>
+__device__ __forceinline__ void sk_wait_loads() {  // until at most N of the wave's loads are in flight
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// NI loads per block: a ring as deep as the LDS allows, with one workgroup of 8 waves or two of 4 on a compute unit
+constexpr int sk_slots(int ni, int waves) {
+  const int fit = ((waves == 8 ? 160 : 80) - 1) / (waves * ni);
+  return fit > 6 ? 6 : fit;
+}
+
+template <int NI, int S>
+__device__ __forceinline__ void sk_wait_block(int behind) {  // `behind` (< S) blocks behind the one that has to be here
+  if (behind == S - 1) return sk_wait_loads<(S - 1) * NI>();
+  if (S > 2 && behind == S - 2) return sk_wait_loads<(S > 2 ? S - 2 : 0) * NI>();
+  if (S > 3 && behind == S - 3) return sk_wait_loads<(S > 3 ? S - 3 : 0) * NI>();
+  if (S > 4 && behind == S - 4) return sk_wait_loads<(S > 4 ? S - 4 : 0) * NI>();
+  if (S > 5 && behind == S - 5) return sk_wait_loads<(S > 5 ? S - 5 : 0) * NI>();
+  sk_wait_loads<0>();
+}
+
+// NW: loads of 8 weight rows per block (of each weight), NA: of 8 activation rows
+template <int NW, int NA, bool GATED, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
     const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N,
-    int K, int epilogue, SkinnyNorm nm, int rows2) {
-  static_assert(!(GATED && TWO) && (!TWO || MT == 1), "a second tile of weight rows: one weight, one tile of rows");
-  constexpr bool DUAL = GATED || TWO;  // a second set of weight registers and sums
-  __shared__ float red[SK_WAVES - 1][MT][64][4];
-  __shared__ float ssq[SK_WAVES][MT][16];  // normed: each wave's share of the rows' sums of squares
-  const int wave = threadIdx.x >> 6;
+    int K, int epilogue, SkinnyNorm nm, int rows) {
+  constexpr int CT = (NW + 1) / 2;                // tiles of 16 weight rows
+  constexpr int TILES = GATED ? 2 : CT;           // accumulators: gate and up, or the weight's tiles
+  constexpr int NI = (GATED ? 2 : 1) * NW + NA;   // loads of a block
+  constexpr int S = sk_slots(NI, WAVES);
+  static_assert(!GATED || CT == 1, "the gated epilogue takes up to 16 rows of each weight");
+  static_assert(S >= 2 && (S - 1) * NI < 63, "the counter of loads in flight");
+  extern __shared__ __align__(1024) unsigned char smem[];   // [WAVES][S][NI KB]; afterwards the waves' sums
+  __shared__ float ssq[WAVES][16];                          // normed: each wave's share of the rows' sums of squares
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int col = lane & 15;
   const int g = lane >> 4;
-  const int n0 = blockIdx.x * (TWO ? 16 + rows2 : 16);
-  const int nblk = K >> 7;
-  const int rot = (int)((blockIdx.x * 7u) % (unsigned)nblk);
-  const bf16_t* wrow = W + (size_t)(n0 + col) * K + g * 8;
-  const bf16_t* urow = GATED ? W2 + (size_t)(n0 + col) * K + g * 8
-                       : TWO ? W + (size_t)(n0 + 16 + min(col, rows2 - 1)) * K + g * 8 : nullptr;
-  const bf16_t* arow[MT];
+  const int n0 = blockIdx.x * rows;
+  const int nblk = K / SK_BLOCK;
+  // gated: workgroups walk K from different starting blocks, so that at any moment they ask the L2 for different parts of
+  // the (shared) activations (12,288 x 4,096 at one row 39.2 -> 37.9 us; without the gate 6,144 x 4,096 12.4 -> 13.4)
+  const int rot = GATED ? (int)((blockIdx.x * 14u) % (unsigned)nblk) : 0;
+  // wave 0 writes the outputs: what it adds into (the residual, the bias) is requested before anything else
+  float prev[CT][4], b[CT], eg[CT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) arow[mt] = A + (size_t)min(mt * 16 + col, M - 1) * lda + g * 8;
-  floatx4 acc[MT];
-  floatx4 acc2[MT];
+  for (int t = 0; t < CT; ++t) {
+    b[t] = eg[t] = 0.f;
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    acc[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    acc2[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 4; ++i) prev[t][i] = 0.f;
   }
-  // wave 0 writes the outputs: what it adds into (the residual, the bias) is requested now, long before it is needed
-  float prev[MT][4];
-  float rscale[MT][4];  // normed: rsqrt(mean of squares + eps) of the rows this lane writes
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) rscale[mt][i] = 1.0f;
-  float b = 0.f, eg = 0.f, b2 = 0.f, eg2 = 0.f;
-  float prev2[4] = {0.f, 0.f, 0.f, 0.f};  // the second tile's share of the residual
   if (wave == 0) {
-    const int n = n0 + col;
-    if (bias) b = (bias_dtype == JLLM_BF16) ? ldf((const bf16_t*)bias, n) : ldf((const float*)bias, n);
-    if (TWO) {
-      const int n2 = n0 + 16 + min(col, rows2 - 1);
-      if (bias) b2 = (bias_dtype == JLLM_BF16) ? ldf((const bf16_t*)bias, n2) : ldf((const float*)bias, n2);
-      if (nm.emit_rows) eg2 = (nm.emit_gain_dtype == JLLM_BF16) ? ldf((const bf16_t*)nm.emit_gain, n2) : ldf((const float*)nm.emit_gain, n2);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = g * 4 + i;
-        prev2[i] = (epilogue == 1 && m < M) ? ((const float*)out)[(size_t)m * ldo + n2] : 0.f;
+    for (int t = 0; t < CT; ++t) {
+      const int n = min(n0 + min(t * 16 + col, rows - 1), N - 1);
+      if (bias) b[t] = (bias_dtype == JLLM_BF16) ? ldf((const bf16_t*)bias, n) : ldf((const float*)bias, n);
+      if (nm.emit_rows) eg[t] = (nm.emit_gain_dtype == JLLM_BF16) ? ldf((const bf16_t*)nm.emit_gain, n) : ldf((const float*)nm.emit_gain, n);
+      if (epilogue == 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (g * 4 + i < M) prev[t][i] = ((const float*)out)[(size_t)(g * 4 + i) * ldo + n];
       }
     }
-    if (nm.emit_rows) eg = (nm.emit_gain_dtype == JLLM_BF16) ? ldf((const bf16_t*)nm.emit_gain, n) : ldf((const float*)nm.emit_gain, n);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = mt * 16 + g * 4 + i;
-        prev[mt][i] = (epilogue == 1 && m < M) ? ((const float*)out)[(size_t)m * ldo + n] : 0.f;
-      }
   }
-  // UB K blocks per turn. What bounds this kernel is how many weight bytes are in flight, so the loads of a turn are
-  // asked for before the turn before it is multiplied. Loads come back in the order they were asked for, and a wait
-  // can only name how many of the latest may still be out: the loads of the next turn therefore stand in straight
-  // code (a branch around them makes the compiler wait for all of them), and the registers of two turns take turns
-  // instead of being copied (a copy waits for its load).
-  constexpr int UB = DUAL ? 1 : 2;
-  constexpr int STEP = UB * SK_WAVES;
-  constexpr bool PINGPONG = MT == 1 && !GATED;
-  auto block_of = [&](int blk, int b) {
-    // past the end: a harmless reload of the last block. Workgroups walk K from different starting blocks, so that
-    // at any moment they ask the L2 for different parts of the (shared) activations
-    int bb = min(blk + b * SK_WAVES, nblk - 1) + rot;
-    return bb >= nblk ? bb - nblk : bb;
-  };
-  // the ping-pong form: weights and activations of a turn together
-  struct Turn {
-    u32x4 w[UB][4], a[UB][4], u[TWO ? UB : 1][4];  // u: the second tile's weights
-  };
-  auto load = [&](Turn& t, int blk) {
+  // normed: the sums of squares of the input rows. Every wave takes a share: lane `col` of wave w the four partials
+  // 4 (16 w + col) .., requested here and added up behind the products, then those 64 WAVES further on
+  floatx4 first[4];
 #pragma unroll
-    for (int b = 0; b < UB; ++b) {
-      const size_t k = (size_t)block_of(blk, b) * 128;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) t.a[b][j] = *(const u32x4*)(arow[0] + k + j * 32);  // rows beyond M: row M - 1 again
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        t.w[b][j] = *(const u32x4*)(wrow + k + j * 32);
-        if (TWO) t.u[b][j] = *(const u32x4*)(urow + k + j * 32);
-      }
-    }
-  };
-  // the other form: the weights a turn ahead, copied into place after the products
-  u32x4 wv[UB][4], uv[UB][4];
-  auto fetch = [&](int blk, u32x4 (*w)[4], u32x4 (*u)[4]) {
-#pragma unroll
-    for (int b = 0; b < UB; ++b) {
-      const size_t k = (size_t)block_of(blk, b) * 128;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        w[b][j] = *(const u32x4*)(wrow + k + j * 32);
-        if (DUAL) u[b][j] = *(const u32x4*)(urow + k + j * 32);
-      }
-    }
-  };
-  Turn t0, t1;
-  if (PINGPONG)
-    load(t0, wave);  // a wave beyond the last block: a harmless load, no products
-  else if (wave < nblk)
-    fetch(wave, wv, uv);
+  for (int i = 0; i < 4; ++i) first[i] = floatx4{0.f, 0.f, 0.f, 0.f};
   if (nm.norm_partial) {
-    // normed: the sums of squares of the input rows, while the first weights are on their way. Every wave takes a
-    // share: lane `col` of wave w the four partials 4 (16 w + col) .., then those 64 SK_WAVES further on; the
-    // shares meet in LDS below, in wave order
-    const int p4n = nm.norm_parts >> 2;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) rscale[mt][i] = 0.f;
-    for (int p4 = wave * 16 + col; p4 < p4n; p4 += SK_WAVES * 16) {
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int m = mt * 16 + g * 4 + i;
-          if (m < M) {
-            const floatx4 v = ((const floatx4*)(nm.norm_partial + (size_t)m * nm.norm_parts))[p4];
-            rscale[mt][i] += (v[0] + v[1]) + (v[2] + v[3]);
-          }
-        }
-    }
+    for (int i = 0; i < 4; ++i)
+      if (g * 4 + i < M && wave * 16 + col < nm.norm_parts >> 2)
+        first[i] = ((const floatx4*)(nm.norm_partial + (size_t)(g * 4 + i) * nm.norm_parts))[wave * 16 + col];
   }
-  const int turns = wave < nblk ? (nblk - wave + STEP - 1) / STEP : 0;
-  if constexpr (PINGPONG) {
-    // every turn but the last has all of its blocks
-    auto products = [&](const Turn& t, int blk, bool whole) {
+  // ---- the loads of a block: a scalar base that advances with the block and a byte offset per lane that never changes
+  uint32_t goff[NI];
+  const int lrow = lane >> 3, lslot = lane & 7;
 #pragma unroll
-      for (int b = 0; b < UB; ++b) {
-        if (whole || blk + b * SK_WAVES < nblk) {
+  for (int c = 0; c < NI; ++c) {
+    const bool of_w = c < NI - NA;
+    const int r = (of_w ? c % NW : c - (NI - NA)) * 8 + lrow;
+    const uint32_t at = of_w ? (uint32_t)(min(n0 + min(r, rows - 1), N - 1) - n0) * (uint32_t)K : (uint32_t)min(r, M - 1) * (uint32_t)lda;
+    goff[c] = at * 2u + (uint32_t)((lslot ^ sk_swz(r)) * 16);
+  }
+  const unsigned char* wbase = (const unsigned char*)(W + (size_t)n0 * K);
+  const unsigned char* ubase = GATED ? (const unsigned char*)(W2 + (size_t)n0 * K) : nullptr;
+  const unsigned char* ring = smem + (size_t)wave * S * NI * 1024;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)ring;
+  const int total = wave < nblk ? (nblk - wave + WAVES - 1) / WAVES : 0;
+  auto issue = [&](int i, int slot) {
+    int bb = wave + i * WAVES + rot;
+    if (bb >= nblk) bb -= nblk;
+    const size_t kbytes = (size_t)bb * SK_ROW_BYTES;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            acc[0] = mfma16(t.a[b][j], t.w[b][j], acc[0]);
-            if (TWO) acc2[0] = mfma16(t.a[b][j], t.u[b][j], acc2[0]);
-          }
-        }
-      }
-    };
-    int i = 0, blk = wave;
-    for (; i + 2 < turns; i += 2, blk += 2 * STEP) {
-      load(t1, blk + STEP);
-      products(t0, blk, true);
-      load(t0, blk + 2 * STEP);
-      products(t1, blk + STEP, true);
+    for (int c = 0; c < NI; ++c) {
+      const unsigned char* base = (c >= NI - NA ? (const unsigned char*)A : GATED && c >= NW ? ubase : wbase) + kbytes;
+      // m0 holds the LDS address of the 1 KB, lane l's 16 bytes land at m0 + 16 l
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                   :
+                   : "v"(goff[c]), "s"(base), "s"(lds0 + (uint32_t)(slot * NI + c) * 1024u)
+                   : "memory", "m0");
     }
-    if (turns - i == 2) {
-      load(t1, blk + STEP);
-      products(t0, blk, true);
-      products(t1, blk + STEP, false);
-    } else if (turns - i == 1) {
-      products(t0, blk, false);
+  };
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+    if (i < total) issue(i, i);
+  // ---- fragments: lane l reads row l % 16, 8 of k at (l / 16) * 8 + 32 j: piece l / 16 + 4 j. Rows that no load fetched
+  // (eight activation rows, up to eight weight rows in a tile) are the last fetched eight again.
+  const int ar = NA == 1 ? col & 7 : col;
+  const int aoff = ((GATED ? 2 : 1) * NW) * 1024 + ar * SK_ROW_BYTES, aswz = sk_swz(ar);
+  int woff[TILES], wswz[TILES];
+#pragma unroll
+  for (int t = 0; t < TILES; ++t) {
+    const int left = GATED ? NW : NW - 2 * t;  // loads that this tile has
+    const int r = (GATED ? 0 : t * 16) + (left == 1 ? col & 7 : col);
+    woff[t] = (GATED ? t * NW * 1024 : 0) + r * SK_ROW_BYTES;
+    wswz[t] = sk_swz(r);
+  }
+  floatx4 acc[TILES];
+#pragma unroll
+  for (int t = 0; t < TILES; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  int slot = 0;
+  for (int i = 0; i < total; ++i) {
+    sk_wait_block<NI, S>(min(S - 1, total - 1 - i));
+    const unsigned char* blk = ring + slot * NI * 1024;
+    u32x4 a[2], w[TILES][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      a[j] = *(const u32x4*)(blk + aoff + (((g + 4 * j) ^ aswz) << 4));
+#pragma unroll
+      for (int t = 0; t < TILES; ++t) w[t][j] = *(const u32x4*)(blk + woff[t] + (((g + 4 * j) ^ wswz[t]) << 4));
     }
-  } else {
-    // several tiles of rows, or two weights: too many registers for two turns of activations, and more activation
-    // loads in flight only crowd out weight loads. The weights a turn ahead, the activations (L2) in their own turn
-    for (int blk = wave; blk < nblk; blk += STEP) {
-      u32x4 wn[UB][4], un[UB][4];
-      if (blk + STEP < nblk) fetch(blk + STEP, wn, un);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot's last reads, before it is filled again
+    __builtin_amdgcn_sched_barrier(0);
+    if (i + S < total) issue(i + S, slot);
 #pragma unroll
-      for (int b = 0; b < UB; ++b) {
-        if (blk + b * SK_WAVES < nblk) {
-          const size_t k = (size_t)block_of(blk, b) * 128;
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) {
-            u32x4 av[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              if (MT == 1)  // rows beyond M read row M - 1 again
-                av[j] = *(const u32x4*)(arow[mt] + k + j * 32);
-              else  // lanes of row tiles beyond M load nothing: their operand rows are zeros
-                av[j] = mt * 16 + col < M ? *(const u32x4*)(arow[mt] + k + j * 32) : u32x4{0u, 0u, 0u, 0u};
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              acc[mt] = mfma16(av[j], wv[b][j], acc[mt]);
-              if (DUAL) acc2[mt] = mfma16(av[j], uv[b][j], acc2[mt]);
-            }
-          }
-        }
-      }
-#pragma unroll
-      for (int b = 0; b < UB; ++b)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          wv[b][j] = wn[b][j];
-          if (DUAL) uv[b][j] = un[b][j];
-        }
-    }
+      for (int t = 0; t < TILES; ++t) acc[t] = mfma16(a[j], w[t][j], acc[t]);
+    if (++slot == S) slot = 0;
   }
   if (nm.norm_partial) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float t = row16_sum(rscale[mt][i]);
-        if (col == 0) ssq[wave][mt][g * 4 + i] = t;
-      }
-  }
-  // sum the 8 partial tiles in wave order (gate first, then up, or the second tile, through the same buffer)
-  for (int pass = 0; pass < (DUAL ? 2 : 1); ++pass) {
-    if (pass == 1) __syncthreads();
-    if (wave > 0) {
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) red[wave - 1][mt][lane][i] = pass == 0 ? acc[mt][i] : acc2[mt][i];
-    }
-    __syncthreads();
-    if (wave == 0) {
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float s = pass == 0 ? acc[mt][i] : acc2[mt][i];
-#pragma unroll
-          for (int w = 0; w < SK_WAVES - 1; ++w) s += red[w][mt][lane][i];
-          if (pass == 0)
-            acc[mt][i] = s;
-          else
-            acc2[mt][i] = s;
+    for (int i = 0; i < 4; ++i) {
+      float t = (first[i][0] + first[i][1]) + (first[i][2] + first[i][3]);
+      if (g * 4 + i < M)
+        for (int p4 = (WAVES + wave) * 16 + col; p4 < nm.norm_parts >> 2; p4 += WAVES * 16) {
+          const floatx4 v = ((const floatx4*)(nm.norm_partial + (size_t)(g * 4 + i) * nm.norm_parts))[p4];
+          t += (v[0] + v[1]) + (v[2] + v[3]);
         }
+      t = row16_sum(t);
+      if (col == 0) ssq[wave][g * 4 + i] = t;
     }
   }
+  // the sums meet in LDS, in wave order
+  __syncthreads();  // every wave is done with its ring
+  floatx4(*red)[TILES][64] = (floatx4(*)[TILES][64])smem;
+  if (wave > 0) {
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) red[wave - 1][t][lane] = acc[t];
+  }
+  __syncthreads();
   if (wave != 0) return;
-  if (nm.norm_partial) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+  for (int t = 0; t < TILES; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float t = 0.f;
+    for (int w = 0; w < WAVES - 1; ++w) acc[t] += red[w][t][lane];
+  float rscale[4];  // normed: rsqrt(mean of squares + eps) of the rows this lane writes
 #pragma unroll
-        for (int w = 0; w < SK_WAVES; ++w) t += ssq[w][mt][g * 4 + i];
-        rscale[mt][i] = 1.0f / sqrtf(t / (float)K + nm.norm_eps);
-      }
+  for (int i = 0; i < 4; ++i) {
+    rscale[i] = 1.0f;
+    if (nm.norm_partial) {
+      float t = 0.f;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) t += ssq[w][g * 4 + i];
+      rscale[i] = 1.0f / sqrtf(t / (float)K + nm.norm_eps);
+    }
   }
-  const int n = n0 + col;
-  float sq2[4] = {0.f, 0.f, 0.f, 0.f};  // the squares of the second tile's columns, per row of this lane
-  if (TWO) {  // the second tile: columns n0 + 16 .. n0 + 16 + rows2 - 1
-    const bool mine = col < rows2;
+  float sq[4] = {0.f, 0.f, 0.f, 0.f};  // emit: the squares of the workgroup's columns, per row of this lane
+#pragma unroll
+  for (int t = CT - 1; t >= 0; --t) {
+    const int n = n0 + t * 16 + col;
+    const bool mine = t * 16 + col < rows && n < N;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int m = g * 4 + i;
-      const float v = acc2[0][i] * rscale[0][i] + b2;
-      const float now = prev2[i] + v;
-      if (nm.emit_rows) sq2[i] = row16_sum(mine && m < M ? now * now : 0.f);
+      float v = acc[t][i] * rscale[i] + b[t];
+      if (GATED) v = gated<false>(v, acc[GATED ? 1 : 0][i] * rscale[i], nm.gate);
+      const float now = prev[t][i] + v;
+      // every lane of the row takes part in the sum, columns and rows that are not there with zeros
+      if (nm.emit_rows) sq[i] = row16_sum(mine && m < M ? now * now : 0.f) + sq[i];
       if (m >= M || !mine) continue;
-      const size_t o = (size_t)m * ldo + n + 16;
-      if (nm.emit_rows) nm.emit_rows[(size_t)m * N + n + 16] = f32_to_bf16(now * eg2);
+      const size_t o = (size_t)m * ldo + n;
+      if (nm.emit_rows) nm.emit_rows[(size_t)m * N + n] = f32_to_bf16(now * eg[t]);
       if (epilogue == 1)
         ((float*)out)[o] = now;
       else if (out_dtype == JLLM_BF16)
@@ -310,131 +268,99 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(
       else
         stf((float*)out, o, v);
     }
-    if (nm.emit_rows && col == 0) {  // the partial sums beyond the workgroups' own: zeros
-      const int spare = (N >> 4) - (int)gridDim.x;
-      if ((int)blockIdx.x < spare)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (g * 4 + i < M) nm.emit_partial[(size_t)(g * 4 + i) * (N >> 4) + gridDim.x + blockIdx.x] = 0.f;
-    }
   }
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+  if (nm.emit_rows && col == 0) {
+    const int spare = nm.emit_parts - (int)gridDim.x;  // partial sums behind the workgroups' own: zeros
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int m = mt * 16 + g * 4 + i;
-      float v = acc[mt][i] * rscale[mt][i] + b;
-      if (GATED) v = gated<false>(v, acc2[mt][i] * rscale[mt][i], nm.gate);
-      const float now = prev[mt][i] + v;
-      if (nm.emit_rows) {  // every lane of the row takes part in the sum, rows beyond M with zeros
-        const float sq = row16_sum(m < M ? now * now : 0.f) + (TWO ? sq2[i] : 0.f);
-        if (m < M) {
-          nm.emit_rows[(size_t)m * N + n] = f32_to_bf16(now * eg);
-          if (col == 0) nm.emit_partial[(size_t)m * (N >> 4) + blockIdx.x] = sq;
-        }
-      }
+      const int m = g * 4 + i;
       if (m >= M) continue;
-      const size_t o = (size_t)m * ldo + n;
-      if (epilogue == 1)
-        ((float*)out)[o] = now;
-      else if (out_dtype == JLLM_BF16)
-        stf((bf16_t*)out, o, v);
-      else
-        stf((float*)out, o, v);
+      nm.emit_partial[(size_t)m * nm.emit_parts + blockIdx.x] = sq[i];
+      for (int z = blockIdx.x; z < spare; z += gridDim.x) nm.emit_partial[(size_t)m * nm.emit_parts + gridDim.x + z] = 0.f;
     }
-}
-
-template <int MT, int WAVES>
-static void launch_skinny(dim3 grid, hipStream_t stream, const void* A, int lda, const void* W, const void* W2,
-                          const void* bias, int bias_dtype, void* out, int out_dtype, int ldo, int M, int N, int K,
-                          int epilogue, const SkinnyNorm& nm) {
-  if (W2)
-    gemm_skinny_kernel<MT, true, WAVES><<<grid, WAVES * 64, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W,
-                                                                         (const bf16_t*)W2, bias, bias_dtype, out,
-                                                                         out_dtype, ldo, M, N, K, epilogue, nm, 0);
-  else
-    gemm_skinny_kernel<MT, false, WAVES><<<grid, WAVES * 64, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W,
-                                                                          nullptr, bias, bias_dtype, out, out_dtype,
-                                                                          ldo, M, N, K, epilogue, nm, 0);
-}
-
-template <int WAVES>
-static void launch_skinny_mt(int mt, dim3 grid, hipStream_t stream, const void* A, int lda, const void* W,
-                             const void* W2, const void* bias, int bias_dtype, void* out, int out_dtype, int ldo, int M,
-                             int N, int K, int epilogue, const SkinnyNorm& nm) {
-  switch (mt) {
-    case 1: launch_skinny<1, WAVES>(grid, stream, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, nm); break;
-    case 2: launch_skinny<2, WAVES>(grid, stream, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, nm); break;
-    case 3: launch_skinny<3, WAVES>(grid, stream, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, nm); break;
-    default: launch_skinny<4, WAVES>(grid, stream, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, nm); break;
   }
+}
+
+struct SkinnyArgs {
+  const bf16_t *A, *W, *W2;
+  const void* bias;
+  int lda, bias_dtype, out_dtype, ldo, M, N, K, epilogue, rows;
+  void* out;
+};
+
+template <int NW, int NA, bool GATED, int WAVES>
+static int launch_skinny(const SkinnyArgs& a, const SkinnyNorm& nm, hipStream_t stream) {
+  constexpr int NI = (GATED ? 2 : 1) * NW + NA;
+  constexpr size_t smem = (size_t)sk_slots(NI, WAVES) * WAVES * NI * 1024;
+  static bool configured = false;
+  if (!configured) {  // above 64 KB the size has to be allowed first
+    if (hipFuncSetAttribute((const void*)gemm_skinny_kernel<NW, NA, GATED, WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+      JLLM_FAIL("gemm_skinny: cannot reserve %zu bytes of LDS", smem);
+    configured = true;
+  }
+  gemm_skinny_kernel<NW, NA, GATED, WAVES><<<(a.N + a.rows - 1) / a.rows, WAVES * 64, smem, stream>>>(
+      a.A, a.lda, a.W, a.W2, a.bias, a.bias_dtype, a.out, a.out_dtype, a.ldo, a.M, a.N, a.K, a.epilogue, nm, a.rows);
+  JLLM_CHECK_LAUNCH("gemm_skinny");
+  return 0;
+}
+
+template <int NW, bool GATED>
+static int launch_skinny_rows(const SkinnyArgs& a, const SkinnyNorm& nm, int waves, hipStream_t stream) {
+  if (waves == 8) return a.M <= 8 ? launch_skinny<NW, 1, GATED, 8>(a, nm, stream) : launch_skinny<NW, 2, GATED, 8>(a, nm, stream);
+  return a.M <= 8 ? launch_skinny<NW, 1, GATED, 4>(a, nm, stream) : launch_skinny<NW, 2, GATED, 4>(a, nm, stream);
 }
 
 static int skinny_checked(const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype,
                           void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue, float gate_limit,
-                          const SkinnyNorm& nm_in, int rows2, hipStream_t stream) {
+                          const SkinnyNorm& nm_in, int rows, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 64 || (K & 127) || (N & 15) || (lda & 7) || K <= 0) return 1;
+  if (M > 16 || (K & 127) || (N & 15) || (lda & 7) || K <= 0 || lda < 0) return 1;
   if (((uintptr_t)A & 15) || ((uintptr_t)W & 15) || (W2 && ((uintptr_t)W2 & 15))) return 1;
+  // a lane's place in an operand is a 32-bit byte offset from the workgroup's first row
+  if ((unsigned long long)lda >= (1ull << 26) || (unsigned long long)K >= (1ull << 25)) return 1;
   JLLM_TAKE_GATE("gemm_skinny", epilogue, gate_limit, gs);
   SkinnyNorm nm = nm_in;
   nm.gate = gs;
   if (epilogue < 0 || epilogue > 2 || (epilogue == 2) != (W2 != nullptr)) JLLM_FAIL("gemm_skinny: epilogue %d", epilogue);
   if (epilogue == 1 && out_dtype != JLLM_F32) JLLM_FAIL("gemm_skinny: the accumulate epilogue adds into fp32");
   if (ldo < N) JLLM_FAIL("gemm_skinny: ldo %d < N %d", ldo, N);
+  if (rows < 1 || rows > (W2 ? 16 : 32)) JLLM_FAIL("gemm_skinny: %d weight rows per workgroup (1 to 32, gated to 16)", rows);
+  const int groups = (N + rows - 1) / rows;
   if (nm.emit_rows && (epilogue != 1 || !nm.emit_gain || !nm.emit_partial)) JLLM_FAIL("gemm_skinny: rows for a norm come from the accumulate epilogue, with gain and partial sums");
+  if (nm.emit_rows && nm.emit_parts < groups) JLLM_FAIL("gemm_skinny: %d places for the partial sums of %d workgroups", nm.emit_parts, groups);
   if (nm.norm_partial && nm.norm_parts <= 0) JLLM_FAIL("gemm_skinny: %d partial sums", nm.norm_parts);
   if (nm.norm_partial && ((nm.norm_parts & 3) || ((uintptr_t)nm.norm_partial & 15))) return 1;
-  const int mt = (M + 15) / 16;
-  int cus = jllm_compute_units();
+  const int cus = jllm_compute_units();
   if (cus <= 0) JLLM_FAIL("gemm_skinny: the GPU's compute units could not be read");
-  // `rows2` > 0: one tile of rows, one weight; a workgroup owns 16 + rows2 weight rows, which the caller asks for
-  // where that many fewer workgroups fill the compute units and N / 16 do not (N = 6144 on 256 compute units: 256
-  // workgroups of 24 against 384, which leaves every other compute unit with two). Measured on that shape: the same
-  // at 1 row, 16.0 -> 14.9 us at 8 rows, 18.8 -> 16.4 at 16 (a third less activation traffic as well). 32 rows per
-  // workgroup for the output head, which has thousands of tiles, were measured too: slower below 8 rows (202 ->
-  // 218 us at one), so it keeps 16.
-  if (rows2 != 0) {
-    if (rows2 < 1 || rows2 > 16 || mt != 1 || W2 || N % (16 + rows2))
-      JLLM_FAIL("gemm_skinny: %d + 16 weight rows per workgroup need one weight, up to 16 rows and N %% (16 + %d) == 0", rows2, rows2);
-    const int groups = N / (16 + rows2);
-    if (groups > cus)
-      gemm_skinny_kernel<1, false, 4, true><<<groups, 4 * 64, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, nullptr, bias, bias_dtype,
-                                                                           out, out_dtype, ldo, M, N, K, epilogue, nm, rows2);
-    else
-      gemm_skinny_kernel<1, false, 8, true><<<groups, 8 * 64, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, nullptr, bias, bias_dtype,
-                                                                           out, out_dtype, ldo, M, N, K, epilogue, nm, rows2);
-    JLLM_CHECK_LAUNCH("gemm_skinny");
-    return 0;
+  const SkinnyArgs a{(const bf16_t*)A, (const bf16_t*)W, (const bf16_t*)W2, bias, lda, bias_dtype, out_dtype, ldo, M, N, K, epilogue, rows, out};
+  // One workgroup of 8 waves per compute unit where there are no more workgroups than those; else two of 4 waves, so that
+  // one streams while the other adds up and stores.
+  const int waves = groups > cus ? 4 : 8;
+  if (W2) return rows <= 8 ? launch_skinny_rows<1, true>(a, nm, waves, stream) : launch_skinny_rows<2, true>(a, nm, waves, stream);
+  switch ((rows + 7) / 8) {
+    case 1: return launch_skinny_rows<1, false>(a, nm, waves, stream);
+    case 2: return launch_skinny_rows<2, false>(a, nm, waves, stream);
+    case 3: return launch_skinny_rows<3, false>(a, nm, waves, stream);
+    default: return launch_skinny_rows<4, false>(a, nm, waves, stream);
   }
-  dim3 grid(N / 16);
-  // Every workgroup should be resident at once (a second round of workgroups starts late and runs at half load):
-  // with more than one 16-row tile per compute unit the K split is 4 waves instead of 8, so that three workgroups
-  // fit on a compute unit.
-  if (N / 16 > cus)
-    launch_skinny_mt<4>(mt, grid, stream, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, nm);
-  else
-    launch_skinny_mt<8>(mt, grid, stream, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, nm);
-  JLLM_CHECK_LAUNCH("gemm_skinny");
-  return 0;
 }
 
-// `rows2`: 0, or the weight rows a workgroup owns beyond its 16 (1 .. 16; one weight, up to 16 rows of activations,
-// N a multiple of 16 + rows2). returns 0 when it ran, 1 when the shape is not one it takes (the caller uses another
-// kernel), -1 on errors
+// `rows`: the weight rows a workgroup owns (1 to 32, with the gated epilogue to 16). returns 0 when it ran, 1 when the
+// shape is not one it takes (the caller uses another kernel), -1 on errors
 extern "C" int jllm_gemm_skinny_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias,
                                      int bias_dtype, void* out, int out_dtype, int ldo, int M, int N, int K,
-                                     int epilogue, float gate_limit, int rows2, hipStream_t stream) {
-  return skinny_checked(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gate_limit, SkinnyNorm{}, rows2, stream);
+                                     int epilogue, float gate_limit, int rows, hipStream_t stream) {
+  return skinny_checked(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gate_limit, SkinnyNorm{}, rows, stream);
 }
 
 // The same with an RMSNorm on either side (see the head of this file). emit_rows [M, N] bf16, emit_gain [N] and
-// emit_partial [M][N / 16] fp32 go with the accumulate epilogue; norm_partial [M][norm_parts] with any.
+// emit_partial [M][emit_parts] fp32 (a sum per workgroup, zeros behind them) go with the accumulate epilogue; norm_partial
+// [M][norm_parts] with any.
 extern "C" int jllm_gemm_skinny_norm_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias,
                                           int bias_dtype, void* out, int out_dtype, int ldo, int M, int N, int K,
-                                          int epilogue, float gate_limit, int rows2, void* emit_rows, const void* emit_gain,
-                                          int emit_gain_dtype, float* emit_partial, const float* norm_partial,
+                                          int epilogue, float gate_limit, int rows, void* emit_rows, const void* emit_gain,
+                                          int emit_gain_dtype, float* emit_partial, int emit_parts, const float* norm_partial,
                                           int norm_parts, float norm_eps, hipStream_t stream) {
-  SkinnyNorm nm{(bf16_t*)emit_rows, emit_gain, emit_gain_dtype, emit_partial, norm_partial, norm_parts, norm_eps, GateSpec{0, 0.f}};
-  return skinny_checked(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gate_limit, nm, rows2, stream);
+  SkinnyNorm nm{(bf16_t*)emit_rows, emit_gain, emit_gain_dtype, emit_partial, emit_parts, norm_partial, norm_parts, norm_eps, GateSpec{0, 0.f}};
+  return skinny_checked(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gate_limit, nm, rows, stream);
 }

@@ -114,7 +114,7 @@ def _declare(lib) -> None:
 
 _OPTIONAL_SIGS = {
     "jllm_gemm_skinny_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P],
-    "jllm_gemm_skinny_norm_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _P, _P, _I, _F, _P],
+    "jllm_gemm_skinny_norm_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _P, _I, _P, _I, _F, _P],
     "jllm_gemm_mfma_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P],
     "jllm_gemm_pingpong_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P, _P],
     "jllm_gemm_stream_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P],
@@ -391,18 +391,18 @@ def _skinny_norm(a, w, w2, bias, out, epilogue, emit=None, normed: Optional[Norm
     n_part = normed.partials if normed is not None else None
     head = (_ptr(a), a.stride(0), _ptr(w), _ptr(w2), _ptr(bias), _code(bias.dtype) if bias is not None else F32,
             _ptr(out), _code(out.dtype), out.stride(0), M, N, K, int(epilogue), float(gate_limit))
-    tail = (_ptr(e_rows), _ptr(e_gain), _code(e_gain.dtype) if e_gain is not None else F32, _ptr(e_part), _ptr(n_part),
-            n_part.shape[1] if n_part is not None else 0, normed.eps if normed is not None else 0.0, _stream())
+    emits = (_ptr(e_rows), _ptr(e_gain), _code(e_gain.dtype) if e_gain is not None else F32, _ptr(e_part))
+    takes = (_ptr(n_part), n_part.shape[1] if n_part is not None else 0, normed.eps if normed is not None else 0.0, _stream())
     few = M <= SKINNY_MAX_ROWS
-    rows2 = _skinny_second_rows(N, w2 is not None) if few else 0
+    emit_parts = e_part.shape[1] if e_part is not None else 0
     if few and not _few_rows_prefer_stream(N, K, w2 is not None):
-        return _try("jllm_gemm_skinny_norm_bf16", *head, rows2, *tail)
+        return _try("jllm_gemm_skinny_norm_bf16", *head, _skinny_rows(N, K, w2 is not None), *emits, emit_parts, *takes)
     parts = _stream_parts(N, K, w2 is not None) if K % 128 == 0 else 0
     if parts >= 2:
         partial = torch.empty((parts * (2 if w2 is not None else 1) * M * N,), dtype=torch.float32, device=a.device)
-        if _try("jllm_gemm_stream_norm_bf16", *head, parts, _ptr(partial), *tail):
+        if _try("jllm_gemm_stream_norm_bf16", *head, parts, _ptr(partial), *emits, *takes):
             return True
-    return few and _try("jllm_gemm_skinny_norm_bf16", *head, rows2, *tail)  # the second kernel declined (N % 256, one part)
+    return few and _try("jllm_gemm_skinny_norm_bf16", *head, 16, *emits, emit_parts, *takes)  # the second kernel declined (N % 256, one part)
 
 
 def gemm_add_then_norm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gain: torch.Tensor, eps: float,
@@ -420,7 +420,7 @@ def gemm_add_then_norm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gain
         _dev(a, w, bias, out, gain)
         M, N = out.shape
         scaled = torch.empty((M, N), dtype=torch.bfloat16, device=out.device)
-        partials = torch.empty((M, N // 16), dtype=torch.float32, device=out.device)
+        partials = torch.empty((M, _norm_partials(M, N, a.shape[1])), dtype=torch.float32, device=out.device)
         if _skinny_norm(a, w, None, bias, out, EPI_ADD, emit=(scaled, gain, partials)):
             return NormedRows(out, gain, eps, norm_dtype, scaled, partials)
     gemm(a, w, bias=bias, out=out, epilogue=EPI_ADD, exact=exact)
@@ -735,11 +735,6 @@ def _stream_parts(N: int, K: int, gated: bool) -> int:
     return best
 
 
-STREAM_BASE = 1.23     # the second kernel's time against the first's at one row, same bytes, both with full rounds
-STREAM_MERGE_MB = 17   # its second launch (the merge of the K parts), in megabytes of streaming time
-SKINNY_ROW_COST = 0.45  # what 16 rows of activations add to the first kernel's time, as a fraction
-
-
 def _round_fill(groups: int) -> float:
     """The share of the compute units' rounds that `groups` workgroups fill."""
     cus = compute_units()
@@ -751,11 +746,8 @@ def _skinny_second_rows(N: int, gated: bool) -> int:
     """Weight rows that a workgroup of the first weight-streaming kernel owns beyond its 16 (0, 4, 8, 12 or 16) for a
     product of up to 16 rows: more than none where N / 16 workgroups leave some compute units with one workgroup more
     than the others and N / (16 + rows) fill their rounds by a fifth more. On 256 compute units N = 6144 gives 24
-    rows (256 workgroups against 384) and N = 5120 gives 20 (256 against 320). Measured at 8 rows on N = 5120: K =
-    5120 19.2 -> 15.1 us, K = 8192 27.9 -> 21.9, K = 17408 56.4 -> 42.1 (the K-cutting kernel: 45.2), K = 25600
-    81.9 -> 60.1 (60.6). Where the rounds fill by less there is nothing to gain: N = 7168 with 28 rows (256 against
-    448) 21.6 -> 20.8 us at 8 rows and 17.2 -> 18.2 at one, N = 10240 with 20 rows 29.2 -> 29.0. The gated product
-    has its second tile taken (the up weight)."""
+    rows (256 workgroups against 384) and N = 5120 gives 20 (256 against 320). The gated product has its second tile taken
+    (the up weight)."""
     if gated or N % 16:
         return 0
     best, best_fill = 0, _round_fill(N // 16) + 0.2
@@ -765,27 +757,53 @@ def _skinny_second_rows(N: int, gated: bool) -> int:
     return best
 
 
+SKINNY_HEAD_ROWS_K = 4096   # below this K a product of many rounds gives its workgroups 32 weight rows instead of 16
+
+
+@functools.lru_cache(maxsize=None)
+def _skinny_rows(N: int, K: int, gated: bool) -> int:
+    """Weight rows that a workgroup of the first weight-streaming kernel owns, from N and K alone: 16 and what
+    `_skinny_second_rows` adds, else the fewest, in steps of four, with which one workgroup per compute unit covers N, or
+    two. Beyond that 16 (gated: 12 where the rounds then fill by a
+    twelfth more), or 32 over a short K, where a workgroup of 16 has too little to stream. Swept over 4 .. 32 rows on the
+    products of six models at 1, 8 and 16 rows; at 8 rows, against 16 per workgroup: 1,024 x 3,072 with four 6.6 -> 5.6 us,
+    2,048 x 6,144 with 8 9.8 -> 8.2, 2,560 x 9,728 with 12 14.2 -> 13.0, 5,120 x 25,600 with 20 61.9 -> 48.8, 7,168 x 5,120
+    with 28 17.4 -> 17.0, gated 6,144 x 2,048 with 12 13.5 -> 12.8; 151,936 x 1,024 with 32 82.9 -> 65.2 (x 4,096: 202.7 ->
+    208.8, so that stays at 16)."""
+    second = _skinny_second_rows(N, gated)
+    if second:
+        return 16 + second
+    cus = compute_units()
+    most = 16 if gated else 32
+    for share in (1, 2):
+        rows = -(-N // (share * cus * 4)) * 4
+        if rows <= most:
+            return rows
+    if gated:
+        return 12 if _round_fill(-(-N // 12)) > _round_fill(-(-N // 16)) + 0.08 else 16
+    return 32 if K < SKINNY_HEAD_ROWS_K else 16
+
+
+def _norm_partials(M: int, N: int, K: int) -> int:
+    """Partial sums of squares per row that a product with N outputs leaves for the norm behind it: one per 16 columns
+    (the kernel for 17 to 64 rows, and the least that the first one is given), or one per workgroup of the first one,
+    in whole fours."""
+    if M > SKINNY_MAX_ROWS or _few_rows_prefer_stream(N, K, False):
+        return N // 16
+    return max(N // 16, -(-(-(-N // _skinny_rows(N, K, False))) // 4) * 4)
+
+
+STREAM_FEW_ROWS = (1280, 8192)   # columns at most, K at least: see `_few_rows_prefer_stream`
+
+
 @functools.lru_cache(maxsize=None)
 def _few_rows_prefer_stream(N: int, K: int, gated: bool) -> bool:
-    """Which weight-streaming kernel takes products of up to 16 rows of this shape. The first kernel gives 16 weight
-    rows to a workgroup and cannot cut K over workgroups: with N / 16 just above a multiple of the compute units a few
-    of them get one workgroup more and everybody waits for those, unless a workgroup can own a few rows more
-    (`_skinny_second_rows`). The second kernel cuts K as well and fills its rounds, at the price of a second launch
-    and of being a little slower byte for byte. From N and K alone (priced at 8 rows), so that all products of up to
-    16 rows of one shape come from one kernel. Measured at 8 rows, first against second kernel, 16 weight rows per
-    workgroup: down product of the 14B shape 56.6 / 46.7 us, of the 32B shape 82.4 / 62.3; every product of the 8B
-    shape is faster in the first, and so are those two with 20 rows per workgroup (42.1 and 60.1 us)."""
-    if K % 128 or N % 16:
-        return False
-    COMPUTE_UNITS = compute_units()
-    fill16 = _round_fill(N // (16 + _skinny_second_rows(N, gated)))
-    parts = _stream_parts(N, K, gated)
-    groups = -(-N // 128) * parts
-    fill = groups / (COMPUTE_UNITS * -(-groups // COMPUTE_UNITS))
-    mb = N * K * 2 * (2 if gated else 1) / 1e6
-    first = mb / fill16 * (1.0 + SKINNY_ROW_COST * 0.5 * (0.5 if gated else 1.0))
-    second = mb / fill * STREAM_BASE + STREAM_MERGE_MB
-    return second < 0.95 * first
+    """Whether products of up to 16 rows of this shape go to the second weight-streaming kernel, which cuts K over
+    workgroups: few columns and a very long K, whose rows then have the same bits in every batch of up to 64. From N and K
+    alone, so that all products of up to 16 rows of one shape come from one kernel. First / second kernel at 8 rows: 1,024 x
+    8,192 7.7 / 11.5 us, x 16,384 11.7 / 14.8 (at 16 rows 15.2 / 15.1), 2,048 x 8,192 9.5 / 13.6: no shape of the served
+    sizes is better off there."""
+    return not gated and K % 128 == 0 and N % 16 == 0 and N <= STREAM_FEW_ROWS[0] and K >= STREAM_FEW_ROWS[1]
 
 
 def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0) -> bool:
@@ -800,7 +818,7 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0) -> bool:
     head = (_ptr(a), a.stride(0), _ptr(w), _ptr(w2), _ptr(bias), _code(bias.dtype) if bias is not None else F32,
             _ptr(out), _code(out.dtype), out.stride(0), M, N, K, int(epilogue), float(gate_limit))
     if M <= SKINNY_MAX_ROWS and not _few_rows_prefer_stream(N, K, w2 is not None) \
-            and _try("jllm_gemm_skinny_bf16", *head, _skinny_second_rows(N, w2 is not None), _stream()):
+            and _try("jllm_gemm_skinny_bf16", *head, _skinny_rows(N, K, w2 is not None), _stream()):
         return True
     if M <= STREAM_MAX_ROWS and K % 128 == 0:
         parts = _stream_parts(N, K, w2 is not None)
@@ -817,7 +835,7 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0) -> bool:
     partial = torch.empty((splits * M * N,), dtype=torch.float32, device=a.device) if splits > 1 else None
     if _try("jllm_gemm_mfma_bf16", *head, splits, _ptr(partial), _stream()):
         return True
-    return M <= 64 and _try("jllm_gemm_skinny_bf16", *head, 0, _stream())
+    return False
 
 
 def qk_norm_rope_store(qkv: torch.Tensor, positions: torch.Tensor, slots: Optional[torch.Tensor],

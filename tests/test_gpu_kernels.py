@@ -275,6 +275,43 @@ def test_norm_between_two_products(ops, M, N, K, N2, gdt):
     assert torch.equal(ops.gemm(p2, w2), ops.gemm(ops.rmsnorm(big_res, gain, eps, torch.bfloat16), w2))
 
 
+@pytest.mark.parametrize("rows", [1, 4, 7, 8, 9, 12, 16, 17, 20, 24, 31, 32])
+@pytest.mark.parametrize("M,N,K", [(1, 96, 128), (8, 4112, 384), (9, 272, 1152), (16, 48, 2560), (5, 8192, 640)])
+def test_few_row_products_at_any_weight_rows_per_workgroup(ops, monkeypatch, M, N, K, rows):
+    """The kernel for up to 16 rows with any number of weight rows per workgroup: last workgroups with fewer rows than the
+    others, loads of eight rows that are not all there, fewer blocks of K than waves and than the ring holds, one and
+    two loads of activations, one and two workgroups a compute unit. Against float64: an fp32 sum of K products, whatever its order, is within
+    K 2^-24 of the sum of their sizes (and twice that for what is summed before the add), the bf16 rows for a norm exactly
+    what the new residual gives. Without the gate the split of K knows nothing of the rows per workgroup: the same bits."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M * N + K + rows)
+    rnd = lambda *shape: torch.randn(*shape, device=DEV, generator=gen)
+    a, w, w2 = rnd(M, K).bfloat16(), (rnd(N, K) / math.sqrt(K)).bfloat16(), (rnd(N, K) / math.sqrt(K)).bfloat16()
+    bias, gain, res0 = rnd(N), rnd(N).abs() + 0.5, rnd(M, N)
+    monkeypatch.setattr(ops, "_few_rows_prefer_stream", lambda *_: False)
+    monkeypatch.setattr(ops, "_skinny_rows", lambda n, k, gated: min(rows, 16) if gated else rows)
+    ops.reset_stats()
+    exact, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    bound = 2 * K * 2.0 ** -24 * size + 1e-6
+    out = ops.gemm(a, w, bias=bias, out_dtype=torch.float32)
+    assert bool(((out.double() - exact - bias.double()).abs() <= bound + 2.0 ** -23 * (exact.abs() + bias.abs())).all())
+    res = res0.clone()
+    promise = ops.gemm_add_then_norm(a, w, res, gain, 1e-3, torch.bfloat16)
+    assert bool(((res.double() - exact - res0.double()).abs() <= bound + 2.0 ** -23 * (exact.abs() + res0.abs())).all())
+    assert torch.equal(promise.scaled, (res * gain).bfloat16())
+    want = (res.double() ** 2).sum(-1)
+    assert bool(((promise.partials.double().sum(-1) - want).abs() <= 32 * 2.0 ** -24 * want).all())
+    gated = ops.gemm(a, w, w2=w2, epilogue=ops.EPI_GATED, out_dtype=torch.float32)
+    up = a.double() @ w2.double().T
+    both = bound * (1.1 * up.abs() + 1) + 2 * K * 2.0 ** -24 * (a.double().abs() @ w2.double().abs().T) * exact.abs() + 1e-5 * (exact * up).abs()
+    assert bool(((gated.double() - torch.nn.functional.silu(exact) * up).abs() <= both).all())
+    assert set(ops.stats()["ran"]) == {"jllm_gemm_skinny_bf16", "jllm_gemm_skinny_norm_bf16"}
+    if (N + rows - 1) // rows > ops.compute_units():  # four waves; the sums of eight differ from theirs
+        return
+    monkeypatch.setattr(ops, "_skinny_rows", lambda n, k, gated: 32)
+    assert torch.equal(out, ops.gemm(a, w, bias=bias, out_dtype=torch.float32))
+
+
 def test_gemm_rows_do_not_depend_on_the_batch(ops):
     """The result of a row is the same bits whether it is alone or among others, within one kernel family (the
     bfloat16 path has one kernel for up to 16 rows, one for up to 64 and one for more; between them results differ
