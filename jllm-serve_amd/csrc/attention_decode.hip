@@ -16,9 +16,12 @@
 // qkv[t] = [q | k | v] as it comes from the product, normalises and rotates q in registers (every workgroup for
 // its own heads), lets the workgroup of a row's last split normalise, rotate and store the new key and copy the
 // new value into their page before the keys are read (the matrix-core kernel for head_dim 128: keeps them in LDS as well
-// and never waits for the store). The splits are merged by the same second kernel. (Merging
-// them in the first kernel, by the workgroup that finishes last, was measured: the device-wide fences it needs
-// cost far more than the launch it saves.)
+// and never waits for the store). At head size 128 the splits are merged by the workgroup of a row and kv head that finishes last
+// (common.h says how it comes to see what the others left), where the caller has counters for that; else by the same second
+// kernel. A launch of its own is 4.2 to 4.8 us a layer; here the last workgroup's way through memory (its stores, its count, the
+// others' parts) adds 2.2 to 3.3. Whole steps: 300 keys of the 0.6B shape 1,022 -> 979 us, one request of 2,048 keys (8B)
+// 3,414 -> 3,343, eight of 900 to 2,500 3,994 -> 3,919, 64 of up to 1,000 6,446 -> 6,385 (runs of one side differ by 0.9 %),
+// four of 6,100 to 8,000 (4B) 3,182 -> 3,105.
 //
 // Needs bf16, head_dim % 8 == 0, head_dim <= 256, G <= 8 (the fused form: rotary width % 16 == 0); the caller
 // falls back to the general kernels otherwise.
@@ -126,6 +129,49 @@ __device__ __forceinline__ void combine_head(const float* part_acc, const float*
   }
 }
 
+// The same for head size 128 inside the launch that made the parts: lane l takes dims 2 l and 2 l + 1 (each dim's sum is the one
+// above), reading what other workgroups of the launch have left.
+__device__ __forceinline__ void combine_arrived(const float* part_acc, const float* part_ml, size_t base, int s_lo, int s_hi, bf16_t* o, int lane) {
+  const int ns = s_hi - s_lo + 1;
+  float ms = -INFINITY, ls = 0.f, m = -INFINITY;
+  if (lane < ns) load_shared2(part_ml + (base + s_lo + lane) * 2, ms, ls);
+  if (ns > 64) {
+    for (int c = 64 + lane; c < ns; c += 64) {
+      float a, b;
+      load_shared2(part_ml + (base + s_lo + c) * 2, a, b);
+      m = fmaxf(m, a);
+    }
+  }
+  float l = 0.f, acc0 = 0.f, acc1 = 0.f;
+  for (int c = 0; c < ns; c += 64) {  // ascending blocks of 64 splits, ascending inside a block
+    if (c > 0) {
+      ms = -INFINITY, ls = 0.f;
+      if (c + lane < ns) load_shared2(part_ml + (base + s_lo + c + lane) * 2, ms, ls);
+    }
+    const int nb = min(64, ns - c);
+    float w = 0.f;
+    for (int j0 = 0; j0 < nb; j0 += 8) {  // eight splits' values are requested before any is used
+      float pv[8][2];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) load_shared2(part_acc + (base + s_lo + c + min(j0 + j, nb - 1)) * 128 + 2 * lane, pv[j][0], pv[j][1]);
+      if (j0 == 0) {
+        if (c == 0) m = wave_max(fmaxf(m, ms));
+        w = c + lane < ns ? __builtin_amdgcn_exp2f(ms - m) : 0.f;
+        l += wave_sum(ls * w);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float wl = __shfl(w, min(j0 + j, 63), 64);
+        const float wj = j0 + j < nb ? wl : 0.f;
+        acc0 = fmaf(pv[j][0], wj, acc0);
+        acc1 = fmaf(pv[j][1], wj, acc1);
+      }
+    }
+  }
+  const float inv = 1.0f / l;
+  ((uint32_t*)o)[lane] = pack2(acc0 * inv, acc1 * inv);
+}
+
 // what the fused form needs beyond the plain one
 struct DecodeFusion {
   const int* slots;       // cache slot of each row's new token, < 0: store nothing
@@ -139,6 +185,7 @@ struct DecodeFusion {
   int write_kv;           // 0: the cache belongs to another layer, which has stored this token already
   bf16_t* kc_w;           // the caches again, writable
   bf16_t* vc_w;
+  int* arrivals;          // [rows][kv heads] zeros, null: the merge of the splits is a launch of its own
 };
 
 template <int LPK, int G, bool FUSED>
@@ -682,6 +729,7 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
   }
   __syncthreads();
   const bool single = s_lo == s_hi;
+  const bool merges = FUSED && fu.arrivals && !single;
   if (wave == 0 && sub < G) {
 #pragma unroll
     for (int w = 0; w < DA_WAVES - 1; ++w) {
@@ -706,13 +754,35 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
     } else {
       const size_t pi = ((size_t)t * H + h) * max_splits + s;
       float* pa = part_acc + pi * hd + 4 * q4;
+      if (merges) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) *(floatx4*)(pa + 16 * j) = acc[j];
-      if (q4 == 0) {
-        part_ml[pi * 2] = m1;
-        part_ml[pi * 2 + 1] = l1;
+        for (int j = 0; j < 8; ++j) {
+          store_shared2(pa + 16 * j, acc[j][0], acc[j][1]);
+          store_shared2(pa + 16 * j + 2, acc[j][2], acc[j][3]);
+        }
+        if (q4 == 0) store_shared2(part_ml + pi * 2, m1, l1);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) *(floatx4*)(pa + 16 * j) = acc[j];
+        if (q4 == 0) {
+          part_ml[pi * 2] = m1;
+          part_ml[pi * 2 + 1] = l1;
+        }
       }
     }
+  }
+  if (!merges) return;
+  // the workgroup of this row and kv head that arrives last merges the splits, a wave per query head
+  __shared__ int last;
+  if (wave == 0) {
+    shared_stores_done();
+    if (lane == 0) last = arrived_last(fu.arrivals + (size_t)t * Hkv + kvh, s_hi - s_lo + 1);
+  }
+  __syncthreads();
+  if (!last) return;
+  for (int g = wave; g < G; g += DA_WAVES) {
+    const int h = kvh * G + g;
+    combine_arrived(part_acc, part_ml, ((size_t)t * H + h) * max_splits, s_lo, s_hi, out + (size_t)t * ldo + (size_t)h * hd, lane);
   }
 }
 
@@ -794,7 +864,7 @@ static int decode_attention(const void* q, int ldq, void* out, int ldo, const vo
 #undef DA_ARGS
   if (rc != 0) return rc;
   JLLM_CHECK_LAUNCH("decode_attention");
-  if (used > 1) {
+  if (used > 1 && !(hd == 128 && fu.arrivals)) {
     dim3 cg(n_rows, H);
     decode_attention_combine_kernel<<<cg, 64, 0, stream>>>(part_acc, part_ml, positions, H, hd, window, max_splits, split,
                                                            (bf16_t*)out, ldo);
@@ -818,7 +888,8 @@ extern "C" int jllm_decode_attention_bf16(const void* q, int ldq, void* out, int
 
 // The whole attention of a decode step from the projection output qkv [rows, (H + 2 Hkv) * hd]: q/k norm (gains
 // null: none), rotation (tables null: none), store of the new key and value at `slots` (write_kv = 0: not stored),
-// attention over the pages, merge of the splits.
+// attention over the pages, merge of the splits. `arrivals` [rows][kv heads], all zero and left so: head size 128 merges in the
+// same launch (null: in a second one); used by one launch at a time.
 extern "C" int jllm_decode_attention_fused_bf16(const void* qkv, int ldqkv, void* out, int ldo, void* kcache,
                                                 void* vcache, const int* block_table, int max_blocks,
                                                 const int* row_req, const int* positions, const int* slots,
@@ -826,14 +897,14 @@ extern "C" int jllm_decode_attention_fused_bf16(const void* qkv, int ldqkv, void
                                                 int gain_dtype, float eps, int rot, int write_kv, int n_rows, int H,
                                                 int Hkv, int hd, int page_size, int window, float scale, int max_pos,
                                                 float* part_acc, float* part_ml, int max_splits, int split,
-                                                hipStream_t stream) {
+                                                int* arrivals, hipStream_t stream) {
   if ((cos_t == nullptr) != (sin_t == nullptr)) JLLM_FAIL("decode attention: cos and sin tables come together");
   if ((gq == nullptr) != (gk == nullptr)) JLLM_FAIL("decode attention: q and k gains come together");
   if (cos_t && (rot < 16 || rot > hd || (rot & 15))) return 1;
   if (ldqkv < (H + 2 * Hkv) * hd) JLLM_FAIL("decode attention: row stride %d < %d", ldqkv, (H + 2 * Hkv) * hd);
   if (write_kv && !slots) JLLM_FAIL("decode attention: cache write without slots");
   if (((uintptr_t)gq & 15) || ((uintptr_t)gk & 15)) return 1;
-  DecodeFusion fu{slots, cos_t, sin_t, gq, gk, gain_dtype, eps, rot, write_kv, (bf16_t*)kcache, (bf16_t*)vcache};
+  DecodeFusion fu{slots, cos_t, sin_t, gq, gk, gain_dtype, eps, rot, write_kv, (bf16_t*)kcache, (bf16_t*)vcache, arrivals};
   return decode_attention<true>(qkv, ldqkv, out, ldo, kcache, vcache, block_table, max_blocks, row_req, positions, n_rows,
                                 H, Hkv, hd, page_size, window, scale, max_pos, part_acc, part_ml, max_splits, split, fu,
                                 stream);

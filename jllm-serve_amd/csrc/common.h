@@ -127,6 +127,30 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return s;
 }
 
+// Values that one workgroup leaves for another of the same launch. The compute units' caches, and the L2s of the eight dies,
+// do not see each other's writes during a kernel; accesses of agent scope pass them by. So the data are stored and read with
+// such accesses, a wave waits for its stores, and only then counts itself as arrived: who sees the count sees the data. (A
+// fence of agent scope would write back and drop the whole L2 instead, which cost more than the launch it saves.) Nobody waits
+// for anybody: the workgroup that arrives last does what is left to do.
+__device__ __forceinline__ void store_shared2(float* p, float a, float b) {  // 8-byte aligned
+  const unsigned long long v = (unsigned long long)__float_as_uint(a) | ((unsigned long long)__float_as_uint(b) << 32);
+  __hip_atomic_store((unsigned long long*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void load_shared2(const float* p, float& a, float& b) {
+  const unsigned long long v = __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  a = __uint_as_float((unsigned)v);
+  b = __uint_as_float((unsigned)(v >> 32));
+}
+__device__ __forceinline__ void shared_stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// Called by one lane whose wave's (or, behind a barrier, whose workgroup's) stores are done: whether it is the last of `all`.
+// The last one leaves the counter at zero for the next launch.
+__device__ __forceinline__ bool arrived_last(int* counter, int all) {
+  const int before = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (before != all - 1) return false;
+  __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
 // host side -----------------------------------------------------------------------------------------------
 void jllm_set_error(const char* fmt, ...);
 extern "C" int jllm_compute_units();  // of the current GPU (elementwise.hip)

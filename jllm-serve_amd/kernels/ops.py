@@ -121,7 +121,7 @@ _OPTIONAL_SIGS = {
     "jllm_gemm_stream_norm_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _P, _I, _P, _P, _I, _F, _P],
     "jllm_decode_attention_bf16": [_P, _I, _P, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _I, _P],
     "jllm_decode_attention_fused_bf16": [_P, _I, _P, _I, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _F, _I, _I, _I, _I, _I,
-                                         _I, _I, _I, _F, _I, _P, _P, _I, _I, _P],
+                                         _I, _I, _I, _F, _I, _P, _P, _I, _I, _P, _P],
     "jllm_prefill_attention_bf16": [_P, _I, _P, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _P],
     "jllm_latent_attention_bf16": [_P, _I, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P, _I, _I, _P, _P],
     "jllm_latent_heads_bf16": [_P, _I, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P],
@@ -984,7 +984,8 @@ def decode_attention_fused(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: to
                            write_kv: bool = True) -> Optional[torch.Tensor]:
     """A decode step's whole attention in one launch, from the projection output ``qkv`` [rows, (H + 2 Hkv) * hd]
     (left as it is): q/k norm, rotation, store of the new key and value at ``slots`` and attention over the pages
-    in one launch, the merge of the key splits in a second. Returns the output [rows, H * hd], or None when the kernel does not take the case
+    and, at head size 128 with ``meta["arrivals"]`` (int32 zeros, one per row and kv head, left zero), the merge of the key
+    splits; else that is a second launch. Returns the output [rows, H * hd], or None when the kernel does not take the case
     (then ``qk_norm_rope_store`` and ``paged_attention`` do the same in three launches."""
     if qkv.dtype != torch.bfloat16 or k_cache.dtype != torch.bfloat16 or meta is None or not meta.get("decode_only"):
         return None
@@ -1023,11 +1024,17 @@ def decode_attention_fused(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: to
         return out
     part_acc = torch.empty((T * heads * splits * head_dim,), dtype=torch.float32, device=device)
     part_ml = torch.empty((T * heads * splits * 2,), dtype=torch.float32, device=device)
+    arrivals = meta.get("arrivals")  # zeros of this step alone: every launch that counts in them leaves them zero
+    if arrivals is not None:
+        _i32(arrivals, arrivals.numel(), "arrival counters")
+        _dev(qkv, arrivals)
+        if arrivals.numel() < T * kv_heads:
+            arrivals = None
     ok = _try("jllm_decode_attention_fused_bf16", _ptr(qkv), qkv.stride(0), _ptr(out), out.stride(0), _ptr(k_cache),
               _ptr(v_cache), _ptr(block_table), block_table.shape[1], _ptr(row_req), _ptr(positions), _ptr(slots),
               _ptr(cos), _ptr(sin), _ptr(gq), _ptr(gk), _code(gq.dtype) if gq is not None else F32, float(eps),
               int(rotary_dim), 1 if write_kv else 0, T, heads, kv_heads, head_dim, k_cache.shape[2], int(window),
-              float(scale), max_ctx - 1, _ptr(part_acc), _ptr(part_ml), splits, split, _stream())
+              float(scale), max_ctx - 1, _ptr(part_acc), _ptr(part_ml), splits, split, _ptr(arrivals), _stream())
     return out if ok else None
 
 

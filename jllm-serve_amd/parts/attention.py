@@ -35,9 +35,13 @@ class GqaStepPlanner:
     single row lie together (then those rows go through the kernel for single rows and the tile list ends before
     them); and whether the portions' runs differ much in their number of keys (one prompt from its start: the last
     run sees 16 times the keys of the first), which is when the portion kernel does well to cut every run's keys over
-    two groups of waves."""
+    two groups of waves. A step of single rows also brings zeroed counters, one per row and
+    kv head, by which the workgroups of the split-key kernel find out which of them merges; the layers, which follow each
+    other in one stream, take turns in them."""
 
-    key = ("gqa", TILE_ROWS)
+    def __init__(self, kv_heads: int = 0):
+        self.kv_heads = kv_heads
+        self.key = ("gqa", TILE_ROWS, kv_heads)
 
     def plan(self, batch):
         from ..engine.step import StepPlan
@@ -60,7 +64,7 @@ class GqaStepPlanner:
                 single_rows = (ones[0], len(ones))
             runs += [(s.index, s.row0, 1, s.pos0) for s in segments if s.n == 1]
             tiles = [v for t in runs for v in t]
-        return StepPlan({"tiles": tiles}, {"decode_only": decode_only, "n_tiles": len(tiles) // 4,
+        return StepPlan({"tiles": tiles, "arrivals": [0] * (batch.rows * self.kv_heads if decode_only else 0)}, {"decode_only": decode_only, "n_tiles": len(tiles) // 4,
                                            "n_tiles_multi": n_multi, "single_rows": single_rows,
                                            "key_groups": key_groups})
 
@@ -134,12 +138,11 @@ class GqaAttention(Part):
         return KvSpec(self.spec.kv_heads, self.spec.head_dim, self.spec.window)
 
     def step_planners(self):
-        return [GqaStepPlanner()]
+        return [GqaStepPlanner(self.spec.kv_heads)]
 
-    @staticmethod
-    def _batch_facts(step):
+    def _batch_facts(self, step):
         """The kernels' view of the batch: the step's own numbers and this mixer's plan of it."""
-        plan = step.plans.get(GqaStepPlanner.key)
+        plan = step.plans.get(GqaStepPlanner(self.spec.kv_heads).key)
         meta = {"max_context": step.max_context, "requests": step.n_requests, "rows": step.n_tokens}
         if plan is None:  # a step put together without the planner: the general kernels take it
             meta["decode_only"] = False
@@ -147,6 +150,8 @@ class GqaAttention(Part):
         meta.update(plan.facts)
         tiles = plan.arrays.get("tiles")
         meta["segments_dev"] = tiles if tiles is not None and tiles.numel() else None
+        arrivals = plan.arrays.get("arrivals")
+        meta["arrivals"] = arrivals if arrivals is not None and arrivals.numel() else None
         return meta
 
     def forward(self, xb, residual, step, slot, then_norm=None):

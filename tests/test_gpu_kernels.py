@@ -914,6 +914,35 @@ def test_decode_fused(ops, H, Hkv, hd, rot, page, window, gdt):
     assert (again.float() - out3.float()).abs().max() <= 1.2e-2 * max(1.0, float(out3.float().abs().max()))
 
 
+@pytest.mark.parametrize("H,Hkv,ctx,window,split", [(16, 8, (300, 1, 128, 129, 1024), 0, 128), (32, 8, (8000, 17, 5000), 0, 0),
+                                                    (5, 1, (9100, 640), 0, 128), (8, 2, (3000, 700, 129), 300, 128), (64, 8, (2500,) * 9, 0, 0)])
+def test_decode_attention_merged_by_its_last_workgroup(ops, monkeypatch, H, Hkv, ctx, window, split):
+    """The splits of a row merged inside the launch by the workgroup that arrives last: bit for bit what the separate merge
+    gives (same sums in the same order), for rows of one split, of up to eight, of more than eight and more than 64, through a
+    window; over several launches that use the same counters, which are zero after each."""
+    hd, page, R = 128, 16, len(ctx)
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(H + sum(ctx))
+    rnd = lambda *shape: torch.randn(*shape, device=DEV, generator=gen)
+    width = -(-max(ctx) // page)
+    table = torch.randperm(R * width, device=DEV, generator=gen).to(torch.int32).view(R, width)
+    kc, vc = rnd(R * width, Hkv, page, hd).bfloat16(), rnd(R * width, Hkv, page, hd).bfloat16()
+    rows = torch.arange(R, dtype=torch.int32, device=DEV)
+    positions = torch.tensor([c - 1 for c in ctx], dtype=torch.int32, device=DEV)
+    slots = torch.stack([table[r, (c - 1) // page] * page + (c - 1) % page for r, c in enumerate(ctx)]).to(torch.int32)
+    if split:
+        monkeypatch.setattr(ops, "_decode_split", lambda *_: split)
+    arrivals = torch.zeros(R * Hkv, dtype=torch.int32, device=DEV)
+    meta = {"max_context": max(ctx), "decode_only": True, "requests": R}
+    for _ in range(3):
+        qkv = rnd(R, (H + 2 * Hkv) * hd).bfloat16()
+        run = lambda m: ops.decode_attention_fused(qkv, kc, vc, table, rows, positions, slots, None, None, None, None, 1e-6, H, Hkv, hd, 0,
+                                                   window, hd ** -0.5, m)
+        want, got = run(meta), run({**meta, "arrivals": arrivals})
+        assert torch.equal(want.view(torch.int16), got.view(torch.int16)) and not torch.isnan(got.float()).any()
+        assert int(arrivals.abs().max()) == 0
+
+
 def _crafted_cache(ks, vs, table, ctx, page, dtype):
     """A cache tensor pair holding exactly the given keys and values of one request, NaN elsewhere."""
     n_pages = int(table.max()) + 2
