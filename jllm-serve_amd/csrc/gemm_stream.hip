@@ -1,350 +1,415 @@
 // out[M,N] = A[M,K] * W[N,K]^T for 17 to 64 rows (decode steps of many requests, small prompt portions): bf16
 // operands, fp32 accumulation on the matrix cores (16x16x32), bound by streaming W from HBM once.
 //
-// A workgroup of 8 waves owns 128 weight rows and a range of K; wave w owns rows 16 w .. 16 w + 15 and keeps their
-// sums for all the activation rows (up to four 16-row tiles), so nothing is reduced inside the workgroup. The weights
-// go straight from memory into the registers that feed the matrix cores, 16 bytes per lane and load, requested
-// two steps of K ahead (lane l, load j of a 128-wide block: row l%16, k = block * 128 + j * 32 + (l/16) * 8 .. + 8;
-// both operands use this k assignment). The activations, which all 8 waves share, go through LDS: the chunk of
-// the next step is requested before this step's products and stored behind them, one barrier per step. Rows are
-// padded by 16 bytes so that the 16 lanes of a tile row read different banks.
+// A workgroup owns CT tiles of 16 weight rows (gated: half of them gate, half up) and a range of K, with two waves per
+// tile: in a block of 64 k one takes the first 32, the other the rest, each for all the activation rows. Both operands go
+// straight from memory into a ring of S blocks in LDS (global_load_lds_dwordx4, 8 rows of 128 bytes per instruction,
+// bank swizzle applied on the global side), S - 1 blocks ahead of the multiplies; one barrier per block.
 //
-// Products with few column tiles cut K over gridDim.y; each part leaves an fp32 partial [part][matrix][M][N] and
-// a second kernel adds the parts in ascending order and applies bias and epilogue (store, add into the fp32
-// residual, gated with two weights). How K is cut depends on N and K only, never on M: a row's result does not
-// depend on the rows beside it.
+// What binds a compute unit here is its load pipe, through which the activations go as well (about 39 bytes a nanosecond
+// for such loads). So a workgroup should own about as many weight rows as there are activation rows, or more, and where
+// that leaves compute units without one, K is cut over gridDim.y. Each part leaves its sums, with accesses that pass the
+// caches by (common.h), and the workgroup of a column tile that arrives last adds the parts in ascending order and applies
+// bias and epilogue: no second launch. How N and K are cut depends on N and K only, never on M: a row's result does
+// not depend on the rows beside it.
+//
+// Inside a graph, us at 20, 32 and 64 rows, before (fragments of the weights straight from memory a step ahead, 128 rows per
+// workgroup, the parts added by a second launch) / now: 8B shape qkv 19.5 19.9 22.6 / 15.6 16.1 19.6, o 13.6 14.1 16.8 /
+// 12.8 13.5 16.7, gate/up 51.3 53.6 58.1 / 42.8 42.6 43.9, down 28.1 29.1 32.7 / 24.1 24.8 29.1; 0.6B shape qkv 11.4 11.7 13.4 /
+// 7.7 8.0 9.8, o 10.3 10.4 11.7 / 7.6 7.9 9.9, gate/up 17.8 18.1 19.8 / 7.8 7.9 11.2, down 11.0 11.4 12.8 / 8.7 8.9 11.4; a step
+// of 64 requests of the 8B shape 6.47 -> 5.49 ms. A large copy's rate (6.2 TB/s) would take 8.1, 5.4, 32.5 and 16.2 us of the
+// 8B shape's four; the rest is the launch and the first bytes (4), the parts' way through memory (3, 4 and more at 64 rows) and
+// at 64 rows the load pipe.
+//
+// The norm forms are those of the kernel for up to 16 rows: "emit" leaves bf16(new residual * gain) and a sum of squares per
+// workgroup for the norm that follows, "normed" multiplies the sums by rsqrt(sum of the input rows' partial sums of squares
+// / K + eps).
 //
 // Needs K % 128 == 0, N % 16 == 0, M <= 64, 16-byte aligned rows; the caller uses another kernel otherwise.
 #include "common.h"
 #include "mfma.h"
 
-#define GS_WAVES 8
-#define GS_COLS (GS_WAVES * 16)
+#define GS_ROW_BYTES 128  // a row of a block in LDS: 64 k = 8 pieces of 16 bytes
 
-template <int MT, bool GATED>
-__global__ __launch_bounds__(GS_WAVES * 64) void gemm_stream_kernel(
-    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
-    const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N, int K,
-    int epilogue, GateSpec gs, float* __restrict__ partial, int blocks_per_part) {
-  constexpr int UB = GATED ? 1 : 2;            // 128-wide K blocks per step
-  constexpr int LD = UB * 128 + 8;             // LDS row stride in elements
-  constexpr int PIECES = MT * 16 * UB * 16;    // 16-byte pieces of an activation chunk
-  constexpr int PPT = (PIECES + GS_WAVES * 64 - 1) / (GS_WAVES * 64);
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  bf16_t(*As)[MT * 16][LD] = (bf16_t(*)[MT * 16][LD])smem_raw;  // [2][MT * 16][LD]
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int col = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * GS_COLS + wave * 16;
-  const bool live = n0 < N;  // N is a multiple of 16: a wave has all of its rows or none
-  const int nblk = K >> 7;
-  const int b_begin = blockIdx.y * blocks_per_part;
-  const int b_end = min(nblk, b_begin + blocks_per_part);
-  const int steps = (b_end - b_begin + UB - 1) / UB;
-  const bf16_t* wrow = W + (size_t)(live ? n0 + col : 0) * K + g * 8;
-  const bf16_t* urow = GATED ? W2 + (size_t)(live ? n0 + col : 0) * K + g * 8 : nullptr;
-  floatx4 acc[MT], acc2[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    acc[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    acc2[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  }
-  // the blocks of step s are b_begin + s UB .. ; past the end of the range: a harmless reload of its last block,
-  // whose products are skipped
-  auto block_of = [&](int s, int b) { return min(b_begin + s * UB + b, b_end - 1); };
-  u32x4 wv[UB][4], uv[UB][4];
-  auto fetch_w = [&](int s, u32x4 (*w)[4], u32x4 (*u)[4]) {
-#pragma unroll
-    for (int b = 0; b < UB; ++b) {
-      const size_t k = (size_t)block_of(s, b) * 128;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        w[b][j] = *(const u32x4*)(wrow + k + j * 32);
-        if (GATED) u[b][j] = *(const u32x4*)(urow + k + j * 32);
-      }
-    }
-  };
-  // activation chunk of a step: piece q = tid + 512 i: row q / (16 UB), 16 bytes number q % (16 UB)
-  u32x4 areg[PPT];
-  auto fetch_a = [&](int s) {
-#pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-      const int q = tid + GS_WAVES * 64 * i;
-      const int row = q / (16 * UB), pc = q % (16 * UB);
-      areg[i] = u32x4{0u, 0u, 0u, 0u};
-      if (q < PIECES && row < M) {
-        const int blk = block_of(s, pc >> 4);
-        areg[i] = *(const u32x4*)(A + (size_t)row * lda + (size_t)blk * 128 + (pc & 15) * 8);
-      }
-    }
-  };
-  auto store_a = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-      const int q = tid + GS_WAVES * 64 * i;
-      if (q < PIECES) *(u32x4*)(&As[buf][q / (16 * UB)][(q % (16 * UB)) * 8]) = areg[i];
-    }
-  };
-  if (steps > 0) {
-    if (live) fetch_w(0, wv, uv);
-    fetch_a(0);
-    store_a(0);
-  }
-  __syncthreads();
-  for (int s = 0; s < steps; ++s) {
-    const int buf = s & 1;
-    u32x4 wn[UB][4], un[UB][4];
-    if (s + 1 < steps) {
-      if (live) fetch_w(s + 1, wn, un);
-      fetch_a(s + 1);
-    }
-    if (live) {
-#pragma unroll
-      for (int b = 0; b < UB; ++b) {
-        if (b_begin + s * UB + b < b_end) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-              const u32x4 a = *(const u32x4*)(&As[buf][mt * 16 + col][b * 128 + j * 32 + g * 8]);
-              acc[mt] = mfma16(a, wv[b][j], acc[mt]);
-              if (GATED) acc2[mt] = mfma16(a, uv[b][j], acc2[mt]);
-            }
-          }
-        }
-      }
-    }
-    if (s + 1 < steps) store_a(buf ^ 1);
-#pragma unroll
-    for (int b = 0; b < UB; ++b)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        wv[b][j] = wn[b][j];
-        if (GATED) uv[b][j] = un[b][j];
-      }
-    __syncthreads();
-  }
-  if (!live) return;
-  const int n = n0 + col;
-  if (gridDim.y > 1) {  // partial sums [part][matrix][M][N]; the second kernel applies bias and epilogue
-    float* pz = partial + (size_t)blockIdx.y * (GATED ? 2 : 1) * M * N;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = mt * 16 + g * 4 + i;
-        if (m >= M) continue;
-        pz[(size_t)m * N + n] = acc[mt][i];
-        if (GATED) pz[(size_t)M * N + (size_t)m * N + n] = acc2[mt][i];
-      }
-    return;
-  }
-  float b = 0.f;
-  if (bias) b = (bias_dtype == JLLM_BF16) ? ldf((const bf16_t*)bias, n) : ldf((const float*)bias, n);
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = mt * 16 + g * 4 + i;
-      if (m >= M) continue;
-      float v = acc[mt][i] + b;
-      if (GATED) v = gated<false>(v, acc2[mt][i], gs);
-      const size_t o = (size_t)m * ldo + n;
-      if (epilogue == 1)
-        ((float*)out)[o] += v;
-      else if (out_dtype == JLLM_BF16)
-        stf((bf16_t*)out, o, v);
-      else
-        stf((float*)out, o, v);
-    }
-}
-
-// what the reduction needs when an RMSNorm rides on the product (the same two forms as in the kernel for up to 16
-// rows): "emit" leaves bf16(new residual * gain) and the sums of squares per 16 columns for the norm that follows,
-// "normed" multiplies the sums by rsqrt(sum of the input rows' partial sums of squares / K + eps)
 struct StreamNorm {
   bf16_t* emit_rows;
   const void* emit_gain;
   int emit_gain_dtype;
-  float* emit_partial;
+  float* emit_partial;  // [M][emit_parts]: a sum per column tile, zeros behind them
+  int emit_parts;
   const float* norm_partial;
   int norm_parts;
   float norm_eps;
-  int K;
-  GateSpec gate;  // the gate function of the gated epilogue
 };
 
-// adds the K parts in ascending order and applies bias and epilogue; `mats` = 2: gate and up sums side by side.
-// One wave per workgroup, V consecutive outputs per lane (4 when rows allow 16-byte accesses): 64 V outputs, which
-// lie in one row when a norm form is asked for (N is then a multiple of 256). The kernel is a chain of memory
-// latencies, so everything it reads (the norm's partial sums, the residual, up to eight parts at a time) is
-// requested before anything is added.
-template <int V>
-__global__ __launch_bounds__(64) void stream_reduce_kernel(const float* __restrict__ partial, int parts, int mats,
-                                                           const void* __restrict__ bias, int bias_dtype,
-                                                           void* __restrict__ out, int out_dtype, int ldo, int M, int N,
-                                                           int epilogue, StreamNorm nm) {
-  typedef float vec_t __attribute__((ext_vector_type(V)));
-  const size_t i = ((size_t)blockIdx.x * 64 + threadIdx.x) * V;
-  const size_t MN = (size_t)M * N;
-  const bool inside = i < MN;  // N is a multiple of V: the V outputs are inside together
-  const size_t ic = inside ? i : MN - V;
-  const int m = (int)(ic / N), n = (int)(ic % N);
-  const size_t o = (size_t)m * ldo + n;
-  float t = 0.f;
-  if (nm.norm_partial)  // lane l adds the partials l, l + 64, ..., then the wave adds up in a fixed order
-    for (int p = threadIdx.x; p < nm.norm_parts; p += 64) t += nm.norm_partial[(size_t)m * nm.norm_parts + p];
-  vec_t res = 0.f;
-  if (epilogue == 1) res = *(const vec_t*)((const float*)out + o);
-  vec_t v = 0.f, u = 0.f;
-  const size_t zs = (size_t)mats * MN;
-  for (int z0 = 0; z0 < parts; z0 += 8) {
-    vec_t pv[8], pu[8];
-#pragma unroll
-    for (int z = 0; z < 8; ++z) {
-      const size_t at = (size_t)min(z0 + z, parts - 1) * zs + ic;
-      pv[z] = *(const vec_t*)(partial + at);
-      if (mats == 2) pu[z] = *(const vec_t*)(partial + at + MN);
-    }
-#pragma unroll
-    for (int z = 0; z < 8; ++z)
-      if (z0 + z < parts) {
-        v += pv[z];
-        if (mats == 2) u += pu[z];
-      }
-  }
-  float scale = 1.0f;
-  if (nm.norm_partial) scale = 1.0f / sqrtf(wave_sum(t) / (float)nm.K + nm.norm_eps);
-  v *= scale;
-  float r[V];
-#pragma unroll
-  for (int e = 0; e < V; ++e) {
-    float x = v[e];
-    if (bias) x += (bias_dtype == JLLM_BF16) ? ldf((const bf16_t*)bias, n + e) : ldf((const float*)bias, n + e);
-    if (mats == 2) x = gated<false>(x, u[e] * scale, nm.gate);
-    r[e] = x;
-  }
-  if (nm.emit_rows) {  // epilogue 1; the lanes of 16 consecutive columns add their squares (all lanes take part)
-    float sq = 0.f;
-#pragma unroll
-    for (int e = 0; e < V; ++e) {
-      r[e] = inside ? res[e] + r[e] : 0.f;
-      sq += r[e] * r[e];
-    }
-    sq += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, sq), 0xB1, 0xF, 0xF, true));
-    sq += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, sq), 0x4E, 0xF, 0xF, true));
-    if (V == 1) {
-      sq += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, sq), 0x141, 0xF, 0xF, true));
-      sq += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, sq), 0x140, 0xF, 0xF, true));
-    }
-    if (!inside) return;
-#pragma unroll
-    for (int e = 0; e < V; ++e) {
-      const float eg = (nm.emit_gain_dtype == JLLM_BF16) ? ldf((const bf16_t*)nm.emit_gain, n + e) : ldf((const float*)nm.emit_gain, n + e);
-      ((float*)out)[o + e] = r[e];
-      nm.emit_rows[(size_t)m * N + n + e] = f32_to_bf16(r[e] * eg);
-    }
-    if ((n & 15) == 0) nm.emit_partial[(size_t)m * (N >> 4) + (n >> 4)] = sq;
-    return;
-  }
-  if (!inside) return;
-#pragma unroll
-  for (int e = 0; e < V; ++e) {
-    if (epilogue == 1)
-      ((float*)out)[o + e] = res[e] + r[e];
-    else if (out_dtype == JLLM_BF16)
-      stf((bf16_t*)out, o + e, r[e]);
-    else
-      stf((float*)out, o + e, r[e]);
+struct StreamArgs {
+  const bf16_t *A, *W, *W2;
+  const void* bias;
+  void* out;
+  float* partial;  // [column tile][part][tile of 16][tile of 16 rows][lane][4]
+  int* arrivals;   // [column tile], zeros, left as zeros
+  int lda, bias_dtype, out_dtype, ldo, M, N, K, epilogue, blocks_per_part;
+  GateSpec gate;
+  StreamNorm nm;
+};
+
+// The piece of row r in slot s is s ^ gs_swz(r): 16 lanes that read one piece of 16 rows cover the 64 banks once, and so do 8
+// lanes of 8 rows half of them.
+__device__ __forceinline__ int gs_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+
+template <int N>
+__device__ __forceinline__ void gs_wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// until at most n of the wave's loads are in flight (more than that may have landed)
+__device__ __forceinline__ void gs_wait_at_most(int n) {
+  switch (n) {
+    case 0: return gs_wait_loads<0>();
+    case 1: return gs_wait_loads<1>();
+    case 2: return gs_wait_loads<2>();
+    case 3: return gs_wait_loads<3>();
+    case 4: return gs_wait_loads<4>();
+    case 5: return gs_wait_loads<5>();
+    case 6: return gs_wait_loads<6>();
+    case 7: return gs_wait_loads<7>();
+    case 8: return gs_wait_loads<8>();
+    case 9: return gs_wait_loads<9>();
+    case 10: return gs_wait_loads<10>();
+    case 11: return gs_wait_loads<11>();
+    case 12: return gs_wait_loads<12>();
+    case 13: case 14: return gs_wait_loads<13>();
+    case 15: case 16: case 17: return gs_wait_loads<15>();
+    default: return gs_wait_loads<18>();
   }
 }
 
-template <int MT>
-static void launch_stream(dim3 grid, hipStream_t stream, const void* A, int lda, const void* W, const void* W2,
-                          const void* bias, int bias_dtype, void* out, int out_dtype, int ldo, int M, int N, int K,
-                          int epilogue, GateSpec gs, float* partial, int bpp) {
-  const size_t smem_g = (size_t)2 * MT * 16 * (128 + 8) * sizeof(bf16_t), smem_p = (size_t)2 * MT * 16 * (256 + 8) * sizeof(bf16_t);
+// blocks in the ring: one workgroup per compute unit, or two (`shared`); 3 KB stay for what is not the ring
+constexpr int gs_slots(int ct, int mt, bool shared) {
+  const int fit = ((shared ? 80 : 160) - 3) / (2 * ct + 2 * mt);
+  return fit > 8 ? 8 : fit;
+}
+
+template <int CT, int MT, bool GATED, bool SHARED>
+__global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
+  constexpr int NW = 2 * CT;                // waves
+  constexpr int BLOCK = (2 * CT + 2 * MT) * 1024;
+  constexpr int S = gs_slots(CT, MT, SHARED);
+  constexpr int OT = GATED ? CT / 2 : CT;   // tiles of outputs
+  constexpr int AL = (2 * MT + NW - 1) / NW;  // activation loads of a wave, at most
+  constexpr int TPR = CT == 2 ? 4 : 8;        // normed: threads that add up a row's squares
+  static_assert(S >= 3 && (S - 1) * (1 + AL) <= 21 && S * BLOCK >= 2 * CT * MT * 1024, "the ring and what it holds afterwards");
+  extern __shared__ __align__(1024) unsigned char smem[];
+  __shared__ float rs[64];                  // normed: the rows' scales
+  __shared__ float rowsq[OT][64];           // emit: the squares of a row's columns, per tile
+  __shared__ int last;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int col = lane & 15, g = lane >> 4;
+  const int ct = wave >> 1, kg = wave & 1;  // the wave's tile of weight rows and its half of a block
+  const int n0 = blockIdx.x * OT * 16;
+  const int nblk = p.K >> 6;
+  const int b_first = blockIdx.y * p.blocks_per_part;
+  const int total = min(nblk - b_first, p.blocks_per_part);
+  const int parts = gridDim.y;
+  // column tiles walk their range of K from different blocks: with rows a multiple of 4 KB apart, workgroups at the same k
+  // would all ask the same memory channels
+  const int rot = parts == 1 ? (int)((blockIdx.x * 5u) % (unsigned)total) : 0;
+  // normed: thread tid % TPR of row tid / TPR adds up the fours of squares number tid % TPR, + TPR, ...; the first two are
+  // requested before anything else and added up behind the products
+  floatx4 first[2];
+  const int sq_row = tid / TPR, sq_at = tid % TPR;
+  const floatx4* squares = (const floatx4*)(p.nm.norm_partial + (size_t)sq_row * p.nm.norm_parts);
+  const int fours = p.nm.norm_partial && sq_row < p.M ? p.nm.norm_parts >> 2 : 0;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) first[j] = sq_at + j * TPR < fours ? squares[sq_at + j * TPR] : floatx4{0.f, 0.f, 0.f, 0.f};
+  // ---- the loads of a block: 8 weight rows per wave, and 8 activation rows for as many waves as that takes
+  const int lrow = lane >> 3, lslot = lane & 7;
+  const int na = (p.M + 7) >> 3;
+  const int nl = 1 + (na > wave ? (na - wave + NW - 1) / NW : 0);  // the wave's loads per block
+  const int wr = wave * 8 + lrow;                                  // row of the block's weights in LDS
+  const bool up = GATED && wave >= CT;
+  const int wn = min(n0 + (up ? wr - CT * 8 : wr), p.N - 1);
+  const uint32_t wlds = (uint32_t)wave * 1024u;
+  const uint32_t woff = (uint32_t)(wn - min(n0, p.N - 1)) * (uint32_t)p.K * 2u + (uint32_t)((lslot ^ gs_swz(wr)) * 16);
+  const unsigned char* wbase = (const unsigned char*)((up ? p.W2 : p.W) + (size_t)min(n0, p.N - 1) * p.K) + (size_t)b_first * GS_ROW_BYTES;
+  const unsigned char* abase = (const unsigned char*)p.A + (size_t)b_first * GS_ROW_BYTES;
+  uint32_t aoff[AL];
+#pragma unroll
+  for (int c = 0; c < AL; ++c) {
+    const int r = (wave + c * NW) * 8 + lrow;
+    aoff[c] = (uint32_t)min(r, p.M - 1) * (uint32_t)p.lda * 2u + (uint32_t)((lslot ^ gs_swz(r)) * 16);
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+  auto issue = [&](int i, int slot) {
+    const uint32_t at = lds0 + (uint32_t)slot * BLOCK;
+    int b = i + rot;
+    if (b >= total) b -= total;
+    const size_t kbytes = (size_t)b * GS_ROW_BYTES;
+    // m0 holds the LDS address of the 1 KB, lane l's 16 bytes land at m0 + 16 l
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(woff), "s"(wbase + kbytes), "s"(at + wlds) : "memory", "m0");
+#pragma unroll
+    for (int c = 0; c < AL; ++c)
+      if (wave + c * NW < na)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                     :
+                     : "v"(aoff[c]), "s"(abase + kbytes), "s"(at + (uint32_t)(2 * CT + wave + c * NW) * 1024u)
+                     : "memory", "m0");
+  };
+#pragma unroll
+  for (int i = 0; i < S - 1; ++i)
+    if (i < total) issue(i, i);
+  // ---- fragments: lane l reads row l % 16, 8 of k at kg * 32 + (l / 16) * 8: piece 4 kg + l / 16
+  const int foff = col * GS_ROW_BYTES + (((4 * kg + g) ^ gs_swz(col)) << 4);  // + 16 rows leave gs_swz unchanged
+  floatx4 acc[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+  int slot = 0, fill = S - 1;
+  for (int i = 0; i < total; ++i) {
+    // block i: issued, with S - 2 behind it where there are as many; the wave's own loads, then everybody's
+    const int behind = min(S - 2, total - 1 - i);
+    if (behind == S - 2 && nl == 2)
+      gs_wait_loads<2 * (S - 2)>();
+    else if (behind == S - 2 && nl == 1)
+      gs_wait_loads<S - 2>();
+    else
+      gs_wait_at_most(behind * nl);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the reads of block i - 1, whose slot is filled next
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (i + S - 1 < total) issue(i + S - 1, fill);
+    const unsigned char* blk = smem + slot * BLOCK + foff;
+    const u32x4 w = *(const u32x4*)(blk + ct * 2048);
+    u32x4 a[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) a[m] = *(const u32x4*)(blk + (CT + m) * 2048);
+    // the weights as the first operand: a lane then holds four consecutive columns of one row
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[m] = mfma16(w, a[m], acc[m]);
+    fill = slot;
+    if (++slot == S) slot = 0;
+  }
+  if (p.nm.norm_partial) {
+    float t = ((first[0][0] + first[0][1]) + (first[0][2] + first[0][3])) + ((first[1][0] + first[1][1]) + (first[1][2] + first[1][3]));
+    for (int q = sq_at + 2 * TPR; q < fours; q += TPR) {
+      const floatx4 v = squares[q];
+      t += (v[0] + v[1]) + (v[2] + v[3]);
+    }
+#pragma unroll
+    for (int o = 1; o < TPR; o <<= 1) t += __shfl_xor(t, o, 64);
+    if (sq_at == 0 && sq_row < p.M) rs[sq_row] = 1.0f / sqrtf(t / (float)p.K + p.nm.norm_eps);
+  }
+  __syncthreads();  // every wave is done with the ring, which now holds the waves' sums
+  floatx4(*red)[CT][MT][64] = (floatx4(*)[CT][MT][64])smem;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) red[kg][ct][m][lane] = acc[m];
+  __syncthreads();
+  constexpr int ITEMS = CT * MT * 64;       // a tile's 16 rows by 16 columns are 64 items of four columns
+  float* mine = p.partial + ((size_t)blockIdx.x * parts) * ITEMS * 4;
+  if (parts > 1) {
+    for (int idx = tid; idx < ITEMS; idx += NW * 64) {
+      if (((idx >> 6) % MT) * 16 + (idx & 15) >= p.M) continue;
+      const floatx4 v = (&red[0][0][0][0])[idx] + (&red[1][0][0][0])[idx];
+      float* dst = mine + ((size_t)blockIdx.y * ITEMS + idx) * 4;
+      store_shared2(dst, v[0], v[1]);
+      store_shared2(dst + 2, v[2], v[3]);
+    }
+    shared_stores_done();
+    __syncthreads();
+    if (tid == 0) last = arrived_last(p.arrivals + blockIdx.x, parts);
+    __syncthreads();
+    if (!last) return;
+  }
+  // a thread's items (64 lanes of a wave: one tile, one tile of rows): everything they read is requested side by side
+  constexpr int IPT = (OT * MT + NW - 1) / NW, MATS = GATED ? 2 : 1;
+  const bool vec = (p.ldo & 3) == 0 && ((uintptr_t)p.out & 15) == 0;
+  floatx4 prev[IPT], sum[IPT][MATS];
+#pragma unroll
+  for (int it = 0; it < IPT; ++it) {
+    const int idx = tid + it * NW * 64, m = ((idx >> 6) % MT) * 16 + col, n = n0 + (idx >> 6) / MT * 16 + g * 4;
+    prev[it] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (p.epilogue == 1 && idx < OT * MT * 64 && m < p.M && n < p.N) {
+      const float* o = (const float*)p.out + (size_t)m * p.ldo + n;
+      if (vec)
+        prev[it] = *(const floatx4*)o;
+      else
+#pragma unroll
+        for (int i = 0; i < 4; ++i) prev[it][i] = o[i];
+    }
+#pragma unroll
+    for (int u = 0; u < MATS; ++u) sum[it][u] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  if (parts == 1) {
+#pragma unroll
+    for (int it = 0; it < IPT; ++it)
+#pragma unroll
+      for (int u = 0; u < MATS; ++u) {
+        const int idx = min(tid + it * NW * 64, OT * MT * 64 - 1) + u * OT * MT * 64;
+        sum[it][u] = (&red[0][0][0][0])[idx] + (&red[1][0][0][0])[idx];
+      }
+  } else {
+    for (int z0 = 0; z0 < parts; z0 += 4) {  // four parts of every item are requested before any is added
+      floatx4 q[4][IPT][MATS];
+#pragma unroll
+      for (int z = 0; z < 4; ++z)
+#pragma unroll
+        for (int it = 0; it < IPT; ++it)
+#pragma unroll
+          for (int u = 0; u < MATS; ++u) {
+            const int idx = min(tid + it * NW * 64, OT * MT * 64 - 1) + u * OT * MT * 64;
+            const float* src = mine + ((size_t)min(z0 + z, parts - 1) * ITEMS + idx) * 4;
+            float x0 = 0.f, x1 = 0.f, x2 = 0.f, x3 = 0.f;
+            if (((idx >> 6) % MT) * 16 + col < p.M) {
+              load_shared2(src, x0, x1);
+              load_shared2(src + 2, x2, x3);
+            }
+            q[z][it][u] = floatx4{x0, x1, x2, x3};
+          }
+#pragma unroll
+      for (int z = 0; z < 4; ++z)
+        if (z0 + z < parts) {
+#pragma unroll
+          for (int it = 0; it < IPT; ++it)
+#pragma unroll
+            for (int u = 0; u < MATS; ++u) sum[it][u] += q[z][it][u];
+        }
+    }
+  }
+#pragma unroll
+  for (int it = 0; it < IPT; ++it) {
+    const int idx = tid + it * NW * 64;
+    if (idx >= OT * MT * 64) continue;
+    const int t = (idx >> 6) / MT, m = ((idx >> 6) % MT) * 16 + col;
+    const int n = n0 + t * 16 + g * 4;
+    float sq = 0.f;
+    if (m < p.M && n < p.N) {
+      const size_t o = (size_t)m * p.ldo + n;
+      const float scale = p.nm.norm_partial ? rs[m] : 1.0f;
+      float r[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x = sum[it][0][i] * scale;
+        if (p.bias) x += (p.bias_dtype == JLLM_BF16) ? ldf((const bf16_t*)p.bias, n + i) : ldf((const float*)p.bias, n + i);
+        if (GATED) x = gated<false>(x, sum[it][MATS - 1][i] * scale, p.gate);
+        r[i] = prev[it][i] + x;
+        sq += r[i] * r[i];
+      }
+      if (p.nm.emit_rows) {
+        float e[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          e[i] = r[i] * ((p.nm.emit_gain_dtype == JLLM_BF16) ? ldf((const bf16_t*)p.nm.emit_gain, n + i) : ldf((const float*)p.nm.emit_gain, n + i));
+        *(u32x2*)(p.nm.emit_rows + (size_t)m * p.N + n) = u32x2{pack_bf16(e[0], e[1]), pack_bf16(e[2], e[3])};
+      }
+      if (p.out_dtype == JLLM_BF16) {
+        if (vec)
+          *(u32x2*)((bf16_t*)p.out + o) = u32x2{pack_bf16(r[0], r[1]), pack_bf16(r[2], r[3])};
+        else
+#pragma unroll
+          for (int i = 0; i < 4; ++i) stf((bf16_t*)p.out, o + i, r[i]);
+      } else {
+        if (vec)
+          *(floatx4*)((float*)p.out + o) = floatx4{r[0], r[1], r[2], r[3]};
+        else
+#pragma unroll
+          for (int i = 0; i < 4; ++i) ((float*)p.out)[o + i] = r[i];
+      }
+    }
+    if (p.nm.emit_rows) {  // over the lanes of one row
+      sq += __shfl_xor(sq, 16, 64);
+      sq += __shfl_xor(sq, 32, 64);
+      if (g == 0) rowsq[t][m] = sq;
+    }
+  }
+  if (p.nm.emit_rows) {
+    __syncthreads();
+    const int spare = p.nm.emit_parts - (int)gridDim.x;
+    for (int m = tid; m < p.M; m += NW * 64) {
+      float t = 0.f;
+#pragma unroll
+      for (int c = 0; c < OT; ++c) t += rowsq[c][m];
+      float* dst = p.nm.emit_partial + (size_t)m * p.nm.emit_parts;
+      dst[blockIdx.x] = t;
+      for (int z = blockIdx.x; z < spare; z += gridDim.x) dst[gridDim.x + z] = 0.f;
+    }
+  }
+}
+
+template <int CT, int MT, bool GATED, bool SHARED>
+static int launch_stream(const StreamArgs& a, dim3 grid, hipStream_t stream) {
+  constexpr size_t smem = (size_t)gs_slots(CT, MT, SHARED) * (2 * CT + 2 * MT) * 1024;
   static bool configured = false;
   if (!configured) {  // above 64 KB the size has to be allowed first
-    (void)hipFuncSetAttribute((const void*)gemm_stream_kernel<MT, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_g);
-    (void)hipFuncSetAttribute((const void*)gemm_stream_kernel<MT, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_p);
+    if (hipFuncSetAttribute((const void*)gemm_stream_kernel<CT, MT, GATED, SHARED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+      JLLM_FAIL("gemm_stream: cannot reserve %zu bytes of LDS", smem);
     configured = true;
   }
-  if (W2)
-    gemm_stream_kernel<MT, true><<<grid, GS_WAVES * 64, smem_g, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W,
-                                                                          (const bf16_t*)W2, bias, bias_dtype, out,
-                                                                          out_dtype, ldo, M, N, K, epilogue, gs, partial, bpp);
-  else
-    gemm_stream_kernel<MT, false><<<grid, GS_WAVES * 64, smem_p, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W,
-                                                                           nullptr, bias, bias_dtype, out, out_dtype, ldo,
-                                                                           M, N, K, epilogue, gs, partial, bpp);
-}
-
-static int stream_checked(const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype,
-                          void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue, float gate_limit, int parts, float* partial,
-                          const StreamNorm& nm_in, hipStream_t stream) {
-  if (M <= 0 || N <= 0) return 0;
-  if (M > 64 || (K & 127) || (N & 15) || (lda & 7) || K <= 0) return 1;
-  if (((uintptr_t)A & 15) || ((uintptr_t)W & 15) || (W2 && ((uintptr_t)W2 & 15))) return 1;
-  JLLM_TAKE_GATE("gemm_stream", epilogue, gate_limit, gs);
-  StreamNorm nm = nm_in;
-  nm.gate = gs;
-  if (epilogue < 0 || epilogue > 2 || (epilogue == 2) != (W2 != nullptr)) JLLM_FAIL("gemm_stream: epilogue %d", epilogue);
-  if (epilogue == 1 && out_dtype != JLLM_F32) JLLM_FAIL("gemm_stream: the accumulate epilogue adds into fp32");
-  if (ldo < N) JLLM_FAIL("gemm_stream: ldo %d < N %d", ldo, N);
-  const int nblk = K >> 7;
-  if (parts < 1) parts = 1;
-  if (parts > nblk) parts = nblk;
-  if (parts > 1 && !partial) JLLM_FAIL("gemm_stream: %d parts of K need a buffer for the partial sums", parts);
-  const int ub = W2 ? 1 : 2;
-  int bpp = (nblk + parts - 1) / parts;
-  bpp = (bpp + ub - 1) / ub * ub;           // whole steps
-  const int used = (nblk + bpp - 1) / bpp;  // parts that have any block
-  const bool with_norm = nm.emit_rows || nm.norm_partial;
-  if (with_norm) {  // the norm forms live in the reduction kernel, one output row per workgroup
-    if (used < 2 || (N & 255)) return 1;
-    if (nm.emit_rows && (epilogue != 1 || !nm.emit_gain || !nm.emit_partial)) JLLM_FAIL("gemm_stream: rows for a norm come from the accumulate epilogue, with gain and partial sums");
-    if (nm.norm_partial && nm.norm_parts <= 0) JLLM_FAIL("gemm_stream: %d partial sums", nm.norm_parts);
-  }
-  dim3 grid((N + GS_COLS - 1) / GS_COLS, used);
-  if (grid.y > 65535) return 1;
-  switch ((M + 15) / 16) {
-    case 1: launch_stream<1>(grid, stream, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, bpp); break;
-    case 2: launch_stream<2>(grid, stream, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, bpp); break;
-    case 3: launch_stream<3>(grid, stream, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, bpp); break;
-    default: launch_stream<4>(grid, stream, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, bpp); break;
-  }
+  gemm_stream_kernel<CT, MT, GATED, SHARED><<<grid, CT * 128, smem, stream>>>(a);
   JLLM_CHECK_LAUNCH("gemm_stream");
-  if (used > 1) {
-    const size_t total = (size_t)M * N;
-    const bool wide = !(N & 3) && !(ldo & 3) && !((uintptr_t)out & 15) && !((uintptr_t)partial & 15);
-    if (wide)
-      stream_reduce_kernel<4><<<(unsigned)((total / 4 + 63) / 64), 64, 0, stream>>>(partial, used, W2 ? 2 : 1, bias, bias_dtype,
-                                                                                  out, out_dtype, ldo, M, N, epilogue, nm);
-    else
-      stream_reduce_kernel<1><<<(unsigned)((total + 63) / 64), 64, 0, stream>>>(partial, used, W2 ? 2 : 1, bias, bias_dtype,
-                                                                              out, out_dtype, ldo, M, N, epilogue, nm);
-    JLLM_CHECK_LAUNCH("gemm_stream_reduce");
-  }
   return 0;
 }
 
-// `parts` > 1 cuts K over gridDim.y; `partial` then holds parts * (W2 ? 2 : 1) * M * N floats.
+template <int CT, bool GATED>
+static int launch_stream_rows(const StreamArgs& a, dim3 grid, bool shared, hipStream_t stream) {
+#define GS_CASE(MT)                                                       \
+  case MT:                                                                \
+    return shared ? launch_stream<CT, MT, GATED, true>(a, grid, stream) : launch_stream<CT, MT, GATED, false>(a, grid, stream);
+  switch ((a.M + 15) / 16) {
+    GS_CASE(1) GS_CASE(2) GS_CASE(3)
+    default: return shared ? launch_stream<CT, 4, GATED, true>(a, grid, stream) : launch_stream<CT, 4, GATED, false>(a, grid, stream);
+  }
+#undef GS_CASE
+}
+
+// `rows`: weight rows per workgroup, both weights' of the gated epilogue together (32, 64, 96 or 128). `parts` > 1 cuts K over
+// gridDim.y in whole blocks of 128; `partial` then holds parts * column tiles * rows * 16 * ceil(M / 16) floats and `arrivals`
+// one int per column tile, zeros, left as zeros. An RMSNorm on either side as in jllm_gemm_skinny_norm_bf16.
 // returns 0 when it ran, 1 when the shape is not one it takes (the caller uses another kernel), -1 on errors
 extern "C" int jllm_gemm_stream_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias,
                                      int bias_dtype, void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue,
-                                     float gate_limit, int parts, float* partial, hipStream_t stream) {
-  return stream_checked(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gate_limit, parts, partial, StreamNorm{},
-                        stream);
-}
-
-// The same with an RMSNorm on either side (the forms of jllm_gemm_skinny_norm_bf16); needs K in at least two parts
-// and N % 256 == 0, declines otherwise.
-extern "C" int jllm_gemm_stream_norm_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias,
-                                          int bias_dtype, void* out, int out_dtype, int ldo, int M, int N, int K,
-                                          int epilogue, float gate_limit, int parts, float* partial, void* emit_rows, const void* emit_gain,
-                                          int emit_gain_dtype, float* emit_partial, const float* norm_partial,
-                                          int norm_parts, float norm_eps, hipStream_t stream) {
-  StreamNorm nm{(bf16_t*)emit_rows, emit_gain, emit_gain_dtype, emit_partial, norm_partial, norm_parts, norm_eps, K, GateSpec{0, 0.f}};
-  return stream_checked(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gate_limit, parts, partial, nm, stream);
+                                     float gate_limit, int rows, int parts, float* partial, int* arrivals, void* emit_rows,
+                                     const void* emit_gain, int emit_gain_dtype, float* emit_partial, int emit_parts,
+                                     const float* norm_partial, int norm_parts, float norm_eps, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (M > 64 || (K & 127) || (N & 15) || (lda & 7) || K <= 0 || lda < 0) return 1;
+  if (((uintptr_t)A & 15) || ((uintptr_t)W & 15) || (W2 && ((uintptr_t)W2 & 15))) return 1;
+  // a lane's place in an operand is a 32-bit byte offset from the workgroup's first row
+  if ((unsigned long long)lda >= (1ull << 24) || (unsigned long long)K >= (1ull << 23)) return 1;
+  JLLM_TAKE_GATE("gemm_stream", epilogue, gate_limit, gs);
+  if (epilogue < 0 || epilogue > 2 || (epilogue == 2) != (W2 != nullptr)) JLLM_FAIL("gemm_stream: epilogue %d", epilogue);
+  if (epilogue == 1 && out_dtype != JLLM_F32) JLLM_FAIL("gemm_stream: the accumulate epilogue adds into fp32");
+  if (ldo < N) JLLM_FAIL("gemm_stream: ldo %d < N %d", ldo, N);
+  if (rows != 32 && rows != 64 && rows != 96 && rows != 128) JLLM_FAIL("gemm_stream: %d weight rows per workgroup (32, 64, 96, 128)", rows);
+  const int cols = W2 ? rows / 2 : rows;
+  const int tiles = (N + cols - 1) / cols;
+  const int nblk = K >> 7;
+  if (parts < 1) parts = 1;
+  if (parts > nblk) parts = nblk;
+  const int bpp = (nblk + parts - 1) / parts;
+  const int used = (nblk + bpp - 1) / bpp;  // parts that have any block
+  if (used > 1 && (!partial || !arrivals || ((uintptr_t)partial & 15))) JLLM_FAIL("gemm_stream: %d parts of K need a buffer for their sums and counters", used);
+  if (emit_rows && (epilogue != 1 || !emit_gain || !emit_partial)) JLLM_FAIL("gemm_stream: rows for a norm come from the accumulate epilogue, with gain and partial sums");
+  if (emit_rows && emit_parts < tiles) JLLM_FAIL("gemm_stream: %d places for the partial sums of %d workgroups", emit_parts, tiles);
+  if (norm_partial && norm_parts <= 0) JLLM_FAIL("gemm_stream: %d partial sums", norm_parts);
+  if (norm_partial && ((norm_parts & 3) || ((uintptr_t)norm_partial & 15))) return 1;
+  const int cus = jllm_compute_units();
+  if (cus <= 0) JLLM_FAIL("gemm_stream: the GPU's compute units could not be read");
+  dim3 grid(tiles, used);
+  if (grid.y > 65535) return 1;
+  const StreamArgs a{(const bf16_t*)A, (const bf16_t*)W, (const bf16_t*)W2, bias, out, partial, arrivals, lda, bias_dtype, out_dtype, ldo, M, N, K,
+                     epilogue, bpp * 2, gs, StreamNorm{(bf16_t*)emit_rows, emit_gain, emit_gain_dtype, emit_partial, emit_parts, norm_partial, norm_parts, norm_eps}};
+  // two workgroups share a compute unit where there are more of them than compute units: one streams while the other adds up
+  const bool shared = (long)tiles * used > cus;
+  if (W2) switch (rows) {
+      case 32: return launch_stream_rows<2, true>(a, grid, shared, stream);
+      case 64: return launch_stream_rows<4, true>(a, grid, shared, stream);
+      case 96: return launch_stream_rows<6, true>(a, grid, shared, stream);
+      default: return launch_stream_rows<8, true>(a, grid, shared, stream);
+    }
+  switch (rows) {
+    case 32: return launch_stream_rows<2, false>(a, grid, shared, stream);
+    case 64: return launch_stream_rows<4, false>(a, grid, shared, stream);
+    case 96: return launch_stream_rows<6, false>(a, grid, shared, stream);
+    default: return launch_stream_rows<8, false>(a, grid, shared, stream);
+  }
 }

@@ -7,6 +7,7 @@ the GPU, they raise.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import functools
 import threading
@@ -117,8 +118,7 @@ _OPTIONAL_SIGS = {
     "jllm_gemm_skinny_norm_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _P, _I, _P, _I, _F, _P],
     "jllm_gemm_mfma_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P],
     "jllm_gemm_pingpong_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P, _P],
-    "jllm_gemm_stream_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P],
-    "jllm_gemm_stream_norm_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _P, _I, _P, _P, _I, _F, _P],
+    "jllm_gemm_stream_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P, _P, _P, _P, _I, _P, _I, _P, _I, _F, _P],
     "jllm_decode_attention_bf16": [_P, _I, _P, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _I, _P],
     "jllm_decode_attention_fused_bf16": [_P, _I, _P, _I, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _F, _I, _I, _I, _I, _I,
                                          _I, _I, _I, _F, _I, _P, _P, _I, _I, _P, _P],
@@ -397,12 +397,11 @@ def _skinny_norm(a, w, w2, bias, out, epilogue, emit=None, normed: Optional[Norm
     emit_parts = e_part.shape[1] if e_part is not None else 0
     if few and not _few_rows_prefer_stream(N, K, w2 is not None):
         return _try("jllm_gemm_skinny_norm_bf16", *head, _skinny_rows(N, K, w2 is not None), *emits, emit_parts, *takes)
-    parts = _stream_parts(N, K, w2 is not None) if K % 128 == 0 else 0
-    if parts >= 2:
-        partial = torch.empty((parts * (2 if w2 is not None else 1) * M * N,), dtype=torch.float32, device=a.device)
-        if _try("jllm_gemm_stream_norm_bf16", *head, parts, _ptr(partial), *emits, *takes):
+    if K % 128 == 0:
+        rows, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a)
+        if _try("jllm_gemm_stream_bf16", *head, rows, parts, _ptr(sums), _ptr(arrivals), *emits, emit_parts, *takes):
             return True
-    return few and _try("jllm_gemm_skinny_norm_bf16", *head, 16, *emits, emit_parts, *takes)  # the second kernel declined (N % 256, one part)
+    return few and _try("jllm_gemm_skinny_norm_bf16", *head, 16, *emits, emit_parts, *takes)  # the second kernel declined
 
 
 def gemm_add_then_norm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gain: torch.Tensor, eps: float,
@@ -709,14 +708,11 @@ STREAM_MIN_BLOCKS = 4           # 128-wide K blocks a part has at least
 
 @functools.lru_cache(maxsize=None)
 def _stream_parts(N: int, K: int, gated: bool) -> int:
-    """How many ways the second weight-streaming kernel cuts K, from N and K alone (never from the number of rows:
-    a row's sum must not depend on its batch). A compute unit streams about as fast with one workgroup as with
-    two, so what counts is the largest number of workgroups any compute unit gets: the count that minimises
-    ceil(workgroups / compute units) / workgroups, times a small price per part. Any count goes, not only powers
-    of two. Against a sweep of every count on the four products of the 8B, 14B and 32B shapes at 32 and 64 rows this
-    choice is 1 % from the best on average (6 % at worst); doubling up to a target was 10 % (down product of the 14B
-    shape: 8 parts, 320 workgroups, 54.9 us; 6 parts 47.2; gate/up: 4 parts, 544 workgroups, 99.1 us; 5 parts
-    88.1)."""
+    """How many ways the second weight-streaming kernel may cut K for a product of ceil(N / 128) column tiles, from N and K
+    alone (never from the number of rows: a row's sum must not depend on its batch; `_stream_plan` asks with the tiles that
+    its workgroups have). A compute unit streams about as fast with one workgroup as with two, so what counts is the largest
+    number of workgroups any compute unit gets: the count that minimises ceil(workgroups / compute units) / workgroups, times
+    a small price per part. Any count goes, not only powers of two."""
     tiles = -(-N // 128)
     nblk = K // 128
     step = 1 if gated else 2
@@ -785,12 +781,73 @@ def _skinny_rows(N: int, K: int, gated: bool) -> int:
 
 
 def _norm_partials(M: int, N: int, K: int) -> int:
-    """Partial sums of squares per row that a product with N outputs leaves for the norm behind it: one per 16 columns
-    (the kernel for 17 to 64 rows, and the least that the first one is given), or one per workgroup of the first one,
-    in whole fours."""
+    """Partial sums of squares per row that a product with N outputs leaves for the norm behind it: room for one per
+    workgroup's columns, in whole fours."""
     if M > SKINNY_MAX_ROWS or _few_rows_prefer_stream(N, K, False):
-        return N // 16
-    return max(N // 16, -(-(-(-N // _skinny_rows(N, K, False))) // 4) * 4)
+        groups = max(N // 16, -(-N // _stream_plan(N, K, False)[0])) if M <= SKINNY_MAX_ROWS else -(-N // _stream_plan(N, K, False)[0])
+    else:
+        groups = -(-N // _skinny_rows(N, K, False))
+    return -(-groups // 4) * 4
+
+
+STREAM_NS_PER_KB = 26.0    # what a compute unit's load pipe takes for 1 KB of weights or activations
+STREAM_MERGE_NS = 1500     # the last workgroup of a column tile: its way through memory ...
+STREAM_SUM_NS_PER_KB = 60  # ... and for 1 KB of sums
+STREAM_PRICED_ROWS = 40
+
+
+@functools.lru_cache(maxsize=None)
+def _stream_plan(N: int, K: int, gated: bool) -> Tuple[int, int]:
+    """(weight rows per workgroup, ways K is cut) of the second weight-streaming kernel, from N and K alone (priced at 40
+    rows). More rows per workgroup share the activations' way into a compute unit, fewer leave more workgroups; parts of K
+    fill what N leaves empty and cost the last workgroup their sums."""
+    cus = compute_units()
+    best, plan = None, (64, 1)
+    for rows in (32, 64, 96, 128):
+        tiles = -(-N // (rows // 2 if gated else rows))
+        for parts in {1, _stream_parts(tiles * 128, K, gated)}:
+            per = -(-(K // 128) // parts) * 128
+            t = -(-tiles * parts // cus) * (rows + STREAM_PRICED_ROWS) * per * 2 / 1024 * STREAM_NS_PER_KB
+            if parts > 1:
+                t += STREAM_MERGE_NS + parts * STREAM_PRICED_ROWS * rows * 4 / 1024 * STREAM_SUM_NS_PER_KB
+            if best is None or t < best:
+                best, plan = t, (rows, parts)
+    return plan
+
+
+_step_scratch = threading.local()  # what a step's products share, see `step_scratch`
+
+
+@contextlib.contextmanager
+def step_scratch(rows: int, device):
+    """Around the launches of one step of ``rows`` rows in one stream: zeroed counters that its products of few rows, which
+    follow each other, take turns in (each leaves them zero). Without them every such product clears counters of its own, as
+    the rare ones do that reach the second kernel with up to 16 rows."""
+    if not SKINNY_MAX_ROWS < rows <= STREAM_MAX_ROWS or device.type != "cuda":
+        yield
+        return
+    before = getattr(_step_scratch, "arrivals", None)
+    _step_scratch.arrivals = (torch.empty(STREAM_COUNTERS, dtype=torch.int32, device=device).zero_(), _stream())
+    try:
+        yield
+    finally:
+        _step_scratch.arrivals = before
+
+
+STREAM_COUNTERS = 1024
+
+
+def _stream_scratch(M: int, N: int, K: int, gated: bool, a: torch.Tensor):
+    """The second weight-streaming kernel's plan and scratch: (rows, parts, sums, counters)."""
+    rows, parts = _stream_plan(N, K, gated)
+    if parts == 1:
+        return rows, 1, None, None
+    tiles = -(-N // (rows // 2 if gated else rows))
+    partial = torch.empty((parts * tiles * rows * 16 * -(-M // 16),), dtype=torch.float32, device=a.device)
+    arrivals, stream = getattr(_step_scratch, "arrivals", None) or (None, None)
+    if arrivals is None or arrivals.device != a.device or arrivals.numel() < tiles or stream != _stream():
+        arrivals = torch.empty(tiles, dtype=torch.int32, device=a.device).zero_()
+    return rows, parts, partial, arrivals
 
 
 STREAM_FEW_ROWS = (1280, 8192)   # columns at most, K at least: see `_few_rows_prefer_stream`
@@ -821,10 +878,8 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0) -> bool:
             and _try("jllm_gemm_skinny_bf16", *head, _skinny_rows(N, K, w2 is not None), _stream()):
         return True
     if M <= STREAM_MAX_ROWS and K % 128 == 0:
-        parts = _stream_parts(N, K, w2 is not None)
-        partial = torch.empty((parts * (2 if w2 is not None else 1) * M * N,), dtype=torch.float32, device=a.device) \
-            if parts > 1 else None
-        if _try("jllm_gemm_stream_bf16", *head, parts, _ptr(partial), _stream()):
+        rows, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a)
+        if _try("jllm_gemm_stream_bf16", *head, rows, parts, _ptr(sums), _ptr(arrivals), None, None, F32, None, 0, None, 0, 0.0, _stream()):
             return True
     tile_rows, cut = _tiled_plan(M, N, K, w2 is not None)
     if tile_rows:

@@ -127,6 +127,10 @@ class DecoderModel:
 
     def forward(self, step, slots) -> torch.Tensor:
         """Runs the step's rows through the schedule; returns fp32 logits [len(step.selected), vocab]."""
+        with ops.step_scratch(step.n_tokens, self.device):
+            return self._forward(step, slots)
+
+    def _forward(self, step, slots) -> torch.Tensor:
         x = ops.embed(self.embed, step.token_ids, self.config.embed_scale)
         for p in self.positions:  # an encoding that is added to the embedded rows rather than applied in the mixers
             if hasattr(p, "embed_add"):

@@ -312,6 +312,46 @@ def test_few_row_products_at_any_weight_rows_per_workgroup(ops, monkeypatch, M, 
     assert torch.equal(out, ops.gemm(a, w, bias=bias, out_dtype=torch.float32))
 
 
+@pytest.mark.parametrize("rows", [32, 64, 96, 128])
+@pytest.mark.parametrize("M,N,K,parts", [(17, 160, 128, 1), (33, 1040, 640, 2), (64, 2064, 1152, 3), (1, 336, 2560, 6), (48, 4112, 256, 1),
+                                         (25, 9728, 384, 1), (64, 192, 4096, 8)])
+def test_products_of_17_to_64_rows_at_any_plan(ops, monkeypatch, M, N, K, rows, parts):
+    """The kernel for 17 to 64 rows at every number of weight rows per workgroup: last column tiles with fewer columns than
+    the others, ranges of K shorter than the ring and of unequal length, one to four tiles of rows, one workgroup a compute
+    unit and two. Against float64 within the bound of an fp32 sum of K products in any order; a row's bits are the same alone as
+    among the others, in the step's shared counters as in counters of its own; the rows for a norm are exactly what
+    the new residual gives."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M * N + K + rows)
+    rnd = lambda *shape: torch.randn(*shape, device=DEV, generator=gen)
+    a, w, w2 = rnd(M, K).bfloat16(), (rnd(N, K) / math.sqrt(K)).bfloat16(), (rnd(N, K) / math.sqrt(K)).bfloat16()
+    bias, gain, res0 = rnd(N), rnd(N).abs() + 0.5, rnd(M, N)
+    monkeypatch.setattr(ops, "_few_rows_prefer_stream", lambda *_: True)
+    monkeypatch.setattr(ops, "_stream_plan", lambda *_: (rows, parts))
+    ops.reset_stats()
+    exact, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    bound = 2 * K * 2.0 ** -24 * size + 1e-6
+    out = ops.gemm(a, w, bias=bias, out_dtype=torch.float32)
+    assert bool(((out.double() - exact - bias.double()).abs() <= bound + 2.0 ** -23 * (exact.abs() + bias.abs())).all())
+    res = res0.clone()
+    with ops.step_scratch(M, a.device):
+        for _ in range(2):  # the second launch finds the counters as the first one left them
+            res = res0.clone()
+            promise = ops.gemm_add_then_norm(a, w, res, gain, 1e-3, torch.bfloat16)
+    assert bool(((res.double() - exact - res0.double()).abs() <= bound + 2.0 ** -23 * (exact.abs() + res0.abs())).all())
+    assert torch.equal(promise.scaled, (res * gain).bfloat16())
+    want = (res.double() ** 2).sum(-1)
+    assert bool(((promise.partials.double().sum(-1) - want).abs() <= 128 * 2.0 ** -24 * want).all())
+    gated = ops.gemm(a, w, w2=w2, epilogue=ops.EPI_GATED, out_dtype=torch.float32)
+    up = a.double() @ w2.double().T
+    both = bound * (1.1 * up.abs() + 1) + 2 * K * 2.0 ** -24 * (a.double().abs() @ w2.double().abs().T) * exact.abs() + 1e-5 * (exact * up).abs()
+    assert bool(((gated.double() - torch.nn.functional.silu(exact) * up).abs() <= both).all())
+    for r in {0, M // 2, M - 1}:
+        assert torch.equal(ops.gemm(a[r:r + 1].contiguous(), w, bias=bias, out_dtype=torch.float32), out[r:r + 1])
+        assert torch.equal(ops.gemm(a[r:r + 1].contiguous(), w, w2=w2, epilogue=ops.EPI_GATED, out_dtype=torch.float32), gated[r:r + 1])
+    assert set(ops.stats()["ran"]) == {"jllm_gemm_stream_bf16"}
+
+
 def test_gemm_rows_do_not_depend_on_the_batch(ops):
     """The result of a row is the same bits whether it is alone or among others, within one kernel family (the
     bfloat16 path has one kernel for up to 16 rows, one for up to 64 and one for more; between them results differ
