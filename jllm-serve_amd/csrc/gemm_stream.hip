@@ -1,5 +1,6 @@
-// out[M,N] = A[M,K] * W[N,K]^T for 17 to 64 rows (decode steps of many requests, small prompt portions): bf16
-// operands, fp32 accumulation on the matrix cores (16x16x32), bound by streaming W from HBM once.
+// out[M,N] = A[M,K] * W[N,K]^T for 17 to 64 rows (decode steps of many requests, small prompt portions), bound by streaming W
+// from HBM once, and for the smaller products of up to about a thousand (gridDim.z tiles of 64 or 128 rows): bf16 operands,
+// fp32 accumulation on the matrix cores (16x16x32).
 //
 // A workgroup owns CT tiles of 16 weight rows (gated: half of them gate, half up) and a range of K, with two waves per
 // tile: in a block of 64 k one takes the first 32, the other the rest, each for all the activation rows. Both operands go
@@ -25,7 +26,7 @@
 // workgroup for the norm that follows, "normed" multiplies the sums by rsqrt(sum of the input rows' partial sums of squares
 // / K + eps).
 //
-// Needs K % 128 == 0, N % 16 == 0, M <= 64, 16-byte aligned rows; the caller uses another kernel otherwise.
+// Needs K % 128 == 0, N % 16 == 0, 16-byte aligned rows; the caller uses another kernel otherwise.
 #include "common.h"
 #include "mfma.h"
 
@@ -33,6 +34,7 @@
 
 struct StreamNorm {
   bf16_t* emit_rows;
+  int emit_ld;
   const void* emit_gain;
   int emit_gain_dtype;
   float* emit_partial;  // [M][emit_parts]: a sum per column tile, zeros behind them
@@ -48,7 +50,7 @@ struct StreamArgs {
   void* out;
   float* partial;  // [column tile][part][tile of 16][tile of 16 rows][lane][4]
   int* arrivals;   // [column tile], zeros, left as zeros
-  int lda, bias_dtype, out_dtype, ldo, M, N, K, epilogue, blocks_per_part;
+  int lda, bias_dtype, out_dtype, ldo, M, N, K, epilogue, blocks_per_part, turn;
   GateSpec gate;
   StreamNorm nm;
 };
@@ -83,9 +85,9 @@ __device__ __forceinline__ void gs_wait_at_most(int n) {
   }
 }
 
-// blocks in the ring: one workgroup per compute unit, or two (`shared`); 3 KB stay for what is not the ring
+// blocks in the ring: one workgroup per compute unit, or two (`shared`); 3 KB (5 for more rows) stay for what is not the ring
 constexpr int gs_slots(int ct, int mt, bool shared) {
-  const int fit = ((shared ? 80 : 160) - 3) / (2 * ct + 2 * mt);
+  const int fit = ((shared ? 80 : 160) - (mt > 4 ? 5 : 3)) / (2 * ct + 2 * mt);
   return fit > 8 ? 8 : fit;
 }
 
@@ -96,11 +98,12 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
   constexpr int S = gs_slots(CT, MT, SHARED);
   constexpr int OT = GATED ? CT / 2 : CT;   // tiles of outputs
   constexpr int AL = (2 * MT + NW - 1) / NW;  // activation loads of a wave, at most
-  constexpr int TPR = CT == 2 ? 4 : 8;        // normed: threads that add up a row's squares
-  static_assert(S >= 3 && (S - 1) * (1 + AL) <= 21 && S * BLOCK >= 2 * CT * MT * 1024, "the ring and what it holds afterwards");
+  constexpr int MAX_ROWS = MT > 4 ? 128 : 64;
+  constexpr int TPR = (CT == 2 ? 4 : 8) * 64 / MAX_ROWS;  // normed: threads that add up a row's squares
+  static_assert(S >= 3 && (S - 1) * (1 + AL) < 63 && S * BLOCK >= 2 * CT * MT * 1024, "the ring and what it holds afterwards");
   extern __shared__ __align__(1024) unsigned char smem[];
-  __shared__ float rs[64];                  // normed: the rows' scales
-  __shared__ float rowsq[OT][64];           // emit: the squares of a row's columns, per tile
+  __shared__ float rs[MAX_ROWS];            // normed: the rows' scales
+  __shared__ float rowsq[OT][MAX_ROWS];     // emit: the squares of a row's columns, per tile
   __shared__ int last;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -111,9 +114,22 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
   const int b_first = blockIdx.y * p.blocks_per_part;
   const int total = min(nblk - b_first, p.blocks_per_part);
   const int parts = gridDim.y;
-  // column tiles walk their range of K from different blocks: with rows a multiple of 4 KB apart, workgroups at the same k
-  // would all ask the same memory channels
-  const int rot = parts == 1 ? (int)((blockIdx.x * 5u) % (unsigned)total) : 0;
+  {  // the workgroup's rows
+    const int m0 = blockIdx.z * MT * 16;
+    p.M = min(p.M - m0, MT * 16);
+    p.A += (size_t)m0 * p.lda;
+    p.out = p.out_dtype == JLLM_BF16 ? (void*)((bf16_t*)p.out + (size_t)m0 * p.ldo) : (void*)((float*)p.out + (size_t)m0 * p.ldo);
+    if (p.nm.norm_partial) p.nm.norm_partial += (size_t)m0 * p.nm.norm_parts;
+    if (p.nm.emit_rows) {
+      p.nm.emit_rows += (size_t)m0 * p.nm.emit_ld;
+      p.nm.emit_partial += (size_t)m0 * p.nm.emit_parts;
+    }
+  }
+  const size_t tile = blockIdx.x + (size_t)gridDim.x * blockIdx.z;
+  // up to 64 rows and K whole: column tiles walk K from different blocks, so that workgroups do not all ask the same memory
+  // channels at once (rows are often a multiple of 4 KB apart; 8B gate/up at 20 rows 45.5 -> 43.3 us; with parts of K the same
+  // or 1 us slower, and for more rows an output's bits would follow the choice of tiles)
+  const int rot = p.turn ? (int)((blockIdx.x * 5u) % (unsigned)total) : 0;
   // normed: thread tid % TPR of row tid / TPR adds up the fours of squares number tid % TPR, + TPR, ...; the first two are
   // requested before anything else and added up behind the products
   floatx4 first[2];
@@ -167,10 +183,10 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
   for (int i = 0; i < total; ++i) {
     // block i: issued, with S - 2 behind it where there are as many; the wave's own loads, then everybody's
     const int behind = min(S - 2, total - 1 - i);
-    if (behind == S - 2 && nl == 2)
-      gs_wait_loads<2 * (S - 2)>();
-    else if (behind == S - 2 && nl == 1)
-      gs_wait_loads<S - 2>();
+    if (behind == S - 2 && nl == 1 + AL)
+      gs_wait_loads<(1 + AL) * (S - 2)>();
+    else if (behind == S - 2 && nl == AL)
+      gs_wait_loads<AL * (S - 2)>();
     else
       gs_wait_at_most(behind * nl);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the reads of block i - 1, whose slot is filled next
@@ -205,7 +221,7 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
   for (int m = 0; m < MT; ++m) red[kg][ct][m][lane] = acc[m];
   __syncthreads();
   constexpr int ITEMS = CT * MT * 64;       // a tile's 16 rows by 16 columns are 64 items of four columns
-  float* mine = p.partial + ((size_t)blockIdx.x * parts) * ITEMS * 4;
+  float* mine = p.partial + tile * parts * ITEMS * 4;
   if (parts > 1) {
     for (int idx = tid; idx < ITEMS; idx += NW * 64) {
       if (((idx >> 6) % MT) * 16 + (idx & 15) >= p.M) continue;
@@ -216,7 +232,7 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
     }
     shared_stores_done();
     __syncthreads();
-    if (tid == 0) last = arrived_last(p.arrivals + blockIdx.x, parts);
+    if (tid == 0) last = arrived_last(p.arrivals + tile, parts);
     __syncthreads();
     if (!last) return;
   }
@@ -248,10 +264,11 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
         sum[it][u] = (&red[0][0][0][0])[idx] + (&red[1][0][0][0])[idx];
       }
   } else {
-    for (int z0 = 0; z0 < parts; z0 += 4) {  // four parts of every item are requested before any is added
-      floatx4 q[4][IPT][MATS];
+    constexpr int Z = IPT * MATS > 2 ? 2 : 4;  // so many parts of every item are requested before any is added
+    for (int z0 = 0; z0 < parts; z0 += Z) {
+      floatx4 q[Z][IPT][MATS];
 #pragma unroll
-      for (int z = 0; z < 4; ++z)
+      for (int z = 0; z < Z; ++z)
 #pragma unroll
         for (int it = 0; it < IPT; ++it)
 #pragma unroll
@@ -266,7 +283,7 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
             q[z][it][u] = floatx4{x0, x1, x2, x3};
           }
 #pragma unroll
-      for (int z = 0; z < 4; ++z)
+      for (int z = 0; z < Z; ++z)
         if (z0 + z < parts) {
 #pragma unroll
           for (int it = 0; it < IPT; ++it)
@@ -299,7 +316,7 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           e[i] = r[i] * ((p.nm.emit_gain_dtype == JLLM_BF16) ? ldf((const bf16_t*)p.nm.emit_gain, n + i) : ldf((const float*)p.nm.emit_gain, n + i));
-        *(u32x2*)(p.nm.emit_rows + (size_t)m * p.N + n) = u32x2{pack_bf16(e[0], e[1]), pack_bf16(e[2], e[3])};
+        *(u32x2*)(p.nm.emit_rows + (size_t)m * p.nm.emit_ld + n) = u32x2{pack_bf16(e[0], e[1]), pack_bf16(e[2], e[3])};
       }
       if (p.out_dtype == JLLM_BF16) {
         if (vec)
@@ -350,29 +367,31 @@ static int launch_stream(const StreamArgs& a, dim3 grid, hipStream_t stream) {
 }
 
 template <int CT, bool GATED>
-static int launch_stream_rows(const StreamArgs& a, dim3 grid, bool shared, hipStream_t stream) {
+static int launch_stream_rows(const StreamArgs& a, dim3 grid, int row_tiles, bool shared, hipStream_t stream) {
 #define GS_CASE(MT)                                                       \
   case MT:                                                                \
     return shared ? launch_stream<CT, MT, GATED, true>(a, grid, stream) : launch_stream<CT, MT, GATED, false>(a, grid, stream);
-  switch ((a.M + 15) / 16) {
-    GS_CASE(1) GS_CASE(2) GS_CASE(3)
-    default: return shared ? launch_stream<CT, 4, GATED, true>(a, grid, stream) : launch_stream<CT, 4, GATED, false>(a, grid, stream);
+  switch (row_tiles) {
+    GS_CASE(1) GS_CASE(2) GS_CASE(3) GS_CASE(4)
+    default: return launch_stream<CT, 8, GATED, false>(a, grid, stream);
   }
 #undef GS_CASE
 }
 
-// `rows`: weight rows per workgroup, both weights' of the gated epilogue together (32, 64, 96 or 128). `parts` > 1 cuts K over
-// gridDim.y in whole blocks of 128; `partial` then holds parts * column tiles * rows * 16 * ceil(M / 16) floats and `arrivals`
-// one int per column tile, zeros, left as zeros. An RMSNorm on either side as in jllm_gemm_skinny_norm_bf16.
+// `rows`: weight rows per workgroup, both weights' of the gated epilogue together (32, 64, 96 or 128). `tile_m`: activation
+// rows per workgroup (64 or 128; up to 64 rows in all take tiles of 16, 32, 48 or 64). `parts` > 1 cuts K over
+// gridDim.y in whole blocks of 128; `partial` then holds parts * column tiles * rows * (tiles of rows in all) * (their rows) floats and `arrivals`
+// one int per column tile (and tile of rows), zeros, left as zeros. An RMSNorm on either side as in jllm_gemm_skinny_norm_bf16.
 // returns 0 when it ran, 1 when the shape is not one it takes (the caller uses another kernel), -1 on errors
 extern "C" int jllm_gemm_stream_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias,
                                      int bias_dtype, void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue,
-                                     float gate_limit, int rows, int parts, float* partial, int* arrivals, void* emit_rows,
+                                     float gate_limit, int rows, int tile_m, int parts, float* partial, int* arrivals, void* emit_rows, int emit_ld,
                                      const void* emit_gain, int emit_gain_dtype, float* emit_partial, int emit_parts,
                                      const float* norm_partial, int norm_parts, float norm_eps, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 64 || (K & 127) || (N & 15) || (lda & 7) || K <= 0 || lda < 0) return 1;
+  if ((K & 127) || (N & 15) || (lda & 7) || K <= 0 || lda < 0) return 1;
   if (((uintptr_t)A & 15) || ((uintptr_t)W & 15) || (W2 && ((uintptr_t)W2 & 15))) return 1;
+  if (tile_m != 64 && tile_m != 128) JLLM_FAIL("gemm_stream: tiles of %d rows (64 and 128)", tile_m);
   // a lane's place in an operand is a 32-bit byte offset from the workgroup's first row
   if ((unsigned long long)lda >= (1ull << 24) || (unsigned long long)K >= (1ull << 23)) return 1;
   JLLM_TAKE_GATE("gemm_stream", epilogue, gate_limit, gs);
@@ -389,27 +408,29 @@ extern "C" int jllm_gemm_stream_bf16(const void* A, int lda, const void* W, cons
   const int used = (nblk + bpp - 1) / bpp;  // parts that have any block
   if (used > 1 && (!partial || !arrivals || ((uintptr_t)partial & 15))) JLLM_FAIL("gemm_stream: %d parts of K need a buffer for their sums and counters", used);
   if (emit_rows && (epilogue != 1 || !emit_gain || !emit_partial)) JLLM_FAIL("gemm_stream: rows for a norm come from the accumulate epilogue, with gain and partial sums");
+  if (emit_rows && (emit_ld < N || (emit_ld & 3) || ((uintptr_t)emit_rows & 7))) JLLM_FAIL("gemm_stream: rows for a norm with stride %d", emit_ld);
   if (emit_rows && emit_parts < tiles) JLLM_FAIL("gemm_stream: %d places for the partial sums of %d workgroups", emit_parts, tiles);
   if (norm_partial && norm_parts <= 0) JLLM_FAIL("gemm_stream: %d partial sums", norm_parts);
   if (norm_partial && ((norm_parts & 3) || ((uintptr_t)norm_partial & 15))) return 1;
   const int cus = jllm_compute_units();
   if (cus <= 0) JLLM_FAIL("gemm_stream: the GPU's compute units could not be read");
-  dim3 grid(tiles, used);
-  if (grid.y > 65535) return 1;
+  dim3 grid(tiles, used, (M + tile_m - 1) / tile_m);
+  if (grid.y > 65535 || grid.z > 65535) return 1;
+  const int row_tiles = M > 64 ? tile_m / 16 : (M + 15) / 16;
   const StreamArgs a{(const bf16_t*)A, (const bf16_t*)W, (const bf16_t*)W2, bias, out, partial, arrivals, lda, bias_dtype, out_dtype, ldo, M, N, K,
-                     epilogue, bpp * 2, gs, StreamNorm{(bf16_t*)emit_rows, emit_gain, emit_gain_dtype, emit_partial, emit_parts, norm_partial, norm_parts, norm_eps}};
+                     epilogue, bpp * 2, M <= 64 && used == 1, gs, StreamNorm{(bf16_t*)emit_rows, emit_ld, emit_gain, emit_gain_dtype, emit_partial, emit_parts, norm_partial, norm_parts, norm_eps}};
   // two workgroups share a compute unit where there are more of them than compute units: one streams while the other adds up
-  const bool shared = (long)tiles * used > cus;
+  const bool shared = (long)tiles * used * grid.z > cus;
   if (W2) switch (rows) {
-      case 32: return launch_stream_rows<2, true>(a, grid, shared, stream);
-      case 64: return launch_stream_rows<4, true>(a, grid, shared, stream);
-      case 96: return launch_stream_rows<6, true>(a, grid, shared, stream);
-      default: return launch_stream_rows<8, true>(a, grid, shared, stream);
+      case 32: return launch_stream_rows<2, true>(a, grid, row_tiles, shared, stream);
+      case 64: return launch_stream_rows<4, true>(a, grid, row_tiles, shared, stream);
+      case 96: return launch_stream_rows<6, true>(a, grid, row_tiles, shared, stream);
+      default: return launch_stream_rows<8, true>(a, grid, row_tiles, shared, stream);
     }
   switch (rows) {
-    case 32: return launch_stream_rows<2, false>(a, grid, shared, stream);
-    case 64: return launch_stream_rows<4, false>(a, grid, shared, stream);
-    case 96: return launch_stream_rows<6, false>(a, grid, shared, stream);
-    default: return launch_stream_rows<8, false>(a, grid, shared, stream);
+    case 32: return launch_stream_rows<2, false>(a, grid, row_tiles, shared, stream);
+    case 64: return launch_stream_rows<4, false>(a, grid, row_tiles, shared, stream);
+    case 96: return launch_stream_rows<6, false>(a, grid, row_tiles, shared, stream);
+    default: return launch_stream_rows<8, false>(a, grid, row_tiles, shared, stream);
   }
 }

@@ -57,46 +57,48 @@ def library_path() -> Optional[str]:
     return _build.find_library()
 
 
+_SIGS = {
+    "jllm_embed": [_P, _I, _P, _P, _I, _I, _F, _P],
+    "jllm_rmsnorm": [_P, _P, _I, _I, _P, _I, _F, _P, _I, _I, _P],
+    "jllm_gemm_generic": [_P, _I, _I, _P, _P, _I, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _P],
+    "jllm_qk_norm_rope_store": [_P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _F, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P],
+    "jllm_paged_attention_generic": [_P, _I, _P, _I, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P, _P],
+    "jllm_argmax": [_P, _I, _I, _I, _P, _P, _P],
+    "jllm_sample": [_P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P],
+    "jllm_adjust_logits": [_P, _I, _P, _P, _I, _F, _F, _F, _P, _P, _I, _P],
+    "jllm_token_logprobs": [_P, _I, _I, _I, _P, _I, _P, _P, _P, _P],
+    "jllm_copy_words": [_P, _P, _L, _P],
+    "jllm_latent_prepare": [_P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _I, _F, _P, _P, _P, _P, _P, _I, _P, _P],
+    "jllm_latent_heads_generic": [_P, _I, _I, _I, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P],
+    "jllm_latent_attention_generic": [_P, _I, _P, _I, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P],
+    "jllm_moe_route": [_P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P],
+    "jllm_moe_gemm_generic": [_P, _I, _I, _P, _P, _I, _P, _I, _I, _I, _I, _P, _P, _I, _I, _I, _I, _I, _F, _I, _F, _P],
+    "jllm_moe_combine": [_P, _P, _I, _I, _I, _F, _P, _P, _P, _P, _I, _I, _I, _P],
+    "jllm_moe_router": [_P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P, _I, _I, _I, _P],
+    "jllm_gather_add": [_P, _I, _P, _I, _I, _P, _I, _I, _P],
+    "jllm_dyntanh_read": [_P, _P, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _P],
+    "jllm_streams_write": [_P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P],
+    "jllm_concat_rows": [_P, _P, _I, _I, _P, _I, _I, _P],
+    "jllm_ssm_scan": [_P, _I, _P, _I, _I, _I, _P, _P, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _P],
+    "jllm_gated_group_norm": [_P, _I, _P, _I, _I, _P, _I, _F, _I, _I, _I, _P, _I, _I, _I, _I, _F, _P],
+    "jllm_linear_scan": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _F, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _F, _P],
+    "jllm_linear_chunks": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _F, _P, _P, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _F, _P, _P],
+    "jllm_rms_seam": [_P, _I, _I, _P, _I, _P, _I, _I, _F, _F, _P, _P, _F, _P, _F, _P, _I, _I, _P, _P, _P, _P],
+    "jllm_rms_between": [_P, _I, _I, _P, _I, _P, _I, _I, _F, _F, _P, _F, _P, _P, _I, _P, _F, _P, _I, _I, _P],
+    "jllm_token_shift": [_P, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _P],
+    "jllm_copy_page_rows": [_P, _I, _I, _I, _I, _L, _I, _I, _I, _P],
+    "jllm_layernorm_seam": [_P, _P, _I, _I, _P, _I, _P, _I, _I, _F, _F, _P, _P, _P, _P, _P, _I, _F, _P, _I, _I, _P],
+    "jllm_qkv_prepare": [_P, _I, _I, _I, _P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _F, _P, _P, _I, _F, _I, _P, _P, _I, _I, _I, _P, _I, _I, _P],
+    "jllm_attention_dv_generic": [_P, _I, _I, _P, _I, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _I, _P, _I, _P, _P],
+    "jllm_heads_finish": [_P, _I, _I, _I, _I, _I, _I, _F, _I, _F, _F, _P, _I, _P, _I, _I, _I, _F, _P, _I, _I, _I, _P],
+    "jllm_heads_finish_split": [_P, _I, _I, _I, _I, _I, _F, _I, _F, _F, _P, _I, _P, _I, _I, _I, _F, _P, _I, _I, _I, _P, _P],
+    "jllm_short_conv": [_P, _I, _P, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _P, _P],
+    "jllm_gated_delta": [_P, _I, _P, _I, _I, _I, _I, _P, _P, _I, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _P],
+}
+
+
 def _declare(lib) -> None:
-    sig = {
-        "jllm_embed": [_P, _I, _P, _P, _I, _I, _F, _P],
-        "jllm_rmsnorm": [_P, _P, _I, _I, _P, _I, _F, _P, _I, _I, _P],
-        "jllm_gemm_generic": [_P, _I, _I, _P, _P, _I, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _P],
-        "jllm_qk_norm_rope_store": [_P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _F, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P],
-        "jllm_paged_attention_generic": [_P, _I, _P, _I, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P, _P],
-        "jllm_argmax": [_P, _I, _I, _I, _P, _P, _P],
-        "jllm_sample": [_P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P],
-        "jllm_adjust_logits": [_P, _I, _P, _P, _I, _F, _F, _F, _P, _P, _I, _P],
-        "jllm_token_logprobs": [_P, _I, _I, _I, _P, _I, _P, _P, _P, _P],
-        "jllm_copy_words": [_P, _P, _L, _P],
-        "jllm_latent_prepare": [_P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _I, _F, _P, _P, _P, _P, _P, _I, _P, _P],
-        "jllm_latent_heads_generic": [_P, _I, _I, _I, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P],
-        "jllm_latent_attention_generic": [_P, _I, _P, _I, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P],
-        "jllm_moe_route": [_P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P],
-        "jllm_moe_gemm_generic": [_P, _I, _I, _P, _P, _I, _P, _I, _I, _I, _I, _P, _P, _I, _I, _I, _I, _I, _F, _I, _F, _P],
-        "jllm_moe_combine": [_P, _P, _I, _I, _I, _F, _P, _P, _P, _P, _I, _I, _I, _P],
-        "jllm_moe_router": [_P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P, _I, _I, _I, _P],
-        "jllm_gather_add": [_P, _I, _P, _I, _I, _P, _I, _I, _P],
-        "jllm_dyntanh_read": [_P, _P, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _P],
-        "jllm_streams_write": [_P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P],
-        "jllm_concat_rows": [_P, _P, _I, _I, _P, _I, _I, _P],
-        "jllm_ssm_scan": [_P, _I, _P, _I, _I, _I, _P, _P, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _P],
-        "jllm_gated_group_norm": [_P, _I, _P, _I, _I, _P, _I, _F, _I, _I, _I, _P, _I, _I, _I, _I, _F, _P],
-        "jllm_linear_scan": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _F, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _F, _P],
-        "jllm_linear_chunks": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _F, _P, _P, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _F, _P, _P],
-        "jllm_rms_seam": [_P, _I, _I, _P, _I, _P, _I, _I, _F, _F, _P, _P, _F, _P, _F, _P, _I, _I, _P, _P, _P, _P],
-        "jllm_rms_between": [_P, _I, _I, _P, _I, _P, _I, _I, _F, _F, _P, _F, _P, _P, _I, _P, _F, _P, _I, _I, _P],
-        "jllm_token_shift": [_P, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _P],
-        "jllm_copy_page_rows": [_P, _I, _I, _I, _I, _L, _I, _I, _I, _P],
-        "jllm_layernorm_seam": [_P, _P, _I, _I, _P, _I, _P, _I, _I, _F, _F, _P, _P, _P, _P, _P, _I, _F, _P, _I, _I, _P],
-        "jllm_qkv_prepare": [_P, _I, _I, _I, _P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _F, _P, _P, _I, _F, _I, _P, _P, _I, _I, _I, _P, _I, _I, _P],
-        "jllm_attention_dv_generic": [_P, _I, _I, _P, _I, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _I, _P, _I, _P, _P],
-        "jllm_heads_finish": [_P, _I, _I, _I, _I, _I, _I, _F, _I, _F, _F, _P, _I, _P, _I, _I, _I, _F, _P, _I, _I, _I, _P],
-        "jllm_heads_finish_split": [_P, _I, _I, _I, _I, _I, _F, _I, _F, _F, _P, _I, _P, _I, _I, _I, _F, _P, _I, _I, _I, _P, _P],
-        "jllm_short_conv": [_P, _I, _P, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _P, _P],
-        "jllm_gated_delta": [_P, _I, _P, _I, _I, _I, _I, _P, _P, _I, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _P],
-    }
-    for name, args in sig.items():
+    for name, args in _SIGS.items():
         fn = getattr(lib, name)
         fn.argtypes = args
         fn.restype = _I
@@ -118,7 +120,7 @@ _OPTIONAL_SIGS = {
     "jllm_gemm_skinny_norm_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _P, _I, _P, _I, _F, _P],
     "jllm_gemm_mfma_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P],
     "jllm_gemm_pingpong_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P, _P],
-    "jllm_gemm_stream_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P, _P, _P, _P, _I, _P, _I, _P, _I, _F, _P],
+    "jllm_gemm_stream_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _P, _P, _I, _P, _I, _P, _I, _P, _I, _F, _P],
     "jllm_decode_attention_bf16": [_P, _I, _P, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _I, _P],
     "jllm_decode_attention_fused_bf16": [_P, _I, _P, _I, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _F, _I, _I, _I, _I, _I,
                                          _I, _I, _I, _F, _I, _P, _P, _I, _I, _P, _P],
@@ -385,7 +387,7 @@ def _skinny_norm(a, w, w2, bias, out, epilogue, emit=None, normed: Optional[Norm
     does not take the case."""
     M, K = a.shape
     N = w.shape[0]
-    if M > STREAM_MAX_ROWS or a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or (M > STREAM_MAX_ROWS and _wide_plan(M, N, K, w2 is not None, epilogue == EPI_ADD) is None):
         return False
     e_rows, e_gain, e_part = emit if emit is not None else (None, None, None)
     n_part = normed.partials if normed is not None else None
@@ -398,10 +400,17 @@ def _skinny_norm(a, w, w2, bias, out, epilogue, emit=None, normed: Optional[Norm
     if few and not _few_rows_prefer_stream(N, K, w2 is not None):
         return _try("jllm_gemm_skinny_norm_bf16", *head, _skinny_rows(N, K, w2 is not None), *emits, emit_parts, *takes)
     if K % 128 == 0:
-        rows, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a)
-        if _try("jllm_gemm_stream_bf16", *head, rows, parts, _ptr(sums), _ptr(arrivals), *emits, emit_parts, *takes):
+        rows, tile, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a, epilogue == EPI_ADD)
+        if _try("jllm_gemm_stream_bf16", *head, rows, tile, parts, _ptr(sums), _ptr(arrivals), _ptr(e_rows), e_rows.stride(0) if e_rows is not None else 0, *emits[1:],
+                emit_parts, *takes):
             return True
     return few and _try("jllm_gemm_skinny_norm_bf16", *head, 16, *emits, emit_parts, *takes)  # the second kernel declined
+
+
+def _norm_rides(M: int, K: int, N: int) -> bool:
+    """Whether the adding product of M rows, K and N prepares the norm that follows. For more than 64 rows it does so where
+    the same kernel takes it, from the row count on at which the rows may be laid out for many rows (`activation_rows`)."""
+    return M <= STREAM_MAX_ROWS or (M >= PAD_ROWS_FROM and _wide_plan(M, N, K, False, True) is not None)
 
 
 def gemm_add_then_norm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gain: torch.Tensor, eps: float,
@@ -410,15 +419,15 @@ def gemm_add_then_norm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gain
     and ``eps``, as a ``NormedRows``: for few bf16 rows the product prepares that norm on its way out."""
     if isinstance(a, NormedRows):
         a = a.tensor()
-    if not exact and norm_dtype == torch.bfloat16 and a.dim() == 2 and a.shape[0] <= STREAM_MAX_ROWS \
-            and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() \
-            and w.shape[1] == a.shape[1] and w.shape[0] % 16 == 0 and a.shape[0] > 0 and a.stride(1) == 1 \
+    if not exact and norm_dtype == torch.bfloat16 and a.dim() == 2 and a.dtype == torch.bfloat16 \
+            and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() \
+            and w.shape[1] == a.shape[1] and w.shape[0] % 16 == 0 and 0 < a.shape[0] and _norm_rides(*a.shape, w.shape[0]) and a.stride(1) == 1 \
             and out.dtype == torch.float32 and out.dim() == 2 and out.shape == (a.shape[0], w.shape[0]) and out.is_contiguous() \
             and gain.numel() == w.shape[0] and gain.is_contiguous() \
             and (bias is None or (bias.numel() == w.shape[0] and bias.is_contiguous())):
         _dev(a, w, bias, out, gain)
         M, N = out.shape
-        scaled = torch.empty((M, N), dtype=torch.bfloat16, device=out.device)
+        scaled = activation_rows(M, N, torch.bfloat16, out.device)
         partials = torch.empty((M, _norm_partials(M, N, a.shape[1])), dtype=torch.float32, device=out.device)
         if _skinny_norm(a, w, None, bias, out, EPI_ADD, emit=(scaled, gain, partials)):
             return NormedRows(out, gain, eps, norm_dtype, scaled, partials)
@@ -783,7 +792,9 @@ def _skinny_rows(N: int, K: int, gated: bool) -> int:
 def _norm_partials(M: int, N: int, K: int) -> int:
     """Partial sums of squares per row that a product with N outputs leaves for the norm behind it: room for one per
     workgroup's columns, in whole fours."""
-    if M > SKINNY_MAX_ROWS or _few_rows_prefer_stream(N, K, False):
+    if M > STREAM_MAX_ROWS:
+        groups = -(-N // _wide_plan(M, N, K, False, True)[0])
+    elif M > SKINNY_MAX_ROWS or _few_rows_prefer_stream(N, K, False):
         groups = max(N // 16, -(-N // _stream_plan(N, K, False)[0])) if M <= SKINNY_MAX_ROWS else -(-N // _stream_plan(N, K, False)[0])
     else:
         groups = -(-N // _skinny_rows(N, K, False))
@@ -823,7 +834,7 @@ def step_scratch(rows: int, device):
     """Around the launches of one step of ``rows`` rows in one stream: zeroed counters that its products of few rows, which
     follow each other, take turns in (each leaves them zero). Without them every such product clears counters of its own, as
     the rare ones do that reach the second kernel with up to 16 rows."""
-    if not SKINNY_MAX_ROWS < rows <= STREAM_MAX_ROWS or device.type != "cuda":
+    if not SKINNY_MAX_ROWS < rows <= WIDE_MOST_ROWS or device.type != "cuda":
         yield
         return
     before = getattr(_step_scratch, "arrivals", None)
@@ -837,17 +848,94 @@ def step_scratch(rows: int, device):
 STREAM_COUNTERS = 1024
 
 
-def _stream_scratch(M: int, N: int, K: int, gated: bool, a: torch.Tensor):
-    """The second weight-streaming kernel's plan and scratch: (rows, parts, sums, counters)."""
-    rows, parts = _stream_plan(N, K, gated)
+def _stream_scratch(M: int, N: int, K: int, gated: bool, a: torch.Tensor, adds: bool):
+    """The plan and scratch of the kernel behind `_stream_plan` and `_wide_plan`: (weight rows, activation rows, parts, sums,
+    counters)."""
+    rows, tile, parts = _plan_of_rows(M, N, K, gated, adds)
     if parts == 1:
-        return rows, 1, None, None
-    tiles = -(-N // (rows // 2 if gated else rows))
-    partial = torch.empty((parts * tiles * rows * 16 * -(-M // 16),), dtype=torch.float32, device=a.device)
+        return rows, tile, 1, None, None
+    row_tiles = -(-M // tile)
+    tiles = -(-N // (rows // 2 if gated else rows)) * row_tiles
+    partial = torch.empty((parts * tiles * rows * (tile if M > STREAM_MAX_ROWS else 16 * -(-M // 16)),), dtype=torch.float32, device=a.device)
     arrivals, stream = getattr(_step_scratch, "arrivals", None) or (None, None)
     if arrivals is None or arrivals.device != a.device or arrivals.numel() < tiles or stream != _stream():
         arrivals = torch.empty(tiles, dtype=torch.int32, device=a.device).zero_()
-    return rows, parts, partial, arrivals
+    return rows, tile, parts, partial, arrivals
+
+
+def _plan_of_rows(M: int, N: int, K: int, gated: bool, adds: bool) -> Tuple[int, int, int]:
+    """(weight rows, activation rows, parts of K) of the second weight-streaming kernel for a product that it takes."""
+    if M > STREAM_MAX_ROWS:
+        return _wide_plan(M, N, K, gated, adds)
+    rows, parts = _stream_plan(N, K, gated)
+    return rows, 64, parts
+
+
+# Estimated times of that kernel for more than 64 rows, in microseconds
+WIDE_MOST_ROWS = 1024
+WIDE_ADD_COLUMNS = 2048           # with the add into the residual (and the rows for a norm) the estimate holds up to here
+WIDE_LEAST_K = 1024               # the shortest K it was measured at
+WIDE_BLOCK_US = (0.275, 0.0198)   # 64 of k on 32 weight and 64 activation rows, and per 8 rows more of either
+WIDE_FIXED_US = {64: 4.8, 128: 7.2}   # the launch, the first blocks and the end, by activation rows per workgroup
+WIDE_PAIR = (1.35, 1.8)           # two workgroups of 64 rows on a compute unit: a few of them, all
+WIDE_MERGE_US = (2.5, 0.06)       # parts of K: the way through memory, and per KB of sums that the last workgroup reads
+WIDE_BYTES_PER_US = 5.3e6         # weights from memory
+TILED_FIXED_US = 6.0              # what the tiled kernels' estimates leave out
+WIDE_AT_MOST = 0.97               # of the tiled kernels' estimate
+NORM_LAUNCH_US = 4.0              # a norm of few rows as a launch of its own
+
+
+def _wide_us(M: int, N: int, K: int, gated: bool, rows: int, tile: int, parts: int) -> float:
+    cus = compute_units()
+    groups = -(-N // (rows // 2 if gated else rows)) * -(-M // tile) * parts
+    blocks = -(-(K // 128) // parts) * 2
+    step = blocks * (WIDE_BLOCK_US[0] + WIDE_BLOCK_US[1] * ((rows + tile) / 8 - 12))
+    if tile == 64:  # two on a compute unit
+        full, last = divmod(groups, 2 * cus)
+        few, all_ = WIDE_PAIR
+        t = full * step * all_
+        if last:
+            t += step if last <= cus else step * (few + (all_ - few) * (last - cus) / cus)
+    else:
+        t = -(-groups // cus) * step
+    t = max(t, N * K * 2 * (2 if gated else 1) / WIDE_BYTES_PER_US) + WIDE_FIXED_US[tile]
+    if parts > 1:
+        t += WIDE_MERGE_US[0] + WIDE_MERGE_US[1] * parts * rows * min(tile, M) * 4 / 1024
+    return t
+
+
+@functools.lru_cache(maxsize=8192)
+def _wide_plan(M: int, N: int, K: int, gated: bool, adds: bool = False) -> Optional[Tuple[int, int, int]]:
+    """(weight rows, activation rows, parts of K) with which the second weight-streaming kernel takes a product of more than
+    64 rows, or None where the tiled kernels are estimated to be faster: they move fewer bytes per multiply through a compute
+    unit, but their tiles of 128 x 128 and larger leave compute units without work where a product is small, and cutting K
+    costs them a second launch. ``adds``: into the residual, where from 128 rows on it prepares the norm behind it, which is then no launch
+    of its own if the product that reads it is taken here too (asked for one over N inputs: as q, k, v behind a long K, gated
+    behind a short one). Here tiles of 64 or 128 rows by 32 to 128 fill the chip with K whole.
+
+    The constants were fitted to a sweep of every choice for the products of the 0.6B, 1.7B, 4B and 8B shapes at 100, 200, 320, 487 and
+    631 rows against what the tiled kernels take. us, tiled / here: 0.6B shape at 487 rows qkv 22.2 / 13.3, o 17.6 / 13.5,
+    gate/up 18.8 / 16.9, down 17.6 / 17.2 (and the norm behind o and down, 4.0, costs no launch of its own); 4B qkv at 631 rows
+    41.6 / 34.5, 8B qkv at 320 39.2 / 35.4. Beyond, the tiled kernels win: 8B gate/up at 200 rows 79.9 / 101, down 44.8 / 54.9."""
+    if not STREAM_MAX_ROWS < M <= WIDE_MOST_ROWS or K % 128 or N % 16 or K < WIDE_LEAST_K or (adds and N > WIDE_ADD_COLUMNS):
+        return None
+    cus = compute_units()
+    rows, cut = _tiled_plan(M, N, K, gated)
+    best = WIDE_AT_MOST * (TILED_FIXED_US + (_large_us(M, N, K, gated, rows, cut) if rows else _small_us(M, N, K, gated, cut)))
+    if adds and M >= PAD_ROWS_FROM and _wide_plan(M, 2 * N if K > N else 3 * N, N, K <= N):
+        best += NORM_LAUNCH_US
+    plan = None
+    for rows in (32, 64, 96, 128):
+        for tile in (64, 128):
+            tiles = -(-N // (rows // 2 if gated else rows)) * -(-M // tile)
+            for parts in (1, 2, 3, 4):
+                per = -(-(K // 128) // parts)
+                if parts > 1 and (tiles * parts > 2 * cus or per < STREAM_MIN_BLOCKS or -(-(K // 128) // per) != parts):
+                    continue
+                t = _wide_us(M, N, K, gated, rows, tile, parts)
+                if t < best:
+                    best, plan = t, (rows, tile, parts)
+    return plan
 
 
 STREAM_FEW_ROWS = (1280, 8192)   # columns at most, K at least: see `_few_rows_prefer_stream`
@@ -877,9 +965,9 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0) -> bool:
     if M <= SKINNY_MAX_ROWS and not _few_rows_prefer_stream(N, K, w2 is not None) \
             and _try("jllm_gemm_skinny_bf16", *head, _skinny_rows(N, K, w2 is not None), _stream()):
         return True
-    if M <= STREAM_MAX_ROWS and K % 128 == 0:
-        rows, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a)
-        if _try("jllm_gemm_stream_bf16", *head, rows, parts, _ptr(sums), _ptr(arrivals), None, None, F32, None, 0, None, 0, 0.0, _stream()):
+    if K % 128 == 0 and (M <= STREAM_MAX_ROWS or _wide_plan(M, N, K, w2 is not None, epilogue == EPI_ADD) is not None):
+        rows, tile, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a, epilogue == EPI_ADD)
+        if _try("jllm_gemm_stream_bf16", *head, rows, tile, parts, _ptr(sums), _ptr(arrivals), None, 0, None, F32, None, 0, None, 0, 0.0, _stream()):
             return True
     tile_rows, cut = _tiled_plan(M, N, K, w2 is not None)
     if tile_rows:

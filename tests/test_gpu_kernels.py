@@ -352,6 +352,43 @@ def test_products_of_17_to_64_rows_at_any_plan(ops, monkeypatch, M, N, K, rows, 
     assert set(ops.stats()["ran"]) == {"jllm_gemm_stream_bf16"}
 
 
+@pytest.mark.parametrize("rows,tile", [(32, 64), (64, 64), (96, 64), (128, 64), (32, 128), (64, 128), (96, 128), (128, 128)])
+@pytest.mark.parametrize("M,N,K,parts", [(128, 1024, 1024, 1), (129, 1040, 1152, 2), (200, 2048, 1024, 3), (321, 528, 3072, 4), (640, 4096, 1024, 1)])
+def test_products_of_more_rows_at_any_plan(ops, monkeypatch, M, N, K, parts, rows, tile):
+    """The same kernel for more than 64 rows in tiles of 64 and 128, the last one with a single row or more, rows with a
+    stride: every epilogue and the norm on both sides, against float64 within the bound of an fp32 sum of K products."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M * N + K + rows + tile)
+    rnd = lambda *shape: torch.randn(*shape, device=DEV, generator=gen)
+    a = ops.activation_rows(M, K, torch.bfloat16, torch.device(DEV))
+    a.copy_(rnd(M, K))
+    w, w2 = (rnd(N, K) / math.sqrt(K)).bfloat16(), (rnd(N, K) / math.sqrt(K)).bfloat16()
+    w3 = (rnd(272, N) / math.sqrt(N)).bfloat16()
+    bias, gain, res0 = rnd(N), rnd(N).abs() + 0.5, rnd(M, N)
+    monkeypatch.setattr(ops, "_wide_plan", lambda m, n, k, gated, adds=False: (rows, tile, parts if k == K else 1))
+    ops.reset_stats()
+    exact, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    bound = 2 * K * 2.0 ** -24 * size + 1e-6
+    out = ops.gemm(a, w, bias=bias, out_dtype=torch.float32)
+    assert bool(((out.double() - exact - bias.double()).abs() <= bound + 2.0 ** -23 * (exact.abs() + bias.abs())).all())
+    assert torch.equal(ops.gemm(a, w, bias=bias), out.bfloat16())
+    res = res0.clone()
+    with ops.step_scratch(M, a.device):
+        promise = ops.gemm_add_then_norm(a, w, res, gain, 1e-3, torch.bfloat16)
+        assert bool(((res.double() - exact - res0.double()).abs() <= bound + 2.0 ** -23 * (exact.abs() + res0.abs())).all())
+        assert torch.equal(promise.scaled, (res * gain).bfloat16())
+        if N % 128 == 0:  # what the consuming product takes as its K
+            scale = torch.rsqrt((res.double() ** 2).mean(-1, keepdim=True) + 1e-3)
+            got = ops.gemm(promise, w3, out_dtype=torch.float32)
+            want = (promise.scaled.double() @ w3.double().T) * scale
+            assert bool(((got.double() - want).abs() <= (2 * N + 256) * 2.0 ** -24 * (promise.scaled.double().abs() @ w3.double().abs().T) * scale + 1e-6).all())
+        gated = ops.gemm(a, w, w2=w2, epilogue=ops.EPI_GATED, out_dtype=torch.float32)
+    up = a.double() @ w2.double().T
+    both = bound * (1.1 * up.abs() + 1) + 2 * K * 2.0 ** -24 * (a.double().abs() @ w2.double().abs().T) * exact.abs() + 1e-5 * (exact * up).abs()
+    assert bool(((gated.double() - torch.nn.functional.silu(exact) * up).abs() <= both).all())
+    assert set(ops.stats()["ran"]) == {"jllm_gemm_stream_bf16"} and promise._rows is None
+
+
 def test_gemm_rows_do_not_depend_on_the_batch(ops):
     """The result of a row is the same bits whether it is alone or among others, within one kernel family (the
     bfloat16 path has one kernel for up to 16 rows, one for up to 64 and one for more; between them results differ

@@ -151,3 +151,49 @@ def test_the_attention_plan_says_whether_the_runs_of_a_step_differ_much_in_keys(
     assert facts((1, 100), (1, 5000))["key_groups"] == 1   # single rows go to the split-key kernel anyway
     f = facts((2048, 0), (1, 77))
     assert f["key_groups"] == 2 and f["n_tiles_multi"] == 16 and f["single_rows"] == (2048, 1)
+
+
+def test_plans_of_the_second_weight_streaming_kernel():
+    """Every plan is one that the kernel has, parts of K are whole blocks that are all there, its counters fit the step's, and
+    for up to 64 rows it knows nothing of their number; few columns and large products of many rows stay with the other kernels."""
+    import inspect
+    assert list(inspect.signature(ops._stream_plan.__wrapped__).parameters) == ["N", "K", "gated"]
+    shapes = [s for v in SHAPES.values() for s in v] + [(4096, 1024, False), (3072, 1024, True), (1024, 3072, False), (2560, 9728, False), (16, 128, False),
+                                                       (48, 1024, True), (151936, 4096, False)]
+    taken = 0
+    for n, k, gated in shapes:
+        rows, parts = ops._stream_plan(n, k, gated)
+        tiles = -(-n // (rows // 2 if gated else rows))
+        assert rows in (32, 64, 96, 128) and 1 <= parts <= k // 128 and (parts == 1 or tiles <= ops.STREAM_COUNTERS), (n, k, gated, rows, parts)
+        for m in (65, 100, 127, 128, 200, 333, 487, 640, 900, 1024, 1025, 4096):
+            for adds in (False, True):
+                plan = ops._wide_plan(m, n, k, gated, adds and not gated)
+                if plan is None:
+                    continue
+                taken += 1
+                rows, tile, parts = plan
+                per = -(-(k // 128) // parts)
+                assert rows in (32, 64, 96, 128) and tile in (64, 128) and m <= ops.WIDE_MOST_ROWS and k >= ops.WIDE_LEAST_K, (m, n, k, plan)
+                assert -(-(k // 128) // per) == parts and (parts == 1 or -(-n // rows) * -(-m // tile) <= ops.STREAM_COUNTERS), (m, n, k, plan)
+    assert taken > 20
+    assert ops._wide_plan(487, 12288, 4096, True) is None and ops._wide_plan(300, 1024, 100, False) is None
+
+
+def test_declared_arguments_are_those_of_the_sources():
+    """Every entry point's declared argument types against its definition: a pointer declared as an int would reach the
+    kernel cut to 32 bits."""
+    import ctypes
+    import os
+    import re
+    from jllm_serve_amd.kernels import build
+    kinds = {ctypes.c_void_p: "pointer", ctypes.c_int: "int", ctypes.c_float: "float", ctypes.c_longlong: "long", ctypes.c_long: "long"}
+    defined = {}
+    for name in build.sources():
+        with open(os.path.join(build.SRC_DIR, name)) as f:
+            for fn, args in re.findall(r'extern "C" int (\w+)\(([^)]*)\)\s*{', f.read()):
+                defined[fn] = ["pointer" if "*" in a or "hipStream_t" in a else "float" if "float" in a else
+                               "long" if re.search(r"\b(long|size_t|int64_t)\b", a) else "int" for a in args.split(",") if a.strip()]
+    declared = {**ops._SIGS, **ops._OPTIONAL_SIGS}
+    assert len(declared) > 40 and set(declared) <= set(defined), set(declared) - set(defined)
+    for fn, args in declared.items():
+        assert [kinds[a] for a in args] == defined[fn], fn
