@@ -195,6 +195,7 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
 def _stream():
@@ -202,7 +203,7 @@ def _stream():
     microseconds each, so the host's time per launch is what such a step costs: the handle is asked of torch's own
     binding (a fraction of a microsecond) where it has one, not through a new Stream object (several)."""
     if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
+        return _raw_stream(_raw_device())
     return torch.cuda.current_stream().cuda_stream
 
 
@@ -354,7 +355,7 @@ def activation_rows(n: int, width: int, dtype: torch.dtype, device) -> torch.Ten
     would queue for it; such rows are laid 64 elements further apart (the tensor is a view with that row stride).
     Measured on the gate/up product of the 8B shape at 2,048 rows: 0.93 -> 1.12 PFLOP/s."""
     if n >= PAD_ROWS_FROM and (width * dtype.itemsize) % 4096 == 0:
-        return torch.empty((n, width + PAD_ELEMENTS), dtype=dtype, device=device)[:, :width]
+        return torch.empty_strided((n, width), (width + PAD_ELEMENTS, 1), dtype=dtype, device=device)
     return torch.empty((n, width), dtype=dtype, device=device)
 
 

@@ -86,6 +86,7 @@ class GqaAttention(Part):
             ops.check_attention_shape(spec.heads, spec.kv_heads, spec.head_dim, rot[2] if rot is not None else 0)
         except ops.KernelError as e:
             raise ValueError(f"{prefix}: {e}") from None
+        self.planner = GqaStepPlanner(spec.kv_heads)
         self.w_qkv = self.b_qkv = self.w_o = self.b_o = self.g_q = self.g_k = None
 
     def _name(self, which: str, ending: str = ".weight") -> str:
@@ -138,20 +139,20 @@ class GqaAttention(Part):
         return KvSpec(self.spec.kv_heads, self.spec.head_dim, self.spec.window)
 
     def step_planners(self):
-        return [GqaStepPlanner(self.spec.kv_heads)]
+        return [self.planner]
 
     def _batch_facts(self, step):
-        """The kernels' view of the batch: the step's own numbers and this mixer's plan of it."""
-        plan = step.plans.get(GqaStepPlanner(self.spec.kv_heads).key)
-        meta = {"max_context": step.max_context, "requests": step.n_requests, "rows": step.n_tokens}
+        """The kernels' view of the batch: the step's own numbers and this mixer's plan of it, put together once per step."""
+        plan = step.plans.get(self.planner.key)
         if plan is None:  # a step put together without the planner: the general kernels take it
-            meta["decode_only"] = False
-            return meta
-        meta.update(plan.facts)
-        tiles = plan.arrays.get("tiles")
-        meta["segments_dev"] = tiles if tiles is not None and tiles.numel() else None
-        arrivals = plan.arrays.get("arrivals")
-        meta["arrivals"] = arrivals if arrivals is not None and arrivals.numel() else None
+            return {"max_context": step.max_context, "requests": step.n_requests, "rows": step.n_tokens, "decode_only": False}
+        meta = plan.facts.get("batch")
+        if meta is None:
+            meta = {"max_context": step.max_context, "requests": step.n_requests, "rows": step.n_tokens, **plan.facts}
+            for name, array in (("segments_dev", "tiles"), ("arrivals", "arrivals")):
+                t = plan.arrays.get(array)
+                meta[name] = t if t is not None and t.numel() else None
+            plan.facts["batch"] = meta
         return meta
 
     def forward(self, xb, residual, step, slot, then_norm=None):
