@@ -351,6 +351,12 @@ static int launch_tiles(dim3 grid, hipStream_t stream, const bf16_t* q, int ldq,
   return 0;
 }
 
+// steps of single rows at key size 128 (attention_dv_rows.hip): true when it ran
+bool jllm_attention_dv_rows(const void* q, int ldq, float* out, int ldo, const void* kcache, const void* vcache, const int* block_table,
+                            int max_blocks, const int* tiles, int n_tiles, const int* positions, int heads, int kv_heads, int maps, int dk,
+                            int dv, int page_shift, int window, float scale, float softcap, int splits, int per_split, float* partial,
+                            int keep_first, const float* sinks, int chunk, const float* slopes, hipStream_t stream);
+
 // Returns 1 (declined) for sizes it does not take: dk a multiple of 16 up to 256, dv a multiple of 8 up to 256, bf16.
 // `splits` > 1 (tiles of single rows only): the workgroups of a tile take `per_split` key blocks each and `partial`
 // (fp32, rows x slots x splits x (dv + 2)) carries their results to the merge (a kernel of its own here, or, with
@@ -378,6 +384,12 @@ extern "C" int jllm_attention_dv_bf16(const void* q, int ldq, float* out, int ld
   dim3 grid(share ? kv_heads * maps : q_slots, n_tiles, partial ? splits : 1);
   const int db = (dv + 31) / 32;
   int rc = 1;
+  if (n_rows == n_tiles && kv_heads * maps <= 65535 &&
+      jllm_attention_dv_rows(q, ldq, out, ldo, kcache, vcache, block_table, max_blocks, tiles, n_tiles, positions, heads, kv_heads, maps, dk, dv,
+                             page_shift, window, scale, softcap, splits, per_split, partial, keep_first, sinks, chunk, slopes, stream)) {
+    JLLM_CHECK_LAUNCH("attention_dv_rows");
+    rc = 0;
+  } else
 #define AT_ARGS grid, stream, (const bf16_t*)q, ldq, out, ldo, (const bf16_t*)kcache, (const bf16_t*)vcache, block_table, max_blocks, \
                 tiles, positions, maps, per_kv, kv_heads * maps, kv_heads, dv, page_shift, window, scale, softcap, partial, per_split, \
                 share, q_slots, keep_first, sinks, chunk, slopes

@@ -1573,7 +1573,8 @@ def _fast_attention_dv(q, out, k_cache, v_cache, block_table, row_req, positions
         # as many workgroups as are resident at once (two per compute unit; one for the instantiations with keys or
         # values beyond 128, whose LDS buffers fill a unit): a second round would start its chains of loads all over.
         # The heads of a key slot share a workgroup
-        resident = (2 if dk <= 128 and dv <= 128 else 1) * compute_units()
+        rows_kernel = dk == 128 and dv in (128, 256) and heads // kv_heads <= 16
+        resident = (2 if rows_kernel or (dk <= 128 and dv <= 128) else 1) * compute_units()
         want = max(1, resident // max(1, n_tiles * kv_heads * maps))
         splits = max(1, min(want, blocks // WIDE_SPLIT_MIN_BLOCKS, 64))
         if splits > 1:

@@ -585,3 +585,55 @@ def test_command_line_runs_the_design(folders, tmp_path):
     assert r.returncode == 0, r.stderr[-2000:]
     out = json.loads(r.stdout.strip().splitlines()[-1])
     assert out["tokens"] == P.greedy(kt.K_C, kt.load_weights(folders["KC"]), [3, 1, 4, 1, 5], 6)
+
+
+@pytest.mark.parametrize("heads,kv_heads,maps,dv", [(16, 8, 1, 128), (8, 4, 2, 256), (4, 4, 1, 256), (32, 2, 1, 128), (20, 1, 1, 128)])
+@pytest.mark.parametrize("kw", [{}, {"softcap": 20.0}, {"window": 100}, {"window": 70, "keep_first": 5}, {"window": 300, "keep_first": 130}, {"chunk": 96},
+                                {"slopes": True}])
+def test_single_rows_at_key_size_128(heads, kv_heads, maps, dv, kw):
+    """Rows of one key, of one block and of many, whole and in key ranges (merged by a launch and by the kernel that finishes the
+    heads), against the general kernel: probabilities rounded to bf16 move an output by at most 2^-8 of the largest value, and a
+    row is the same alone as beside others. Values and keys outside what a row sees are infinite: they must not reach it. (20
+    heads over one key slot: more than the kernel has columns, the tile kernel takes them.)"""
+    from jllm_serve_amd.kernels import ops
+    dk, page, ctx = 128, 16, (1, 64, 65, 700, 1999)
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(heads + dv + len(str(kw)))
+    rnd = lambda *shape: torch.randn(*shape, device=DEV, generator=gen)
+    T, width = len(ctx), -(-max(ctx) // page)
+    table = torch.randperm(T * width, device=DEV, generator=gen).to(torch.int32).view(T, width)
+    kc, vc = rnd(T * width, kv_heads * maps, page, dk).bfloat16(), rnd(T * width, kv_heads, page, dv).bfloat16()
+    kw = dict(kw)
+    window, keep, chunk = kw.get("window", 0), kw.get("keep_first", 0), kw.get("chunk", 0)
+    if kw.pop("slopes", False):
+        kw["slopes"] = rnd(heads).abs() * 0.02
+    if maps == 1 and window:
+        kw["sinks"] = rnd(heads)
+    q = rnd(T, heads * maps * dk).bfloat16()
+    rows, pos = torch.arange(T, dtype=torch.int32, device=DEV), torch.tensor([c - 1 for c in ctx], dtype=torch.int32, device=DEV)
+    args = (q, kc, vc, table, rows, pos, heads, kv_heads, maps, dk, dv, dk ** -0.5)
+    want = ops.attention_dv(*args, exact=True, out_dtype=torch.float32, **kw)
+    for r, c in enumerate(ctx):
+        first = max(0, c - window) if window else (c - 1) // chunk * chunk if chunk else 0
+        for p in range(width * page):
+            if p >= c or (p < first and p >= keep):
+                kc[table[r, p // page], :, p % page] = float("inf")
+                vc[table[r, p // page], :, p % page] = float("inf")
+    tiles = torch.tensor([[r, r, 1, -1] for r in range(T)], dtype=torch.int32, device=DEV).flatten()
+    bound = 2.0 ** -8 * 6.0
+    for longest in (64, max(ctx)):  # the step's longest request decides the key ranges; rows beyond it are left out
+        n = sum(c <= longest for c in ctx)
+        meta = {"tiles_dev": tiles[:4 * n].contiguous(), "n_tiles": n, "single_rows": True, "max_context": longest}
+        part = (q[:n].contiguous(), kc, vc, table, rows[:n].contiguous(), pos[:n].contiguous(), *args[6:])
+        got = ops.attention_dv(*part, meta=meta, out_dtype=torch.float32, **kw)
+        assert bool(torch.isfinite(got).all()) and float((got - want[:n]).abs().max()) <= bound
+        split = ops.attention_dv(*part, meta=meta, out_dtype=torch.float32, defer_merge=True, **kw)
+        assert isinstance(split, ops.SplitHeads) or longest == 64 or window or chunk
+        if isinstance(split, ops.SplitHeads):
+            done = ops.heads_finish(split, heads, maps, dv, torch.float32, lam=0.3)
+            ref = ops.heads_finish(want[:n].contiguous(), heads, maps, dv, torch.float32, lam=0.3)
+            assert float((done - ref).abs().max()) <= 2 * bound
+            one = {**meta, "n_tiles": 1, "tiles_dev": torch.tensor([n - 1, 0, 1, -1], dtype=torch.int32, device=DEV)}
+            alone = ops.attention_dv(q[n - 1:n].contiguous(), kc, vc, table, rows[n - 1:n].contiguous(), pos[n - 1:n].contiguous(), *args[6:],
+                                     meta=one, out_dtype=torch.float32, **kw)
+            assert float((alone - got[n - 1:n]).abs().max()) <= bound
