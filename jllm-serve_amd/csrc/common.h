@@ -158,6 +158,10 @@ extern "C" int jllm_compute_units();  // of the current GPU (elementwise.hip)
 int jllm_splitk_reduce(const float* partial, int splits, const void* bias, int bias_dtype, void* out, int out_dtype,
                        int ldo, int M, int N, int epilogue, hipStream_t stream);
 
+// the same for the accumulate epilogue, with the RMSNorm of the new rows (gemm_mfma.hip)
+int jllm_splitk_reduce_norm(const float* partial, int splits, const void* bias, int bias_dtype, void* out, int out_dtype, int ldo, int M, int N,
+                            int epilogue, const void* gain, int gain_dtype, float eps, void* rows, int ldr, hipStream_t stream);
+
 #define JLLM_FAIL(...)           \
   do {                           \
     jllm_set_error(__VA_ARGS__); \

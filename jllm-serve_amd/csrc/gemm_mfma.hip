@@ -281,6 +281,96 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   }
 }
 
+// The reduction of a product that adds into the residual, and the RMSNorm of the new rows, in one pass: a workgroup per row,
+// which stays in registers (N <= 8,192, a multiple of 4, rows without gaps), everything it reads requested before the first
+// sum. The bits are those of the reduction above followed by the norm kernel (elementwise.hip): parts in ascending order, bias,
+// residual, then the squares by thread, wave and block. Bound by its bytes; the norm's own pass read the rows again
+// and cost a launch: 2,048 rows of 4,096 in two parts 22.4 + 13.4 -> 25.7 us, 631 in four 10.1 + 6.6 -> 12.5. (With a branch
+// around every load, as in the kernels it replaces, 46 and 22.)
+template <typename TG, int J>
+__global__ __launch_bounds__(256) void splitk_reduce_norm_kernel(const float* __restrict__ partial, int splits, const void* __restrict__ bias,
+                                                                 int bias_dtype, float* __restrict__ out, int M, int N,
+                                                                 const TG* __restrict__ gain, float eps, bf16_t* __restrict__ rows, int ldr) {
+  __shared__ float red[4];
+  const int nv = N >> 2;  // fours of a row: thread t has number t, t + 256, ..; beyond the end it reads the last one again (no
+                          // branch around a load: the compiler would wait for everything behind one)
+  const size_t row = (size_t)blockIdx.x * N;
+  int at[J];
+  floatx4 v[J], res[J];
+  TG g[J][4];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    at[j] = 4 * min((int)threadIdx.x + 256 * j, nv - 1);
+    v[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    res[j] = *(const floatx4*)(out + row + at[j]);
+    if (sizeof(TG) == 2)
+      *(uint2*)g[j] = *(const uint2*)(gain + at[j]);
+    else
+      *(uint4*)g[j] = *(const uint4*)(gain + at[j]);
+  }
+  int z = 0;
+  for (; z + 2 <= splits; z += 2) {
+    const float* p = partial + (size_t)z * M * N + row;
+    const float* p2 = p + (size_t)M * N;
+    floatx4 a[J], b[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) a[j] = *(const floatx4*)(p + at[j]);
+#pragma unroll
+    for (int j = 0; j < J; ++j) b[j] = *(const floatx4*)(p2 + at[j]);
+#pragma unroll
+    for (int j = 0; j < J; ++j) v[j] = (v[j] + a[j]) + b[j];
+  }
+  if (z < splits) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) v[j] += *(const floatx4*)(partial + (size_t)z * M * N + row + at[j]);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    if (bias)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[j][e] += (bias_dtype == JLLM_BF16) ? ldf((const bf16_t*)bias, at[j] + e) : ldf((const float*)bias, at[j] + e);
+    v[j] = res[j] + v[j];
+    if ((int)threadIdx.x + 256 * j < nv) {
+      *(floatx4*)(out + row + at[j]) = v[j];
+      ss += v[j][0] * v[j][0] + v[j][1] * v[j][1] + v[j][2] * v[j][2] + v[j][3] * v[j][3];
+    }
+  }
+  ss = block_sum<4>(ss, red);
+  const float s = norm_scale(ss, N, eps);
+  bf16_t* o = rows + (size_t)blockIdx.x * ldr;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    if ((int)threadIdx.x + 256 * j >= nv) continue;
+    float r[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = (v[j][e] * s) * ldf(g[j], e);
+    *(uint2*)(o + at[j]) = uint2{(uint32_t)f32_to_bf16(r[0]).bits | ((uint32_t)f32_to_bf16(r[1]).bits << 16),
+                                 (uint32_t)f32_to_bf16(r[2]).bits | ((uint32_t)f32_to_bf16(r[3]).bits << 16)};
+  }
+}
+
+int jllm_splitk_reduce_norm(const float* partial, int splits, const void* bias, int bias_dtype, void* out, int out_dtype, int ldo, int M, int N,
+                            int epilogue, const void* gain, int gain_dtype, float eps, void* rows, int ldr, hipStream_t stream) {
+  if (epilogue != 1 || out_dtype != JLLM_F32 || ldo != N || (N & 3) || N > 8192 || ldr < N || (ldr & 3) || !gain || (((uintptr_t)out | (uintptr_t)partial) & 15) ||
+      ((uintptr_t)rows & 7))
+    JLLM_FAIL("splitk_reduce_norm: rows of %d (stride %d) and a norm's of stride %d", N, ldo, ldr);
+  if ((uintptr_t)gain & 15) JLLM_FAIL("splitk_reduce_norm: a gain that is not aligned to 16 bytes");
+#define SRN_CASE(J)                                                                                                                                    \
+  case J:                                                                                                                                              \
+    splitk_reduce_norm_kernel<TG, J><<<M, 256, 0, stream>>>(partial, splits, bias, bias_dtype, (float*)out, M, N, (const TG*)gain, eps, (bf16_t*)rows, ldr); \
+    break;
+  JLLM_DISPATCH_1(gain_dtype, TG, {
+    switch ((N / 4 + 255) / 256) {
+      SRN_CASE(1) SRN_CASE(2) SRN_CASE(3) SRN_CASE(4) SRN_CASE(5) SRN_CASE(6) SRN_CASE(7) SRN_CASE(8)
+    }
+  })
+#undef SRN_CASE
+  JLLM_CHECK_LAUNCH("splitk_reduce_norm");
+  return 0;
+}
+
 int jllm_splitk_reduce(const float* partial, int splits, const void* bias, int bias_dtype, void* out, int out_dtype,
                        int ldo, int M, int N, int epilogue, hipStream_t stream) {
   const size_t total = (size_t)M * N;
@@ -321,10 +411,12 @@ static int launch_tiled(const void* A, int lda, const void* W, const void* W2, c
 }
 
 // `splits` > 1 cuts K over gridDim.z (not with the gated epilogue); `partial` then holds splits * M * N floats.
+// `norm_rows` [M][norm_ld] bf16 (with cuts of K and the accumulate epilogue): the RMSNorm of the new rows, made by the reduction.
 // returns 0 when it ran, 1 when the shape is not one it takes, -1 on errors
 extern "C" int jllm_gemm_mfma_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias,
                                    int bias_dtype, void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue,
-                                   float gate_limit, int splits, float* partial, hipStream_t stream) {
+                                   float gate_limit, int splits, float* partial, const void* norm_gain, int norm_gain_dtype, float norm_eps,
+                                   void* norm_rows, int norm_ld, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || (K % TBK) || (lda & 7)) return 1;
   if (((uintptr_t)A & 15) || ((uintptr_t)W & 15) || (W2 && ((uintptr_t)W2 & 15))) return 1;
@@ -334,6 +426,7 @@ extern "C" int jllm_gemm_mfma_bf16(const void* A, int lda, const void* W, const 
   if (ldo < N) JLLM_FAIL("gemm_mfma: ldo %d < N %d", ldo, N);
   if (splits < 1) splits = 1;
   if (splits > 1 && (W2 || !partial || (K / TBK) % splits != 0)) JLLM_FAIL("gemm_mfma: %d K splits are not possible here", splits);
+  if (norm_rows && splits == 1) JLLM_FAIL("gemm_mfma: the norm is the reduction's, and K is whole");
   // the large tile when it still gives every compute unit two rounds of work, or when one round of it fills three
   // quarters of the compute units or more (the small tile would then need a second, half-empty round)
   const long big_tiles = (long)((N + (W2 ? 127 : 255)) / (W2 ? 128 : 256)) * ((M + 255) / 256);
@@ -354,6 +447,8 @@ extern "C" int jllm_gemm_mfma_bf16(const void* A, int lda, const void* W, const 
   }
   if (rc != 0) return rc;
   JLLM_CHECK_LAUNCH("gemm_mfma");
+  if (splits > 1 && norm_rows)
+    return jllm_splitk_reduce_norm(partial, splits, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, norm_gain, norm_gain_dtype, norm_eps, norm_rows, norm_ld, stream);
   if (splits > 1) return jllm_splitk_reduce(partial, splits, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, stream);
   return 0;
 }

@@ -257,10 +257,12 @@ static int launch_pingpong(const void* A, int lda, const void* W, const void* W2
 
 // `tile_rows`: 256 or 192 (rows of the output tile; 256 columns, 128 outputs with the gated epilogue).
 // `splits` > 1 cuts K over gridDim.z (not with the gated epilogue): `partial` then holds splits * M * N floats, summed
-// in ascending order of the split by the other tiled kernel's reduction. Returns 0 when it ran, 1 when the shape is not one it takes, -1 on errors.
+// in ascending order of the split by the other tiled kernel's reduction, which also makes the RMSNorm of the new rows where
+// `norm_rows` is given (as there). Returns 0 when it ran, 1 when the shape is not one it takes, -1 on errors.
 extern "C" int jllm_gemm_pingpong_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias,
                                        int bias_dtype, void* out, int out_dtype, int ldo, int M, int N, int K,
-                                       int epilogue, float gate_limit, int tile_rows, int splits, float* partial, hipStream_t stream) {
+                                       int epilogue, float gate_limit, int tile_rows, int splits, float* partial, const void* norm_gain,
+                                       int norm_gain_dtype, float norm_eps, void* norm_rows, int norm_ld, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || (K % PP_BK) || (lda & 7)) return 1;
   if (((uintptr_t)A & 15) || ((uintptr_t)W & 15) || (W2 && ((uintptr_t)W2 & 15))) return 1;
@@ -272,6 +274,7 @@ extern "C" int jllm_gemm_pingpong_bf16(const void* A, int lda, const void* W, co
   if ((unsigned long long)M * (unsigned)lda * 2ull >= (1ull << 32) || (unsigned long long)N * (unsigned)K * 2ull >= (1ull << 32)) return 1;
   if (splits < 1) splits = 1;
   if (splits > 1 && (W2 || !partial)) JLLM_FAIL("gemm_pingpong: %d K splits are not possible here", splits);
+  if (norm_rows && splits == 1) JLLM_FAIL("gemm_pingpong: the norm is the reduction's, and K is whole");
   if (splits > 65535 || (K / PP_BK) / splits < 4) return 1;
   int rc;
   if (tile_rows == 256)
@@ -282,6 +285,8 @@ extern "C" int jllm_gemm_pingpong_bf16(const void* A, int lda, const void* W, co
     JLLM_FAIL("gemm_pingpong: tile of %d rows (256 and 192 are built)", tile_rows);
   if (rc != 0) return rc;
   JLLM_CHECK_LAUNCH("gemm_pingpong");
+  if (splits > 1 && norm_rows)
+    return jllm_splitk_reduce_norm(partial, splits, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, norm_gain, norm_gain_dtype, norm_eps, norm_rows, norm_ld, stream);
   if (splits > 1) return jllm_splitk_reduce(partial, splits, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, stream);
   return 0;
 }

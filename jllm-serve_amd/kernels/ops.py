@@ -118,8 +118,8 @@ def _declare(lib) -> None:
 _OPTIONAL_SIGS = {
     "jllm_gemm_skinny_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P],
     "jllm_gemm_skinny_norm_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _P, _I, _P, _I, _F, _P],
-    "jllm_gemm_mfma_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P],
-    "jllm_gemm_pingpong_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P, _P],
+    "jllm_gemm_mfma_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _F, _P, _I, _P],
+    "jllm_gemm_pingpong_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P, _P, _I, _F, _P, _I, _P],
     "jllm_gemm_stream_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _P, _P, _I, _P, _I, _P, _I, _P, _I, _F, _P],
     "jllm_decode_attention_bf16": [_P, _I, _P, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _I, _P],
     "jllm_decode_attention_fused_bf16": [_P, _I, _P, _I, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _F, _I, _I, _I, _I, _I,
@@ -420,20 +420,27 @@ def gemm_add_then_norm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gain
     and ``eps``, as a ``NormedRows``: for few bf16 rows the product prepares that norm on its way out."""
     if isinstance(a, NormedRows):
         a = a.tensor()
-    if not exact and norm_dtype == torch.bfloat16 and a.dim() == 2 and a.dtype == torch.bfloat16 \
-            and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() \
-            and w.shape[1] == a.shape[1] and w.shape[0] % 16 == 0 and 0 < a.shape[0] and _norm_rides(*a.shape, w.shape[0]) and a.stride(1) == 1 \
-            and out.dtype == torch.float32 and out.dim() == 2 and out.shape == (a.shape[0], w.shape[0]) and out.is_contiguous() \
-            and gain.numel() == w.shape[0] and gain.is_contiguous() \
-            and (bias is None or (bias.numel() == w.shape[0] and bias.is_contiguous())):
+    fits = not exact and norm_dtype == torch.bfloat16 and a.dim() == 2 and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 \
+        and w.dim() == 2 and w.is_contiguous() and w.shape[1] == a.shape[1] and w.shape[0] % 16 == 0 and 0 < a.shape[0] and a.stride(1) == 1 \
+        and out.dtype == torch.float32 and out.dim() == 2 and out.shape == (a.shape[0], w.shape[0]) and out.is_contiguous() \
+        and gain.numel() == w.shape[0] and gain.is_contiguous() and (bias is None or (bias.numel() == w.shape[0] and bias.is_contiguous()))
+    if fits:
         _dev(a, w, bias, out, gain)
+    if fits and _norm_rides(*a.shape, w.shape[0]):
         M, N = out.shape
         scaled = activation_rows(M, N, torch.bfloat16, out.device)
         partials = torch.empty((M, _norm_partials(M, N, a.shape[1])), dtype=torch.float32, device=out.device)
         if _skinny_norm(a, w, None, bias, out, EPI_ADD, emit=(scaled, gain, partials)):
             return NormedRows(out, gain, eps, norm_dtype, scaled, partials)
+    promise = NormedRows(out, gain, eps, norm_dtype)
+    if fits and _cut_takes_norm(*out.shape, a.shape[1]) and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and a.stride(0) % 8 == 0 \
+            and out.data_ptr() % 16 == 0 and gain.data_ptr() % 16 == 0:
+        rows = activation_rows(*out.shape, norm_dtype, out.device)
+        if _fast_gemm(a, w, None, bias, out, EPI_ADD, norm=(_ptr(gain), _code(gain.dtype), float(eps), _ptr(rows), rows.stride(0))):
+            promise._rows = rows
+            return promise
     gemm(a, w, bias=bias, out=out, epilogue=EPI_ADD, exact=exact)
-    return NormedRows(out, gain, eps, norm_dtype)
+    return promise
 
 
 def gemm(a: torch.Tensor, w: torch.Tensor, *, w2: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None,
@@ -952,10 +959,23 @@ def _few_rows_prefer_stream(N: int, K: int, gated: bool) -> bool:
     return not gated and K % 128 == 0 and N % 16 == 0 and N <= STREAM_FEW_ROWS[0] and K >= STREAM_FEW_ROWS[1]
 
 
-def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0) -> bool:
+_NO_NORM = (None, F32, 0.0, None, 0)
+
+
+def _cut_takes_norm(M: int, N: int, K: int) -> bool:
+    """Whether the adding product of M rows goes to a tiled kernel that cuts K: its reduction then makes the norm of the new
+    rows as well."""
+    if M <= STREAM_MAX_ROWS or K % 64 or N % 4 or N > 8192 or _wide_plan(M, N, K, False, True) is not None:
+        return False
+    rows, cut = _tiled_plan(M, N, K, False)
+    return (cut if rows else _k_splits(M, N, K, False)) > 1
+
+
+def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0, norm=_NO_NORM) -> bool:
     """The bf16 matrix-core kernels: a weight-streaming one for up to 16 rows, another for up to 64; for many rows
     the two-group kernel with tiles of 256 or 192 rows by 256 columns or the small tile, either with K cut over several
-    workgroups when the output has few tiles (`_tiled_plan`). Each declines shapes it does
+    workgroups when the output has few tiles (`_tiled_plan`); then the reduction makes the ``norm`` (gain, its type, eps, rows,
+    their stride) of the new rows where one is asked for. Each declines shapes it does
     not take; then the fp32 kernel runs."""
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         return False
@@ -973,11 +993,13 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0) -> bool:
     tile_rows, cut = _tiled_plan(M, N, K, w2 is not None)
     if tile_rows:
         partial = torch.empty((cut * M * N,), dtype=torch.float32, device=a.device) if cut > 1 else None
-        if _try("jllm_gemm_pingpong_bf16", *head, tile_rows, cut, _ptr(partial), _stream()):
+        if _try("jllm_gemm_pingpong_bf16", *head, tile_rows, cut, _ptr(partial), *norm, _stream()):
             return True
     splits = _k_splits(M, N, K, w2 is not None) if K % 64 == 0 else 1
+    if splits == 1 and norm is not _NO_NORM:
+        return False  # (the other kernel declined, and here K stays whole: no reduction to make the norm)
     partial = torch.empty((splits * M * N,), dtype=torch.float32, device=a.device) if splits > 1 else None
-    if _try("jllm_gemm_mfma_bf16", *head, splits, _ptr(partial), _stream()):
+    if _try("jllm_gemm_mfma_bf16", *head, splits, _ptr(partial), *norm, _stream()):
         return True
     return False
 

@@ -389,6 +389,27 @@ def test_products_of_more_rows_at_any_plan(ops, monkeypatch, M, N, K, parts, row
     assert set(ops.stats()["ran"]) == {"jllm_gemm_stream_bf16"} and promise._rows is None
 
 
+@pytest.mark.parametrize("M,N,K,tile,cut", [(65, 1024, 2048, 0, 4), (631, 4096, 4096, 256, 2), (300, 2560, 4096, 192, 2), (130, 8192, 1024, 0, 2),
+                                            (700, 96, 2048, 0, 8), (70, 1040, 1024, 0, 1)])
+@pytest.mark.parametrize("gdt", [torch.bfloat16, torch.float32])
+def test_the_reduction_makes_the_norm(ops, monkeypatch, M, N, K, tile, cut, gdt):
+    """An adding product of many rows with K cut: the residual and the rows for the next product have the bits of the reduction
+    and the norm as launches of their own, with and without a bias, in rows with a stride; with K whole the norm stays a launch."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M + N + K)
+    rnd = lambda *shape: torch.randn(*shape, device=DEV, generator=gen)
+    a, w, res0, gain = rnd(M, K).bfloat16(), (rnd(N, K) / math.sqrt(K)).bfloat16(), rnd(M, N), (rnd(N).abs() + 0.5).to(gdt)
+    monkeypatch.setattr(ops, "_wide_plan", lambda *_: None)
+    monkeypatch.setattr(ops, "_tiled_plan", lambda *_: (tile, cut))
+    monkeypatch.setattr(ops, "_k_splits", lambda *_: cut)
+    for bias in (None, rnd(N), rnd(N).bfloat16()):
+        want, got = res0.clone(), res0.clone()
+        ops.gemm(a, w, bias=bias, out=want, epilogue=ops.EPI_ADD)
+        promise = ops.gemm_add_then_norm(a, w, got, gain, 1e-5, torch.bfloat16, bias=bias)
+        assert torch.equal(got, want) and promise.scaled is None and (promise._rows is not None) == (cut > 1)
+        assert torch.equal(promise.tensor().view(torch.int16), ops.rmsnorm(want, gain, 1e-5, torch.bfloat16).view(torch.int16))
+
+
 def test_gemm_rows_do_not_depend_on_the_batch(ops):
     """The result of a row is the same bits whether it is alone or among others, within one kernel family (the
     bfloat16 path has one kernel for up to 16 rows, one for up to 64 and one for more; between them results differ
