@@ -55,10 +55,10 @@ extern "C" int jllm_embed(const void* table, int table_dtype, const int* ids, fl
 // ---------------------------------------------------------------------------------------------------------
 // RMSNorm of fp32 rows: y = (x * rsqrt(mean(x^2) + eps)) * g. One block per output row; `rows` (optional)
 // picks the input row of each output row; output rows lie `ldo` elements apart. Sum of squares, the reciprocal root and both products are fp32.
-// Rows of up to 8192 values whose width is a multiple of 4 are read once, 16 bytes per lane, and held in
-// registers (every load is in flight at the same time: the kernel is bound by latency, not by bytes);
-// other widths take the two-pass loop.
-template <typename TG, typename TO>
+// Rows of up to 8192 values whose width is a multiple of 4 are read once, 16 bytes per lane, and held in J vectors of registers
+// per thread (J = 0: other widths and gains that are not 16-byte aligned take the two-pass loop). 2,048 rows of 4,096 13.4 ->
+// 9.7 us (50 MB: 5.2 TB/s) since no branch stands around a load.
+template <typename TG, typename TO, int J>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ x, const int* __restrict__ rows,
                                                       const TG* __restrict__ gain, TO* __restrict__ out, int ldo, int d,
                                                       float eps) {
@@ -66,39 +66,35 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ 
   const int r = blockIdx.x;
   const float* xi = x + (size_t)(rows ? rows[r] : r) * d;
   TO* o = out + (size_t)r * ldo;
-  if ((d & 3) == 0 && d <= 8192) {
+  if constexpr (J > 0) {
+    constexpr int JN = J > 0 ? J : 1;
     const int nv = d >> 2;
-    float4 v[8], gn[8];
+    float4 v[JN];
+    TG gn[JN][4];
+    int at[JN];
     float ss = 0.f;
-    // the gains are requested together with the row, as 8- or 16-byte loads, so that nothing is waited for twice
-    const bool gvec = (((uintptr_t)gain) & 15) == 0;
+    // the gains are requested together with the row; beyond the row's end its last four again (a branch around a load makes
+    // the compiler wait for everything behind it)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int i = threadIdx.x + 256 * j;
-      v[j] = i < nv ? ((const float4*)xi)[i] : float4{0.f, 0.f, 0.f, 0.f};
-      gn[j] = float4{0.f, 0.f, 0.f, 0.f};
-      if (i < nv) {
-        if (!gvec) {
-          gn[j] = float4{ldf(gain, 4 * i), ldf(gain, 4 * i + 1), ldf(gain, 4 * i + 2), ldf(gain, 4 * i + 3)};
-        } else if (sizeof(TG) == 2) {
-          const uint2 u = ((const uint2*)gain)[i];
-          gn[j] = float4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
-                         __uint_as_float(u.y & 0xffff0000u)};
-        } else {
-          gn[j] = ((const float4*)gain)[i];
-        }
-      }
+    for (int j = 0; j < J; ++j) {
+      at[j] = min((int)threadIdx.x + 256 * j, nv - 1);
+      v[j] = ((const float4*)xi)[at[j]];
+      if (sizeof(TG) == 2)
+        *(uint2*)gn[j] = ((const uint2*)gain)[at[j]];
+      else
+        *(uint4*)gn[j] = ((const uint4*)gain)[at[j]];
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+    for (int j = 0; j < J; ++j)
+      if ((int)threadIdx.x + 256 * j < nv) ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
     ss = block_sum<4>(ss, red);
     const float s = norm_scale(ss, d, eps);
     const bool ovec = (((uintptr_t)o) & 15) == 0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < J; ++j) {
       const int i = threadIdx.x + 256 * j;
       if (i < nv) {
-        const float a = (v[j].x * s) * gn[j].x, b = (v[j].y * s) * gn[j].y, c = (v[j].z * s) * gn[j].z, e = (v[j].w * s) * gn[j].w;
+        const float a = (v[j].x * s) * ldf(gn[j], 0), b = (v[j].y * s) * ldf(gn[j], 1), c = (v[j].z * s) * ldf(gn[j], 2), e = (v[j].w * s) * ldf(gn[j], 3);
         if (!ovec) {
           stf(o, 4 * i, a);
           stf(o, 4 * i + 1, b);
@@ -129,11 +125,18 @@ extern "C" int jllm_rmsnorm(const float* x, const int* rows, int n_rows, int d, 
   if (n_rows <= 0) return 0;
   if (d <= 0) JLLM_FAIL("rmsnorm: width %d", d);
   if (ldo < d) JLLM_FAIL("rmsnorm: output row stride %d < width %d", ldo, d);
+#define RN_CASE(J)                                                                                            \
+  case J:                                                                                                      \
+    rmsnorm_kernel<TG, TO, J><<<n_rows, 256, 0, stream>>>(x, rows, (const TG*)gain, (TO*)out, ldo, d, eps);     \
+    break;
   JLLM_DISPATCH_1(gain_dtype, TG, {
     JLLM_DISPATCH_1(out_dtype, TO, {
-      rmsnorm_kernel<TG, TO><<<n_rows, 256, 0, stream>>>(x, rows, (const TG*)gain, (TO*)out, ldo, d, eps);
+      switch ((d & 3) == 0 && d <= 8192 && ((uintptr_t)gain & 15) == 0 && ((uintptr_t)x & 15) == 0 ? (d / 4 + 255) / 256 : 0) {
+        RN_CASE(0) RN_CASE(1) RN_CASE(2) RN_CASE(3) RN_CASE(4) RN_CASE(5) RN_CASE(6) RN_CASE(7) RN_CASE(8)
+      }
     })
   })
+#undef RN_CASE
   JLLM_CHECK_LAUNCH("rmsnorm");
   return 0;
 }
