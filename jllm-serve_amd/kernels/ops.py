@@ -388,9 +388,10 @@ def _skinny_norm(a, w, w2, bias, out, epilogue, emit=None, normed: Optional[Norm
     does not take the case."""
     M, K = a.shape
     N = w.shape[0]
-    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or (M > STREAM_MAX_ROWS and _wide_plan(M, N, K, w2 is not None, epilogue == EPI_ADD) is None):
-        return False
     e_rows, e_gain, e_part = emit if emit is not None else (None, None, None)
+    adds = _adds(epilogue, emit is not None)
+    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or (M > STREAM_MAX_ROWS and _wide_plan(M, N, K, w2 is not None, adds) is None):
+        return False
     n_part = normed.partials if normed is not None else None
     head = (_ptr(a), a.stride(0), _ptr(w), _ptr(w2), _ptr(bias), _code(bias.dtype) if bias is not None else F32,
             _ptr(out), _code(out.dtype), out.stride(0), M, N, K, int(epilogue), float(gate_limit))
@@ -401,23 +402,37 @@ def _skinny_norm(a, w, w2, bias, out, epilogue, emit=None, normed: Optional[Norm
     if few and not _few_rows_prefer_stream(N, K, w2 is not None):
         return _try("jllm_gemm_skinny_norm_bf16", *head, _skinny_rows(N, K, w2 is not None), *emits, emit_parts, *takes)
     if K % 128 == 0:
-        rows, tile, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a, epilogue == EPI_ADD)
+        rows, tile, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a, adds)
         if _try("jllm_gemm_stream_bf16", *head, rows, tile, parts, _ptr(sums), _ptr(arrivals), _ptr(e_rows), e_rows.stride(0) if e_rows is not None else 0, *emits[1:],
                 emit_parts, *takes):
             return True
     return few and _try("jllm_gemm_skinny_norm_bf16", *head, 16, *emits, emit_parts, *takes)  # the second kernel declined
 
 
-def _norm_rides(M: int, K: int, N: int) -> bool:
-    """Whether the adding product of M rows, K and N prepares the norm that follows. For more than 64 rows it does so where
-    the same kernel takes it, from the row count on at which the rows may be laid out for many rows (`activation_rows`)."""
-    return M <= STREAM_MAX_ROWS or (M >= PAD_ROWS_FROM and _wide_plan(M, N, K, False, True) is not None)
+ADDS, ADDS_AND_NORM = 1, 2  # `adds` of a plan: into the residual, and with the rows for the norm behind it
+
+
+def _adds(epilogue: int, emits: bool = False) -> int:
+    return 0 if epilogue != EPI_ADD else ADDS_AND_NORM if emits else ADDS
+
+
+def _norm_rides(M: int, N: int, K: int, reader: Optional[Tuple[int, bool]]) -> bool:
+    """Whether the adding product of M rows, N outputs and K inputs prepares the norm that follows. For more than 64 rows it
+    does so where the same kernel takes both it and the product that reads the norm (``reader``: its outputs and whether it is
+    gated; not known: plain, with N outputs), from the row count on at which the rows may be laid out for many rows
+    (`activation_rows`). A norm that is prepared for a reader which does not take it is made again by a launch of its own."""
+    if M <= STREAM_MAX_ROWS:
+        return True
+    outputs, gated = reader if reader is not None else (N, False)
+    return M >= PAD_ROWS_FROM and _wide_plan(M, outputs, N, gated, 0) is not None and _wide_plan(M, N, K, False, ADDS_AND_NORM) is not None
 
 
 def gemm_add_then_norm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gain: torch.Tensor, eps: float,
-                       norm_dtype: torch.dtype, *, bias: Optional[torch.Tensor] = None, exact: bool = False) -> NormedRows:
+                       norm_dtype: torch.dtype, *, bias: Optional[torch.Tensor] = None, exact: bool = False,
+                       reader: Optional[Tuple[int, bool]] = None) -> NormedRows:
     """``out += a @ w.T (+ bias)`` (the fp32 residual), returning the RMSNorm of the new ``out`` rows, with ``gain``
-    and ``eps``, as a ``NormedRows``: for few bf16 rows the product prepares that norm on its way out."""
+    and ``eps``, as a ``NormedRows``: for few bf16 rows the product prepares that norm on its way out. ``reader``: the product
+    that the norm is for, as (outputs, whether gated), where the caller knows it."""
     if isinstance(a, NormedRows):
         a = a.tensor()
     fits = not exact and norm_dtype == torch.bfloat16 and a.dim() == 2 and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 \
@@ -426,7 +441,7 @@ def gemm_add_then_norm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gain
         and gain.numel() == w.shape[0] and gain.is_contiguous() and (bias is None or (bias.numel() == w.shape[0] and bias.is_contiguous()))
     if fits:
         _dev(a, w, bias, out, gain)
-    if fits and _norm_rides(*a.shape, w.shape[0]):
+    if fits and _norm_rides(*out.shape, a.shape[1], reader):
         M, N = out.shape
         scaled = activation_rows(M, N, torch.bfloat16, out.device)
         partials = torch.empty((M, _norm_partials(M, N, a.shape[1])), dtype=torch.float32, device=out.device)
@@ -801,7 +816,7 @@ def _norm_partials(M: int, N: int, K: int) -> int:
     """Partial sums of squares per row that a product with N outputs leaves for the norm behind it: room for one per
     workgroup's columns, in whole fours."""
     if M > STREAM_MAX_ROWS:
-        groups = -(-N // _wide_plan(M, N, K, False, True)[0])
+        groups = -(-N // _wide_plan(M, N, K, False, ADDS_AND_NORM)[0])
     elif M > SKINNY_MAX_ROWS or _few_rows_prefer_stream(N, K, False):
         groups = max(N // 16, -(-N // _stream_plan(N, K, False)[0])) if M <= SKINNY_MAX_ROWS else -(-N // _stream_plan(N, K, False)[0])
     else:
@@ -856,7 +871,7 @@ def step_scratch(rows: int, device):
 STREAM_COUNTERS = 1024
 
 
-def _stream_scratch(M: int, N: int, K: int, gated: bool, a: torch.Tensor, adds: bool):
+def _stream_scratch(M: int, N: int, K: int, gated: bool, a: torch.Tensor, adds: int):
     """The plan and scratch of the kernel behind `_stream_plan` and `_wide_plan`: (weight rows, activation rows, parts, sums,
     counters)."""
     rows, tile, parts = _plan_of_rows(M, N, K, gated, adds)
@@ -871,7 +886,7 @@ def _stream_scratch(M: int, N: int, K: int, gated: bool, a: torch.Tensor, adds: 
     return rows, tile, parts, partial, arrivals
 
 
-def _plan_of_rows(M: int, N: int, K: int, gated: bool, adds: bool) -> Tuple[int, int, int]:
+def _plan_of_rows(M: int, N: int, K: int, gated: bool, adds: int) -> Tuple[int, int, int]:
     """(weight rows, activation rows, parts of K) of the second weight-streaming kernel for a product that it takes."""
     if M > STREAM_MAX_ROWS:
         return _wide_plan(M, N, K, gated, adds)
@@ -913,13 +928,12 @@ def _wide_us(M: int, N: int, K: int, gated: bool, rows: int, tile: int, parts: i
 
 
 @functools.lru_cache(maxsize=8192)
-def _wide_plan(M: int, N: int, K: int, gated: bool, adds: bool = False) -> Optional[Tuple[int, int, int]]:
+def _wide_plan(M: int, N: int, K: int, gated: bool, adds: int = 0) -> Optional[Tuple[int, int, int]]:
     """(weight rows, activation rows, parts of K) with which the second weight-streaming kernel takes a product of more than
     64 rows, or None where the tiled kernels are estimated to be faster: they move fewer bytes per multiply through a compute
     unit, but their tiles of 128 x 128 and larger leave compute units without work where a product is small, and cutting K
-    costs them a second launch. ``adds``: into the residual, where from 128 rows on it prepares the norm behind it, which is then no launch
-    of its own if the product that reads it is taken here too (asked for one over N inputs: as q, k, v behind a long K, gated
-    behind a short one). Here tiles of 64 or 128 rows by 32 to 128 fill the chip with K whole.
+    costs them a second launch. ``adds``: into the residual (`ADDS`), or there with the norm behind it prepared, which is then no
+    launch of its own (`ADDS_AND_NORM`, see `_norm_rides`). Here tiles of 64 or 128 rows by 32 to 128 fill the chip with K whole.
 
     The constants were fitted to a sweep of every choice for the products of the 0.6B, 1.7B, 4B and 8B shapes at 100, 200, 320, 487 and
     631 rows against what the tiled kernels take. us, tiled / here: 0.6B shape at 487 rows qkv 22.2 / 13.3, o 17.6 / 13.5,
@@ -930,7 +944,7 @@ def _wide_plan(M: int, N: int, K: int, gated: bool, adds: bool = False) -> Optio
     cus = compute_units()
     rows, cut = _tiled_plan(M, N, K, gated)
     best = WIDE_AT_MOST * (TILED_FIXED_US + (_large_us(M, N, K, gated, rows, cut) if rows else _small_us(M, N, K, gated, cut)))
-    if adds and M >= PAD_ROWS_FROM and _wide_plan(M, 2 * N if K > N else 3 * N, N, K <= N):
+    if adds == ADDS_AND_NORM:
         best += NORM_LAUNCH_US
     plan = None
     for rows in (32, 64, 96, 128):
@@ -965,7 +979,7 @@ _NO_NORM = (None, F32, 0.0, None, 0)
 def _cut_takes_norm(M: int, N: int, K: int) -> bool:
     """Whether the adding product of M rows goes to a tiled kernel that cuts K: its reduction then makes the norm of the new
     rows as well."""
-    if M <= STREAM_MAX_ROWS or K % 64 or N % 4 or N > 8192 or _wide_plan(M, N, K, False, True) is not None:
+    if M <= STREAM_MAX_ROWS or K % 64 or N % 4 or N > 8192 or _wide_plan(M, N, K, False, ADDS) is not None:
         return False
     rows, cut = _tiled_plan(M, N, K, False)
     return (cut if rows else _k_splits(M, N, K, False)) > 1
@@ -986,8 +1000,8 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0, norm=_NO_
     if M <= SKINNY_MAX_ROWS and not _few_rows_prefer_stream(N, K, w2 is not None) \
             and _try("jllm_gemm_skinny_bf16", *head, _skinny_rows(N, K, w2 is not None), _stream()):
         return True
-    if K % 128 == 0 and (M <= STREAM_MAX_ROWS or _wide_plan(M, N, K, w2 is not None, epilogue == EPI_ADD) is not None):
-        rows, tile, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a, epilogue == EPI_ADD)
+    if K % 128 == 0 and (M <= STREAM_MAX_ROWS or _wide_plan(M, N, K, w2 is not None, _adds(epilogue)) is not None):
+        rows, tile, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a, _adds(epilogue))
         if _try("jllm_gemm_stream_bf16", *head, rows, tile, parts, _ptr(sums), _ptr(arrivals), None, 0, None, F32, None, 0, None, 0, 0.0, _stream()):
             return True
     tile_rows, cut = _tiled_plan(M, N, K, w2 is not None)

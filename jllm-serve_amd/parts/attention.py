@@ -138,6 +138,9 @@ class GqaAttention(Part):
     def cache_spec(self):
         return KvSpec(self.spec.kv_heads, self.spec.head_dim, self.spec.window)
 
+    def normed_rows_product(self):
+        return self.w_qkv.shape[0], False
+
     def step_planners(self):
         return [self.planner]
 

@@ -6,9 +6,11 @@ xb = norm_post(x); x += ffn(xb). The residual stream x is fp32 and is never norm
 Norms between two products need no launch of their own when both sides agree (optional, by attributes of the
 parts; a part that knows nothing of this works as before):
 * a mixer / feed-forward with ``takes_normed_rows = True`` only feeds its input to ``ops.gemm`` and so may get the
-  norm as a promise (``norm.defer`` / ``ops.NormedRows``) instead of a tensor;
+  norm as a promise (``norm.defer`` / ``ops.NormedRows``) instead of a tensor; ``normed_rows_product()``, where it has one,
+  says what product that is, as (outputs, whether gated);
 * one with ``prepares_next_norm = True`` takes ``then_norm=<norm part>`` in ``forward``, ends with
-  ``then_norm.after_add(...)`` instead of the add into the residual, and returns that promise.
+  ``then_norm.after_add(...)`` instead of the add into the residual, and returns that promise. It is asked only for a
+  norm whose reader takes promises (``norm.reader``, set here).
 """
 from __future__ import annotations
 
@@ -34,6 +36,8 @@ class PreNormBlock(Part):
                                                                 f"{prefix}.{spec.norm_post_name}{ending}", build)
             self.ffn = part_factory("ffn", spec.ffn.kind)(spec.ffn, prefix, build)
             self.parts = (self.norm_in, self.mixer, self.norm_post, self.ffn)
+            self.norm_post.reader = self.ffn
+        self.norm_in.reader = self.mixer
         self.capturable = all(getattr(p, "capturable", True) for p in self.parts)
 
     def weight_specs(self):
@@ -62,22 +66,29 @@ class PreNormBlock(Part):
             return norm.defer(x)
         return norm.forward(x)
 
+    @staticmethod
+    def _prepares(part, norm):
+        """Whether ``part``'s adding product is asked for ``norm`` of what it leaves (a reader that nobody named: yes)."""
+        reader = getattr(norm, "reader", None)
+        return getattr(part, "prepares_next_norm", False) and hasattr(norm, "after_add") \
+            and (reader is None or getattr(reader, "takes_normed_rows", False))
+
     def forward(self, x, step, slot, normed_in=None, next_norm=None):
         """``normed_in``: norm_in of x, prepared by whoever wrote x last (or None); ``next_norm``: the norm part that
         will read x next. Returns that norm of the new x as a promise when the feed-forward prepared it."""
         xb = self._input(self.norm_in, self.mixer, x, normed_in)
         if self.ffn is None:
-            if next_norm is not None and getattr(self.mixer, "prepares_next_norm", False) and hasattr(next_norm, "after_add"):
+            if self._prepares(self.mixer, next_norm):
                 return self.mixer.forward(xb, x, step, slot, then_norm=next_norm)
             self.mixer.forward(xb, x, step, slot)
             return None
-        if getattr(self.mixer, "prepares_next_norm", False) and hasattr(self.norm_post, "after_add"):
+        if self._prepares(self.mixer, self.norm_post):
             mid = self.mixer.forward(xb, x, step, slot, then_norm=self.norm_post)
         else:
             self.mixer.forward(xb, x, step, slot)
             mid = None
         xb = self._input(self.norm_post, self.ffn, x, mid)
-        if next_norm is not None and getattr(self.ffn, "prepares_next_norm", False) and hasattr(next_norm, "after_add"):
+        if self._prepares(self.ffn, next_norm):
             return self.ffn.forward(xb, x, step, then_norm=next_norm)
         self.ffn.forward(xb, x, step)
         return None

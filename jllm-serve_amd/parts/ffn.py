@@ -45,6 +45,9 @@ class GatedMlp(Part):
             self.w_up = get(self._name("up"))
         self.w_down = get(self._name("down"))
 
+    def normed_rows_product(self):
+        return self.hidden, True
+
     def forward(self, xb, residual, step, then_norm=None):
         h = ops.gemm(xb, self.w_gate, w2=self.w_up, epilogue=ops.EPI_GATED, out_dtype=self.build.dtype,
                      exact=self.build.exact, gate=self.gate, gate_limit=self.limit)

@@ -140,6 +140,9 @@ class LatentAttention(Part):
         # one row per position: [latent | rotated key part]; the pages honour the widest window that reads them
         return PageSpec((CacheRow("ckr", (self.kv_width,), 0),), self.spec.keep)
 
+    def normed_rows_product(self):
+        return self.w_in.shape[0], False
+
     def step_planners(self):
         return [LatentStepPlanner()]
 

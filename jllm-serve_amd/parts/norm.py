@@ -19,6 +19,7 @@ class RMSNorm(Part):
         self.out_dtype = build.dtype
         self.one_plus = bool(getattr(spec, "one_plus", False))
         self.gain = self.gain32 = None
+        self.reader = None  # the part whose input this norm makes, where the arrangement says so
 
     def weight_specs(self):
         return [WeightSpec(self.weight_name, (self.dim,), init="bias" if self.one_plus else "gain")]
@@ -48,7 +49,9 @@ class RMSNorm(Part):
     def after_add(self, a, w, residual, bias=None, exact=False):
         """residual += a @ w.T (+ bias), and this norm of the result as a promise: the product that makes the new
         residual rows can prepare their norm on its way out (``ops.gemm_add_then_norm``)."""
-        return ops.gemm_add_then_norm(a, w, residual, self.gain, self.eps, self.out_dtype, bias=bias, exact=exact)
+        reads = getattr(self.reader, "normed_rows_product", None)
+        return ops.gemm_add_then_norm(a, w, residual, self.gain, self.eps, self.out_dtype, bias=bias, exact=exact,
+                                      reader=reads() if reads is not None else None)
 
     def join(self, residual, branches, scales=(1.0, 1.0), branch_gains=None, branch_eps=0.0, then=None):
         """``residual += this norm of a sublayer's output`` in one launch. ``branches``: the output, or two branches'

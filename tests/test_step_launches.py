@@ -1,0 +1,46 @@
+"""What a step asks the kernels for, from the shapes alone: launches recorded over tensors without memory."""
+import pytest
+
+import recorded
+from jllm_serve_amd.kernels import ops
+
+SHAPES = {"0.6b": (1024, 16, 8, 3072), "1.7b": (2048, 16, 8, 6144), "4b": (2560, 32, 8, 9728)}  # width, heads, kv heads, feed-forward
+
+
+@pytest.mark.parametrize("size", SHAPES)
+def test_a_norm_is_prepared_only_where_its_reader_takes_it(monkeypatch, size):
+    """The adding product of many rows leaves scaled rows and partial sums only for a product that reads them; and it is not
+    credited for a norm that is a launch of its own."""
+    seen = recorded.record(monkeypatch)
+    m = recorded.model(*SHAPES[size], layers=3)
+    rode = 0
+    for rows in (65, 127, 128, 200, 321, 400, 487, 512, 513, 600, 640, 750, 897, 960, 1009, 1024, 1500):
+        del seen[:]
+        recorded.forward(m, (rows, 0))
+        left = read = 0
+        for name, args in seen:
+            if name == "jllm_gemm_stream_bf16":
+                left += args[19] is not None   # emit_rows
+                read += args[25] is not None   # norm_partial
+        assert left == read, (rows, left, read)
+        rode += left
+        norms = [args for name, args in seen if name == "jllm_rmsnorm"]
+        made = sum(name in ("jllm_gemm_mfma_bf16", "jllm_gemm_pingpong_bf16") and args[-3] is not None for name, args in seen)
+        assert len(norms) + made + left == 2 * 3 + 1, rows  # two norms a layer and the last one, each of them once
+    assert rode or size == "4b"
+
+
+def test_no_norm_is_asked_for_when_its_reader_takes_rows_only():
+    """A feed-forward that gathers its rows (routed experts) gets the norm as a launch: the product in front of it is not
+    asked to prepare one that would be thrown away."""
+    from types import SimpleNamespace
+    from jllm_serve_amd.parts.block import PreNormBlock
+    asked = []
+    for takes in (False, True):
+        block = PreNormBlock.__new__(PreNormBlock)
+        block.ffn = SimpleNamespace(takes_normed_rows=takes, forward=lambda xb, x, step: None)
+        block.mixer = SimpleNamespace(prepares_next_norm=True, forward=lambda xb, x, step, slot, then_norm=None: asked.append(then_norm))
+        block.norm_in = SimpleNamespace(forward=lambda x: x)
+        block.norm_post = SimpleNamespace(forward=lambda x: x, after_add=None, reader=block.ffn)
+        block.forward("x", None, None)
+    assert asked == [None, block.norm_post]
