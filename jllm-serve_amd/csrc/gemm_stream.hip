@@ -372,14 +372,14 @@ static int launch_stream_rows(const StreamArgs& a, dim3 grid, int row_tiles, boo
   case MT:                                                                \
     return shared ? launch_stream<CT, MT, GATED, true>(a, grid, stream) : launch_stream<CT, MT, GATED, false>(a, grid, stream);
   switch (row_tiles) {
-    GS_CASE(1) GS_CASE(2) GS_CASE(3) GS_CASE(4)
+    GS_CASE(2) GS_CASE(3) GS_CASE(4)
     default: return launch_stream<CT, 8, GATED, false>(a, grid, stream);
   }
 #undef GS_CASE
 }
 
 // `rows`: weight rows per workgroup, both weights' of the gated epilogue together (32, 64, 96 or 128). `tile_m`: activation
-// rows per workgroup (64 or 128; up to 64 rows in all take tiles of 16, 32, 48 or 64). `parts` > 1 cuts K over
+// rows per workgroup (64 or 128; up to 64 rows in all take tiles of 32, 48 or 64). `parts` > 1 cuts K over
 // gridDim.y in whole blocks of 128; `partial` then holds parts * column tiles * rows * (tiles of rows in all) * (their rows) floats and `arrivals`
 // one int per column tile (and tile of rows), zeros, left as zeros. An RMSNorm on either side as in jllm_gemm_skinny_norm_bf16.
 // returns 0 when it ran, 1 when the shape is not one it takes (the caller uses another kernel), -1 on errors
@@ -416,7 +416,7 @@ extern "C" int jllm_gemm_stream_bf16(const void* A, int lda, const void* W, cons
   if (cus <= 0) JLLM_FAIL("gemm_stream: the GPU's compute units could not be read");
   dim3 grid(tiles, used, (M + tile_m - 1) / tile_m);
   if (grid.y > 65535 || grid.z > 65535) return 1;
-  const int row_tiles = M > 64 ? tile_m / 16 : (M + 15) / 16;
+  const int row_tiles = M > 64 ? tile_m / 16 : M > 32 ? (M + 15) / 16 : 2;
   const StreamArgs a{(const bf16_t*)A, (const bf16_t*)W, (const bf16_t*)W2, bias, out, partial, arrivals, lda, bias_dtype, out_dtype, ldo, M, N, K,
                      epilogue, bpp * 2, M <= 64 && used == 1, gs, StreamNorm{(bf16_t*)emit_rows, emit_ld, emit_gain, emit_gain_dtype, emit_partial, emit_parts, norm_partial, norm_parts, norm_eps}};
   // two workgroups share a compute unit where there are more of them than compute units: one streams while the other adds up

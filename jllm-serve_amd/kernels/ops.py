@@ -397,16 +397,14 @@ def _skinny_norm(a, w, w2, bias, out, epilogue, emit=None, normed: Optional[Norm
             _ptr(out), _code(out.dtype), out.stride(0), M, N, K, int(epilogue), float(gate_limit))
     emits = (_ptr(e_rows), _ptr(e_gain), _code(e_gain.dtype) if e_gain is not None else F32, _ptr(e_part))
     takes = (_ptr(n_part), n_part.shape[1] if n_part is not None else 0, normed.eps if normed is not None else 0.0, _stream())
-    few = M <= SKINNY_MAX_ROWS
     emit_parts = e_part.shape[1] if e_part is not None else 0
-    if few and not _few_rows_prefer_stream(N, K, w2 is not None):
+    if M <= SKINNY_MAX_ROWS:
         return _try("jllm_gemm_skinny_norm_bf16", *head, _skinny_rows(N, K, w2 is not None), *emits, emit_parts, *takes)
-    if K % 128 == 0:
-        rows, tile, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a, adds)
-        if _try("jllm_gemm_stream_bf16", *head, rows, tile, parts, _ptr(sums), _ptr(arrivals), _ptr(e_rows), e_rows.stride(0) if e_rows is not None else 0, *emits[1:],
-                emit_parts, *takes):
-            return True
-    return few and _try("jllm_gemm_skinny_norm_bf16", *head, 16, *emits, emit_parts, *takes)  # the second kernel declined
+    if K % 128:
+        return False
+    rows, tile, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a, adds)
+    return _try("jllm_gemm_stream_bf16", *head, rows, tile, parts, _ptr(sums), _ptr(arrivals), _ptr(e_rows), e_rows.stride(0) if e_rows is not None else 0, *emits[1:],
+                emit_parts, *takes)
 
 
 ADDS, ADDS_AND_NORM = 1, 2  # `adds` of a plan: into the residual, and with the rows for the norm behind it
@@ -817,8 +815,8 @@ def _norm_partials(M: int, N: int, K: int) -> int:
     workgroup's columns, in whole fours."""
     if M > STREAM_MAX_ROWS:
         groups = -(-N // _wide_plan(M, N, K, False, ADDS_AND_NORM)[0])
-    elif M > SKINNY_MAX_ROWS or _few_rows_prefer_stream(N, K, False):
-        groups = max(N // 16, -(-N // _stream_plan(N, K, False)[0])) if M <= SKINNY_MAX_ROWS else -(-N // _stream_plan(N, K, False)[0])
+    elif M > SKINNY_MAX_ROWS:
+        groups = -(-N // _stream_plan(N, K, False)[0])
     else:
         groups = -(-N // _skinny_rows(N, K, False))
     return -(-groups // 4) * 4
@@ -855,8 +853,7 @@ _step_scratch = threading.local()  # what a step's products share, see `step_scr
 @contextlib.contextmanager
 def step_scratch(rows: int, device):
     """Around the launches of one step of ``rows`` rows in one stream: zeroed counters that its products of few rows, which
-    follow each other, take turns in (each leaves them zero). Without them every such product clears counters of its own, as
-    the rare ones do that reach the second kernel with up to 16 rows."""
+    follow each other, take turns in (each leaves them zero). Without them every such product clears counters of its own."""
     if not SKINNY_MAX_ROWS < rows <= WIDE_MOST_ROWS or device.type != "cuda":
         yield
         return
@@ -879,7 +876,7 @@ def _stream_scratch(M: int, N: int, K: int, gated: bool, a: torch.Tensor, adds: 
         return rows, tile, 1, None, None
     row_tiles = -(-M // tile)
     tiles = -(-N // (rows // 2 if gated else rows)) * row_tiles
-    partial = torch.empty((parts * tiles * rows * (tile if M > STREAM_MAX_ROWS else 16 * -(-M // 16)),), dtype=torch.float32, device=a.device)
+    partial = torch.empty((parts * tiles * rows * (tile if M > STREAM_MAX_ROWS else max(32, 16 * -(-M // 16))),), dtype=torch.float32, device=a.device)
     arrivals, stream = getattr(_step_scratch, "arrivals", None) or (None, None)
     if arrivals is None or arrivals.device != a.device or arrivals.numel() < tiles or stream != _stream():
         arrivals = torch.empty(tiles, dtype=torch.int32, device=a.device).zero_()
@@ -960,19 +957,6 @@ def _wide_plan(M: int, N: int, K: int, gated: bool, adds: int = 0) -> Optional[T
     return plan
 
 
-STREAM_FEW_ROWS = (1280, 8192)   # columns at most, K at least: see `_few_rows_prefer_stream`
-
-
-@functools.lru_cache(maxsize=None)
-def _few_rows_prefer_stream(N: int, K: int, gated: bool) -> bool:
-    """Whether products of up to 16 rows of this shape go to the second weight-streaming kernel, which cuts K over
-    workgroups: few columns and a very long K, whose rows then have the same bits in every batch of up to 64. From N and K
-    alone, so that all products of up to 16 rows of one shape come from one kernel. First / second kernel at 8 rows: 1,024 x
-    8,192 7.7 / 11.5 us, x 16,384 11.7 / 14.8 (at 16 rows 15.2 / 15.1), 2,048 x 8,192 9.5 / 13.6: no shape of the served
-    sizes is better off there."""
-    return not gated and K % 128 == 0 and N % 16 == 0 and N <= STREAM_FEW_ROWS[0] and K >= STREAM_FEW_ROWS[1]
-
-
 _NO_NORM = (None, F32, 0.0, None, 0)
 
 
@@ -997,10 +981,10 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0, norm=_NO_
     N = w.shape[0]
     head = (_ptr(a), a.stride(0), _ptr(w), _ptr(w2), _ptr(bias), _code(bias.dtype) if bias is not None else F32,
             _ptr(out), _code(out.dtype), out.stride(0), M, N, K, int(epilogue), float(gate_limit))
-    if M <= SKINNY_MAX_ROWS and not _few_rows_prefer_stream(N, K, w2 is not None) \
-            and _try("jllm_gemm_skinny_bf16", *head, _skinny_rows(N, K, w2 is not None), _stream()):
-        return True
-    if K % 128 == 0 and (M <= STREAM_MAX_ROWS or _wide_plan(M, N, K, w2 is not None, _adds(epilogue)) is not None):
+    if M <= SKINNY_MAX_ROWS:
+        if _try("jllm_gemm_skinny_bf16", *head, _skinny_rows(N, K, w2 is not None), _stream()):
+            return True
+    elif K % 128 == 0 and (M <= STREAM_MAX_ROWS or _wide_plan(M, N, K, w2 is not None, _adds(epilogue)) is not None):
         rows, tile, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a, _adds(epilogue))
         if _try("jllm_gemm_stream_bf16", *head, rows, tile, parts, _ptr(sums), _ptr(arrivals), None, 0, None, F32, None, 0, None, 0, 0.0, _stream()):
             return True

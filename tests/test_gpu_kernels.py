@@ -217,7 +217,7 @@ def test_the_small_tile_gives_the_bits_of_the_two_group_kernel(ops, monkeypatch,
                                       (40, 1024, 1024, 512), (64, 2048, 2048, 768), (17, 1024, 4096, 256),
                                       # few rows, N / 16 just above the compute units: 20 weight rows per workgroup
                                       (8, 5120, 3072, 5120), (16, 5120, 4096, 640), (3, 5120, 3072, 5120), (11, 5120, 128, 7168),
-                                      # few rows, few columns and a long K: the K-cutting kernel takes them
+                                      # few rows, few columns and a long K
                                       (8, 1024, 8192, 512), (3, 1280, 8192, 1024),
                                       # the consuming product with 24 weight rows per workgroup, and with thousands of tiles
                                       (8, 1024, 512, 6144), (13, 256, 256, 32768)])
@@ -231,8 +231,6 @@ def test_norm_between_two_products(ops, M, N, K, N2, gdt):
     torch.manual_seed(M * N + K)
     if N == 5120 and M <= 16:
         assert ops._skinny_second_rows(N, False) == 4, "this case is meant for workgroups with 20 weight rows"
-    if K == 8192 and M <= 16:
-        assert ops._few_rows_prefer_stream(N, K, False), "this case is meant for the K-cutting kernel"
     a = torch.randn(M, K, device=DEV).bfloat16()
     w = (torch.randn(N, K, device=DEV) / math.sqrt(K)).bfloat16()
     bias = torch.randn(N, device=DEV)
@@ -288,7 +286,6 @@ def test_few_row_products_at_any_weight_rows_per_workgroup(ops, monkeypatch, M, 
     rnd = lambda *shape: torch.randn(*shape, device=DEV, generator=gen)
     a, w, w2 = rnd(M, K).bfloat16(), (rnd(N, K) / math.sqrt(K)).bfloat16(), (rnd(N, K) / math.sqrt(K)).bfloat16()
     bias, gain, res0 = rnd(N), rnd(N).abs() + 0.5, rnd(M, N)
-    monkeypatch.setattr(ops, "_few_rows_prefer_stream", lambda *_: False)
     monkeypatch.setattr(ops, "_skinny_rows", lambda n, k, gated: min(rows, 16) if gated else rows)
     ops.reset_stats()
     exact, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
@@ -326,7 +323,7 @@ def test_products_of_17_to_64_rows_at_any_plan(ops, monkeypatch, M, N, K, rows, 
     rnd = lambda *shape: torch.randn(*shape, device=DEV, generator=gen)
     a, w, w2 = rnd(M, K).bfloat16(), (rnd(N, K) / math.sqrt(K)).bfloat16(), (rnd(N, K) / math.sqrt(K)).bfloat16()
     bias, gain, res0 = rnd(N), rnd(N).abs() + 0.5, rnd(M, N)
-    monkeypatch.setattr(ops, "_few_rows_prefer_stream", lambda *_: True)
+    monkeypatch.setattr(ops, "SKINNY_MAX_ROWS", 0)  # up to 16 rows as well
     monkeypatch.setattr(ops, "_stream_plan", lambda *_: (rows, parts))
     ops.reset_stats()
     exact, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
@@ -418,12 +415,10 @@ def test_gemm_rows_do_not_depend_on_the_batch(ops):
     for dtype, K, full_rows, parts in ((torch.float32, 200, 64, (1, 2, 7, 16, 33)), (torch.float32, 203, 40, (1, 3, 16, 17)),
                                        (torch.bfloat16, 512, 16, (1, 7, 11)),
                                        (torch.bfloat16, 1024, 64, (17, 33, 48)), (torch.bfloat16, 512, 128, (65, 100)),
-                                       (torch.bfloat16, 8192, 64, (1, 8, 16, 17, 40)),  # with N = 1024: one kernel up to 64 rows
+                                       (torch.bfloat16, 8192, 16, (1, 8)), (torch.bfloat16, 8192, 64, (17, 40)),  # with N = 1024
                                        (torch.bfloat16, 3072, 16, (1, 8, 11)),  # with N = 5120: 20 weight rows per workgroup
                                        (torch.bfloat16, 384, 16, (1, 5, 9))):  # with N = 6144: 24 weight rows per workgroup
         N = {8192: 1024, 3072: 5120, 384: 6144}.get(K, 96)
-        if K == 8192:
-            assert ops._few_rows_prefer_stream(N, K, False), "this case is meant for the K-cutting kernel at few rows"
         a = torch.randn(full_rows, K, device=DEV).to(dtype)
         w = torch.randn(N, K, device=DEV).to(dtype)
         full = ops.gemm(a, w, out_dtype=torch.float32, exact=dtype == torch.float32)

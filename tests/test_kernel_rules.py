@@ -33,13 +33,25 @@ def test_k_parts_do_not_depend_on_rows():
     """The rule has no argument for the number of rows: a row's sum is the same bits in any batch."""
     import inspect
     assert list(inspect.signature(ops._stream_parts.__wrapped__).parameters) == ["N", "K", "gated"]
-    assert list(inspect.signature(ops._few_rows_prefer_stream.__wrapped__).parameters) == ["N", "K", "gated"]
 
 
-def test_kernel_for_few_rows():
-    assert not ops._few_rows_prefer_stream(96, 512, False), "small products: the second launch costs more than it saves"
-    assert not ops._few_rows_prefer_stream(5120, 100, False), "a K the kernels do not take"
-    assert not ops._few_rows_prefer_stream(4096, 4096, False), "N / 16 fills the compute units exactly: nothing to gain"
+def test_kernel_for_few_rows(monkeypatch):
+    """Products of up to 16 rows go to one kernel whatever their shape (cutting K over workgroups was slower at every one that
+    was measured, a launch for its counters aside), and have no scratch; those of 17 to 64 rows to the other."""
+    import torch
+
+    import recorded
+    seen = recorded.record(monkeypatch)
+    shapes = [(n, k) for v in SHAPES.values() for n, k, _ in v] + [(128, 512), (1024, 8192), (1280, 8192), (1024, 16384), (256, 32768)]
+    for n, k in shapes:
+        for rows in (1, 8, 16, 17, 64):
+            a, w, res = recorded.tensor(rows, k), recorded.tensor(n, k), recorded.tensor(rows, n, dtype=torch.float32)
+            del seen[:]
+            promise = ops.gemm_add_then_norm(a, w, res, recorded.tensor(n), 1e-5, torch.bfloat16)
+            ops.gemm(promise, recorded.tensor(512, n))
+            ops.gemm(a, w)
+            few = rows <= 16
+            assert [name for name, _ in seen] == (["jllm_gemm_skinny_norm_bf16"] * 2 + ["jllm_gemm_skinny_bf16"] if few else ["jllm_gemm_stream_bf16"] * 3), (n, k, rows)
 
 
 def test_rows_of_a_workgroup_of_the_first_weight_streaming_kernel():
