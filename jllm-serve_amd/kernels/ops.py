@@ -732,35 +732,6 @@ def compute_units() -> int:
 _compute_units = 0
 
 
-STREAM_PART_COST = 0.02         # what one more part costs (partial sums, a shorter K range), as a fraction, per weight
-STREAM_MIN_BLOCKS = 4           # 128-wide K blocks a part has at least
-
-
-@functools.lru_cache(maxsize=None)
-def _stream_parts(N: int, K: int, gated: bool) -> int:
-    """How many ways the second weight-streaming kernel may cut K for a product of ceil(N / 128) column tiles, from N and K
-    alone (never from the number of rows: a row's sum must not depend on its batch; `_stream_plan` asks with the tiles that
-    its workgroups have). A compute unit streams about as fast with one workgroup as with two, so what counts is the largest
-    number of workgroups any compute unit gets: the count that minimises ceil(workgroups / compute units) / workgroups, times
-    a small price per part. Any count goes, not only powers of two."""
-    tiles = -(-N // 128)
-    nblk = K // 128
-    step = 1 if gated else 2
-    best, best_cost = 1, None
-    COMPUTE_UNITS = compute_units()
-    most = 1 if tiles >= 2 * COMPUTE_UNITS else min(nblk, 32)  # many column tiles: rounds are full enough as they are
-    for parts in range(1, most + 1):
-        per = -(-nblk // parts)
-        per = -(-per // step) * step  # whole steps, as the kernel rounds
-        if -(-nblk // per) != parts or (parts > 1 and per < STREAM_MIN_BLOCKS):
-            continue
-        groups = tiles * parts
-        cost = -(-groups // COMPUTE_UNITS) / groups * (1.0 + STREAM_PART_COST * parts * (2 if gated else 1))
-        if best_cost is None or cost < best_cost - 1e-12:
-            best, best_cost = parts, cost
-    return best
-
-
 def _round_fill(groups: int) -> float:
     """The share of the compute units' rounds that `groups` workgroups fill."""
     cus = compute_units()
@@ -822,26 +793,55 @@ def _norm_partials(M: int, N: int, K: int) -> int:
     return -(-groups // 4) * 4
 
 
-STREAM_NS_PER_KB = 26.0    # what a compute unit's load pipe takes for 1 KB of weights or activations
-STREAM_MERGE_NS = 1500     # the last workgroup of a column tile: its way through memory ...
-STREAM_SUM_NS_PER_KB = 60  # ... and for 1 KB of sums
+# Estimated times of the second weight-streaming kernel for 17 to 64 rows, in ns (priced at 40 rows)
+STREAM_MIN_BLOCKS = 4             # 128-wide K blocks a part has at least
+STREAM_MOST_PARTS = 32
 STREAM_PRICED_ROWS = 40
+STREAM_BLOCK_NS = (148.0, 4.12)    # 64 of k, and per weight row
+STREAM_PAIR = (1.59, 1.9)         # two workgroups on a compute unit: a few of them, all
+STREAM_BYTES_PER_NS = 5600.0      # weights from memory
+STREAM_MERGE_NS = 1940.0          # parts of K: the last workgroup's way through memory ...
+STREAM_SUM_NS_PER_KB = 56.6       # ... per KB of sums that it reads ...
+STREAM_PARTS_NS_PER_KB = 0.45     # ... and per KB that all workgroups leave
+
+
+def _stream_ns(N: int, K: int, gated: bool, rows: int, parts: int) -> float:
+    cus = compute_units()
+    groups = -(-N // (rows // 2 if gated else rows)) * parts
+    step = -(-(K // 128) // parts) * 2 * (STREAM_BLOCK_NS[0] + STREAM_BLOCK_NS[1] * rows)
+    full, last = divmod(groups, 2 * cus)
+    few, all_ = STREAM_PAIR
+    t = full * step * all_
+    if last:
+        t += step if last <= cus else step * (few + (all_ - few) * (last - cus) / cus)
+    t = max(t, N * K * 2 * (2 if gated else 1) / STREAM_BYTES_PER_NS)
+    if parts > 1:
+        kb = rows * STREAM_PRICED_ROWS * 4 / 1024
+        t += STREAM_MERGE_NS + kb * (parts * STREAM_SUM_NS_PER_KB + groups * STREAM_PARTS_NS_PER_KB)
+    return t
 
 
 @functools.lru_cache(maxsize=None)
 def _stream_plan(N: int, K: int, gated: bool) -> Tuple[int, int]:
-    """(weight rows per workgroup, ways K is cut) of the second weight-streaming kernel, from N and K alone (priced at 40
-    rows). More rows per workgroup share the activations' way into a compute unit, fewer leave more workgroups; parts of K
-    fill what N leaves empty and cost the last workgroup their sums."""
-    cus = compute_units()
+    """(weight rows per workgroup, ways K is cut) of the second weight-streaming kernel, the cheapest by the estimate, from N
+    and K alone (never from the number of rows: a row's sum must not depend on its batch). More rows per workgroup share the
+    activations' way into a compute unit, fewer leave more workgroups; parts of K, any count of them, fill what N leaves
+    empty and cost the last workgroup their sums, and all of them their way through memory.
+
+    The constants were fitted to a sweep of every choice for the products of 17 models' shapes at 17, 32 and 64 rows, with
+    what a change has to gain before it is one: 1.4 % behind the best on average (2.3 % before, when each tile width had one
+    count, chosen by the fill of the rounds, and parts were priced by the last workgroup's sums only). us at those rows,
+    before / now: gated 6,144 x 2,048 17.2 17.6 20.2 / 14.4 15.0 17.3, plain 5,120 x 17,408 41.1 42.4 48.3 / 39.1 40.5 48.4,
+    15,360 x 5,120 36.6 37.3 42.6 / 34.4 35.6 41.6. It misses: 12,288 x 4,096 30.8 31.2 34.0 where 64 rows with K whole take
+    24.7 25.7 30.2, 8,192 x 8,192 39.5 40.3 44.4 where 32 with K whole take 32.9 32.1 41.0."""
     best, plan = None, (64, 1)
     for rows in (32, 64, 96, 128):
         tiles = -(-N // (rows // 2 if gated else rows))
-        for parts in {1, _stream_parts(tiles * 128, K, gated)}:
-            per = -(-(K // 128) // parts) * 128
-            t = -(-tiles * parts // cus) * (rows + STREAM_PRICED_ROWS) * per * 2 / 1024 * STREAM_NS_PER_KB
-            if parts > 1:
-                t += STREAM_MERGE_NS + parts * STREAM_PRICED_ROWS * rows * 4 / 1024 * STREAM_SUM_NS_PER_KB
+        for parts in range(1, (STREAM_MOST_PARTS if tiles <= STREAM_COUNTERS else 1) + 1):
+            per = -(-(K // 128) // parts)
+            if parts > 1 and (per < STREAM_MIN_BLOCKS or -(-(K // 128) // per) != parts):
+                continue
+            t = _stream_ns(N, K, gated, rows, parts)
             if best is None or t < best:
                 best, plan = t, (rows, parts)
     return plan

@@ -11,28 +11,32 @@ SHAPES = {  # (N, K, gated): qkv, o, gate/up, down
 
 
 def test_k_parts_fill_the_rounds():
-    """Whatever the tuning: every part keeps the minimum length, the kernel's rounding of a part's blocks gives back
-    the count, and the chosen count never leaves the busiest compute unit with a larger share of the product than
-    no cut at all would."""
+    """Whatever the tuning: every part keeps the minimum length, a part's blocks give back the count, the chosen count never
+    leaves the busiest compute unit with a larger share of the product than no cut at all would, and the choice is the
+    cheapest by the estimate over every number of weight rows and every count of parts that the kernel can do."""
     cus = ops.compute_units()
-    shapes = [s for v in SHAPES.values() for s in v] + [(96, 128, False), (256, 256, False), (384, 1024, True), (5120, 640, False)]
+    shapes = [s for v in SHAPES.values() for s in v] + [(96, 128, False), (256, 256, False), (384, 1024, True), (5120, 640, False),
+                                                       (1024, 3072, False), (4608, 3584, False), (18944, 3584, True), (6144, 2048, True)]
     for n, k, gated in shapes:
-        parts = ops._stream_parts(n, k, gated)
-        step = 1 if gated else 2
+        rows, parts = ops._stream_plan(n, k, gated)
         nblk = k // 128
-        per = -(-(-(-nblk // parts)) // step) * step  # whole steps, as the kernel rounds
+        per = -(-nblk // parts)
         assert parts >= 1 and (parts == 1 or per >= ops.STREAM_MIN_BLOCKS), (n, k, gated, parts)
         assert -(-nblk // per) == parts, (n, k, gated, parts)
-        tiles = -(-n // 128)
+        tiles = -(-n // (rows // 2 if gated else rows))
         share = lambda p: -(-(tiles * p) // cus) / (tiles * p)
         assert share(parts) <= share(1) + 1e-12, (n, k, gated, parts)
-    assert ops._stream_parts(151936, 4096, False) == 1, "many column tiles: no cut"
+        cheapest = min(ops._stream_ns(n, k, gated, r, p) for r in (32, 64, 96, 128) for p in range(1, ops.STREAM_MOST_PARTS + 1)
+                       if p == 1 or (-(-nblk // p) >= ops.STREAM_MIN_BLOCKS and -(-nblk // -(-nblk // p)) == p and
+                                     -(-n // (r // 2 if gated else r)) <= ops.STREAM_COUNTERS))
+        assert ops._stream_ns(n, k, gated, rows, parts) == cheapest, (n, k, gated)
+    assert ops._stream_plan(151936, 4096, False)[1] == 1, "many column tiles: no cut"
 
 
 def test_k_parts_do_not_depend_on_rows():
     """The rule has no argument for the number of rows: a row's sum is the same bits in any batch."""
     import inspect
-    assert list(inspect.signature(ops._stream_parts.__wrapped__).parameters) == ["N", "K", "gated"]
+    assert list(inspect.signature(ops._stream_plan.__wrapped__).parameters) == ["N", "K", "gated"]
 
 
 def test_kernel_for_few_rows(monkeypatch):
