@@ -852,20 +852,32 @@ _step_scratch = threading.local()  # what a step's products share, see `step_scr
 
 @contextlib.contextmanager
 def step_scratch(rows: int, device):
-    """Around the launches of one step of ``rows`` rows in one stream: zeroed counters that its products of few rows, which
-    follow each other, take turns in (each leaves them zero). Without them every such product clears counters of its own."""
-    if not SKINNY_MAX_ROWS < rows <= WIDE_MOST_ROWS or device.type != "cuda":
+    """Around the launches of one step of ``rows`` rows: the products of few rows with K cut, which follow each other in their
+    stream, take turns in one set of zeroed counters (each leaves them zero), made and cleared for the first of them; a step
+    without any launches nothing for it. Outside, every such product clears counters of its own."""
+    if not SKINNY_MAX_ROWS < rows <= WIDE_MOST_ROWS:
         yield
         return
-    before = getattr(_step_scratch, "arrivals", None)
-    _step_scratch.arrivals = (torch.empty(STREAM_COUNTERS, dtype=torch.int32, device=device).zero_(), _stream())
+    before = getattr(_step_scratch, "counters", None)
+    _step_scratch.counters = {}  # (device, stream, whether it is captured) -> counters
     try:
         yield
     finally:
-        _step_scratch.arrivals = before
+        _step_scratch.counters = before
 
 
 STREAM_COUNTERS = 1024
+
+
+def _arrival_counters(tiles: int, device) -> torch.Tensor:
+    shared = getattr(_step_scratch, "counters", None)
+    if shared is None or tiles > STREAM_COUNTERS:
+        return torch.empty(tiles, dtype=torch.int32, device=device).zero_()
+    # memory that a capture has recorded the clearing of is not clear for launches beside it, nor the other way round
+    key = (device, _stream(), torch.cuda.is_current_stream_capturing())
+    if key not in shared:
+        shared[key] = torch.empty(STREAM_COUNTERS, dtype=torch.int32, device=device).zero_()
+    return shared[key]
 
 
 def _stream_scratch(M: int, N: int, K: int, gated: bool, a: torch.Tensor, adds: int):
@@ -877,10 +889,7 @@ def _stream_scratch(M: int, N: int, K: int, gated: bool, a: torch.Tensor, adds: 
     row_tiles = -(-M // tile)
     tiles = -(-N // (rows // 2 if gated else rows)) * row_tiles
     partial = torch.empty((parts * tiles * rows * (tile if M > STREAM_MAX_ROWS else max(32, 16 * -(-M // 16))),), dtype=torch.float32, device=a.device)
-    arrivals, stream = getattr(_step_scratch, "arrivals", None) or (None, None)
-    if arrivals is None or arrivals.device != a.device or arrivals.numel() < tiles or stream != _stream():
-        arrivals = torch.empty(tiles, dtype=torch.int32, device=a.device).zero_()
-    return rows, tile, parts, partial, arrivals
+    return rows, tile, parts, partial, _arrival_counters(tiles, a.device)
 
 
 def _plan_of_rows(M: int, N: int, K: int, gated: bool, adds: int) -> Tuple[int, int, int]:

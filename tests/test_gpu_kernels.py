@@ -349,6 +349,38 @@ def test_products_of_17_to_64_rows_at_any_plan(ops, monkeypatch, M, N, K, rows, 
     assert set(ops.stats()["ran"]) == {"jllm_gemm_stream_bf16"}
 
 
+def test_counters_of_parts_belong_to_a_stream(ops, monkeypatch):
+    """Products with K cut over workgroups inside one step's scope on two streams at once, and recorded into a graph beside
+    eager ones: each stream, and the capture, counts in zeroed counters of its own, and every result has the same bits."""
+    M, N, K = 40, 1024, 2048
+    monkeypatch.setattr(ops, "_stream_plan", lambda *_: (32, 4))
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(3)
+    a, w = torch.randn(M, K, device=DEV, generator=gen).bfloat16(), (torch.randn(N, K, device=DEV, generator=gen) / math.sqrt(K)).bfloat16()
+    want = ops.gemm(a, w, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    side, graph, got = torch.cuda.Stream(), torch.cuda.CUDAGraph(), []
+    with ops.step_scratch(M, a.device):
+        for _ in range(4):
+            got.append(ops.gemm(a, w, out_dtype=torch.float32))
+            with torch.cuda.stream(side):
+                got.append(ops.gemm(a, w, out_dtype=torch.float32))
+        assert len(ops._step_scratch.counters) == 2
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            recorded = ops.gemm(a, w, out_dtype=torch.float32)
+        assert len(ops._step_scratch.counters) == 3
+        with torch.cuda.stream(side):  # in front of the first replay, which clears what the capture counts in
+            got.append(ops.gemm(a, w, out_dtype=torch.float32))
+        torch.cuda.synchronize()
+    for _ in range(3):
+        graph.replay()
+        got.append(recorded.clone())
+        got.append(ops.gemm(a, w, out_dtype=torch.float32))
+        torch.cuda.synchronize()
+    assert all(torch.equal(g, want) for g in got)
+
+
 @pytest.mark.parametrize("rows,tile", [(32, 64), (64, 64), (96, 64), (128, 64), (32, 128), (64, 128), (96, 128), (128, 128)])
 @pytest.mark.parametrize("M,N,K,parts", [(128, 1024, 1024, 1), (129, 1040, 1152, 2), (200, 2048, 1024, 3), (321, 528, 3072, 4), (640, 4096, 1024, 1)])
 def test_products_of_more_rows_at_any_plan(ops, monkeypatch, M, N, K, parts, rows, tile):

@@ -1,5 +1,7 @@
 """What a step asks the kernels for, from the shapes alone: launches recorded over tensors without memory."""
 import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 import recorded
 from jllm_serve_amd.kernels import ops
@@ -44,3 +46,31 @@ def test_no_norm_is_asked_for_when_its_reader_takes_rows_only():
         block.norm_post = SimpleNamespace(forward=lambda x: x, after_add=None, reader=block.ffn)
         block.forward("x", None, None)
     assert asked == [None, block.norm_post]
+
+
+class Clears(TorchDispatchMode):
+    """Counts the fill launches inside."""
+
+    def __init__(self):
+        super().__init__()
+        self.n = 0
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.n += func in (torch.ops.aten.zero_.default, torch.ops.aten.zeros.default, torch.ops.aten.fill_.Scalar)
+        return func(*args, **(kwargs or {}))
+
+
+def test_a_step_clears_counters_once_and_only_for_products_that_count(monkeypatch):
+    """The products with K cut over workgroups share the step's counters, cleared for the first of them; a step that has none,
+    in 32 bits or with every K whole, launches nothing for them."""
+    with ops.step_scratch(40, torch.device("cuda")):
+        pass  # nothing is made, so this needs no GPU
+    seen = recorded.record(monkeypatch)
+    for dtype, rows, counts in ((torch.bfloat16, 40, True), (torch.float32, 40, False), (torch.float32, 487, False), (torch.bfloat16, 16, False), (torch.bfloat16, 487, None)):
+        m = recorded.model(*SHAPES["0.6b"], dtype=dtype)
+        del seen[:]
+        with Clears() as clears:
+            recorded.forward(m, (rows, 0))
+        counters = [args[18] for name, args in seen if name == "jllm_gemm_stream_bf16" and args[16] > 1]
+        assert counts is None or bool(counters) == counts
+        assert clears.n == bool(counters) and all(c is counters[0] for c in counters), (dtype, rows, clears.n)
