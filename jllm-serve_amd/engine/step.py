@@ -13,7 +13,8 @@ indices, uploaded in one copy; then the model runs once over all rows.
 
 The step function knows nothing of any mixer's kernels. A part that wants more about the batch on the device
 or on the host (attention: its rows cut into tiles, whether every request brings one row) gives the model a
-*step planner*: ``key`` (planners with equal keys plan once per step) and ``plan(StepBatch) -> StepPlan`` with
+*step planner*: ``key`` (planners with equal keys plan once per step; ``join(other)``, where the first of them has it,
+tells it whom else it plans for) and ``plan(StepBatch) -> StepPlan`` with
 int32 arrays, which ride in the same upload, and host-side facts. Parts find their plan in ``step.plans[key]``.
 """
 from __future__ import annotations
@@ -164,12 +165,12 @@ class ModelRunner:
     def planners(self) -> list:
         """The model's step planners, one per distinct key (36 equal attention layers plan once)."""
         if self._planners is None:
-            seen, out = set(), []
+            by_key = {}
             for pl in (self.model.step_planners() if hasattr(self.model, "step_planners") else []):
-                if pl.key not in seen:
-                    seen.add(pl.key)
-                    out.append(pl)
-            self._planners = out
+                first = by_key.setdefault(pl.key, pl)
+                if first is not pl and hasattr(first, "join"):
+                    first.join(pl)
+            self._planners = list(by_key.values())
         return self._planners
 
     def _layout(self, entries: Sequence[StepEntry], pad_rows: int = 0, width: int = 0):

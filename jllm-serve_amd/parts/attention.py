@@ -11,6 +11,7 @@ of the output product.
 """
 from __future__ import annotations
 
+import numpy as np
 import torch
 
 from ..cache.manager import KvSpec
@@ -37,11 +38,15 @@ class GqaStepPlanner:
     run sees 16 times the keys of the first), which is when the portion kernel does well to cut every run's keys over
     two groups of waves. A step of single rows also brings zeroed counters, one per row and
     kv head, by which the workgroups of the split-key kernel find out which of them merges; the layers, which follow each
-    other in one stream, take turns in them."""
+    other in one stream, take turns in them (with several head counts: in as many as the largest takes)."""
+
+    key = ("gqa", TILE_ROWS)
 
     def __init__(self, kv_heads: int = 0):
         self.kv_heads = kv_heads
-        self.key = ("gqa", TILE_ROWS, kv_heads)
+
+    def join(self, other):
+        self.kv_heads = max(self.kv_heads, other.kv_heads)
 
     def plan(self, batch):
         from ..engine.step import StepPlan
@@ -64,9 +69,10 @@ class GqaStepPlanner:
                 single_rows = (ones[0], len(ones))
             runs += [(s.index, s.row0, 1, s.pos0) for s in segments if s.n == 1]
             tiles = [v for t in runs for v in t]
-        return StepPlan({"tiles": tiles, "arrivals": [0] * (batch.rows * self.kv_heads if decode_only else 0)}, {"decode_only": decode_only, "n_tiles": len(tiles) // 4,
-                                           "n_tiles_multi": n_multi, "single_rows": single_rows,
-                                           "key_groups": key_groups})
+        arrivals = np.zeros(batch.rows * self.kv_heads if decode_only else 0, np.int32)
+        return StepPlan({"tiles": tiles, "arrivals": arrivals},
+                        {"decode_only": decode_only, "n_tiles": len(tiles) // 4, "n_tiles_multi": n_multi,
+                         "single_rows": single_rows, "key_groups": key_groups})
 
 
 class GqaAttention(Part):
@@ -146,7 +152,7 @@ class GqaAttention(Part):
 
     def _batch_facts(self, step):
         """The kernels' view of the batch: the step's own numbers and this mixer's plan of it, put together once per step."""
-        plan = step.plans.get(self.planner.key)
+        plan = step.plans.get(GqaStepPlanner.key)
         if plan is None:  # a step put together without the planner: the general kernels take it
             return {"max_context": step.max_context, "requests": step.n_requests, "rows": step.n_tokens, "decode_only": False}
         meta = plan.facts.get("batch")

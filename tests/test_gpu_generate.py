@@ -382,3 +382,41 @@ def test_eos_and_penalties_through_the_engine(model_folders):
         assert got[i] == t
         toks.append(t)
         gen[t] = gen.get(t, 0) + 1
+
+
+def test_layers_of_two_kv_head_counts_share_a_step_plan(monkeypatch):
+    """A model whose layers differ in kv heads: captured decode steps over several key ranges, whose last workgroup merges them by
+    the step's counters, against the same steps with the merge as a launch of its own: the same bits, step after step."""
+    import dataclasses
+    from jllm_serve_amd.config import parse_config
+    from jllm_serve_amd.engine import StepEntry, build_model, build_runner
+    from jllm_serve_amd.kernels import ops
+    from jllm_serve_amd.parts.model import DecoderModel
+    from jllm_serve_amd.weights.loader import TensorSource
+    cfg = parse_config({"architectures": ["Qwen3ForCausalLM"], "model_type": "qwen3", "hidden_size": 256, "num_hidden_layers": 3, "vocab_size": 512,
+                        "num_attention_heads": 4, "num_key_value_heads": 4, "head_dim": 128, "intermediate_size": 256, "rms_norm_eps": 1e-6,
+                        "rope_theta": 1e6, "tie_word_embeddings": False, "max_position_embeddings": 1024})
+    layers = tuple(dataclasses.replace(l, mixer=dataclasses.replace(l.mixer, kv_heads=n)) for l, n in zip(cfg.layers, (2, 4, 1)))
+    cfg = dataclasses.replace(cfg, layers=layers)
+    gen = torch.Generator().manual_seed(11)
+    specs = DecoderModel(cfg, torch.bfloat16, "meta", 1024).weight_specs()
+    source = TensorSource({s.name: (torch.randn(tuple(s.shape), generator=gen) * 0.06 + (len(s.shape) == 1)).bfloat16() for s in specs})
+    prompts = [torch.randint(0, 512, (n,), generator=gen).tolist() for n in (700, 130, 5)]
+    monkeypatch.setattr(ops, "_decode_split", lambda *_: 128)
+    fused, got = ops.decode_attention_fused, []
+    for merged in (True, False):
+        counted = []
+
+        def attention(*args, **kw):
+            meta = args[18]
+            counted.append(meta["arrivals"].numel())
+            return fused(*args[:18], meta if merged else {**meta, "arrivals": None}, *args[19:], **kw)
+
+        monkeypatch.setattr(ops, "decode_attention_fused", attention)
+        runner = build_runner(build_model(cfg, source, torch.bfloat16, torch.device("cuda:0"), 1024), page_size=16, max_requests=4)
+        assert len(runner.planners()) == 1
+        runner.step([StepEntry(i, p, [len(p) - 1]) for i, p in enumerate(prompts)])
+        steps = [runner.step([StepEntry(i, [7 * t + i], [0]) for i in range(3)]).clone() for t in range(4)]
+        assert counted and set(counted) == {4 * 4}  # rows of the captured step, by the most kv heads
+        got.append(steps)
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and not torch.isnan(got[0][-1]).any()

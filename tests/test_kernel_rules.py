@@ -169,6 +169,22 @@ def test_the_attention_plan_says_whether_the_runs_of_a_step_differ_much_in_keys(
     assert f["key_groups"] == 2 and f["n_tiles_multi"] == 16 and f["single_rows"] == (2048, 1)
 
 
+def test_attention_layers_of_several_head_counts_plan_once():
+    """The runs of a step are cut and uploaded once whatever the layers' kv heads, under a key that any part can ask for by the
+    planner's class; the counters are as many as the layer with the most kv heads takes."""
+    from types import SimpleNamespace
+
+    import torch
+    from jllm_serve_amd.engine.step import ModelRunner, Segment, StepBatch
+    from jllm_serve_amd.parts.attention import GqaStepPlanner
+    planners = [GqaStepPlanner(n) for n in (2, 8, 4)]
+    model = SimpleNamespace(step_planners=lambda: planners, device=torch.device("cpu"), config=SimpleNamespace(vocab=8))
+    got = ModelRunner(model, None, 64).planners()
+    assert [pl.key for pl in got] == [GqaStepPlanner.key]
+    batch = StepBatch([Segment(i, i, i, 1, 9, i) for i in range(3)], 3, 3, 10, 16, None, False)
+    assert len(got[0].plan(batch).arrays["arrivals"]) == 3 * 8
+
+
 def test_plans_of_the_second_weight_streaming_kernel():
     """Every plan is one that the kernel has, parts of K are whole blocks that are all there, its counters fit the step's, and
     for up to 64 rows it knows nothing of their number; few columns and large products of many rows stay with the other kernels."""
