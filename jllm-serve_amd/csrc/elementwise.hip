@@ -56,8 +56,9 @@ extern "C" int jllm_embed(const void* table, int table_dtype, const int* ids, fl
 // RMSNorm of fp32 rows: y = (x * rsqrt(mean(x^2) + eps)) * g. One block per output row; `rows` (optional)
 // picks the input row of each output row; output rows lie `ldo` elements apart. Sum of squares, the reciprocal root and both products are fp32.
 // Rows of up to 8192 values whose width is a multiple of 4 are read once, 16 bytes per lane, and held in J vectors of registers
-// per thread (J = 0: other widths and gains that are not 16-byte aligned take the two-pass loop). 2,048 rows of 4,096 13.4 ->
-// 9.7 us (50 MB: 5.2 TB/s) since no branch stands around a load.
+// per thread (J = 0: other widths take the two-pass loop); the loads are declared as aligned to an element only, which costs
+// nothing, so that a row has the same bits wherever it and the gains lie. 2,048 rows of 4,096 13.4 -> 9.7 us (50 MB:
+// 5.2 TB/s) since no branch stands around a load.
 template <typename TG, typename TO, int J>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ x, const int* __restrict__ rows,
                                                       const TG* __restrict__ gain, TO* __restrict__ out, int ldo, int d,
@@ -78,11 +79,8 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ 
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       at[j] = min((int)threadIdx.x + 256 * j, nv - 1);
-      v[j] = ((const float4*)xi)[at[j]];
-      if (sizeof(TG) == 2)
-        *(uint2*)gn[j] = ((const uint2*)gain)[at[j]];
-      else
-        *(uint4*)gn[j] = ((const uint4*)gain)[at[j]];
+      __builtin_memcpy(&v[j], xi + 4 * at[j], 16);
+      __builtin_memcpy(gn[j], gain + 4 * at[j], 4 * sizeof(TG));
     }
 #pragma unroll
     for (int j = 0; j < J; ++j)
@@ -131,7 +129,7 @@ extern "C" int jllm_rmsnorm(const float* x, const int* rows, int n_rows, int d, 
     break;
   JLLM_DISPATCH_1(gain_dtype, TG, {
     JLLM_DISPATCH_1(out_dtype, TO, {
-      switch ((d & 3) == 0 && d <= 8192 && ((uintptr_t)gain & 15) == 0 && ((uintptr_t)x & 15) == 0 ? (d / 4 + 255) / 256 : 0) {
+      switch ((d & 3) == 0 && d <= 8192 ? (d / 4 + 255) / 256 : 0) {
         RN_CASE(0) RN_CASE(1) RN_CASE(2) RN_CASE(3) RN_CASE(4) RN_CASE(5) RN_CASE(6) RN_CASE(7) RN_CASE(8)
       }
     })

@@ -51,6 +51,24 @@ def test_rmsnorm(ops, d, gdt, odt):
     assert torch.equal(ops.rmsnorm(x, g, eps, odt, rows), out[rows.long()])
 
 
+@pytest.mark.parametrize("d", [4, 1020, 1024, 4096, 8192])
+@pytest.mark.parametrize("gdt", [torch.float32, torch.bfloat16])
+def test_rmsnorm_has_the_same_bits_at_any_alignment(ops, d, gdt):
+    """Rows and gains that begin anywhere in a 16-byte piece (pieces of a larger tensor) against those that begin with one."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(d)
+    x = torch.randn(9, d, device=DEV, generator=gen) * 3
+    g = (torch.rand(d, device=DEV, generator=gen) + 0.5).to(gdt)
+    want = ops.rmsnorm(x, g, 1e-5, torch.float32)
+    for at in (1, 2, 3, 5):
+        gains = torch.zeros(d + 8, device=DEV, dtype=gdt)[at:at + d]
+        gains.copy_(g)
+        rows = torch.zeros(9 * d + 8, device=DEV)[at:at + 9 * d].view(9, d)
+        rows.copy_(x)
+        assert gains.data_ptr() % 16 and rows.data_ptr() % 16
+        assert torch.equal(ops.rmsnorm(x, gains, 1e-5, torch.float32), want) and torch.equal(ops.rmsnorm(rows, g, 1e-5, torch.float32), want)
+
+
 GEMM_SHAPES = [(1, 16, 128), (5, 48, 384), (16, 4096, 128), (17, 80, 256), (33, 16, 1024), (64, 304, 640), (50, 144, 2176),
                (20, 4112, 512),
                (8, 6144, 256), (3, 6144, 128), (16, 6144, 1152),  # 24 weight rows per workgroup (N / 24 = 256 of them)
