@@ -14,7 +14,7 @@
 // had to share. In LDS the activations of up to 8 rows cost half as much, and K blocks of 64 keep the waves even.
 // Inside a graph, before / now, in us at 1, 8 and 16 rows: 8B shape qkv 14.0 15.7 16.0 / 12.4 13.0 13.4, o 8.7 9.8 11.3 / 8.6
 // 9.0 9.6, gate/up 39.6 41.9 45.7 / 37.6 39.0 39.5, down 21.0 25.0 30.4 / 19.9 20.6 22.5; 32B down 51.2 58.6 68.4 / 47.3 48.8
-// 50.8; 0.6B o 4.7 5.8 6.4 / 4.1 4.5 4.8, down 7.4 9.0 10.4 / 5.0 5.6 6.3; slower: 1.7B qkv at one row 6.0 / 6.7.
+// 50.8; 0.6B o 4.7 5.8 6.4 / 4.1 4.5 4.8, down 7.4 9.0 10.4 / 5.0 5.6 6.3.
 // What a large copy reaches (6.2 TB/s) would take 8.1, 5.4, 32.5 and 16.2 us of the 8B shape's four: what is left is the
 // launch, the first bytes' latency and the sum over the waves, about 4 us each. Measured and not taken: three blocks in
 // flight instead of up to six (8B gate/up at one row 37.9 -> 38.2), a contiguous range of K per wave (42.2).
@@ -208,9 +208,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
       for (int t = 0; t < TILES; ++t) acc[t] = mfma16(a[j], w[t][j], acc[t]);
     if (++slot == S) slot = 0;
   }
+  // (of one row three in four are no lane's: left out, a normed product of one row takes 0.5 us less; a branch for each of
+  // the four made more rows 1 to 2 % slower)
   if (nm.norm_partial) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    auto squares = [&](int i) {
       float t = (first[i][0] + first[i][1]) + (first[i][2] + first[i][3]);
       if (g * 4 + i < M)
         for (int p4 = (WAVES + wave) * 16 + col; p4 < nm.norm_parts >> 2; p4 += WAVES * 16) {
@@ -219,7 +220,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
         }
       t = row16_sum(t);
       if (col == 0) ssq[wave][g * 4 + i] = t;
-    }
+    };
+    squares(0);
+    if (M > 1) squares(1), squares(2), squares(3);
   }
   // the sums meet in LDS, in wave order
   __syncthreads();  // every wave is done with its ring
@@ -236,14 +239,16 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
     for (int w = 0; w < WAVES - 1; ++w) acc[t] += red[w][t][lane];
   float rscale[4];  // normed: rsqrt(mean of squares + eps) of the rows this lane writes
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    rscale[i] = 1.0f;
-    if (nm.norm_partial) {
+  for (int i = 0; i < 4; ++i) rscale[i] = 1.0f;
+  if (nm.norm_partial) {
+    auto scale = [&](int i) {
       float t = 0.f;
 #pragma unroll
       for (int w = 0; w < WAVES; ++w) t += ssq[w][g * 4 + i];
       rscale[i] = 1.0f / sqrtf(t / (float)K + nm.norm_eps);
-    }
+    };
+    scale(0);
+    if (M > 1) scale(1), scale(2), scale(3);
   }
   float sq[4] = {0.f, 0.f, 0.f, 0.f};  // emit: the squares of the workgroup's columns, per row of this lane
 #pragma unroll
