@@ -70,9 +70,9 @@ __device__ __forceinline__ void sk_wait_loads() {  // until at most N of the wav
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// NI loads per block: a ring as deep as the LDS allows, with one workgroup of 8 waves or two of 4 on a compute unit
-constexpr int sk_slots(int ni, int waves) {
-  const int fit = ((waves == 8 ? 160 : 80) - 1) / (waves * ni);
+// NI loads per block: a ring as deep as the LDS allows, with `per_cu` workgroups on a compute unit
+constexpr int sk_slots(int ni, int waves, int per_cu) {
+  const int fit = (160 / per_cu - 1) / (waves * ni);
   return fit > 6 ? 6 : fit;
 }
 
@@ -87,7 +87,7 @@ __device__ __forceinline__ void sk_wait_block(int behind) {  // `behind` (< S) b
 }
 
 // NW: loads of 8 weight rows per block (of each weight), NA: of 8 activation rows
-template <int NW, int NA, bool GATED, int WAVES>
+template <int NW, int NA, bool GATED, int WAVES, int PER_CU>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
     const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N,
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
   constexpr int CT = (NW + 1) / 2;                // tiles of 16 weight rows
   constexpr int TILES = GATED ? 2 : CT;           // accumulators: gate and up, or the weight's tiles
   constexpr int NI = (GATED ? 2 : 1) * NW + NA;   // loads of a block
-  constexpr int S = sk_slots(NI, WAVES);
+  constexpr int S = sk_slots(NI, WAVES, PER_CU);
   static_assert(!GATED || CT == 1, "the gated epilogue takes up to 16 rows of each weight");
   static_assert(S >= 2 && (S - 1) * NI < 63, "the counter of loads in flight");
   extern __shared__ __align__(1024) unsigned char smem[];   // [WAVES][S][NI KB]; afterwards the waves' sums
@@ -293,26 +293,34 @@ struct SkinnyArgs {
   void* out;
 };
 
-template <int NW, int NA, bool GATED, int WAVES>
+template <int NW, int NA, bool GATED, int WAVES, int PER_CU>
 static int launch_skinny(const SkinnyArgs& a, const SkinnyNorm& nm, hipStream_t stream) {
   constexpr int NI = (GATED ? 2 : 1) * NW + NA;
-  constexpr size_t smem = (size_t)sk_slots(NI, WAVES) * WAVES * NI * 1024;
+  constexpr size_t smem = (size_t)sk_slots(NI, WAVES, PER_CU) * WAVES * NI * 1024;
   static bool configured = false;
   if (!configured) {  // above 64 KB the size has to be allowed first
-    if (hipFuncSetAttribute((const void*)gemm_skinny_kernel<NW, NA, GATED, WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)gemm_skinny_kernel<NW, NA, GATED, WAVES, PER_CU>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
       JLLM_FAIL("gemm_skinny: cannot reserve %zu bytes of LDS", smem);
     configured = true;
   }
-  gemm_skinny_kernel<NW, NA, GATED, WAVES><<<(a.N + a.rows - 1) / a.rows, WAVES * 64, smem, stream>>>(
+  gemm_skinny_kernel<NW, NA, GATED, WAVES, PER_CU><<<(a.N + a.rows - 1) / a.rows, WAVES * 64, smem, stream>>>(
       a.A, a.lda, a.W, a.W2, a.bias, a.bias_dtype, a.out, a.out_dtype, a.ldo, a.M, a.N, a.K, a.epilogue, nm, a.rows);
   JLLM_CHECK_LAUNCH("gemm_skinny");
   return 0;
 }
 
+template <int NW, bool GATED, int WAVES, int PER_CU>
+static int launch_skinny_rows(const SkinnyArgs& a, const SkinnyNorm& nm, hipStream_t stream) {
+  return a.M <= 8 ? launch_skinny<NW, 1, GATED, WAVES, PER_CU>(a, nm, stream) : launch_skinny<NW, 2, GATED, WAVES, PER_CU>(a, nm, stream);
+}
+
 template <int NW, bool GATED>
-static int launch_skinny_rows(const SkinnyArgs& a, const SkinnyNorm& nm, int waves, hipStream_t stream) {
-  if (waves == 8) return a.M <= 8 ? launch_skinny<NW, 1, GATED, 8>(a, nm, stream) : launch_skinny<NW, 2, GATED, 8>(a, nm, stream);
-  return a.M <= 8 ? launch_skinny<NW, 1, GATED, 4>(a, nm, stream) : launch_skinny<NW, 2, GATED, 4>(a, nm, stream);
+static int launch_skinny_waves(const SkinnyArgs& a, const SkinnyNorm& nm, int per_cu, hipStream_t stream) {
+  switch (per_cu) {
+    case 1: return launch_skinny_rows<NW, GATED, 8, 1>(a, nm, stream);
+    case 2: return launch_skinny_rows<NW, GATED, 4, 2>(a, nm, stream);
+    default: return launch_skinny_rows<NW, GATED, 4, 3>(a, nm, stream);
+  }
 }
 
 static int skinny_checked(const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype,
@@ -339,14 +347,17 @@ static int skinny_checked(const void* A, int lda, const void* W, const void* W2,
   if (cus <= 0) JLLM_FAIL("gemm_skinny: the GPU's compute units could not be read");
   const SkinnyArgs a{(const bf16_t*)A, (const bf16_t*)W, (const bf16_t*)W2, bias, lda, bias_dtype, out_dtype, ldo, M, N, K, epilogue, rows, out};
   // One workgroup of 8 waves per compute unit where there are no more workgroups than those; else two of 4 waves, so that
-  // one streams while the other adds up and stores.
-  const int waves = groups > cus ? 4 : 8;
-  if (W2) return rows <= 8 ? launch_skinny_rows<1, true>(a, nm, waves, stream) : launch_skinny_rows<2, true>(a, nm, waves, stream);
+  // one streams while the other adds up and stores; three, with a shallower ring, where there are more than two of them and K
+  // is so short that a wave has no use for a deep one. Two / three at 1, 8 and 16 rows, us: 151,936 x 1,024 60.7 64.2 67.8 /
+  // 54.0 58.1 61.3 (53.4 80.2 91.2 from memory into registers), gated 8,960 x 1,536 15.3 16.4 16.6 / 13.5 14.6 15.0; from K =
+  // 2,048 on three are the same to 2 % slower (gated 8,192 x 2,048).
+  const int per_cu = groups <= cus ? 1 : groups > 2 * cus && K < 2048 ? 3 : 2;
+  if (W2) return rows <= 8 ? launch_skinny_waves<1, true>(a, nm, per_cu, stream) : launch_skinny_waves<2, true>(a, nm, per_cu, stream);
   switch ((rows + 7) / 8) {
-    case 1: return launch_skinny_rows<1, false>(a, nm, waves, stream);
-    case 2: return launch_skinny_rows<2, false>(a, nm, waves, stream);
-    case 3: return launch_skinny_rows<3, false>(a, nm, waves, stream);
-    default: return launch_skinny_rows<4, false>(a, nm, waves, stream);
+    case 1: return launch_skinny_waves<1, false>(a, nm, per_cu, stream);
+    case 2: return launch_skinny_waves<2, false>(a, nm, per_cu, stream);
+    case 3: return launch_skinny_waves<3, false>(a, nm, per_cu, stream);
+    default: return launch_skinny_waves<4, false>(a, nm, per_cu, stream);
   }
 }
 
