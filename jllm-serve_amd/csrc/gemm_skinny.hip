@@ -86,8 +86,8 @@ __device__ __forceinline__ void sk_wait_block(int behind) {  // `behind` (< S) b
   sk_wait_loads<0>();
 }
 
-// NW: loads of 8 weight rows per block (of each weight), NA: of 8 activation rows
-template <int NW, int NA, bool GATED, int WAVES, int PER_CU>
+// NW: loads of 8 weight rows per block (of each weight), NA: of 8 activation rows; TURN: see the host's rule
+template <int NW, int NA, bool GATED, int WAVES, int PER_CU, bool TURN>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
     const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N,
@@ -107,8 +107,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
   const int n0 = blockIdx.x * rows;
   const int nblk = K / SK_BLOCK;
   // gated: workgroups walk K from different starting blocks, so that at any moment they ask the L2 for different parts of
-  // the (shared) activations (12,288 x 4,096 at one row 39.2 -> 37.9 us; without the gate 6,144 x 4,096 12.4 -> 13.4)
-  const int rot = GATED ? (int)((blockIdx.x * 14u) % (unsigned)nblk) : 0;
+  // the (shared) activations (12,288 x 4,096 at one row 39.2 -> 37.9 us); without the gate from a power of two of them
+  // (which needs no division) where the host says so
+  const int rot = GATED  ? (int)((blockIdx.x * 14u) % (unsigned)nblk)
+                  : TURN ? (int)(blockIdx.x & ((1u << (31 - __builtin_clz((unsigned)nblk))) - 1u))
+                         : 0;
   // wave 0 writes the outputs: what it adds into (the residual, the bias) is requested before anything else
   float prev[CT][4], b[CT], eg[CT];
 #pragma unroll
@@ -293,33 +296,36 @@ struct SkinnyArgs {
   void* out;
 };
 
-template <int NW, int NA, bool GATED, int WAVES, int PER_CU>
+template <int NW, int NA, bool GATED, int WAVES, int PER_CU, bool TURN>
 static int launch_skinny(const SkinnyArgs& a, const SkinnyNorm& nm, hipStream_t stream) {
   constexpr int NI = (GATED ? 2 : 1) * NW + NA;
   constexpr size_t smem = (size_t)sk_slots(NI, WAVES, PER_CU) * WAVES * NI * 1024;
   static bool configured = false;
   if (!configured) {  // above 64 KB the size has to be allowed first
-    if (hipFuncSetAttribute((const void*)gemm_skinny_kernel<NW, NA, GATED, WAVES, PER_CU>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)gemm_skinny_kernel<NW, NA, GATED, WAVES, PER_CU, TURN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
       JLLM_FAIL("gemm_skinny: cannot reserve %zu bytes of LDS", smem);
     configured = true;
   }
-  gemm_skinny_kernel<NW, NA, GATED, WAVES, PER_CU><<<(a.N + a.rows - 1) / a.rows, WAVES * 64, smem, stream>>>(
+  gemm_skinny_kernel<NW, NA, GATED, WAVES, PER_CU, TURN><<<(a.N + a.rows - 1) / a.rows, WAVES * 64, smem, stream>>>(
       a.A, a.lda, a.W, a.W2, a.bias, a.bias_dtype, a.out, a.out_dtype, a.ldo, a.M, a.N, a.K, a.epilogue, nm, a.rows);
   JLLM_CHECK_LAUNCH("gemm_skinny");
   return 0;
 }
 
 template <int NW, bool GATED, int WAVES, int PER_CU>
-static int launch_skinny_rows(const SkinnyArgs& a, const SkinnyNorm& nm, hipStream_t stream) {
-  return a.M <= 8 ? launch_skinny<NW, 1, GATED, WAVES, PER_CU>(a, nm, stream) : launch_skinny<NW, 2, GATED, WAVES, PER_CU>(a, nm, stream);
+static int launch_skinny_rows(const SkinnyArgs& a, const SkinnyNorm& nm, bool turn, hipStream_t stream) {
+  if constexpr (!GATED && PER_CU < 3) {
+    if (turn) return a.M <= 8 ? launch_skinny<NW, 1, GATED, WAVES, PER_CU, true>(a, nm, stream) : launch_skinny<NW, 2, GATED, WAVES, PER_CU, true>(a, nm, stream);
+  }
+  return a.M <= 8 ? launch_skinny<NW, 1, GATED, WAVES, PER_CU, false>(a, nm, stream) : launch_skinny<NW, 2, GATED, WAVES, PER_CU, false>(a, nm, stream);
 }
 
 template <int NW, bool GATED>
-static int launch_skinny_waves(const SkinnyArgs& a, const SkinnyNorm& nm, int per_cu, hipStream_t stream) {
+static int launch_skinny_waves(const SkinnyArgs& a, const SkinnyNorm& nm, int per_cu, bool turn, hipStream_t stream) {
   switch (per_cu) {
-    case 1: return launch_skinny_rows<NW, GATED, 8, 1>(a, nm, stream);
-    case 2: return launch_skinny_rows<NW, GATED, 4, 2>(a, nm, stream);
-    default: return launch_skinny_rows<NW, GATED, 4, 3>(a, nm, stream);
+    case 1: return launch_skinny_rows<NW, GATED, 8, 1>(a, nm, turn, stream);
+    case 2: return launch_skinny_rows<NW, GATED, 4, 2>(a, nm, turn, stream);
+    default: return launch_skinny_rows<NW, GATED, 4, 3>(a, nm, turn, stream);
   }
 }
 
@@ -352,12 +358,18 @@ static int skinny_checked(const void* A, int lda, const void* W, const void* W2,
   // 54.0 58.1 61.3 (53.4 80.2 91.2 from memory into registers), gated 8,960 x 1,536 15.3 16.4 16.6 / 13.5 14.6 15.0; from K =
   // 2,048 on three are the same to 2 % slower (gated 8,192 x 2,048).
   const int per_cu = groups <= cus ? 1 : groups > 2 * cus && K < 2048 ? 3 : 2;
-  if (W2) return rows <= 8 ? launch_skinny_waves<1, true>(a, nm, per_cu, stream) : launch_skinny_waves<2, true>(a, nm, per_cu, stream);
+  // Rows of W that lie a multiple of 4 KB apart, and long rows in workgroups of up to 16 of them: the workgroups begin at
+  // different blocks. All at one block, they ask the memory for the same piece of every row at once. One / different at 1, 8 and 16 rows, us:
+  // 12,288 x 4,096 22.0 23.4 24.0 / 20.7 22.2 22.6, 4,096 x 11,008 23.2 24.0 25.1 / 19.7 20.3 21.4, 8,192 x 8,192 32.0 34.2
+  // 35.4 / 27.7 28.2 28.7, 32,768 x 2,048 30.4 32.1 33.0 / 26.9 29.7 29.8, 4,096 x 4,096 8.9 9.5 10.1 / 8.7 9.1 9.7; slower so:
+  // 5,120 x 17,408 (20 rows a workgroup) by 9 %, 7,168 x 5,120 (28) by 4 %.
+  const bool turn = K % 2048 == 0 || (rows <= 16 && K >= 8192);
+  if (W2) return rows <= 8 ? launch_skinny_waves<1, true>(a, nm, per_cu, false, stream) : launch_skinny_waves<2, true>(a, nm, per_cu, false, stream);
   switch ((rows + 7) / 8) {
-    case 1: return launch_skinny_waves<1, false>(a, nm, per_cu, stream);
-    case 2: return launch_skinny_waves<2, false>(a, nm, per_cu, stream);
-    case 3: return launch_skinny_waves<3, false>(a, nm, per_cu, stream);
-    default: return launch_skinny_waves<4, false>(a, nm, per_cu, stream);
+    case 1: return launch_skinny_waves<1, false>(a, nm, per_cu, turn, stream);
+    case 2: return launch_skinny_waves<2, false>(a, nm, per_cu, turn, stream);
+    case 3: return launch_skinny_waves<3, false>(a, nm, per_cu, turn, stream);
+    default: return launch_skinny_waves<4, false>(a, nm, per_cu, turn, stream);
   }
 }
 

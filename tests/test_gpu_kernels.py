@@ -327,6 +327,29 @@ def test_few_row_products_at_any_weight_rows_per_workgroup(ops, monkeypatch, M, 
     assert torch.equal(out, ops.gemm(a, w, bias=bias, out_dtype=torch.float32))
 
 
+@pytest.mark.parametrize("M,N,K,rows", [(1, 160, 2048, 32), (9, 4096, 4096, 16), (8, 4112, 2048, 8), (16, 8192, 4096, 20), (3, 48, 8320, 4), (13, 272, 11008, 16),
+                                        (5, 6144, 2048, 24), (16, 96, 16384, 12)])
+def test_few_row_products_that_begin_at_different_blocks(ops, monkeypatch, M, N, K, rows):
+    """Rows a multiple of 4 KB apart, and long ones: workgroups that begin anywhere in K, with as many blocks as a power of two
+    and more, for every number of loads per block, one and two workgroups a compute unit. Against float64 within the bound of an
+    fp32 sum of K products; a row has the same bits alone as beside others, and adding as storing."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M * N + K + rows)
+    rnd = lambda *shape: torch.randn(*shape, device=DEV, generator=gen)
+    a, w, res0 = rnd(M, K).bfloat16(), (rnd(N, K) / math.sqrt(K)).bfloat16(), rnd(M, N)
+    monkeypatch.setattr(ops, "_skinny_rows", lambda *_: rows)
+    ops.reset_stats()
+    out = ops.gemm(a, w, out_dtype=torch.float32)
+    bound = 2 * K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T) + 1e-6
+    assert bool(((out.double() - a.double() @ w.double().T).abs() <= bound).all())
+    res = res0.clone()
+    promise = ops.gemm_add_then_norm(a, w, res, torch.ones(N, device=DEV), 1e-5, torch.bfloat16)
+    assert torch.equal(res, res0 + out) and torch.equal(promise.scaled, res.bfloat16())
+    for r in {0, M // 2, M - 1}:
+        assert torch.equal(ops.gemm(a[r:r + 1].contiguous(), w, out_dtype=torch.float32), out[r:r + 1])
+    assert set(ops.stats()["ran"]) == {"jllm_gemm_skinny_bf16", "jllm_gemm_skinny_norm_bf16"}
+
+
 @pytest.mark.parametrize("rows", [32, 64, 96, 128])
 @pytest.mark.parametrize("M,N,K,parts", [(17, 160, 128, 1), (33, 1040, 640, 2), (64, 2064, 1152, 3), (1, 336, 2560, 6), (48, 4112, 256, 1),
                                          (25, 9728, 384, 1), (64, 192, 4096, 8)])
