@@ -933,6 +933,27 @@ def _wide_us(M: int, N: int, K: int, gated: bool, rows: int, tile: int, parts: i
     return t
 
 
+@functools.lru_cache(maxsize=None)
+def _wide_best(tiles64: int, most: int, N: int, K: int, gated: bool) -> Tuple[float, Tuple[int, int, int]]:
+    """The cheapest (weight rows, activation rows, parts of K) by the estimate, and its time, for ``tiles64`` tiles of 64 rows
+    (``most``: rows of the fullest tile). It is the same for all row counts that have these tiles, so that a prompt of a
+    length that was not seen before does not weigh 30 choices per product anew (some 45 us of the host's time each)."""
+    cus = compute_units()
+    M = tiles64 * 64 if most == 128 else most
+    best, plan = float("inf"), (64, 64, 1)
+    for rows in (32, 64, 96, 128):
+        for tile in (64, 128):
+            tiles = -(-N // (rows // 2 if gated else rows)) * -(-M // tile)
+            for parts in (1, 2, 3, 4):
+                per = -(-(K // 128) // parts)
+                if parts > 1 and (tiles * parts > 2 * cus or per < STREAM_MIN_BLOCKS or -(-(K // 128) // per) != parts):
+                    continue
+                t = _wide_us(M, N, K, gated, rows, tile, parts)
+                if t < best:
+                    best, plan = t, (rows, tile, parts)
+    return best, plan
+
+
 @functools.lru_cache(maxsize=8192)
 def _wide_plan(M: int, N: int, K: int, gated: bool, adds: int = 0) -> Optional[Tuple[int, int, int]]:
     """(weight rows, activation rows, parts of K) with which the second weight-streaming kernel takes a product of more than
@@ -947,23 +968,12 @@ def _wide_plan(M: int, N: int, K: int, gated: bool, adds: int = 0) -> Optional[T
     41.6 / 34.5, 8B qkv at 320 39.2 / 35.4. Beyond, the tiled kernels win: 8B gate/up at 200 rows 79.9 / 101, down 44.8 / 54.9."""
     if not STREAM_MAX_ROWS < M <= WIDE_MOST_ROWS or K % 128 or N % 16 or K < WIDE_LEAST_K or (adds and N > WIDE_ADD_COLUMNS):
         return None
-    cus = compute_units()
     rows, cut = _tiled_plan(M, N, K, gated)
     best = WIDE_AT_MOST * (TILED_FIXED_US + (_large_us(M, N, K, gated, rows, cut) if rows else _small_us(M, N, K, gated, cut)))
     if adds == ADDS_AND_NORM:
         best += NORM_LAUNCH_US
-    plan = None
-    for rows in (32, 64, 96, 128):
-        for tile in (64, 128):
-            tiles = -(-N // (rows // 2 if gated else rows)) * -(-M // tile)
-            for parts in (1, 2, 3, 4):
-                per = -(-(K // 128) // parts)
-                if parts > 1 and (tiles * parts > 2 * cus or per < STREAM_MIN_BLOCKS or -(-(K // 128) // per) != parts):
-                    continue
-                t = _wide_us(M, N, K, gated, rows, tile, parts)
-                if t < best:
-                    best, plan = t, (rows, tile, parts)
-    return plan
+    t, plan = _wide_best(-(-M // 64), min(M, 128), N, K, gated)
+    return plan if t < best else None
 
 
 _NO_NORM = (None, F32, 0.0, None, 0)

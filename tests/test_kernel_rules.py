@@ -211,6 +211,21 @@ def test_plans_of_the_second_weight_streaming_kernel():
     assert ops._wide_plan(487, 12288, 4096, True) is None and ops._wide_plan(300, 1024, 100, False) is None
 
 
+def test_a_new_row_count_does_not_weigh_every_choice_again(monkeypatch):
+    """The choices of the ring kernel for many rows cost the same for all row counts with the same tiles: the host weighs them once."""
+    weighed = []
+    estimate = ops._wide_us
+    monkeypatch.setattr(ops, "_wide_us", lambda *args: weighed.append(args) or estimate(*args))
+    for cached in (ops._wide_plan, getattr(ops, "_wide_best", ops._wide_plan)):
+        cached.cache_clear()
+    ops._wide_plan(449, 4096, 1024, False, 0)
+    once = len(weighed)
+    for m in range(450, 513):
+        for adds in (0, 1, 2):
+            ops._wide_plan(m, 4096, 1024, False, adds)
+    assert 0 < once == len(weighed)
+
+
 def test_declared_arguments_are_those_of_the_sources():
     """Every entry point's declared argument types against its definition: a pointer declared as an int would reach the
     kernel cut to 32 bits."""
