@@ -592,9 +592,12 @@ def test_command_line_runs_the_design(folders, tmp_path):
                                 {"slopes": True}])
 def test_single_rows_at_key_size_128(heads, kv_heads, maps, dv, kw):
     """Rows of one key, of one block and of many, whole and in key ranges (merged by a launch and by the kernel that finishes the
-    heads), against the general kernel: probabilities rounded to bf16 move an output by at most 2^-8 of the largest value, and a
-    row is the same alone as beside others. Values and keys outside what a row sees are infinite: they must not reach it. (20
-    heads over one key slot: more than the kernel has columns, the tile kernel takes them.)"""
+    heads), against the general kernel, each output within its own rounding: a probability rounded to bf16 (eight significant
+    bits) is off by 2^-8 of itself at most, so an output by 2^-8 of sum(p |v|), beside the scores' sums in fp32 (2^-13 of it, and
+    more than they are off). A row alone, whose keys are cut into other ranges, is within the same of the general kernel. Values and keys outside
+    what a row sees are infinite: they must not reach it. The newest key and those on either side of the seams of blocks and of
+    the waves' shares have values a hundred times the others': left out, each would move its row by far more than the bound, which
+    the general kernel shows. (20 heads over one key slot: more than the kernel has columns, the tile kernel takes them.)"""
     from jllm_serve_amd.kernels import ops
     dk, page, ctx = 128, 16, (1, 64, 65, 700, 1999)
     gen = torch.Generator(device=DEV)
@@ -612,7 +615,27 @@ def test_single_rows_at_key_size_128(heads, kv_heads, maps, dv, kw):
     q = rnd(T, heads * maps * dk).bfloat16()
     rows, pos = torch.arange(T, dtype=torch.int32, device=DEV), torch.tensor([c - 1 for c in ctx], dtype=torch.int32, device=DEV)
     args = (q, kc, vc, table, rows, pos, heads, kv_heads, maps, dk, dv, dk ** -0.5)
+    marked = {}
+    for r, c in enumerate(ctx):
+        last = (c - 1) // 64 * 64
+        seams = {c - 1, last, last - 1, last + 16, (c - 1) // 16 * 16 - 1, last // 2 // 64 * 64} if c > 64 else {c - 1}
+        first = max(0, c - window) if window else (c - 1) // chunk * chunk if chunk else 0
+        marked[r] = sorted(p for p in seams if first <= p < c)
+        for p in marked[r]:
+            kc[table[r, p // page], :, p % page] = 0
+            vc[table[r, p // page], :, p % page] *= 100
     want = ops.attention_dv(*args, exact=True, out_dtype=torch.float32, **kw)
+    general = lambda values: ops.attention_dv(q, kc, values, *args[3:], exact=True, out_dtype=torch.float32, **kw)
+    bound = (2.0 ** -8 + 2.0 ** -13) * general(vc.abs()) + 1e-6
+    for nth in range(max(len(m) for m in marked.values())):  # the nth marked key of every row left out
+        without, rows_left = vc.clone(), []
+        for r, m in marked.items():
+            if nth < len(m) and (ctx[r] - 1 - m[nth]) < 200:  # (with slopes, far keys hardly count)
+                without[table[r, m[nth] // page], :, m[nth] % page] = 0
+                rows_left.append(r)
+        moved = (general(without) - want).abs() / bound
+        for r in rows_left:
+            assert float(moved[r].max()) > 3, (r, m[nth])
     for r, c in enumerate(ctx):
         first = max(0, c - window) if window else (c - 1) // chunk * chunk if chunk else 0
         for p in range(width * page):
@@ -620,20 +643,20 @@ def test_single_rows_at_key_size_128(heads, kv_heads, maps, dv, kw):
                 kc[table[r, p // page], :, p % page] = float("inf")
                 vc[table[r, p // page], :, p % page] = float("inf")
     tiles = torch.tensor([[r, r, 1, -1] for r in range(T)], dtype=torch.int32, device=DEV).flatten()
-    bound = 2.0 ** -8 * 6.0
     for longest in (64, max(ctx)):  # the step's longest request decides the key ranges; rows beyond it are left out
         n = sum(c <= longest for c in ctx)
         meta = {"tiles_dev": tiles[:4 * n].contiguous(), "n_tiles": n, "single_rows": True, "max_context": longest}
         part = (q[:n].contiguous(), kc, vc, table, rows[:n].contiguous(), pos[:n].contiguous(), *args[6:])
         got = ops.attention_dv(*part, meta=meta, out_dtype=torch.float32, **kw)
-        assert bool(torch.isfinite(got).all()) and float((got - want[:n]).abs().max()) <= bound
+        assert bool(((got - want[:n]).abs() <= bound[:n]).all())
         split = ops.attention_dv(*part, meta=meta, out_dtype=torch.float32, defer_merge=True, **kw)
         assert isinstance(split, ops.SplitHeads) or longest == 64 or window or chunk
         if isinstance(split, ops.SplitHeads):
             done = ops.heads_finish(split, heads, maps, dv, torch.float32, lam=0.3)
             ref = ops.heads_finish(want[:n].contiguous(), heads, maps, dv, torch.float32, lam=0.3)
-            assert float((done - ref).abs().max()) <= 2 * bound
+            room = ops.heads_finish(bound[:n].contiguous(), heads, maps, dv, torch.float32, lam=-0.3)
+            assert bool(((done - ref).abs() <= room + 1e-6 * (1 + ref.abs())).all())
             one = {**meta, "n_tiles": 1, "tiles_dev": torch.tensor([n - 1, 0, 1, -1], dtype=torch.int32, device=DEV)}
             alone = ops.attention_dv(q[n - 1:n].contiguous(), kc, vc, table, rows[n - 1:n].contiguous(), pos[n - 1:n].contiguous(), *args[6:],
                                      meta=one, out_dtype=torch.float32, **kw)
-            assert float((alone - got[n - 1:n]).abs().max()) <= bound
+            assert bool(((alone - want[n - 1:n]).abs() <= bound[n - 1:n]).all())
