@@ -44,11 +44,6 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
 }
 
-// scores are kept in units of log2(e), so the exponentials are single v_exp_f32 instructions
-__device__ __forceinline__ float safe_exp_diff(float a, float m) {
-  return a == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(a - m);
-}
-
 // merges the splits s_lo..s_hi of one (row, head) in ascending order and writes the normalised output; one wave,
 // lane s reads the (max, sum) of split s, so all of them are requested at once
 __device__ __forceinline__ void combine_head(const float* part_acc, const float* part_ml, size_t base, int s_lo, int s_hi,
@@ -367,12 +362,12 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(G
       float mn = m1;
 #pragma unroll
       for (int u = 0; u < DA_U; ++u) mn = fmaxf(mn, sc1[u]);
-      const float alpha1 = safe_exp_diff(m1, mn);  // mn is finite for real heads: a group's first key is valid
+      const float alpha1 = exp2_diff(m1, mn);  // mn is finite for real heads: a group's first key is valid
       float p[DA_U];
       float ps = 0.f;
 #pragma unroll
       for (int u = 0; u < DA_U; ++u) {
-        p[u] = safe_exp_diff(sc1[u], mn);
+        p[u] = exp2_diff(sc1[u], mn);
         ps += p[u];
       }
       l1 = l1 * alpha1 + ps;
@@ -402,12 +397,12 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(G
 #pragma unroll
       for (int u = 0; u < DA_U; ++u) mn = fmaxf(mn, sc[u][g]);
       // the first key of a group is always valid, so mn is finite here
-      const float alpha = safe_exp_diff(m[g], mn);
+      const float alpha = exp2_diff(m[g], mn);
       float p[DA_U];
       float ps = 0.f;
 #pragma unroll
       for (int u = 0; u < DA_U; ++u) {
-        p[u] = safe_exp_diff(sc[u][g], mn);
+        p[u] = exp2_diff(sc[u][g], mn);
         ps += p[u];
       }
       l[g] = l[g] * alpha + ps;
@@ -448,7 +443,7 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(G
       const float om = __shfl_xor(m[g], o, 64);
       const float ol = __shfl_xor(l[g], o, 64);
       const float mn = fmaxf(m[g], om);
-      const float a = safe_exp_diff(m[g], mn), b = safe_exp_diff(om, mn);
+      const float a = exp2_diff(m[g], mn), b = exp2_diff(om, mn);
       l[g] = l[g] * a + ol * b;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -477,7 +472,7 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(G
       for (int w = 0; w < DA_WAVES - 1; ++w) {
         const float om = mrg[w][g][lane][0], ol = mrg[w][g][lane][1];
         const float mn = fmaxf(m[g], om);
-        const float a = safe_exp_diff(m[g], mn), b = safe_exp_diff(om, mn);
+        const float a = exp2_diff(m[g], mn), b = exp2_diff(om, mn);
         l[g] = l[g] * a + ol * b;
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc[g][i] = acc[g][i] * a + mrg[w][g][lane][2 + i] * b;
@@ -684,7 +679,7 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));  // over the four key groups: the head's maximum in this turn
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     if (mx > m1 + 8.0f) {  // also the first turn with a visible key (m1 = -inf)
-      const float alpha = safe_exp_diff(m1, mx);
+      const float alpha = exp2_diff(m1, mx);
       l1 *= alpha;
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[j] *= alpha;
@@ -693,7 +688,7 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
     float p[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      p[i] = safe_exp_diff(z[i], m1);  // m1 = -inf only while every key so far was beyond the end: then z is too
+      p[i] = exp2_diff(z[i], m1);  // m1 = -inf only while every key so far was beyond the end: then z is too
       l1 += p[i];
     }
     const u32x2 pb = u32x2{pack2(p[0], p[1]), pack2(p[2], p[3])};
@@ -736,7 +731,7 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
       const float* src = &mrg[w][lane][0];
       const float om = src[0], ol = src[1];
       const float mn = fmaxf(m1, om);
-      const float a = safe_exp_diff(m1, mn), b = safe_exp_diff(om, mn);
+      const float a = exp2_diff(m1, mn), b = exp2_diff(om, mn);
       l1 = l1 * a + ol * b;
 #pragma unroll
       for (int j = 0; j < 8; ++j)

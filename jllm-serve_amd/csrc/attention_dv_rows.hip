@@ -25,8 +25,6 @@
 #define AR_WAVES 4
 #define AR_KEYS 64
 
-__device__ __forceinline__ float exp2_diff(float a, float m) { return a == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(a - m); }
-
 template <int DVB>
 __global__ __launch_bounds__(AR_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, 2))) void attention_dv_rows_kernel(
     const bf16_t* __restrict__ q, int ldq, float* __restrict__ out, int ldo, const bf16_t* __restrict__ kc,

@@ -35,6 +35,7 @@
 #include <math.h>
 
 #include "common.h"
+#include "lds_ring.h"
 #include "mfma.h"
 
 #define PA_ROWS 128
@@ -308,19 +309,8 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void prefill_attention_k
 #define PA_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
 #define PA_LGKMCNT0() __builtin_amdgcn_s_waitcnt((15) | (3 << 14) | (7 << 4) | (0 << 8))
 
-// One load of 16 bytes per lane from global memory straight into LDS, written as the instruction itself. Through the
-// compiler's builtin the compiler knows of a load into LDS that is on its way, and from then on it waits for all
-// outstanding loads and LDS reads before every use of either (it cannot tell which of them that load might be): the
-// waits below are written out by hand instead, as the pipeline needs them, and nothing else in the loop of the kernel
-// is a vector memory load (table entries come through the scalar cache where pages hold 16 positions or more).
-// `lds` is the byte address in LDS of the wave's 1 KB (lane l's 16 bytes land at lds + 16 l).
-__device__ __forceinline__ void load_to_lds_16(const void* base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ void load_to_lds_16(const void* address, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(address), "s"(lds) : "memory", "m0");
-}
-
+// Keys and values come straight into LDS (lds_ring.h); nothing else in the loop of the kernel is a vector memory load (table
+// entries come through the scalar cache where pages hold 16 positions or more).
 // WIDE: pages hold 16 positions or more, so the 16 keys a wave brings per block lie in one page and its table entry is
 // the same in all lanes
 template <bool WIDE>

@@ -100,6 +100,10 @@ __device__ __forceinline__ float norm_scale(float ss, int n, float eps) {
   return (float)(1.0 / sqrt((double)(ss / (float)n + eps)));
 }
 
+// 2^(a - m), zero for a = -infinity whatever m is: the attention kernels keep scores in units of log2(e), so that the
+// exponentials are single v_exp_f32 instructions
+__device__ __forceinline__ float exp2_diff(float a, float m) { return a == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(a - m); }
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = JLLM_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, JLLM_WAVE);

@@ -31,6 +31,7 @@
 // Epilogues as in the other tiled kernel (gemm_epilogue.h). Needs K % 32 == 0 and at least NS - 1 stages, 16-byte
 // aligned rows; any M and N (rows beyond the end are read as the last row and never stored).
 #include "common.h"
+#include "lds_ring.h"
 #include "gemm_epilogue.h"
 #include "mfma.h"
 
@@ -112,11 +113,7 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
 #pragma unroll
     for (int c = 0; c < L0; ++c) {
       if (c >= LA1 && c < LA && group != 0) continue;
-      // the instruction itself: m0 holds the LDS address of the wave's 1 KB, lane l's 16 bytes land at m0 + 16 l
-      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                   :
-                   : "v"(goff[c]), "s"(gbase[c] + kbytes), "s"(ldst[c] + slot)
-                   : "memory", "m0");
+      load_to_lds_16(gbase[c] + kbytes, goff[c], ldst[c] + slot);
     }
   };
 

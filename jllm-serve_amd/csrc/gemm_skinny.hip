@@ -6,7 +6,7 @@
 // of S blocks in LDS that belongs to the wave alone (global_load_lds_dwordx4, 1 KB per instruction: 8 rows of 128 bytes),
 // S - 1 blocks ahead of the multiplies; nothing but the wave's own counter of loads in flight stands between a load and its
 // use, so there is no barrier before the end. A lane's place in LDS is fixed by its number, so the bank swizzle is
-// applied on the global side: the lane that fills slot s of row r fetches the row's 16-byte piece s ^ sk_swz(r).
+// applied on the global side: the lane that fills slot s of row r fetches the row's 16-byte piece s ^ ring_swz(r).
 //
 // Why not from memory into the registers that feed the matrix cores, as this kernel used to: such a load takes 64 bytes of
 // each of 16 rows, and a compute unit's load pipe then passes 25 bytes a clock (6.6 TB/s of the whole chip with everything in
@@ -34,6 +34,7 @@
 //
 // Needs K % 128 == 0, N % 16 == 0, M <= 16, 16-byte aligned rows; the caller falls back otherwise.
 #include "common.h"
+#include "lds_ring.h"
 #include "mfma.h"
 
 #define SK_BLOCK 64                    // k per block
@@ -61,15 +62,6 @@ __device__ __forceinline__ float row16_sum(float d) {
   return d;
 }
 
-// The piece of row r in slot s is s ^ sk_swz(r): 16 lanes that read one piece of 16 rows cover the 64 banks once, and so do 8
-// lanes of 8 rows half of them.
-__device__ __forceinline__ int sk_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-
-template <int N>
-__device__ __forceinline__ void sk_wait_loads() {  // until at most N of the wave's loads are in flight
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 // NI loads per block: a ring as deep as the LDS allows, with `per_cu` workgroups on a compute unit
 constexpr int sk_slots(int ni, int waves, int per_cu) {
   const int fit = (160 / per_cu - 1) / (waves * ni);
@@ -78,12 +70,12 @@ constexpr int sk_slots(int ni, int waves, int per_cu) {
 
 template <int NI, int S>
 __device__ __forceinline__ void sk_wait_block(int behind) {  // `behind` (< S) blocks behind the one that has to be here
-  if (behind == S - 1) return sk_wait_loads<(S - 1) * NI>();
-  if (S > 2 && behind == S - 2) return sk_wait_loads<(S > 2 ? S - 2 : 0) * NI>();
-  if (S > 3 && behind == S - 3) return sk_wait_loads<(S > 3 ? S - 3 : 0) * NI>();
-  if (S > 4 && behind == S - 4) return sk_wait_loads<(S > 4 ? S - 4 : 0) * NI>();
-  if (S > 5 && behind == S - 5) return sk_wait_loads<(S > 5 ? S - 5 : 0) * NI>();
-  sk_wait_loads<0>();
+  if (behind == S - 1) return wait_loads<(S - 1) * NI>();
+  if (S > 2 && behind == S - 2) return wait_loads<(S > 2 ? S - 2 : 0) * NI>();
+  if (S > 3 && behind == S - 3) return wait_loads<(S > 3 ? S - 3 : 0) * NI>();
+  if (S > 4 && behind == S - 4) return wait_loads<(S > 4 ? S - 4 : 0) * NI>();
+  if (S > 5 && behind == S - 5) return wait_loads<(S > 5 ? S - 5 : 0) * NI>();
+  wait_loads<0>();
 }
 
 // NW: loads of 8 weight rows per block (of each weight), NA: of 8 activation rows; TURN: see the host's rule
@@ -152,7 +144,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
     const bool of_w = c < NI - NA;
     const int r = (of_w ? c % NW : c - (NI - NA)) * 8 + lrow;
     const uint32_t at = of_w ? (uint32_t)(min(n0 + min(r, rows - 1), N - 1) - n0) * (uint32_t)K : (uint32_t)min(r, M - 1) * (uint32_t)lda;
-    goff[c] = at * 2u + (uint32_t)((lslot ^ sk_swz(r)) * 16);
+    goff[c] = at * 2u + (uint32_t)((lslot ^ ring_swz(r)) * 16);
   }
   const unsigned char* wbase = (const unsigned char*)(W + (size_t)n0 * K);
   const unsigned char* ubase = GATED ? (const unsigned char*)(W2 + (size_t)n0 * K) : nullptr;
@@ -166,11 +158,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
 #pragma unroll
     for (int c = 0; c < NI; ++c) {
       const unsigned char* base = (c >= NI - NA ? (const unsigned char*)A : GATED && c >= NW ? ubase : wbase) + kbytes;
-      // m0 holds the LDS address of the 1 KB, lane l's 16 bytes land at m0 + 16 l
-      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                   :
-                   : "v"(goff[c]), "s"(base), "s"(lds0 + (uint32_t)(slot * NI + c) * 1024u)
-                   : "memory", "m0");
+      load_to_lds_16(base, goff[c], lds0 + (uint32_t)(slot * NI + c) * 1024u);
     }
   };
 #pragma unroll
@@ -179,14 +167,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
   // ---- fragments: lane l reads row l % 16, 8 of k at (l / 16) * 8 + 32 j: piece l / 16 + 4 j. Rows that no load fetched
   // (eight activation rows, up to eight weight rows in a tile) are the last fetched eight again.
   const int ar = NA == 1 ? col & 7 : col;
-  const int aoff = ((GATED ? 2 : 1) * NW) * 1024 + ar * SK_ROW_BYTES, aswz = sk_swz(ar);
+  const int aoff = ((GATED ? 2 : 1) * NW) * 1024 + ar * SK_ROW_BYTES, aswz = ring_swz(ar);
   int woff[TILES], wswz[TILES];
 #pragma unroll
   for (int t = 0; t < TILES; ++t) {
     const int left = GATED ? NW : NW - 2 * t;  // loads that this tile has
     const int r = (GATED ? 0 : t * 16) + (left == 1 ? col & 7 : col);
     woff[t] = (GATED ? t * NW * 1024 : 0) + r * SK_ROW_BYTES;
-    wswz[t] = sk_swz(r);
+    wswz[t] = ring_swz(r);
   }
   floatx4 acc[TILES];
 #pragma unroll

@@ -28,6 +28,7 @@
 //
 // Needs K % 128 == 0, N % 16 == 0, 16-byte aligned rows; the caller uses another kernel otherwise.
 #include "common.h"
+#include "lds_ring.h"
 #include "mfma.h"
 
 #define GS_ROW_BYTES 128  // a row of a block in LDS: 64 k = 8 pieces of 16 bytes
@@ -55,33 +56,25 @@ struct StreamArgs {
   StreamNorm nm;
 };
 
-// The piece of row r in slot s is s ^ gs_swz(r): 16 lanes that read one piece of 16 rows cover the 64 banks once, and so do 8
-// lanes of 8 rows half of them.
-__device__ __forceinline__ int gs_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-
-template <int N>
-__device__ __forceinline__ void gs_wait_loads() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 // until at most n of the wave's loads are in flight (more than that may have landed)
 __device__ __forceinline__ void gs_wait_at_most(int n) {
   switch (n) {
-    case 0: return gs_wait_loads<0>();
-    case 1: return gs_wait_loads<1>();
-    case 2: return gs_wait_loads<2>();
-    case 3: return gs_wait_loads<3>();
-    case 4: return gs_wait_loads<4>();
-    case 5: return gs_wait_loads<5>();
-    case 6: return gs_wait_loads<6>();
-    case 7: return gs_wait_loads<7>();
-    case 8: return gs_wait_loads<8>();
-    case 9: return gs_wait_loads<9>();
-    case 10: return gs_wait_loads<10>();
-    case 11: return gs_wait_loads<11>();
-    case 12: return gs_wait_loads<12>();
-    case 13: case 14: return gs_wait_loads<13>();
-    case 15: case 16: case 17: return gs_wait_loads<15>();
-    default: return gs_wait_loads<18>();
+    case 0: return wait_loads<0>();
+    case 1: return wait_loads<1>();
+    case 2: return wait_loads<2>();
+    case 3: return wait_loads<3>();
+    case 4: return wait_loads<4>();
+    case 5: return wait_loads<5>();
+    case 6: return wait_loads<6>();
+    case 7: return wait_loads<7>();
+    case 8: return wait_loads<8>();
+    case 9: return wait_loads<9>();
+    case 10: return wait_loads<10>();
+    case 11: return wait_loads<11>();
+    case 12: return wait_loads<12>();
+    case 13: case 14: return wait_loads<13>();
+    case 15: case 16: case 17: return wait_loads<15>();
+    default: return wait_loads<18>();
   }
 }
 
@@ -159,14 +152,14 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
   const bool up = GATED && wave >= CT;
   const int wn = min(n0 + (up ? wr - CT * 8 : wr), p.N - 1);
   const uint32_t wlds = (uint32_t)wave * 1024u;
-  const uint32_t woff = (uint32_t)(wn - min(n0, p.N - 1)) * (uint32_t)p.K * 2u + (uint32_t)((lslot ^ gs_swz(wr)) * 16);
+  const uint32_t woff = (uint32_t)(wn - min(n0, p.N - 1)) * (uint32_t)p.K * 2u + (uint32_t)((lslot ^ ring_swz(wr)) * 16);
   const unsigned char* wbase = (const unsigned char*)((up ? p.W2 : p.W) + (size_t)min(n0, p.N - 1) * p.K) + (size_t)b_first * GS_ROW_BYTES;
   const unsigned char* abase = (const unsigned char*)p.A + (size_t)b_first * GS_ROW_BYTES;
   uint32_t aoff[AL];
 #pragma unroll
   for (int c = 0; c < AL; ++c) {
     const int r = (wave + c * NW) * 8 + lrow;
-    aoff[c] = (uint32_t)min(r, p.M - 1) * (uint32_t)p.lda * 2u + (uint32_t)((lslot ^ gs_swz(r)) * 16);
+    aoff[c] = (uint32_t)min(r, p.M - 1) * (uint32_t)p.lda * 2u + (uint32_t)((lslot ^ ring_swz(r)) * 16);
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
   auto issue = [&](int i, int slot) {
@@ -174,21 +167,16 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
     int b = i + rot;
     if (b >= total) b -= total;
     const size_t kbytes = (size_t)b * GS_ROW_BYTES;
-    // m0 holds the LDS address of the 1 KB, lane l's 16 bytes land at m0 + 16 l
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(woff), "s"(wbase + kbytes), "s"(at + wlds) : "memory", "m0");
+    load_to_lds_16(wbase + kbytes, woff, at + wlds);
 #pragma unroll
     for (int c = 0; c < AL; ++c)
-      if (wave + c * NW < na)
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                     :
-                     : "v"(aoff[c]), "s"(abase + kbytes), "s"(at + (uint32_t)(2 * CT + wave + c * NW) * 1024u)
-                     : "memory", "m0");
+      if (wave + c * NW < na) load_to_lds_16(abase + kbytes, aoff[c], at + (uint32_t)(2 * CT + wave + c * NW) * 1024u);
   };
 #pragma unroll
   for (int i = 0; i < S - 1; ++i)
     if (i < total) issue(i, i);
   // ---- fragments: lane l reads row l % 16, 8 of k at kg * 32 + (l / 16) * 8: piece 4 kg + l / 16
-  const int foff = col * GS_ROW_BYTES + (((4 * kg + g) ^ gs_swz(col)) << 4);  // + 16 rows leave gs_swz unchanged
+  const int foff = col * GS_ROW_BYTES + (((4 * kg + g) ^ ring_swz(col)) << 4);  // + 16 rows leave ring_swz unchanged
   floatx4 acc[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -215,7 +203,7 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
   // loop they made products with such a tile slower than full ones (6,144 x 4,096 at 400 rows 49.2 us, at 512 45.0; now 42.3)
   gs_with_loads<1 + AL>(nl, [&](auto loads) {
     for (; i + S - 2 < total; ++i) {
-      gs_wait_loads<decltype(loads)::n * (S - 2)>();
+      wait_loads<decltype(loads)::n * (S - 2)>();
       block();
     }
   });
