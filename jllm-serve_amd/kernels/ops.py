@@ -852,32 +852,33 @@ _step_scratch = threading.local()  # what a step's products share, see `step_scr
 
 @contextlib.contextmanager
 def step_scratch(rows: int, device):
-    """Around the launches of one step of ``rows`` rows: the products of few rows with K cut, which follow each other in their
-    stream, take turns in one set of zeroed counters (each leaves them zero), made and cleared for the first of them; a step
-    without any launches nothing for it. Outside, every such product clears counters of its own."""
+    """Around the launches of one step of ``rows`` rows (all of them inside a capture, or none): the products of few rows with K
+    cut that follow each other in the stream of the first of them take turns in one set of zeroed counters (each leaves them
+    zero), made and cleared for that first one; a step without any launches nothing for it. Outside, and in other streams, every
+    such product clears counters of its own."""
     if not SKINNY_MAX_ROWS < rows <= WIDE_MOST_ROWS:
         yield
         return
-    before = getattr(_step_scratch, "counters", None)
-    _step_scratch.counters = {}  # (device, stream, whether it is captured) -> counters
+    before = getattr(_step_scratch, "shared", None)
+    _step_scratch.shared = []  # [counters, the stream they are used in] from the first product on
     try:
         yield
     finally:
-        _step_scratch.counters = before
+        _step_scratch.shared = before
 
 
 STREAM_COUNTERS = 1024
 
 
 def _arrival_counters(tiles: int, device) -> torch.Tensor:
-    shared = getattr(_step_scratch, "counters", None)
+    shared = getattr(_step_scratch, "shared", None)
     if shared is None or tiles > STREAM_COUNTERS:
         return torch.empty(tiles, dtype=torch.int32, device=device).zero_()
-    # memory that a capture has recorded the clearing of is not clear for launches beside it, nor the other way round
-    key = (device, _stream(), torch.cuda.is_current_stream_capturing())
-    if key not in shared:
-        shared[key] = torch.empty(STREAM_COUNTERS, dtype=torch.int32, device=device).zero_()
-    return shared[key]
+    if not shared:
+        shared += [torch.empty(STREAM_COUNTERS, dtype=torch.int32, device=device).zero_(), _stream()]
+    elif shared[1] != _stream() or shared[0].device != device:
+        return torch.empty(tiles, dtype=torch.int32, device=device).zero_()
+    return shared[0]
 
 
 def _stream_scratch(M: int, N: int, K: int, gated: bool, a: torch.Tensor, adds: int):

@@ -132,6 +132,7 @@ class GqaAttention(Part):
             del parts
             if s.bias:
                 self.b_qkv = torch.cat([get(self._name(n, ".bias")).to(torch.float32) for n in "qkv"]).contiguous()
+        self.normed_rows_product = (self.w_qkv.shape[0], False)
         self.w_o = get(self._name("o"))
         if s.out_bias:
             self.b_o = get(self._name("o", ".bias"))
@@ -143,9 +144,6 @@ class GqaAttention(Part):
 
     def cache_spec(self):
         return KvSpec(self.spec.kv_heads, self.spec.head_dim, self.spec.window)
-
-    def normed_rows_product(self):
-        return self.w_qkv.shape[0], False
 
     def step_planners(self):
         return [self.planner]

@@ -6,8 +6,8 @@ xb = norm_post(x); x += ffn(xb). The residual stream x is fp32 and is never norm
 Norms between two products need no launch of their own when both sides agree (optional, by attributes of the
 parts; a part that knows nothing of this works as before):
 * a mixer / feed-forward with ``takes_normed_rows = True`` only feeds its input to ``ops.gemm`` and so may get the
-  norm as a promise (``norm.defer`` / ``ops.NormedRows``) instead of a tensor; ``normed_rows_product()``, where it has one,
-  says what product that is, as (outputs, whether gated);
+  norm as a promise (``norm.defer`` / ``ops.NormedRows``) instead of a tensor; ``normed_rows_product``, where it has one,
+  says what product that is, as (outputs, whether gated), once its weights are loaded;
 * one with ``prepares_next_norm = True`` takes ``then_norm=<norm part>`` in ``forward``, ends with
   ``then_norm.after_add(...)`` instead of the add into the residual, and returns that promise. It is asked only for a
   norm whose reader takes promises (``norm.reader``, set here).

@@ -20,6 +20,7 @@ class GatedMlp(Part):
         self.gate = ops.GATE_FUNCTIONS[spec.activation]
         self.limit = float(getattr(spec, "limit", 0.0))
         self.hidden = spec.hidden
+        self.normed_rows_product = (self.hidden, True)
         self.names = spec.names
         self.dim = build.hidden
         self.prefix = prefix
@@ -44,9 +45,6 @@ class GatedMlp(Part):
             self.w_gate = get(self._name("gate"))
             self.w_up = get(self._name("up"))
         self.w_down = get(self._name("down"))
-
-    def normed_rows_product(self):
-        return self.hidden, True
 
     def forward(self, xb, residual, step, then_norm=None):
         h = ops.gemm(xb, self.w_gate, w2=self.w_up, epilogue=ops.EPI_GATED, out_dtype=self.build.dtype,

@@ -124,6 +124,7 @@ class LatentAttention(Part):
             stack.append(get(self._name("gate")))
         dt = stack[0].dtype if all(t.dtype == stack[0].dtype for t in stack) else torch.float32
         self.w_in = torch.cat([t.to(dt) for t in stack], dim=0).contiguous()  # [dq | dkv | g] rows
+        self.normed_rows_product = (self.w_in.shape[0], False)
         del stack
         self.g_q = get(self._name("dq_norm")) if s.q_rank > 0 else None
         if self.g_kv is not None and self.g_q is not None and self.g_kv.dtype != self.g_q.dtype:
@@ -139,9 +140,6 @@ class LatentAttention(Part):
     def cache_spec(self):
         # one row per position: [latent | rotated key part]; the pages honour the widest window that reads them
         return PageSpec((CacheRow("ckr", (self.kv_width,), 0),), self.spec.keep)
-
-    def normed_rows_product(self):
-        return self.w_in.shape[0], False
 
     def step_planners(self):
         return [LatentStepPlanner()]

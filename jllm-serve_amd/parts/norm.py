@@ -49,9 +49,8 @@ class RMSNorm(Part):
     def after_add(self, a, w, residual, bias=None, exact=False):
         """residual += a @ w.T (+ bias), and this norm of the result as a promise: the product that makes the new
         residual rows can prepare their norm on its way out (``ops.gemm_add_then_norm``)."""
-        reads = getattr(self.reader, "normed_rows_product", None)
         return ops.gemm_add_then_norm(a, w, residual, self.gain, self.eps, self.out_dtype, bias=bias, exact=exact,
-                                      reader=reads() if reads is not None else None)
+                                      reader=getattr(self.reader, "normed_rows_product", None))
 
     def join(self, residual, branches, scales=(1.0, 1.0), branch_gains=None, branch_eps=0.0, then=None):
         """``residual += this norm of a sublayer's output`` in one launch. ``branches``: the output, or two branches'

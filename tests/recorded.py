@@ -21,7 +21,6 @@ def record(monkeypatch):
     monkeypatch.setattr(ops, "_call", lambda name, *args: seen.append((name, args)))
     monkeypatch.setattr(ops, "_dev", lambda *tensors: None)
     monkeypatch.setattr(ops, "_stream", lambda: 0)
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     monkeypatch.setattr(ops, "_ptr", lambda t: t)
     return seen
 
