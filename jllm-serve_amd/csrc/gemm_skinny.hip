@@ -12,9 +12,9 @@
 // each of 16 rows, and a compute unit's load pipe then passes 25 bytes a clock (6.6 TB/s of the whole chip with everything in
 // L2, against 10 for 8 rows of 128 bytes), which the activations, once per workgroup and as many as the weights at 16 rows,
 // had to share. In LDS the activations of up to 8 rows cost half as much, and K blocks of 64 keep the waves even.
-// Inside a graph, before / now, in us at 1, 8 and 16 rows: 8B shape qkv 14.0 15.7 16.0 / 12.4 13.0 13.4, o 8.7 9.8 11.3 / 8.6
-// 9.0 9.6, gate/up 39.6 41.9 45.7 / 37.6 39.0 39.5, down 21.0 25.0 30.4 / 19.9 20.6 22.5; 32B down 51.2 58.6 68.4 / 47.3 48.8
-// 50.8; 0.6B o 4.7 5.8 6.4 / 4.1 4.5 4.8, down 7.4 9.0 10.4 / 5.0 5.6 6.3.
+// Inside a graph, before / now, in us at 1, 8 and 16 rows: 8B shape qkv 13.9 15.6 16.1 / 11.6 12.9 13.1, o 8.7 9.8 11.3 / 8.3
+// 8.7 9.4, gate/up 40.1 41.4 45.6 / 37.2 38.4 39.1, down 20.9 25.2 30.6 / 20.2 21.0 23.1; 32B down 52.3 61.5 71.5 / 48.8 50.1
+// 52.9; 0.6B o 4.7 5.7 6.4 / 4.0 4.4 4.7, down 7.4 9.1 10.4 / 4.8 5.4 5.9; 1.7B qkv 6.0 7.2 7.6 / 6.0 6.8 7.1.
 // What a large copy reaches (6.2 TB/s) would take 8.1, 5.4, 32.5 and 16.2 us of the 8B shape's four: what is left is the
 // launch, the first bytes' latency and the sum over the waves, about 4 us each. Measured and not taken: three blocks in
 // flight instead of up to six (8B gate/up at one row 37.9 -> 38.2), a contiguous range of K per wave (42.2).

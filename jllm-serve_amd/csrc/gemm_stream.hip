@@ -11,14 +11,15 @@
 // for such loads). So a workgroup should own about as many weight rows as there are activation rows, or more, and where
 // that leaves compute units without one, K is cut over gridDim.y. Each part leaves its sums, with accesses that pass the
 // caches by (common.h), and the workgroup of a column tile that arrives last adds the parts in ascending order and applies
-// bias and epilogue: no second launch. How N and K are cut depends on N and K only, never on M: a row's result does
-// not depend on the rows beside it.
+// bias and epilogue: no second launch. Up to 64 rows, how N and K are cut depends on N and K only, never on M: a row's result
+// does not depend on the rows beside it. Beyond, tiles and parts follow M, and with them the order of a row's sums and of the
+// squares that a norm adds up.
 //
 // Inside a graph, us at 20, 32 and 64 rows, before (fragments of the weights straight from memory a step ahead, 128 rows per
-// workgroup, the parts added by a second launch) / now: 8B shape qkv 19.5 19.9 22.6 / 15.6 16.1 19.6, o 13.6 14.1 16.8 /
-// 12.8 13.5 16.7, gate/up 51.3 53.6 58.1 / 42.8 42.6 43.9, down 28.1 29.1 32.7 / 24.1 24.8 29.1; 0.6B shape qkv 11.4 11.7 13.4 /
-// 7.7 8.0 9.8, o 10.3 10.4 11.7 / 7.6 7.9 9.9, gate/up 17.8 18.1 19.8 / 7.8 7.9 11.2, down 11.0 11.4 12.8 / 8.7 8.9 11.4; a step
-// of 64 requests of the 8B shape 6.47 -> 5.49 ms. A large copy's rate (6.2 TB/s) would take 8.1, 5.4, 32.5 and 16.2 us of the
+// workgroup, the parts added by a second launch) / now: 8B shape qkv 19.4 20.0 22.6 / 16.7 17.3 20.8, o 13.5 14.1 16.7 /
+// 12.4 13.1 16.3, gate/up 51.8 53.7 58.6 / 41.9 41.7 43.1, down 28.2 29.1 32.7 / 24.4 25.2 30.3; 0.6B shape qkv 11.6 11.7 13.5 /
+// 6.7 6.9 8.4, o 10.2 10.4 11.7 / 7.1 7.4 9.2, gate/up 17.8 18.1 19.8 / 7.5 8.2 9.3, down 11.2 11.4 12.9 / 8.4 8.6 10.7; a step
+// of 64 requests of the 8B shape 6.47 -> 5.42 ms. A large copy's rate (6.2 TB/s) would take 8.1, 5.4, 32.5 and 16.2 us of the
 // 8B shape's four; the rest is the launch and the first bytes (4), the parts' way through memory (3, 4 and more at 64 rows) and
 // at 64 rows the load pipe.
 //

@@ -903,7 +903,11 @@ def _plan_of_rows(M: int, N: int, K: int, gated: bool, adds: int) -> Tuple[int, 
 
 # Estimated times of that kernel for more than 64 rows, in microseconds
 WIDE_MOST_ROWS = 1024
-WIDE_ADD_COLUMNS = 2048           # with the add into the residual (and the rows for a norm) the estimate holds up to here
+# Into the residual: up to here. The estimates count the norm behind such a product as a launch that only this kernel saves,
+# but the tiled kernels' reduction makes it too where they cut K, as they do for wider rows. o and gate/up in turn without this
+# limit, us: 4B at 128 rows 58.2 -> 55.3, 8B at 832 239.6 -> 228.7; down and qkv: 4B at 160 rows 55.7 -> 58.1, 14B at 192
+# 128.3 -> 131.0. Taking the credit away instead made the narrow ones slower (0.6B down and qkv at 160 rows 21.9 -> 24.8).
+WIDE_ADD_COLUMNS = 2048
 WIDE_LEAST_K = 1024               # the shortest K it was measured at
 WIDE_BLOCK_US = (0.275, 0.0198)   # 64 of k on 32 weight and 64 activation rows, and per 8 rows more of either
 WIDE_FIXED_US = {64: 4.8, 128: 7.2}   # the launch, the first blocks and the end, by activation rows per workgroup
@@ -964,9 +968,11 @@ def _wide_plan(M: int, N: int, K: int, gated: bool, adds: int = 0) -> Optional[T
     launch of its own (`ADDS_AND_NORM`, see `_norm_rides`). Here tiles of 64 or 128 rows by 32 to 128 fill the chip with K whole.
 
     The constants were fitted to a sweep of every choice for the products of the 0.6B, 1.7B, 4B and 8B shapes at 100, 200, 320, 487 and
-    631 rows against what the tiled kernels take. us, tiled / here: 0.6B shape at 487 rows qkv 22.2 / 13.3, o 17.6 / 13.5,
-    gate/up 18.8 / 16.9, down 17.6 / 17.2 (and the norm behind o and down, 4.0, costs no launch of its own); 4B qkv at 631 rows
-    41.6 / 34.5, 8B qkv at 320 39.2 / 35.4. Beyond, the tiled kernels win: 8B gate/up at 200 rows 79.9 / 101, down 44.8 / 54.9."""
+    631 rows against what the tiled kernels take, when a last tile of few rows still made a launch slower than a full one; of the
+    480 choices between 65 and 1,024 rows of nine shapes one is now behind the tiled kernels (gated 8,960 x 1,536 at 128 rows,
+    25.9 / 26.6). us, tiled / here: 0.6B shape at 487 rows qkv 22.4 / 12.6, o 18.3 / 10.6, gate/up 18.7 / 15.7 (and the norm
+    behind o, 4.0, costs no launch of its own); 4B qkv at 640 rows 41.5 / 33.8, 8B qkv at 320 39.4 / 34.1. Beyond, the tiled
+    kernels win: 8B gate/up at 200 rows 79.9 / 101, down 44.8 / 54.9."""
     if not STREAM_MAX_ROWS < M <= WIDE_MOST_ROWS or K % 128 or N % 16 or K < WIDE_LEAST_K or (adds and N > WIDE_ADD_COLUMNS):
         return None
     rows, cut = _tiled_plan(M, N, K, gated)
