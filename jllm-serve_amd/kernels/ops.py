@@ -383,15 +383,18 @@ class NormedRows:
 
 
 def _skinny_norm(a, w, w2, bias, out, epilogue, emit=None, normed: Optional[NormedRows] = None,
-                 gate_limit: float = 0.0) -> bool:
-    """The weight-streaming products (up to 16 rows, up to 64 rows) with a norm on either side; False when the kernel
-    does not take the case."""
+                 gate_limit: float = 0.0, plan: Optional[Tuple[int, int, int]] = None) -> bool:
+    """The weight-streaming products (up to 16 rows, up to 64 rows, some of up to 1,024) with a norm on either side; False when
+    the kernel does not take the case. ``plan``: what `_row_plan` says, where the caller has asked."""
     M, K = a.shape
     N = w.shape[0]
-    e_rows, e_gain, e_part = emit if emit is not None else (None, None, None)
-    adds = _adds(epilogue, emit is not None)
-    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or (M > STREAM_MAX_ROWS and _wide_plan(M, N, K, w2 is not None, adds) is None):
+    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         return False
+    if plan is None:
+        plan = _row_plan(M, N, K, w2 is not None, _adds(epilogue))
+        if plan is None:
+            return False
+    e_rows, e_gain, e_part = emit if emit is not None else (None, None, None)
     n_part = normed.partials if normed is not None else None
     head = (_ptr(a), a.stride(0), _ptr(w), _ptr(w2), _ptr(bias), _code(bias.dtype) if bias is not None else F32,
             _ptr(out), _code(out.dtype), out.stride(0), M, N, K, int(epilogue), float(gate_limit))
@@ -399,30 +402,32 @@ def _skinny_norm(a, w, w2, bias, out, epilogue, emit=None, normed: Optional[Norm
     takes = (_ptr(n_part), n_part.shape[1] if n_part is not None else 0, normed.eps if normed is not None else 0.0, _stream())
     emit_parts = e_part.shape[1] if e_part is not None else 0
     if M <= SKINNY_MAX_ROWS:
-        return _try("jllm_gemm_skinny_norm_bf16", *head, _skinny_rows(N, K, w2 is not None), *emits, emit_parts, *takes)
+        return _try("jllm_gemm_skinny_norm_bf16", *head, plan[0], *emits, emit_parts, *takes)
     if K % 128:
         return False
-    rows, tile, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a, adds)
-    return _try("jllm_gemm_stream_bf16", *head, rows, tile, parts, _ptr(sums), _ptr(arrivals), _ptr(e_rows), e_rows.stride(0) if e_rows is not None else 0, *emits[1:],
+    sums, arrivals = _stream_scratch(M, N, w2 is not None, a, plan)
+    return _try("jllm_gemm_stream_bf16", *head, *plan, _ptr(sums), _ptr(arrivals), _ptr(e_rows), e_rows.stride(0) if e_rows is not None else 0, *emits[1:],
                 emit_parts, *takes)
 
 
 ADDS, ADDS_AND_NORM = 1, 2  # `adds` of a plan: into the residual, and with the rows for the norm behind it
 
 
-def _adds(epilogue: int, emits: bool = False) -> int:
-    return 0 if epilogue != EPI_ADD else ADDS_AND_NORM if emits else ADDS
+def _adds(epilogue: int) -> int:
+    return ADDS if epilogue == EPI_ADD else 0
 
 
-def _norm_rides(M: int, N: int, K: int, reader: Optional[Tuple[int, bool]]) -> bool:
-    """Whether the adding product of M rows, N outputs and K inputs prepares the norm that follows. For more than 64 rows it
-    does so where the same kernel takes both it and the product that reads the norm (``reader``: its outputs and whether it is
-    gated; not known: plain, with N outputs), from the row count on at which the rows may be laid out for many rows
-    (`activation_rows`). A norm that is prepared for a reader which does not take it is made again by a launch of its own."""
-    if M <= STREAM_MAX_ROWS:
-        return True
-    outputs, gated = reader if reader is not None else (N, False)
-    return M >= PAD_ROWS_FROM and _wide_plan(M, outputs, N, gated, 0) is not None and _wide_plan(M, N, K, False, ADDS_AND_NORM) is not None
+def _ride_plan(M: int, N: int, K: int, reader: Optional[Tuple[int, bool]]) -> Optional[Tuple[int, int, int]]:
+    """The plan (`_row_plan`) of an adding product of M rows, N outputs and K inputs that prepares the norm that follows, or
+    None where it does not. For more than 64 rows it does so where the same kernel takes both it and the product that reads
+    the norm (``reader``: its outputs and whether it is gated; not known: plain, with N outputs), from the row count on at
+    which the rows may be laid out for many rows (`activation_rows`). A norm that is prepared for a reader which does not
+    take it is made again by a launch of its own."""
+    if M > STREAM_MAX_ROWS:
+        outputs, gated = reader if reader is not None else (N, False)
+        if M < PAD_ROWS_FROM or _wide_plan(M, outputs, N, gated, 0) is None:
+            return None
+    return _row_plan(M, N, K, False, ADDS_AND_NORM)
 
 
 def gemm_add_then_norm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gain: torch.Tensor, eps: float,
@@ -439,11 +444,13 @@ def gemm_add_then_norm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gain
         and gain.numel() == w.shape[0] and gain.is_contiguous() and (bias is None or (bias.numel() == w.shape[0] and bias.is_contiguous()))
     if fits:
         _dev(a, w, bias, out, gain)
-    if fits and _norm_rides(*out.shape, a.shape[1], reader):
+    plan = _ride_plan(*out.shape, a.shape[1], reader) if fits else None
+    if plan is not None:
         M, N = out.shape
         scaled = activation_rows(M, N, torch.bfloat16, out.device)
-        partials = torch.empty((M, _norm_partials(M, N, a.shape[1])), dtype=torch.float32, device=out.device)
-        if _skinny_norm(a, w, None, bias, out, EPI_ADD, emit=(scaled, gain, partials)):
+        # a sum of squares per row and workgroup's columns, in whole fours
+        partials = torch.empty((M, -(-N // (4 * plan[0])) * 4), dtype=torch.float32, device=out.device)
+        if _skinny_norm(a, w, None, bias, out, EPI_ADD, emit=(scaled, gain, partials), plan=plan):
             return NormedRows(out, gain, eps, norm_dtype, scaled, partials)
     promise = NormedRows(out, gain, eps, norm_dtype)
     if fits and _cut_takes_norm(*out.shape, a.shape[1]) and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and a.stride(0) % 8 == 0 \
@@ -781,18 +788,6 @@ def _skinny_rows(N: int, K: int, gated: bool) -> int:
     return 32 if K < SKINNY_HEAD_ROWS_K else 16
 
 
-def _norm_partials(M: int, N: int, K: int) -> int:
-    """Partial sums of squares per row that a product with N outputs leaves for the norm behind it: room for one per
-    workgroup's columns, in whole fours."""
-    if M > STREAM_MAX_ROWS:
-        groups = -(-N // _wide_plan(M, N, K, False, ADDS_AND_NORM)[0])
-    elif M > SKINNY_MAX_ROWS:
-        groups = -(-N // _stream_plan(N, K, False)[0])
-    else:
-        groups = -(-N // _skinny_rows(N, K, False))
-    return -(-groups // 4) * 4
-
-
 # Estimated times of the second weight-streaming kernel for 17 to 64 rows, in ns (priced at 40 rows)
 STREAM_MIN_BLOCKS = 4             # 128-wide K blocks a part has at least
 STREAM_MOST_PARTS = 32
@@ -881,22 +876,23 @@ def _arrival_counters(tiles: int, device) -> torch.Tensor:
     return shared[0]
 
 
-def _stream_scratch(M: int, N: int, K: int, gated: bool, a: torch.Tensor, adds: int):
-    """The plan and scratch of the kernel behind `_stream_plan` and `_wide_plan`: (weight rows, activation rows, parts, sums,
-    counters)."""
-    rows, tile, parts = _plan_of_rows(M, N, K, gated, adds)
+def _stream_scratch(M: int, N: int, gated: bool, a: torch.Tensor, plan: Tuple[int, int, int]):
+    """What the kernel behind `_stream_plan` and `_wide_plan` needs for parts of K: (sums, counters)."""
+    rows, tile, parts = plan
     if parts == 1:
-        return rows, tile, 1, None, None
-    row_tiles = -(-M // tile)
-    tiles = -(-N // (rows // 2 if gated else rows)) * row_tiles
+        return None, None
+    tiles = -(-N // (rows // 2 if gated else rows)) * -(-M // tile)
     partial = torch.empty((parts * tiles * rows * (tile if M > STREAM_MAX_ROWS else max(32, 16 * -(-M // 16))),), dtype=torch.float32, device=a.device)
-    return rows, tile, parts, partial, _arrival_counters(tiles, a.device)
+    return partial, _arrival_counters(tiles, a.device)
 
 
-def _plan_of_rows(M: int, N: int, K: int, gated: bool, adds: int) -> Tuple[int, int, int]:
-    """(weight rows, activation rows, parts of K) of the second weight-streaming kernel for a product that it takes."""
+def _row_plan(M: int, N: int, K: int, gated: bool, adds: int) -> Optional[Tuple[int, int, int]]:
+    """(weight rows, activation rows, parts of K) per workgroup of the weight-streaming kernel for M rows, or None where the
+    tiled kernels take more than 64."""
     if M > STREAM_MAX_ROWS:
         return _wide_plan(M, N, K, gated, adds)
+    if M <= SKINNY_MAX_ROWS:
+        return _skinny_rows(N, K, gated), 0, 1
     rows, parts = _stream_plan(N, K, gated)
     return rows, 64, parts
 
@@ -965,7 +961,7 @@ def _wide_plan(M: int, N: int, K: int, gated: bool, adds: int = 0) -> Optional[T
     64 rows, or None where the tiled kernels are estimated to be faster: they move fewer bytes per multiply through a compute
     unit, but their tiles of 128 x 128 and larger leave compute units without work where a product is small, and cutting K
     costs them a second launch. ``adds``: into the residual (`ADDS`), or there with the norm behind it prepared, which is then no
-    launch of its own (`ADDS_AND_NORM`, see `_norm_rides`). Here tiles of 64 or 128 rows by 32 to 128 fill the chip with K whole.
+    launch of its own (`ADDS_AND_NORM`, see `_ride_plan`). Here tiles of 64 or 128 rows by 32 to 128 fill the chip with K whole.
 
     The constants were fitted to a sweep of every choice for the products of the 0.6B, 1.7B, 4B and 8B shapes at 100, 200, 320, 487 and
     631 rows against what the tiled kernels take, when a last tile of few rows still made a launch slower than a full one; of the
@@ -1007,12 +1003,13 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0, norm=_NO_
     N = w.shape[0]
     head = (_ptr(a), a.stride(0), _ptr(w), _ptr(w2), _ptr(bias), _code(bias.dtype) if bias is not None else F32,
             _ptr(out), _code(out.dtype), out.stride(0), M, N, K, int(epilogue), float(gate_limit))
+    plan = _row_plan(M, N, K, w2 is not None, _adds(epilogue))
     if M <= SKINNY_MAX_ROWS:
-        if _try("jllm_gemm_skinny_bf16", *head, _skinny_rows(N, K, w2 is not None), _stream()):
+        if _try("jllm_gemm_skinny_bf16", *head, plan[0], _stream()):
             return True
-    elif K % 128 == 0 and (M <= STREAM_MAX_ROWS or _wide_plan(M, N, K, w2 is not None, _adds(epilogue)) is not None):
-        rows, tile, parts, sums, arrivals = _stream_scratch(M, N, K, w2 is not None, a, _adds(epilogue))
-        if _try("jllm_gemm_stream_bf16", *head, rows, tile, parts, _ptr(sums), _ptr(arrivals), None, 0, None, F32, None, 0, None, 0, 0.0, _stream()):
+    elif plan is not None and K % 128 == 0:
+        sums, arrivals = _stream_scratch(M, N, w2 is not None, a, plan)
+        if _try("jllm_gemm_stream_bf16", *head, *plan, _ptr(sums), _ptr(arrivals), None, 0, None, F32, None, 0, None, 0, 0.0, _stream()):
             return True
     tile_rows, cut = _tiled_plan(M, N, K, w2 is not None)
     if tile_rows:
