@@ -1,7 +1,7 @@
 // out[M,N] = A[M,K] * W[N,K]^T for many rows, bf16 on the matrix cores (v_mfma_f32_16x16x32_bf16), built so that the
 // matrix cores of a compute unit never wait for operands:
 //
-//  * A workgroup of 8 waves (2 x 4) owns a 256 x 256 output tile (a wave 128 x 64: 8 by 4 accumulators of 16 x 16). K
+//  * A workgroup of 8 waves (2 x 4; 1 x 8 for the wide tiles further down) owns a 256 x 256 output tile (a wave 128 x 64: 8 by 4 accumulators of 16 x 16). K
 //    advances in stages of 32 through a ring of NS stages in LDS. (The 16 x 16 x 32 form rather than 32 x 32 x 16: the
 //    full chip is bound by its power, and a multiply-add of the smaller form reads and writes half as many accumulator
 //    bytes. MFMAs alone on random operands run at 2.04 PFLOP/s against 1.85; this kernel with either form: 2,048 rows of
@@ -38,7 +38,6 @@
 #define PP_BK 32
 #define PP_ROW_BYTES (PP_BK * 2)  // a tile row in LDS: 64 bytes = 4 pieces of 16
 #define PP_WAVES 8
-#define PP_MUL 3  // multiplies between two LDS reads of the multiply phase
 
 // The piece of row r that lies in slot s is s ^ pp_swz(r): 16 lanes that read the same piece of 16 consecutive rows,
 // and 8 lanes of 8 rows, then cover every bank once, whichever of the two the LDS takes per pass. (With fragments of 32 rows
@@ -48,19 +47,20 @@ __device__ __forceinline__ int pp_swz(int r) { return (((r >> 1) ^ (r >> 3)) & 1
 #define PP_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
 #define PP_LGKMCNT0() __builtin_amdgcn_s_waitcnt((15) | (3 << 14) | (7 << 4) | (0 << 8))
 
-template <bool GATED, int FM, int NS>
-__global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
+// WGM x 8 / WGM waves of 32 FM rows by 64 columns each: the tile whose first row and first output are m0 and n0
+template <bool GATED, int FM, int NS, int WGM>
+__device__ __forceinline__ void pingpong_tile(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
     const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N, int K,
-    int epilogue, GateSpec gs, float* __restrict__ partial) {
-  constexpr int WGM = 2, WGN = 4, RM = 2 * FM, CN = 4;  // a wave's blocks of 16 rows and of 16 columns
+    int epilogue, GateSpec gs, float* __restrict__ partial, int m0, int n0) {
+  constexpr int WGN = PP_WAVES / WGM, RM = 2 * FM, CN = 4;  // a wave's blocks of 16 rows and of 16 columns
   constexpr int TBM = WGM * RM * 16, TBN = WGN * CN * 16;
   constexpr int STAGE = (TBM + TBN) * PP_ROW_BYTES;
   // load instructions (16 rows each) per wave and stage. Tiles of 192 rows are twelve chunks of A: two for each wave of the
   // first group, one for each of the second's.
   constexpr int LA = (TBM / 16 + PP_WAVES - 1) / PP_WAVES, LB = TBN / 16 / PP_WAVES, LA1 = TBM / 16 * 2 / PP_WAVES - LA;
   constexpr int L0 = LA + LB, L1 = LA1 + LB;
-  static_assert(LA1 >= 1 && LB >= 1 && (LA + LA1) * PP_WAVES / 2 == TBM / 16, "every wave loads rows of both operands");
+  static_assert(LA1 >= 0 && LB >= 1 && (LA + LA1) * PP_WAVES / 2 == TBM / 16, "every wave loads rows of both operands");
   extern __shared__ __align__(1024) unsigned char smem[];
   const int tid = threadIdx.x;
   // the wave's number is the same in all its lanes: said so, its group, its part of the tile and the places in LDS it
@@ -68,8 +68,6 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int group = wave >> 2;  // waves 0..3 and 4..7: one of each on every SIMD
   const int wm = wave / WGN, wn = wave % WGN;
-  const int m0 = blockIdx.y * TBM;
-  const int n0 = blockIdx.x * (GATED ? TBN / 2 : TBN);
   const int nk_all = K / PP_BK;
   const int nk_per = (nk_all + gridDim.z - 1) / gridDim.z;
   const int kt0 = blockIdx.z * nk_per;
@@ -146,6 +144,7 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
   // second half of the rows' (read in the memory phase); the loop is unrolled by two so that a stage's and the next
   // one's swap names instead of being copied
   constexpr int RH = RM / 2;
+  constexpr int PP_MUL = RM > 4 ? 3 : 2;  // multiplies between two LDS reads of the multiply phase
   u32x4 a0[RH], b0[CN], a1[RH], an[RH], bn[CN];
   auto read_rows = [&](int t, int half, u32x4 (&af)[RH]) {
     const unsigned char* st = smem + (t % NS) * STAGE + aoff + half * RH * 16 * PP_ROW_BYTES;
@@ -227,6 +226,38 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
                                          (int)blockIdx.z, (int)gridDim.z);
 }
 
+template <bool GATED, int FM, int NS>
+__global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
+    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
+    const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N, int K,
+    int epilogue, GateSpec gs, float* __restrict__ partial) {
+  pingpong_tile<GATED, FM, NS, 2>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial,
+                                  blockIdx.y * 64 * FM, blockIdx.x * (GATED ? 128 : 256));
+}
+
+// Tiles of 256 x 256 and, for the last rows where those are at most 128, of 128 x 512 (64 x 512 where they are at most 64): `wide`
+// of the latter, which come first because they take longer, then rows of `cols` of the former. A tile of 256 rows of which a few
+// are there takes as long as a full one, and so does the round of workgroups that it begins. A wide tile takes half as many
+// workgroups; its stage moves a quarter (an eighth) more bytes into LDS and takes 1.25 (1.17) times as long. us, what was chosen
+// among whole tiles / this: gate/up of the 8B shape at 560 rows (288 tiles / 240) 167 / 122, at 631 171 / 131, of the 14B shape at 300 223 / 153,
+// at 1,320 522 / 457, at 4,614 (10.1 rounds / 9.8) 1,558 / 1,498, of the 32B shape at 600 412 / 345; 14B down at 3,111 620 / 501, 4B
+// qkv at 2,600 106 / 75. Last rows of 129 to 192 in a tile of either kind gained nothing (8B gate/up at 700 rows 169 / 196).
+template <bool GATED, int NS>
+__global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_mixed_kernel(
+    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
+    const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N, int K,
+    int epilogue, GateSpec gs, float* __restrict__ partial, int wide, int cols) {
+  const int whole = M >> 8 << 8, b = blockIdx.x;
+  if (b >= wide) {
+    const int row = (b - wide) / cols, col = b - wide - row * cols;
+    pingpong_tile<GATED, 4, NS, 2>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, row * 256, col * (GATED ? 128 : 256));
+  } else if (M - whole > 64) {
+    pingpong_tile<GATED, 4, NS, 1>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, whole, b * (GATED ? 256 : 512));
+  } else {
+    pingpong_tile<GATED, 2, NS, 1>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, whole, b * (GATED ? 256 : 512));
+  }
+}
+
 template <int FM, int NS>
 static int launch_pingpong(const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype,
                            void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue, GateSpec gs, int splits,
@@ -252,8 +283,34 @@ static int launch_pingpong(const void* A, int lda, const void* W, const void* W2
   return 0;
 }
 
-// `tile_rows`: 256 or 192 (rows of the output tile; 256 columns, 128 outputs with the gated epilogue).
-// `splits` > 1 cuts K over gridDim.z (not with the gated epilogue): `partial` then holds splits * M * N floats, summed
+static int launch_mixed(const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype,
+                        void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue, GateSpec gs, int splits,
+                        float* partial, hipStream_t stream) {
+  constexpr int NS = 4;
+  const int cols = (N + (W2 ? 127 : 255)) / (W2 ? 128 : 256), wide = (cols + 1) / 2;
+  const long groups = (long)(M / 256) * cols + wide;
+  if (groups > 0x7fffffffl) return 1;
+  constexpr size_t smem = (size_t)NS * (128 + 512) * PP_ROW_BYTES;  // of the wider stage
+  static bool configured = false;
+  if (!configured) {
+    hipError_t e1 = hipFuncSetAttribute((const void*)gemm_pingpong_mixed_kernel<true, NS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    hipError_t e2 = hipFuncSetAttribute((const void*)gemm_pingpong_mixed_kernel<false, NS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e1 != hipSuccess || e2 != hipSuccess) JLLM_FAIL("gemm_pingpong: cannot reserve %zu bytes of LDS", smem);
+    configured = true;
+  }
+  dim3 grid((unsigned)groups, 1, splits);
+  if (W2)
+    gemm_pingpong_mixed_kernel<true, NS><<<grid, PP_WAVES * 64, smem, stream>>>(
+        (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, wide, cols);
+  else
+    gemm_pingpong_mixed_kernel<false, NS><<<grid, PP_WAVES * 64, smem, stream>>>(
+        (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, wide, cols);
+  return 0;
+}
+
+// `tile_rows`: 256 or 192 (rows of the output tile; 256 columns, 128 outputs with the gated epilogue), or 384: tiles of 256 rows and
+// wide ones for the last at most 128 rows.
+// `splits` > 1 cuts K over gridDim.z (not with the gated epilogue; any count that leaves every part four stages): `partial` then holds splits * M * N floats, summed
 // in ascending order of the split by the other tiled kernel's reduction, which also makes the RMSNorm of the new rows where
 // `norm_rows` is given (as there). Returns 0 when it ran, 1 when the shape is not one it takes, -1 on errors.
 extern "C" int jllm_gemm_pingpong_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias,
@@ -273,13 +330,18 @@ extern "C" int jllm_gemm_pingpong_bf16(const void* A, int lda, const void* W, co
   if (splits > 1 && (W2 || !partial)) JLLM_FAIL("gemm_pingpong: %d K splits are not possible here", splits);
   if (norm_rows && splits == 1) JLLM_FAIL("gemm_pingpong: the norm is the reduction's, and K is whole");
   if (splits > 65535 || (K / PP_BK) / splits < 4) return 1;
+  // (an uneven cut: the last part is what the others, rounded up, leave)
+  const int per = (K / PP_BK + splits - 1) / splits;
+  if (K / PP_BK - per * (splits - 1) < 4) return 1;
   int rc;
   if (tile_rows == 256)
     rc = launch_pingpong<4, 4>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, splits, partial, stream);
   else if (tile_rows == 192)
     rc = launch_pingpong<3, 4>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, splits, partial, stream);
+  else if (tile_rows == (256 | 128) && M % 256 >= 1 && M % 256 <= 128)
+    rc = launch_mixed(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, splits, partial, stream);
   else
-    JLLM_FAIL("gemm_pingpong: tile of %d rows (256 and 192 are built)", tile_rows);
+    JLLM_FAIL("gemm_pingpong: tile of %d rows for %d (256 and 192 are built; 384: 256 and, where the last rows are at most 128, wide ones for them)", tile_rows, M);
   if (rc != 0) return rc;
   JLLM_CHECK_LAUNCH("gemm_pingpong");
   if (splits > 1 && norm_rows)

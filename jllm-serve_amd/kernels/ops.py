@@ -715,6 +715,73 @@ def _tiled_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int]:
     return rows, cut
 
 
+_own_tiled_plan = _tiled_plan  # as it is, whoever puts another in its place
+
+
+WIDE_LAST = 384                     # tile code: 256 rows, and the last at most 128 in tiles of half the rows and twice the columns
+WIDE_LAST_EXTRA = (0.17, 0.25)      # of a tile's time that a wide one takes longer: up to 64 rows, beyond
+FINER_CUTS = 8                      # the two-group kernel's parts of K, any count up to this
+FINER_AT_MOST = 0.95                # of the plan's estimate
+NORM_PASS_US = (4.0, 0.6e-6)        # the norm behind an adding product with K whole (a cut's reduction makes it): launch, per element
+
+
+def _wide_last_us(M: int, N: int, K: int, gated: bool, cut: int) -> float:
+    """The two-group kernel with wide tiles for the last rows."""
+    cus = compute_units()
+    lone, full = LARGE_STEP_US[256]
+    steps = K / 32 / cut
+    cols = -(-N // (128 if gated else 256))
+    rounds, last = divmod((M // 256 * cols + -(-cols // 2)) * cut, cus)
+    t = rounds * (steps * full + LARGE_ROUND_US)
+    step = lone + (full - lone) * last / cus
+    if last:
+        t += steps * step + LARGE_ROUND_US
+    t += WIDE_LAST_EXTRA[M % 256 > 64] * steps * (full if rounds else step)
+    return t + (CUT_US[0] + CUT_US[1] * M * N * cut if cut > 1 else 0.0)
+
+
+@functools.lru_cache(maxsize=8192)
+def _tiles(M: int, N: int, K: int, gated: bool, normed: bool, rows: int, cut: int) -> Tuple[int, int]:
+    """(rows of the two-group kernel's tile, `WIDE_LAST`, or 0 for the small tile, ways K is cut): the plan (``rows``, ``cut``) of
+    `_tiled_plan`, or what is estimated to take at most `FINER_AT_MOST` of its time among tiles of 256, 192 and wide last rows
+    with K in any number of parts up to `FINER_CUTS`; ``normed``: the product adds into the residual and the RMSNorm of the new
+    rows follows, which the reduction of a cut product makes on its way. A plan that is not `_tiled_plan`'s own stands.
+
+    Against the times, inside a graph, of every choice for 142 products (six shapes at 280 to 4,614 rows): 1.7 % behind the best
+    on average, where the plan is 4.7 % behind; of 25 choices that change none is slower than the plan's (with 0.97 for 0.95 4B
+    down at 700 rows went to 192 rows in six parts, and the pass took 2.7 % longer). Whole passes: 560 rows of the 8B shape 12 %
+    faster, 280 to 340 of the 14B 18 %, 2,600 of the 8B 7 %, of the 0.6B 3.5 %. us, plan / now: 8B down at 1,100 rows
+    139.8 (192 rows, two parts) / 120.5 (256, three), at 280 64.1 (small tile, four) / 54.0 (192, eight), 14B qkv at 631 77.0 (256,
+    two) / 67.1 (three), down at 900 195.6 (192, two) / 174.9 (256, three); wide last rows: csrc/gemm_pingpong.hip."""
+    if K % 64 or M < PINGPONG_MIN_ROWS or (rows, cut) != _own_tiled_plan(M, N, K, gated):
+        return rows, cut
+    return _finer_tiles(-(-M // 64) * 64, N, K, gated, normed, rows, cut)
+
+
+@functools.lru_cache(maxsize=8192)
+def _finer_tiles(M: int, N: int, K: int, gated: bool, normed: bool, rows: int, cut: int) -> Tuple[int, int]:
+    """The same for row counts up to M in whole 64s, which all have M's tiles (so that a prompt of a new length does not weigh
+    two dozen choices per product anew)."""
+
+    def us(tile, c):
+        t = _wide_last_us(M, N, K, gated, c) if tile == WIDE_LAST else _large_us(M, N, K, gated, tile, c) if tile else _small_us(M, N, K, gated, c)
+        return t + (NORM_PASS_US[0] + NORM_PASS_US[1] * M * N if normed and c == 1 else 0.0)
+
+    least, best = FINER_AT_MOST * us(rows, cut), (rows, cut)
+    for tile in (192, 256, WIDE_LAST):
+        if tile == WIDE_LAST and M % 256 not in (64, 128):
+            continue
+        for c in range(1, 1 + (1 if gated else FINER_CUTS)):
+            if c > 1 and K // c < PINGPONG_SPLIT_MIN_K:
+                break
+            if tile == 192 and c in (1, 2, 4):  # the plan has weighed these against 256 rows, with exceptions of its own
+                continue
+            t = us(tile, c)
+            if t < least:
+                least, best = t, (tile, c)
+    return best
+
+
 STREAM_MAX_ROWS = 64   # up to here the second weight-streaming kernel (activations through LDS)
 
 
@@ -987,14 +1054,14 @@ def _cut_takes_norm(M: int, N: int, K: int) -> bool:
     rows as well."""
     if M <= STREAM_MAX_ROWS or K % 64 or N % 4 or N > 8192 or _wide_plan(M, N, K, False, ADDS) is not None:
         return False
-    rows, cut = _tiled_plan(M, N, K, False)
+    rows, cut = _tiles(M, N, K, False, True, *_tiled_plan(M, N, K, False))
     return (cut if rows else _k_splits(M, N, K, False)) > 1
 
 
 def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0, norm=_NO_NORM) -> bool:
     """The bf16 matrix-core kernels: a weight-streaming one for up to 16 rows, another for up to 64; for many rows
     the two-group kernel with tiles of 256 or 192 rows by 256 columns or the small tile, either with K cut over several
-    workgroups when the output has few tiles (`_tiled_plan`); then the reduction makes the ``norm`` (gain, its type, eps, rows,
+    workgroups when the output has few tiles (`_tiled_plan`, `_tiles`); then the reduction makes the ``norm`` (gain, its type, eps, rows,
     their stride) of the new rows where one is asked for. Each declines shapes it does
     not take; then the fp32 kernel runs."""
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
@@ -1011,7 +1078,7 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0, norm=_NO_
         sums, arrivals = _stream_scratch(M, N, w2 is not None, a, plan)
         if _try("jllm_gemm_stream_bf16", *head, *plan, _ptr(sums), _ptr(arrivals), None, 0, None, F32, None, 0, None, 0, 0.0, _stream()):
             return True
-    tile_rows, cut = _tiled_plan(M, N, K, w2 is not None)
+    tile_rows, cut = _tiles(M, N, K, w2 is not None, norm is not _NO_NORM, *_tiled_plan(M, N, K, w2 is not None))
     if tile_rows:
         partial = torch.empty((cut * M * N,), dtype=torch.float32, device=a.device) if cut > 1 else None
         if _try("jllm_gemm_pingpong_bf16", *head, tile_rows, cut, _ptr(partial), *norm, _stream()):

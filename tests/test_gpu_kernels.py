@@ -210,6 +210,33 @@ def test_gemm_two_group_kernel_with_tiles_of_192_rows(ops, monkeypatch, M, N, K,
     assert bool(((got[1].double() - ref).abs() <= K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
 
 
+@pytest.mark.parametrize("M,N,K,cut", [(257, 520, 128, 1), (320, 131, 160, 1), (321, 1300, 192, 1), (640, 700, 3200, 3), (512 + 60, 2500, 5376, 5)])
+def test_gemm_two_group_kernel_with_wide_last_rows(ops, monkeypatch, M, N, K, cut):
+    """The last 1 to 64 or 65 to 128 rows in tiles of twice the columns against tiles of 256 rows throughout, bit for bit: both
+    edges of either kind, an odd number of column tiles (the last wide one is half beyond the end), K from four stages on and in
+    parts of unequal length, every epilogue."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M + K)
+    a = torch.randn(M, K, device=DEV, generator=gen).bfloat16()
+    w, w2 = ((torch.randn(N, K, device=DEV, generator=gen) * K ** -0.5).bfloat16() for _ in range(2))
+    bias = torch.randn(N, device=DEV, generator=gen)
+
+    def outputs(rows):
+        monkeypatch.setattr(ops, "_tiles", lambda m, n, k, gated, *plan: (rows, 1 if gated else cut))
+        ops.reset_stats()
+        res = torch.ones(M, N, device=DEV)
+        ops.gemm(a, w, bias=bias, out=res, epilogue=ops.EPI_ADD)
+        got = [res, ops.gemm(a, w, out_dtype=torch.float32), ops.gemm(a, w, bias=bias), ops.gemm(a, w, w2=w2, epilogue=ops.EPI_GATED)]
+        assert ops.stats()["ran"] == {"jllm_gemm_pingpong_bf16": 4}
+        return got
+
+    monkeypatch.setattr(ops, "_wide_plan", lambda *_: None)
+    tall, got = outputs(256), outputs(ops.WIDE_LAST)
+    assert all(torch.equal(x, y) for x, y in zip(got, tall))
+    ref = a.double() @ w.double().T  # fp32 sums of K rounded products: K 2^-24 of the sum of magnitudes at most
+    assert bool(((got[1].double() - ref).abs() <= K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 520, 128), (130, 516, 192), (256, 1024, 256), (385, 131, 576)])
 def test_the_small_tile_gives_the_bits_of_the_two_group_kernel(ops, monkeypatch, M, N, K):
     """The small tile's accumulators lie otherwise over the lanes (32 x 32) than the two-group kernel's (16 x 16): every

@@ -145,6 +145,31 @@ def test_plan_of_the_tiled_products():
     assert {(192, 1), (192, 2), (192, 4), (256, 1), (256, 2), (256, 4)} <= taken, taken
 
 
+def test_tiles_that_the_dispatch_asks_for():
+    """Beside the plan's own: tiles the kernel has, wide last rows only for at most 128 of them, K in at most eight parts that
+    all keep four stages or more, never for the gated product; few rows, K that is no multiple of 64 and a plan that
+    was put in the place of the rule's own are left alone."""
+    shapes = [s for group in SHAPES.values() for s in group] + [(100, 8256, False), (4100, 1056, False), (5120, 17408, False)]
+    taken = set()
+    for n, k, gated in shapes:
+        for rows in (65, 256, 257, 280, 320, 385, 560, 631, 700, 900, 1100, 1320, 2100, 2600, 3111, 4614, 8192):
+            plan = ops._tiled_plan(rows, n, k, gated)
+            for normed in (False, True):
+                tile, cut = ops._tiles(rows, n, k, gated, normed and not gated, *plan)
+                where = (rows, n, k, gated, tile, cut)
+                if (tile, cut) == plan:
+                    continue
+                assert rows >= ops.PINGPONG_MIN_ROWS and k % 64 == 0 and tile in (192, 256, ops.WIDE_LAST) and 1 <= cut <= ops.FINER_CUTS, where
+                assert tile != ops.WIDE_LAST or 1 <= rows % 256 <= 128, where
+                assert not gated or cut == 1, where
+                stages = k // 32
+                assert cut == 1 or (k // cut >= ops.PINGPONG_SPLIT_MIN_K and stages - -(-stages // cut) * (cut - 1) >= 4), where
+                taken.add((tile, cut))
+            other = (256, 2) if plan != (256, 2) else (192, 1)
+            assert ops._tiles(rows, n, k, gated, False, *other) == other
+    assert {t for t, _ in taken} == {192, 256, ops.WIDE_LAST} and {3, 5} <= {c for _, c in taken}, taken
+
+
 def test_the_attention_plan_says_whether_the_runs_of_a_step_differ_much_in_keys():
     """One prompt from its start has runs of 128 to 2,048 keys (the portion kernel then cuts every run's keys over two
     groups of waves); a portion deep inside a long request, or several of them, has runs of about the same length."""
