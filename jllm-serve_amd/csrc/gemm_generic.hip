@@ -14,6 +14,7 @@
 // Epilogues: 0 store (fp32 or bf16), 1 add into an fp32 matrix (the residual stream), 2 gated:
 // out = gate(A*Wg^T, A*Wu^T) (the gate functions of common.h) with two weight matrices sharing the A tile.
 #include "common.h"
+#include "lds_ring.h"
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
@@ -306,7 +307,142 @@ __global__ __launch_bounds__(GATED ? 320 : 256) void gemm_f32_rows_kernel(const 
   if (r < M) finish_four<GATED>(acc, up, r, n, N, bias, bias_dtype, out, out_dtype, ldo, epilogue, gs);
 }
 
+// Up to four rows, fp32 operands: the same chains on the vector units, where a multiply-add takes 4 cycles and not 8. A lane owns one
+// output (16 weight rows x 4 activation rows per wave; gate and up are a wave each), so that nothing but its own chain orders its
+// sums. A wave issues one instruction every 4 cycles, so what the chain needs besides has to be little: the four lanes of a
+// weight row hold four pieces of it, 16 k in all, from one LDS read, and a multiply-add takes its weight from the quad's lane q by
+// DPP; the activations are a read per four k.
+// Four other waves keep the operands on their way, straight from memory into a ring of turns of 128 k in LDS. One barrier a turn:
+// in front of it the loading waves wait for their part of the turn, behind it they refill the turn that was read before. us inside
+// a graph at three rows, the kernel above / this: 4,096 x 2,048 15.1 / 9.9, 1,024 x 2,048 12.7 / 8.8, 1,024 x 3,072 19.0 / 12.3,
+// 2,048 x 6,144 35.0 / 22.4 (3.3 ns a k, where the kernel above takes 5.3), gated 3,072 x 1,024 14.4 / 7.9, gated 6,144 x 2,048
+// 42.4 / 20.2, 151,936 x 1,024 160 / 107 (5.8 TB/s). Turns of 256 k in a ring of six (144 KB): 7 to 17 % slower, twice as slow
+// where compute units then hold one workgroup instead of three.
+template <bool GATED>
+struct F32Few {
+  static constexpr int NC = GATED ? 2 : 1, LOADERS = 4;
+  static constexpr int BLOCKS = 4, RING = GATED ? 3 : 4;  // blocks of 32 k per turn, turns
+  static constexpr int BLOCK_KB = 2 * NC + 1, TURN_KB = BLOCKS * BLOCK_KB;
+  static constexpr int LOADS = TURN_KB / LOADERS;  // of 1 KB: 8 rows x 128 bytes
+  static constexpr int THREADS = (NC + LOADERS) * 64;
+  static constexpr size_t LDS = (size_t)RING * TURN_KB * 1024;
+  static_assert(TURN_KB % LOADERS == 0 && RING * LOADS < 63, "whole loads per wave, as many in flight as the counter holds");
+};
+// sixteen links of a chain: k = 4 q + j takes w[j] of the quad's lane q and a[q][j]. Written as instructions, which the compiler
+// would each make two of (a move by DPP, then the multiply-add); what a DPP operand needs between it and a vector instruction
+// that wrote it is waited for here, since the compiler does not look into this.
+__device__ __forceinline__ float chain16(floatx4 w, const floatx4 (&a)[4], float acc) {
+#define LINK(W, A, Q) "v_fmac_f32_dpp %0, %" #W ", %" #A " quad_perm:[" #Q "," #Q "," #Q "," #Q "] row_mask:0xf bank_mask:0xf\n\t"
+  asm("s_nop 1\n\t" LINK(1, 5, 0) LINK(2, 6, 0) LINK(3, 7, 0) LINK(4, 8, 0) LINK(1, 9, 1) LINK(2, 10, 1) LINK(3, 11, 1) LINK(4, 12, 1)
+          LINK(1, 13, 2) LINK(2, 14, 2) LINK(3, 15, 2) LINK(4, 16, 2) LINK(1, 17, 3) LINK(2, 18, 3) LINK(3, 19, 3) LINK(4, 20, 3)
+      : "+v"(acc)
+      : "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(a[0][0]), "v"(a[0][1]), "v"(a[0][2]), "v"(a[0][3]), "v"(a[1][0]), "v"(a[1][1]), "v"(a[1][2]),
+        "v"(a[1][3]), "v"(a[2][0]), "v"(a[2][1]), "v"(a[2][2]), "v"(a[2][3]), "v"(a[3][0]), "v"(a[3][1]), "v"(a[3][2]), "v"(a[3][3]));
+#undef LINK
+  return acc;
+}
+template <bool GATED>
+__global__ __launch_bounds__((GATED ? 6 : 5) * 64) void gemm_f32_few_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W,
+                                                                             const float* __restrict__ W2, const void* __restrict__ bias, int bias_dtype,
+                                                                             void* __restrict__ out, int out_dtype, int ldo, int M, int N, int K,
+                                                                             int epilogue, GateSpec gs) {
+  using F = F32Few<GATED>;
+  extern __shared__ __align__(1024) float lds[];  // [RING][BLOCKS][a block: 16 rows of W, of W2, 8 of A; 128 bytes a row]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * 16;
+  const int turns = K / (F::BLOCKS * 32);
+  if (wave >= F::NC) {
+    const int me = wave - F::NC, row = lane >> 3, slot = lane & 7;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)lds;
+    const float* at[F::LOADS];  // this lane's piece of each of the wave's loads of a turn
+#pragma unroll
+    for (int i = 0; i < F::LOADS; ++i) {
+      const int u = me * F::LOADS + i, block = u / F::BLOCK_KB, part = u % F::BLOCK_KB;
+      const int r = (part & 1) * 8 + row, k = block * 32 + (slot ^ ring_swz(part == 2 * F::NC ? row : r)) * 4;
+      at[i] = (part == 2 * F::NC ? A + (size_t)min(row, M - 1) * lda : (part < 2 ? W : W2) + (size_t)min(n0 + r, N - 1) * K) + k;
+    }
+    auto issue = [&](int t, int place) {
+#pragma unroll
+      for (int i = 0; i < F::LOADS; ++i)
+        load_to_lds_16(at[i] + (size_t)t * F::BLOCKS * 32, lds0 + (uint32_t)(place * F::TURN_KB + me * F::LOADS + i) * 1024u);
+    };
+#pragma unroll
+    for (int t = 0; t < F::RING; ++t)
+      if (t < turns) issue(t, t);
+    int asked = min(F::RING, turns), place = 0;  // the place of turn t - 1
+    for (int t = 0; t < turns; ++t) {
+      switch (asked - 1 - t) {  // turns that may still be on their way
+        case 3: wait_loads<(F::RING > 3 ? 3 : 0) * F::LOADS>(); break;
+        case 2: wait_loads<2 * F::LOADS>(); break;
+        case 1: wait_loads<1 * F::LOADS>(); break;
+        default: wait_loads<0>();
+      }
+      __builtin_amdgcn_s_barrier();
+      if (t == 0) continue;
+      if (asked < turns) issue(asked++, place);
+      if (++place == F::RING) place = 0;
+    }
+    if (GATED) __syncthreads();
+    return;
+  }
+  const int r = lane >> 2, m = lane & 3, n = n0 + r;
+  const bool mine = m < M && n < N;
+  float prev = 0.f;
+  if (epilogue == 1 && mine) prev = ((const float*)out)[(size_t)m * ldo + n];
+  const float* wrow = lds + wave * 512 + r * 32;  // of a block
+  const float* arow = lds + F::NC * 512 + m * 32;
+  const int wswz = ring_swz(r), aswz = ring_swz(m);
+  float acc = 0.f;
+  for (int t0 = 0; t0 < turns; t0 += F::RING) {
+#pragma unroll
+    for (int place = 0; place < F::RING; ++place) {  // (each with its own addresses: an addition per read costs 7 %)
+      if (t0 + place >= turns) break;
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const int at = place * F::TURN_KB * 256;
+      constexpr int CHUNKS = 2 * F::BLOCKS;  // of 16 k, each requested two ahead of its multiply-adds
+      floatx4 w[3], a[3][4];
+      auto read = [&](int i) {
+        const int block = at + (i >> 1) * F::BLOCK_KB * 256, c = 4 * (i & 1);
+        w[i % 3] = *(const floatx4*)(wrow + block + (((c + m) ^ wswz) << 2));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[i % 3][q] = *(const floatx4*)(arow + block + (((c + q) ^ aswz) << 2));
+      };
+      read(0);
+      read(1);
+#pragma unroll
+      for (int i = 0; i < CHUNKS; ++i) {
+        if (i + 2 < CHUNKS) read(i + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        acc = chain16(w[i % 3], a[i % 3], acc);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the turn's last reads, before the barrier behind which it is filled again
+    }
+  }
+  float up = 0.f;
+  if (GATED) {
+    __shared__ float meet[64];
+    if (wave) meet[lane] = acc;
+    __syncthreads();
+    if (wave) return;
+    up = meet[lane];
+  }
+  if (!mine) return;
+  if (bias) acc += (bias_dtype == JLLM_BF16) ? ldf((const bf16_t*)bias, n) : ldf((const float*)bias, n);
+  if (GATED) acc = gated<false>(acc, up, gs);
+  const size_t o = (size_t)m * ldo + n;
+  if (epilogue == 1)
+    ((float*)out)[o] = prev + acc;
+  else if (out_dtype == JLLM_BF16)
+    stf((bf16_t*)out, o, acc);
+  else
+    stf((float*)out, o, acc);
+}
+
 #define GEMM_ROWS_MAX 16
+#define GEMM_FEW_MAX 4
 
 // Measured (fp32 operands, one product alone, against the vector-unit kernels that stood here): 2,048 x 4,096 x 4,096 1,029 ->
 // 590 us (117 TFLOP/s; a library product reaches 154), 847 rows of N = 1,024 and K = 2,048 337 -> 51, K = 3,072 503 -> 73,
@@ -356,8 +492,25 @@ static int launch_f32_tile(const F32Args& g, hipStream_t stream) {
   return 0;
 }
 
+template <bool GATED>
+static int launch_f32_few(const F32Args& g, hipStream_t stream) {
+  using F = F32Few<GATED>;
+  static bool configured = false;
+  if (!configured) {  // above 64 KB the size has to be allowed first
+    if (hipFuncSetAttribute((const void*)gemm_f32_few_kernel<GATED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)F::LDS) != hipSuccess)
+      JLLM_FAIL("gemm: cannot reserve %zu bytes of LDS", F::LDS);
+    configured = true;
+  }
+  gemm_f32_few_kernel<GATED><<<(g.N + 15) / 16, F::THREADS, F::LDS, stream>>>((const float*)g.A, g.lda, (const float*)g.W, (const float*)g.W2, g.bias,
+                                                                          g.bias_dtype, g.out, g.out_dtype, g.ldo, g.M, g.N, g.K, g.epilogue, g.gs);
+  return 0;
+}
+
 template <typename TA, typename TW, bool WIDE>
 static int launch_f32(const F32Args& g, hipStream_t stream) {
+  if constexpr (WIDE && sizeof(TA) == 4 && sizeof(TW) == 4) {
+    if (g.M <= GEMM_FEW_MAX && g.K % (F32Few<false>::BLOCKS * 32) == 0) return g.W2 ? launch_f32_few<true>(g, stream) : launch_f32_few<false>(g, stream);
+  }
   if (g.M <= GEMM_ROWS_MAX) {
     dim3 grid((g.N + 15) / 16);
     if (g.W2)

@@ -571,6 +571,30 @@ def test_float32_products_are_one_chain_of_multiply_adds(ops, M, N, K, wdt):
         assert torch.equal(few, gated[at:at + 16])
 
 
+@pytest.mark.parametrize("N,K", [(1, 128), (16, 256), (17, 384), (40, 512), (300, 640), (4100, 1152)])
+def test_float32_products_of_few_rows(ops, N, K):
+    """Up to four rows, K in turns of 128 (one, fewer than the ring holds, exactly those, more, not a multiple of them), weight
+    rows that end inside a workgroup, every epilogue: the bits of the same rows among six, which the other kernel takes, also with
+    an infinity in one row; a stride between the rows."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(N + K)
+    a = torch.randn(6, K + 4, device=DEV, generator=gen)[:, :K]
+    w, w2 = (torch.randn(N, K, device=DEV, generator=gen) * K ** -0.5 for _ in range(2))
+    a[1, K // 2] = float("inf")
+    bias = torch.randn(N, device=DEV, generator=gen)
+    res = torch.randn(6, N, device=DEV, generator=gen)
+    add = ops.gemm(a, w, bias=bias, out=res.clone(), epilogue=ops.EPI_ADD, exact=True)
+    many = [ops.gemm(a, w, bias=bias, exact=True), ops.gemm(a, w, w2=w2, epilogue=ops.EPI_GATED, exact=True), ops.gemm(a, w, out_dtype=torch.bfloat16, exact=True)]
+    for first, rows in ((0, 1), (1, 2), (0, 3), (2, 4)):
+        x, r = a[first:first + rows], res[first:first + rows].clone()
+        few = [ops.gemm(x, w, bias=bias, exact=True), ops.gemm(x, w, w2=w2, epilogue=ops.EPI_GATED, exact=True), ops.gemm(x, w, out_dtype=torch.bfloat16, exact=True)]
+        ops.gemm(x, w, bias=bias, out=r, epilogue=ops.EPI_ADD, exact=True)
+        for got, want in zip(few + [r], many + [add]):
+            assert torch.equal(torch.nan_to_num(got, nan=7.0), torch.nan_to_num(want[first:first + rows], nan=7.0)), (rows, first)
+    tiny, small = a.nan_to_num(posinf=1.0) * 2.0 ** -68, w * 2.0 ** -68  # denormal products and sums
+    assert torch.equal(ops.gemm(tiny[:3], small, exact=True), ops.gemm(tiny, small, exact=True)[:3])
+
+
 @pytest.mark.parametrize("M,N,K,exponent", [(3, 17, 67, 0), (16, 20, 200, -70), (20, 33, 70, 0), (40, 35, 68, -71), (130, 40, 36, -70)])
 def test_float32_products_round_once_per_multiply_add(ops, M, N, K, exponent):
     """The 32-bit products on operands of 24 bits, whose products a multiply-add must not round, against the C library's
