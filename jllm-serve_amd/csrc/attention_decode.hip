@@ -31,6 +31,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "layer_launches.h"
 #include "head_lanes.h"
 #include "mfma.h"
 #include "no_alloc.h"

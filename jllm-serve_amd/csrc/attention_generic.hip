@@ -19,6 +19,7 @@
 #include <math.h>
 
 #include "common.h"
+#include "layer_launches.h"
 
 #define ATT_MAX_ACC 8  // head_dim <= 512
 #define ATT_WAVES 4

@@ -35,6 +35,7 @@
 #include <math.h>
 
 #include "common.h"
+#include "layer_launches.h"
 #include "lds_ring.h"
 #include "mfma.h"
 

@@ -3,6 +3,7 @@
 #include <string.h>
 
 #include "common.h"
+#include "layer_launches.h"
 
 static thread_local char g_error[512] = "";
 

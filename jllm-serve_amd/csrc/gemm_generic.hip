@@ -14,6 +14,7 @@
 // Epilogues: 0 store (fp32 or bf16), 1 add into an fp32 matrix (the residual stream), 2 gated:
 // out = gate(A*Wg^T, A*Wu^T) (the gate functions of common.h) with two weight matrices sharing the A tile.
 #include "common.h"
+#include "layer_launches.h"
 #include "lds_ring.h"
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));

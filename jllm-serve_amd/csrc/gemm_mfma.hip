@@ -20,6 +20,7 @@
 //
 // Needs K % 64 == 0 and 16-byte aligned rows; any M and N. The caller falls back otherwise.
 #include "common.h"
+#include "layer_launches.h"
 #include "gemm_epilogue.h"
 #include "mfma.h"
 

@@ -31,6 +31,7 @@
 // Epilogues as in the other tiled kernel (gemm_epilogue.h). Needs K % 32 == 0 and at least NS - 1 stages, 16-byte
 // aligned rows; any M and N (rows beyond the end are read as the last row and never stored).
 #include "common.h"
+#include "layer_launches.h"
 #include "lds_ring.h"
 #include "gemm_epilogue.h"
 #include "mfma.h"

@@ -34,6 +34,7 @@
 //
 // Needs K % 128 == 0, N % 16 == 0, M <= 16, 16-byte aligned rows; the caller falls back otherwise.
 #include "common.h"
+#include "layer_launches.h"
 #include "lds_ring.h"
 #include "mfma.h"
 

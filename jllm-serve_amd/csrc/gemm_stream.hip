@@ -29,6 +29,7 @@
 //
 // Needs K % 128 == 0, N % 16 == 0, 16-byte aligned rows; the caller uses another kernel otherwise.
 #include "common.h"
+#include "layer_launches.h"
 #include "lds_ring.h"
 #include "mfma.h"
 

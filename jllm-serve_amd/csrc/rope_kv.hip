@@ -8,6 +8,7 @@
 // Cache layout of one layer: [page][kv_head][page_size][head_dim]; `slots[t]` = page * page_size + offset
 // of token t, or < 0 for "do not store".
 #include "common.h"
+#include "layer_launches.h"
 #include "head_lanes.h"
 
 template <typename T, typename TG>

@@ -7,9 +7,11 @@ the GPU, they raise.
 """
 from __future__ import annotations
 
+import bisect
 import contextlib
 import ctypes
 import functools
+import struct
 import threading
 from typing import Optional, Tuple
 
@@ -108,6 +110,10 @@ def _declare(lib) -> None:
     lib.jllm_probe_read.restype = _I
     lib.jllm_probe_mfma.argtypes = [_I, _P, ctypes.POINTER(ctypes.c_double), _P]
     lib.jllm_probe_mfma.restype = _I
+    for name, args in _LAYER_ENTRIES.items():
+        fn = getattr(lib, name)
+        fn.argtypes = args
+        fn.restype = _I
     for name, args in _OPTIONAL_SIGS.items():
         if hasattr(lib, name):
             fn = getattr(lib, name)
@@ -133,11 +139,100 @@ _OPTIONAL_SIGS = {
 }
 
 
+# While a layer's launches are kept (`kept_launches`): how many threads do so, and of each its list
+_keeping = 0
+_kept = threading.local()
+
+
+class KeptLaunches:
+    """The launches of the block of statements behind ``with kept_launches()``: (entry point, its arguments, whether it may
+    decline), and every tensor that one of them was given, which stays alive as long as this object."""
+
+    def __init__(self):
+        self.calls, self.tensors = [], []
+
+
+@contextlib.contextmanager
+def kept_launches():
+    global _keeping
+    before, mine = getattr(_kept, "now", None), KeptLaunches()
+    with _lock:
+        _keeping += 1
+    _kept.now = mine
+    try:
+        yield mine
+    finally:
+        _kept.now = before
+        with _lock:
+            _keeping -= 1
+
+
+def _keep(name: str, args: tuple, may_decline: bool) -> None:
+    mine = getattr(_kept, "now", None)
+    if mine is not None:
+        mine.calls.append((name, args, may_decline))
+
+
+_LAYER_ENTRIES = {"jllm_layer_entry": [ctypes.c_char_p, _I], "jllm_layer_launches": [_P, _L, _P, _I, _P]}
+_layer_entries: dict = {}  # entry point -> (its number in csrc/layer_launches.hip, its arguments: 1 address, 2 float)
+
+
+class RepeatedLaunches:
+    """The kept launches, to be made again with some addresses moved. ``spans``: (first address, the one behind the last) of what moves;
+    what lay inside the i-th lies as far behind ``addresses[i]`` when they are made. ``able``: whether all of them can be repeated."""
+
+    def __init__(self, kept: KeptLaunches, spans):
+        self.lib, self.kept, self.able = library(), kept, bool(kept.calls)
+        order = sorted(range(len(spans)), key=spans.__getitem__)
+        begins, ends = [spans[i][0] for i in order], [spans[i][1] for i in order]
+        if any(b < e for b, e in zip(begins[1:], ends)):  # memory that two of them share: whose an address is would not be clear
+            self.able = False
+            return
+        words, places, self.moved = [], [], []
+        for name, args, _ in kept.calls:
+            entry = _layer_entries.get(name)
+            if entry is None:
+                types = _SIGS.get(name) or _OPTIONAL_SIGS.get(name) or ()
+                number = self.lib.jllm_layer_entry(name.encode(), len(types))
+                entry = _layer_entries[name] = (number, len(types), [i for i, t in enumerate(types) if t is _P], [i for i, t in enumerate(types) if t is _F])
+            number, count, addresses, floats = entry
+            if number < 0 or count != len(args):
+                self.able = False
+                return
+            words += (number, count)
+            first = len(words)
+            words += args
+            for i in floats:
+                words[first + i] = struct.unpack("<I", struct.pack("<f", args[i]))[0]
+            for i in addresses:
+                a = args[i]
+                if a is None:
+                    words[first + i] = 0
+                    continue
+                at = bisect.bisect_right(begins, a) - 1
+                if at >= 0 and a < ends[at]:
+                    places.append(first + i)
+                    self.moved.append((order[at], a - begins[at]))
+        # (an int below zero in its two's complement, as the conversion to the array's type leaves it)
+        self.words, self.places = (ctypes.c_ulonglong * len(words))(*words), (ctypes.c_longlong * len(places))(*places)
+        self.room = ctypes.c_ulonglong * len(places)
+
+    def make(self, addresses) -> None:
+        values = self.room(*[addresses[i] + offset for i, offset in self.moved])
+        if self.lib.jllm_layer_launches(self.words, len(self.words), self.places, len(self.places), values) != 0:
+            raise KernelError(self.lib.jllm_last_error().decode("utf-8", "replace"))
+        for name, _, may_decline in self.kept.calls:
+            if may_decline:
+                _count("ran", name)
+
+
 def _call(name: str, *args) -> None:
     lib = library()
     rc = getattr(lib, name)(*args)
     if rc != 0:
         raise KernelError(lib.jllm_last_error().decode("utf-8", "replace"))
+    if _keeping:
+        _keep(name, args, False)
 
 
 _counts: dict = {}
@@ -172,6 +267,8 @@ def _try(name: str, *args) -> bool:
     if rc < 0:
         raise KernelError(lib.jllm_last_error().decode("utf-8", "replace"))
     _count("ran" if rc == 0 else "declined", name)
+    if _keeping and rc == 0:
+        _keep(name, args, True)
     return rc == 0
 
 
@@ -191,6 +288,10 @@ def _dev(*tensors) -> None:
 
 def _ptr(t: Optional[torch.Tensor]):
     """The tensor's address as the entry points take it (their pointer arguments are declared, so a plain int does)."""
+    if _keeping and t is not None:
+        mine = getattr(_kept, "now", None)
+        if mine is not None:
+            mine.tensors.append(t)
     return None if t is None else t.data_ptr()
 
 

@@ -19,6 +19,7 @@ from ..config.schema import GqaSpec
 from ..kernels import ops
 from ..weights.loader import WeightSpec
 from .base import BuildContext, Part, register_part
+from .equal_layers import own_forward
 
 
 TILE_ROWS = 128  # rows of one request that the portion-attention kernel takes per workgroup
@@ -161,6 +162,12 @@ class GqaAttention(Part):
                 meta[name] = t if t is not None and t.numel() else None
             plan.facts["batch"] = meta
         return meta
+
+    def launch_key(self):
+        return ("gqa", self.spec, id(self.position), self.build.dtype, self.build.exact) if own_forward(self, GqaAttention) else None
+
+    def launch_tensors(self):
+        return [self.w_qkv, self.b_qkv, self.w_o, self.b_o, self.g_q, self.g_k]
 
     def forward(self, xb, residual, step, slot, then_norm=None):
         s = self.spec

@@ -19,6 +19,7 @@ import torch
 from ..kernels import ops
 from ..weights.loader import WeightSpec
 from .base import Part, StateShare, part_factory, register_part
+from .equal_layers import own_forward
 from .shift import TokenShift
 
 
@@ -55,6 +56,15 @@ class PreNormBlock(Part):
 
     def step_planners(self):
         return [pl for p in self.parts for pl in (p.step_planners() if hasattr(p, "step_planners") else [])]
+
+    def launch_key(self):
+        if not own_forward(self, PreNormBlock) or self.ffn is None:
+            return None
+        keys = tuple(getattr(p, "launch_key", lambda: None)() for p in self.parts)
+        return None if None in keys else keys
+
+    def launch_tensors(self):
+        return [t for p in self.parts for t in p.launch_tensors()]
 
     chains_norms = True  # forward takes normed_in / next_norm and returns the next block's input promise
 

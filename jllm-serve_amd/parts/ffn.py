@@ -8,6 +8,7 @@ from ..config.schema import GatedMlpSpec
 from ..kernels import ops
 from ..weights.loader import WeightSpec
 from .base import BuildContext, Part, register_part
+from .equal_layers import own_forward
 
 
 class GatedMlp(Part):
@@ -45,6 +46,12 @@ class GatedMlp(Part):
             self.w_gate = get(self._name("gate"))
             self.w_up = get(self._name("up"))
         self.w_down = get(self._name("down"))
+
+    def launch_key(self):
+        return ("gated_mlp", self.hidden, self.dim, self.gate, self.limit, self.build.dtype, self.build.exact) if own_forward(self, GatedMlp) else None
+
+    def launch_tensors(self):
+        return [self.w_gate, self.w_up, self.w_down]
 
     def forward(self, xb, residual, step, then_norm=None):
         h = ops.gemm(xb, self.w_gate, w2=self.w_up, epilogue=ops.EPI_GATED, out_dtype=self.build.dtype,

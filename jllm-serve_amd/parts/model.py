@@ -19,6 +19,7 @@ from ..config.schema import ModelConfig
 from ..kernels import ops
 from ..weights import loader
 from ..weights.loader import WeightSpec
+from . import equal_layers
 from .base import BuildContext, part_factory
 
 
@@ -58,6 +59,7 @@ class DecoderModel:
         self.stream_mix_names = sorted({e.mix_before.name for e in config.schedule if e.mix_before is not None})
         self.stream_mixes = {}
         self.keeps_embedding = bool(self.stream_mix_names) or any(getattr(e, "add_embedding", False) for e in config.schedule)
+        self.equal_runs = [0] * len(config.schedule)  # (known once the weights are)
         self.watch = None  # a function (run, x) called with the stream after every run (tests, debugging)
         # a part that walks the step's requests on the host sets ``capturable = False``; then decode steps are
         # never recorded as graphs
@@ -105,6 +107,7 @@ class DecoderModel:
                 raise ValueError(f"a logit scale needs a final norm that can scale its output, '{self.config.final_norm.kind}' cannot")
             self.final_norm.scale_output(self.config.logit_scale)
         self.lm_head = get(names.head) if names.head in set(source.names()) else self.embed
+        self.equal_runs = equal_layers.equal_runs(self.config.schedule, self.layers)
 
     # -------------------------------------------------------------------------------------------- cache plan
 
@@ -142,8 +145,18 @@ class DecoderModel:
         x0 = x.clone() if self.keeps_embedding else None  # the embedding output, for the runs that bring it back in
         carry = None  # the next block's input norm, when the block before prepared it (parts/block.py)
         added = False  # what joins the stream before this run already did (the block before added it on its way out)
+        native = self.watch is None and equal_layers.launches(x)
+        walked = 0  # runs below this one are done
         for run, e in enumerate(schedule):
+            if run < walked:
+                continue
             layer = self.layers[e.layer]
+            end = self.equal_runs[run]
+            if native and end - run >= equal_layers.LEAST and (run == 0 or self.equal_runs[run - 1] == run) and not added \
+                    and equal_layers.pays(layer, step.n_tokens):
+                walked, carry = equal_layers.walk([self.layers[s.layer] for s in schedule], slots, run, end, x, step, carry,
+                                                  lambda r: self.layers[schedule[r + 1].layer].norm_in)
+                continue
             if e.mix_before is not None:
                 # x <- W [x; x0] (+ the run's vector, as the product's bias): a new stream tensor
                 vec = self._stream_vector(e.add_before) if e.add_before is not None and not added else None

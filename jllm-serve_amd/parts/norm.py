@@ -9,6 +9,7 @@ from ..config.schema import DynTanhSpec, LayerNormSpec, NormSpec
 from ..kernels import ops
 from ..weights.loader import WeightSpec
 from .base import BuildContext, Part, register_part
+from .equal_layers import own_forward
 
 
 class RMSNorm(Part):
@@ -29,6 +30,12 @@ class RMSNorm(Part):
         if self.one_plus:  # the stored weight lies around zero; in fp32, since 1 + w has more digits than a bf16 holds
             self.gain = (self.gain.float() + 1.0).contiguous()
         self.gain32 = self.gain.float().contiguous()  # what the launches between two sublayers take
+
+    def launch_key(self):
+        return ("rmsnorm", self.dim, self.eps, self.out_dtype) if own_forward(self, RMSNorm) else None
+
+    def launch_tensors(self):
+        return [self.gain]
 
     def forward(self, x, rows=None):
         return ops.rmsnorm(x, self.gain, self.eps, self.out_dtype, rows)
