@@ -79,6 +79,8 @@ class GqaStepPlanner:
 class GqaAttention(Part):
     takes_normed_rows = True    # the input goes into ops.gemm and nowhere else
     prepares_next_norm = True   # forward(then_norm=...) ends with then_norm.after_add and returns its promise
+    takes_only = True           # forward(only=rows): behind the attention those rows alone, into ``residual`` of as many
+
     def __init__(self, spec: GqaSpec, prefix: str, build: BuildContext, positions):
         if spec.kv_heads <= 0 or spec.heads % spec.kv_heads != 0:
             raise ValueError(f"{spec.kv_heads} kv heads do not divide {spec.heads} query heads")
@@ -169,7 +171,7 @@ class GqaAttention(Part):
     def launch_tensors(self):
         return [self.w_qkv, self.b_qkv, self.w_o, self.b_o, self.g_q, self.g_k]
 
-    def forward(self, xb, residual, step, slot, then_norm=None):
+    def forward(self, xb, residual, step, slot, then_norm=None, only=None):
         s = self.spec
         g = step.groups[slot.group]
         k_cache, v_cache = slot.rows["k"], slot.rows["v"]
@@ -185,15 +187,17 @@ class GqaAttention(Part):
                                              g.slots, cos, sin, self.g_q, self.g_k, s.qk_norm_eps, s.heads, s.kv_heads,
                                              s.head_dim, rdim, s.window, s.scale, meta, write_kv=slot.writes)
             if att is not None:
-                return self._project_out(att, residual, then_norm)
+                return self._project_out(att, residual, then_norm, only)
         ops.qk_norm_rope_store(qkv, step.positions, g.slots, cos, sin, self.g_q, self.g_k, s.qk_norm_eps, s.heads,
                                s.kv_heads, s.head_dim, rdim, slot.page_size, k_cache, v_cache, write_kv=slot.writes)
         att = ops.paged_attention(qkv[:, :s.q_dim], k_cache, v_cache, g.block_table, step.row_req,
                                   step.positions, s.heads, s.kv_heads, s.head_dim, s.window, s.scale, meta=meta,
                                   exact=self.build.exact, slopes=slopes)
-        return self._project_out(att, residual, then_norm)
+        return self._project_out(att, residual, then_norm, only)
 
-    def _project_out(self, att, residual, then_norm):
+    def _project_out(self, att, residual, then_norm, only=None):
+        if only is not None:
+            att = att.index_select(0, only)
         if then_norm is not None:
             return then_norm.after_add(att, self.w_o, residual, bias=self.b_o, exact=self.build.exact)
         ops.gemm(att, self.w_o, bias=self.b_o, out=residual, epilogue=ops.EPI_ADD, exact=self.build.exact)

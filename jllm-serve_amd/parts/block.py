@@ -14,6 +14,8 @@ parts; a part that knows nothing of this works as before):
 """
 from __future__ import annotations
 
+from types import SimpleNamespace
+
 import torch
 
 from ..kernels import ops
@@ -103,8 +105,36 @@ class PreNormBlock(Part):
         self.ffn.forward(xb, x, step)
         return None
 
+    def ends_rows(self):
+        return own_forward(self, PreNormBlock) and rows_alone(self.ffn)
+
+    def forward_last(self, x, step, slot, normed_in=None):
+        """As the last layer: the mixer runs over all rows (its cache is written for all of them), what follows its heads over
+        the step's selected rows only, as nobody reads the others. Returns the stream of those, [n_selected, width]."""
+        xb = self._input(self.norm_in, self.mixer, x, normed_in)
+        if step.n_selected and type(self.mixer).__dict__.get("takes_only") and "forward" not in vars(self.mixer):
+            some = x.index_select(0, step.selected)
+            self.mixer.forward(xb, some, step, slot, only=step.selected)
+        else:
+            self.mixer.forward(xb, x, step, slot)
+            some = x.index_select(0, step.selected)
+        if step.n_selected:
+            self.ffn.forward(self._input(self.norm_post, self.ffn, some, None), some, selected_step(step))
+        return some
+
 
 register_part("arrangement", "prenorm", PreNormBlock, replace=True)
+
+
+def rows_alone(ffn) -> bool:
+    """Whether this is a feed-forward (of exactly a class that says so, with its methods) whose output for a row depends on that row
+    and its token alone."""
+    return ffn is not None and bool(type(ffn).__dict__.get("rows_alone")) and not {"forward", "output"} & set(vars(ffn))
+
+
+def selected_step(step):
+    """What such a feed-forward asks of a step, of its selected rows."""
+    return SimpleNamespace(n_tokens=step.n_selected, token_ids=step.token_ids.index_select(0, step.selected))
 
 
 def sublayer_output(part, xb, step, slot, width):
@@ -198,26 +228,51 @@ class SandwichBlock(Part):
             x += add_vec.float()
         return None
 
+    def _branches(self, xb, step, slot, then, add_rows):
+        """The mixer's output, as ([rows], None), or as two branches and their weights, whose sum the seam's launch then takes."""
+        scales = getattr(getattr(self.mixer, "spec", None), "scales", ())
+        if hasattr(self.mixer, "outputs") and not getattr(self.mixer, "fused", False) and len(scales) == 2 \
+                and not getattr(self.mixer, "out_names", None) and self._seams(self.norm_mixer_out, then, add_rows):
+            return self.mixer.outputs(xb, step, slot), list(scales)
+        return [sublayer_output(self.mixer, xb, step, slot, self.width)], None
+
     def forward(self, x, step, slot, normed_in=None, next_norm=None, add_after=None, add_rows_after=None):
         """``normed_in``: norm_in of x as the block before left it (a tensor) or None; ``next_norm``: the norm part that
         reads x next; ``add_after``: a vector that joins the stream behind this layer, ``add_rows_after``: rows that join
         it before that. Returns ``next_norm`` of the new x when the last seam prepared it."""
         xb = normed_in if isinstance(normed_in, torch.Tensor) else self.norm_in.forward(x)
         then, rows, vec = (next_norm, add_rows_after, add_after) if self.ffn is None else (self.norm_post, None, None)
-        scales = getattr(getattr(self.mixer, "spec", None), "scales", ())
-        if hasattr(self.mixer, "outputs") and not getattr(self.mixer, "fused", False) and len(scales) == 2 \
-                and not getattr(self.mixer, "out_names", None) and self._seams(self.norm_mixer_out, then, rows):
-            # two weighted branches: their sum is taken inside the seam's launch
+        branches, scales = self._branches(xb, step, slot, then, rows)
+        if scales:
             more = {"add_rows": rows} if rows is not None else {}
-            xb = self.norm_mixer_out.seam(x, self.mixer.outputs(xb, step, slot), list(scales), add_vec=vec, then=then, **more)
+            xb = self.norm_mixer_out.seam(x, branches, scales, add_vec=vec, then=then, **more)
         else:
-            xb = self._join(self.norm_mixer_out, x, sublayer_output(self.mixer, xb, step, slot, self.width), rows, vec, then)
+            xb = self._join(self.norm_mixer_out, x, branches[0], rows, vec, then)
         if self.ffn is None:
             return xb
         if xb is None:
             xb = self.norm_post.forward(x)
         branch = sublayer_output(self.ffn, xb, step, None, self.width)
         return self._join(self.norm_ffn_out, x, branch, add_rows_after, add_after, next_norm)
+
+    def ends_rows(self):
+        return own_forward(self, SandwichBlock) and rows_alone(self.ffn)
+
+    def forward_last(self, x, step, slot, normed_in=None):
+        """As ``PreNormBlock.forward_last``: behind the mixer's output only the selected rows go on."""
+        xb = normed_in if isinstance(normed_in, torch.Tensor) else self.norm_in.forward(x)
+        branches, scales = self._branches(xb, step, slot, self.norm_post, None)
+        some = x.index_select(0, step.selected)
+        if step.n_selected:
+            branches = [b.index_select(0, step.selected) for b in branches]
+            if scales:
+                xb = self.norm_mixer_out.seam(some, branches, scales, then=self.norm_post)
+            else:
+                xb = self._join(self.norm_mixer_out, some, branches[0], None, None, self.norm_post)
+            if xb is None:
+                xb = self.norm_post.forward(some)
+            self._join(self.norm_ffn_out, some, sublayer_output(self.ffn, xb, selected_step(step), None, self.width), None, None, None)
+        return some
 
 
 register_part("arrangement", "sandwich", SandwichBlock, replace=True)

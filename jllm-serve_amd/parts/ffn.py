@@ -14,6 +14,8 @@ from .equal_layers import own_forward
 class GatedMlp(Part):
     takes_normed_rows = True    # the input goes into ops.gemm and nowhere else
     prepares_next_norm = True   # forward(then_norm=...) ends with then_norm.after_add and returns its promise
+    rows_alone = True  # a row's output depends on that row and its token alone
+
     def __init__(self, spec: GatedMlpSpec, prefix: str, build: BuildContext):
         if spec.activation not in ops.GATE_FUNCTIONS:
             raise ValueError(f"unsupported activation '{spec.activation}': the product kernels have "

@@ -154,7 +154,9 @@ class LatentAttention(Part):
             meta["tiles_dev"] = tiles if tiles is not None and tiles.numel() else None
         return meta
 
-    def forward(self, xb, residual, step, slot, then_norm=None):
+    takes_only = True  # forward(only=rows): behind the attention those rows alone, into ``residual`` of as many
+
+    def forward(self, xb, residual, step, slot, then_norm=None, only=None):
         s, exact = self.spec, self.build.exact
         g = step.groups[slot.group]
         cache = slot.rows["ckr"]
@@ -175,8 +177,11 @@ class LatentAttention(Part):
                               exact=exact)
         lat = ops.latent_attention(qa, cache, g.block_table, step.row_req, step.positions, s.heads, s.kv_rank, s.window,
                                    s.scale, self.sink, meta=self._batch_facts(step), exact=exact)
+        gate = y[:, gate_off:gate_off + s.heads * s.vdim] if s.out_gate else None
+        if only is not None:
+            lat, gate = lat.index_select(0, only), gate.index_select(0, only) if gate is not None else None
         if s.out_gate:
-            att = ops.latent_heads(lat, self.w_uv, gate=y[:, gate_off:gate_off + s.heads * s.vdim], exact=exact)
+            att = ops.latent_heads(lat, self.w_uv, gate=gate, exact=exact)
         else:
             att = ops.latent_heads(lat, self.w_uv, exact=exact)
         if then_norm is not None:

@@ -147,6 +147,7 @@ class DecoderModel:
         added = False  # what joins the stream before this run already did (the block before added it on its way out)
         native = self.watch is None and equal_layers.launches(x)
         walked = 0  # runs below this one are done
+        selected = step.selected  # rows of x that are wanted; None: x is those already
         for run, e in enumerate(schedule):
             if run < walked:
                 continue
@@ -171,7 +172,10 @@ class DecoderModel:
                 ops.layernorm_seam(x, 0.0, add_vec=self._stream_vector(e.add_before))
                 carry = None
             added = False
-            if not getattr(layer, "chains_norms", False):
+            if run + 1 == len(schedule) and step.n_selected < step.n_tokens and self.watch is None and self.streams == 1 \
+                    and hasattr(layer, "ends_rows") and layer.ends_rows():
+                x, selected = layer.forward_last(x, step, slots[run], normed_in=carry), None
+            elif not getattr(layer, "chains_norms", False):
                 layer.forward(x, step, slots[run])
                 carry = None
             else:
@@ -194,6 +198,6 @@ class DecoderModel:
                 self.watch(run, x if self.streams == 1 else x.view(x.shape[0], self.streams, -1).sum(dim=1))
         if step.n_selected == 0:
             return torch.empty((0, self.config.vocab), dtype=torch.float32, device=self.device)
-        xs = self.final_norm.forward(x, rows=step.selected) if self.streams == 1 else \
-            self.final_norm.forward(x, rows=step.selected, read=self.streams_sum)
+        xs = self.final_norm.forward(x, rows=selected) if self.streams == 1 else \
+            self.final_norm.forward(x, rows=selected, read=self.streams_sum)
         return ops.gemm(xs, self.lm_head, out_dtype=torch.float32, exact=self.build.exact)

@@ -20,6 +20,8 @@ from .base import BuildContext, Part, pad_rows, part_factory, register_part
 
 
 class TableMoe(Part):
+    rows_alone = True  # a row's output depends on that row and its token alone
+
     def __init__(self, spec: TableMoeSpec, prefix: str, build: BuildContext):
         if not 0 < spec.top <= spec.experts:
             raise ValueError(f"{prefix}: top {spec.top} of {spec.experts} experts")
@@ -103,6 +105,8 @@ class RoutedMoe(Part):
     table-routed one with the step's own table: ``ops.moe_route`` groups the assignments by expert, the grouped products
     run gate/up and down, ``ops.moe_combine`` takes the weighted sum into the residual. Nothing waits for the GPU, so a
     decode step with this feed-forward can be captured."""
+
+    rows_alone = True  # a row's output depends on that row and its token alone
 
     def __init__(self, spec: RoutedMoeSpec, prefix: str, build: BuildContext):
         if not 0 < spec.top <= spec.experts or spec.experts % spec.groups or not 0 < spec.keep <= spec.groups \

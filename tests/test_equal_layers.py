@@ -87,7 +87,7 @@ def test_the_launches_and_what_they_read_are_those_of_every_layer_by_itself(monk
     """For prompts, single rows and both, one layer beyond the least up to several, an even and an odd number of layers between: the
     same entry points with the same numbers, every address in the same tensor of the same layer or where the same earlier call wrote."""
     held = []
-    monkeypatch.setattr(recorded, "tensor", lambda *shape, dtype=torch.bfloat16: held.append(torch.empty(shape, dtype=dtype)) or held[-1])
+    monkeypatch.setattr(recorded, "tensor", lambda *shape, dtype=torch.bfloat16: held.append(torch.zeros(shape, dtype=dtype)) or held[-1])
     monkeypatch.setattr(recorded, "DecoderModel", lambda config, dtype, device, positions: DecoderModel(config, dtype, "cpu", positions))
     m = recorded.model(1024, 4, 2, 512, layers=layers, dtype=dtype)
     library = Library()
