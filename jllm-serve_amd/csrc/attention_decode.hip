@@ -38,6 +38,7 @@
 
 #define DA_MAX_SPLIT 2048  // keys per split: a power of two up to this, chosen by the caller
 #define DA_WAVES 4
+#define DA_WHOLE 384  // rows of up to so many keys are one range
 #define DA_U 4  // keys per group and turn; the packed weighted sum below is written for exactly four
 
 // a.lo * b.lo + a.hi * b.hi + c with a, b holding two bf16 each (v_dot2_f32_bf16: exact products, fp32 sum)
@@ -499,6 +500,13 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(G
   }
 }
 
+// for what lies in LDS alone: loads from memory stay on their way
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // The same for head_dim 128 with the scores on the matrix cores. A wave takes 16 consecutive keys per turn (the
 // workgroup 64): S^T[key][head] = K Q^T is four v_mfma_f32_16x16x32_bf16 with K straight from the cache as the A
 // operand (lane l: key l%16, dims 32 j + (l/16) 8 .. + 8) and Q as the B operand (column = head; columns beyond G
@@ -511,48 +519,98 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(G
 // receives dim i of the group's four keys). One running maximum per head serves all four key groups of a wave; it
 // moves only when a turn's maximum exceeds it by more than 2^8, so the accumulators are rarely rescaled.
 //
-// A step of few rows is one chain of latencies: position and table, then q and the new key, then the first keys, then the
-// products. So position, request and slot are asked for together, the new key is another wave's work than q, and its
-// readers take it from LDS, so that nobody waits for its store. Whole steps, before and after: 300 keys of
-// the 0.6B shape 1,106 -> 1,089 to 1,096 us, one request of 2,048 keys (8B) 3,562 -> 3,544; eight of 900 to 2,500 keys (8B, 20.1
-// / 20.4 us a layer), 64 of up to 1,000 and four of 6,100 to 8,000 (4B) as before, within what two runs of one side differ (0.7
-// to 1.6 %). The first keys straight through the table, before q is prepared, were slower (300 keys of the 0.6B shape 1,089
-// -> 1,104).
+// A step of few rows is one chain of latencies, about 6 us of a launch however short the rows are: the launch and its arguments,
+// then all that needs only those (position, request and slot; the table entries, as if the row were the request of its number;
+// q, the new key and value, their gains), then the first keys, while q and the new key are prepared by a wave each (the new
+// key's readers take it from LDS, so that nobody waits for its store), then the products and the meeting of the waves, in which
+// each sums a quarter of the dims. Rows of up to DA_WHOLE keys are one range: handing a part through memory and counting its
+// arrival costs 1.7 us, the further turns 0.35 each. 12 layers of a decode step, before and after: 300 keys of the 0.6B shape 446
+// -> 422 us (of it 12 from the one range), 500 keys 451 -> 436, 1,200 keys 451 -> 436; 300 keys of the 8B 1,223 -> 1,190, eight
+// of 900 1,357 -> 1,308, 64 of 500 1,967 -> 1,930; four of 7,000 (4B) 1,108 -> 1,087. DA_WHOLE by the sweep: 300 keys 446.6 us
+// cut against 434.2 whole, 350 keys 447.3 / 440.1, 400 keys 444.8 / 445.4, 500 keys 451.0 / 461.7.
 template <int G, bool FUSED>
 __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, 3))) void decode_attention_mfma_kernel(
-    const bf16_t* q, int ldq, const bf16_t* kc, const bf16_t* vc, const int* __restrict__ block_table, int max_blocks,
-    const int* __restrict__ row_req, const int* __restrict__ positions, int Hkv, int page_size, int window, float scale,
-    float* part_acc, float* part_ml, int max_splits, int split, bf16_t* out, int ldo, DecodeFusion fu) {
+    const int* __restrict__ positions, const int* __restrict__ row_req, const int* __restrict__ block_table, int max_blocks,
+    int table_rows, const bf16_t* q, int ldq, int split, int page_size, int window, const bf16_t* kc, const bf16_t* vc, int Hkv,
+    float scale, float* part_acc, float* part_ml, int max_splits, int whole_keys, bf16_t* out, int ldo, DecodeFusion fu) {
   constexpr int hd = 128, LPK = 16;
   constexpr int VLD = hd + 16;  // row stride of the V copy: 72 words, so the 16 rows of a transposing load spread over the banks
   __shared__ int tb[DA_MAX_SPLIT + 4];
-  // the waves' copies of a turn's values during the loop; afterwards, per lane of the waves 1..: maximum, sum, 32 accumulators
-  constexpr int VS_BYTES = DA_WAVES * 16 * VLD * 2, MRG_BYTES = (DA_WAVES - 1) * 64 * 34 * 4;
+  // the waves' copies of a turn's values during the loop; afterwards every wave's accumulators, and per head its maximum and sum
+  constexpr int VS_BYTES = DA_WAVES * 16 * VLD * 2, MRG_BYTES = DA_WAVES * 8 * 64 * 16;
   __shared__ __align__(16) unsigned char pool[VS_BYTES > MRG_BYTES ? VS_BYTES : MRG_BYTES];
-  float (*mrg)[64][34] = (float (*)[64][34])pool;
+  floatx4 (*mrg)[8][64] = (floatx4 (*)[8][64])pool;
+  __shared__ float ml[DA_WAVES][2][16];
   __shared__ __align__(16) bf16_t qs[G][hd];  // fused form: q after norm and rotation, to be read as the B operand
   __shared__ __align__(16) bf16_t new_kv[2][hd];  // fused form: the new token's key and value
   const int t = blockIdx.x;
   const int kvh = blockIdx.y;
   const int s = blockIdx.z;
-  // requested together; the compiler would otherwise ask for what follows the return only behind it
-  const int pos = positions[t], req = row_req[t];
-  const int slot = FUSED && fu.write_kv ? fu.slots[t] : -1;
-  asm volatile("" ::"s"(pos), "s"(req), "s"(slot));
-  const int first = window > 0 ? max(0, pos + 1 - window) : 0;
-  const int s_lo = first / split, s_hi = pos / split;
-  if (s < s_lo || s > s_hi) return;
-  const int kb = max(first, s * split);
-  const int ke = min(pos, s * split + split - 1);
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = lane & 15, q4 = lane >> 4;
   const int H = Hkv * G;
-  const int* tbl = block_table + (size_t)req * max_blocks;
   const int psh = __builtin_ctz(page_size);  // pages hold a power of two of positions: shifts, not divisions
+  // Everything that does not depend on the row's position is requested together with it: the table entries of the range as they
+  // lie where a row is the request of its number and no window moves the start (else they are read again), the fused form's q,
+  // new key and value and their gains.
+  const int b_ahead = (s * split) >> psh;
+  const int req_ahead = min(t, table_rows - 1);
+  const int entry = block_table[(size_t)req_ahead * max_blocks + min(b_ahead + (int)threadIdx.x, max_blocks - 1)];
+  const bf16_t* qrow = q + (size_t)t * ldq + (size_t)kvh * G * hd;
+  constexpr int QV = (G + 3) / 4, RAW = 2;
+  uint4 raw[RAW];  // wave 0: the heads q4, q4 + 4, ..; wave 1: the new key, the new value; 8 dims a lane
+  uint4 gain_raw[2];
+  const int d0 = sub * 8;
+  const void* gains = wave == 0 ? fu.gq : fu.gk;
+  if (FUSED && wave < 2) {
+    const bf16_t* kin = q + (size_t)t * ldq + (size_t)(H + kvh) * hd + d0;
+#pragma unroll
+    for (int i = 0; i < RAW; ++i) {
+      const bf16_t* at = wave == 0 ? qrow + (size_t)min(q4 + 4 * i, G - 1) * hd + d0 : kin + (i ? (size_t)Hkv * hd : 0);
+      raw[i] = *(const uint4*)at;
+    }
+    // the bytes of the gains of 8 dims: 16 of bf16 (read twice), 32 of float32
+    const uint4* at = (const uint4*)(gains ? gains : (const void*)q) + (fu.gain_dtype == JLLM_BF16 ? sub : 2 * sub);
+    gain_raw[0] = at[0];
+    gain_raw[1] = at[fu.gain_dtype == JLLM_BF16 ? 0 : 1];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const int pos = positions[t], req = row_req[t];
+  const int slot_at = FUSED ? (fu.write_kv ? fu.slots : positions)[t] : -1;
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::"s"(pos), "s"(req), "s"(slot_at));
+  const int slot = FUSED && fu.write_kv ? slot_at : -1;
+  const int first = window > 0 ? max(0, pos + 1 - window) : 0;
+  // a short row is one range, whatever the launch was cut into: no way through memory to merge it
+  const bool whole = pos - first < whole_keys;
+  const int ssh = __builtin_ctz(split);  // and so is a range's length
+  const int s_lo = whole ? 0 : first >> ssh, s_hi = whole ? 0 : pos >> ssh;
+  if (s < s_lo || s > s_hi) return;
+  asm volatile("" ::"v"(entry));  // waited for here, where all that is on its way was requested with it
+  const int kb = whole ? first : max(first, s * split);
+  const int ke = whole ? pos : min(pos, s * split + split - 1);
   const int b0 = kb >> psh;
   const int nb = (ke >> psh) - b0 + 1;
-  for (int i = threadIdx.x; i < nb; i += DA_WAVES * 64) tb[i] = tbl[b0 + i];
+  const bool has_new = slot >= 0 && s == s_hi;
+  if (req != req_ahead || b0 != b_ahead || nb > DA_WAVES * 64) {
+    const int* tbl = block_table + (size_t)req * max_blocks;
+    for (int i = threadIdx.x; i < nb; i += DA_WAVES * 64) tb[i] = tbl[b0 + i];
+  } else if ((int)threadIdx.x < nb) {
+    tb[threadIdx.x] = entry;
+  }
+  LaneAngles an;
+  const bool rotate = FUSED && fu.cos_t != nullptr;
+  if (FUSED && wave < 2) {
+    const int half = fu.rot >> 1;
+    an.low = rotate && d0 < half;
+    an.high = rotate && d0 >= half && d0 < fu.rot;
+    an.src = lane + (an.low ? (half >> 3) : an.high ? -(half >> 3) : 0);
+    // (lanes without a rotation read something else: a branch around the loads would wait for them where it ends)
+    const size_t at = an.low || an.high ? (size_t)pos * half + (an.low ? d0 : d0 - half) : 0;
+    load8(rotate ? (const void*)fu.cos_t : q, JLLM_F32, at, an.c);
+    load8(rotate ? (const void*)fu.sin_t : q, JLLM_F32, at, an.s);
+  }
   // a turn: keys k0 .. k0 + 15 of this wave. K for the scores: key k0 + sub, dims 32 j + 8 q4; V for the sums: key
   // k0 + 4 q4 + u, dims 8 sub. The next turn's are requested before this turn's are used.
   struct Turn {
@@ -587,7 +645,6 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
   };
   // The token that is only now stored is the range's last key (and stands in for those beyond). Whatever lies in its place is
   // read with the others and replaced here by what wave 1 left in LDS.
-  const bool has_new = slot >= 0 && s == s_hi;
   auto with_new = [&](int k0, Turn& tn) {
     if (!has_new || k0 + 15 < ke) return;
     if (k0 + sub >= ke) {
@@ -600,58 +657,49 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
   };
   const int k_first = kb + wave * 16;
   Turn ta, tb2;
-  const bf16_t* qrow = q + (size_t)t * ldq + (size_t)kvh * G * hd;
   u32x4 qf[4];  // B operand: head `sub`, dims 32 j + 8 q4 .. + 8
-  if (FUSED) {
-    // wave 0 prepares q: lane group q4 takes heads q4, q4 + 4, ..; norm and rotation in the 8-dims-per-lane layout. Wave 1 of
-    // the last split prepares the new key meanwhile.
-    const bool rotate = fu.cos_t != nullptr;
-    const bool stores = wave == 1 && has_new;
-    if (wave == 0 || stores) {
-      LaneAngles an;
-      float gain[8];
-      const int d0 = sub * 8, half = fu.rot >> 1;
-      an.low = rotate && d0 < half;
-      an.high = rotate && d0 >= half && d0 < fu.rot;
-      an.src = lane + (an.low ? (half >> 3) : an.high ? -(half >> 3) : 0);
-      if (an.low || an.high) {
-        const size_t at = (size_t)pos * half + (an.low ? d0 : d0 - half);
-        load8(fu.cos_t, JLLM_F32, at, an.c);
-        load8(fu.sin_t, JLLM_F32, at, an.s);
-      }
-      if (wave == 0) {
-        if (fu.gq) load8(fu.gq, fu.gain_dtype, d0, gain);
-#pragma unroll
-        for (int g0 = 0; g0 < G; g0 += 4) {
-          const int g = g0 + q4;
-          uint4 v = uint4{0u, 0u, 0u, 0u};
-          if (g < G) v = *(const uint4*)(qrow + (size_t)g * hd + d0);
-          float x[8];
-          unpack8(v, x);
-          norm_rope8<LPK>(x, gain, fu.gq != nullptr, an, rotate, fu.eps, hd, true);
-          if (g < G) *(uint4*)(&qs[g][d0]) = uint4{pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
-        }
-      } else if (q4 == 0) {
-        const int page = slot >> psh;
-        const size_t dst = ((((size_t)page * Hkv + kvh) << psh) + (slot & (page_size - 1))) * hd + d0;
-        const bf16_t* kin = q + (size_t)t * ldq + (size_t)(H + kvh) * hd + d0;
-        const uint4 kv_ = *(const uint4*)kin;
-        const uint4 vv = *(const uint4*)(kin + (size_t)Hkv * hd);
-        if (fu.gk) load8(fu.gk, fu.gain_dtype, d0, gain);
-        float x[8];
-        unpack8(kv_, x);
-        norm_rope8<LPK>(x, gain, fu.gk != nullptr, an, rotate, fu.eps, hd, true);
-        const uint4 kn = uint4{pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
-        *(uint4*)(&new_kv[0][d0]) = kn;
-        *(uint4*)(&new_kv[1][d0]) = vv;
-        *(uint4*)(fu.kc_w + dst) = kn;
-        *(uint4*)(fu.vc_w + dst) = vv;
-      }
-    }
-  } else {
+  if (!FUSED) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       qf[j] = sub < G ? *(const u32x4*)(qrow + (size_t)sub * hd + j * 32 + q4 * 8) : u32x4{0u, 0u, 0u, 0u};
+  }
+  lds_barrier();  // the table is there
+  fetch(k_first, ta);
+  if (FUSED) {
+    // while the first keys are on their way wave 0 prepares q: lane group q4 takes heads q4, q4 + 4, ..; norm and rotation in the
+    // 8-dims-per-lane layout. Wave 1 of the last range prepares the new key meanwhile.
+    float gain[8];
+    if (wave < 2 && gains) {
+      if (fu.gain_dtype == JLLM_BF16) {
+        unpack8(gain_raw[0], gain);
+      } else {
+        gain[0] = __uint_as_float(gain_raw[0].x), gain[1] = __uint_as_float(gain_raw[0].y);
+        gain[2] = __uint_as_float(gain_raw[0].z), gain[3] = __uint_as_float(gain_raw[0].w);
+        gain[4] = __uint_as_float(gain_raw[1].x), gain[5] = __uint_as_float(gain_raw[1].y);
+        gain[6] = __uint_as_float(gain_raw[1].z), gain[7] = __uint_as_float(gain_raw[1].w);
+      }
+    }
+    if (wave == 0) {
+#pragma unroll
+      for (int i = 0; i < QV; ++i) {
+        const int g = q4 + 4 * i;
+        float x[8];
+        unpack8(raw[i], x);
+        norm_rope8<LPK>(x, gain, fu.gq != nullptr, an, rotate, fu.eps, hd, true);
+        if (g < G) *(uint4*)(&qs[g][d0]) = uint4{pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
+      }
+    } else if (wave == 1 && has_new && q4 == 0) {
+      const int page = slot >> psh;
+      const size_t dst = ((((size_t)page * Hkv + kvh) << psh) + (slot & (page_size - 1))) * hd + d0;
+      float x[8];
+      unpack8(raw[0], x);
+      norm_rope8<LPK>(x, gain, fu.gk != nullptr, an, rotate, fu.eps, hd, true);
+      const uint4 kn = uint4{pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
+      *(uint4*)(&new_kv[0][d0]) = kn;
+      *(uint4*)(&new_kv[1][d0]) = raw[1];
+      *(uint4*)(fu.kc_w + dst) = kn;
+      *(uint4*)(fu.vc_w + dst) = raw[1];
+    }
   }
   floatx4 acc[8];  // O^T: dims 16 j + 4 q4 .. + 3 of head `sub`
 #pragma unroll
@@ -659,9 +707,8 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
   float m1 = -INFINITY, l1 = 0.f;  // of head `sub`: the wave's running maximum, and the sum over this lane's key group
   bf16_t* vw = (bf16_t*)pool + wave * 16 * VLD;
   const bf16_t* v_tr = vw + (4 * q4 + (sub >> 2)) * VLD + 4 * (sub & 3);  // what this lane names in a transposing load
-  __syncthreads();
-  fetch(k_first, ta);
   if (FUSED) {
+    lds_barrier();
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       qf[j] = sub < G ? *(const u32x4*)(&qs[sub < G ? sub : 0][j * 32 + q4 * 8]) : u32x4{0u, 0u, 0u, 0u};
@@ -710,68 +757,55 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
     with_new(k0 + DA_WAVES * 16, tb2);
     turn(k0 + DA_WAVES * 16, tb2);
   }
-  // the sum over the four key groups; then the waves merge, in order, through LDS
+  // the sum over the four key groups; then the waves meet in LDS, and each merges its share of the dims
   l1 += __shfl_xor(l1, 16, 64);
   l1 += __shfl_xor(l1, 32, 64);
   __syncthreads();  // every wave is done with its copy of the values: the memory now carries the merge
-  if (wave > 0) {
-    float* dst = &mrg[wave - 1][lane][0];
-    dst[0] = m1;
-    dst[1] = l1;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dst[2 + 4 * j + i] = acc[j][i];
-  }
+  for (int j = 0; j < 8; ++j) mrg[wave][j][lane] = acc[j];
+  if (q4 == 0) ml[wave][0][sub] = m1, ml[wave][1][sub] = l1;
   __syncthreads();
   const bool single = s_lo == s_hi;
   const bool merges = FUSED && fu.arrivals && !single;
-  if (wave == 0 && sub < G) {
+  if (sub < G) {
+    float mw[DA_WAVES], l = 0.f, m = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < DA_WAVES - 1; ++w) {
-      const float* src = &mrg[w][lane][0];
-      const float om = src[0], ol = src[1];
-      const float mn = fmaxf(m1, om);
-      const float a = exp2_diff(m1, mn), b = exp2_diff(om, mn);
-      l1 = l1 * a + ol * b;
+    for (int w = 0; w < DA_WAVES; ++w) mw[w] = ml[w][0][sub], m = fmaxf(m, mw[w]);
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[j][i] = acc[j][i] * a + src[2 + 4 * j + i] * b;
-      m1 = mn;
-    }
+    for (int w = 0; w < DA_WAVES; ++w) mw[w] = exp2_diff(mw[w], m), l += ml[w][1][sub] * mw[w];
     const int h = kvh * G + sub;
-    if (single) {
-      const float inv = 1.0f / l1;
-      bf16_t* o = out + (size_t)t * ldo + (size_t)h * hd + 4 * q4;
+    const size_t pi = ((size_t)t * H + h) * max_splits + s;
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        *(u32x2*)(o + 16 * j) = u32x2{pack2(acc[j][0] * inv, acc[j][1] * inv), pack2(acc[j][2] * inv, acc[j][3] * inv)};
-    } else {
-      const size_t pi = ((size_t)t * H + h) * max_splits + s;
-      float* pa = part_acc + pi * hd + 4 * q4;
-      if (merges) {
+    for (int j = wave; j < 8; j += DA_WAVES) {
+      floatx4 v = mrg[0][j][lane] * mw[0];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          store_shared2(pa + 16 * j, acc[j][0], acc[j][1]);
-          store_shared2(pa + 16 * j + 2, acc[j][2], acc[j][3]);
-        }
-        if (q4 == 0) store_shared2(part_ml + pi * 2, m1, l1);
+      for (int w = 1; w < DA_WAVES; ++w) v += mrg[w][j][lane] * mw[w];
+      if (single) {
+        const float inv = 1.0f / l;
+        *(u32x2*)(out + (size_t)t * ldo + (size_t)h * hd + 16 * j + 4 * q4) = u32x2{pack2(v[0] * inv, v[1] * inv), pack2(v[2] * inv, v[3] * inv)};
+      } else if (merges) {
+        float* pa = part_acc + pi * hd + 16 * j + 4 * q4;
+        store_shared2(pa, v[0], v[1]);
+        store_shared2(pa + 2, v[2], v[3]);
       } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) *(floatx4*)(pa + 16 * j) = acc[j];
-        if (q4 == 0) {
-          part_ml[pi * 2] = m1;
-          part_ml[pi * 2 + 1] = l1;
-        }
+        *(floatx4*)(part_acc + pi * hd + 16 * j + 4 * q4) = v;
+      }
+    }
+    if (!single && wave == 0 && q4 == 0) {
+      if (merges) {
+        store_shared2(part_ml + pi * 2, m, l);
+      } else {
+        part_ml[pi * 2] = m;
+        part_ml[pi * 2 + 1] = l;
       }
     }
   }
   if (!merges) return;
   // the workgroup of this row and kv head that arrives last merges the splits, a wave per query head
   __shared__ int last;
+  shared_stores_done();
+  __syncthreads();
   if (wave == 0) {
-    shared_stores_done();
     if (lane == 0) last = arrived_last(fu.arrivals + (size_t)t * Hkv + kvh, s_hi - s_lo + 1);
   }
   __syncthreads();
@@ -786,14 +820,14 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
 __global__ __launch_bounds__(64) void decode_attention_combine_kernel(const float* __restrict__ part_acc,
                                                                       const float* __restrict__ part_ml,
                                                                       const int* __restrict__ positions, int H, int hd,
-                                                                      int window, int max_splits, int split,
+                                                                      int window, int max_splits, int split, int whole,
                                                                       bf16_t* __restrict__ out, int ldo) {
   const int t = blockIdx.x;
   const int h = blockIdx.y;
   const int pos = positions[t];
   const int first = window > 0 ? max(0, pos + 1 - window) : 0;
   const int s_lo = first / split, s_hi = pos / split;
-  if (s_lo == s_hi) return;
+  if (s_lo == s_hi || pos - first < whole) return;
   combine_head(part_acc, part_ml, ((size_t)t * H + h) * max_splits, s_lo, s_hi, hd, out + (size_t)t * ldo + (size_t)h * hd,
                threadIdx.x);
 }
@@ -817,8 +851,8 @@ static int launch_decode(int G, dim3 grid, hipStream_t st, const bf16_t* q, int 
 
 template <bool FUSED>
 static int decode_attention(const void* q, int ldq, void* out, int ldo, const void* kcache, const void* vcache,
-                            const int* block_table, int max_blocks, const int* row_req, const int* positions, int n_rows,
-                            int H, int Hkv, int hd, int page_size, int window, float scale, int max_pos, float* part_acc,
+                            const int* block_table, int max_blocks, int table_rows, const int* row_req, const int* positions,
+                            int n_rows, int H, int Hkv, int hd, int page_size, int window, float scale, int max_pos, float* part_acc,
                             float* part_ml, int max_splits, int split, const DecodeFusion& fu, hipStream_t stream) {
   if (n_rows <= 0) return 0;
   if (Hkv <= 0 || H % Hkv != 0) JLLM_FAIL("decode attention: %d query heads over %d kv heads", H, Hkv);
@@ -833,6 +867,7 @@ static int decode_attention(const void* q, int ldq, void* out, int ldo, const vo
   while (lpk * 8 < hd) lpk <<= 1;
   const int used = max_pos / split + 1;
   dim3 grid(n_rows, Hkv, used);
+  const int whole_keys = hd == 128 ? DA_WHOLE : 0;
   int rc;
 #define DA_ARGS G, grid, stream, (const bf16_t*)q, ldq, (const bf16_t*)kcache, (const bf16_t*)vcache, block_table,    \
                 max_blocks, row_req, positions, Hkv, hd, page_size, window, scale * 1.4426950408889634f, part_acc,  \
@@ -841,8 +876,9 @@ static int decode_attention(const void* q, int ldq, void* out, int ldo, const vo
 #define DA_MCASE(GG)                                                                                                    \
   case GG:                                                                                                              \
     decode_attention_mfma_kernel<GG, FUSED><<<grid, DA_WAVES * 64, 0, stream>>>(                                        \
-        (const bf16_t*)q, ldq, (const bf16_t*)kcache, (const bf16_t*)vcache, block_table, max_blocks, row_req, positions, \
-        Hkv, page_size, window, scale * 1.4426950408889634f, part_acc, part_ml, max_splits, split, (bf16_t*)out, ldo, fu); \
+        positions, row_req, block_table, max_blocks, table_rows, (const bf16_t*)q, ldq, split, page_size, window,        \
+        (const bf16_t*)kcache, (const bf16_t*)vcache, Hkv, scale * 1.4426950408889634f, part_acc, part_ml, max_splits,   \
+        whole_keys, (bf16_t*)out, ldo, fu);                                                                              \
     break;
     switch (G) {
       DA_MCASE(1) DA_MCASE(2) DA_MCASE(3) DA_MCASE(4) DA_MCASE(5) DA_MCASE(6) DA_MCASE(7) DA_MCASE(8)
@@ -863,7 +899,7 @@ static int decode_attention(const void* q, int ldq, void* out, int ldo, const vo
   if (used > 1 && !(hd == 128 && fu.arrivals)) {
     dim3 cg(n_rows, H);
     decode_attention_combine_kernel<<<cg, 64, 0, stream>>>(part_acc, part_ml, positions, H, hd, window, max_splits, split,
-                                                           (bf16_t*)out, ldo);
+                                                           whole_keys, (bf16_t*)out, ldo);
     JLLM_CHECK_LAUNCH("decode_attention_combine");
   }
   return 0;
@@ -877,7 +913,7 @@ extern "C" int jllm_decode_attention_bf16(const void* q, int ldq, void* out, int
                                           const int* row_req, const int* positions, int n_rows, int H, int Hkv, int hd,
                                           int page_size, int window, float scale, int max_pos, float* part_acc,
                                           float* part_ml, int max_splits, int split, hipStream_t stream) {
-  return decode_attention<false>(q, ldq, out, ldo, kcache, vcache, block_table, max_blocks, row_req, positions, n_rows, H,
+  return decode_attention<false>(q, ldq, out, ldo, kcache, vcache, block_table, max_blocks, 1, row_req, positions, n_rows, H,
                                  Hkv, hd, page_size, window, scale, max_pos, part_acc, part_ml, max_splits, split,
                                  DecodeFusion{}, stream);
 }
@@ -887,7 +923,7 @@ extern "C" int jllm_decode_attention_bf16(const void* q, int ldq, void* out, int
 // attention over the pages, merge of the splits. `arrivals` [rows][kv heads], all zero and left so: head size 128 merges in the
 // same launch (null: in a second one); used by one launch at a time.
 extern "C" int jllm_decode_attention_fused_bf16(const void* qkv, int ldqkv, void* out, int ldo, void* kcache,
-                                                void* vcache, const int* block_table, int max_blocks,
+                                                void* vcache, const int* block_table, int max_blocks, int table_rows,
                                                 const int* row_req, const int* positions, const int* slots,
                                                 const float* cos_t, const float* sin_t, const void* gq, const void* gk,
                                                 int gain_dtype, float eps, int rot, int write_kv, int n_rows, int H,
@@ -901,7 +937,7 @@ extern "C" int jllm_decode_attention_fused_bf16(const void* qkv, int ldqkv, void
   if (write_kv && !slots) JLLM_FAIL("decode attention: cache write without slots");
   if (((uintptr_t)gq & 15) || ((uintptr_t)gk & 15)) return 1;
   DecodeFusion fu{slots, cos_t, sin_t, gq, gk, gain_dtype, eps, rot, write_kv, (bf16_t*)kcache, (bf16_t*)vcache, arrivals};
-  return decode_attention<true>(qkv, ldqkv, out, ldo, kcache, vcache, block_table, max_blocks, row_req, positions, n_rows,
+  return decode_attention<true>(qkv, ldqkv, out, ldo, kcache, vcache, block_table, max_blocks, table_rows, row_req, positions, n_rows,
                                 H, Hkv, hd, page_size, window, scale, max_pos, part_acc, part_ml, max_splits, split, fu,
                                 stream);
 }
@@ -950,7 +986,7 @@ extern "C" int jllm_decode_attention_bf16_no_alloc(const void* q, int ldq, void*
               n_rows, H, max_splits, hd, need, (unsigned)JLLM_NO_ALLOC_SCRATCH_FLOATS);
   float* base = nullptr;
   if (scratch_of_current_device(&base) != 0) return -1;
-  return decode_attention<false>(q, ldq, out, ldo, kcache, vcache, block_table, max_blocks, row_req, positions, n_rows, H,
+  return decode_attention<false>(q, ldq, out, ldo, kcache, vcache, block_table, max_blocks, 1, row_req, positions, n_rows, H,
                                  Hkv, hd, page_size, window, scale, max_pos, base, base + acc_floats, (int)max_splits, split,
                                  DecodeFusion{}, stream);
 }

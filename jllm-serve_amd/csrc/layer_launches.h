@@ -34,8 +34,8 @@ int jllm_decode_attention_bf16(const void* q, int ldq, void* out, int ldo, const
         int max_blocks, const int* row_req, const int* positions, int n_rows, int H, int Hkv, int hd, int page_size, int window, float
         scale, int max_pos, float* part_acc, float* part_ml, int max_splits, int split, hipStream_t stream);
 int jllm_decode_attention_fused_bf16(const void* qkv, int ldqkv, void* out, int ldo, void* kcache, void* vcache, const int* block_table, int
-        max_blocks, const int* row_req, const int* positions, const int* slots, const float* cos_t, const float* sin_t, const void* gq,
-        const void* gk, int gain_dtype, float eps, int rot, int write_kv, int n_rows, int H, int Hkv, int hd, int page_size, int window,
+        max_blocks, int table_rows, const int* row_req, const int* positions, const int* slots, const float* cos_t, const float* sin_t,
+        const void* gq, const void* gk, int gain_dtype, float eps, int rot, int write_kv, int n_rows, int H, int Hkv, int hd, int page_size, int window,
         float scale, int max_pos, float* part_acc, float* part_ml, int max_splits, int split, int* arrivals, hipStream_t stream);
 int jllm_prefill_attention_bf16(const void* q, int ldq, void* out, int ldo, const void* kcache, const void* vcache, const int* block_table,
         int max_blocks, const int* tiles, const int* positions, int n_tiles, int n_requests, int H, int Hkv, int hd, int page_size, int

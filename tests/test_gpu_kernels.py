@@ -1130,6 +1130,40 @@ def test_decode_fused(ops, H, Hkv, hd, rot, page, window, gdt):
     assert (again.float() - out3.float()).abs().max() <= 1.2e-2 * max(1.0, float(out3.float().abs().max()))
 
 
+@pytest.mark.parametrize("page", [1, 16])
+@pytest.mark.parametrize("window", [0, 300, 385])
+@pytest.mark.parametrize("order", [(0, 1, 2, 3, 4, 5), (5, 2, 0, 4, 1, 3), (1, 0)])
+def test_decode_rows_of_one_range_and_of_several(ops, page, window, order):
+    """Head size 128 takes rows of up to 384 keys (seen through the window) as one range and cuts longer ones: the rows on both
+    sides of that line in one launch, rows that are the requests of their numbers (whose table entries are asked for ahead) and
+    others, more requests in the table than rows, more entries in a range than threads (pages of one position). The bound: the
+    probabilities that weight the values and the result are rounded to bf16 once each, by 2^-8 of their size at most; the sums
+    are 32-bit (1e-4 covers them and the scores)."""
+    H, Hkv, hd = 8, 2, 128
+    ctx = [384, 385, 1, 383, 1100, 386]
+    R = len(order)
+    kc, vc, table, ks, vs = make_cache(len(ctx), ctx, Hkv, hd, page, torch.bfloat16, seed=page + window)
+    gen = torch.Generator().manual_seed(R)
+    positions = torch.tensor([ctx[r] - 1 for r in order], dtype=torch.int32, device=DEV)
+    row_req = torch.tensor(order, dtype=torch.int32, device=DEV)
+    slots = torch.tensor([int(table[r, (ctx[r] - 1) // page]) * page + (ctx[r] - 1) % page for r in order], dtype=torch.int32, device=DEV)
+    qkv = (torch.randn(R, (H + 2 * Hkv) * hd, generator=gen) * 1.5).bfloat16()
+    plain = ops.paged_attention(qkv[:, :H * hd].to(DEV), kc, vc, table, row_req, positions, H, Hkv, hd, window, hd ** -0.5,
+                                meta={"max_context": max(ctx), "decode_only": True, "requests": R})
+    meta = {"max_context": max(ctx), "decode_only": True, "requests": R, "arrivals": torch.zeros(R * Hkv, dtype=torch.int32, device=DEV)}
+    fused = ops.decode_attention_fused(qkv.to(DEV), kc, vc, table, row_req, positions, slots, None, None, None, None, 1e-6, H, Hkv, hd,
+                                       0, window, hd ** -0.5, meta)
+    for i, r in enumerate(order):
+        q, k, v = qkv[i, :H * hd].view(H, hd), ks[r].clone(), vs[r].clone()
+        for got, name in ((plain, "plain"), (fused, "fused")):
+            if name == "fused":
+                k[-1], v[-1] = qkv[i, H * hd:(H + Hkv) * hd].view(Hkv, hd), qkv[i, (H + Hkv) * hd:].view(Hkv, hd)
+            ref = attention_reference(q, k, v, ctx[r] - 1, H, window, hd ** -0.5)
+            size = attention_reference(q, k, v.abs(), ctx[r] - 1, H, window, hd ** -0.5) + ref.abs()
+            assert bool(((got[i].view(H, hd).cpu().double() - ref).abs() <= 2.0 ** -8 * size + 1e-4).all()), (name, r)
+    assert int(meta["arrivals"].abs().max()) == 0
+
+
 @pytest.mark.parametrize("H,Hkv,ctx,window,split", [(16, 8, (300, 1, 128, 129, 1024), 0, 128), (32, 8, (8000, 17, 5000), 0, 0),
                                                     (5, 1, (9100, 640), 0, 128), (8, 2, (3000, 700, 129), 300, 128), (64, 8, (2500,) * 9, 0, 0)])
 def test_decode_attention_merged_by_its_last_workgroup(ops, monkeypatch, H, Hkv, ctx, window, split):
