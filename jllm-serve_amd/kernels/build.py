@@ -24,6 +24,10 @@ ARCH = "gfx950"
 # packed fp32 VALU forms are switched off for every device compile of this project
 FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
          "-packed-fp32-ops", "-Wno-unused-command-line-argument", "-Wno-unused-result",
+         # a kernel's first arguments (up to 14 words; none of a struct's) are in scalar registers when it starts, not fetched by
+         # it: a step of 300 keys of the 0.6B shape 883.5 -> 876.2 us, one request of 2,048 keys (8B) 3,224 -> 3,205, a prompt of
+         # 487 rows (0.6B) 2,430 -> 2,416; nothing slower
+         "-mllvm", "-amdgpu-kernarg-preload-count=16",
          # the loads that write LDS directly are written out as instructions and name m0 among what they change,
          # which the compiler remarks on at every use
          "-Wno-inline-asm"]
