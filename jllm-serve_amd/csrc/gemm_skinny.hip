@@ -63,6 +63,12 @@ __device__ __forceinline__ float row16_sum(float d) {
   return d;
 }
 
+// one entry of a bf16 or float32 vector as it lies in memory, and its value
+__device__ __forceinline__ uint32_t sk_raw(const void* p, int dtype, int at) {
+  return dtype == JLLM_BF16 ? (uint32_t)((const uint16_t*)p)[at] : ((const uint32_t*)p)[at];
+}
+__device__ __forceinline__ float sk_value(uint32_t raw, int dtype) { return __uint_as_float(dtype == JLLM_BF16 ? raw << 16 : raw); }
+
 // NI loads per block: a ring as deep as the LDS allows, with `per_cu` workgroups on a compute unit
 constexpr int sk_slots(int ni, int waves, int per_cu) {
   const int fit = (160 / per_cu - 1) / (waves * ni);
@@ -82,9 +88,8 @@ __device__ __forceinline__ void sk_wait_block(int behind) {  // `behind` (< S) b
 // NW: loads of 8 weight rows per block (of each weight), NA: of 8 activation rows; TURN: see the host's rule
 template <int NW, int NA, bool GATED, int WAVES, int PER_CU, bool TURN>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
-    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
-    const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N,
-    int K, int epilogue, SkinnyNorm nm, int rows) {
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2, int lda, int M, int N, int K, int rows,
+    int epilogue, const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, SkinnyNorm nm) {
   constexpr int CT = (NW + 1) / 2;                // tiles of 16 weight rows
   constexpr int TILES = GATED ? 2 : CT;           // accumulators: gate and up, or the weight's tiles
   constexpr int NI = (GATED ? 2 : 1) * NW + NA;   // loads of a block
@@ -105,11 +110,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
   const int rot = GATED  ? (int)((blockIdx.x * 14u) % (unsigned)nblk)
                   : TURN ? (int)(blockIdx.x & ((1u << (31 - __builtin_clz((unsigned)nblk))) - 1u))
                          : 0;
-  // wave 0 writes the outputs: what it adds into (the residual, the bias) is requested before anything else
-  float prev[CT][4], b[CT], eg[CT];
+  // Wave 0 writes the outputs: what it adds into (the residual, the bias) is requested before anything else, as it lies in memory
+  // and from rows that are there: a conversion, or a branch of single lanes, waits for its load before the next request goes out,
+  // and wave 0 begins its share of K two latencies behind the others: 0.8 us a launch of the two in each layer that add (a step of
+  // 300 keys of the 0.6B shape 875 -> 831 us, four of 6,100 to 8,000 keys (4B) 3,028 -> 2,970; 8B, whose rows are longer, as before).
+  float prev[CT][4];
+  uint32_t raw_b[CT], raw_eg[CT];
 #pragma unroll
   for (int t = 0; t < CT; ++t) {
-    b[t] = eg[t] = 0.f;
+    raw_b[t] = raw_eg[t] = 0u;
 #pragma unroll
     for (int i = 0; i < 4; ++i) prev[t][i] = 0.f;
   }
@@ -117,25 +126,24 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
 #pragma unroll
     for (int t = 0; t < CT; ++t) {
       const int n = min(n0 + min(t * 16 + col, rows - 1), N - 1);
-      if (bias) b[t] = (bias_dtype == JLLM_BF16) ? ldf((const bf16_t*)bias, n) : ldf((const float*)bias, n);
-      if (nm.emit_rows) eg[t] = (nm.emit_gain_dtype == JLLM_BF16) ? ldf((const bf16_t*)nm.emit_gain, n) : ldf((const float*)nm.emit_gain, n);
+      if (bias) raw_b[t] = sk_raw(bias, bias_dtype, n);
+      if (nm.emit_rows) raw_eg[t] = sk_raw(nm.emit_gain, nm.emit_gain_dtype, n);
       if (epilogue == 1) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (g * 4 + i < M) prev[t][i] = ((const float*)out)[(size_t)(g * 4 + i) * ldo + n];
+        for (int i = 0; i < 4; ++i) prev[t][i] = ((const float*)out)[(size_t)min(g * 4 + i, M - 1) * ldo + n];
       }
     }
   }
   // normed: the sums of squares of the input rows. Every wave takes a share: lane `col` of wave w the four partials
   // 4 (16 w + col) .., requested here and added up behind the products, then those 64 WAVES further on
   floatx4 first[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) first[i] = floatx4{0.f, 0.f, 0.f, 0.f};
   if (nm.norm_partial) {
+    const int p4 = min(wave * 16 + col, (nm.norm_parts >> 2) - 1);
+    first[0] = ((const floatx4*)(nm.norm_partial + (size_t)min(g * 4, M - 1) * nm.norm_parts))[p4];
+    if (M > 1) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (g * 4 + i < M && wave * 16 + col < nm.norm_parts >> 2)
-        first[i] = ((const floatx4*)(nm.norm_partial + (size_t)(g * 4 + i) * nm.norm_parts))[wave * 16 + col];
+      for (int i = 1; i < 4; ++i) first[i] = ((const floatx4*)(nm.norm_partial + (size_t)min(g * 4 + i, M - 1) * nm.norm_parts))[p4];
+    }
   }
   // ---- the loads of a block: a scalar base that advances with the block and a byte offset per lane that never changes
   uint32_t goff[NI];
@@ -204,7 +212,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
   // the four made more rows 1 to 2 % slower)
   if (nm.norm_partial) {
     auto squares = [&](int i) {
-      float t = (first[i][0] + first[i][1]) + (first[i][2] + first[i][3]);
+      float t = wave * 16 + col < nm.norm_parts >> 2 ? (first[i][0] + first[i][1]) + (first[i][2] + first[i][3]) : 0.f;
       if (g * 4 + i < M)
         for (int p4 = (WAVES + wave) * 16 + col; p4 < nm.norm_parts >> 2; p4 += WAVES * 16) {
           const floatx4 v = ((const floatx4*)(nm.norm_partial + (size_t)(g * 4 + i) * nm.norm_parts))[p4];
@@ -242,6 +250,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
     scale(0);
     if (M > 1) scale(1), scale(2), scale(3);
   }
+  float b[CT], eg[CT];
+#pragma unroll
+  for (int t = 0; t < CT; ++t) b[t] = sk_value(raw_b[t], bias_dtype), eg[t] = sk_value(raw_eg[t], nm.emit_gain_dtype);
   float sq[4] = {0.f, 0.f, 0.f, 0.f};  // emit: the squares of the workgroup's columns, per row of this lane
 #pragma unroll
   for (int t = CT - 1; t >= 0; --t) {
@@ -296,7 +307,7 @@ static int launch_skinny(const SkinnyArgs& a, const SkinnyNorm& nm, hipStream_t 
     configured = true;
   }
   gemm_skinny_kernel<NW, NA, GATED, WAVES, PER_CU, TURN><<<(a.N + a.rows - 1) / a.rows, WAVES * 64, smem, stream>>>(
-      a.A, a.lda, a.W, a.W2, a.bias, a.bias_dtype, a.out, a.out_dtype, a.ldo, a.M, a.N, a.K, a.epilogue, nm, a.rows);
+      a.A, a.W, a.W2, a.lda, a.M, a.N, a.K, a.rows, a.epilogue, a.bias, a.bias_dtype, a.out, a.out_dtype, a.ldo, nm);
   JLLM_CHECK_LAUNCH("gemm_skinny");
   return 0;
 }
