@@ -31,6 +31,11 @@ __device__ __forceinline__ bf16_t f32_to_bf16(float f) {
 
 __device__ __forceinline__ float ldf(const float* p, size_t i) { return p[i]; }
 __device__ __forceinline__ float ldf(const bf16_t* p, size_t i) { return bf16_to_f32(p[i]); }
+// an entry of a bf16 or float32 vector as it lies in memory, for requests ahead of their use, and its value
+__device__ __forceinline__ uint32_t raw_entry(const void* p, int dtype, int i) {
+  return dtype == JLLM_BF16 ? (uint32_t)((const uint16_t*)p)[i] : ((const uint32_t*)p)[i];
+}
+__device__ __forceinline__ float raw_value(uint32_t raw, int dtype) { return __uint_as_float(dtype == JLLM_BF16 ? raw << 16 : raw); }
 __device__ __forceinline__ void stf(float* p, size_t i, float v) { p[i] = v; }
 __device__ __forceinline__ void stf(bf16_t* p, size_t i, float v) { p[i] = f32_to_bf16(v); }
 

@@ -63,12 +63,6 @@ __device__ __forceinline__ float row16_sum(float d) {
   return d;
 }
 
-// one entry of a bf16 or float32 vector as it lies in memory, and its value
-__device__ __forceinline__ uint32_t sk_raw(const void* p, int dtype, int at) {
-  return dtype == JLLM_BF16 ? (uint32_t)((const uint16_t*)p)[at] : ((const uint32_t*)p)[at];
-}
-__device__ __forceinline__ float sk_value(uint32_t raw, int dtype) { return __uint_as_float(dtype == JLLM_BF16 ? raw << 16 : raw); }
-
 // NI loads per block: a ring as deep as the LDS allows, with `per_cu` workgroups on a compute unit
 constexpr int sk_slots(int ni, int waves, int per_cu) {
   const int fit = (160 / per_cu - 1) / (waves * ni);
@@ -126,8 +120,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
 #pragma unroll
     for (int t = 0; t < CT; ++t) {
       const int n = min(n0 + min(t * 16 + col, rows - 1), N - 1);
-      if (bias) raw_b[t] = sk_raw(bias, bias_dtype, n);
-      if (nm.emit_rows) raw_eg[t] = sk_raw(nm.emit_gain, nm.emit_gain_dtype, n);
+      if (bias) raw_b[t] = raw_entry(bias, bias_dtype, n);
+      if (nm.emit_rows) raw_eg[t] = raw_entry(nm.emit_gain, nm.emit_gain_dtype, n);
       if (epilogue == 1) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) prev[t][i] = ((const float*)out)[(size_t)min(g * 4 + i, M - 1) * ldo + n];
@@ -252,7 +246,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
   }
   float b[CT], eg[CT];
 #pragma unroll
-  for (int t = 0; t < CT; ++t) b[t] = sk_value(raw_b[t], bias_dtype), eg[t] = sk_value(raw_eg[t], nm.emit_gain_dtype);
+  for (int t = 0; t < CT; ++t) b[t] = raw_value(raw_b[t], bias_dtype), eg[t] = raw_value(raw_eg[t], nm.emit_gain_dtype);
   float sq[4] = {0.f, 0.f, 0.f, 0.f};  // emit: the squares of the workgroup's columns, per row of this lane
 #pragma unroll
   for (int t = CT - 1; t >= 0; --t) {

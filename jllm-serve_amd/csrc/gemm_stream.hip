@@ -100,7 +100,7 @@ constexpr int gs_slots(int ct, int mt, bool shared) {
 }
 
 template <int CT, int MT, bool GATED, bool SHARED>
-__global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
+__global__ __launch_bounds__(CT * 128, SHARED ? CT : 1) void gemm_stream_kernel(StreamArgs p) {
   constexpr int NW = 2 * CT;                // waves
   constexpr int BLOCK = (2 * CT + 2 * MT) * 1024;
   constexpr int S = gs_slots(CT, MT, SHARED);
@@ -142,10 +142,54 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
   // requested before anything else and added up behind the products
   floatx4 first[2];
   const int sq_row = tid / TPR, sq_at = tid % TPR;
-  const floatx4* squares = (const floatx4*)(p.nm.norm_partial + (size_t)sq_row * p.nm.norm_parts);
-  const int fours = p.nm.norm_partial && sq_row < p.M ? p.nm.norm_parts >> 2 : 0;
+  const floatx4* squares = (const floatx4*)(p.nm.norm_partial + (size_t)min(sq_row, p.M - 1) * p.nm.norm_parts);
+  const int fours = p.nm.norm_parts >> 2;
+  if (p.nm.norm_partial) {
 #pragma unroll
-  for (int j = 0; j < 2; ++j) first[j] = sq_at + j * TPR < fours ? squares[sq_at + j * TPR] : floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < 2; ++j) first[j] = squares[min(sq_at + j * TPR, fours - 1)];
+  }
+  // What the epilogue adds into, gains and bias, as they lie in memory, from rows and columns that are there (a branch of lanes
+  // or a conversion would wait for each load): the sums before the first block where this workgroup writes them, else, with the
+  // rest, while it counts its arrival. A step of 64 rows (8B) 5,395 -> 5,347 us against requests where they are used, a prompt of 487 rows
+  // (0.6B) 2,394 -> 2,361.
+  constexpr int IPT = (OT * MT + NW - 1) / NW, MATS = GATED ? 2 : 1;  // a thread's items of four columns of a row
+  const bool vec = (p.ldo & 3) == 0 && ((uintptr_t)p.out & 15) == 0;
+  floatx4 prev[IPT];
+  uint32_t raw_b[IPT][4], raw_eg[IPT][4];
+#pragma unroll
+  for (int it = 0; it < IPT; ++it) prev[it] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto request_sums = [&]() {
+    if (p.epilogue != 1) return;
+#pragma unroll
+    for (int it = 0; it < IPT; ++it) {
+      const int idx = min(tid + it * NW * 64, OT * MT * 64 - 1);
+      const float* o = (const float*)p.out + (size_t)min(((idx >> 6) % MT) * 16 + col, p.M - 1) * p.ldo + min(n0 + (idx >> 6) / MT * 16 + g * 4, p.N - 4);
+      if (vec)
+        prev[it] = *(const floatx4*)o;
+      else
+        prev[it] = floatx4{o[0], o[1], o[2], o[3]};
+    }
+  };
+  auto request_vector = [&](const void* vector, int dtype, uint32_t (&raw)[IPT][4]) {
+    auto entries = [&](auto* v) {
+#pragma unroll
+      for (int it = 0; it < IPT; ++it) {
+        const int n = min(n0 + (min(tid + it * NW * 64, OT * MT * 64 - 1) >> 6) / MT * 16 + g * 4, p.N - 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) raw[it][i] = v[n + i];
+      }
+    };
+    if (dtype == JLLM_BF16)
+      entries((const uint16_t*)vector);
+    else
+      entries((const uint32_t*)vector);
+  };
+  auto request_vectors = [&]() {
+    if (p.nm.emit_rows) request_vector(p.nm.emit_gain, p.nm.emit_gain_dtype, raw_eg);
+    if (p.bias) request_vector(p.bias, p.bias_dtype, raw_b);
+  };
+  constexpr bool AHEAD = GATED || CT < 8 || !SHARED;  // two workgroups of 16 waves: 64 registers a thread, too few for it
+  if (AHEAD && parts == 1) request_sums();
   // ---- the loads of a block: 8 weight rows per wave, and 8 activation rows for as many waves as that takes
   const int lrow = lane >> 3, lslot = lane & 7;
   const int na = (p.M + 7) >> 3;
@@ -213,9 +257,11 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
     gs_wait_at_most((total - 1 - i) * nl);
     block();
   }
+  if (AHEAD && parts == 1) request_vectors();
   if (p.nm.norm_partial) {
-    float t = ((first[0][0] + first[0][1]) + (first[0][2] + first[0][3])) + ((first[1][0] + first[1][1]) + (first[1][2] + first[1][3]));
-    for (int q = sq_at + 2 * TPR; q < fours; q += TPR) {
+    float t = sq_at < fours ? (first[0][0] + first[0][1]) + (first[0][2] + first[0][3]) : 0.f;
+    t += sq_at + TPR < fours ? (first[1][0] + first[1][1]) + (first[1][2] + first[1][3]) : 0.f;
+    for (int q = sq_at + 2 * TPR; q < (sq_row < p.M ? fours : 0); q += TPR) {
       const floatx4 v = squares[q];
       t += (v[0] + v[1]) + (v[2] + v[3]);
     }
@@ -239,30 +285,21 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
       store_shared2(dst + 2, v[2], v[3]);
     }
     shared_stores_done();
+    if (AHEAD) {
+      request_sums();
+      request_vectors();
+    }
     __syncthreads();
     if (tid == 0) last = arrived_last(p.arrivals + tile, parts);
     __syncthreads();
     if (!last) return;
   }
   // a thread's items (64 lanes of a wave: one tile, one tile of rows): everything they read is requested side by side
-  constexpr int IPT = (OT * MT + NW - 1) / NW, MATS = GATED ? 2 : 1;
-  const bool vec = (p.ldo & 3) == 0 && ((uintptr_t)p.out & 15) == 0;
-  floatx4 prev[IPT], sum[IPT][MATS];
+  floatx4 sum[IPT][MATS];
 #pragma unroll
-  for (int it = 0; it < IPT; ++it) {
-    const int idx = tid + it * NW * 64, m = ((idx >> 6) % MT) * 16 + col, n = n0 + (idx >> 6) / MT * 16 + g * 4;
-    prev[it] = floatx4{0.f, 0.f, 0.f, 0.f};
-    if (p.epilogue == 1 && idx < OT * MT * 64 && m < p.M && n < p.N) {
-      const float* o = (const float*)p.out + (size_t)m * p.ldo + n;
-      if (vec)
-        prev[it] = *(const floatx4*)o;
-      else
-#pragma unroll
-        for (int i = 0; i < 4; ++i) prev[it][i] = o[i];
-    }
+  for (int it = 0; it < IPT; ++it)
 #pragma unroll
     for (int u = 0; u < MATS; ++u) sum[it][u] = floatx4{0.f, 0.f, 0.f, 0.f};
-  }
   if (parts == 1) {
 #pragma unroll
     for (int it = 0; it < IPT; ++it)
@@ -281,13 +318,12 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
         for (int it = 0; it < IPT; ++it)
 #pragma unroll
           for (int u = 0; u < MATS; ++u) {
-            const int idx = min(tid + it * NW * 64, OT * MT * 64 - 1) + u * OT * MT * 64;
+            int idx = min(tid + it * NW * 64, OT * MT * 64 - 1) + u * OT * MT * 64;
+            if (((idx >> 6) % MT) * 16 + col >= p.M) idx = 0;  // a row that is not there: any that is
             const float* src = mine + ((size_t)min(z0 + z, parts - 1) * ITEMS + idx) * 4;
-            float x0 = 0.f, x1 = 0.f, x2 = 0.f, x3 = 0.f;
-            if (((idx >> 6) % MT) * 16 + col < p.M) {
-              load_shared2(src, x0, x1);
-              load_shared2(src + 2, x2, x3);
-            }
+            float x0, x1, x2, x3;
+            load_shared2(src, x0, x1);
+            load_shared2(src + 2, x2, x3);
             q[z][it][u] = floatx4{x0, x1, x2, x3};
           }
 #pragma unroll
@@ -299,6 +335,10 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
             for (int u = 0; u < MATS; ++u) sum[it][u] += q[z][it][u];
         }
     }
+  }
+  if (!AHEAD) {
+    request_sums();
+    request_vectors();
   }
 #pragma unroll
   for (int it = 0; it < IPT; ++it) {
@@ -314,7 +354,7 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float x = sum[it][0][i] * scale;
-        if (p.bias) x += (p.bias_dtype == JLLM_BF16) ? ldf((const bf16_t*)p.bias, n + i) : ldf((const float*)p.bias, n + i);
+        if (p.bias) x += raw_value(raw_b[it][i], p.bias_dtype);
         if (GATED) x = gated<false>(x, sum[it][MATS - 1][i] * scale, p.gate);
         r[i] = prev[it][i] + x;
         sq += r[i] * r[i];
@@ -323,7 +363,7 @@ __global__ __launch_bounds__(CT * 128) void gemm_stream_kernel(StreamArgs p) {
         float e[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          e[i] = r[i] * ((p.nm.emit_gain_dtype == JLLM_BF16) ? ldf((const bf16_t*)p.nm.emit_gain, n + i) : ldf((const float*)p.nm.emit_gain, n + i));
+          e[i] = r[i] * raw_value(raw_eg[it][i], p.nm.emit_gain_dtype);
         *(u32x2*)(p.nm.emit_rows + (size_t)m * p.nm.emit_ld + n) = u32x2{pack_bf16(e[0], e[1]), pack_bf16(e[2], e[3])};
       }
       if (p.out_dtype == JLLM_BF16) {
