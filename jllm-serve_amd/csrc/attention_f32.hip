@@ -6,8 +6,8 @@
 // in the order of the waves) and what is one multiply-add are the general kernel's. Cache layout and table as there.
 //
 //  * single rows (decode steps): a workgroup per row and up to four heads of a kv head, a lane per key. The general kernel
-//    waits for a handful of 16-byte loads at a time (three rows of 90 to 400 keys, 16 heads: 52 us, here 16); here a lane requests its whole
-//    key row at once, and a block's values in four groups of 16 keys, each on its way while the one before is used.
+//    waits for a handful of 16-byte loads at a time (three rows of 400 keys, 16 heads: 52 us, here 14, 12 with the keys by way of LDS);
+//    here a lane requests its whole key row at once, and a block's values in four groups of 16 keys, each on its way while the one before is used.
 //  * many rows (portions): a workgroup takes 16 query vectors (rows of one request x the heads of a kv head), so a key is
 //    read once for all of them instead of once per row, and both products run on the matrix cores' fp32 form, whose sums
 //    are chains of multiply-adds in ascending order (see gemm_generic.hip). Three prompts of 847 rows in all, 16 heads over 8:
@@ -15,6 +15,7 @@
 #include <math.h>
 
 #include "common.h"
+#include "lds_ring.h"
 
 #define AF_HD 128
 #define AF_WAVES 4
@@ -37,8 +38,15 @@ __device__ __forceinline__ int cache_row(const AttF32& A, const int* __restrict_
 
 // ---------------------------------------------------------------------------------------------- single rows
 
-template <int GC>
-__global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_rows_kernel(AttF32 A) {
+// STAGED: the keys come by way of LDS. A lane that reads a key's row takes 16 bytes of a line at a time, 64 lines at once: the
+// four waves' 128 KB do not stay in the first-level cache (32 KB) until a line's other pieces are asked for, so each crosses from
+// the L2 several times. In LDS they come once, in whole lines, and the next block's while this one's values are weighted; but a
+// compute unit then holds one workgroup. Registers / LDS, 16 heads over 8: 300 keys 12.1 / 11.2 us, three rows of 400 14.2 /
+// 11.8, of 2,000 56.1 / 41.1, 16 of 1,000 30.6 / 25.6; where there are more workgroups than compute units, 64 of 1,000 93.2 / 94.8
+// and 64 of 100 12.1 / 17.7; one block a wave, 60 keys, 5.6 / 6.5.
+template <int GC, bool STAGED>
+__global__ __launch_bounds__(64 * AF_WAVES, STAGED ? 1 : 2) void attention_f32_rows_kernel(AttF32 A) {
+  extern __shared__ __align__(1024) unsigned char key_rows[];  // STAGED: [AF_WAVES][64 keys][512 bytes]
   __shared__ __align__(16) float qs[GC][AF_HD];
   __shared__ float mg[AF_WAVES][GC][2 + AF_HD];  // every wave's maximum, sum and weighted sums
   const int t = blockIdx.x, lane = threadIdx.x & 63;
@@ -61,14 +69,24 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_rows_kernel(At
   float acc[GC][2], m[GC], l[GC];
 #pragma unroll
   for (int g = 0; g < GC; ++g) m[g] = -INFINITY, l[g] = 0.f, acc[g][0] = acc[g][1] = 0.f;
+  // A block's keys go into the wave's own 32 KB of LDS, two rows (1 KB) a load, piece j (16 bytes) of key k at place j ^ (k % 32):
+  // read back a lane per key, a row apart, neighbouring lanes meet different banks.
+  unsigned char* keys = key_rows + wave * 64 * AF_HD * 4;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)keys;
+  auto request_keys = [&](int row) {
+#pragma unroll
+    for (int c = 0; c < 32; ++c) {
+      const int r0 = __builtin_amdgcn_readlane(row, 2 * c), r1 = __builtin_amdgcn_readlane(row, 2 * c + 1);
+      const int piece = (lane & 31) ^ ((2 * c + (lane >> 5)) & 31);
+      const float* src = A.k + (size_t)(lane < 32 ? r0 : r1) * AF_HD + piece * 4;
+      load_to_lds_16(src, lds0 + c * 1024u);
+    }
+  };
+  if (STAGED && blk * 64 <= pos) request_keys(row);
   for (; blk * 64 <= pos; blk += AF_WAVES) {
     const int c0 = blk * 64, kj = c0 + lane;
     const bool valid = kj >= first && kj <= pos;
-    const floatx4* kr = (const floatx4*)(A.k + (size_t)row * AF_HD);
-    floatx4 kv[AF_HD / 4];
-#pragma unroll
-    for (int i = 0; i < AF_HD / 4; ++i) kv[i] = kr[i];
-    __builtin_amdgcn_sched_barrier(0);
+    const int next = blk + AF_WAVES;
     auto fetch = [&](float (&vv)[16][2], int jb) {
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
@@ -77,26 +95,50 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_rows_kernel(At
         vv[u][1] = vr[lane + 64];
       }
     };
+    const floatx4* kr = (const floatx4*)(A.k + (size_t)row * AF_HD);
+    floatx4 kv[STAGED ? 1 : AF_HD / 4];
+    float va[16][2], vb[16][2];
+    int next_row = row;
+    if constexpr (STAGED) {
+      wait_loads<0>();  // the block's keys
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(va, 0);
+      next_row = row_of(next);
+    } else {
+#pragma unroll
+      for (int i = 0; i < AF_HD / 4; ++i) kv[i] = kr[i];
+    }
+    __builtin_amdgcn_sched_barrier(0);
     float d[GC], p[GC];
 #pragma unroll
     for (int g = 0; g < GC; ++g) d[g] = 0.f;
+    constexpr int AT_ONCE = STAGED ? 8 : 4;  // pieces at a time: all of the queries' (and the keys') LDS reads would take all registers
 #pragma unroll
-    for (int i0 = 0; i0 < AF_HD / 4; i0 += 4) {  // (four at a time: the queries' LDS reads would take all registers)
+    for (int i0 = 0; i0 < AF_HD / 4; i0 += AT_ONCE) {
+      floatx4 part[AT_ONCE];
 #pragma unroll
-      for (int i = i0; i < i0 + 4; ++i)
+      for (int i = 0; i < AT_ONCE; ++i) {
+        if constexpr (STAGED)
+          part[i] = *(const floatx4*)(keys + lane * AF_HD * 4 + (((i0 + i) ^ (lane & 31)) << 4));
+        else
+          part[i] = kv[i0 + i];
+      }
+#pragma unroll
+      for (int i = 0; i < AT_ONCE; ++i)
 #pragma unroll
         for (int g = 0; g < GC; ++g) {
-          const floatx4 qv = *(const floatx4*)&qs[g][4 * i];
+          const floatx4 qv = *(const floatx4*)&qs[g][4 * (i0 + i)];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) d[g] = fmaf(qv[e], kv[i][e], d[g]);
+          for (int e = 0; e < 4; ++e) d[g] = fmaf(qv[e], part[i][e], d[g]);
         }
 #pragma unroll
       for (int g = 0; g < GC; ++g) asm volatile("" : "+v"(d[g]));  // (nor does the chain sink below to where its sum is used)
       __builtin_amdgcn_sched_barrier(0);
     }
-    float va[16][2], vb[16][2];
-    fetch(va, 0);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!STAGED) {
+      fetch(va, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int g = 0; g < GC; ++g) {
 #pragma clang fp contract(off)
@@ -131,8 +173,16 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_rows_kernel(At
     __builtin_amdgcn_sched_barrier(0);
     use(vb, 16);
     fetch(vb, 48);
-    const int next = blk + AF_WAVES;
-    if (next * 64 <= pos) row = row_of(next);
+    if constexpr (STAGED) {
+      // The next keys go out with nothing else on its way: the compiler does not count loads into LDS, and would wait for these
+      // where it waits for values. Every read of the last keys is done, their products are.
+      __builtin_amdgcn_sched_barrier(0);
+      row = next_row;
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+      if (next * 64 <= pos) request_keys(row);
+    } else {
+      if (next * 64 <= pos) row = row_of(next);
+    }
     __builtin_amdgcn_sched_barrier(0);
     use(va, 32);
     use(vb, 48);
@@ -422,13 +472,29 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_tiles_kernel(A
   }
 }
 
+template <int GC, bool STAGED>
+static int launch_rows(const AttF32& A, dim3 grid, hipStream_t stream) {
+  constexpr int smem = STAGED ? AF_WAVES * 64 * AF_HD * 4 : 0;
+  if constexpr (STAGED) {
+    static bool configured = false;
+    if (!configured) {  // above 64 KB the size has to be allowed first
+      if (hipFuncSetAttribute((const void*)attention_f32_rows_kernel<GC, true>, hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess)
+        JLLM_FAIL("attention_f32: cannot reserve %d bytes of LDS", smem);
+      configured = true;
+    }
+  }
+  attention_f32_rows_kernel<GC, STAGED><<<grid, 64 * AF_WAVES, smem, stream>>>(A);
+  JLLM_CHECK_LAUNCH("attention_f32");
+  return 0;
+}
+
 // fp32, head size 128, 16-byte aligned rows; returns 1 for what it leaves to the general kernel. `n_requests` bounds
 // row_req, the block table's width the keys. Which kernel: a tile holds 16 / G rows of one request, and reads their keys
 // once; where the rows are spread over as many requests (steps of single tokens) there is nothing to share and a workgroup
 // per row has more waves. A portion of few rows goes row by row too: a tile's chain is about 12 us for the first 64 keys, a
 // row's 5.5, as long as its workgroups (row x head) are one per compute unit, a few where the keys are few. 16 heads over
 // 8, rows / tiles (the general kernel): 4 rows of a new prompt 5.5 / 11.7 us (6.8), 20 rows 5.9 / 12.1 (10.2), 64 rows 8.4 /
-// 12.3, 96 rows 16.0 / 13.1; 20 rows behind 200 keys 13.2 / 15.1, 40 rows 17.6 / 15.3; 16 rows behind 1,000 keys 31.6 / 39.6,
+// 12.3, 96 rows 16.0 / 13.1; 20 rows behind 200 keys 13.2 / 15.1, 40 rows 17.6 / 15.3; 16 rows behind 1,000 keys 31.6 (25.6 by way of LDS) / 39.6,
 // 20 rows 46.7 / 41.6. Up to 16 keys the general kernel lies between: 64 rows of eight new prompts, 24 heads over 3, 9.8 us,
 // 11.8 by rows, 12.5 by tiles.
 extern "C" int jllm_attention_f32(const void* q, int ldq, void* out, int ldo, const void* kcache, const void* vcache, const int* block_table,
@@ -454,13 +520,15 @@ extern "C" int jllm_attention_f32(const void* q, int ldq, void* out, int ldo, co
       attention_f32_tiles_kernel<true><<<dim3(tiles + n_requests, Hkv), 64 * AF_WAVES, 0, stream>>>(A, rows, n_requests);
     else
       attention_f32_tiles_kernel<false><<<dim3(tiles, Hkv), 64 * AF_WAVES, 0, stream>>>(A, rows, 0);
+  } else if (pairs <= cus && keys > 256) {  // one round of workgroups, more than a block a wave
+    return launch_rows<1, true>(A, dim3(n_tokens, H), stream);
   } else {  // heads share a workgroup where the step still has two workgroups for every compute unit, as in the general kernel
     if (G >= 3 && (long)n_tokens * Hkv * ((G + 3) / 4) >= 2L * cus)
-      attention_f32_rows_kernel<4><<<dim3(n_tokens, Hkv * ((G + 3) / 4)), 64 * AF_WAVES, 0, stream>>>(A);
+      return launch_rows<4, false>(A, dim3(n_tokens, Hkv * ((G + 3) / 4)), stream);
     else if (G >= 2 && (G <= 4 || keys > 64) && (long)n_tokens * Hkv * ((G + 1) / 2) >= 2L * cus)
-      attention_f32_rows_kernel<2><<<dim3(n_tokens, Hkv * ((G + 1) / 2)), 64 * AF_WAVES, 0, stream>>>(A);
+      return launch_rows<2, false>(A, dim3(n_tokens, Hkv * ((G + 1) / 2)), stream);
     else
-      attention_f32_rows_kernel<1><<<dim3(n_tokens, H), 64 * AF_WAVES, 0, stream>>>(A);
+      return launch_rows<1, false>(A, dim3(n_tokens, H), stream);
   }
   JLLM_CHECK_LAUNCH("attention_f32");
   return 0;

@@ -886,6 +886,20 @@ def test_float32_attention_of_rows_in_any_order_gives_the_general_kernels_bits(o
     assert torch.equal(attend(), attend(torch.zeros(H, device=DEV)))
 
 
+@pytest.mark.parametrize("H,Hkv,page,window", [(16, 8, 16, 0), (3, 3, 1, 0), (8, 1, 64, 300), (32, 8, 16, 65)])
+def test_float32_rows_with_their_keys_by_way_of_lds(ops, H, Hkv, page, window):
+    """float32 rows at head size 128 with more than 256 keys in the table and no more workgroups than compute units take their
+    keys by way of LDS: bit for bit the general kernel (here by slopes of zero), at the edges of a wave's blocks and of a window."""
+    lens = [1, 63, 64, 65, 257, 321, 1000]
+    kc, vc, table, _, _ = make_cache(len(lens), lens, Hkv, 128, page, torch.float32, seed=H + page)
+    q = torch.randn(len(lens), H * 128, generator=torch.Generator().manual_seed(H)).to(DEV)
+    req = torch.arange(len(lens), dtype=torch.int32, device=DEV)
+    pos = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    attend = lambda slopes: ops.paged_attention(q, kc, vc, table, req, pos, H, Hkv, 128, window, 128 ** -0.5, exact=True, slopes=slopes)
+    got = attend(None)
+    assert not torch.isnan(got).any() and torch.equal(got, attend(torch.zeros(H, device=DEV)))
+
+
 @pytest.mark.parametrize("H,Hkv,hd,window", [(12, 3, 32, 0), (10, 2, 48, 70), (6, 3, 64, 0), (8, 8, 16, 0)])
 def test_general_attention_gives_a_row_the_same_bits_in_any_step(ops, H, Hkv, hd, window):
     """The general kernel (the 32-bit path) takes up to four query heads of a kv head in one workgroup when the step
