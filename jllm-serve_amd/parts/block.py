@@ -128,8 +128,11 @@ register_part("arrangement", "prenorm", PreNormBlock, replace=True)
 
 def rows_alone(ffn) -> bool:
     """Whether this is a feed-forward (of exactly a class that says so, with its methods) whose output for a row depends on that row
-    and its token alone."""
-    return ffn is not None and bool(type(ffn).__dict__.get("rows_alone")) and not {"forward", "output"} & set(vars(ffn))
+    and its token alone. One that has a shared feed-forward says so of itself: the shared one, of whatever kind, is asked too."""
+    if ffn is None or not type(ffn).__dict__.get("rows_alone") or {"forward", "output"} & set(vars(ffn)):
+        return False
+    shared = getattr(ffn, "shared", None)
+    return shared is None or rows_alone(shared)
 
 
 def selected_step(step):
