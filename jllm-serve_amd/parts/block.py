@@ -21,7 +21,7 @@ import torch
 from ..kernels import ops
 from ..weights.loader import WeightSpec
 from .base import Part, StateShare, part_factory, register_part
-from .equal_layers import own_forward
+from .equal_layers import key_of, own_forward
 from .shift import TokenShift
 
 
@@ -62,11 +62,14 @@ class PreNormBlock(Part):
     def launch_key(self):
         if not own_forward(self, PreNormBlock) or self.ffn is None:
             return None
-        keys = tuple(getattr(p, "launch_key", lambda: None)() for p in self.parts)
+        keys = tuple(key_of(p) for p in self._runs())
         return None if None in keys else keys
 
     def launch_tensors(self):
-        return [t for p in self.parts for t in p.launch_tensors()]
+        return [t for p in self._runs() for t in p.launch_tensors()]
+
+    def _runs(self):  # (what ``forward`` uses now, not what was built)
+        return self.norm_in, self.mixer, self.norm_post, self.ffn
 
     chains_norms = True  # forward takes normed_in / next_norm and returns the next block's input promise
 

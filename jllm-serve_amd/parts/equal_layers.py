@@ -6,9 +6,13 @@ natively from another layer's (``ops.RepeatedLaunches``) it costs 40 in all. So 
 the last, and the launches of the second, the first whose input norm the layer before prepared, are made again for those between.
 
 A part whose launches follow from its sizes and its tensors alone says so: ``launch_key()``, equal for parts that launch alike
-(None: not known), and ``launch_tensors()``, what they differ in, in an order of the part's own. Nothing is kept between steps.
+(None: not known), and ``launch_tensors()``, what they differ in, in an order of the part's own. Nothing is kept between steps: which runs
+may be alike is known when the weights are, but a layer's key is asked for again in every step, since a part may have been given a
+method, a number or a part of its own meanwhile (4 us a layer, while the GPU is at work on the one before).
 """
 from __future__ import annotations
+
+import functools
 
 import torch
 
@@ -31,8 +35,15 @@ def launches(x) -> bool:
     return x.is_cuda and not torch.cuda.is_current_stream_capturing()
 
 
+def key_of(part):
+    """What the part says of its launches now (None: nothing)."""
+    return part.launch_key() if hasattr(part, "launch_key") else None
+
+
 def pays(layer, rows: int) -> bool:
     """Whether the host is what a step of so many rows waits for in such a layer."""
+    if key_of(layer) is None:
+        return False
     us = BESIDE_US
     for t in layer.launch_tensors():
         if t is not None and t.dim() == 2:
@@ -40,9 +51,14 @@ def pays(layer, rows: int) -> bool:
     return us < PYTHON_LAYER_US
 
 
+@functools.lru_cache(maxsize=None)
+def _methods(kind):
+    return frozenset(n for n in dir(kind) if not n.startswith("__") and callable(getattr(kind, n)))
+
+
 def own_forward(part, kind) -> bool:
     """Whether the part is of exactly this class, with its methods."""
-    return type(part) is kind and "forward" not in vars(part)
+    return type(part) is kind and _methods(kind).isdisjoint(vars(part))
 
 
 def equal_runs(schedule, layers):
@@ -50,8 +66,7 @@ def equal_runs(schedule, layers):
     keys = []
     for e in schedule:
         plain = e.cache_from is None and e.add_before is None and e.mix_before is None and not e.add_embedding
-        key = getattr(layers[e.layer], "launch_key", lambda: None)() if plain else None
-        keys.append(key)
+        keys.append(key_of(layers[e.layer]) if plain else None)
     ends = [0] * len(keys)
     for i in range(len(keys) - 1, -1, -1):
         same = i + 1 < len(keys) and keys[i] is not None and keys[i] == keys[i + 1]
@@ -78,7 +93,10 @@ def walk(layers, slots, first, last, x, step, carry, next_norm_of):
     run = first
     carry = layers[run].forward(x, step, slots[run], normed_in=carry, next_norm=next_norm_of(run))
     run += 1
-    norm = next_norm_of(run)
+    norm, key = next_norm_of(run), key_of(layers[run])
+    norm_key = key_of(norm)
+    if key is None or norm_key is None:
+        return run, carry
     own, taken = _tensors(layers[run], slots[run], norm), _carried(carry)
     with ops.kept_launches() as kept:
         left = layers[run].forward(x, step, slots[run], normed_in=carry, next_norm=norm)
@@ -97,6 +115,8 @@ def walk(layers, slots, first, last, x, step, carry, next_norm_of):
     forms, mine = [_form(t) for t in own], slots[run - 1]
     for n, run in enumerate(between):  # (one by one: the GPU is at work on one while the host looks at the next)
         slot, norm = slots[run], next_norm_of(run)
+        if key_of(layers[run]) != key or key_of(norm) != norm_key:
+            return run, carry
         tensors = _tensors(layers[run], slot, norm)
         if (slot.group, slot.writes, slot.page_size) != (mine.group, mine.writes, mine.page_size) or [_form(t) for t in tensors] != forms:
             return run, carry

@@ -1,8 +1,10 @@
 """Layers whose launches are made natively from another layer's: the same launches, over the same data."""
+import copy
 import ctypes
 import os
 import re
 import struct
+import types
 
 import pytest
 import torch
@@ -80,12 +82,9 @@ def data_flow(calls, tensors):
     return seen
 
 
-@pytest.mark.parametrize("layers", [5, 6, 9, 10])
-@pytest.mark.parametrize("dtype,requests", [(torch.bfloat16, [(40, 0)]), (torch.bfloat16, [(487, 0)]), (torch.bfloat16, [(1, 9), (1, 30)]),
-                                            (torch.bfloat16, [(300, 0), (1, 20), (1, 7)]), (torch.float32, [(3, 0)]), (torch.float32, [(100, 0)])])
-def test_the_launches_and_what_they_read_are_those_of_every_layer_by_itself(monkeypatch, layers, dtype, requests):
-    """For prompts, single rows and both, one layer beyond the least up to several, an even and an odd number of layers between: the
-    same entry points with the same numbers, every address in the same tensor of the same layer or where the same earlier call wrote."""
+def stand_ins(monkeypatch, layers, dtype):
+    """A model on the CPU whose launches are noted (every layer of it natively where it may be), its library, and all that was
+    given to a launch (kept, so that no memory is given out twice and an address says which tensor)."""
     held = []
     monkeypatch.setattr(recorded, "tensor", lambda *shape, dtype=torch.bfloat16: held.append(torch.zeros(shape, dtype=dtype)) or held[-1])
     monkeypatch.setattr(recorded, "DecoderModel", lambda config, dtype, device, positions: DecoderModel(config, dtype, "cpu", positions))
@@ -98,7 +97,17 @@ def test_the_launches_and_what_they_read_are_those_of_every_layer_by_itself(monk
     monkeypatch.setattr(equal_layers, "launches", lambda x: True)
     monkeypatch.setattr(equal_layers, "PYTHON_LAYER_US", 1e9)
     real = ops._ptr
-    monkeypatch.setattr(ops, "_ptr", lambda t: held.append(t) or real(t))  # (no memory twice, so that an address says which tensor)
+    monkeypatch.setattr(ops, "_ptr", lambda t: held.append(t) or real(t))
+    return m, library, held
+
+
+@pytest.mark.parametrize("layers", [5, 6, 9, 10])
+@pytest.mark.parametrize("dtype,requests", [(torch.bfloat16, [(40, 0)]), (torch.bfloat16, [(487, 0)]), (torch.bfloat16, [(1, 9), (1, 30)]),
+                                            (torch.bfloat16, [(300, 0), (1, 20), (1, 7)]), (torch.float32, [(3, 0)]), (torch.float32, [(100, 0)])])
+def test_the_launches_and_what_they_read_are_those_of_every_layer_by_itself(monkeypatch, layers, dtype, requests):
+    """For prompts, single rows and both, one layer beyond the least up to several, an even and an odd number of layers between: the
+    same entry points with the same numbers, every address in the same tensor of the same layer or where the same earlier call wrote."""
+    m, library, held = stand_ins(monkeypatch, layers, dtype)
     tensors = {(i, n): t for i, layer in enumerate(m.layers) for n, t in enumerate(layer.launch_tensors()) if t is not None}
 
     caches, forward = {}, type(m).forward
@@ -121,3 +130,39 @@ def test_the_launches_and_what_they_read_are_those_of_every_layer_by_itself(monk
     assert none == 0 and some % (layers - 3) == 0 and some > 0
     at = lambda calls: [(n, tuple("step" if isinstance(x, tuple) and x[0] == "at" else x for x in args)) for n, args in calls]
     assert at(native) == at(one_by_one)
+
+
+def with_a_limit(part):
+    part.limit = 3.0
+
+
+def with_a_method(part):
+    part.forward = types.MethodType(type(part).forward, part)
+
+
+CHANGES = {"a method of the feed-forward": lambda layer: with_a_method(layer.ffn), "a method of the layer": with_a_method,
+           "a method of the norm": lambda layer: setattr(layer.norm_in, "after_add", types.MethodType(type(layer.norm_in).after_add, layer.norm_in)),
+           "the norm's number": lambda layer: setattr(layer.norm_post, "eps", 1e-3), "the gate's limit": lambda layer: with_a_limit(layer.ffn),
+           "another feed-forward": lambda layer: setattr(layer, "ffn", copy.copy(layer.ffn)) or with_a_limit(layer.ffn)}
+
+
+@pytest.mark.parametrize("change", CHANGES)
+@pytest.mark.parametrize("at", [1, 4])
+def test_a_layer_that_was_changed_after_the_load_is_walked(monkeypatch, change, at):
+    """What a program does to one layer of a loaded model is asked for by its own walk, whether that layer is the one whose launches
+    would be kept or one of those between."""
+    m, library, _ = stand_ins(monkeypatch, 9, torch.bfloat16)
+    walked = []
+    # (a layer that Python walks asks for the step's facts)
+    real = type(m.layers[0].mixer)._batch_facts
+    monkeypatch.setattr(type(m.layers[0].mixer), "_batch_facts", lambda self, *a: walked.append([l.mixer for l in m.layers].index(self)) or real(self, *a))
+    recorded.forward(m, (40, 0))
+    assert walked == [0, 1, 8]
+    plain = library.calls[:]
+    CHANGES[change](m.layers[at])
+    walked.clear()
+    library.calls.clear()
+    recorded.forward(m, (40, 0))
+    # (the norm of a changed layer is made by the layer before it)
+    assert at in walked and (at == 4 or 2 in walked) and ("norm" not in change or "number" in change or at - 1 in walked)
+    assert [c[0] for c in library.calls] == [c[0] for c in plain]
