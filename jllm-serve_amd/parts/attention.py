@@ -79,7 +79,7 @@ class GqaStepPlanner:
 class GqaAttention(Part):
     takes_normed_rows = True    # the input goes into ops.gemm and nowhere else
     prepares_next_norm = True   # forward(then_norm=...) ends with then_norm.after_add and returns its promise
-    takes_only = True           # forward(only=rows): behind the attention those rows alone, into ``residual`` of as many
+    takes_only = True           # forward(only=WantedRows): behind the attention those rows alone, into the stream of theirs
 
     def __init__(self, spec: GqaSpec, prefix: str, build: BuildContext, positions):
         if spec.kv_heads <= 0 or spec.heads % spec.kv_heads != 0:
@@ -197,7 +197,7 @@ class GqaAttention(Part):
 
     def _project_out(self, att, residual, then_norm, only=None):
         if only is not None:
-            att = att.index_select(0, only)
+            att, residual = only.take(att)
         if then_norm is not None:
             return then_norm.after_add(att, self.w_o, residual, bias=self.b_o, exact=self.build.exact)
         ops.gemm(att, self.w_o, bias=self.b_o, out=residual, epilogue=ops.EPI_ADD, exact=self.build.exact)

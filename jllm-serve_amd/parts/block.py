@@ -14,8 +14,6 @@ parts; a part that knows nothing of this works as before):
 """
 from __future__ import annotations
 
-from types import SimpleNamespace
-
 import torch
 
 from ..kernels import ops
@@ -115,14 +113,16 @@ class PreNormBlock(Part):
         """As the last layer: the mixer runs over all rows (its cache is written for all of them), what follows its heads over
         the step's selected rows only, as nobody reads the others. Returns the stream of those, [n_selected, width]."""
         xb = self._input(self.norm_in, self.mixer, x, normed_in)
+        wanted, mid = WantedRows(step, x), None
         if step.n_selected and type(self.mixer).__dict__.get("takes_only") and "forward" not in vars(self.mixer):
-            some = x.index_select(0, step.selected)
-            self.mixer.forward(xb, some, step, slot, only=step.selected)
+            more = {"then_norm": self.norm_post} if self._prepares(self.mixer, self.norm_post) else {}
+            mid = self.mixer.forward(xb, x, step, slot, only=wanted, **more)
         else:
             self.mixer.forward(xb, x, step, slot)
-            some = x.index_select(0, step.selected)
+            wanted.take()
+        some = wanted.stream
         if step.n_selected:
-            self.ffn.forward(self._input(self.norm_post, self.ffn, some, None), some, selected_step(step))
+            self.ffn.forward(self._input(self.norm_post, self.ffn, some, mid), some, SelectedStep(step))
         return some
 
 
@@ -138,9 +138,29 @@ def rows_alone(ffn) -> bool:
     return shared is None or rows_alone(shared)
 
 
-def selected_step(step):
-    """What such a feed-forward asks of a step, of its selected rows."""
-    return SimpleNamespace(n_tokens=step.n_selected, token_ids=step.token_ids.index_select(0, step.selected))
+class WantedRows:
+    """The rows of a step that somebody reads behind its last layer, and, once they are taken, their stream."""
+
+    def __init__(self, step, x):
+        self.rows, self.x, self.stream = step.selected, x, None
+
+    def take(self, *tensors):
+        """Those rows of the tensors and, last, of the stream: one launch."""
+        *some, self.stream = ops.gather_rows(self.rows, *tensors, self.x)
+        return *some, self.stream
+
+
+class SelectedStep:
+    """What a feed-forward whose rows stand alone asks of a step, of its selected rows."""
+
+    def __init__(self, step):
+        self.n_tokens, self._step, self._ids = step.n_selected, step, None
+
+    @property
+    def token_ids(self):  # (few ask)
+        if self._ids is None:
+            self._ids = ops.gather_rows(self._step.selected, self._step.token_ids.view(-1, 1))[0].view(-1)
+        return self._ids
 
 
 def sublayer_output(part, xb, step, slot, width):
@@ -268,16 +288,15 @@ class SandwichBlock(Part):
         """As ``PreNormBlock.forward_last``: behind the mixer's output only the selected rows go on."""
         xb = normed_in if isinstance(normed_in, torch.Tensor) else self.norm_in.forward(x)
         branches, scales = self._branches(xb, step, slot, self.norm_post, None)
-        some = x.index_select(0, step.selected)
+        *branches, some = WantedRows(step, x).take(*branches)
         if step.n_selected:
-            branches = [b.index_select(0, step.selected) for b in branches]
             if scales:
                 xb = self.norm_mixer_out.seam(some, branches, scales, then=self.norm_post)
             else:
                 xb = self._join(self.norm_mixer_out, some, branches[0], None, None, self.norm_post)
             if xb is None:
                 xb = self.norm_post.forward(some)
-            self._join(self.norm_ffn_out, some, sublayer_output(self.ffn, xb, selected_step(step), None, self.width), None, None, None)
+            self._join(self.norm_ffn_out, some, sublayer_output(self.ffn, xb, SelectedStep(step), None, self.width), None, None, None)
         return some
 
 

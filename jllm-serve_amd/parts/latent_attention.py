@@ -154,7 +154,7 @@ class LatentAttention(Part):
             meta["tiles_dev"] = tiles if tiles is not None and tiles.numel() else None
         return meta
 
-    takes_only = True  # forward(only=rows): behind the attention those rows alone, into ``residual`` of as many
+    takes_only = True  # forward(only=WantedRows): behind the attention those rows alone, into the stream of theirs
 
     def forward(self, xb, residual, step, slot, then_norm=None, only=None):
         s, exact = self.spec, self.build.exact
@@ -179,7 +179,8 @@ class LatentAttention(Part):
                                    s.scale, self.sink, meta=self._batch_facts(step), exact=exact)
         gate = y[:, gate_off:gate_off + s.heads * s.vdim] if s.out_gate else None
         if only is not None:
-            lat, gate = lat.index_select(0, only), gate.index_select(0, only) if gate is not None else None
+            lat, *gates, residual = only.take(lat, *([gate] if s.out_gate else []))
+            gate = gates[0] if s.out_gate else None
         if s.out_gate:
             att = ops.latent_heads(lat, self.w_uv, gate=gate, exact=exact)
         else:

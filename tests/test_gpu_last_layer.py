@@ -6,6 +6,7 @@ import kebepel_tiny
 import miforax_tiny
 import tiny
 from jllm_serve_amd.engine import StepEntry, build_runner, load_model
+from jllm_serve_amd.kernels import ops
 from jllm_serve_amd.parts.model import DecoderModel
 from jllm_serve_amd.weights import write_random_model
 
@@ -50,3 +51,21 @@ def test_logits_are_those_of_a_last_layer_over_all_rows(tmp_path, monkeypatch, f
             # both sides are within the family's bound of the plain implementation
             assert float((a.double() - b.double()).abs().max()) <= 2 * kind.tolerance(dtype, b.cpu().double())
     assert isinstance(load_model(folder, dtype, torch.device("cuda:0"), max_positions=256), DecoderModel)
+
+
+@pytest.mark.parametrize("n", [1, 3, 200])
+@pytest.mark.parametrize("width", [1, 7, 64, 2048, 2050])
+def test_rows_are_gathered_as_they_are(n, width):
+    """Row lengths of every unit that the kernel copies in, one, a few and many rows, with repeats and in any order, of contiguous matrices
+    and of views that begin at an odd element, one to four at once."""
+    gen = torch.Generator(device="cuda").manual_seed(n * width)
+    held = [torch.randn(37, width + 3, device="cuda", generator=gen).to(t) for t in (torch.bfloat16, torch.float32, torch.bfloat16)]
+    tensors = [held[0][:, 1:1 + width], held[1][:, :width], held[2][:, :width].contiguous(), torch.arange(37, device="cuda", dtype=torch.int32).view(-1, 1)]
+    rows = torch.randint(0, 37, (n,), device="cuda", generator=gen, dtype=torch.int32)
+    rows[0] = 36
+    for k in (1, 2, 4):
+        got = ops.gather_rows(rows, *tensors[:k])
+        assert len(got) == k and all(torch.equal(g, t[rows.long()]) for g, t in zip(got, tensors))
+    assert ops.gather_rows(rows[:0], *tensors)[1].shape == (0, width)
+    with pytest.raises(ops.KernelError):
+        ops.gather_rows(rows, *tensors, tensors[0])

@@ -1,7 +1,9 @@
 """Where the last layer goes on with the wanted rows alone."""
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
+import recorded
 from jllm_serve_amd.config.schema import GatedMlpSpec, RoutedMoeSpec, TableMoeSpec
 from jllm_serve_amd.parts.base import BuildContext, Part, part_factory
 from jllm_serve_amd.parts.block import rows_alone
@@ -30,3 +32,29 @@ def test_a_shared_feed_forward_is_asked_too(spec):
     assert not rows_alone(ffn)
     ffn.shared = None
     assert rows_alone(ffn)
+
+
+class Noted(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, kinds, args=(), kwargs=None):
+        self.names.append(func.overloadpacket.__name__)
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("rows", [40, 300])
+def test_the_wanted_rows_are_taken_by_one_launch(monkeypatch, rows):
+    """The heads' rows and the stream's together, by the project's own kernel; token ids are not gathered for a feed-forward that
+    does not read them; and the norm behind the o product is made on its way, as in every other layer."""
+    m = recorded.model(4096, 32, 8, 12288, layers=2)
+    seen = recorded.record(monkeypatch)
+    with Noted() as noted:
+        recorded.forward(m, (rows, 0), (1, 9))
+    names = [name for name, _ in seen]
+    assert names.count("jllm_gather_rows") == 1 and names.count("jllm_embed") == 1
+    assert names[-1].startswith("jllm_gemm") and names.count("jllm_rmsnorm") == 2  # in front of the layers and behind them
+    assert not {"index_select", "index", "gather", "take"} & set(noted.names), noted.names
+    _, n_matrices, picked, n, height, _ = next(args for name, args in seen if name == "jllm_gather_rows")
+    assert (n_matrices, n, height) == (2, 2, rows + 1)
