@@ -367,7 +367,8 @@ def gather_rows(rows: torch.Tensor, *tensors: torch.Tensor) -> Tuple[torch.Tenso
     if n and outs[0].shape[1]:
         if not 1 <= len(tensors) <= 4 or not height:
             raise KernelError(f"gather_rows takes one to four matrices, not {len(tensors)} of {height} rows")
-        _call("jllm_gather_rows", (_L * len(words))(*words), len(tensors), _ptr(rows), n, height, _stream())
+        matrices = (_L * len(words))(*words)
+        _call("jllm_gather_rows", ctypes.addressof(matrices), len(tensors), _ptr(rows), n, height, _stream())
     return tuple(outs)
 
 
