@@ -79,7 +79,7 @@ class GqaStepPlanner:
 class GqaAttention(Part):
     takes_normed_rows = True    # the input goes into ops.gemm and nowhere else
     prepares_next_norm = True   # forward(then_norm=...) ends with then_norm.after_add and returns its promise
-    takes_only = True           # forward(only=WantedRows): behind the attention those rows alone, into the stream of theirs
+    takes_only = True           # forward(only=WantedRows): behind the attention those rows alone, into the stream of theirs; none: the cache alone
 
     def __init__(self, spec: GqaSpec, prefix: str, build: BuildContext, positions):
         if spec.kv_heads <= 0 or spec.heads % spec.kv_heads != 0:
@@ -190,6 +190,8 @@ class GqaAttention(Part):
                 return self._project_out(att, residual, then_norm, only)
         ops.qk_norm_rope_store(qkv, step.positions, g.slots, cos, sin, self.g_q, self.g_k, s.qk_norm_eps, s.heads,
                                s.kv_heads, s.head_dim, rdim, slot.page_size, k_cache, v_cache, write_kv=slot.writes)
+        if only is not None and not only.n:
+            return None
         att = ops.paged_attention(qkv[:, :s.q_dim], k_cache, v_cache, g.block_table, step.row_req,
                                   step.positions, s.heads, s.kv_heads, s.head_dim, s.window, s.scale, meta=meta,
                                   exact=self.build.exact, slopes=slopes)
@@ -197,6 +199,8 @@ class GqaAttention(Part):
 
     def _project_out(self, att, residual, then_norm, only=None):
         if only is not None:
+            if not only.n:
+                return None
             att, residual = only.take(att)
         if then_norm is not None:
             return then_norm.after_add(att, self.w_o, residual, bias=self.b_o, exact=self.build.exact)

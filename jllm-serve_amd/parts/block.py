@@ -111,18 +111,20 @@ class PreNormBlock(Part):
 
     def forward_last(self, x, step, slot, normed_in=None):
         """As the last layer: the mixer runs over all rows (its cache is written for all of them), what follows its heads over
-        the step's selected rows only, as nobody reads the others. Returns the stream of those, [n_selected, width]."""
+        the step's selected rows only, as nobody reads the others; where none is wanted (the portions of a prompt in front of its last)
+        nothing follows what its cache gets. Returns the stream of those rows, [n_selected, width]."""
         xb = self._input(self.norm_in, self.mixer, x, normed_in)
         wanted, mid = WantedRows(step, x), None
-        if step.n_selected and type(self.mixer).__dict__.get("takes_only") and "forward" not in vars(self.mixer):
+        if type(self.mixer).__dict__.get("takes_only") and "forward" not in vars(self.mixer):
             more = {"then_norm": self.norm_post} if self._prepares(self.mixer, self.norm_post) else {}
             mid = self.mixer.forward(xb, x, step, slot, only=wanted, **more)
         else:
             self.mixer.forward(xb, x, step, slot)
             wanted.take()
+        if not step.n_selected:
+            return x[:0]
         some = wanted.stream
-        if step.n_selected:
-            self.ffn.forward(self._input(self.norm_post, self.ffn, some, mid), some, SelectedStep(step))
+        self.ffn.forward(self._input(self.norm_post, self.ffn, some, mid), some, SelectedStep(step))
         return some
 
 
@@ -142,7 +144,7 @@ class WantedRows:
     """The rows of a step that somebody reads behind its last layer, and, once they are taken, their stream."""
 
     def __init__(self, step, x):
-        self.rows, self.x, self.stream = step.selected, x, None
+        self.n, self.rows, self.x, self.stream = step.n_selected, step.selected, x, None
 
     def take(self, *tensors):
         """Those rows of the tensors and, last, of the stream: one launch."""

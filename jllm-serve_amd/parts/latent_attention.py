@@ -154,7 +154,7 @@ class LatentAttention(Part):
             meta["tiles_dev"] = tiles if tiles is not None and tiles.numel() else None
         return meta
 
-    takes_only = True  # forward(only=WantedRows): behind the attention those rows alone, into the stream of theirs
+    takes_only = True  # forward(only=WantedRows): behind the attention those rows alone, into the stream of theirs; none: the cache alone
 
     def forward(self, xb, residual, step, slot, then_norm=None, only=None):
         s, exact = self.spec, self.build.exact
@@ -172,6 +172,8 @@ class LatentAttention(Part):
                                     sin=sin, cache=cache)
         elif s.q_rank > 0:
             cq = ops.latent_prepare(y, s.q_rank, self.g_q, s.eps)
+        if only is not None and not only.n:
+            return None
         q = ops.gemm(cq, self.w_uq, out_dtype=self.build.dtype, exact=exact) if s.q_rank > 0 else y[:, :self.q_width]
         qa = ops.latent_heads(q, self.w_ukt, tail=s.rot_dim, rot_dims=rdims, positions=step.positions, cos=cos, sin=sin,
                               exact=exact)

@@ -35,8 +35,8 @@ def model(width, heads, kv_heads, ff, layers=2, dtype=torch.bfloat16):
     return m
 
 
-def forward(m, *requests):
-    """One step of ``requests`` (rows, first position): its logits' rows are the requests' last ones."""
+def forward(m, *requests, wanted=None):
+    """One step of ``requests`` (rows, first position): its logits' rows are the requests' last ones, or ``wanted`` in number."""
     i32 = lambda *shape: tensor(*shape, dtype=torch.int32)
     segments, rows = [], 0
     for i, (n, pos0) in enumerate(requests):
@@ -48,7 +48,8 @@ def forward(m, *requests):
     for planner in m.step_planners():
         plan = planner.plan(batch)
         plans[planner.key] = StepPlan({name: i32(len(a)) for name, a in plan.arrays.items()}, plan.facts)
-    step = StepContext(rows, len(segments), i32(rows), i32(rows), i32(rows), i32(len(segments)), i32(len(segments)), len(segments),
+    wanted = len(segments) if wanted is None else wanted
+    step = StepContext(rows, len(segments), i32(rows), i32(rows), i32(rows), i32(len(segments)), i32(wanted), wanted,
                        [GroupStep(i32(len(segments), -(-context // 16)), i32(rows))], segments, context, plans)
     slots = []
     for layer in m.layers:

@@ -58,3 +58,14 @@ def test_the_wanted_rows_are_taken_by_one_launch(monkeypatch, rows):
     assert not {"index_select", "index", "gather", "take"} & set(noted.names), noted.names
     _, n_matrices, picked, n, height, _ = next(args for name, args in seen if name == "jllm_gather_rows")
     assert (n_matrices, n, height) == (2, 2, rows + 1)
+
+
+def test_a_portion_that_wants_nothing_ends_with_the_cache(monkeypatch):
+    """Of the last layer only what its cache gets is made; for single rows that is inside their attention's launch."""
+    m = recorded.model(4096, 32, 8, 12288, layers=2)
+    seen = recorded.record(monkeypatch)
+    for requests, last in (([(300, 0), (1, 9)], "jllm_qk_norm_rope_store"), ([(1, 9), (1, 30)], "jllm_decode_attention_fused_bf16")):
+        del seen[:]
+        assert recorded.forward(m, *requests, wanted=0).shape == (0, 4096)
+        names = [name for name, _ in seen]
+        assert names[-1] == last and names.count(last) == 2, names
