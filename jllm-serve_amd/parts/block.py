@@ -19,7 +19,7 @@ import torch
 from ..kernels import ops
 from ..weights.loader import WeightSpec
 from .base import Part, StateShare, part_factory, register_part
-from .equal_layers import key_of, own_forward
+from .equal_layers import FLOPS_PER_US, WEIGHT_BYTES_PER_US, key_of, own_forward
 from .shift import TokenShift
 
 
@@ -39,6 +39,7 @@ class PreNormBlock(Part):
             self.parts = (self.norm_in, self.mixer, self.norm_post, self.ffn)
             self.norm_post.reader = self.ffn
         self.norm_in.reader = self.mixer
+        self.dtype = build.dtype
         self.capturable = all(getattr(p, "capturable", True) for p in self.parts)
 
     def weight_specs(self):
@@ -112,7 +113,10 @@ class PreNormBlock(Part):
     def forward_last(self, x, step, slot, normed_in=None):
         """As the last layer: the mixer runs over all rows (its cache is written for all of them), what follows its heads over
         the step's selected rows only, as nobody reads the others; where none is wanted (the portions of a prompt in front of its last)
-        nothing follows what its cache gets. Returns the stream of those rows, [n_selected, width]."""
+        nothing follows what its cache gets. Returns the stream and which of its rows are the selected ones (None: it holds no others)."""
+        if not wanted_pay(self, step):
+            self.forward(x, step, slot, normed_in=normed_in)
+            return x, step.selected
         xb = self._input(self.norm_in, self.mixer, x, normed_in)
         wanted, mid = WantedRows(step, x), None
         if type(self.mixer).__dict__.get("takes_only") and "forward" not in vars(self.mixer):
@@ -122,10 +126,10 @@ class PreNormBlock(Part):
             self.mixer.forward(xb, x, step, slot)
             wanted.take()
         if not step.n_selected:
-            return x[:0]
+            return x[:0], None
         some = wanted.stream
         self.ffn.forward(self._input(self.norm_post, self.ffn, some, mid), some, SelectedStep(step))
-        return some
+        return some, None
 
 
 register_part("arrangement", "prenorm", PreNormBlock, replace=True)
@@ -138,6 +142,39 @@ def rows_alone(ffn) -> bool:
         return False
     shared = getattr(ffn, "shared", None)
     return shared is None or rows_alone(shared)
+
+
+# What it costs a step to take the wanted rows apart, and what it has to save, in us. Behind layers whose launches may be made natively
+# (or that the GPU takes longer for than Python) it is a launch: 28 layers of the 0.6B shape, one row wanted, whole / taken apart: 40
+# rows 1,681 / 1,671 us, 200 2,088 / 2,060, 1,500 4,449 / 4,394; fp32, 17 rows 3,147 / 3,111. Other layers wait for Python, to which the
+# rows cost 15 to 35 us more: four of the Kebepel shape, 40 rows 809 / 826 us, 100 831 / 849, 200 891 / 866; of the Miforax shape, 5
+# rows 757 / 787, 40 863 / 855, 100 900 / 820. Two rows of a token each, one of them wanted: 513 / 523 (0.6B, four layers), 760 / 799
+# (Miforax); 63 of 64 768 / 784; 99 rows of 100 689 / 705.
+WANTED_SAVE_US = {True: 4.0, False: 20.0}
+WANTED_LEAST_ROWS = {True: 0, False: 49}
+FEW_ROWS_SAVE_US = 8.0  # where the others keep three products from the kernel for up to 16 rows
+
+
+def _weights_read(ffn, rows):
+    """Elements of the weights that a feed-forward reads for so many rows, by what it says (nothing: 0)."""
+    return ffn.weights_read(rows) if hasattr(ffn, "weights_read") else 0
+
+
+def wanted_pay(layer, step) -> bool:
+    """Whether the last layer is faster with the step's selected rows taken apart: by the feed-forward's weights and sums that the others
+    cost. (With none selected there is nothing to take.)"""
+    rows, some = step.n_tokens, step.n_selected
+    if some == 0:
+        return True
+    native = key_of(layer) is not None
+    if rows < WANTED_LEAST_ROWS[native]:
+        return False
+    size = layer.dtype.itemsize
+    read = _weights_read(layer.ffn, rows) - _weights_read(layer.ffn, some)
+    saved = read * size / WEIGHT_BYTES_PER_US + 2.0 * (rows - some) * _weights_read(layer.ffn, 1) / FLOPS_PER_US[size]
+    if native and rows > ops.SKINNY_MAX_ROWS >= some:
+        saved += FEW_ROWS_SAVE_US
+    return saved > WANTED_SAVE_US[native]
 
 
 class WantedRows:
@@ -196,6 +233,7 @@ class SandwichBlock(Part):
             return make(spec.norm, build.hidden, f"{prefix}.{name}{ending}", build)
 
         self.width = build.hidden
+        self.dtype = build.dtype
         self.norm_in = norm(spec.norm_in_name)
         self.norm_mixer_out = norm(spec.norm_mixer_out_name)
         mixer_prefix = f"{prefix}.{spec.mixer_prefix}" if getattr(spec, "mixer_prefix", "") else prefix
@@ -288,6 +326,9 @@ class SandwichBlock(Part):
 
     def forward_last(self, x, step, slot, normed_in=None):
         """As ``PreNormBlock.forward_last``: behind the mixer's output only the selected rows go on."""
+        if not wanted_pay(self, step):
+            self.forward(x, step, slot, normed_in=normed_in)
+            return x, step.selected
         xb = normed_in if isinstance(normed_in, torch.Tensor) else self.norm_in.forward(x)
         branches, scales = self._branches(xb, step, slot, self.norm_post, None)
         *branches, some = WantedRows(step, x).take(*branches)
@@ -299,7 +340,7 @@ class SandwichBlock(Part):
             if xb is None:
                 xb = self.norm_post.forward(some)
             self._join(self.norm_ffn_out, some, sublayer_output(self.ffn, xb, SelectedStep(step), None, self.width), None, None, None)
-        return some
+        return some, None
 
 
 register_part("arrangement", "sandwich", SandwichBlock, replace=True)

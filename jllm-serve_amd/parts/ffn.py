@@ -49,6 +49,9 @@ class GatedMlp(Part):
             self.w_up = get(self._name("up"))
         self.w_down = get(self._name("down"))
 
+    def weights_read(self, rows):
+        return 3 * self.hidden * self.dim
+
     def launch_key(self):
         return ("gated_mlp", self.hidden, self.dim, self.gate, self.limit, self.build.dtype, self.build.exact) if own_forward(self, GatedMlp) else None
 

@@ -174,7 +174,7 @@ class DecoderModel:
             added = False
             if run + 1 == len(schedule) and step.n_selected < step.n_tokens and self.watch is None and self.streams == 1 \
                     and hasattr(layer, "ends_rows") and layer.ends_rows():
-                x, selected = layer.forward_last(x, step, slots[run], normed_in=carry), None
+                x, selected = layer.forward_last(x, step, slots[run], normed_in=carry)
             elif not getattr(layer, "chains_norms", False):
                 layer.forward(x, step, slots[run])
                 carry = None

@@ -19,7 +19,15 @@ from ..weights.loader import WeightSpec
 from .base import BuildContext, Part, pad_rows, part_factory, register_part
 
 
+def _weights_read(ffn, rows):
+    """Elements of the weights that the experts of ``rows`` rows have, chosen evenly, and of the shared feed-forward's."""
+    s = ffn.spec
+    shared = ffn.shared.weights_read(rows) if hasattr(ffn.shared, "weights_read") else 0
+    return 3 * s.hidden * ffn.build.hidden * s.experts * (1.0 - (1.0 - s.top / s.experts) ** rows) + shared
+
+
 class TableMoe(Part):
+    weights_read = _weights_read
     rows_alone = True  # a row's output depends on that row and its token alone
 
     def __init__(self, spec: TableMoeSpec, prefix: str, build: BuildContext):
@@ -106,6 +114,7 @@ class RoutedMoe(Part):
     run gate/up and down, ``ops.moe_combine`` takes the weighted sum into the residual. Nothing waits for the GPU, so a
     decode step with this feed-forward can be captured."""
 
+    weights_read = _weights_read
     rows_alone = True  # a row's output depends on that row and its token alone
 
     def __init__(self, spec: RoutedMoeSpec, prefix: str, build: BuildContext):

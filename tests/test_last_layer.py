@@ -69,3 +69,22 @@ def test_a_portion_that_wants_nothing_ends_with_the_cache(monkeypatch):
         assert recorded.forward(m, *requests, wanted=0).shape == (0, 4096)
         names = [name for name, _ in seen]
         assert names[-1] == last and names.count(last) == 2, names
+
+
+def test_rows_are_taken_apart_only_where_that_saves_something(monkeypatch):
+    """Steps that drop few rows, and those of few rows altogether, keep the last layer whole: no gather, and the final norm takes the
+    row list; a prompt whose last row is wanted does not."""
+    m = recorded.model(1024, 16, 8, 3072, layers=2)
+    seen = recorded.record(monkeypatch)
+
+    def apart(*requests, wanted=None):
+        del seen[:]
+        recorded.forward(m, *requests, wanted=wanted)
+        picked = [args for name, args in seen if name == "jllm_rmsnorm"][-1][1]
+        some = any(name == "jllm_gather_rows" for name, _ in seen)
+        assert some == (picked is None)
+        return some
+
+    assert not any(apart((n, 0)) for n in (2, 5, 16))
+    assert not apart(*[(1, 100)] * 64, wanted=63) and not apart((100, 0), wanted=99) and not apart(*[(1, 9)] * 2, wanted=1)
+    assert all(apart((n, 0)) for n in (17, 64, 300, 2000)) and apart((300, 0), (1, 9))
