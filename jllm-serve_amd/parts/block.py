@@ -166,15 +166,14 @@ def wanted_pay(layer, step) -> bool:
     rows, some = step.n_tokens, step.n_selected
     if some == 0:
         return True
-    native = key_of(layer) is not None
-    if rows < WANTED_LEAST_ROWS[native]:
-        return False
     size = layer.dtype.itemsize
     read = _weights_read(layer.ffn, rows) - _weights_read(layer.ffn, some)
     saved = read * size / WEIGHT_BYTES_PER_US + 2.0 * (rows - some) * _weights_read(layer.ffn, 1) / FLOPS_PER_US[size]
-    if native and rows > ops.SKINNY_MAX_ROWS >= some:
-        saved += FEW_ROWS_SAVE_US
-    return saved > WANTED_SAVE_US[native]
+    few = FEW_ROWS_SAVE_US if rows > ops.SKINNY_MAX_ROWS >= some else 0.0
+    if saved + few <= min(WANTED_SAVE_US.values()):
+        return False
+    native = key_of(layer) is not None
+    return rows >= WANTED_LEAST_ROWS[native] and saved + native * few > WANTED_SAVE_US[native]
 
 
 class WantedRows:
