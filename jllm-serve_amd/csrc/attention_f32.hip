@@ -43,12 +43,10 @@ __device__ __forceinline__ int cache_row(const AttF32& A, const int* __restrict_
 // the L2 several times. In LDS they come once, in whole lines, and the next block's while this one's values are weighted; but a
 // compute unit then holds one workgroup. Registers / LDS, 16 heads over 8: 300 keys 12.1 / 11.2 us, three rows of 400 14.2 /
 // 11.8, of 2,000 56.1 / 41.1, 16 of 1,000 30.6 / 25.6; where there are more workgroups than compute units, 64 of 1,000 93.2 / 94.8
-// and 64 of 100 12.1 / 17.7; one block a wave, 60 keys, 5.6 / 6.5.
+// and 64 of 100 12.1 / 17.7.
+// `key_rows`, where STAGED: [AF_WAVES][64 keys][512 bytes]; `mg`: every wave's maximum, sum and weighted sums.
 template <int GC, bool STAGED>
-__global__ __launch_bounds__(64 * AF_WAVES, STAGED ? 1 : 2) void attention_f32_rows_kernel(AttF32 A) {
-  extern __shared__ __align__(1024) unsigned char key_rows[];  // STAGED: [AF_WAVES][64 keys][512 bytes]
-  __shared__ __align__(16) float qs[GC][AF_HD];
-  __shared__ float mg[AF_WAVES][GC][2 + AF_HD];  // every wave's maximum, sum and weighted sums
+__device__ __forceinline__ void attention_rows(const AttF32& A, unsigned char* key_rows, float (&qs)[GC][AF_HD], float (&mg)[AF_WAVES][GC][2 + AF_HD]) {
   const int t = blockIdx.x, lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = A.H / A.Hkv, chunks = (G + GC - 1) / GC;
@@ -210,6 +208,25 @@ __global__ __launch_bounds__(64 * AF_WAVES, STAGED ? 1 : 2) void attention_f32_r
     }
     A.out[(size_t)t * A.ldo + (size_t)(h0 + g) * AF_HD + dim] = x * (1.0f / ll);
   }
+}
+
+// STAGED: rows of more than two blocks of keys by way of LDS. The host knows the table's width alone, and a captured step's is that
+// of its bucket, however short the rows are: the row itself decides. Registers / LDS in that kernel, a row of 16 heads over 8: 20 keys
+// 4.9 / 6.0 us, 60 keys 5.6 / 6.3, 120 keys 6.6 / 6.6, 200 keys 8.3 / 7.3, 256 keys 8.9 / 7.3; 16 rows of 60 5.7 / 6.5, of 250 9.7 / 8.4.
+template <int GC, bool STAGED>
+__global__ __launch_bounds__(64 * AF_WAVES, STAGED ? 1 : 2) void attention_f32_rows_kernel(AttF32 A) {
+  extern __shared__ __align__(1024) unsigned char key_rows[];
+  __shared__ __align__(16) float qs[GC][AF_HD];
+  __shared__ float mg[AF_WAVES][GC][2 + AF_HD];
+  if constexpr (STAGED) {
+    const int pos = A.positions[blockIdx.x];
+    const int first = A.window > 0 ? max(0, pos + 1 - A.window) : 0;
+    if ((pos >> 6) - (first >> 6) >= 2) {
+      attention_rows<GC, true>(A, key_rows, qs, mg);
+      return;
+    }
+  }
+  attention_rows<GC, false>(A, nullptr, qs, mg);
 }
 
 // ---------------------------------------------------------------------------------------------- many rows

@@ -900,6 +900,20 @@ def test_float32_rows_with_their_keys_by_way_of_lds(ops, H, Hkv, page, window):
     assert not torch.isnan(got).any() and torch.equal(got, attend(torch.zeros(H, device=DEV)))
 
 
+@pytest.mark.parametrize("window", [0, 1, 65, 66, 128, 129, 257])
+def test_float32_rows_of_a_wide_table_choose_by_their_own_keys(ops, window):
+    """Rows of one to five blocks of keys in a table of many, as a captured step has them: up to two blocks the keys go into registers,
+    beyond by way of LDS; on either side of that line, without a window and with ones that reach over two and three blocks."""
+    lens = [1, 2, 64, 65, 127, 128, 129, 192, 193, 257, 1500]
+    kc, vc, table, _, _ = make_cache(len(lens), lens, 2, 128, 16, torch.float32, seed=window)
+    q = torch.randn(len(lens), 4 * 128, generator=torch.Generator().manual_seed(window)).to(DEV)
+    req = torch.arange(len(lens), dtype=torch.int32, device=DEV)
+    pos = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    attend = lambda slopes: ops.paged_attention(q, kc, vc, table, req, pos, 4, 2, 128, window, 128 ** -0.5, exact=True, slopes=slopes)
+    got = attend(None)
+    assert not torch.isnan(got).any() and torch.equal(got, attend(torch.zeros(4, device=DEV)))
+
+
 @pytest.mark.parametrize("H,Hkv,hd,window", [(12, 3, 32, 0), (10, 2, 48, 70), (6, 3, 64, 0), (8, 8, 16, 0)])
 def test_general_attention_gives_a_row_the_same_bits_in_any_step(ops, H, Hkv, hd, window):
     """The general kernel (the 32-bit path) takes up to four query heads of a kv head in one workgroup when the step
