@@ -551,12 +551,12 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
   const int sub = lane & 15, q4 = lane >> 4;
   const int H = Hkv * G;
   const int psh = __builtin_ctz(page_size);  // pages hold a power of two of positions: shifts, not divisions
-  // Everything that does not depend on the row's position is requested together with it: the table entries of the range as they
-  // lie where a row is the request of its number and no window moves the start (else they are read again), the fused form's q,
-  // new key and value and their gains.
+  // Everything that does not depend on the row's position is requested together with it, in the fused form: the table entries of the
+  // range as they lie where a row is the request of its number and no window moves the start (else they are read again), q, the new
+  // key and value and their gains. The rows of the other form are some of a step's, whose requests have any number.
   const int b_ahead = (s * split) >> psh;
-  const int req_ahead = min(t, table_rows - 1);
-  const int entry = block_table[(size_t)req_ahead * max_blocks + min(b_ahead + (int)threadIdx.x, max_blocks - 1)];
+  const int req_ahead = FUSED ? min(t, table_rows - 1) : 0;
+  const int entry = FUSED ? block_table[(size_t)req_ahead * max_blocks + min(b_ahead + (int)threadIdx.x, max_blocks - 1)] : 0;
   const bf16_t* qrow = q + (size_t)t * ldq + (size_t)kvh * G * hd;
   constexpr int QV = (G + 3) / 4, RAW = 2;
   uint4 raw[RAW];  // wave 0: the heads q4, q4 + 4, ..; wave 1: the new key, the new value; 8 dims a lane
@@ -587,13 +587,13 @@ __global__ __launch_bounds__(DA_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1
   const int ssh = __builtin_ctz(split);  // and so is a range's length
   const int s_lo = whole ? 0 : first >> ssh, s_hi = whole ? 0 : pos >> ssh;
   if (s < s_lo || s > s_hi) return;
-  asm volatile("" ::"v"(entry));  // waited for here, where all that is on its way was requested with it
+  if (FUSED) asm volatile("" ::"v"(entry));  // waited for here, where all that is on its way was requested with it
   const int kb = whole ? first : max(first, s * split);
   const int ke = whole ? pos : min(pos, s * split + split - 1);
   const int b0 = kb >> psh;
   const int nb = (ke >> psh) - b0 + 1;
   const bool has_new = slot >= 0 && s == s_hi;
-  if (req != req_ahead || b0 != b_ahead || nb > DA_WAVES * 64) {
+  if (!FUSED || req != req_ahead || b0 != b_ahead || nb > DA_WAVES * 64) {
     const int* tbl = block_table + (size_t)req * max_blocks;
     for (int i = threadIdx.x; i < nb; i += DA_WAVES * 64) tb[i] = tbl[b0 + i];
   } else if ((int)threadIdx.x < nb) {
@@ -913,7 +913,7 @@ extern "C" int jllm_decode_attention_bf16(const void* q, int ldq, void* out, int
                                           const int* row_req, const int* positions, int n_rows, int H, int Hkv, int hd,
                                           int page_size, int window, float scale, int max_pos, float* part_acc,
                                           float* part_ml, int max_splits, int split, hipStream_t stream) {
-  return decode_attention<false>(q, ldq, out, ldo, kcache, vcache, block_table, max_blocks, 1, row_req, positions, n_rows, H,
+  return decode_attention<false>(q, ldq, out, ldo, kcache, vcache, block_table, max_blocks, 0, row_req, positions, n_rows, H,
                                  Hkv, hd, page_size, window, scale, max_pos, part_acc, part_ml, max_splits, split,
                                  DecodeFusion{}, stream);
 }
@@ -986,7 +986,7 @@ extern "C" int jllm_decode_attention_bf16_no_alloc(const void* q, int ldq, void*
               n_rows, H, max_splits, hd, need, (unsigned)JLLM_NO_ALLOC_SCRATCH_FLOATS);
   float* base = nullptr;
   if (scratch_of_current_device(&base) != 0) return -1;
-  return decode_attention<false>(q, ldq, out, ldo, kcache, vcache, block_table, max_blocks, 1, row_req, positions, n_rows, H,
+  return decode_attention<false>(q, ldq, out, ldo, kcache, vcache, block_table, max_blocks, 0, row_req, positions, n_rows, H,
                                  Hkv, hd, page_size, window, scale, max_pos, base, base + acc_floats, (int)max_splits, split,
                                  DecodeFusion{}, stream);
 }
