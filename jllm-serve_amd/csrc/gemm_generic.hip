@@ -496,12 +496,7 @@ static int launch_f32_tile(const F32Args& g, hipStream_t stream) {
 template <bool GATED>
 static int launch_f32_few(const F32Args& g, hipStream_t stream) {
   using F = F32Few<GATED>;
-  static bool configured = false;
-  if (!configured) {  // above 64 KB the size has to be allowed first
-    if (hipFuncSetAttribute((const void*)gemm_f32_few_kernel<GATED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)F::LDS) != hipSuccess)
-      JLLM_FAIL("gemm: cannot reserve %zu bytes of LDS", F::LDS);
-    configured = true;
-  }
+  static_assert(F::LDS + 64 * sizeof(float) <= 64 * 1024, "no launch needs leave for more");
   gemm_f32_few_kernel<GATED><<<(g.N + 15) / 16, F::THREADS, F::LDS, stream>>>((const float*)g.A, g.lda, (const float*)g.W, (const float*)g.W2, g.bias,
                                                                           g.bias_dtype, g.out, g.out_dtype, g.ldo, g.M, g.N, g.K, g.epilogue, g.gs);
   return 0;
