@@ -39,7 +39,8 @@ decoding at batch 8 and 64 with full windows, each with the fraction of the publ
 
 A decode step must read every weight once and the keys and values of the live requests: bytes = weights + KV bytes
 per token x tokens held (mean over the timed steps). A prefill must do 2 flops per weight and row, plus 4 x heads x
-head size per (row, key) pair and layer, plus the head for the rows whose logits are wanted.
+head size per (row, key) pair and layer, plus the head for the rows whose logits are wanted; behind the last layer's attention
+(its output product and feed-forward) only those rows count.
 """
 import argparse
 import json
@@ -82,7 +83,8 @@ class Work:
         self.F, self.V = shape["intermediate_size"], shape["vocab_size"]
         self.esize = 2 if dtype == "bf16" else 4
         self.dtype = dtype
-        self.layer_params = (self.H * self.hd + 2 * self.Hkv * self.hd) * self.d + self.d * self.H * self.hd + 3 * self.d * self.F
+        self.behind_heads = self.d * self.H * self.hd + 3 * self.d * self.F  # a layer's output product and feed-forward
+        self.layer_params = (self.H * self.hd + 2 * self.Hkv * self.hd) * self.d + self.behind_heads
         self.weight_bytes = (self.L * self.layer_params + self.V * self.d) * self.esize
         self.kv_bytes_per_token = 2 * self.L * self.Hkv * self.hd * self.esize
         self.window = shape.get("sliding_window", 0) if shape.get("use_sliding_window") else 0
@@ -98,9 +100,10 @@ class Work:
         return sum(min(i + 1, w) for i in range(T))
 
     def flops(self, rows: float, pairs: float, selected: float) -> float:
-        """``rows`` through every layer, ``pairs`` of (row, key) in the attention of every layer, ``selected`` rows
-        through the head."""
-        return 2.0 * rows * self.L * self.layer_params + 4.0 * self.H * self.hd * self.L * pairs + 2.0 * self.V * self.d * selected
+        """``rows`` through every layer, but behind the last one's heads ``selected`` of them, ``pairs`` of (row, key) in the
+        attention of every layer, ``selected`` rows through the head."""
+        return 2.0 * (rows * self.L * self.layer_params - (rows - selected) * self.behind_heads) + 4.0 * self.H * self.hd * self.L * pairs \
+            + 2.0 * self.V * self.d * selected
 
     def pass_seconds(self, ones: int, one_keys: int, rows: int, pairs: int) -> float:
         """The least time one pass can take at the published peaks: the larger of the time to read what it must
@@ -144,7 +147,8 @@ class LatentWork:
     """Bytes and flops of passes over a Miforax model of the sizes ``z`` (the interface of ``Work``). A decode step
     reads every weight outside the experts, of the experts at most batch x top per layer, and per request the cached
     rows its window holds; a row costs 2 flops per weight it passes through (of the experts: top), and per (row, key)
-    pair and head 2 x (kv_rank + rot) for the score and 2 x kv_rank for the weighted sum."""
+    pair and head 2 x (kv_rank + rot) for the score and 2 x kv_rank for the weighted sum; behind the last layer's attention
+    only the rows whose logits are wanted count."""
 
     def __init__(self, z: dict, dtype: str):
         self.z = z
@@ -161,6 +165,7 @@ class LatentWork:
         self.expert = 3 * d * z["expert_ff"]
         self.n_moe = self.L // 2
         self.n_dense = self.L - self.n_moe
+        self.behind_heads = H * z["vdim"] * (r + d) + (self.dense_ff if self.L % 2 else self.shared_ff + z["top"] * self.expert)
         self.kv_bytes_per_token = self.L * self.hd * self.esize
         self.weight_bytes = (self.L * self.mixer + self.n_dense * self.dense_ff + self.n_moe * (self.shared_ff + z["experts"] * self.expert)
                              + self.V * d) * self.esize
@@ -178,7 +183,8 @@ class LatentWork:
 
     def flops(self, rows: float, pairs: float, selected: float) -> float:
         per_row = self.L * self.mixer + self.n_dense * self.dense_ff + self.n_moe * (self.shared_ff + self.z["top"] * self.expert)
-        return 2.0 * rows * per_row + 2.0 * self.H * (self.hd + self.z["kv_rank"]) * self.L * pairs + 2.0 * self.V * self.d * selected
+        return 2.0 * (rows * per_row - (rows - selected) * self.behind_heads) + 2.0 * self.H * (self.hd + self.z["kv_rank"]) * self.L * pairs \
+            + 2.0 * self.V * self.d * selected
 
 
 KEBEPEL_SIZES = {  # layer sizes that resemble released models with a delta-rule mixer beside attention
@@ -207,7 +213,8 @@ class KebepelWork:
     """Bytes and flops of passes over a Kebepel model of the sizes ``z`` (the interface of ``Work``). A decode step reads
     every weight, per request the cached keys and values of every layer, and reads and writes the delta rule's matrices
     (fp32); a row costs 2 flops per weight, per (row, key) pair 2 (dk + dv) per score map, and in the delta rule 6 dk
-    dv per head (two products with the matrix and its update)."""
+    dv per head (two products with the matrix and its update); through the last layer's feed-forward only the rows whose logits are
+    wanted go."""
 
     def __init__(self, z: dict, dtype: str):
         self.z = z
@@ -234,7 +241,8 @@ class KebepelWork:
         return T * (T + 1) / 2.0
 
     def flops(self, rows: float, pairs: float, selected: float) -> float:
-        return rows * (2.0 * self.per_row + self.row_flops) + self.pair_flops * pairs + 2.0 * self.V * self.d * selected
+        return rows * (2.0 * self.per_row + self.row_flops) - (rows - selected) * 6.0 * self.d * self.F + self.pair_flops * pairs \
+            + 2.0 * self.V * self.d * selected
 
 
 GUBOTAR_CHUNK = 2048  # positions of an attention chunk: as long as the measured prompts, so that both models see every key
@@ -545,7 +553,8 @@ class DazilixWork:
     """Bytes and flops of passes over a Dazilix model of the sizes ``z`` (the interface of ``Work``). A decode step reads
     every weight outside the experts, of the experts at most batch x top per layer, per request the keys and values (cached
     as two tensors) of its chunk, and reads and writes the recurrent matrices (fp32); a row costs 2 flops per weight it
-    passes through, per (row, key) pair and head 4 dim, and in a recurrence 4 dim vdim per head."""
+    passes through, per (row, key) pair and head 4 dim, and in a recurrence 4 dim vdim per head; through the last layer's
+    feed-forward only the rows whose logits are wanted go."""
 
     def __init__(self, z: dict, dtype: str):
         self.z = z
@@ -576,8 +585,9 @@ class DazilixWork:
         return sum(i % GUBOTAR_CHUNK + 1 for i in range(T))
 
     def flops(self, rows: float, pairs: float, selected: float) -> float:
-        per_row = self.mixers + self.L * (self.router + self.z["top"] * self.expert)
-        return rows * (2.0 * per_row + self.row_flops) + self.pair_flops * pairs + 2.0 * self.V * self.d * selected
+        ffn = self.router + self.z["top"] * self.expert
+        return rows * (2.0 * (self.mixers + self.L * ffn) + self.row_flops) - 2.0 * (rows - selected) * ffn + self.pair_flops * pairs \
+            + 2.0 * self.V * self.d * selected
 
 
 def compare_dazilix(args) -> dict:
