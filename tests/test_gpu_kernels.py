@@ -241,6 +241,26 @@ def test_gemm_two_group_kernel_with_wide_last_rows(ops, monkeypatch, M, N, K, cu
     assert bool(((got[1].double() - ref).abs() <= K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
 
 
+@pytest.mark.parametrize("M,N,K,cut", [(256, 256, 128, 1), (257, 300, 160, 1), (320, 700, 288, 2), (300, 516, 1056, 3), (330, 260, 2080, 5)])
+def test_gemm_ring_of_half_stages(ops, monkeypatch, M, N, K, cut):
+    """A ring of halves of stages of 64: K of two stages, of whole ones and with a last one of 32, alone and as the end of the last of
+    several parts of unequal length, shorter than the ring and longer, in all three tilings, which give the same bits."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M + K)
+    a = torch.randn(M, K, device=DEV, generator=gen).bfloat16()
+    w = (torch.randn(N, K, device=DEV, generator=gen) * K ** -0.5).bfloat16()
+    monkeypatch.setattr(ops, "_wide_plan", lambda *_: None)
+    got = []
+    for rows in (256, 192) + ((ops.WIDE_LAST,) if 1 <= M % 256 <= 128 else ()):
+        monkeypatch.setattr(ops, "_tiles", lambda m, n, k, gated, *plan: (rows, cut))
+        ops.reset_stats()
+        got.append(ops.gemm(a, w, out_dtype=torch.float32))
+        assert ops.stats()["ran"] == {"jllm_gemm_pingpong_bf16": 1}
+    assert all(torch.equal(got[0], x) for x in got[1:])
+    ref = a.double() @ w.double().T  # fp32 sums of K rounded products: K 2^-24 of the sum of magnitudes at most
+    assert bool(((got[0].double() - ref).abs() <= K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 520, 128), (130, 516, 192), (256, 1024, 256), (385, 131, 576)])
 def test_the_small_tile_gives_the_bits_of_the_two_group_kernel(ops, monkeypatch, M, N, K):
     """The small tile's accumulators lie otherwise over the lanes (32 x 32) than the two-group kernel's (16 x 16): every
