@@ -1,34 +1,39 @@
-// out[M,N] = A[M,K] * W[N,K]^T for many rows (prompt portions): bf16 operands staged through LDS, fp32
-// accumulation on the matrix cores (v_mfma_f32_32x32x16_bf16). Two of its products give the bits of one of
-// v_mfma_f32_16x16x32_bf16, which gemm_pingpong.hip uses, so both kernels give the same outputs. That form saves power
-// where the whole chip multiplies, but reads twice the fragments out of LDS, which is what binds here: with it 400 rows of 9,728
-// x 2,560 took 55.6 us instead of 51.3, 193 rows of the gated 2,560 x 9,728 52.7 instead of 49.3, 300 rows of 12,288 x 4,096
-// 68.0 instead of 63.6, and whole prompts of 129 rows of the 4B shape 5.64 ms instead of 5.52.
+// out[M,N] = A[M,K] * W[N,K]^T in tiles of 64 x 64 to 256 x 128, for products that the large tiles of gemm_pingpong.hip would leave
+// most compute units without: bf16 on the matrix cores (v_mfma_f32_16x16x32_bf16, in the order of that kernel, so both give the
+// same outputs).
 //
-// Two tile shapes. The small one: 4 waves in a 2 x 2 arrangement over a 128 x 128 output tile, each wave owning
-// 64 x 64 = four 32 x 32 accumulators; two such workgroups share a compute unit. The large one, for products
-// with many tiles: 8 waves in a 2 x 4 arrangement over 256 x 256, each wave owning 128 x 64 (fewer LDS bytes per
-// multiply). K advances in steps of 64 through two LDS buffers: while the waves multiply out of
-// one, the 16-byte global loads of the next step are already in registers and are stored into the other.
-// LDS rows are padded by 16 bytes so that the 16-byte operand reads of neighbouring rows fall into
-// different banks. With gridDim.x a multiple of 8, the workgroups that share a weight tile run on the same
-// XCD (workgroups go round-robin to the 8 XCDs by linear id), so the tile is fetched into one L2.
+// A wave owns RM x CN accumulators of 16 x 16, WGM x WGN waves a tile. K advances in stages of 64 through a ring of NS stages in
+// LDS, filled without registers (global_load_lds_dwordx4, whole lines of 128 bytes, eight rows to an instruction, the bank
+// swizzle applied on the global side). A stage's fragments are all in registers before its multiplies begin; between these,
+// evenly, a wave reads the next stage's fragments (a second set of registers) and asks for its share of the stage that takes the
+// place of the one it is multiplying. One barrier a stage.
 //
-// Epilogues: store, add into the fp32 residual, gated. For the gated one the LDS rows of the weight tile are,
-// per 64 rows, 32 gate rows and the 32 matching up rows, so that every wave holds gate and up of the same 32
-// outputs in neighbouring accumulators and silu(gate) * up is formed in registers.
+// What binds is the pipe through which a compute unit fills its LDS (32 bytes a clock at best: 1,024 clocks for a stage of 128 x 128,
+// whose MFMAs take 512; a stage takes 0.55 to 0.65 us, some 1,350 clocks, with a tile on nearly every compute unit), and where
+// there are few stages the launch, the first bytes and the parts of a cut K. The smaller tiles share a compute unit (two of 64 x 128,
+// 72 KB each, two of 64 x 64), which hides one's start and end behind the other.
 //
+// What stood here before (128 x 128 through registers and two LDS buffers, 32 x 32 x 16; below a thousand rows mostly gemm_stream.hip,
+// with LDS reads of 144 KB a stage) / this, us inside a graph, products alone: 0.6B shape at 487 rows qkv 12.2 / 8.9, gate/up 16.8 /
+// 14.6, 8B qkv at 128 rows 25.7 / 20.5, at 631 50.9 / 41.4, o at 128 20.1 / 15.
+//
+// Epilogues as in gemm_epilogue.h; K cut over gridDim.z leaves fp32 partial tiles that the reduction below adds up. Two further
+// forms: grouped (a workgroup's rows belong to one group, with weights of its own, gathered by an index list) and per head.
 // Needs K % 64 == 0 and 16-byte aligned rows; any M and N. The caller falls back otherwise.
+#include <type_traits>
 #include "common.h"
 #include "layer_launches.h"
+#include "lds_ring.h"
 #include "gemm_epilogue.h"
 #include "mfma.h"
 
 #define TBK 64
-#define TPCS (TBK / 8)  // 16-byte pieces per tile row
-#define TLD (TBK + 8)   // LDS row stride in elements
+#define T_ROW_BYTES (TBK * 2)  // a tile row in LDS: 128 bytes = 8 pieces of 16
+#define T_FENCE() __builtin_amdgcn_sched_barrier(0)
 
-// What the per-head form (HEADS) takes beside the operands: head h = blockIdx.z multiplies the rows at A + h * a_stride with
+enum { FORM_PLAIN = 0, FORM_GROUPED = 1, FORM_HEADS = 2 };
+
+// What the per-head form takes beside the operands: head h = blockIdx.z multiplies the rows at A + h * a_stride with
 // its own weights (W [heads][N][K]) and writes bf16 at out + h * o_stride, times sigmoid(gate[row][h * N + column]) where a
 // gate is given.
 struct HeadsArgs {
@@ -36,190 +41,185 @@ struct HeadsArgs {
   const bf16_t* gate;
   int ld_gate;
 };
+// The grouped form: (group, first row, rows) per blockIdx.y, rows = 0 for an unused entry: the workgroup's rows are first ..
+// first + rows - 1, its weights those of its group ([groups][N][K]); with `row_map` input row i is row row_map[i] / row_div of A,
+// the output rows stay i.
+struct GroupArgs {
+  const int *groups, *row_map;
+  int row_div;
+};
 
-// WGM x WGN waves, each with FM x FN accumulators of 32 x 32 (FN = 2 for the gated epilogue: gate and up)
-template <bool GATED, int WGM, int WGN, int FM, int FN, bool DEEP, bool HEADS = false>
+template <bool GATED, int FORM, int RM, int CN, int WGM, int WGN, int NS>
 __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
     const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N, int K,
-    int epilogue, GateSpec gs, float* __restrict__ partial, const int* __restrict__ groups, const int* __restrict__ row_map,
-    int row_div, HeadsArgs ha) {
-  static_assert(FN == 2, "a wave's columns are two 32-wide accumulators (gate and up with the gated epilogue)");
-  constexpr int NT = WGM * WGN * 64;
-  constexpr int TBM = WGM * FM * 32, TBN = WGN * FN * 32;
-  constexpr int TRSTEP = NT / TPCS;        // rows between a thread's pieces
-  constexpr int PA = TBM / TRSTEP, PB = TBN / TRSTEP;  // pieces per thread
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  bf16_t* As = (bf16_t*)smem_raw;             // [2][TBM][TLD]
-  bf16_t* Bs = As + 2 * TBM * TLD;            // [2][TBN][TLD]
+    int epilogue, GateSpec gs, float* __restrict__ partial, GroupArgs ga, HeadsArgs ha) {
+  constexpr int WAVES = WGM * WGN, TBM = WGM * RM * 16, TBN = WGN * CN * 16, STAGE = (TBM + TBN) * T_ROW_BYTES;
+  constexpr int LA = TBM / 8 / WAVES, L = LA + TBN / 8 / WAVES;  // load instructions (8 rows each) per wave and stage
+  constexpr int NM = 2 * RM * CN, NR = 2 * (RM + CN);            // multiplies and LDS reads of a stage
+  constexpr int EVERY = NM / L;
+  static_assert(LA * 8 * WAVES == TBM && (L - LA) * 8 * WAVES == TBN && EVERY >= 1, "every wave loads as many rows of either operand");
+  static_assert(NS >= 3 && NS <= 6, "one stage being read, one that has landed or is about to, one on its way");
+  extern __shared__ __align__(1024) unsigned char smem[];
   const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int wm = wave / WGN, wn = wave % WGN;
-  // Grouped form (`groups`: (group, first row, rows) per blockIdx.y, rows = 0 for an unused entry): the workgroup's rows
-  // are first .. first + rows - 1, its weights those of its group ([groups][N][K]); with `row_map` input row i is row
-  // row_map[i] / row_div of A (rows gathered by an index list), the output rows stay i.
-  int m0 = blockIdx.y * TBM;
-  if (groups) {
-    const int g_rows = groups[3 * blockIdx.y + 2];
-    if (g_rows == 0) return;
-    m0 = groups[3 * blockIdx.y + 1];
-    M = m0 + g_rows;
-    const size_t at = (size_t)groups[3 * blockIdx.y] * N * K;
+  // (no order of the tiles by dies here: these products gain nothing by it, and its divisions cost 0.3 us)
+  const int row = blockIdx.y, col = blockIdx.x;
+  int m0 = row * TBM;
+  if (FORM == FORM_GROUPED) {
+    const int rows = ga.groups[3 * row + 2];
+    if (rows == 0) return;
+    m0 = ga.groups[3 * row + 1];
+    M = m0 + rows;
+    const size_t at = (size_t)ga.groups[3 * row] * N * K;
     W += at;
     if (GATED) W2 += at;
   }
-  if (HEADS) {
+  if (FORM == FORM_HEADS) {
     A += (size_t)blockIdx.z * ha.a_stride;
     W += (size_t)blockIdx.z * N * K;
   }
-  const int n0 = blockIdx.x * (GATED ? TBN / 2 : TBN);  // output columns covered by this workgroup start here
-  // global -> register staging: piece c = tid + NT j: row c / TPCS, 16 bytes number c % TPCS
-  const int lrow = tid / TPCS, lpc = tid % TPCS;
-  const bf16_t* aptr[PA];
-  const bf16_t* bptr[PB];
-#pragma unroll
-  for (int j = 0; j < PA; ++j) {
-    int row = min(m0 + lrow + TRSTEP * j, M - 1);
-    if (row_map) row = row_map[row] / row_div;
-    aptr[j] = A + (size_t)row * lda + lpc * 8;
-  }
-#pragma unroll
-  for (int j = 0; j < PB; ++j) {
-    const int r = lrow + TRSTEP * j;
-    int wr;
-    const bf16_t* wb = W;
-    if (GATED) {  // LDS row r: quarter r / 32: even = gate, odd = up of the outputs n0 + (quarter / 2) * 32 ..
-      const int quarter = r >> 5;
-      wr = n0 + (quarter >> 1) * 32 + (r & 31);
-      wb = (quarter & 1) ? W2 : W;
-    } else {
-      wr = n0 + r;
-    }
-    bptr[j] = wb + (size_t)min(wr, N - 1) * K + lpc * 8;
-  }
+  const int n0 = col * (GATED ? TBN / 2 : TBN);  // output columns covered by this workgroup start here
   // gridDim.z > 1: this workgroup multiplies only its share of K and leaves an fp32 partial tile
   const int nk_all = K / TBK;
-  const int nk_per = HEADS ? nk_all : (nk_all + gridDim.z - 1) / gridDim.z;
-  const int kt0 = HEADS ? 0 : blockIdx.z * nk_per;
+  const int nk_per = FORM == FORM_HEADS ? nk_all : (nk_all + gridDim.z - 1) / gridDim.z;
+  const int kt0 = FORM == FORM_HEADS ? 0 : blockIdx.z * nk_per;
   const int nk = max(0, min(nk_all, kt0 + nk_per) - kt0);
-  floatx16 acc[FM][FN];
+
+  // ---- global side of the loads: the tile's start at its first stage (the same in all lanes, advanced by scalar arithmetic) and a
+  // 32-bit byte offset per lane that never changes (row of the tile and piece; rows of less than 8 MB: checked on the host).
+  // Rows gathered by a list lie anywhere: an address per lane.
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+  const unsigned char* abase = (const unsigned char*)(A + (size_t)m0 * lda) + (size_t)kt0 * T_ROW_BYTES;
+  const unsigned char* wbase[2] = {(const unsigned char*)(W + (size_t)n0 * K) + (size_t)kt0 * T_ROW_BYTES,
+                                   (const unsigned char*)((GATED ? W2 : W) + (size_t)n0 * K) + (size_t)kt0 * T_ROW_BYTES};
+  const unsigned char *base[L], *gathered[LA];
+  uint32_t off[L];
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-#pragma unroll
-  for (int j = 0; j < PA; ++j) aptr[j] += (size_t)kt0 * TBK;
-#pragma unroll
-  for (int j = 0; j < PB; ++j) bptr[j] += (size_t)kt0 * TBK;
-  struct Staged {
-    u32x4 a[PA], b[PB];
-  };
-  auto request = [&](Staged& r, int kt) {  // the global loads of K step kt
-#pragma unroll
-    for (int j = 0; j < PA; ++j) r.a[j] = *(const u32x4*)(aptr[j] + (size_t)kt * TBK);
-#pragma unroll
-    for (int j = 0; j < PB; ++j) r.b[j] = *(const u32x4*)(bptr[j] + (size_t)kt * TBK);
-  };
-  auto put = [&](const Staged& r, int buf) {  // into LDS buffer buf
-#pragma unroll
-    for (int j = 0; j < PA; ++j) *(u32x4*)(As + (size_t)buf * TBM * TLD + (size_t)(lrow + TRSTEP * j) * TLD + lpc * 8) = r.a[j];
-#pragma unroll
-    for (int j = 0; j < PB; ++j) *(u32x4*)(Bs + (size_t)buf * TBN * TLD + (size_t)(lrow + TRSTEP * j) * TLD + lpc * 8) = r.b[j];
-  };
-  const int fr = lane & 31;        // fragment row / column
-  const int fk = (lane >> 5) * 8;  // fragment k offset
-  auto multiply = [&](int cur) {
-    const bf16_t* Ac = As + (size_t)cur * TBM * TLD + (size_t)(wm * FM * 32 + fr) * TLD + fk;
-    const bf16_t* Bc = Bs + (size_t)cur * TBN * TLD + (size_t)(wn * FN * 32 + fr) * TLD + fk;
-    // the weight fragment goes in as the first operand: the accumulator then holds the tile transposed (rows =
-    // output columns), so a lane owns four consecutive output columns of one row and stores them at once
-    constexpr int KS = DEEP ? 2 : TBK / 16;  // k16 steps whose fragments are in registers together
-#pragma unroll
-    for (int k0 = 0; k0 < TBK / 16; k0 += KS) {
-      u32x4 af[KS][FM], bf[KS][FN];
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-        for (int i = 0; i < FM; ++i) af[ks][i] = *(const u32x4*)(Ac + i * 32 * TLD + (k0 + ks) * 16);
-#pragma unroll
-        for (int j = 0; j < FN; ++j) bf[ks][j] = *(const u32x4*)(Bc + j * 32 * TLD + (k0 + ks) * 16);
+  for (int c = 0; c < L; ++c) {
+    const int chunk = c < LA ? wave * LA + c : wave * (L - LA) + c - LA, r = chunk * 8 + (lane >> 3);
+    const uint32_t piece = (uint32_t)(((lane & 7) ^ ring_swz(r)) * 16);
+    if (c < LA) {
+      const int m = min(r, M - 1 - m0);
+      base[c] = abase;
+      off[c] = (uint32_t)m * (uint32_t)lda * 2u + piece;
+      if (FORM == FORM_GROUPED) {
+        const int from = ga.row_map ? ga.row_map[m0 + m] / ga.row_div : m0 + m;
+        gathered[c] = (const unsigned char*)(A + (size_t)from * lda) + piece;
       }
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j) acc[i][j] = mfma32(bf[ks][j], af[ks][i], acc[i][j]);
-      }
-      // the order of issue: the LDS reads of step ks + 1 go out before the multiplies of step ks
-      __builtin_amdgcn_sched_group_barrier(0x100, FM + FN, 0);
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        if (ks + 1 < KS) __builtin_amdgcn_sched_group_barrier(0x100, FM + FN, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, FM * FN, 0);
-      }
-    }
-  };
-  if (nk > 0) {
-    if constexpr (DEEP) {
-      // Two K steps on their way while a third is multiplied: a step of the small tile is 0.2 us of work, and with
-      // one step in flight every step waited a memory latency (1.1 us a step for weights that come from HBM once).
-      // Two register sets take turns, so the wait before a set is stored names only the older of the two requests.
-      // No branch stands around a request (the compiler would wait for every load behind one): a step beyond the
-      // last is the last step once more, stored where nobody reads it again.
-      Staged r0, r1;
-      const int last = nk - 1;
-      request(r0, 0);
-      request(r1, min(1, last));
-      put(r0, 0);
-      request(r0, min(2, last));
-      __syncthreads();
-      for (int kt = 0; kt < nk; kt += 2) {
-        multiply(0);
-        put(r1, 1);
-        request(r1, min(kt + 3, last));
-        __syncthreads();
-        if (kt + 1 >= nk) break;
-        multiply(1);
-        put(r0, 0);
-        request(r0, min(kt + 4, last));
-        __syncthreads();
-      }
-    } else {
-      Staged r;
-      request(r, 0);
-      put(r, 0);
-      __syncthreads();
-      for (int kt = 0; kt < nk; ++kt) {
-        const int cur = kt & 1;
-        if (kt + 1 < nk) request(r, kt + 1);
-        multiply(cur);
-        if (kt + 1 < nk) put(r, cur ^ 1);
-        __syncthreads();
-      }
+    } else {  // gated: of a wave's CN blocks of 16 the first half is gate rows, the second the up rows of the same outputs
+      const int block = chunk % (2 * CN) / 2;  // the same in all lanes
+      const int n = GATED ? chunk / (2 * CN) * CN * 8 + block % (CN / 2) * 16 + (r & 15) : r;
+      base[c] = wbase[GATED && block >= CN / 2];
+      off[c] = (uint32_t)min(n, N - 1 - n0) * (uint32_t)K * 2u + piece;
     }
   }
-  constexpr int CN = 4 * FN;  // a lane's runs of four columns per row block
-  floatx4 runs[FM][CN];
+  auto load = [&](int t, uint32_t slot, int c) {  // the wave's load c of stage t into the slot at byte `slot`
+    const size_t kbytes = (size_t)t * T_ROW_BYTES;
+    const uint32_t to = lds0 + slot + (c < LA ? (wave * LA + c) * 1024 : TBM * T_ROW_BYTES + (wave * (L - LA) + c - LA) * 1024);
+    if (FORM == FORM_GROUPED && c < LA)
+      load_to_lds_16(gathered[c < LA ? c : 0] + kbytes, to);
+    else
+      load_to_lds_16(base[c] + kbytes, off[c], to);
+  };
+  auto landed = [&](int left) {  // until at most `left` stages of the wave's loads are on their way
+    if (NS >= 6 && left >= 4) wait_loads<4 * L>();
+    else if (NS >= 5 && left >= 3) wait_loads<3 * L>();
+    else if (NS >= 4 && left >= 2) wait_loads<2 * L>();
+    else if (left >= 1) wait_loads<L>();
+    else wait_loads<0>();
+  };
+  auto meet = [&] {  // behind the wave's own reads: the stage that it has in registers now is free for the loads of all
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    T_FENCE();
+    __builtin_amdgcn_s_barrier();
+    T_FENCE();
+  };
+
+  // ---- LDS side: fragment of a block of 16 rows: row = block * 16 + lane % 16, piece = lane / 16 (16 bytes: 8 of 32 k), + 4 for the
+  // stage's second 32 (bit 6 of the address); 16 rows further leaves ring_swz unchanged
+  const int ra = wm * RM * 16 + (lane & 15), rb = wn * CN * 16 + (lane & 15);
+  const int aread = ra * T_ROW_BYTES + (((lane >> 4) ^ ring_swz(ra)) * 16);
+  const int bread = TBM * T_ROW_BYTES + rb * T_ROW_BYTES + (((lane >> 4) ^ ring_swz(rb)) * 16);
+  u32x4 fa[2][2][RM], fb[2][2][CN];  // [set][32 of k][block]
+  auto read = [&](int set, uint32_t slot, int x) {  // read x of a stage, in the order of use
+    const int kk = x / (RM + CN), y = x % (RM + CN);
+    if (y < CN) fb[set][kk][y] = *(const u32x4*)(smem + slot + (bread ^ (kk * 64)) + y * 16 * T_ROW_BYTES);
+    else fa[set][kk][y - CN] = *(const u32x4*)(smem + slot + (aread ^ (kk * 64)) + (y - CN) * 16 * T_ROW_BYTES);
+  };
+  floatx4 acc[RM][CN];
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+  for (int i = 0; i < RM; ++i)
 #pragma unroll
-    for (int j = 0; j < CN; ++j)
+    for (int j = 0; j < CN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  // ---- prologue: every stage of the ring on its way, the first in registers, the second landed
 #pragma unroll
-      for (int c = 0; c < 4; ++c) runs[i][j][c] = acc[i][j / 4][4 * (j % 4) + c];
-  if (HEADS) {
+  for (int s = 0; s < NS; ++s)
+    if (s < nk) {
+#pragma unroll
+      for (int c = 0; c < L; ++c) load(s, s * STAGE, c);
+    }
+  if (nk >= NS) wait_loads<(NS - 1) * L>();
+  else wait_loads<0>();
+  meet();
+#pragma unroll
+  for (int x = 0; x < NR; ++x) read(0, 0, x);
+  if (nk >= NS) wait_loads<(NS - 2) * L>();
+  meet();
+  // Stage t is multiplied from one set of registers while stage t + 1 (its slot: rs) is read into the other and stage t + NS loaded into
+  // the slot of stage t (ws). At its end stage t + 2 has landed: each wave waits for its own loads, the barrier for all waves.
+  uint32_t rs = STAGE, ws = 0;
+  auto stage = [&](auto which, auto full, int t) {
+    constexpr int SET = decltype(which)::value;
+    constexpr bool FULL = decltype(full)::value;  // not among the last stages: every load is asked for
+    const int p = t + NS;
+#pragma unroll
+    for (int n = 0; n < NM; ++n) {
+      const int kk = n / (RM * CN), i = n % (RM * CN) / CN, j = n % CN;
+      // the weight fragment goes in as the first operand: the accumulator then holds the tile transposed (rows = output
+      // columns), so a lane owns four consecutive output columns of one row and stores them at once
+      acc[i][j] = mfma16(fb[SET][kk][j], fa[SET][kk][i], acc[i][j]);
+      T_FENCE();
+      if (n < NR) {
+        read(1 - SET, rs, n);
+        T_FENCE();
+      }
+      if (n == NM - 1) {
+#pragma unroll
+        for (int x = NM; x < NR; ++x) read(1 - SET, rs, x);
+      }
+      if (n % EVERY == EVERY / 2 && n / EVERY < L && (FULL || p < nk)) {
+        load(p, ws, n / EVERY);
+        T_FENCE();
+      }
+    }
+    landed(FULL ? NS - 2 : min(p, nk - 1) - (t + 2));
+    meet();
+    rs = rs == (NS - 1) * STAGE ? 0 : rs + STAGE;
+    ws = ws == (NS - 1) * STAGE ? 0 : ws + STAGE;
+  };
+  int t = 0;
+  for (; t + 1 < nk - NS; t += 2) {
+    stage(std::integral_constant<int, 0>{}, std::true_type{}, t);
+    stage(std::integral_constant<int, 1>{}, std::true_type{}, t + 1);
+  }
+  for (; t < nk; t += 2) {  // (the reads behind the last stage fetch some slot's bytes, which are never multiplied)
+    stage(std::integral_constant<int, 0>{}, std::false_type{}, t);
+    if (t + 1 < nk) stage(std::integral_constant<int, 1>{}, std::false_type{}, t + 1);
+  }
+  if (FORM == FORM_HEADS) {
     bf16_t* o = (bf16_t*)out + (size_t)blockIdx.z * ha.o_stride;
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      const int m = m0 + (wm * FM + i) * 32 + (lane & 31);
+    for (int i = 0; i < RM; ++i) {
+      const int m = m0 + (wm * RM + i) * 16 + (lane & 15);
       if (m >= M) continue;
 #pragma unroll
       for (int j = 0; j < CN; ++j) {
-        const int n = n0 + (wn * CN + j) * 8 + (lane >> 5) * 4;
+        const int n = n0 + (wn * CN + j) * 16 + (lane >> 4) * 4;
         if (n >= N) continue;  // N is a multiple of four
-        floatx4 v = runs[i][j];
+        floatx4 v = acc[i][j];
         if (ha.gate) {
           const u32x2 g = *(const u32x2*)(ha.gate + (size_t)m * ha.ld_gate + (size_t)blockIdx.z * N + n);
           const float gv[4] = {__uint_as_float(g[0] << 16), __uint_as_float(g[0] & 0xffff0000u), __uint_as_float(g[1] << 16),
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
     }
     return;
   }
-  tile_epilogue<GATED, 32, FM, CN, TBM, TBN>(runs, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
+  tile_epilogue<GATED, 16, RM, CN, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
                                              (int)blockIdx.z, (int)gridDim.z);
 }
 
@@ -386,66 +386,77 @@ int jllm_splitk_reduce(const float* partial, int splits, const void* bias, int b
   return 0;
 }
 
-template <int WGM, int WGN, int FM, int FN, bool DEEP>
+// the kernel of a tile, its dynamic LDS allowed for
+template <bool GATED, int FORM, int RM, int CN, int WGM, int WGN, int NS>
+struct Tiled {
+  static constexpr int ROWS = WGM * RM * 16, COLS = WGN * CN * 16 / (GATED ? 2 : 1), THREADS = WGM * WGN * 64;
+  static constexpr int LDS = (WGM * RM * 16 + WGN * CN * 16) * T_ROW_BYTES * NS;
+  static_assert(LDS <= 160 * 1024, "the ring fits");
+  static bool allow() {
+    static bool allowed = false;
+    if (!allowed)
+      allowed = hipFuncSetAttribute((const void*)gemm_mfma_kernel<GATED, FORM, RM, CN, WGM, WGN, NS>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) == hipSuccess;
+    return allowed;
+  }
+};
+
+template <bool GATED, int RM, int CN, int WGM, int WGN, int NS>
 static int launch_tiled(const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype,
                         void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue, GateSpec gs, int splits,
                         float* partial, hipStream_t stream) {
-  constexpr int TBM = WGM * FM * 32, TBN = WGN * FN * 32;
-  const int cols = W2 ? TBN / 2 : TBN;
-  dim3 grid((N + cols - 1) / cols, (M + TBM - 1) / TBM, splits);
+  using T = Tiled<GATED, FORM_PLAIN, RM, CN, WGM, WGN, NS>;
+  dim3 grid((N + T::COLS - 1) / T::COLS, (M + T::ROWS - 1) / T::ROWS, splits);
   if (grid.y > 65535) return 1;
-  const size_t smem = (size_t)2 * (TBM + TBN) * TLD * sizeof(bf16_t);
-  static bool configured = false;
-  if (!configured) {
-    hipError_t e1 = hipFuncSetAttribute((const void*)gemm_mfma_kernel<true, WGM, WGN, FM, FN, DEEP>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    hipError_t e2 = hipFuncSetAttribute((const void*)gemm_mfma_kernel<false, WGM, WGN, FM, FN, DEEP>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    if (e1 != hipSuccess || e2 != hipSuccess) JLLM_FAIL("gemm_mfma: cannot reserve %zu bytes of LDS", smem);
-    configured = true;
-  }
-  if (W2)
-    gemm_mfma_kernel<true, WGM, WGN, FM, FN, DEEP><<<grid, WGM * WGN * 64, smem, stream>>>(
-        (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, nullptr, nullptr, 1, HeadsArgs{});
-  else
-    gemm_mfma_kernel<false, WGM, WGN, FM, FN, DEEP><<<grid, WGM * WGN * 64, smem, stream>>>(
-        (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, nullptr, nullptr, 1, HeadsArgs{});
+  if (!T::allow()) JLLM_FAIL("gemm_mfma: cannot reserve %d bytes of LDS", T::LDS);
+  gemm_mfma_kernel<GATED, FORM_PLAIN, RM, CN, WGM, WGN, NS><<<grid, T::THREADS, T::LDS, stream>>>(
+      (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, GroupArgs{}, HeadsArgs{});
   return 0;
 }
 
-// `splits` > 1 cuts K over gridDim.z (not with the gated epilogue); `partial` then holds splits * M * N floats.
+static bool tiled_rows_fit(int lda, int K) { return lda < (1 << 22) && K < (1 << 22); }  // 256 rows of 8 MB are a 32-bit offset
+
+// `tile`: rows * 1000 + columns of the output tile (of both products' columns with the gated epilogue): 64064 (not gated), 64128, 128128,
+// 128256, 256128.
+// `splits` > 1 cuts K over gridDim.z (not with the gated epilogue; any count that leaves no part without); `partial` then holds
+// splits * M * N floats.
 // `norm_rows` [M][norm_ld] bf16 (with cuts of K and the accumulate epilogue): the RMSNorm of the new rows, made by the reduction.
 // returns 0 when it ran, 1 when the shape is not one it takes, -1 on errors
 extern "C" int jllm_gemm_mfma_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias,
                                    int bias_dtype, void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue,
-                                   float gate_limit, int splits, float* partial, const void* norm_gain, int norm_gain_dtype, float norm_eps,
+                                   float gate_limit, int tile, int splits, float* partial, const void* norm_gain, int norm_gain_dtype, float norm_eps,
                                    void* norm_rows, int norm_ld, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (K <= 0 || (K % TBK) || (lda & 7)) return 1;
+  if (K <= 0 || (K % TBK) || (lda & 7) || !tiled_rows_fit(lda, K)) return 1;
   if (((uintptr_t)A & 15) || ((uintptr_t)W & 15) || (W2 && ((uintptr_t)W2 & 15))) return 1;
   JLLM_TAKE_GATE("gemm_mfma", epilogue, gate_limit, gs);
   if (epilogue < 0 || epilogue > 2 || (epilogue == 2) != (W2 != nullptr)) JLLM_FAIL("gemm_mfma: epilogue %d", epilogue);
   if (epilogue == 1 && out_dtype != JLLM_F32) JLLM_FAIL("gemm_mfma: the accumulate epilogue adds into fp32");
   if (ldo < N) JLLM_FAIL("gemm_mfma: ldo %d < N %d", ldo, N);
   if (splits < 1) splits = 1;
-  if (splits > 1 && (W2 || !partial || (K / TBK) % splits != 0)) JLLM_FAIL("gemm_mfma: %d K splits are not possible here", splits);
+  const int stages = K / TBK, per = (stages + splits - 1) / splits;
+  if (splits > 1 && (W2 || !partial || splits > 65535 || stages <= per * (splits - 1))) JLLM_FAIL("gemm_mfma: %d K splits are not possible here", splits);
   if (norm_rows && splits == 1) JLLM_FAIL("gemm_mfma: the norm is the reduction's, and K is whole");
-  // the large tile when it still gives every compute unit two rounds of work, or when one round of it fills three
-  // quarters of the compute units or more (the small tile would then need a second, half-empty round)
-  const long big_tiles = (long)((N + (W2 ? 127 : 255)) / (W2 ? 128 : 256)) * ((M + 255) / 256);
   int rc;
-  if (splits == 1 && (big_tiles >= 512 || (big_tiles >= 192 && big_tiles <= 256)))
-    rc = launch_tiled<2, 4, 4, 2, false>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, 1, partial, stream);
-  else {
-    // The small tile with two K steps requested ahead where every workgroup has a compute unit to itself: then a step
-    // takes 0.85 us instead of 1.1 (gate/up at 128 rows of the 8B shape, 192 workgroups: 68 -> 54 us; down, 256: 38 ->
-    // 33). Where compute units hold two workgroups the deeper requests of both only crowd the one path into LDS
-    // (384 workgroups: 73 -> 89 us), so those keep one step ahead.
-    const long groups = (long)((N + (W2 ? 63 : 127)) / (W2 ? 64 : 128)) * ((M + 127) / 128) * splits;
-    const int cus = jllm_compute_units();
-    if (cus > 0 && groups <= cus)
-      rc = launch_tiled<2, 2, 2, 2, true>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, splits, partial, stream);
-    else
-      rc = launch_tiled<2, 2, 2, 2, false>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, splits, partial, stream);
+#define TILED_CASE(CODE, ...)                                                                                                                       \
+  case CODE:                                                                                                                                        \
+    rc = W2 ? launch_tiled<true, __VA_ARGS__>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, 1, partial, stream)       \
+            : launch_tiled<false, __VA_ARGS__>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, splits, partial, stream); \
+    break;
+  switch (tile) {
+    TILED_CASE(64128, 2, 4, 2, 2, 3)
+    TILED_CASE(128128, 2, 4, 4, 2, 5)
+    TILED_CASE(128256, 4, 4, 2, 4, 3)
+    TILED_CASE(256128, 4, 4, 4, 2, 3)
+    case 64064:
+      if (!W2) {
+        rc = launch_tiled<false, 2, 2, 2, 2, 4>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, splits, partial, stream);
+        break;
+      }
+      [[fallthrough]];
+    default:
+      JLLM_FAIL("gemm_mfma: no tile of %d rows x %d columns here", tile / 1000, tile % 1000);
   }
+#undef TILED_CASE
   if (rc != 0) return rc;
   JLLM_CHECK_LAUNCH("gemm_mfma");
   if (splits > 1 && norm_rows)
@@ -454,7 +465,7 @@ extern "C" int jllm_gemm_mfma_bf16(const void* A, int lda, const void* W, const 
   return 0;
 }
 
-// The grouped form of the small tile: `tiles` holds (group, first row, rows <= 128) per entry (rows = 0: unused), the
+// The grouped form in tiles of 128 x 128: `tiles` holds (group, first row, rows <= 128) per entry (rows = 0: unused), the
 // weights are [groups][N][K] (and W2 likewise for the gated epilogue), row i of the input is A[row_map[i] / row_div]
 // when `row_map` is given, and output row i is row i of `out`. K whole, epilogues store and gated.
 // returns 0 when it ran, 1 when the shape is not one it takes, -1 on errors
@@ -463,29 +474,24 @@ extern "C" int jllm_gemm_mfma_grouped_bf16(const void* A, int lda, const void* W
                                            int max_tiles, int tile_rows, const int* row_map, int row_div,
                                            hipStream_t stream) {
   if (max_tiles <= 0 || M <= 0) return 0;
-  if ((K & 63) || K <= 0 || N <= 0 || (lda & 7) || max_tiles > 65535) return 1;
+  if ((K & 63) || K <= 0 || N <= 0 || (lda & 7) || max_tiles > 65535 || !tiled_rows_fit(lda, K)) return 1;
   if (((uintptr_t)A & 15) || ((uintptr_t)W & 15) || (W2 && ((uintptr_t)W2 & 15))) return 1;
   JLLM_TAKE_GATE("gemm_mfma_grouped", epilogue, gate_limit, gs);
   if ((epilogue != 0 && epilogue != 2) || (epilogue == 2) != (W2 != nullptr)) JLLM_FAIL("gemm_mfma_grouped: epilogue %d", epilogue);
-  constexpr int TBM = 128, TBN = 128;
-  if (tile_rows != TBM) JLLM_FAIL("gemm_mfma_grouped: tiles of %d rows, this kernel takes %d", tile_rows, TBM);
+  using Plain = Tiled<false, FORM_GROUPED, 2, 4, 4, 2, 5>;
+  using Gated = Tiled<true, FORM_GROUPED, 2, 4, 4, 2, 5>;
+  if (tile_rows != Plain::ROWS) JLLM_FAIL("gemm_mfma_grouped: tiles of %d rows, this kernel takes %d", tile_rows, Plain::ROWS);
   if (ldo < N || row_div < 1) JLLM_FAIL("gemm_mfma_grouped: ldo %d < N %d", ldo, N);
-  const int cols = W2 ? TBN / 2 : TBN;
+  const int cols = W2 ? Gated::COLS : Plain::COLS;
   dim3 grid((N + cols - 1) / cols, max_tiles, 1);
-  const size_t smem = (size_t)2 * (TBM + TBN) * TLD * sizeof(bf16_t);
-  static bool configured = false;
-  if (!configured) {
-    hipError_t e1 = hipFuncSetAttribute((const void*)gemm_mfma_kernel<true, 2, 2, 2, 2, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    hipError_t e2 = hipFuncSetAttribute((const void*)gemm_mfma_kernel<false, 2, 2, 2, 2, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    if (e1 != hipSuccess || e2 != hipSuccess) JLLM_FAIL("gemm_mfma_grouped: cannot reserve %zu bytes of LDS", smem);
-    configured = true;
-  }
+  if (!Plain::allow() || !Gated::allow()) JLLM_FAIL("gemm_mfma_grouped: cannot reserve %d bytes of LDS", Plain::LDS);
+  const GroupArgs ga{tiles, row_map, row_div};
   if (W2)
-    gemm_mfma_kernel<true, 2, 2, 2, 2, false><<<grid, 256, smem, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, nullptr, 0, out,
-                                                                           out_dtype, ldo, M, N, K, epilogue, gs, nullptr, tiles, row_map, row_div, HeadsArgs{});
+    gemm_mfma_kernel<true, FORM_GROUPED, 2, 4, 4, 2, 5><<<grid, Gated::THREADS, Gated::LDS, stream>>>(
+        (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, nullptr, 0, out, out_dtype, ldo, M, N, K, epilogue, gs, nullptr, ga, HeadsArgs{});
   else
-    gemm_mfma_kernel<false, 2, 2, 2, 2, false><<<grid, 256, smem, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, nullptr, nullptr, 0, out, out_dtype,
-                                                                            ldo, M, N, K, epilogue, gs, nullptr, tiles, row_map, row_div, HeadsArgs{});
+    gemm_mfma_kernel<false, FORM_GROUPED, 2, 4, 4, 2, 5><<<grid, Plain::THREADS, Plain::LDS, stream>>>(
+        (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, nullptr, 0, out, out_dtype, ldo, M, N, K, epilogue, gs, nullptr, ga, HeadsArgs{});
   JLLM_CHECK_LAUNCH("gemm_mfma_grouped");
   return 0;
 }
@@ -496,18 +502,13 @@ extern "C" int jllm_gemm_mfma_grouped_bf16(const void* A, int lda, const void* W
 // at 128 x 512 with a gate, here (the tail a launch of its own) 35 and 21.
 int jllm_gemm_mfma_heads(const void* in, int ld_in, int in_hstride, const void* W, void* out, int ld_out, int out_hstride, int M,
                          int H, int N, int K, const void* gate, int ld_gate, hipStream_t stream) {
-  constexpr int TB = 128;
-  const size_t smem = (size_t)2 * (TB + TB) * TLD * sizeof(bf16_t);
-  static bool configured = false;
-  if (!configured) {
-    if (hipFuncSetAttribute((const void*)gemm_mfma_kernel<false, 2, 2, 2, 2, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
-      JLLM_FAIL("gemm_mfma_heads: cannot reserve %zu bytes of LDS", smem);
-    configured = true;
-  }
-  dim3 grid((N + TB - 1) / TB, (M + TB - 1) / TB, H);
+  using T = Tiled<false, FORM_HEADS, 2, 4, 2, 2, 3>;
+  if (!tiled_rows_fit(ld_in, K)) return 1;
+  dim3 grid((N + T::COLS - 1) / T::COLS, (M + T::ROWS - 1) / T::ROWS, H);
   if (grid.y > 65535) return 1;
-  gemm_mfma_kernel<false, 2, 2, 2, 2, false, true><<<grid, 256, smem, stream>>>(
-      (const bf16_t*)in, ld_in, (const bf16_t*)W, nullptr, nullptr, 0, out, JLLM_BF16, ld_out, M, N, K, 0, GateSpec{}, nullptr, nullptr, nullptr, 1,
+  if (!T::allow()) JLLM_FAIL("gemm_mfma_heads: cannot reserve %d bytes of LDS", T::LDS);
+  gemm_mfma_kernel<false, FORM_HEADS, 2, 4, 2, 2, 3><<<grid, T::THREADS, T::LDS, stream>>>(
+      (const bf16_t*)in, ld_in, (const bf16_t*)W, nullptr, nullptr, 0, out, JLLM_BF16, ld_out, M, N, K, 0, GateSpec{}, nullptr, GroupArgs{},
       HeadsArgs{in_hstride, out_hstride, (const bf16_t*)gate, ld_gate});
   JLLM_CHECK_LAUNCH("gemm_mfma_heads");
   return 0;

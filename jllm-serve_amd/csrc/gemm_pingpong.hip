@@ -215,7 +215,7 @@ __device__ __forceinline__ void pingpong_tile(
 
 // Which tile workgroup b of rows x cols takes: workgroups b, b + 8, b + 16 .. share a die, which gets a run of neighbouring tiles,
 // in bands of four columns, row by row inside a band
-__device__ __forceinline__ void pingpong_place(int b, int rows, int cols, int& row, int& col) {
+__device__ __forceinline__ void die_tile(int b, int rows, int cols, int& row, int& col) {
   const int tiles = rows * cols, each = tiles >> 3, more = tiles & 7, die = b & 7;
   const int i = die * each + min(die, more) + (b >> 3);
   const int band = i / (4 * rows), r = i - band * 4 * rows, width = min(4, cols - band * 4);
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
     const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N, int K,
     int epilogue, GateSpec gs, float* __restrict__ partial) {
   int row, col;
-  pingpong_place(blockIdx.x + blockIdx.y * gridDim.x, gridDim.y, gridDim.x, row, col);
+  die_tile(blockIdx.x + blockIdx.y * gridDim.x, gridDim.y, gridDim.x, row, col);
   pingpong_tile<GATED, FM, 2>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, row * 64 * FM, col * (GATED ? 128 : 256));
 }
 
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_mixed_kernel(
   const int whole = M >> 8 << 8, b = blockIdx.x;
   if (b >= wide) {
     int row, col;
-    pingpong_place(b - wide, M >> 8, cols, row, col);
+    die_tile(b - wide, M >> 8, cols, row, col);
     pingpong_tile<GATED, 4, 2>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, row * 256, col * (GATED ? 128 : 256));
   } else if (M - whole > 64) {
     pingpong_tile<GATED, 4, 1>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, whole, b * (GATED ? 256 : 512));

@@ -15,7 +15,7 @@ int jllm_gemm_skinny_norm_bf16(const void* A, int lda, const void* W, const void
         emit_gain_dtype, float* emit_partial, int emit_parts, const float* norm_partial, int norm_parts, float norm_eps, hipStream_t
         stream);
 int jllm_gemm_mfma_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype, void* out, int out_dtype,
-        int ldo, int M, int N, int K, int epilogue, float gate_limit, int splits, float* partial, const void* norm_gain, int
+        int ldo, int M, int N, int K, int epilogue, float gate_limit, int tile, int splits, float* partial, const void* norm_gain, int
         norm_gain_dtype, float norm_eps, void* norm_rows, int norm_ld, hipStream_t stream);
 int jllm_gemm_pingpong_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype, void* out, int
         out_dtype, int ldo, int M, int N, int K, int epilogue, float gate_limit, int tile_rows, int splits, float* partial, const void*

@@ -34,7 +34,7 @@ FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-std=c++17", "-Xclang", "-ta
 # per source: the decode attention multiplies its MFMA accumulators by the softmax rescale now and then; kept in
 # the accumulator half of the register file they would be moved there and back at every turn of the loop
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-FILE_FLAGS = {"attention_decode.hip": VGPR_FORM, "attention_dv_rows.hip": VGPR_FORM, "gemm_skinny.hip": VGPR_FORM}
+FILE_FLAGS = {"attention_decode.hip": VGPR_FORM, "attention_dv_rows.hip": VGPR_FORM, "gemm_skinny.hip": VGPR_FORM, "gemm_mfma.hip": VGPR_FORM}
 
 
 def sources():

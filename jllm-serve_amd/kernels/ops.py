@@ -11,6 +11,7 @@ import bisect
 import contextlib
 import ctypes
 import functools
+import math
 import struct
 import threading
 from typing import Optional, Tuple
@@ -125,7 +126,7 @@ def _declare(lib) -> None:
 _OPTIONAL_SIGS = {
     "jllm_gemm_skinny_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P],
     "jllm_gemm_skinny_norm_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _P, _I, _P, _I, _F, _P],
-    "jllm_gemm_mfma_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _F, _P, _I, _P],
+    "jllm_gemm_mfma_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P, _P, _I, _F, _P, _I, _P],
     "jllm_gemm_pingpong_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P, _P, _I, _F, _P, _I, _P],
     "jllm_gemm_stream_bf16": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _P, _P, _I, _P, _I, _P, _I, _P, _I, _F, _P],
     "jllm_decode_attention_bf16": [_P, _I, _P, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _I, _P],
@@ -757,44 +758,83 @@ def _pingpong_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int]:
     return plan
 
 
-# Estimated times of the tiled products for the choice of `_tiled_plan`, in microseconds. A step's time grows with the compute
-# units at work (they share the memory and the chip's power): "lone" for a few, "full" for all.
-SMALL_DEEP_STEP_US = (0.665, 0.092)   # 64 of K on 128 x 128 tiles, a workgroup per compute unit at most: lone, + for all
-SMALL_STEP_US = (0.629, 1.125)        # the same, two workgroups to a compute unit: a round of few, a full one
-SMALL_ROUND_US = 1.2                  # what a round of workgroups costs beside its steps
-LARGE_STEP_US = {256: (0.576, 0.808), 192: (0.45, 0.687)}  # 32 of K on tiles of 256 or 192 rows by 256 columns: lone, full
-LARGE_ROUND_US = 2.33
-CUT_US = (2.2, 1.255e-6)              # a cut of K: the reduction's launch, and per element of a partial result
+# Estimated times of the tiled products, in microseconds, by tile: 256 and 192 are the rows of the large tiles (256 columns), rows * 1000 +
+# columns the tiles of `jllm_gemm_mfma_bf16`. (fixed, 64 of K with a few compute units at work, with all, a round of workgroups beside
+# its steps), and for the two tiles of which a compute unit holds two: 64 of K where a few compute units hold two, where all do.
+TILE_US = {256: (1.98, 1.043, 1.384, 5.97), 192: (3.19, 0.851, 1.149, 4.49),
+           64064: (3.85, 0.139, 0.275, 0.0, 0.367, 0.483), 64128: (4.30, 0.302, 0.468, 0.0, 0.569, 0.727),
+           128128: (4.11, 0.399, 0.557, 2.39), 128256: (5.0, 0.725, 0.890, 1.84), 256128: (3.99, 0.604, 0.849, 2.87)}
+TILE_CUT_US = (2.07, 1.422e-6)        # a cut of K: the reduction's launch, and per element of a partial result
+TILE_BYTES_PER_US = 5.91e6            # weights from memory; both at once take the root of the sum of squares
 GATED_192_AT_MOST = 0.97              # of the other choice's estimate, for the gated product
+SMALL_TILES = (64064, 64128, 128128, 128256, 256128)
+SMALL_CUTS = (1, 2, 3, 4, 6, 8)
+SMALL_CUT_MIN_K = 256                 # of a part
+SMALL_AT_MOST = 0.96                  # of the large tiles' estimate
+WIDE_LAST = 384                       # tile code: 256 rows, and the last at most 128 in tiles of half the rows and twice the columns
+WIDE_LAST_EXTRA = (0.025, 0.132)      # of a tile's time that a wide one takes longer: up to 64 rows, beyond
 
 
-def _small_us(M: int, N: int, K: int, gated: bool, splits: int) -> float:
-    """The small tile (128 x 128; 128 x 64 outputs of the gated product): one workgroup per compute unit with two K steps
-    requested ahead, or rounds of two per compute unit."""
+def _tile_us(tile: int, M: int, N: int, K: int, gated: bool, cut: int) -> float:
+    """The product in tiles of one kind with K in ``cut`` parts, the reduction included: rounds of workgroups, one or two to a compute
+    unit, against the weights' way from memory.
+
+    The constants were fitted to the times, inside a graph over as many weights as do not fit the caches, of all choices for 25
+    products (0.6B to 14B shapes and five others) at 18 row counts from 70 to 3,000, 9,300 in all: 5 % off on average, and the
+    cheapest by the estimate 2.0 % behind the best of a product's choices on average, 11 % at the 95th of a hundred, 38 % at worst
+    (the best of what the tiles of 256 and 192 rows and gemm_stream.hip offer is 15 % behind on average)."""
     cus = compute_units()
-    groups = -(-N // (64 if gated else 128)) * -(-M // 128) * splits
-    steps = K / 64 / splits
-    if groups <= cus:
-        t = steps * (SMALL_DEEP_STEP_US[0] + SMALL_DEEP_STEP_US[1] * groups / cus)
-    else:
-        lone, full = SMALL_STEP_US
-        rounds, last = divmod(groups, 2 * cus)
-        t = rounds * (steps * full + SMALL_ROUND_US)
-        if last:
-            t += steps * (lone + (full - lone) * last / (2 * cus)) + SMALL_ROUND_US
-    return t + (CUT_US[0] + CUT_US[1] * M * N * splits if splits > 1 else 0.0)
+    fixed, lone, full, round_us, *pair = TILE_US[256 if tile == WIDE_LAST else tile]
+    rows, columns = divmod(tile, 1000) if tile > 1000 else (256 if tile == WIDE_LAST else tile, 256)
+    across = -(-N // (columns // 2 if gated else columns))
+    groups = (M // 256 * across + -(-across // 2) if tile == WIDE_LAST else across * -(-M // rows)) * cut
+    steps = -(-K // (64 * cut))
+    rounds, last = divmod(groups, 2 * cus if pair else cus)
+    t = rounds * (steps * (pair[1] if pair else full) + round_us)
+    step = lone + (full - lone) * min(last, cus) / cus
+    if last > cus:
+        step = pair[0] + (pair[1] - pair[0]) * (last - cus) / cus
+    if last:
+        t += steps * step + round_us
+    if tile == WIDE_LAST:
+        t += WIDE_LAST_EXTRA[M % 256 > 64] * steps * (full if rounds else step)
+    t = fixed + math.hypot(t, N * K * (4 if gated else 2) / TILE_BYTES_PER_US)
+    return t + (TILE_CUT_US[0] + TILE_CUT_US[1] * M * N * cut if cut > 1 else 0.0)
 
 
 def _large_us(M: int, N: int, K: int, gated: bool, rows: int, cut: int) -> float:
-    """The two-group kernel: rounds of one workgroup per compute unit."""
-    cus = compute_units()
-    lone, full = LARGE_STEP_US[rows]
-    steps = K / 32 / cut
-    rounds, last = divmod(-(-N // (128 if gated else 256)) * -(-M // rows) * cut, cus)
-    t = rounds * (steps * full + LARGE_ROUND_US)
-    if last:
-        t += steps * (lone + (full - lone) * last / cus) + LARGE_ROUND_US
-    return t + (CUT_US[0] + CUT_US[1] * M * N * cut if cut > 1 else 0.0)
+    return _tile_us(rows, M, N, K, gated, cut)
+
+
+@functools.lru_cache(maxsize=8192)
+def _small_best(tiles64: int, N: int, K: int, gated: bool, normed: bool) -> Tuple[float, int, int]:
+    """(estimated time, tile, parts of K) of the cheapest choice of `jllm_gemm_mfma_bf16` for ``tiles64`` times 64 rows (and so for all
+    row counts that have these tiles); ``normed``: the norm of the new rows included, which the reduction makes where K is cut."""
+    M, cus = 64 * tiles64, compute_units()
+    best = (float("inf"), 128128, 1)
+    for tile in SMALL_TILES:
+        if gated and tile == 64064:
+            continue
+        rows, columns = divmod(tile, 1000)
+        groups = -(-N // (columns // 2 if gated else columns)) * -(-M // rows)
+        for cut in SMALL_CUTS:
+            if cut > 1 and (gated or K // cut < SMALL_CUT_MIN_K or groups * cut > 3 * cus or K // 64 <= -(-(K // 64) // cut) * (cut - 1)):
+                continue
+            t = _tile_us(tile, M, N, K, gated, cut) + (_norm_us(M, N) if normed and cut == 1 else 0.0)
+            if t < best[0]:
+                best = t, tile, cut
+    return best
+
+
+def _small_us(M: int, N: int, K: int, gated: bool) -> float:
+    return _small_best(-(-M // 64), N, K, gated, False)[0]
+
+
+NORM_PASS_US = (4.0, 0.6e-6)        # the norm behind an adding product with K whole (a cut's reduction makes it): launch, per element
+
+
+def _norm_us(M: int, N: int) -> float:
+    return NORM_PASS_US[0] + NORM_PASS_US[1] * M * N
 
 
 @functools.lru_cache(maxsize=8192)
@@ -821,7 +861,7 @@ def _tiled_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int]:
     rows, cut = _pingpong_plan(M, N, K, gated)
     if K % 64 == 0:
         cut = cut if rows else _k_splits(M, N, K, gated)
-        least = _large_us(M, N, K, gated, rows, cut) if rows else _small_us(M, N, K, gated, cut)
+        least = _large_us(M, N, K, gated, rows, cut) if rows else _small_us(M, N, K, gated)
         if gated:
             least *= GATED_192_AT_MOST
         if K >= 128 and (gated or M >= PINGPONG_MIN_ROWS):
@@ -842,26 +882,8 @@ def _tiled_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int]:
 _own_tiled_plan = _tiled_plan  # as it is, whoever puts another in its place
 
 
-WIDE_LAST = 384                     # tile code: 256 rows, and the last at most 128 in tiles of half the rows and twice the columns
-WIDE_LAST_EXTRA = (0.17, 0.25)      # of a tile's time that a wide one takes longer: up to 64 rows, beyond
-FINER_CUTS = 8                      # the two-group kernel's parts of K, any count up to this
+FINER_CUTS = 8                      # the large tiles' parts of K, any count up to this
 FINER_AT_MOST = 0.95                # of the plan's estimate
-NORM_PASS_US = (4.0, 0.6e-6)        # the norm behind an adding product with K whole (a cut's reduction makes it): launch, per element
-
-
-def _wide_last_us(M: int, N: int, K: int, gated: bool, cut: int) -> float:
-    """The two-group kernel with wide tiles for the last rows."""
-    cus = compute_units()
-    lone, full = LARGE_STEP_US[256]
-    steps = K / 32 / cut
-    cols = -(-N // (128 if gated else 256))
-    rounds, last = divmod((M // 256 * cols + -(-cols // 2)) * cut, cus)
-    t = rounds * (steps * full + LARGE_ROUND_US)
-    step = lone + (full - lone) * last / cus
-    if last:
-        t += steps * step + LARGE_ROUND_US
-    t += WIDE_LAST_EXTRA[M % 256 > 64] * steps * (full if rounds else step)
-    return t + (CUT_US[0] + CUT_US[1] * M * N * cut if cut > 1 else 0.0)
 
 
 @functools.lru_cache(maxsize=8192)
@@ -888,8 +910,9 @@ def _finer_tiles(M: int, N: int, K: int, gated: bool, normed: bool, rows: int, c
     two dozen choices per product anew)."""
 
     def us(tile, c):
-        t = _wide_last_us(M, N, K, gated, c) if tile == WIDE_LAST else _large_us(M, N, K, gated, tile, c) if tile else _small_us(M, N, K, gated, c)
-        return t + (NORM_PASS_US[0] + NORM_PASS_US[1] * M * N if normed and c == 1 else 0.0)
+        if not tile:
+            return _small_best(-(-M // 64), N, K, gated, normed)[0]
+        return _tile_us(tile, M, N, K, gated, c) + (_norm_us(M, N) if normed and c == 1 else 0.0)
 
     least, best = FINER_AT_MOST * us(rows, cut), (rows, cut)
     for tile in (192, 256, WIDE_LAST):
@@ -1097,13 +1120,13 @@ WIDE_MOST_ROWS = 1024
 WIDE_ADD_COLUMNS = 2048
 WIDE_LEAST_K = 1024               # the shortest K it was measured at
 WIDE_BLOCK_US = (0.275, 0.0198)   # 64 of k on 32 weight and 64 activation rows, and per 8 rows more of either
-WIDE_FIXED_US = {64: 4.8, 128: 7.2}   # the launch, the first blocks and the end, by activation rows per workgroup
+WIDE_FIXED_US = {64: 3.9, 128: 7.2}   # the launch, the first blocks and the end, by activation rows per workgroup
 WIDE_PAIR = (1.35, 1.8)           # two workgroups of 64 rows on a compute unit: a few of them, all
 WIDE_MERGE_US = (2.5, 0.06)       # parts of K: the way through memory, and per KB of sums that the last workgroup reads
 WIDE_BYTES_PER_US = 5.3e6         # weights from memory
-TILED_FIXED_US = 6.0              # what the tiled kernels' estimates leave out
-WIDE_AT_MOST = 0.97               # of the tiled kernels' estimate
-NORM_LAUNCH_US = 4.0              # a norm of few rows as a launch of its own
+# a norm that rides on a product of 128 rows, of the tiled kernels' estimate (o and gate/up in turn, us, here / tiled: 0.6B 19.3 / 18.2,
+# 1.7B 30.1 / 29.7; beyond 128 rows 2 to 30 behind)
+WIDE_NORM_AT_MOST = 1.25
 
 
 def _wide_us(M: int, N: int, K: int, gated: bool, rows: int, tile: int, parts: int) -> float:
@@ -1162,24 +1185,50 @@ def _wide_plan(M: int, N: int, K: int, gated: bool, adds: int = 0) -> Optional[T
     kernels win: 8B gate/up at 200 rows 79.9 / 101, down 44.8 / 54.9."""
     if not STREAM_MAX_ROWS < M <= WIDE_MOST_ROWS or K % 128 or N % 16 or K < WIDE_LEAST_K or (adds and N > WIDE_ADD_COLUMNS):
         return None
-    rows, cut = _tiled_plan(M, N, K, gated)
-    best = WIDE_AT_MOST * (TILED_FIXED_US + (_large_us(M, N, K, gated, rows, cut) if rows else _small_us(M, N, K, gated, cut)))
-    if adds == ADDS_AND_NORM:
-        best += NORM_LAUNCH_US
     t, plan = _wide_best(-(-M // 64), min(M, 128), N, K, gated)
-    return plan if t < best else None
+    limit = _own_choice(M, N, K, gated, adds == ADDS_AND_NORM)[2]
+    return plan if t < (limit * WIDE_NORM_AT_MOST if adds == ADDS_AND_NORM and M <= 128 else limit) else None
 
 
 _NO_NORM = (None, F32, 0.0, None, 0)
 
 
+_own_k_splits, _own_tiles = _k_splits, _tiles  # as they are, whoever puts others in their place
+
+
+@functools.lru_cache(maxsize=8192)
+def _own_choice(M: int, N: int, K: int, gated: bool, normed: bool) -> Tuple[int, int, float]:
+    """(tile, ways K is cut, estimated time) of a product that the tiled kernels take: a large tile (256, 192 or `WIDE_LAST`:
+    `_tiles`), or one of `SMALL_TILES` where its estimate is below `SMALL_AT_MOST` of the large one's or no large one fits. The time
+    counts the norm behind the product where one is asked for."""
+    tile, cut = _own_tiles(M, N, K, gated, normed, *_own_tiled_plan(M, N, K, gated))
+    if K % 64:
+        return tile or 128128, cut, float("inf")
+    us, small, small_cut = _small_best(-(-M // 64), N, K, gated, normed)
+    if tile:
+        large = _tile_us(tile, M, N, K, gated, cut) + (_norm_us(M, N) if normed and cut == 1 else 0.0)
+        if us >= SMALL_AT_MOST * large:
+            return tile, cut, large
+    return small, small_cut, us
+
+
+def _tiled_choice(M: int, N: int, K: int, gated: bool, normed: bool) -> Tuple[int, int]:
+    """The choice's tile and cut; a plan or a count of cuts that was put in the place of the rules' own stands (where it names no
+    large tile, with tiles of 128 x 128)."""
+    if _tiled_plan is _own_tiled_plan and _k_splits is _own_k_splits and _tiles is _own_tiles:
+        return _own_choice(M, N, K, gated, normed)[:2]
+    tile, cut = _tiles(M, N, K, gated, normed, *_tiled_plan(M, N, K, gated))
+    return (tile, cut) if tile else (128128, _k_splits(M, N, K, gated) if K % 64 == 0 else 1)
+
+
 def _cut_takes_norm(M: int, N: int, K: int) -> bool:
     """Whether the adding product of M rows goes to a tiled kernel that cuts K: its reduction then makes the norm of the new
-    rows as well."""
-    if M <= STREAM_MAX_ROWS or K % 64 or N % 4 or N > 8192 or _wide_plan(M, N, K, False, ADDS) is not None:
+    rows as well. The weight-streaming kernel, where it takes such a product, leaves the norm to a launch."""
+    if M <= STREAM_MAX_ROWS or K % 64 or N % 4 or N > 8192 or _tiled_choice(M, N, K, False, True)[1] == 1:
         return False
-    rows, cut = _tiles(M, N, K, False, True, *_tiled_plan(M, N, K, False))
-    return (cut if rows else _k_splits(M, N, K, False)) > 1
+    if _wide_plan(M, N, K, False, ADDS) is None:
+        return True
+    return _own_choice(M, N, K, False, True)[2] < _wide_best(-(-M // 64), min(M, 128), N, K, False)[0] + _norm_us(M, N)
 
 
 def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0, norm=_NO_NORM) -> bool:
@@ -1194,26 +1243,28 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0, norm=_NO_
     N = w.shape[0]
     head = (_ptr(a), a.stride(0), _ptr(w), _ptr(w2), _ptr(bias), _code(bias.dtype) if bias is not None else F32,
             _ptr(out), _code(out.dtype), out.stride(0), M, N, K, int(epilogue), float(gate_limit))
-    plan = _row_plan(M, N, K, w2 is not None, _adds(epilogue))
-    if M <= SKINNY_MAX_ROWS:
+    plan = _row_plan(M, N, K, w2 is not None, _adds(epilogue)) if norm is _NO_NORM else None  # (the norm is a tiled kernel's reduction's)
+    if plan is None:
+        pass
+    elif M <= SKINNY_MAX_ROWS:
         if _try("jllm_gemm_skinny_bf16", *head, plan[0], _stream()):
             return True
-    elif plan is not None and K % 128 == 0:
+    elif K % 128 == 0:
         sums, arrivals = _stream_scratch(M, N, w2 is not None, a, plan)
         if _try("jllm_gemm_stream_bf16", *head, *plan, _ptr(sums), _ptr(arrivals), None, 0, None, F32, None, 0, None, 0, 0.0, _stream()):
             return True
-    tile_rows, cut = _tiles(M, N, K, w2 is not None, norm is not _NO_NORM, *_tiled_plan(M, N, K, w2 is not None))
-    if tile_rows:
+    tile, cut = _tiled_choice(M, N, K, w2 is not None, norm is not _NO_NORM)
+    if cut == 1 and norm is not _NO_NORM:
+        return False  # (K stays whole: no reduction to make the norm)
+    if tile < 1000:
         partial = torch.empty((cut * M * N,), dtype=torch.float32, device=a.device) if cut > 1 else None
-        if _try("jllm_gemm_pingpong_bf16", *head, tile_rows, cut, _ptr(partial), *norm, _stream()):
+        if _try("jllm_gemm_pingpong_bf16", *head, tile, cut, _ptr(partial), *norm, _stream()):
             return True
-    splits = _k_splits(M, N, K, w2 is not None) if K % 64 == 0 else 1
-    if splits == 1 and norm is not _NO_NORM:
-        return False  # (the other kernel declined, and here K stays whole: no reduction to make the norm)
-    partial = torch.empty((splits * M * N,), dtype=torch.float32, device=a.device) if splits > 1 else None
-    if _try("jllm_gemm_mfma_bf16", *head, splits, _ptr(partial), *norm, _stream()):
-        return True
-    return False
+        tile, cut = 128128, _k_splits(M, N, K, w2 is not None) if K % 64 == 0 else 1
+        if cut == 1 and norm is not _NO_NORM:
+            return False
+    partial = torch.empty((cut * M * N,), dtype=torch.float32, device=a.device) if cut > 1 else None
+    return _try("jllm_gemm_mfma_bf16", *head, tile, cut, _ptr(partial), *norm, _stream())
 
 
 def qk_norm_rope_store(qkv: torch.Tensor, positions: torch.Tensor, slots: Optional[torch.Tensor],

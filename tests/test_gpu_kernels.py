@@ -241,6 +241,35 @@ def test_gemm_two_group_kernel_with_wide_last_rows(ops, monkeypatch, M, N, K, cu
     assert bool(((got[1].double() - ref).abs() <= K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
 
 
+@pytest.mark.parametrize("M,N,K,cut", [(65, 68, 64, 1), (129, 131, 128, 1), (255, 260, 320, 2), (257, 516, 448, 3), (300, 1028, 1088, 5)])
+def test_gemm_small_tiles(ops, monkeypatch, M, N, K, cut):
+    """Every tile of the small kernel against every other, bit for bit, and float64: one row beyond a tile and one short of it, K of one
+    stage, shorter than the rings and longer, an odd number of stages, whole and in parts of unequal length, every epilogue. (Gated:
+    tiles that lie inside the output take the hardware's exponential and reciprocal, others the library's, some 2^-22 of the value.)"""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M + K)
+    a = torch.randn(M, K, device=DEV, generator=gen).bfloat16()
+    w, w2 = ((torch.randn(N, K, device=DEV, generator=gen) * K ** -0.5).bfloat16() for _ in range(2))
+    bias = torch.randn(N, device=DEV, generator=gen)
+    monkeypatch.setattr(ops, "_wide_plan", lambda *_: None)
+    got = []
+    for tile in ops.SMALL_TILES:
+        monkeypatch.setattr(ops, "_tiled_choice", lambda m, n, k, gated, normed: (128128 if gated and tile == 64064 else tile, 1 if gated else cut))
+        ops.reset_stats()
+        res = torch.ones(M, N, device=DEV)
+        ops.gemm(a, w, bias=bias, out=res, epilogue=ops.EPI_ADD)
+        got.append([res, ops.gemm(a, w, out_dtype=torch.float32), ops.gemm(a, w, bias=bias), ops.gemm(a, w, w2=w2, epilogue=ops.EPI_GATED)])
+        assert ops.stats()["ran"] == {"jllm_gemm_mfma_bf16": 4}
+    for other in got[1:]:
+        assert all(torch.equal(x, y) for x, y in zip(got[0][:3], other[:3]))
+        x, y = got[0][3].double(), other[3].double()
+        assert bool(((x - y).abs() <= 2.0 ** -7 * torch.maximum(x.abs(), y.abs())).all())
+    ref = a.double() @ w.double().T  # fp32 sums of K rounded products: K 2^-24 of the sum of magnitudes at most
+    assert bool(((got[0][1].double() - ref).abs() <= K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
+    u = a.double() @ w2.double().T
+    assert bf16_close(got[0][3], ref / (1 + torch.exp(-ref)) * u, ulps=1.01)[0]
+
+
 @pytest.mark.parametrize("M,N,K,cut", [(256, 256, 128, 1), (257, 300, 160, 1), (320, 700, 288, 2), (300, 516, 1056, 3), (330, 260, 2080, 5)])
 def test_gemm_ring_of_half_stages(ops, monkeypatch, M, N, K, cut):
     """A ring of halves of stages of 64: K of two stages, of whole ones and with a last one of 32, alone and as the end of the last of
