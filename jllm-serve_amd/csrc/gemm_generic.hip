@@ -217,6 +217,124 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_f32_tile_kernel(const TA* _
   }
 }
 
+// The same tiles with fp32 operands whose rows are whole lines (K a multiple of 32, rows on 16 bytes): stages of 32 k go straight from
+// memory into a ring of RING places in LDS (lds_ring.h), RING - 1 of them on their way. Nothing is transposed on the way: a step of a
+// fragment is one word a lane, and of the rows of 128 bytes with their pieces turned by ring_swz the 64 words that a read names (16
+// rows at k = 4 s .. 4 s + 3) fall into all 64 banks. One barrier a stage, two steps before the stage ends: in front of it a wave waits
+// for its own share of the next stage, behind it the place of the stage before is asked for again, and the next stage's first fragments
+// are read while the last steps are multiplied. The sums are those of the kernel above, bit for bit.
+// It is bound by the matrix cores (32 cycles a step and accumulator: 157 TFLOP/s) and by what rounds of workgroups leave idle; the kernel
+// above also waits for its four 4-byte writes to LDS for every 16 bytes, and once a step for its fragments. us, the kernel above / this:
+// 1,000 rows of 4,096 x 1,024 76.6 / 65.9, of 4,096 x 2,048 146 / 125 (134 TFLOP/s), of 1,024 x 3,072 68.6 / 52.4, gated 3,072 x 1,024
+// 119.7 / 101.3; 487 of 2,048 x 6,144 132 / 101, of 1,024 x 2,048 (32 x 32) 29.6 / 22.9; 40 rows of 1,024 x 3,072 28.1 / 25.1 (a chain of
+// 768 steps, three times its cycles: four waves alone on a compute unit, bound by the wait for memory). With the barrier behind the last step and the
+// compiler's own order of reads and multiplies: 71.6, 137, 65.3, 113.9.
+template <bool GATED, int WM, int WN, int FM, int FN, int RING>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_f32_ring_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W,
+                                                            const float* __restrict__ W2, const void* __restrict__ bias,
+                                                            int bias_dtype, void* __restrict__ out, int out_dtype, int ldo,
+                                                            int M, int N, int K, int epilogue, GateSpec gs) {
+  constexpr int TM = WM * FM * 16, TN = WN * FN * 16, NW = GATED ? 2 : 1;
+  constexpr int ROWS = TM + NW * TN, STAGE = ROWS * 32;  // rows of a stage; floats of one place of the ring
+  constexpr int LOADS = ROWS / 8 / (WM * WN);            // of 1 KB, eight rows each, per wave and stage
+  static_assert(ROWS % (8 * WM * WN) == 0 && RING >= 3 && RING <= 8, "whole loads per wave");
+  extern __shared__ __align__(1024) float lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
+  const int stages = K / 32;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)lds;
+  const float* at[LOADS];  // this lane's piece of each of the wave's loads of the next stage
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int row = (wave * LOADS + i) * 8 + (lane >> 3);  // the tile's rows: A, then W, then W2
+    const int piece = (lane & 7) ^ ring_swz(row & 15);
+    const int r = row - TM, n = min(n0 + (r >= TN ? r - TN : r), N - 1);
+    at[i] = (row < TM ? A + (size_t)min(m0 + row, M - 1) * lda : (GATED && r >= TN ? W2 : W) + (size_t)n * K) + piece * 4;
+  }
+  auto issue = [&](int place) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      load_to_lds_16(at[i], lds0 + (uint32_t)(place * STAGE * 4 + (wave * LOADS + i) * 1024));
+      at[i] += 32;
+    }
+  };
+  floatx4 acc[NW][FM][FN];
+#pragma unroll
+  for (int z = 0; z < NW; ++z)
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[z][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int fr = lane & 15;
+  const float* word[8];  // of step s: row `fr`, k = 4 s + lane / 16 of the first block of a place
+#pragma unroll
+  for (int s = 0; s < 8; ++s) word[s] = lds + fr * 32 + ((s ^ ring_swz(fr)) << 2) + (lane >> 4);
+  // A step's fragments are asked for two steps ahead, also across stages (behind the last one what lies in the ring, which nothing
+  // multiplies), and the compiler is held to that order: left to itself it reads in front of the use and waits there.
+  float a[4][FM], w[4][NW][FN];
+  auto read = [&](int place, int s) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i) a[s & 3][i] = word[s][place * STAGE + (wm * FM + i) * 512];
+#pragma unroll
+    for (int z = 0; z < NW; ++z)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) w[s & 3][z][j] = word[s][place * STAGE + TM * 32 + ((z * WN + wn) * FN + j) * 512];
+  };
+  auto landed = [&](int behind) {  // what is next is there for all waves, with so many stages behind it still on their way
+    switch (min(RING - 2, behind)) {
+      case 6: wait_loads<6 * LOADS>(); break;
+      case 5: wait_loads<5 * LOADS>(); break;
+      case 4: wait_loads<4 * LOADS>(); break;
+      case 3: wait_loads<3 * LOADS>(); break;
+      case 2: wait_loads<2 * LOADS>(); break;
+      case 1: wait_loads<1 * LOADS>(); break;
+      default: wait_loads<0>();
+    }
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+#pragma unroll
+  for (int t = 0; t < RING - 1; ++t)
+    if (t < stages) issue(t);
+  landed(stages - 1);
+  read(0, 0);
+  read(0, 1);
+  for (int t0 = 0; t0 < stages; t0 += RING) {
+#pragma unroll
+    for (int place = 0; place < RING; ++place) {
+      const int t = t0 + place;
+      if (t >= stages) break;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {  // k = 32 t + 4 s .. + 3
+        if (s == 6 && t + 1 < stages) {
+          landed(min(RING - 3, stages - 2 - t));
+          if (t + RING - 1 < stages) issue((place + RING - 1) % RING);  // where stage t - 1 was: all waves are in stage t
+        }
+        read(s < 6 ? place : (place + 1) % RING, (s + 2) & 7);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int z = 0; z < NW; ++z)
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[z][i][j] = mfma_f32(w[s & 3][z][j], a[s & 3][i], acc[z][i][j]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    const int m = m0 + (wm * FM + i) * 16 + fr;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int n = n0 + (wn * FN + j) * 16 + (lane >> 4) * 4;
+      if (m < M) finish_four<GATED>(acc[0][i][j], acc[NW - 1][i][j], m, n, N, bias, bias_dtype, out, out_dtype, ldo, epilogue, gs);
+    }
+  }
+}
+
 // Up to 16 rows (decode steps of the 32-bit path). An output's chain is 8 cycles per k (a 16 x 16 x 4 product takes 32), so
 // a product of few weight rows is bound by that chain (3,072 k: 11 us) as long as nothing else stands in it: a workgroup
 // owns 16 weight rows and all activation rows, one wave (two with the gated epilogue, one per weight matrix) does nothing
@@ -452,7 +570,8 @@ __global__ __launch_bounds__((GATED ? 6 : 5) * 64) void gemm_f32_few_kernel(cons
 //
 // The tile is the one with the smallest estimated time: rounds of workgroups (one per compute unit) times the tile's
 // products, the smaller tiles a little dearer for their share of loads. K cannot be cut (one accumulator per output), so
-// where large tiles leave compute units idle only smaller ones fill them.
+// where large tiles leave compute units idle only smaller ones fill them. The prices hold for both kernels: a full round of 64 x 64 takes
+// 16.4 us per 1,024 k through the ring, one of 128 x 128 59.7.
 struct F32Tile {
   int rows, cols;  // of the output
 };
@@ -493,6 +612,23 @@ static int launch_f32_tile(const F32Args& g, hipStream_t stream) {
   return 0;
 }
 
+template <bool GATED, int WM, int WN, int FM, int FN, int RING>
+static int launch_f32_ring(const F32Args& g, hipStream_t stream) {
+  constexpr int TM = WM * FM * 16, TN = WN * FN * 16;
+  constexpr size_t smem = (size_t)RING * (TM + (GATED ? 2 : 1) * TN) * 128;
+  static bool configured = smem <= 65536;
+  if (!configured) {
+    if (hipFuncSetAttribute((const void*)gemm_f32_ring_kernel<GATED, WM, WN, FM, FN, RING>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+      JLLM_FAIL("gemm: cannot reserve %zu bytes of LDS", smem);
+    configured = true;
+  }
+  dim3 grid((g.N + TN - 1) / TN, (g.M + TM - 1) / TM);
+  if (grid.y > 65535) JLLM_FAIL("gemm: M=%d is too large for this kernel", g.M);
+  gemm_f32_ring_kernel<GATED, WM, WN, FM, FN, RING><<<grid, WM * WN * 64, smem, stream>>>(
+      (const float*)g.A, g.lda, (const float*)g.W, (const float*)g.W2, g.bias, g.bias_dtype, g.out, g.out_dtype, g.ldo, g.M, g.N, g.K, g.epilogue, g.gs);
+  return 0;
+}
+
 template <bool GATED>
 static int launch_f32_few(const F32Args& g, hipStream_t stream) {
   using F = F32Few<GATED>;
@@ -518,6 +654,18 @@ static int launch_f32(const F32Args& g, hipStream_t stream) {
     return 0;
   }
   const int tile = f32_tile(g.M, g.N, g.W2 != nullptr);
+  if constexpr (WIDE && sizeof(TA) == 4 && sizeof(TW) == 4) {
+    // whole lines of 128 bytes of every row: the ring, faster at all of 17 .. 1,000 rows and eight shapes of products (by 6 to 25 %)
+    if (g.K % 32 == 0) {
+      if (g.W2)
+        return tile == 0   ? launch_f32_ring<true, 2, 4, 4, 1, 3>(g, stream)
+               : tile == 1 ? launch_f32_ring<true, 4, 2, 1, 1, 4>(g, stream)
+                           : launch_f32_ring<true, 2, 2, 1, 1, 5>(g, stream);
+      return tile == 0   ? launch_f32_ring<false, 2, 4, 4, 2, 3>(g, stream)
+             : tile == 1 ? launch_f32_ring<false, 2, 4, 2, 1, 4>(g, stream)
+                         : launch_f32_ring<false, 2, 2, 1, 1, 8>(g, stream);
+    }
+  }
   if (g.W2)
     return tile == 0   ? launch_f32_tile<TA, TW, true, 2, 4, 4, 1, 32, WIDE>(g, stream)
            : tile == 1 ? launch_f32_tile<TA, TW, true, 4, 2, 1, 1, 64, WIDE>(g, stream)

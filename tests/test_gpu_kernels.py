@@ -650,6 +650,32 @@ def test_float32_products_of_few_rows(ops, N, K):
     assert torch.equal(ops.gemm(tiny[:3], small, exact=True), ops.gemm(tiny, small, exact=True)[:3])
 
 
+@pytest.mark.parametrize("M,N,tile", [(17, 33, 2), (33, 1030, 2), (700, 1100, 1), (769, 1030, 1), (2041, 4090, 0), (1921, 4092, 0)])
+@pytest.mark.parametrize("K", [32, 64, 96, 128, 352])
+def test_float32_products_of_whole_lines(ops, M, N, tile, K):
+    """Many rows, K in stages of 32 (one, fewer than a ring holds, exactly those, more), edges of tiles, every epilogue: the bits of
+    the same rows in batches of 16, which another kernel takes, also with an infinity in one row; a stride between the rows."""
+    assert [ops.library().jllm_f32_tile(M, N, gated) for gated in (0, 1)] == [tile, tile]
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M + K)
+    a = torch.randn(M, K + 4, device=DEV, generator=gen)[:, :K]
+    w, w2 = (torch.randn(N, K, device=DEV, generator=gen) * K ** -0.5 for _ in range(2))
+    a[1, K // 2] = float("inf")
+    bias = torch.randn(N, device=DEV, generator=gen)
+    res = torch.randn(M, N, device=DEV, generator=gen)
+
+    def forms(x, r):
+        r = r.clone()
+        ops.gemm(x, w, bias=bias, out=r, epilogue=ops.EPI_ADD, exact=True)
+        return [r, ops.gemm(x, w, bias=bias, exact=True), ops.gemm(x, w, out_dtype=torch.bfloat16, exact=True),
+                ops.gemm(x, w, w2=w2, epilogue=ops.EPI_GATED, exact=True)]
+
+    many = forms(a, res)
+    for at in {0, min(16, M - 16), M // 2 if M > 100 else 0, M - 16}:
+        for got, want in zip(many, forms(a[at:at + 16], res[at:at + 16])):
+            assert torch.equal(torch.nan_to_num(got[at:at + 16], nan=7.0), torch.nan_to_num(want, nan=7.0)), at
+
+
 @pytest.mark.parametrize("M,N,K,exponent", [(3, 17, 67, 0), (16, 20, 200, -70), (20, 33, 70, 0), (40, 35, 68, -71), (130, 40, 36, -70)])
 def test_float32_products_round_once_per_multiply_add(ops, M, N, K, exponent):
     """The 32-bit products on operands of 24 bits, whose products a multiply-add must not round, against the C library's
