@@ -235,9 +235,10 @@ struct GdrArgs {
   const int* row_req;
   const int* state_slots;
   int n_rows, heads, kv_heads, dk, dv;
+  int req0;  // the launch's first request
 };
 
-// thread = wave * 64 + c * 16 + part: column blockIdx.z * 16 + wave * 4 + c, key rows part * E .. + E
+// thread = wave * 64 + c * 16 + part: column blockIdx.x * 16 + wave * 4 + c, key rows part * E .. + E
 // CHANNEL: the decay is a vector over the key channels (S's rows) instead of one number per head:
 //   S <- diag(g) S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q = (diag(g) S_old)^T q + (k . q) u
 // FEW: the form for steps of few rows per request (decoding). It leaves out the interleaved walk over a full chunk, whose
@@ -254,8 +255,8 @@ __global__ __launch_bounds__(256) void gated_delta_kernel(GdrArgs A) {
   __shared__ __align__(16) float sm[C * ROWF];
   const int tid = threadIdx.x;
   const int part = tid & 15, cw = tid >> 4;  // cw: the column within the workgroup
-  const int req = blockIdx.x, h = blockIdx.y;
-  const int col0 = blockIdx.z * GDR_COLS;
+  const int req = A.req0 + blockIdx.z, h = blockIdx.y;
+  const int col0 = blockIdx.x * GDR_COLS;
   const int col = col0 + cw;
   const bool col_on = col < A.dv;
   int lo, n;
@@ -439,12 +440,17 @@ extern "C" int jllm_gated_delta(const void* qkv, int ldc, const void* proj, int 
                                                                             kv_heads, dk, decay_rows, ldd);
     })
   })
-  GdrArgs A{qkv, ldc, prep, ldq, state, out, ldo, row_req, state_slots, n_rows, heads, kv_heads, dk, dv};
-  dim3 grid(n_requests, heads, (dv + GDR_COLS - 1) / GDR_COLS);
+  GdrArgs A{qkv, ldc, prep, ldq, state, out, ldo, row_req, state_slots, n_rows, heads, kv_heads, dk, dv, 0};
+  // The requests come last in the order of dispatch. Neighbouring workgroups go to different dies: with the requests first, four
+  // requests of 16 heads x 128 columns had all workgroups of the longest one on two of the eight dies, two to a compute unit to
+  // the end; now the two are of different requests, and the longer one's has the unit alone for its rest (150 .. 1,390 rows: 388 -> 328
+  // us). Single rows of four requests take 6.6 us so, 7.0 with the requests first.
+  const int col_groups = (dv + GDR_COLS - 1) / GDR_COLS;
   const int per_lane = (dk + GDR_PARTS - 1) / GDR_PARTS;
   const bool few = n_rows <= 2 * n_requests;
 #define GDR_LAUNCH(E)                                                           \
-  do {                                                                          \
+  for (A.req0 = 0; A.req0 < n_requests; A.req0 += 65535) {                      \
+    const dim3 grid(col_groups, heads, min(n_requests - A.req0, 65535));        \
     if (channel && few)                                                         \
       gated_delta_kernel<T, E, true, true><<<grid, 256, 0, stream>>>(A);        \
     else if (channel)                                                           \
@@ -453,16 +459,17 @@ extern "C" int jllm_gated_delta(const void* qkv, int ldc, const void* proj, int 
       gated_delta_kernel<T, E, false, true><<<grid, 256, 0, stream>>>(A);       \
     else                                                                        \
       gated_delta_kernel<T, E, false, false><<<grid, 256, 0, stream>>>(A);      \
-  } while (0)
+  }
   JLLM_DISPATCH_1(dtype, T, {
-    if (per_lane <= 2)
-      GDR_LAUNCH(2);
-    else if (per_lane <= 4)
-      GDR_LAUNCH(4);
-    else if (per_lane <= 8)
-      GDR_LAUNCH(8);
-    else
-      GDR_LAUNCH(16);
+    if (per_lane <= 2) {
+      GDR_LAUNCH(2)
+    } else if (per_lane <= 4) {
+      GDR_LAUNCH(4)
+    } else if (per_lane <= 8) {
+      GDR_LAUNCH(8)
+    } else {
+      GDR_LAUNCH(16)
+    }
   })
 #undef GDR_LAUNCH
   JLLM_CHECK_LAUNCH("gated_delta");
