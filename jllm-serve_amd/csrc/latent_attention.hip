@@ -34,7 +34,12 @@
 __device__ __forceinline__ float lm_exp_diff(float a, float b) { return a == -INFINITY ? 0.f : __expf(a - b); }
 
 // RT: 16-dim blocks of the latent the accumulators hold at most; DKS: 32-dim steps of a key row at most
-template <int RT, int DKS>
+// WHOLE: the sizes are exactly those, and nothing in the loops is conditional on them: a step behind a condition waits for its own LDS
+// read, eighteen times a score and sixteen a sum. Single rows of 512 + 64 entries, us with the merge, before / so (a workgroup is a chain
+// of blocks of 64 keys, 2.8 -> 1.9 us each at 16 heads, 7.3 -> 4.0 at 32): 8 rows of 16 heads and a window of 1,024 in ranges of 128 keys
+// 20.2 / 16.2, in ranges of 64 18.1 / 14.7; 32 heads 24.4 / 18.2 and 18.1 / 14.7; 24 rows of 32 heads and 2,000 keys in ranges of 384 58 / 39.
+// Sizes in between keep the conditions: padded to these they would multiply up to three times their entries and hold a compute unit's LDS.
+template <int RT, int DKS, bool WHOLE>
 __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
     const bf16_t* __restrict__ qa, int ldq, bf16_t* __restrict__ out, int ldo, const bf16_t* __restrict__ cache,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ tiles,
@@ -63,9 +68,10 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
   const int my_h = hb * HB + v;
   const bool live = v < HB && my_h < H;
   const bool wave_live = kpar || qwave * 16 < HB;  // (a wave without a live query vector only helps to load)
-  const int dks = (Dk + 31) >> 5, r16 = R >> 4;
+  const int dks = WHOLE ? DKS : (Dk + 31) >> 5, r16 = WHOLE ? RT : R >> 4;
   constexpr int RTH = (RT + 1) / 2;  // accumulators of one wave: its half of the latent's 16-dim blocks
-  const int j_lo = rhalf ? (r16 + 1) / 2 : 0, nj = rhalf ? r16 - (r16 + 1) / 2 : (r16 + 1) / 2;
+  static_assert(!WHOLE || RT % 2 == 0, "two equal halves");
+  const int j_lo = rhalf ? (r16 + 1) / 2 : 0, nj = WHOLE ? RTH : rhalf ? r16 - (r16 + 1) / 2 : (r16 + 1) / 2;
   const int psh = __builtin_ctz(page_size);
   const int* tbl = block_table + (size_t)req * max_blocks;
 
@@ -75,7 +81,7 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
 #pragma unroll
     for (int j = 0; j < DKS; ++j) {
       const int d = 32 * j + 8 * q4;
-      qf[j] = (live && j < dks && d < Dk) ? *(const u32x4*)(qrow + d) : u32x4{0u, 0u, 0u, 0u};
+      qf[j] = (WHOLE || (live && j < dks && d < Dk)) ? *(const u32x4*)(qrow + d) : u32x4{0u, 0u, 0u, 0u};  // (WHOLE: another head's where not live, unused)
     }
   }
   floatx4 acc[RTH];
@@ -95,13 +101,13 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
     const int key = min(max(blk * LM_KEYS + srow, kb), ke);  // a key outside the range is masked below and reads one inside it
     const bf16_t* src = cache + ((((size_t)tbl[key >> psh]) << psh) + (key & (page_size - 1))) * Dk + scol;
 #pragma unroll
-    for (int i = 0; i < CPT; ++i) staged[i] = (scol + 64 * i < Dk) ? *(const uint4*)(src + 64 * i) : uint4{0u, 0u, 0u, 0u};
+    for (int i = 0; i < CPT; ++i) staged[i] = (WHOLE || scol + 64 * i < Dk) ? *(const uint4*)(src + 64 * i) : uint4{0u, 0u, 0u, 0u};
   };
   auto put = [&](bf16_t* buf) {
     bf16_t* dst = buf + srow * LD + scol;
 #pragma unroll
     for (int i = 0; i < CPT; ++i)
-      if (scol + 64 * i < dks * 32) *(uint4*)(dst + 64 * i) = staged[i];
+      if (WHOLE || scol + 64 * i < dks * 32) *(uint4*)(dst + 64 * i) = staged[i];
   };
   const int blk_last = ke >> 6;
   int cur = 0;
@@ -610,21 +616,30 @@ __global__ __launch_bounds__(256) void latent_attention_merge_kernel(const float
   }
 }
 
-template <int RT, int DKS>
-static int lm_launch(dim3 grid, size_t smem, hipStream_t stream, const void* qa, int ldq, void* out, int ldo, const void* cache,
+template <int RT, int DKS, bool WHOLE>
+static int lm_launch_as(dim3 grid, size_t smem, hipStream_t stream, const void* qa, int ldq, void* out, int ldo, const void* cache,
                      const int* block_table, int max_blocks, const int* tiles, const int* positions, int H, int R, int Dk,
                      int page_size, int window, float scale, const float* sink, int HB, int LD, int split, float* part) {
   static size_t reserved = 0;
   if (smem > 48 * 1024 && smem > reserved) {
-    if (hipFuncSetAttribute((const void*)latent_attention_mfma_kernel<RT, DKS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (hipFuncSetAttribute((const void*)latent_attention_mfma_kernel<RT, DKS, WHOLE>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)smem) != hipSuccess)
       JLLM_FAIL("latent_attention: cannot reserve %zu bytes of LDS", smem);
     reserved = smem;
   }
-  latent_attention_mfma_kernel<RT, DKS><<<grid, LM_WAVES * 64, smem, stream>>>(
+  latent_attention_mfma_kernel<RT, DKS, WHOLE><<<grid, LM_WAVES * 64, smem, stream>>>(
       (const bf16_t*)qa, ldq, (bf16_t*)out, ldo, (const bf16_t*)cache, block_table, max_blocks, tiles, positions, H, R, Dk,
       page_size, window, scale, sink, HB, LD, split, part);
   return 0;
+}
+
+template <int RT, int DKS>
+static int lm_launch(dim3 grid, size_t smem, hipStream_t stream, const void* qa, int ldq, void* out, int ldo, const void* cache,
+                     const int* block_table, int max_blocks, const int* tiles, const int* positions, int H, int R, int Dk,
+                     int page_size, int window, float scale, const float* sink, int HB, int LD, int split, float* part) {
+  return R == RT * 16 && Dk == DKS * 32
+             ? lm_launch_as<RT, DKS, true>(grid, smem, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, LD, split, part)
+             : lm_launch_as<RT, DKS, false>(grid, smem, stream, qa, ldq, out, ldo, cache, block_table, max_blocks, tiles, positions, H, R, Dk, page_size, window, scale, sink, HB, LD, split, part);
 }
 
 template <int NJ, int DKS>

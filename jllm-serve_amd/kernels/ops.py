@@ -1623,7 +1623,12 @@ def _fast_latent_attention(qa, out, cache, block_table, row_req, positions, head
                 split, n_z, _ptr(part), _stream())
 
 
-LATENT_SPLIT_MIN = 128  # keys a workgroup takes at least when a row's keys are cut over several
+# keys a workgroup takes at least when a row's keys are cut over several: one block of the kernel, since a workgroup is a chain of blocks. us
+# at ranges of 64 / 128 / 256: 16 heads of 512 + 64 entries, a window of 1,024, 1 row 13.4 / 15.6 / 19.3, 8 rows 14.7 / 16.2 / 19.4, 16 rows
+# 15.8 / 16.2 / 19.6; 32 heads 12.5 / 17.2 / 25.3, 14.7 / 18.2 / 25.6, 18.9 / 18.8 / 26.1. One row that may reach 8,192 keys, at
+# 2,000: 18.5 in 44 ranges of 192, 19.3 in 33 of 256 (32 heads 22.1 / 25.2)
+LATENT_SPLIT_MIN = 64
+LATENT_SPAN_MIN = 256  # shorter spans are not cut
 
 
 def _latent_split(rows: int, heads: int, window: int, max_ctx: int):
@@ -1633,12 +1638,12 @@ def _latent_split(rows: int, heads: int, window: int, max_ctx: int):
     span = min(window, max_ctx) if window > 0 else max_ctx
     groups = rows * -(-heads // 64)
     want = -(-2 * compute_units() // max(groups, 1))
-    if span < 2 * LATENT_SPLIT_MIN or want < 2:
+    if span < LATENT_SPAN_MIN or want < 2:
         return 0, 1
     split = max(LATENT_SPLIT_MIN, -(-(-(-span // want)) // 64) * 64)
     n_z = -(-span // split) + 1  # a span of that many keys touches at most this many absolute ranges
     while n_z > 64:  # the merge takes up to 64 ranges
-        split *= 2
+        split += 64
         n_z = -(-span // split) + 1
     return (split, n_z) if n_z > 2 else (0, 1)
 

@@ -370,6 +370,38 @@ def test_latent_attention_of_runs_of_rows(H, R, Dk, window):
     assert bool(((got.view(-1, H, R).double().cpu() - torch.cat(want)).abs() <= torch.cat(room)).all())
 
 
+@pytest.mark.parametrize("H, R, Dk", [(16, 512, 576), (40, 512, 576), (5, 64, 128), (70, 128, 256), (16, 512, 568)])
+@pytest.mark.parametrize("window", [0, 100, 300])
+def test_latent_attention_of_single_rows_of_whole_sizes(H, R, Dk, window):
+    """Single rows at the sizes whose loops carry no condition (and one entry group short of them), in ranges of one block and uncut:
+    keys that end one below, at and one beyond a block or a range, places without keys hold NaN; the definition in 64 bits."""
+    from jllm_serve_amd.kernels import ops
+    g = torch.Generator().manual_seed(H + R + window)
+    page, width, pos = 16, 48, [0, 62, 63, 64, 255, 256, 699, 767]
+    n = len(pos)
+    assert ops._latent_split(n, H, window, width * page) == ((0, 1) if window == 100 else (64, 6) if window == 300 else (64, 13))
+    cache = torch.full((n * width, page, Dk), float("nan"), dtype=torch.bfloat16)
+    table = torch.randperm(n * width, generator=g).to(torch.int32).view(n, width)
+    q, sink, scale = torch.randn(n, H, Dk, generator=g).bfloat16(), torch.randn(H, generator=g), 1.5 * Dk ** -0.5
+    want, room = [], []
+    for r, at in enumerate(pos):
+        keys = torch.randn(at + 1, Dk, generator=g).bfloat16()
+        for k in range(0, at + 1, page):
+            part = keys[k:k + page]
+            cache[int(table[r, k // page]), :len(part)] = part
+        keys = keys[max(0, at + 1 - window) if window else 0:].double()
+        z = q[r].double() @ keys.T * scale
+        p = torch.softmax(torch.cat([z, sink.double()[:, None]], dim=1), dim=1)[:, :-1]
+        want.append(p @ keys[:, :R])
+        # a score: Dk products' fp32 sum, in any order, and its part in exp; the probabilities and the result as bf16
+        size = (q[r].double().abs() @ keys.abs().T).amax(dim=1, keepdim=True) * scale
+        room.append((2.0 ** -9 + 2.0 * Dk * 2.0 ** -24 * size + 2.0 ** -18) * (p @ keys[:, :R].abs()) + 2.0 ** -8 * want[-1].abs())
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    meta = {"tiles_dev": i32([(i, i, 1, p) for i, p in enumerate(pos)]).flatten(), "n_tiles": n, "single_rows": True, "max_context": width * page}
+    got = ops.latent_attention(q.view(n, -1).to(DEV), cache.to(DEV), table.to(DEV), i32(list(range(n))), i32(pos), H, R, window, scale, sink.to(DEV), meta=meta)
+    assert bool(((got.view(n, H, R).double().cpu() - torch.stack(want)).abs() <= torch.stack(room)).all())
+
+
 @pytest.mark.parametrize("H, R, Dk, window, single_runs", [(40, 512, 576, 0, False), (40, 144, 168, 90, False), (17, 128, 256, 33, False),
                                                            (16, 512, 576, 0, True), (16, 512, 576, 70, True), (3, 96, 128, 0, True), (20, 64, 96, 0, False)])
 def test_latent_attention_gives_a_row_the_same_bits_in_runs_and_alone(H, R, Dk, window, single_runs):
