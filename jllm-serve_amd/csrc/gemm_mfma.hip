@@ -31,7 +31,7 @@
 #define T_ROW_BYTES (TBK * 2)  // a tile row in LDS: 128 bytes = 8 pieces of 16
 #define T_FENCE() __builtin_amdgcn_sched_barrier(0)
 
-enum { FORM_PLAIN = 0, FORM_GROUPED = 1, FORM_HEADS = 2 };
+enum { FORM_PLAIN = 0, FORM_GROUPED = 1, FORM_HEADS = 2, FORM_BY_COLUMNS = 3 };  // the last: plain, in another order of the tiles
 
 // What the per-head form takes beside the operands: head h = blockIdx.z multiplies the rows at A + h * a_stride with
 // its own weights (W [heads][N][K]) and writes bf16 at out + h * o_stride, times sigmoid(gate[row][h * N + column]) where a
@@ -49,11 +49,26 @@ struct GroupArgs {
   int row_div;
 };
 
+// Workgroups go to the eight dies in turn, so with a multiple of eight columns those that share a weight tile are on one die and with
+// four more on two; with an odd number every die fetches every weight tile. There workgroups b, b + 8, b + 16 .. (one die) take a
+// run of neighbouring tiles, column by column (`by_rows`: 2^32 / rows rounded up; a division would cost 0.3 us). us, by number / so:
+// 400 rows of 3,392 x 2,048 in tiles of 64 x 64 (53 columns) 20.4 / 14.1, 1,100 in 64 x 128 (27) 36.6 / 22.5, 1,025 of 6,208 x 4,096 in
+// 128 x 256 (25) 74.1 / 54.4, 900 of 22,592 x 4,096 (89) 234.8 / 168.3; ten columns (2,560 x 9,728, 400 rows) 51.4 / 46.2.
+// Where the number is a multiple of four it gains nothing (2,560 x 4,096, K whole, in 20 columns of 128: 6 % slower).
+static bool by_columns(int rows, int cols) { return rows > 1 && cols % 4 != 0 && (unsigned long long)rows * rows * cols < (1ull << 32); }
+static uint32_t by_rows_of(uint32_t rows) { return (uint32_t)(((1ull << 32) + rows - 1) / rows); }
+__host__ __device__ __forceinline__ void column_tile(uint32_t b, uint32_t rows, uint32_t cols, uint32_t by_rows, int& row, int& col) {
+  const uint32_t tiles = rows * cols, each = tiles >> 3, more = tiles & 7, die = b & 7;
+  const uint32_t i = die * each + (die < more ? die : more) + (b >> 3);
+  col = (int)(((uint64_t)i * by_rows) >> 32);
+  row = (int)(i - col * rows);
+}
+
 template <bool GATED, int FORM, int RM, int CN, int WGM, int WGN, int NS>
 __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
     const void* __restrict__ bias, int bias_dtype, void* __restrict__ out, int out_dtype, int ldo, int M, int N, int K,
-    int epilogue, GateSpec gs, float* __restrict__ partial, GroupArgs ga, HeadsArgs ha) {
+    int epilogue, GateSpec gs, float* __restrict__ partial, GroupArgs ga, HeadsArgs ha, uint32_t by_rows) {
   constexpr int WAVES = WGM * WGN, TBM = WGM * RM * 16, TBN = WGN * CN * 16, STAGE = (TBM + TBN) * T_ROW_BYTES;
   constexpr int LA = TBM / 8 / WAVES, L = LA + TBN / 8 / WAVES;  // load instructions (8 rows each) per wave and stage
   constexpr int NM = 2 * RM * CN, NR = 2 * (RM + CN);            // multiplies and LDS reads of a stage
@@ -64,8 +79,8 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int wm = wave / WGN, wn = wave % WGN;
-  // (no order of the tiles by dies here: these products gain nothing by it, and its divisions cost 0.3 us)
-  const int row = blockIdx.y, col = blockIdx.x;
+  int row = blockIdx.y, col = blockIdx.x;
+  if (FORM == FORM_BY_COLUMNS) column_tile(blockIdx.x + blockIdx.y * gridDim.x, gridDim.y, gridDim.x, by_rows, row, col);
   int m0 = row * TBM;
   if (FORM == FORM_GROUPED) {
     const int rows = ga.groups[3 * row + 2];
@@ -386,6 +401,14 @@ int jllm_splitk_reduce(const float* partial, int splits, const void* bias, int b
   return 0;
 }
 
+// For tests: the row and column (out[0], out[1]) of the tile that workgroup b of a plain product's rows x cols takes
+extern "C" int jllm_tiled_place(int rows, int cols, int b, int* out) {
+  if (rows < 1 || cols < 1 || b < 0 || b >= rows * cols) return -1;
+  out[0] = b / cols, out[1] = b % cols;
+  if (by_columns(rows, cols)) column_tile(b, rows, cols, by_rows_of(rows), out[0], out[1]);
+  return 0;
+}
+
 // the kernel of a tile, its dynamic LDS allowed for
 template <bool GATED, int FORM, int RM, int CN, int WGM, int WGN, int NS>
 struct Tiled {
@@ -400,17 +423,26 @@ struct Tiled {
   }
 };
 
+template <bool GATED, int FORM, int RM, int CN, int WGM, int WGN, int NS>
+static int launch_tiled_as(dim3 grid, uint32_t by_rows, const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype,
+                           void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue, GateSpec gs, float* partial, hipStream_t stream) {
+  using T = Tiled<GATED, FORM, RM, CN, WGM, WGN, NS>;
+  if (!T::allow()) JLLM_FAIL("gemm_mfma: cannot reserve %d bytes of LDS", T::LDS);
+  gemm_mfma_kernel<GATED, FORM, RM, CN, WGM, WGN, NS><<<grid, T::THREADS, T::LDS, stream>>>(
+      (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, GroupArgs{}, HeadsArgs{}, by_rows);
+  return 0;
+}
+
 template <bool GATED, int RM, int CN, int WGM, int WGN, int NS>
 static int launch_tiled(const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype,
                         void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue, GateSpec gs, int splits,
                         float* partial, hipStream_t stream) {
   using T = Tiled<GATED, FORM_PLAIN, RM, CN, WGM, WGN, NS>;
-  dim3 grid((N + T::COLS - 1) / T::COLS, (M + T::ROWS - 1) / T::ROWS, splits);
+  const dim3 grid((N + T::COLS - 1) / T::COLS, (M + T::ROWS - 1) / T::ROWS, splits);
   if (grid.y > 65535) return 1;
-  if (!T::allow()) JLLM_FAIL("gemm_mfma: cannot reserve %d bytes of LDS", T::LDS);
-  gemm_mfma_kernel<GATED, FORM_PLAIN, RM, CN, WGM, WGN, NS><<<grid, T::THREADS, T::LDS, stream>>>(
-      (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, GroupArgs{}, HeadsArgs{});
-  return 0;
+  if (by_columns(grid.y, grid.x))
+    return launch_tiled_as<GATED, FORM_BY_COLUMNS, RM, CN, WGM, WGN, NS>(grid, by_rows_of(grid.y), A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, stream);
+  return launch_tiled_as<GATED, FORM_PLAIN, RM, CN, WGM, WGN, NS>(grid, 0, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, stream);
 }
 
 static bool tiled_rows_fit(int lda, int K) { return lda < (1 << 22) && K < (1 << 22); }  // 256 rows of 8 MB are a 32-bit offset
@@ -488,10 +520,10 @@ extern "C" int jllm_gemm_mfma_grouped_bf16(const void* A, int lda, const void* W
   const GroupArgs ga{tiles, row_map, row_div};
   if (W2)
     gemm_mfma_kernel<true, FORM_GROUPED, 2, 4, 4, 2, 5><<<grid, Gated::THREADS, Gated::LDS, stream>>>(
-        (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, nullptr, 0, out, out_dtype, ldo, M, N, K, epilogue, gs, nullptr, ga, HeadsArgs{});
+        (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, nullptr, 0, out, out_dtype, ldo, M, N, K, epilogue, gs, nullptr, ga, HeadsArgs{}, 0);
   else
     gemm_mfma_kernel<false, FORM_GROUPED, 2, 4, 4, 2, 5><<<grid, Plain::THREADS, Plain::LDS, stream>>>(
-        (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, nullptr, 0, out, out_dtype, ldo, M, N, K, epilogue, gs, nullptr, ga, HeadsArgs{});
+        (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, nullptr, 0, out, out_dtype, ldo, M, N, K, epilogue, gs, nullptr, ga, HeadsArgs{}, 0);
   JLLM_CHECK_LAUNCH("gemm_mfma_grouped");
   return 0;
 }
@@ -509,7 +541,7 @@ int jllm_gemm_mfma_heads(const void* in, int ld_in, int in_hstride, const void* 
   if (!T::allow()) JLLM_FAIL("gemm_mfma_heads: cannot reserve %d bytes of LDS", T::LDS);
   gemm_mfma_kernel<false, FORM_HEADS, 2, 4, 2, 2, 3><<<grid, T::THREADS, T::LDS, stream>>>(
       (const bf16_t*)in, ld_in, (const bf16_t*)W, nullptr, nullptr, 0, out, JLLM_BF16, ld_out, M, N, K, 0, GateSpec{}, nullptr, GroupArgs{},
-      HeadsArgs{in_hstride, out_hstride, (const bf16_t*)gate, ld_gate});
+      HeadsArgs{in_hstride, out_hstride, (const bf16_t*)gate, ld_gate}, 0);
   JLLM_CHECK_LAUNCH("gemm_mfma_heads");
   return 0;
 }

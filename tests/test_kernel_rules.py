@@ -251,6 +251,25 @@ def test_a_new_row_count_does_not_weigh_every_choice_again(monkeypatch):
     assert 0 < once == len(weighed)
 
 
+def test_order_of_the_tiles_of_odd_numbers_of_columns():
+    """Every tile is taken once, whatever the numbers; with an odd number of columns, and with two more than a multiple of four, the
+    workgroups of a die (every eighth) share the weights of as few columns as their number allows."""
+    import ctypes
+    place = ops.library().jllm_tiled_place
+    out = (ctypes.c_int * 2)()
+    for rows, cols in ((1, 1), (1, 53), (2, 3), (5, 53), (7, 53), (7, 27), (18, 27), (3, 97), (9, 25), (8, 89), (13, 10), (4, 20), (5, 16), (40, 9), (300, 7), (70, 177)):
+        taken, dies = set(), [set() for _ in range(8)]
+        for b in range(rows * cols):
+            assert place(rows, cols, b, out) == 0
+            taken.add((out[0], out[1]))
+            dies[b % 8].add(out[1])
+        assert taken == {(r, c) for r in range(rows) for c in range(cols)}, (rows, cols)
+        if rows > 1 and cols % 4:
+            most = -(-rows * cols // 8)
+            assert max(map(len, dies)) <= (most + rows - 2) // rows + 1, (rows, cols)
+    assert place(4, 20, 80, out) == -1
+
+
 def test_declared_arguments_are_those_of_the_sources():
     """Every entry point's declared argument types against its definition: a pointer declared as an int would reach the
     kernel cut to 32 bits."""
