@@ -1,4 +1,4 @@
-// Hammers the native host library (page pool, step layout) with random work, for a build under AddressSanitizer and
+// Hammers the native host library (page pool, step layout, products' choices) with random work, for a build under AddressSanitizer and
 // UndefinedBehaviorSanitizer on the CPU: every buffer handed to the library is allocated at exactly its stated
 // length, so a read or write one element too far is a report. The reference hammers its pool the same way
 // (src/test/java/org/robomiri/jllm/KvPoolTest.java:147). Prints "hammer ok" and returns 0, or says what disagreed.
@@ -223,6 +223,37 @@ void hammer_layout(std::mt19937& rng, int rounds) {
   }
 }
 
+// The estimates and walks over the products' choices, at sizes from one row to beyond 32 bits of elements: what a walk returns is one
+// of the kinds, priced as the estimate prices it.
+void hammer_tiles(std::mt19937& rng, int rounds) {
+  std::vector<JllmTileKind> kinds(4);
+  const int32_t shapes[4][2] = {{64, 64}, {128, 128}, {192, 256}, {256, 256}};
+  for (int i = 0; i < 4; ++i)
+    kinds[i] = JllmTileKind{2.0 + i, 0.2 * (i + 1), 0.3 * (i + 1), 1.0, 0.4 * (i + 1), 0.5 * (i + 1), 1000 + i, shapes[i][0], shapes[i][1], i == 0, i == 3, i == 0, i == 2};
+  const std::vector<int32_t> cuts = {1, 2, 3};
+  const JllmTileRules rules{kinds.data(), cuts.data(), 2, 2, 3, 256, 1001, 256, 1024, 8, 5e6, 2.0, 1e-6, 4.0, 1e-6, {0.1, 0.2}};
+  const JllmStreamRules stream{0.3, 0.02, 4.0, 7.0, 1.3, 1.8, 2.5, 0.06, 5e6, 256, 4};
+  auto any = [&](int most) { return 1 + (int)(rng() % (1u << (1 + rng() % most))); };
+  for (int round = 0; round < rounds; ++round) {
+    const int M = any(22), N = any(18), K = any(16), gated = (int)(rng() & 1), normed = (int)(rng() & 1);
+    std::vector<JllmTileChoice> out(2);
+    jllm_small_tiles(&rules, M, N, K, gated, out.data());
+    for (int i = 0; i < 2; ++i) {
+      const double us = jllm_tile_us(&rules, out[i].tile - 1000, M, N, K, gated, out[i].cut);
+      const double norm = i == 1 && out[i].cut == 1 ? rules.norm_us + rules.norm_element_us * M * (double)N : 0.0;
+      EXPECT((out[i].tile == 1000 && !gated) || out[i].tile == 1001, "round %d: tile %d", round, out[i].tile);
+      EXPECT(out[i].us == us + norm && us > 0, "round %d: %f us, priced at %f", round, out[i].us, us);
+    }
+    std::vector<JllmTileChoice> best = {{1e30, 0, 0}};
+    jllm_large_tiles(&rules, M, N, K, gated, normed, best.data());
+    if (best[0].tile) EXPECT(best[0].tile == 1003 ? M % 256 >= 1 && M % 256 <= 128 : best[0].tile == 1002, "round %d: tile %d of %d rows", round, best[0].tile, M);
+    EXPECT(jllm_tile_us(&rules, 4, M, N, K, gated, 1) == -1.0, "round %d: a tile that is not there", round);
+    std::vector<int32_t> plan(3);
+    jllm_stream_tiles(&stream, M, N, 128 * any(8), gated, plan.data());
+    EXPECT(plan[0] >= 32 && plan[0] <= 128 && (plan[1] == 64 || plan[1] == 128) && plan[2] >= 1 && plan[2] <= 4, "round %d: plan %d %d %d", round, plan[0], plan[1], plan[2]);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -231,6 +262,7 @@ int main(int argc, char** argv) {
   std::mt19937 rng(seed);
   for (int pages : {1, 2, 37, 300}) hammer_pool(rng, pages, 20000);
   hammer_layout(rng, rounds);
+  hammer_tiles(rng, rounds);
   if (failures) {
     std::fprintf(stderr, "hammer: %d checks failed\n", failures);
     return 1;

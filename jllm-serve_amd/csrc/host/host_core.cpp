@@ -21,7 +21,7 @@ inline int ctz32(int v) { return __builtin_ctz((unsigned)v); }
 
 extern "C" {
 
-int jllm_host_abi_version() { return 2; }
+int jllm_host_abi_version() { return 3; }
 
 void* jllm_pool_new(int num_pages) {
   if (num_pages < 1) return nullptr;

@@ -61,5 +61,42 @@ struct JllmStepBatch {
 // power of two): nothing is read beyond the stated lengths.
 int64_t jllm_step_layout(const JllmStepBatch* batch, int32_t* out, int64_t capacity, JllmStepSizes* sizes);
 
+// ---- estimated times of the tiled products: what a tile costs, and what all of them do (kernels/ops.py says how)
+struct JllmTileKind {
+  double fixed, lone, full, round_us, few, all;
+  int32_t code, rows, columns;
+  int32_t two;         // a compute unit holds two workgroups
+  int32_t wide_last;   // the last rows, at most 128 of them, in tiles of half the rows and twice the columns
+  int32_t plain_only;  // not with the gated epilogue
+  int32_t odd_cuts;    // K in one, two or four parts is not weighed
+};
+struct JllmTileRules {
+  const JllmTileKind* kinds;  // n_small of the small kernel, then n_large of the large one
+  const int32_t* small_cuts;
+  int32_t n_small, n_large, n_small_cuts, cus;
+  int32_t fallback;               // the tile where none has a time
+  int32_t small_part, large_part; // K of a part at least
+  int32_t large_cuts;             // parts at most
+  double bytes_per_us, cut_us, cut_element_us, norm_us, norm_element_us, wide_extra[2];
+};
+struct JllmTileChoice {
+  double us;
+  int32_t tile, cut;
+};
+double jllm_tile_us(const JllmTileRules* rules, int kind, int M, int N, int K, int gated, int cut);  // -1: no such tile or cut
+// the cheapest of the small kernel's: out[0] of the product alone, out[1] with the norm behind it where K stays whole
+void jllm_small_tiles(const JllmTileRules* rules, int M, int N, int K, int gated, JllmTileChoice* out);
+// the cheapest of the large kernel's where it takes less than best->us; `normed`: with that norm
+void jllm_large_tiles(const JllmTileRules* rules, int M, int N, int K, int gated, int normed, JllmTileChoice* best);
+
+// ---- the same for the weight-streaming kernel on more than 64 rows: (weight rows, activation rows, parts of K) per workgroup
+struct JllmStreamRules {
+  double block_us, block_row_us;  // 64 of k, on 32 weight and 64 activation rows; per 8 rows more of either
+  double fixed_64, fixed_128, pair_few, pair_all, merge_us, merge_kb_us, bytes_per_us;
+  int32_t cus, least_blocks;      // 128-wide blocks of K that a part has at least
+};
+double jllm_stream_us(const JllmStreamRules* rules, int M, int N, int K, int gated, int rows, int tile, int parts);
+void jllm_stream_tiles(const JllmStreamRules* rules, int M, int N, int K, int gated, int32_t* plan);  // the cheapest
+
 int jllm_host_abi_version();
 }

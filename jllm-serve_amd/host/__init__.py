@@ -1,4 +1,4 @@
-"""The native host library (csrc/host/): page pool and step layout, reached through ctypes.
+"""The native host library (csrc/host/): page pool, step layout and the estimates of the tiled products, reached through ctypes.
 
 It holds no GPU code, so it builds with the C++ compiler alone and loads on a machine without a GPU; it is built at
 its first use when no current build is found (a second or two).
@@ -10,7 +10,7 @@ import threading
 
 from ..kernels import build as _build
 
-ABI_VERSION = 2
+ABI_VERSION = 3
 _lock = threading.Lock()
 _lib = None
 
@@ -31,6 +31,28 @@ class StepBatchArgs(ctypes.Structure):
                 ("page_size", ctypes.c_int32), ("n_groups", ctypes.c_int32), ("arena_rows", ctypes.c_int32),
                 ("arena", ctypes.c_void_p), ("arena_stride", ctypes.c_void_p), ("table_rows", ctypes.c_void_p),
                 ("table_lens", ctypes.c_void_p)]
+
+
+class TileKind(ctypes.Structure):
+    """JllmTileKind of csrc/host/host_core.h; the next three likewise."""
+    _fields_ = [(n, ctypes.c_double) for n in ("fixed", "lone", "full", "round_us", "few", "all")] + \
+               [(n, ctypes.c_int32) for n in ("code", "rows", "columns", "two", "wide_last", "plain_only", "odd_cuts")]
+
+
+class TileRules(ctypes.Structure):
+    _fields_ = [("kinds", ctypes.POINTER(TileKind)), ("small_cuts", i32p)] + \
+               [(n, ctypes.c_int32) for n in ("n_small", "n_large", "n_small_cuts", "cus", "fallback", "small_part", "large_part", "large_cuts")] + \
+               [(n, ctypes.c_double) for n in ("bytes_per_us", "cut_us", "cut_element_us", "norm_us", "norm_element_us")] + \
+               [("wide_extra", ctypes.c_double * 2)]
+
+
+class StreamRules(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_double) for n in ("block_us", "block_row_us", "fixed_64", "fixed_128", "pair_few", "pair_all", "merge_us", "merge_kb_us", "bytes_per_us")] + \
+               [("cus", ctypes.c_int32), ("least_blocks", ctypes.c_int32)]
+
+
+class TileChoice(ctypes.Structure):
+    _fields_ = [("us", ctypes.c_double), ("tile", ctypes.c_int32), ("cut", ctypes.c_int32)]
 
 
 def step_layout(n_tokens, pos0, state_slots, tokens, want_counts, wants, pad_rows: int, pad_state_slot: int,
@@ -72,6 +94,11 @@ def _declare(lib) -> None:
         "jllm_pool_set_free_list": (c_int, [vp, vp, c_int]),
         "jllm_pool_check": (c_int, [vp, ctypes.POINTER(c_int)]),
         "jllm_step_layout": (c_i64, [ctypes.POINTER(StepBatchArgs), vp, c_i64, ctypes.POINTER(StepSizes)]),
+        "jllm_tile_us": (ctypes.c_double, [vp] + [c_int] * 6),
+        "jllm_small_tiles": (None, [vp] + [c_int] * 4 + [ctypes.POINTER(TileChoice)]),
+        "jllm_large_tiles": (None, [vp] + [c_int] * 5 + [ctypes.POINTER(TileChoice)]),
+        "jllm_stream_us": (ctypes.c_double, [vp] + [c_int] * 7),
+        "jllm_stream_tiles": (None, [vp] + [c_int] * 4 + [i32p]),
     }
     for name, (res, args) in sig.items():
         fn = getattr(lib, name)

@@ -11,7 +11,6 @@ import bisect
 import contextlib
 import ctypes
 import functools
-import math
 import struct
 import threading
 from typing import Optional, Tuple
@@ -19,6 +18,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import build as _build
+from .. import host as _host
 
 F32, BF16 = 0, 1
 EPI_STORE, EPI_ADD, EPI_GATED = 0, 1, 2
@@ -669,7 +669,6 @@ TILE_COLS = 128
 SPLIT_LONG_STEPS = 16     # ... where each still has this many 64-wide K steps
 
 
-@functools.lru_cache(maxsize=8192)
 def _k_splits(M: int, N: int, K: int, gated: bool) -> int:
     """How many ways the tiled kernel cuts K so that a product with few output tiles still fills the GPU. Splits are
     doubled until every compute unit has a workgroup, and further, up to two per compute unit, only while the K range
@@ -704,7 +703,6 @@ PINGPONG_SUM_US = 2.3e-6       # per element of a partial result: written in 32-
 TILED_SUM_US = 1.9e-6
 
 
-@functools.lru_cache(maxsize=8192)
 def _pingpong_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int]:
     """(rows of the output tile, ways K is cut) with which the two-group kernel takes a product, or (0, 1) when the
     other tiled kernel is the better choice. The 256 x 256 tile moves the fewest bytes per multiply (a compute unit
@@ -775,6 +773,24 @@ WIDE_LAST = 384                       # tile code: 256 rows, and the last at mos
 WIDE_LAST_EXTRA = (0.025, 0.132)      # of a tile's time that a wide one takes longer: up to 64 rows, beyond
 
 
+@functools.lru_cache(maxsize=None)
+def _tile_rules(cus: int):
+    """What the native estimates and walks (csrc/host/tile_times.cpp) work with, and each tile's place in it."""
+    large = (192, 256, WIDE_LAST)
+    kinds = (_host.TileKind * (len(SMALL_TILES) + len(large)))()
+    for k, tile in zip(kinds, SMALL_TILES + large):
+        k.fixed, k.lone, k.full, k.round_us, *pair = TILE_US[256 if tile == WIDE_LAST else tile]
+        k.few, k.all = pair or (0.0, 0.0)
+        k.rows, k.columns = divmod(tile, 1000) if tile > 1000 else (192 if tile == 192 else 256, 256)
+        k.code, k.two, k.wide_last = tile, len(pair) > 0, tile == WIDE_LAST
+        k.plain_only = tile == 64064
+        k.odd_cuts = tile == 192  # `_tiled_plan` has weighed the others against 256 rows, with exceptions of its own
+    cuts = (ctypes.c_int32 * len(SMALL_CUTS))(*SMALL_CUTS)
+    rules = _host.TileRules(kinds, cuts, len(SMALL_TILES), len(large), len(SMALL_CUTS), cus, 128128, SMALL_CUT_MIN_K, PINGPONG_SPLIT_MIN_K, FINER_CUTS,
+                            TILE_BYTES_PER_US, *TILE_CUT_US, *NORM_PASS_US, WIDE_LAST_EXTRA)
+    return ctypes.addressof(rules), {k.code: i for i, k in enumerate(kinds)}, _host.library(), (rules, kinds, cuts)
+
+
 def _tile_us(tile: int, M: int, N: int, K: int, gated: bool, cut: int) -> float:
     """The product in tiles of one kind with K in ``cut`` parts, the reduction included: rounds of workgroups, one or two to a compute
     unit, against the weights' way from memory.
@@ -783,51 +799,12 @@ def _tile_us(tile: int, M: int, N: int, K: int, gated: bool, cut: int) -> float:
     products (0.6B to 14B shapes and five others) at 18 row counts from 70 to 3,000, 9,300 in all: 5 % off on average, and the
     cheapest by the estimate 2.0 % behind the best of a product's choices on average, 11 % at the 95th of a hundred, 38 % at worst
     (the best of what the tiles of 256 and 192 rows and gemm_stream.hip offer is 15 % behind on average)."""
-    cus = compute_units()
-    fixed, lone, full, round_us, *pair = TILE_US[256 if tile == WIDE_LAST else tile]
-    rows, columns = divmod(tile, 1000) if tile > 1000 else (256 if tile == WIDE_LAST else tile, 256)
-    across = -(-N // (columns // 2 if gated else columns))
-    groups = (M // 256 * across + -(-across // 2) if tile == WIDE_LAST else across * -(-M // rows)) * cut
-    steps = -(-K // (64 * cut))
-    rounds, last = divmod(groups, 2 * cus if pair else cus)
-    t = rounds * (steps * (pair[1] if pair else full) + round_us)
-    step = lone + (full - lone) * min(last, cus) / cus
-    if last > cus:
-        step = pair[0] + (pair[1] - pair[0]) * (last - cus) / cus
-    if last:
-        t += steps * step + round_us
-    if tile == WIDE_LAST:
-        t += WIDE_LAST_EXTRA[M % 256 > 64] * steps * (full if rounds else step)
-    t = fixed + math.hypot(t, N * K * (4 if gated else 2) / TILE_BYTES_PER_US)
-    return t + (TILE_CUT_US[0] + TILE_CUT_US[1] * M * N * cut if cut > 1 else 0.0)
+    rules, places, lib, _ = _tile_rules(compute_units())
+    return lib.jllm_tile_us(rules, places[tile], M, N, K, gated, cut)
 
 
 def _large_us(M: int, N: int, K: int, gated: bool, rows: int, cut: int) -> float:
     return _tile_us(rows, M, N, K, gated, cut)
-
-
-@functools.lru_cache(maxsize=8192)
-def _small_best(tiles64: int, N: int, K: int, gated: bool, normed: bool) -> Tuple[float, int, int]:
-    """(estimated time, tile, parts of K) of the cheapest choice of `jllm_gemm_mfma_bf16` for ``tiles64`` times 64 rows (and so for all
-    row counts that have these tiles); ``normed``: the norm of the new rows included, which the reduction makes where K is cut."""
-    M, cus = 64 * tiles64, compute_units()
-    best = (float("inf"), 128128, 1)
-    for tile in SMALL_TILES:
-        if gated and tile == 64064:
-            continue
-        rows, columns = divmod(tile, 1000)
-        groups = -(-N // (columns // 2 if gated else columns)) * -(-M // rows)
-        for cut in SMALL_CUTS:
-            if cut > 1 and (gated or K // cut < SMALL_CUT_MIN_K or groups * cut > 3 * cus or K // 64 <= -(-(K // 64) // cut) * (cut - 1)):
-                continue
-            t = _tile_us(tile, M, N, K, gated, cut) + (_norm_us(M, N) if normed and cut == 1 else 0.0)
-            if t < best[0]:
-                best = t, tile, cut
-    return best
-
-
-def _small_us(M: int, N: int, K: int, gated: bool) -> float:
-    return _small_best(-(-M // 64), N, K, gated, False)[0]
 
 
 NORM_PASS_US = (4.0, 0.6e-6)        # the norm behind an adding product with K whole (a cut's reduction makes it): launch, per element
@@ -838,6 +815,20 @@ def _norm_us(M: int, N: int) -> float:
 
 
 @functools.lru_cache(maxsize=8192)
+def _small_bests(tiles64: int, N: int, K: int, gated: bool):
+    """(estimated time, tile, parts of K) of the cheapest choice of `jllm_gemm_mfma_bf16` for ``tiles64`` times 64 rows (and so for all
+    row counts that have these tiles), twice: of the product alone, and with the norm of the new rows, which the reduction makes where
+    K is cut, or a launch behind it."""
+    rules, _, lib, _ = _tile_rules(compute_units())
+    out = (_host.TileChoice * 2)()
+    lib.jllm_small_tiles(rules, 64 * tiles64, N, K, gated, out)
+    return tuple((c.us, c.tile, c.cut) for c in out)
+
+
+def _small_us(M: int, N: int, K: int, gated: bool, normed: bool = False) -> float:
+    return _small_bests(-(-M // 64), N, K, gated)[normed][0]
+
+
 def _tiled_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int]:
     """(rows of the two-group kernel's tile or 0 for the small tile, ways K is cut): what `_pingpong_plan` and `_k_splits`
     choose between 256 rows and the small tile, or tiles of 192 rows where these are estimated to be faster. A tile of
@@ -886,7 +877,6 @@ FINER_CUTS = 8                      # the large tiles' parts of K, any count up 
 FINER_AT_MOST = 0.95                # of the plan's estimate
 
 
-@functools.lru_cache(maxsize=8192)
 def _tiles(M: int, N: int, K: int, gated: bool, normed: bool, rows: int, cut: int) -> Tuple[int, int]:
     """(rows of the two-group kernel's tile, `WIDE_LAST`, or 0 for the small tile, ways K is cut): the plan (``rows``, ``cut``) of
     `_tiled_plan`, or what is estimated to take at most `FINER_AT_MOST` of its time among tiles of 256, 192 and wide last rows
@@ -899,34 +889,24 @@ def _tiles(M: int, N: int, K: int, gated: bool, normed: bool, rows: int, cut: in
     now: 560 rows of the 8B shape 12.7 / 11.2 ms, 280 to 340 of the 14B 16.7 to 17.6 / 13.9 to 14.5, 2,600 of the 8B 40.7 / 37.5, of
     the 0.6B 3.5 % less. us, plan / now: 8B down at 1,100 rows 139.8 (192 rows, two parts) / 120.5 (256, three), at 280 64.1 (small tile, four) / 54.0 (192, eight), 14B qkv at 631 77.0 (256,
     two) / 67.1 (three), down at 900 195.6 (192, two) / 174.9 (256, three); wide last rows: csrc/gemm_pingpong.hip."""
-    if K % 64 or M < PINGPONG_MIN_ROWS or (rows, cut) != _own_tiled_plan(M, N, K, gated):
-        return rows, cut
-    return _finer_tiles(-(-M // 64) * 64, N, K, gated, normed, rows, cut)
+    return _finer_tiles(M, N, K, gated, normed, rows, cut)[:2] if (rows, cut) == _own_tiled_plan(M, N, K, gated) else (rows, cut)
 
 
-@functools.lru_cache(maxsize=8192)
-def _finer_tiles(M: int, N: int, K: int, gated: bool, normed: bool, rows: int, cut: int) -> Tuple[int, int]:
-    """The same for row counts up to M in whole 64s, which all have M's tiles (so that a prompt of a new length does not weigh
-    two dozen choices per product anew)."""
-
-    def us(tile, c):
-        if not tile:
-            return _small_best(-(-M // 64), N, K, gated, normed)[0]
-        return _tile_us(tile, M, N, K, gated, c) + (_norm_us(M, N) if normed and c == 1 else 0.0)
-
-    least, best = FINER_AT_MOST * us(rows, cut), (rows, cut)
-    for tile in (192, 256, WIDE_LAST):
-        if tile == WIDE_LAST and M % 256 not in (64, 128):
-            continue
-        for c in range(1, 1 + (1 if gated else FINER_CUTS)):
-            if c > 1 and K // c < PINGPONG_SPLIT_MIN_K:
-                break
-            if tile == 192 and c in (1, 2, 4):  # the plan has weighed these against 256 rows, with exceptions of its own
-                continue
-            t = us(tile, c)
-            if t < least:
-                least, best = t, (tile, c)
-    return best
+def _finer_tiles(M: int, N: int, K: int, gated: bool, normed: bool, rows: int, cut: int) -> Tuple[int, int, float]:
+    """The same for a plan that is `_tiled_plan`'s own, and the time of what it chose (of the small tiles' best where that is none)."""
+    if K % 64:
+        return rows, cut, float("inf")
+    if rows:
+        us = _tile_us(rows, M, N, K, gated, cut) + (_norm_us(M, N) if normed and cut == 1 else 0.0)
+    else:
+        us = _small_us(M, N, K, gated, normed)
+    if M >= PINGPONG_MIN_ROWS and K >= 128:
+        rules, _, lib, _ = _tile_rules(compute_units())
+        best = _host.TileChoice(FINER_AT_MOST * us, 0, 0)
+        lib.jllm_large_tiles(rules, M, N, K, gated, normed, best)
+        if best.tile:
+            return best.tile, best.cut, best.us
+    return rows, cut, us
 
 
 STREAM_MAX_ROWS = 64   # up to here the second weight-streaming kernel (activations through LDS)
@@ -1129,44 +1109,28 @@ WIDE_BYTES_PER_US = 5.3e6         # weights from memory
 WIDE_NORM_AT_MOST = 1.25
 
 
+@functools.lru_cache(maxsize=None)
+def _wide_rules(cus: int):
+    rules = _host.StreamRules(*WIDE_BLOCK_US, WIDE_FIXED_US[64], WIDE_FIXED_US[128], *WIDE_PAIR, *WIDE_MERGE_US, WIDE_BYTES_PER_US, cus, STREAM_MIN_BLOCKS)
+    return ctypes.addressof(rules), _host.library(), rules
+
+
 def _wide_us(M: int, N: int, K: int, gated: bool, rows: int, tile: int, parts: int) -> float:
-    cus = compute_units()
-    groups = -(-N // (rows // 2 if gated else rows)) * -(-M // tile) * parts
-    blocks = -(-(K // 128) // parts) * 2
-    step = blocks * (WIDE_BLOCK_US[0] + WIDE_BLOCK_US[1] * ((rows + tile) / 8 - 12))
-    if tile == 64:  # two on a compute unit
-        full, last = divmod(groups, 2 * cus)
-        few, all_ = WIDE_PAIR
-        t = full * step * all_
-        if last:
-            t += step if last <= cus else step * (few + (all_ - few) * (last - cus) / cus)
-    else:
-        t = -(-groups // cus) * step
-    t = max(t, N * K * 2 * (2 if gated else 1) / WIDE_BYTES_PER_US) + WIDE_FIXED_US[tile]
-    if parts > 1:
-        t += WIDE_MERGE_US[0] + WIDE_MERGE_US[1] * parts * rows * min(tile, M) * 4 / 1024
-    return t
+    """A product of M rows with that many weight rows, activation rows and parts of K per workgroup (csrc/host/tile_times.cpp)."""
+    rules, lib, _ = _wide_rules(compute_units())
+    return lib.jllm_stream_us(rules, M, N, K, gated, rows, tile, parts)
 
 
 @functools.lru_cache(maxsize=None)
 def _wide_best(tiles64: int, most: int, N: int, K: int, gated: bool) -> Tuple[float, Tuple[int, int, int]]:
     """The cheapest (weight rows, activation rows, parts of K) by the estimate, and its time, for ``tiles64`` tiles of 64 rows
     (``most``: rows of the fullest tile). It is the same for all row counts that have these tiles, so that a prompt of a
-    length that was not seen before does not weigh 30 choices per product anew (some 45 us of the host's time each)."""
-    cus = compute_units()
+    length that was not seen before does not weigh 30 choices per product anew."""
     M = tiles64 * 64 if most == 128 else most
-    best, plan = float("inf"), (64, 64, 1)
-    for rows in (32, 64, 96, 128):
-        for tile in (64, 128):
-            tiles = -(-N // (rows // 2 if gated else rows)) * -(-M // tile)
-            for parts in (1, 2, 3, 4):
-                per = -(-(K // 128) // parts)
-                if parts > 1 and (tiles * parts > 2 * cus or per < STREAM_MIN_BLOCKS or -(-(K // 128) // per) != parts):
-                    continue
-                t = _wide_us(M, N, K, gated, rows, tile, parts)
-                if t < best:
-                    best, plan = t, (rows, tile, parts)
-    return best, plan
+    rules, lib, _ = _wide_rules(compute_units())
+    plan = (ctypes.c_int32 * 3)()
+    lib.jllm_stream_tiles(rules, M, N, K, gated, plan)
+    return _wide_us(M, N, K, gated, *plan), tuple(plan)
 
 
 @functools.lru_cache(maxsize=8192)
@@ -1198,18 +1162,30 @@ _own_k_splits, _own_tiles = _k_splits, _tiles  # as they are, whoever puts other
 
 @functools.lru_cache(maxsize=8192)
 def _own_choice(M: int, N: int, K: int, gated: bool, normed: bool) -> Tuple[int, int, float]:
-    """(tile, ways K is cut, estimated time) of a product that the tiled kernels take: a large tile (256, 192 or `WIDE_LAST`:
-    `_tiles`), or one of `SMALL_TILES` where its estimate is below `SMALL_AT_MOST` of the large one's or no large one fits. The time
-    counts the norm behind the product where one is asked for."""
-    tile, cut = _own_tiles(M, N, K, gated, normed, *_own_tiled_plan(M, N, K, gated))
+    """(tile, ways K is cut, estimated time) of a product that the tiled kernels take. The time counts the norm behind the product
+    where one is asked for. The choice is that of M rounded up to whole 32s, which has the same tiles: a prompt of a new length looks
+    it up."""
+    rows32 = -(-M // 32)
+    tile, cut, us = _choice_of(rows32, N, K, gated, normed)
+    return tile, cut, us - (32 * rows32 - M) * N * _row_us(cut, normed)
+
+
+@functools.lru_cache(maxsize=8192)
+def _choice_of(rows32: int, N: int, K: int, gated: bool, normed: bool) -> Tuple[int, int, float]:
+    """A large tile (256, 192 or `WIDE_LAST`: `_tiles`), or one of `SMALL_TILES` where its estimate is below `SMALL_AT_MOST` of the large
+    one's or no large one fits."""
+    M = 32 * rows32
+    tile, cut, large = _finer_tiles(M, N, K, gated, normed, *_own_tiled_plan(M, N, K, gated))
     if K % 64:
-        return tile or 128128, cut, float("inf")
-    us, small, small_cut = _small_best(-(-M // 64), N, K, gated, normed)
-    if tile:
-        large = _tile_us(tile, M, N, K, gated, cut) + (_norm_us(M, N) if normed and cut == 1 else 0.0)
-        if us >= SMALL_AT_MOST * large:
-            return tile, cut, large
-    return small, small_cut, us
+        return tile or 128128, cut, large
+    us, small, small_cut = _small_bests(-(-M // 64), N, K, gated)[normed]
+    us -= -M % 64 * N * _row_us(small_cut, normed)
+    return (tile, cut, large) if tile and us >= SMALL_AT_MOST * large else (small, small_cut, us)
+
+
+def _row_us(cut: int, normed: bool) -> float:
+    """What an estimate grows by, per element of the output, within the same tiles: a reduction's or a norm's pass."""
+    return TILE_CUT_US[1] * cut if cut > 1 else NORM_PASS_US[1] if normed else 0.0
 
 
 def _tiled_choice(M: int, N: int, K: int, gated: bool, normed: bool) -> Tuple[int, int]:

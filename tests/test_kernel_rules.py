@@ -251,6 +251,87 @@ def test_a_new_row_count_does_not_weigh_every_choice_again(monkeypatch):
     assert 0 < once == len(weighed)
 
 
+MANY = [s for v in SHAPES.values() for s in v] + [  # the smaller models' products, and odd sizes
+    (4096, 1024, False), (1024, 2048, False), (3072, 1024, True), (1024, 3072, False), (6144, 2560, False), (2560, 9728, False), (3392, 2048, False),
+    (12320, 2048, False), (22592, 4096, False), (8192, 2048, True)] + [(n, k, g) for n in (8, 131, 1000, 4100) for k in (32, 64, 96, 128, 192, 320, 1056, 4160, 8256)
+                                                                      for g in (False, True)]
+
+
+def test_choices_of_the_tiled_products():
+    """What the dispatch asks for, at every row count of some and many of all shapes: a tile of a kernel that takes the sizes, K in no
+    more parts than leave each one stages and never for the gated product, the norm's time counted where one is asked for; the same
+    for all row counts of 32 with the same tiles, and the cheapest of the small kernel's choices by the estimate."""
+    taken = set()
+    for n, k, gated in MANY:
+        rows_of = range(65, 1100, 7) if (n, k) in ((4096, 4096), (3392, 2048)) else (65, 96, 97, 128, 129, 192, 257, 288, 384, 385, 487, 513, 700, 1025, 1318, 1800, 2100, 3000, 8192)
+        for rows in rows_of:
+            for normed in (False,) if gated else (False, True):
+                tile, cut, us = ops._own_choice(rows, n, k, gated, normed)
+                where = (rows, n, k, gated, normed, tile, cut)
+                taken.add((tile, cut))
+                stages = -(-k // 64)
+                assert cut == 1 or (not gated and stages > -(-stages // cut) * (cut - 1)), where
+                if tile in (192, 256, ops.WIDE_LAST):
+                    assert k % 32 == 0 and k >= 128 and k // cut >= 128, where
+                    assert tile != ops.WIDE_LAST or (rows > 256 and 1 <= rows % 256 <= 128), where
+                else:
+                    assert tile in ops.SMALL_TILES and not (gated and tile == 64064), where
+                assert ops._own_choice(-(-rows // 32) * 32, n, k, gated, normed)[:2] == (tile, cut), where
+                if k % 64:
+                    continue
+                norm = ops._norm_us(rows, n) if normed and cut == 1 else 0.0
+                assert abs(us - ops._tile_us(tile, rows, n, k, gated, cut) - norm) < 1e-6 * us, where
+    assert len(taken) > 25 and {t for t, _ in taken} == {192, 256, ops.WIDE_LAST, *ops.SMALL_TILES}, taken
+
+
+def test_the_native_walks_find_the_cheapest():
+    """The walks over the choices against every single one's time."""
+    cus = ops.compute_units()
+    for n, k, gated in MANY:
+        if k % 64:
+            continue
+        for rows in (128, 320, 512, 832, 1344, 2112):
+            for normed in (False, True):
+                norm = lambda c: ops._norm_us(rows, n) if normed and c == 1 else 0.0
+                all_ = []
+                for tile in ops.SMALL_TILES:
+                    r, c = divmod(tile, 1000)
+                    groups = -(-n // (c // 2 if gated else c)) * -(-rows // r)
+                    all_ += [(ops._tile_us(tile, rows, n, k, gated, cut) + norm(cut), tile, cut) for cut in ops.SMALL_CUTS if not (gated and tile == 64064)
+                             and (cut == 1 or (not gated and k // cut >= ops.SMALL_CUT_MIN_K and groups * cut <= 3 * cus and k // 64 > -(-(k // 64) // cut) * (cut - 1)))]
+                got = ops._small_bests(rows // 64, n, k, gated)[normed]
+                assert got[1:] == min(all_)[1:] and abs(got[0] - min(all_)[0]) < 1e-9 * got[0], (rows, n, k, gated, normed)
+                plan = ops._tiled_plan(rows, n, k, gated)
+                if rows < ops.PINGPONG_MIN_ROWS or k < 128:
+                    continue
+                us = ops._tile_us(plan[0], rows, n, k, gated, plan[1]) + norm(plan[1]) if plan[0] else got[0]
+                large = [(ops.FINER_AT_MOST * us, 0, 0)] + [
+                    (ops._tile_us(tile, rows, n, k, gated, cut) + norm(cut), tile, cut) for tile in (192, 256, ops.WIDE_LAST) for cut in range(1, 2 if gated else ops.FINER_CUTS + 1)
+                    if (cut == 1 or k // cut >= ops.PINGPONG_SPLIT_MIN_K) and not (tile == 192 and cut in (1, 2, 4)) and (tile != ops.WIDE_LAST or rows % 256 in (64, 128))]
+                want = min(large)
+                assert ops._finer_tiles(rows, n, k, gated, normed, *plan)[:2] == (want[1:] if want[1] else plan), (rows, n, k, gated, normed)
+
+
+def test_a_prompt_of_a_new_length_costs_the_host_little(monkeypatch):
+    """Of the tiled kernels' choices few are priced one by one in Python for a row count whose tiles were not seen, none for one whose
+    tiles were."""
+    priced = []
+    estimate = ops._tile_us
+    monkeypatch.setattr(ops, "_tile_us", lambda *args: priced.append(args) or estimate(*args))
+    for cached in (f for f in vars(ops).values() if hasattr(f, "cache_clear") and f.__name__ in ("_own_choice", "_choice_of", "_small_bests", "_wide_plan", "_wide_best")):
+        cached.cache_clear()
+    for n, k, gated in ((4096, 1024, False), (1024, 2048, False), (3072, 1024, True), (4096, 4096, False), (4096, 12288, False)):
+        for rows in (487, 833, 1500):
+            ask = lambda m: [ops._cut_takes_norm(m, n, k) if not gated else None, ops._wide_plan(m, n, k, gated, 0), ops._tiled_choice(m, n, k, gated, False)]
+            del priced[:]
+            ask(rows)
+            assert len(priced) <= 16, (n, k, gated, rows, len(priced))
+            del priced[:]
+            for m in range(-(-rows // 32) * 32 - 31, -(-rows // 32) * 32 + 1):
+                ask(m)
+            assert not priced, (n, k, gated, rows)
+
+
 def test_order_of_the_tiles_of_odd_numbers_of_columns():
     """Every tile is taken once, whatever the numbers; with an odd number of columns, and with two more than a multiple of four, the
     workgroups of a die (every eighth) share the weights of as few columns as their number allows."""
