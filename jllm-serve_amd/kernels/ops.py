@@ -874,7 +874,7 @@ _own_tiled_plan = _tiled_plan  # as it is, whoever puts another in its place
 
 
 FINER_CUTS = 8                      # the large tiles' parts of K, any count up to this
-FINER_AT_MOST = 0.95                # of the plan's estimate
+FINER_AT_MOST = 0.96                # of the plan's estimate
 
 
 def _tiles(M: int, N: int, K: int, gated: bool, normed: bool, rows: int, cut: int) -> Tuple[int, int]:
@@ -884,8 +884,9 @@ def _tiles(M: int, N: int, K: int, gated: bool, normed: bool, rows: int, cut: in
     rows follows, which the reduction of a cut product makes on its way. A plan that is not `_tiled_plan`'s own stands.
 
     Against the times, inside a graph, of every choice for 142 products (six shapes at 280 to 4,614 rows): 1.7 % behind the best
-    on average, where the plan is 4.7 % behind; of 25 choices that change none is slower than the plan's (with 0.97 for 0.95 4B
-    down at 700 rows went to 192 rows in six parts, and the pass took 2.7 % longer). Whole passes, plan /
+    on average, where the plan is 4.7 % behind. With 0.95 for 0.96 8B o at 1,200 rows stays with two parts for three (68.4 / 64.3 us, the
+    pass 17.65 / 17.46 ms) and 2,500 rows of 2,048 x 4,096 likewise (68.7 / 65.4); with 1.0 and no exception 4B down at 900 goes to 192
+    rows in five parts (the pass 10.02 / 10.14). Whole passes, plan /
     now: 560 rows of the 8B shape 12.7 / 11.2 ms, 280 to 340 of the 14B 16.7 to 17.6 / 13.9 to 14.5, 2,600 of the 8B 40.7 / 37.5, of
     the 0.6B 3.5 % less. us, plan / now: 8B down at 1,100 rows 139.8 (192 rows, two parts) / 120.5 (256, three), at 280 64.1 (small tile, four) / 54.0 (192, eight), 14B qkv at 631 77.0 (256,
     two) / 67.1 (three), down at 900 195.6 (192, two) / 174.9 (256, three); wide last rows: csrc/gemm_pingpong.hip."""

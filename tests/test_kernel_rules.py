@@ -290,7 +290,7 @@ def test_the_native_walks_find_the_cheapest():
     for n, k, gated in MANY:
         if k % 64:
             continue
-        for rows in (128, 320, 512, 832, 1344, 2112):
+        for rows in (128, 320, 512, 832, 1216, 1344, 2112, 2560):
             for normed in (False, True):
                 norm = lambda c: ops._norm_us(rows, n) if normed and c == 1 else 0.0
                 all_ = []
@@ -310,6 +310,7 @@ def test_the_native_walks_find_the_cheapest():
                     if (cut == 1 or k // cut >= ops.PINGPONG_SPLIT_MIN_K) and not (tile == 192 and cut in (1, 2, 4)) and (tile != ops.WIDE_LAST or rows % 256 in (64, 128))]
                 want = min(large)
                 assert ops._finer_tiles(rows, n, k, gated, normed, *plan)[:2] == (want[1:] if want[1] else plan), (rows, n, k, gated, normed)
+                assert ops._own_choice(rows, n, k, gated, normed)[2] < 1.05 * min(t for t, tile, _ in large if tile), (rows, n, k, gated, normed)
 
 
 def test_a_prompt_of_a_new_length_costs_the_host_little(monkeypatch):
