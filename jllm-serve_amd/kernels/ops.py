@@ -1600,29 +1600,38 @@ def _fast_latent_attention(qa, out, cache, block_table, row_req, positions, head
                 split, n_z, _ptr(part), _stream())
 
 
-# keys a workgroup takes at least when a row's keys are cut over several: one block of the kernel, since a workgroup is a chain of blocks. us
-# at ranges of 64 / 128 / 256: 16 heads of 512 + 64 entries, a window of 1,024, 1 row 13.4 / 15.6 / 19.3, 8 rows 14.7 / 16.2 / 19.4, 16 rows
-# 15.8 / 16.2 / 19.6; 32 heads 12.5 / 17.2 / 25.3, 14.7 / 18.2 / 25.6, 18.9 / 18.8 / 26.1. One row that may reach 8,192 keys, at
-# 2,000: 18.5 in 44 ranges of 192, 19.3 in 33 of 256 (32 heads 22.1 / 25.2)
-LATENT_SPLIT_MIN = 64
+# Keys a workgroup of single rows takes at least, in blocks of 64 (it is a chain of them): one block only where the compute units then
+# have one workgroup each (of 512 + 64 entries they hold no more), since otherwise some wait for others' ends. us with the merge at ranges
+# of 64 / 128 / 192 / 256 keys, 16 heads of 512 + 64 entries (32 heads), a window of 1,024: 1 row 15.0 / 16.6 / 18.0 / 19.8 (14.2 / 18.1 /
+# 21.5 / 25.8), 8 rows 15.3 / 16.8 / 18.2 / 19.8 (15.1 / 18.7 / 22.2 / 25.9), 16 rows 25.4 / 17.2 / 18.4 / 20.1 (24.5 / 20.1 / 23.0 / 26.6), 24
+# rows 29.0 / 19.8 / 20.2 / 21.3 (30.8 / 24.3 / 25.8 / 28.8), 64 rows of 400 keys 29.4 / 20.4 / 21.2 / 22.6; 24 rows of 1,000 keys without
+# a window 28.3 / 18.7 / 19.9 / 21.1.
+LATENT_BLOCK = 64
 LATENT_SPAN_MIN = 256  # shorter spans are not cut
+LATENT_MOST_RANGES = 64  # what the merge takes
 
 
 def _latent_split(rows: int, heads: int, window: int, max_ctx: int):
     """(keys per range, ranges per row) for a step of single rows, or (0, 1): a row's keys are cut over several
-    workgroups where the step would otherwise leave most compute units idle (few rows, long spans). From the number of
-    rows, the heads, the window and the longest context only (what a captured step's bucket fixes)."""
-    span = min(window, max_ctx) if window > 0 else max_ctx
-    groups = rows * -(-heads // 64)
-    want = -(-2 * compute_units() // max(groups, 1))
+    workgroups where the step would otherwise leave most compute units idle (few rows, long spans), two a compute unit if all rows were
+    as long as they may be. From the number of rows, the heads, the window and the longest context only (what a captured
+    step's bucket fixes)."""
+    windowed = 0 < window < max_ctx  # the span then begins anywhere in a range
+    span = window if windowed else max_ctx
+    groups, cus = rows * -(-heads // 64), compute_units()
+    want = -(-2 * cus // max(groups, 1))
     if span < LATENT_SPAN_MIN or want < 2:
         return 0, 1
-    split = max(LATENT_SPLIT_MIN, -(-(-(-span // want)) // 64) * 64)
-    n_z = -(-span // split) + 1  # a span of that many keys touches at most this many absolute ranges
-    while n_z > 64:  # the merge takes up to 64 ranges
-        split += 64
-        n_z = -(-span // split) + 1
-    return (split, n_z) if n_z > 2 else (0, 1)
+    blocks = -(-span // LATENT_BLOCK)
+    per = max(1 if groups * (blocks + windowed) <= cus else 2, -(-blocks // want))
+    least = -(-blocks // (LATENT_MOST_RANGES - 1))
+    if per < least:
+        # up to twice as long where the compute units then have one workgroup each: 8 rows of 7,000 keys that may reach 8,192, 43 ranges of
+        # 192 40.1 us, 32 of 256 27.5 (1 and 8 rows of 2,000 18.8 / 19.8, 18.9 / 20.2)
+        alone = -(-blocks // max(1, cus // groups - windowed))
+        per = alone if least < alone < 2 * least else least
+    n_z = -(-blocks // per) + 1  # a span of that many keys touches at most this many absolute ranges
+    return (per * LATENT_BLOCK, n_z) if n_z > 2 else (0, 1)
 
 
 # ------------------------------------------------------------------------------------------------ table-routed experts

@@ -333,6 +333,27 @@ def test_a_prompt_of_a_new_length_costs_the_host_little(monkeypatch):
             assert not priced, (n, k, gated, rows)
 
 
+def test_ranges_of_the_latent_attention_of_single_rows():
+    """Whole blocks of 64 keys, no more ranges than the merge takes and enough for the span wherever it lies, about two workgroups a compute
+    unit at most; ranges of one block only where rows as long as they may be have one compute unit each."""
+    cus = ops.compute_units()
+    for rows in (1, 2, 3, 5, 8, 11, 15, 16, 17, 24, 31, 32, 48, 64, 100, 128, 200, 255, 256, 257, 600):
+        for heads in (1, 5, 16, 32, 64, 65, 128, 200):
+            for window in (0, 100, 256, 300, 1000, 1024, 4096, 50000):
+                for longest in (16, 255, 256, 257, 512, 768, 1024, 2048, 8192, 16000, 131072, 1 << 20):
+                    split, n_z = ops._latent_split(rows, heads, window, longest)
+                    where = (rows, heads, window, longest, split, n_z)
+                    windowed = 0 < window < longest
+                    span = window if windowed else longest
+                    groups = rows * -(-heads // 64)
+                    if split == 0:
+                        assert n_z == 1 and (span < ops.LATENT_SPAN_MIN or span <= 256 or groups >= cus), where
+                        continue
+                    assert split % 64 == 0 and 2 < n_z <= 64 and (n_z - 1) * split >= span, where
+                    assert split > 64 or groups * (n_z - 1 + windowed) <= cus, where
+                    assert groups * (n_z - 1) < 2 * cus + groups, where
+
+
 def test_order_of_the_tiles_of_odd_numbers_of_columns():
     """Every tile is taken once, whatever the numbers; with an odd number of columns, and with two more than a multiple of four, the
     workgroups of a die (every eighth) share the weights of as few columns as their number allows."""
