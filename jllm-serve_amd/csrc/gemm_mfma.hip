@@ -72,9 +72,11 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
   constexpr int WAVES = WGM * WGN, TBM = WGM * RM * 16, TBN = WGN * CN * 16, STAGE = (TBM + TBN) * T_ROW_BYTES;
   constexpr int LA = TBM / 8 / WAVES, L = LA + TBN / 8 / WAVES;  // load instructions (8 rows each) per wave and stage
   constexpr int NM = 2 * RM * CN, NR = 2 * (RM + CN);            // multiplies and LDS reads of a stage
-  constexpr int EVERY = NM / L;
+  // Loads are asked for evenly between the multiplies; with a ring of two stages, where they have to land within this one, at once (4,096
+  // rows through 32 experts 199 -> 191 us, 64 experts 800 -> 776)
+  constexpr int EVERY = NS == 2 ? 1 : NM / L;
   static_assert(LA * 8 * WAVES == TBM && (L - LA) * 8 * WAVES == TBN && EVERY >= 1, "every wave loads as many rows of either operand");
-  static_assert(NS >= 3 && NS <= 6, "one stage being read, one that has landed or is about to, one on its way");
+  static_assert(NS >= 2 && NS <= 6, "one stage being read, the others on their way");
   extern __shared__ __align__(1024) unsigned char smem[];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -497,7 +499,13 @@ extern "C" int jllm_gemm_mfma_bf16(const void* A, int lda, const void* W, const 
   return 0;
 }
 
-// The grouped form in tiles of 128 x 128: `tiles` holds (group, first row, rows <= 128) per entry (rows = 0: unused), the
+// The grouped form in tiles of 128 x 128, four waves and a ring of two stages, so that two workgroups share a compute unit: at few rows an
+// expert the weights' way from memory is what binds, at many the tiles' starts and ends, and either needs another workgroup beside. us, what
+// stood here before the rings / a ring of five stages, one workgroup a compute unit / this (rows x 4 through 32 experts of 1,024 x 2,048,
+// x 6 through 64 of 1,536 x 4,096): gate/up of 512 rows 47.8 / 56.7 / 49.6, of 1,024 89.5 / 88.4 / 84.9, of 4,096 222 / 212 / 191 and 877 /
+// 857 / 776; down 31.2 / 35.9 / 32.3, 47.8 / 56.3 / 43.5, 128 / 143 / 121 and 514 / 555 / 466. Tiles of 128 x 64 in rings of three: gate/up 59.4,
+// 84.6, 224 and 986.
+// `tiles` holds (group, first row, rows <= 128) per entry (rows = 0: unused), the
 // weights are [groups][N][K] (and W2 likewise for the gated epilogue), row i of the input is A[row_map[i] / row_div]
 // when `row_map` is given, and output row i is row i of `out`. K whole, epilogues store and gated.
 // returns 0 when it ran, 1 when the shape is not one it takes, -1 on errors
@@ -510,8 +518,8 @@ extern "C" int jllm_gemm_mfma_grouped_bf16(const void* A, int lda, const void* W
   if (((uintptr_t)A & 15) || ((uintptr_t)W & 15) || (W2 && ((uintptr_t)W2 & 15))) return 1;
   JLLM_TAKE_GATE("gemm_mfma_grouped", epilogue, gate_limit, gs);
   if ((epilogue != 0 && epilogue != 2) || (epilogue == 2) != (W2 != nullptr)) JLLM_FAIL("gemm_mfma_grouped: epilogue %d", epilogue);
-  using Plain = Tiled<false, FORM_GROUPED, 2, 4, 4, 2, 5>;
-  using Gated = Tiled<true, FORM_GROUPED, 2, 4, 4, 2, 5>;
+  using Plain = Tiled<false, FORM_GROUPED, 4, 4, 2, 2, 2>;
+  using Gated = Tiled<true, FORM_GROUPED, 4, 4, 2, 2, 2>;
   if (tile_rows != Plain::ROWS) JLLM_FAIL("gemm_mfma_grouped: tiles of %d rows, this kernel takes %d", tile_rows, Plain::ROWS);
   if (ldo < N || row_div < 1) JLLM_FAIL("gemm_mfma_grouped: ldo %d < N %d", ldo, N);
   const int cols = W2 ? Gated::COLS : Plain::COLS;
@@ -519,10 +527,10 @@ extern "C" int jllm_gemm_mfma_grouped_bf16(const void* A, int lda, const void* W
   if (!Plain::allow() || !Gated::allow()) JLLM_FAIL("gemm_mfma_grouped: cannot reserve %d bytes of LDS", Plain::LDS);
   const GroupArgs ga{tiles, row_map, row_div};
   if (W2)
-    gemm_mfma_kernel<true, FORM_GROUPED, 2, 4, 4, 2, 5><<<grid, Gated::THREADS, Gated::LDS, stream>>>(
+    gemm_mfma_kernel<true, FORM_GROUPED, 4, 4, 2, 2, 2><<<grid, Gated::THREADS, Gated::LDS, stream>>>(
         (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)W2, nullptr, 0, out, out_dtype, ldo, M, N, K, epilogue, gs, nullptr, ga, HeadsArgs{}, 0);
   else
-    gemm_mfma_kernel<false, FORM_GROUPED, 2, 4, 4, 2, 5><<<grid, Plain::THREADS, Plain::LDS, stream>>>(
+    gemm_mfma_kernel<false, FORM_GROUPED, 4, 4, 2, 2, 2><<<grid, Plain::THREADS, Plain::LDS, stream>>>(
         (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, nullptr, 0, out, out_dtype, ldo, M, N, K, epilogue, gs, nullptr, ga, HeadsArgs{}, 0);
   JLLM_CHECK_LAUNCH("gemm_mfma_grouped");
   return 0;

@@ -254,6 +254,37 @@ def test_experts_rows_have_the_same_bits_in_few_and_in_many(N, K):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
+@pytest.mark.parametrize("K", [64, 128, 192, 320, 704])
+@pytest.mark.parametrize("N", [64, 132, 260])
+def test_experts_tiles_at_their_edges(N, K):
+    """Experts with no row, one, one short of a tile, a whole tile, one beyond it and two tiles and one, K of one stage, of the ring's two
+    and of even and odd numbers beyond: gathered rows and rows by place, plain and gated, against float64."""
+    from jllm_serve_amd.kernels import ops
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(N + K)
+    counts = [0, 1, 127, 128, 129, 257]
+    E, T = len(counts), sum(counts)
+    w, w2 = ((torch.randn(E, N, K, device="cuda", generator=gen) * K ** -0.5).bfloat16() for _ in range(2))
+    experts = torch.repeat_interleave(torch.arange(E, device="cuda"), torch.tensor(counts, device="cuda"))[torch.randperm(T, device="cuda", generator=gen)]
+    routing = ops.moe_route(None, experts.to(torch.int32).view(T, 1).contiguous(), E, many_ok=True)
+    assert routing.many
+    x = torch.randn(T, K, device="cuda", generator=gen).bfloat16()
+    y, u = (torch.einsum("ak,ank->an", x.double(), t.double()[experts]) for t in (w, w2))
+    room = K * 2.0 ** -24 * torch.einsum("ak,ank->an", x.double().abs(), w.double()[experts].abs())
+    place = routing.place_of.long()
+    by_place = torch.empty_like(x)
+    by_place[place] = x
+    for a, in_map in ((x, 1), (by_place, 0)):
+        out = torch.full((T, N), float("nan"), device="cuda")
+        ops.moe_gemm(a, w, routing, out=out, in_map=in_map, out_map=0)
+        assert bool(((out[place].double() - y).abs() <= room + 1e-30).all())
+        h = torch.full((T, N), float("nan"), device="cuda", dtype=torch.bfloat16)
+        ops.moe_gemm(a, w, routing, w2=w2, out=h, in_map=in_map, out_map=0)
+        want = y * torch.sigmoid(y) * u
+        scale = (y.abs() + 1.0) * (u.abs() + 1.0)
+        assert bool(((h[place].double() - want).abs() <= 2.0 ** -8 * want.abs() + 4.0 * room.max() * scale + 2.0 ** -20 * scale).all())
+
+
 @pytest.mark.parametrize("dtype, fast", [("float32", False), ("bfloat16", True), ("bfloat16", False)])
 @pytest.mark.parametrize("H, R, Dr, page", [(4, 32, 16, 8), (5, 48, 8, 16), (16, 64, 32, 32), (40, 16, 16, 4), (3, 24, 6, 8)])
 def test_attention_kernels_on_crafted_keys(dtype, fast, H, R, Dr, page):
