@@ -235,10 +235,11 @@ struct GdrArgs {
   const int* row_req;
   const int* state_slots;
   int n_rows, heads, kv_heads, dk, dv;
-  int req0;  // the launch's first request
+  int req0;             // the launch's first request
+  bool requests_first;  // in the order of dispatch: (request, head, columns), or (head, columns, request)
 };
 
-// thread = wave * 64 + c * 16 + part: column blockIdx.x * 16 + wave * 4 + c, key rows part * E .. + E
+// thread = wave * 64 + c * 16 + part: column 16 * the workgroup's columns + wave * 4 + c, key rows part * E .. + E
 // CHANNEL: the decay is a vector over the key channels (S's rows) instead of one number per head:
 //   S <- diag(g) S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q = (diag(g) S_old)^T q + (k . q) u
 // FEW: the form for steps of few rows per request (decoding). It leaves out the interleaved walk over a full chunk, whose
@@ -255,8 +256,8 @@ __global__ __launch_bounds__(256) void gated_delta_kernel(GdrArgs A) {
   __shared__ __align__(16) float sm[C * ROWF];
   const int tid = threadIdx.x;
   const int part = tid & 15, cw = tid >> 4;  // cw: the column within the workgroup
-  const int req = A.req0 + blockIdx.z, h = blockIdx.y;
-  const int col0 = blockIdx.x * GDR_COLS;
+  const int req = A.requests_first ? blockIdx.x : A.req0 + blockIdx.z, h = A.requests_first ? blockIdx.y : blockIdx.x;
+  const int col0 = (A.requests_first ? blockIdx.z : blockIdx.y) * GDR_COLS;
   const int col = col0 + cw;
   const bool col_on = col < A.dv;
   int lo, n;
@@ -440,17 +441,21 @@ extern "C" int jllm_gated_delta(const void* qkv, int ldc, const void* proj, int 
                                                                             kv_heads, dk, decay_rows, ldd);
     })
   })
-  GdrArgs A{qkv, ldc, prep, ldq, state, out, ldo, row_req, state_slots, n_rows, heads, kv_heads, dk, dv, 0};
-  // The requests come last in the order of dispatch. Neighbouring workgroups go to different dies: with the requests first, four
-  // requests of 16 heads x 128 columns had all workgroups of the longest one on two of the eight dies, two to a compute unit to
-  // the end; now the two are of different requests, and the longer one's has the unit alone for its rest (150 .. 1,390 rows: 388 -> 328
-  // us). Single rows of four requests take 6.6 us so, 7.0 with the requests first.
+  // Neighbouring workgroups go to different dies. With the requests first, four requests of 16 heads x 128 columns had all workgroups of
+  // the longest one on two of the eight dies, two to a compute unit to the end; with the heads first the two are of different requests,
+  // the longer one's has the unit alone for its rest, and a die reads the q and k of few heads. Where all workgroups of a request fit the
+  // compute units of a die that costs nothing, and a die that reads few requests is ahead. us, requests first / columns first / heads
+  // first: 150 .. 1,390 rows, 16 heads of 128 x 128, 362 / 302 / 305, 32 heads 653 / 367 / 360, three prompts of 300 to 900 beside five
+  // single rows 427 / 196 / 198 and 750 / 260 / 230, 16 heads of 64 x 64 with channel decays at 500 rows 89 / 93 / 89, 24 prompts of 60 57.6 /
+  // 60.6 / 58.9; 6 heads of 96 x 40 (18 workgroups a request), 8 prompts of 256 63.0 / 69.0 / 68.9, 16 of 100 38.0 / 42.8 / 42.7.
   const int col_groups = (dv + GDR_COLS - 1) / GDR_COLS;
+  const bool requests_first = (long)heads * col_groups <= 32;
+  GdrArgs A{qkv, ldc, prep, ldq, state, out, ldo, row_req, state_slots, n_rows, heads, kv_heads, dk, dv, 0, requests_first};
   const int per_lane = (dk + GDR_PARTS - 1) / GDR_PARTS;
   const bool few = n_rows <= 2 * n_requests;
 #define GDR_LAUNCH(E)                                                           \
-  for (A.req0 = 0; A.req0 < n_requests; A.req0 += 65535) {                      \
-    const dim3 grid(col_groups, heads, min(n_requests - A.req0, 65535));        \
+  for (A.req0 = 0; A.req0 < n_requests; A.req0 += requests_first ? n_requests : 65535) {                                                    \
+    const dim3 grid = requests_first ? dim3(n_requests, heads, col_groups) : dim3(heads, col_groups, min(n_requests - A.req0, 65535)); \
     if (channel && few)                                                         \
       gated_delta_kernel<T, E, true, true><<<grid, 256, 0, stream>>>(A);        \
     else if (channel)                                                           \

@@ -407,6 +407,33 @@ def test_delta_rule_recalls_a_far_memory(dtype, H, G, dk, dv):
         assert torch.equal(results[0][i], results[1][i]), "the recurrence depends on how the tokens were cut"
 
 
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("H, G, dk, dv", [(6, 3, 40, 24), (8, 4, 32, 64), (8, 8, 32, 80), (33, 11, 16, 16)])
+def test_delta_rule_of_many_requests_is_that_of_each(H, G, dk, dv, channel):
+    """Workgroups are dispatched by requests where those of one are at most 32 (12, 32), by heads where they are more (40, 33): requests of
+    one row to some dozens beside each other have the bits of each alone, outputs and states, and no other state is touched."""
+    from jllm_serve_amd.kernels import ops
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(H + dv)
+    rnd = lambda *shape: torch.randn(*shape, device=DEV, generator=gen)
+    lens = [1, 37, 1, 70, 2, 5, 1, 1, 16, 33, 1]
+    T, B = sum(lens), len(lens)
+    qkv, proj, decay = rnd(T, 2 * G * dk + H * dv).bfloat16(), rnd(T, 2 * H).bfloat16(), rnd(T, H * dk) if channel else None
+    a_log, bias = rnd(H), rnd(H * dk if channel else H)
+    before = rnd(2 * B + 1, H, dv, dk)
+    state, alone = before.clone(), before.clone()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    slots = [2 * i + 1 for i in range(B)]
+    out = ops.gated_delta(qkv, proj, 0, H, a_log, bias, state, i32([i for i, n in enumerate(lens) for _ in range(n)]), i32(slots), B, H, G, dk, dv, decay)
+    at = 0
+    for i, n in enumerate(lens):
+        part = slice(at, at + n)
+        one = ops.gated_delta(qkv[part], proj[part], 0, H, a_log, bias, alone, i32([0] * n), i32(slots[i:i + 1]), 1, H, G, dk, dv, decay[part] if channel else None)
+        assert torch.equal(one, out[part]), (i, n)
+        at += n
+    assert bool(torch.isfinite(out).all()) and torch.equal(state, alone) and torch.equal(state[::2], before[::2])
+
+
 @pytest.mark.parametrize("taps", [1, 2, 4, 7])
 def test_short_convolution_across_steps_and_slots(taps):
     """Two requests of unequal lengths in steps of unequal portions (down to one row, shorter than the taps), their
