@@ -31,7 +31,7 @@
 #define T_ROW_BYTES (TBK * 2)  // a tile row in LDS: 128 bytes = 8 pieces of 16
 #define T_FENCE() __builtin_amdgcn_sched_barrier(0)
 
-enum { FORM_PLAIN = 0, FORM_GROUPED = 1, FORM_HEADS = 2, FORM_BY_COLUMNS = 3 };  // the last: plain, in another order of the tiles
+enum { FORM_PLAIN = 0, FORM_GROUPED = 1, FORM_HEADS = 2, FORM_BY_COLUMNS = 3, FORM_FAR = 4 };  // the last two: plain, in another order of the tiles; of rows of any length
 
 // What the per-head form takes beside the operands: head h = blockIdx.z multiplies the rows at A + h * a_stride with
 // its own weights (W [heads][N][K]) and writes bf16 at out + h * o_stride, times sigmoid(gate[row][h * N + column]) where a
@@ -105,13 +105,13 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
   const int nk = max(0, min(nk_all, kt0 + nk_per) - kt0);
 
   // ---- global side of the loads: the tile's start at its first stage (the same in all lanes, advanced by scalar arithmetic) and a
-  // 32-bit byte offset per lane that never changes (row of the tile and piece; rows of less than 8 MB: checked on the host).
-  // Rows gathered by a list lie anywhere: an address per lane.
+  // 32-bit byte offset per lane that never changes (row of the tile and piece: checked on the host). Rows gathered by a list, and those
+  // too long for that, lie anywhere: an address per lane.
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
   const unsigned char* abase = (const unsigned char*)(A + (size_t)m0 * lda) + (size_t)kt0 * T_ROW_BYTES;
   const unsigned char* wbase[2] = {(const unsigned char*)(W + (size_t)n0 * K) + (size_t)kt0 * T_ROW_BYTES,
                                    (const unsigned char*)((GATED ? W2 : W) + (size_t)n0 * K) + (size_t)kt0 * T_ROW_BYTES};
-  const unsigned char *base[L], *gathered[LA];
+  const unsigned char *base[L], *at[L];
   uint32_t off[L];
 #pragma unroll
   for (int c = 0; c < L; ++c) {
@@ -123,20 +123,22 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
       off[c] = (uint32_t)m * (uint32_t)lda * 2u + piece;
       if (FORM == FORM_GROUPED) {
         const int from = ga.row_map ? ga.row_map[m0 + m] / ga.row_div : m0 + m;
-        gathered[c] = (const unsigned char*)(A + (size_t)from * lda) + piece;
+        at[c] = (const unsigned char*)(A + (size_t)from * lda) + piece;
       }
+      if (FORM == FORM_FAR) at[c] = base[c] + (size_t)m * lda * 2 + piece;
     } else {  // gated: of a wave's CN blocks of 16 the first half is gate rows, the second the up rows of the same outputs
       const int block = chunk % (2 * CN) / 2;  // the same in all lanes
       const int n = GATED ? chunk / (2 * CN) * CN * 8 + block % (CN / 2) * 16 + (r & 15) : r;
       base[c] = wbase[GATED && block >= CN / 2];
       off[c] = (uint32_t)min(n, N - 1 - n0) * (uint32_t)K * 2u + piece;
+      if (FORM == FORM_FAR) at[c] = base[c] + (size_t)min(n, N - 1 - n0) * K * 2 + piece;
     }
   }
   auto load = [&](int t, uint32_t slot, int c) {  // the wave's load c of stage t into the slot at byte `slot`
     const size_t kbytes = (size_t)t * T_ROW_BYTES;
     const uint32_t to = lds0 + slot + (c < LA ? (wave * LA + c) * 1024 : TBM * T_ROW_BYTES + (wave * (L - LA) + c - LA) * 1024);
-    if (FORM == FORM_GROUPED && c < LA)
-      load_to_lds_16(gathered[c < LA ? c : 0] + kbytes, to);
+    if (FORM == FORM_FAR || (FORM == FORM_GROUPED && c < LA))
+      load_to_lds_16(at[c] + kbytes, to);
     else
       load_to_lds_16(base[c] + kbytes, off[c], to);
   };
@@ -435,32 +437,36 @@ static int launch_tiled_as(dim3 grid, uint32_t by_rows, const void* A, int lda, 
   return 0;
 }
 
-template <bool GATED, int RM, int CN, int WGM, int WGN, int NS>
+template <bool GATED, int RM, int CN, int WGM, int WGN, int NS, bool FAR = false>
 static int launch_tiled(const void* A, int lda, const void* W, const void* W2, const void* bias, int bias_dtype,
                         void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue, GateSpec gs, int splits,
                         float* partial, hipStream_t stream) {
   using T = Tiled<GATED, FORM_PLAIN, RM, CN, WGM, WGN, NS>;
   const dim3 grid((N + T::COLS - 1) / T::COLS, (M + T::ROWS - 1) / T::ROWS, splits);
   if (grid.y > 65535) return 1;
+  if constexpr (FAR)
+    return launch_tiled_as<GATED, FORM_FAR, RM, CN, WGM, WGN, NS>(grid, 0, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, stream);
   if (by_columns(grid.y, grid.x))
     return launch_tiled_as<GATED, FORM_BY_COLUMNS, RM, CN, WGM, WGN, NS>(grid, by_rows_of(grid.y), A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, stream);
   return launch_tiled_as<GATED, FORM_PLAIN, RM, CN, WGM, WGN, NS>(grid, 0, A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, partial, stream);
 }
 
-static bool tiled_rows_fit(int lda, int K) { return lda < (1 << 22) && K < (1 << 22); }  // 256 rows of 8 MB are a 32-bit offset
+// a tile's rows of either operand, of which there are at most so many, lie within 32-bit byte offsets
+static bool tiled_rows_fit(int a_rows, int lda, int w_rows, int K) { return (uint64_t)a_rows * lda * 2 < (1ull << 32) && (uint64_t)w_rows * K * 2 < (1ull << 32); }
 
 // `tile`: rows * 1000 + columns of the output tile (of both products' columns with the gated epilogue): 64064 (not gated), 64128, 128128,
 // 128256, 256128.
 // `splits` > 1 cuts K over gridDim.z (not with the gated epilogue; any count that leaves no part without); `partial` then holds
 // splits * M * N floats.
 // `norm_rows` [M][norm_ld] bf16 (with cuts of K and the accumulate epilogue): the RMSNorm of the new rows, made by the reduction.
+// Rows of 16 MB and more go through tiles of 128 x 128 with an address per lane, whatever the tile.
 // returns 0 when it ran, 1 when the shape is not one it takes, -1 on errors
 extern "C" int jllm_gemm_mfma_bf16(const void* A, int lda, const void* W, const void* W2, const void* bias,
                                    int bias_dtype, void* out, int out_dtype, int ldo, int M, int N, int K, int epilogue,
                                    float gate_limit, int tile, int splits, float* partial, const void* norm_gain, int norm_gain_dtype, float norm_eps,
                                    void* norm_rows, int norm_ld, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (K <= 0 || (K % TBK) || (lda & 7) || !tiled_rows_fit(lda, K)) return 1;
+  if (K <= 0 || (K % TBK) || (lda & 7)) return 1;
   if (((uintptr_t)A & 15) || ((uintptr_t)W & 15) || (W2 && ((uintptr_t)W2 & 15))) return 1;
   JLLM_TAKE_GATE("gemm_mfma", epilogue, gate_limit, gs);
   if (epilogue < 0 || epilogue > 2 || (epilogue == 2) != (W2 != nullptr)) JLLM_FAIL("gemm_mfma: epilogue %d", epilogue);
@@ -476,7 +482,8 @@ extern "C" int jllm_gemm_mfma_bf16(const void* A, int lda, const void* W, const 
     rc = W2 ? launch_tiled<true, __VA_ARGS__>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, 1, partial, stream)       \
             : launch_tiled<false, __VA_ARGS__>(A, lda, W, W2, bias, bias_dtype, out, out_dtype, ldo, M, N, K, epilogue, gs, splits, partial, stream); \
     break;
-  switch (tile) {
+  switch (tiled_rows_fit(256, lda, 256, K) ? tile : -1) {
+    TILED_CASE(-1, 2, 4, 4, 2, 5, true)
     TILED_CASE(64128, 2, 4, 2, 2, 3)
     TILED_CASE(128128, 2, 4, 4, 2, 5)
     TILED_CASE(128256, 4, 4, 2, 4, 3)
@@ -514,7 +521,7 @@ extern "C" int jllm_gemm_mfma_grouped_bf16(const void* A, int lda, const void* W
                                            int max_tiles, int tile_rows, const int* row_map, int row_div,
                                            hipStream_t stream) {
   if (max_tiles <= 0 || M <= 0) return 0;
-  if ((K & 63) || K <= 0 || N <= 0 || (lda & 7) || max_tiles > 65535 || !tiled_rows_fit(lda, K)) return 1;
+  if ((K & 63) || K <= 0 || N <= 0 || (lda & 7) || max_tiles > 65535 || !tiled_rows_fit(0, lda, 128, K)) return 1;
   if (((uintptr_t)A & 15) || ((uintptr_t)W & 15) || (W2 && ((uintptr_t)W2 & 15))) return 1;
   JLLM_TAKE_GATE("gemm_mfma_grouped", epilogue, gate_limit, gs);
   if ((epilogue != 0 && epilogue != 2) || (epilogue == 2) != (W2 != nullptr)) JLLM_FAIL("gemm_mfma_grouped: epilogue %d", epilogue);
@@ -543,7 +550,7 @@ extern "C" int jllm_gemm_mfma_grouped_bf16(const void* A, int lda, const void* W
 int jllm_gemm_mfma_heads(const void* in, int ld_in, int in_hstride, const void* W, void* out, int ld_out, int out_hstride, int M,
                          int H, int N, int K, const void* gate, int ld_gate, hipStream_t stream) {
   using T = Tiled<false, FORM_HEADS, 2, 4, 2, 2, 3>;
-  if (!tiled_rows_fit(ld_in, K)) return 1;
+  if (!tiled_rows_fit(T::ROWS, ld_in, T::COLS, K)) return 1;
   dim3 grid((N + T::COLS - 1) / T::COLS, (M + T::ROWS - 1) / T::ROWS, H);
   if (grid.y > 65535) return 1;
   if (!T::allow()) JLLM_FAIL("gemm_mfma_heads: cannot reserve %d bytes of LDS", T::LDS);

@@ -290,6 +290,29 @@ def test_gemm_ring_of_half_stages(ops, monkeypatch, M, N, K, cut):
     assert bool(((got[0].double() - ref).abs() <= K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
 
 
+@pytest.mark.parametrize("M,N,K,stride", [(66, 72, 128, (1 << 22) + 8), (130, 72, 192, (1 << 23) + 8), (65, 24, (1 << 23) + 64, (1 << 23) + 64)])
+def test_gemm_of_very_long_rows(ops, M, N, K, stride):
+    """Rows 8 and 16 MB and more apart, beyond the 32-bit offsets of a tile: still the tiled kernel. Small whole numbers, so that every sum
+    is exact, at the ends of K and in between."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(M)
+    at = sorted({0, 1, 63, 64, K // 2 - 1, K // 2, K - 65, K - 64, K - 1} & set(range(K)))
+    whole = torch.zeros(M * stride, dtype=torch.bfloat16, device=DEV)
+    a = whole.as_strided((M, K), (stride, 1))
+    a[:, at] = torch.randint(-3, 4, (M, len(at)), device=DEV, generator=gen).bfloat16()
+    w, w2 = (torch.zeros(N, K, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    for x in (w, w2):
+        x[:, at] = torch.randint(-3, 4, (N, len(at)), device=DEV, generator=gen).bfloat16()
+    g, u = (a[:, at].double() @ x[:, at].double().T for x in (w, w2))
+    ops.reset_stats()
+    assert torch.equal(ops.gemm(a, w, out_dtype=torch.float32).double(), g)
+    res = torch.ones(M, N, device=DEV)
+    ops.gemm(a, w, out=res, epilogue=ops.EPI_ADD)
+    assert torch.equal(res.double(), g + 1)
+    assert bf16_close(ops.gemm(a, w, w2=w2, epilogue=ops.EPI_GATED), g / (1 + torch.exp(-g)) * u, ulps=1.01)[0]
+    assert ops.stats()["ran"] == {"jllm_gemm_mfma_bf16": 3} and not ops.stats()["general"], ops.stats()
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 520, 128), (130, 516, 192), (256, 1024, 256), (385, 131, 576)])
 def test_the_small_tile_gives_the_bits_of_the_two_group_kernel(ops, monkeypatch, M, N, K):
     """The small tile's accumulators lie otherwise over the lanes (32 x 32) than the two-group kernel's (16 x 16): every
