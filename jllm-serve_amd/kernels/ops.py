@@ -1209,9 +1209,9 @@ def _cut_takes_norm(M: int, N: int, K: int) -> bool:
 
 
 def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0, norm=_NO_NORM) -> bool:
-    """The bf16 matrix-core kernels: a weight-streaming one for up to 16 rows, another for up to 64; for many rows
-    the two-group kernel with tiles of 256 or 192 rows by 256 columns or the small tile, either with K cut over several
-    workgroups when the output has few tiles (`_tiled_plan`, `_tiles`); then the reduction makes the ``norm`` (gain, its type, eps, rows,
+    """The bf16 matrix-core kernels: a weight-streaming one for up to 16 rows, another for up to 64 and for some products of more
+    (`_row_plan`); for the others tiles of 256 or 192 rows by 256 columns or one of five smaller ones, either with K cut over several
+    workgroups where the output has few tiles (`_tiled_choice`); then the reduction makes the ``norm`` (gain, its type, eps, rows,
     their stride) of the new rows where one is asked for. Each declines shapes it does
     not take; then the fp32 kernel runs."""
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
@@ -1237,7 +1237,9 @@ def _fast_gemm(a, w, w2, bias, out, epilogue, gate_limit: float = 0.0, norm=_NO_
         partial = torch.empty((cut * M * N,), dtype=torch.float32, device=a.device) if cut > 1 else None
         if _try("jllm_gemm_pingpong_bf16", *head, tile, cut, _ptr(partial), *norm, _stream()):
             return True
-        tile, cut = 128128, _k_splits(M, N, K, w2 is not None) if K % 64 == 0 else 1
+        if K % 64:
+            return False  # (the other kernel takes whole stages only)
+        _, tile, cut = _small_bests(-(-M // 64), N, K, w2 is not None)[norm is not _NO_NORM]  # (it declines operands of 4 GB)
         if cut == 1 and norm is not _NO_NORM:
             return False
     partial = torch.empty((cut * M * N,), dtype=torch.float32, device=a.device) if cut > 1 else None

@@ -284,6 +284,37 @@ def test_choices_of_the_tiled_products():
     assert len(taken) > 25 and {t for t, _ in taken} == {192, 256, ops.WIDE_LAST, *ops.SMALL_TILES}, taken
 
 
+def test_what_the_large_tiles_decline_goes_to_the_best_small_one(monkeypatch):
+    """An operand of 4 GB is none of the large tiles': the smaller ones take it in the tile and cut that are the cheapest of theirs, also with
+    the norm of the new rows."""
+    import torch
+
+    import recorded
+    seen = recorded.record(monkeypatch)
+    monkeypatch.setattr(ops, "_try", lambda name, *args: seen.append((name, args)) or name != "jllm_gemm_pingpong_bf16")
+    asked = 0
+    for m, n, k in ((2048, 4096, 12288), (1800, 6144, 4096), (600, 5120, 17408), (8192, 4096, 4096)):
+        a, w, res, gain = recorded.tensor(m, k), recorded.tensor(n, k), recorded.tensor(m, n, dtype=torch.float32), recorded.tensor(n)
+        for normed, gated in ((False, False), (False, True), (True, False)):
+            if ops._own_choice(m, n, k, gated, normed)[0] > 1000 or (normed and not ops._cut_takes_norm(m, n, k)):
+                continue
+            asked += 1
+            small = ops._small_bests(-(-m // 64), n, k, gated)[normed][1:]
+            del seen[:]
+            if normed:
+                with monkeypatch.context() as mp:
+                    mp.setattr(torch.Tensor, "data_ptr", lambda self: 0)
+                    ops.gemm_add_then_norm(a, w, res, gain, 1e-5, torch.bfloat16)
+            else:
+                ops.gemm(a, w, w2=w if gated else None, epilogue=ops.EPI_GATED if gated else ops.EPI_STORE)
+            assert [name for name, _ in seen][0] == "jllm_gemm_pingpong_bf16", (m, n, k)
+            if normed and small[1] == 1:
+                continue  # K stays whole: the norm is a launch behind it
+            name, args = seen[1]
+            assert name == "jllm_gemm_mfma_bf16" and args[14:16] == small, (m, n, k, gated, normed, args[14:16], small)
+    assert asked >= 6
+
+
 def test_the_native_walks_find_the_cheapest():
     """The walks over the choices against every single one's time."""
     cus = ops.compute_units()
