@@ -546,7 +546,8 @@ def _ride_plan(M: int, N: int, K: int, reader: Optional[Tuple[int, bool]]) -> Op
     """The plan (`_row_plan`) of an adding product of M rows, N outputs and K inputs that prepares the norm that follows, or
     None where it does not. For more than 64 rows it does so where the same kernel takes both it and the product that reads
     the norm (``reader``: its outputs and whether it is gated; not known: plain, with N outputs), from the row count on at
-    which the rows may be laid out for many rows (`activation_rows`). A norm that is prepared for a reader which does not
+    which the rows may be laid out for many rows (`activation_rows`); since the tiled kernels cut such products and make the norm in
+    their reduction, hardly any of the models' are among these. A norm that is prepared for a reader which does not
     take it is made again by a launch of its own."""
     if M > STREAM_MAX_ROWS:
         outputs, gated = reader if reader is not None else (N, False)
@@ -1094,10 +1095,8 @@ def _row_plan(M: int, N: int, K: int, gated: bool, adds: int) -> Optional[Tuple[
 
 # Estimated times of that kernel for more than 64 rows, in microseconds
 WIDE_MOST_ROWS = 1024
-# Into the residual: up to here. The estimates count the norm behind such a product as a launch that only this kernel saves,
-# but the tiled kernels' reduction makes it too where they cut K, as they do for wider rows. o and gate/up in turn without this
-# limit, us: 4B at 128 rows 58.2 -> 55.3, 8B at 832 239.6 -> 228.7; down and qkv: 4B at 160 rows 55.7 -> 58.1, 14B at 192
-# 128.3 -> 131.0. Taking the credit away instead made the narrow ones slower (0.6B down and qkv at 160 rows 21.9 -> 24.8).
+# Into the residual: up to here (wider ones are cut by the tiled kernels, whose reduction makes the norm as well; without this limit 4B o
+# and gate/up in turn at 128 rows 50.0 -> 52.8 us, the others as they are)
 WIDE_ADD_COLUMNS = 2048
 WIDE_LEAST_K = 1024               # the shortest K it was measured at
 WIDE_BLOCK_US = (0.275, 0.0198)   # 64 of k on 32 weight and 64 activation rows, and per 8 rows more of either
@@ -1105,9 +1104,6 @@ WIDE_FIXED_US = {64: 3.9, 128: 7.2}   # the launch, the first blocks and the end
 WIDE_PAIR = (1.35, 1.8)           # two workgroups of 64 rows on a compute unit: a few of them, all
 WIDE_MERGE_US = (2.5, 0.06)       # parts of K: the way through memory, and per KB of sums that the last workgroup reads
 WIDE_BYTES_PER_US = 5.3e6         # weights from memory
-# a norm that rides on a product of 128 rows, of the tiled kernels' estimate (o and gate/up in turn, us, here / tiled: 0.6B 19.3 / 18.2,
-# 1.7B 30.1 / 29.7; beyond 128 rows 2 to 30 behind)
-WIDE_NORM_AT_MOST = 1.25
 
 
 @functools.lru_cache(maxsize=None)
@@ -1152,7 +1148,7 @@ def _wide_plan(M: int, N: int, K: int, gated: bool, adds: int = 0) -> Optional[T
         return None
     t, plan = _wide_best(-(-M // 64), min(M, 128), N, K, gated)
     limit = _own_choice(M, N, K, gated, adds == ADDS_AND_NORM)[2]
-    return plan if t < (limit * WIDE_NORM_AT_MOST if adds == ADDS_AND_NORM and M <= 128 else limit) else None
+    return plan if t < limit else None
 
 
 _NO_NORM = (None, F32, 0.0, None, 0)

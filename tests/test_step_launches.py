@@ -16,7 +16,7 @@ def test_a_norm_is_prepared_only_where_its_reader_takes_it(monkeypatch, size):
     seen = recorded.record(monkeypatch)
     m = recorded.model(*SHAPES[size], layers=3)
     rode = 0
-    for rows in (65, 127, 128, 200, 321, 400, 487, 512, 513, 600, 640, 750, 897, 960, 1009, 1024, 1500):
+    for rows in (17, 40, 64, 65, 127, 128, 200, 321, 400, 487, 512, 513, 600, 640, 750, 897, 960, 1009, 1024, 1500):
         del seen[:]
         recorded.forward(m, (rows, 0))
         left = read = 0
