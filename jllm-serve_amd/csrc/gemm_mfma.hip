@@ -251,7 +251,7 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(
     }
     return;
   }
-  tile_epilogue<GATED, 16, RM, CN, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
+  tile_epilogue<GATED, RM, CN, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
                                              (int)blockIdx.z, (int)gridDim.z);
 }
 

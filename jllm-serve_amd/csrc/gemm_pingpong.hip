@@ -209,7 +209,7 @@ __device__ __forceinline__ void pingpong_tile(
     half(std::integral_constant<int, 0>{}, std::false_type{}, t);
     half(std::integral_constant<int, 1>{}, std::false_type{}, t);
   }
-  tile_epilogue<GATED, 16, 2 * FM, 4, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
+  tile_epilogue<GATED, 2 * FM, 4, TBM, TBN>(acc, lane, wm, wn, m0, n0, bias, bias_dtype, out, out_dtype, ldo, M, N, epilogue, gs, partial,
                                                 (int)blockIdx.z, (int)gridDim.z);
 }
 

@@ -70,7 +70,7 @@ __global__ __launch_bounds__(LM_WAVES * 64) void latent_attention_mfma_kernel(
   const bool wave_live = kpar || qwave * 16 < HB;  // (a wave without a live query vector only helps to load)
   const int dks = WHOLE ? DKS : (Dk + 31) >> 5, r16 = WHOLE ? RT : R >> 4;
   constexpr int RTH = (RT + 1) / 2;  // accumulators of one wave: its half of the latent's 16-dim blocks
-  static_assert(!WHOLE || RT % 2 == 0, "two equal halves");
+  static_assert(!WHOLE || (RT % 2 == 0 && DKS % 2 == 0), "two equal halves of the latent, and a row in loads of 64 entries");
   const int j_lo = rhalf ? (r16 + 1) / 2 : 0, nj = WHOLE ? RTH : rhalf ? r16 - (r16 + 1) / 2 : (r16 + 1) / 2;
   const int psh = __builtin_ctz(page_size);
   const int* tbl = block_table + (size_t)req * max_blocks;
