@@ -543,20 +543,35 @@ extern "C" int jllm_gemm_mfma_grouped_bf16(const void* A, int lda, const void* W
   return 0;
 }
 
-// The per-head products of latent attention for many rows (latent_heads.hip, which checks the arguments): K a multiple of
-// 64, N of 4. Through LDS in tiles of 128 x 128 a row's and a weight's loads are shared by a workgroup; read straight
-// from memory by every wave (64 x 64 outputs each) 2,556 rows of 16 heads took 76 us at 512 x 128 with a rotated tail and 41
-// at 128 x 512 with a gate, here (the tail a launch of its own) 35 and 21.
-int jllm_gemm_mfma_heads(const void* in, int ld_in, int in_hstride, const void* W, void* out, int ld_out, int out_hstride, int M,
-                         int H, int N, int K, const void* gate, int ld_gate, hipStream_t stream) {
-  using T = Tiled<false, FORM_HEADS, 2, 4, 2, 2, 3>;
+template <int RM, int CN, int WGM, int WGN, int NS>
+static int launch_heads(const void* in, int ld_in, int in_hstride, const void* W, void* out, int ld_out, int out_hstride, int M,
+                        int H, int N, int K, const void* gate, int ld_gate, hipStream_t stream) {
+  using T = Tiled<false, FORM_HEADS, RM, CN, WGM, WGN, NS>;
   if (!tiled_rows_fit(T::ROWS, ld_in, T::COLS, K)) return 1;
   dim3 grid((N + T::COLS - 1) / T::COLS, (M + T::ROWS - 1) / T::ROWS, H);
   if (grid.y > 65535) return 1;
   if (!T::allow()) JLLM_FAIL("gemm_mfma_heads: cannot reserve %d bytes of LDS", T::LDS);
-  gemm_mfma_kernel<false, FORM_HEADS, 2, 4, 2, 2, 3><<<grid, T::THREADS, T::LDS, stream>>>(
+  gemm_mfma_kernel<false, FORM_HEADS, RM, CN, WGM, WGN, NS><<<grid, T::THREADS, T::LDS, stream>>>(
       (const bf16_t*)in, ld_in, (const bf16_t*)W, nullptr, nullptr, 0, out, JLLM_BF16, ld_out, M, N, K, 0, GateSpec{}, nullptr, GroupArgs{},
       HeadsArgs{in_hstride, out_hstride, (const bf16_t*)gate, ld_gate}, 0);
   JLLM_CHECK_LAUNCH("gemm_mfma_heads");
   return 0;
+}
+
+// The per-head products of latent attention for many rows (latent_heads.hip, which checks the arguments): K a multiple of
+// 64, N of 4. Through LDS a row's and a weight's loads are shared by a workgroup, two of which share a compute unit: tiles of 64 x 128 in
+// rings of three stages, or of 128 x 128 in rings of two where these take fewer rounds of workgroups (a round of one to a compute unit
+// 0.6 of one of two; one of 128 x 128 1.66 of 64 x 128). us, straight from memory by every wave (64 x 64 outputs each) / 64 x 128 / 128 x
+// 128, 512 x 128: 16 heads at 500 rows 11.9 / 7.4 / 7.5, at 2,556 42.2 / 24.9 / 24.0, 64 heads at 65 rows - / 8.2 / 6.7, 32 heads at 2,556
+// - / 55.2 / 41.9; 128 x 512 with a gate: 16 heads at 65 rows 14.4 / 8.6 / 11.9, at 2,556 41 / 21.2 / 22.3, 64 heads at 800 - / 29.0 / 28.0.
+int jllm_gemm_mfma_heads(const void* in, int ld_in, int in_hstride, const void* W, void* out, int ld_out, int out_hstride, int M,
+                         int H, int N, int K, const void* gate, int ld_gate, hipStream_t stream) {
+  const long cus = jllm_compute_units(), cols = (N + 127) / 128;
+  auto rounds = [&](int rows) {  // of two workgroups to a compute unit
+    const long groups = ((M + rows - 1) / rows) * cols * H, last = groups % (2 * cus);
+    return groups / (2 * cus) + (last == 0 ? 0.0 : last <= cus ? 0.6 : 1.0);
+  };
+  if (rounds(64) < 1.66 * rounds(128))
+    return launch_heads<2, 4, 2, 2, 3>(in, ld_in, in_hstride, W, out, ld_out, out_hstride, M, H, N, K, gate, ld_gate, stream);
+  return launch_heads<4, 4, 2, 2, 2>(in, ld_in, in_hstride, W, out, ld_out, out_hstride, M, H, N, K, gate, ld_gate, stream);
 }

@@ -118,11 +118,11 @@ extern "C" int jllm_latent_heads_bf16(const void* in, int ld_in, int in_hstride,
   if (mode == 1 && ((ld_gate & 3) || ((uintptr_t)gate & 7) || !gate)) return 1;
   if (mode == 0 && tail > 0 && (!positions || (rot_dims && (!cos_t || !sin_t)))) JLLM_FAIL("latent_heads: the rotated tail needs positions and tables");
   const bool few = M <= 16;
-  // Tiles of 128 rows (the same bits: one accumulator per output, K in steps of 32); the rotated tail then is the only column
-  // of workgroups of the kernel above, a launch of its own. 16 heads of 512 x 128 with a tail: 70 rows 11 us in one
-  // launch, 13 in two, 100 rows 14.1 / 13.8, 300 38 / 14, 2,556 76 / 35; of 128 x 512 without one: 70 rows 14.8 / 13.8,
-  // 2,556 41 / 21.
-  const bool tiled = M > (mode == 0 && tail > 0 ? 96 : 64) && (K & 63) == 0;
+  // Tiles through LDS (the same bits: one accumulator per output, K in steps of 32); the rotated tail then is the only column
+  // of workgroups of the kernel above, a launch of its own. us, straight from memory / through LDS, 16 heads of 512 x 128 with a tail (32
+  // heads): 32 rows 6.5 / 8.0 (7.2 / 8.1), 40 7.5 / 8.1 (8.2 / 8.2), 48 8.4 / 8.1 (9.4 / 8.4), 64 10.4 / 8.4 (11.5 / 8.6), 96 14.3 / 8.5 (16.3 / 10.3);
+  // without one 17 rows 4.7 / 4.5, 64 5.6 / 4.9 (64 heads 7.5 / 6.4); of 128 x 512 17 rows 10.6 / 8.2, 64 14.3 / 8.2.
+  const bool tiled = M > (mode == 0 && tail > 0 ? 40 : 16) && (K & 63) == 0;
   if (tiled) {
     const int rc = jllm_gemm_mfma_heads(in, ld_in, in_hstride, W, out, ld_out, out_hstride, M, H, N, K, mode == 1 ? gate : nullptr, ld_gate, stream);
     if (rc != 0) return rc;

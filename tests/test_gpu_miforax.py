@@ -161,7 +161,7 @@ def _attend_plain(qa, rows, R, window, scale, sink, q_pos):
 @pytest.mark.parametrize("N,K,tail,gated", [(512, 128, 64, False), (128, 512, 0, True), (36, 64, 24, False), (132, 192, 0, True),
                                             (20, 40, 8, False), (100, 256, 0, True), (68, 320, 16, False)])
 def test_heads_products_at_every_row_count(N, K, tail, gated):
-    """The per-head products where their kernel changes (up to 16 rows, up to 64 or 96, tiles of 128 rows beyond) and at odd
+    """The per-head products where their kernel changes (up to 16 rows, up to 40 with a tail, tiles of 64 or 128 rows beyond) and at odd
     sizes: against float64, and a row's bits are those it has in any other batch."""
     from jllm_serve_amd.kernels import ops
     gen = torch.Generator(device="cuda")
@@ -180,7 +180,7 @@ def test_heads_products_at_every_row_count(N, K, tail, gated):
                                 cos=cos if tail else None, sin=sin if tail else None, gate=gate[:n].contiguous() if gated else None)
 
     whole = heads(M)
-    for n in (1, 16, 17, 64, 65, 96, 97, 128, 129):
+    for n in (1, 16, 17, 40, 41, 64, 65, 96, 97, 128, 129):
         assert torch.equal(heads(n), whole[:n]), n
     rows = x.double().view(M, H, K + tail)
     want = torch.einsum("mhk,hnk->mhn", rows[..., :K], w.double())
@@ -195,6 +195,28 @@ def test_heads_products_at_every_row_count(N, K, tail, gated):
         a, b = t[..., :rot // 2], t[..., rot // 2:rot]
         turned = torch.cat([a * c - b * s, b * c + a * s, t[..., rot:]], dim=-1)
         assert bool(((got[..., N:] - turned).abs() <= 2.0 ** -8 * turned.abs() + 2.0 ** -22 * (a.abs().max() + b.abs().max())).all())
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320])
+@pytest.mark.parametrize("M", [65, 193, 257])
+def test_heads_products_in_tall_tiles(M, K):
+    """Heads enough for tiles of 128 x 128 (a ring of two stages: K of one, of two and of more, even and odd) have the bits of a few of them,
+    which go through tiles of 64 x 128, with a gate and without."""
+    from jllm_serve_amd.kernels import ops
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + K)
+    H, N = 256, 132  # 512 tiles of either kind for each of their rows
+    x = torch.randn(M, H * K, device="cuda", generator=gen).bfloat16()
+    w = (torch.randn(H, N, K, device="cuda", generator=gen) * K ** -0.5).bfloat16()
+    gate = torch.randn(M, H * N, device="cuda", generator=gen).bfloat16()
+    plain, gated = ops.latent_heads(x, w), ops.latent_heads(x, w, gate=gate)
+    want = torch.einsum("mhk,hnk->mhn", x.double().view(M, H, K), w.double())
+    room = 2.0 ** -8 * want.abs() + (K * 2.0 ** -24) * torch.einsum("mhk,hnk->mhn", x.double().abs().view(M, H, K), w.double().abs())
+    assert bool(((plain.double().view(M, H, N) - want).abs() <= room).all())
+    for h in (0, 137, H - 2):
+        at, to = slice(h * K, (h + 2) * K), slice(h * N, (h + 2) * N)
+        assert torch.equal(ops.latent_heads(x[:, at].contiguous(), w[h:h + 2].contiguous()), plain[:, to])
+        assert torch.equal(ops.latent_heads(x[:, at].contiguous(), w[h:h + 2].contiguous(), gate=gate[:, to].contiguous()), gated[:, to])
 
 
 @pytest.mark.parametrize("N,K", [(16, 8), (20, 72), (33 * 4, 520), (48, 1096), (36, 2048), (64, 2128)])
