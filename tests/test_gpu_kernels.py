@@ -74,7 +74,7 @@ GEMM_SHAPES = [(1, 16, 128), (5, 48, 384), (16, 4096, 128), (17, 80, 256), (33, 
                (8, 6144, 256), (3, 6144, 128), (16, 6144, 1152),  # 24 weight rows per workgroup (N / 24 = 256 of them)
                (8, 5120, 256), (1, 5120, 1152), (13, 7168, 384), (16, 10240, 128),  # 20 weight rows per workgroup for N = 5120
                (5, 32768, 128), (16, 32800, 256),  # thousands of 16-row tiles
-               (100, 256, 64), (70, 200, 192), (90, 136, 320),  # one, three and five K steps of the tiled kernel's two-ahead form
+               (100, 256, 64), (70, 200, 192), (90, 136, 320),  # one, three and five stages of the tiled kernel's rings
                (3, 50, 70), (65, 96, 128), (200, 130, 96), (128, 256, 512), (300, 384, 4096), (1000, 192, 136)]
 
 
@@ -114,19 +114,23 @@ def test_gemm_epilogues(ops, M, N, K, dtype):
         assert bf16_close(out, want, ulps=1.01)[0]
 
 
-def test_gemm_large_tile(ops):
-    """Products with at least 512 tiles of 256 x 256 go through the 8-wave tile: all three epilogues at sizes that
-    leave partial tiles in both directions, and the same bits as the small tile gives for the same rows."""
+def test_gemm_large_tile(ops, monkeypatch):
+    """Products of many tiles in tiles of 256 rows, whatever the choice between tiles makes of so short a K: all three epilogues at sizes that
+    leave partial tiles in both directions, and the same bits as the smaller tiles give for the same rows."""
+    own = ops._tiled_choice
+    monkeypatch.setattr(ops, "_tiled_choice", lambda m, *rest: (256, 1) if m > 128 else own(m, *rest))
     torch.manual_seed(5)
     M, N, K = 530, 43800, 192
     a = torch.randn(M, K, device=DEV).bfloat16()
     w = (torch.randn(N, K, device=DEV) / math.sqrt(K)).bfloat16()
     bias = torch.randn(N, device=DEV)
     ref = a.double() @ w.double().T
+    ops.reset_stats()
     out = ops.gemm(a, w, out_dtype=torch.float32)
     assert torch.allclose(out.double(), ref, rtol=1e-5, atol=2e-5 * ref.abs().max())
-    small = ops.gemm(a[:100].contiguous(), w, out_dtype=torch.float32)   # few tiles: the 4-wave kernel
+    small = ops.gemm(a[:100].contiguous(), w, out_dtype=torch.float32)
     assert torch.equal(small, out[:100])
+    assert ops.stats()["ran"] == {"jllm_gemm_pingpong_bf16": 1, "jllm_gemm_mfma_bf16": 1}
     assert bf16_close(ops.gemm(a, w, bias=bias), ref + bias.double())[0]
     res = torch.randn(M, N, device=DEV)
     want = res.double() + ref
@@ -155,7 +159,7 @@ def test_gemm_large_tile(ops):
                                         (520, 16400, 4096, (256, 1)), (2000, 4096, 8192, (256, 2)), (1024, 6140, 8256, (256, 2)),
                                         (1000, 4100, 8192, (256, 2)), (640, 4100, 8192, (256, 4)), (1024, 6144, 4096, (256, 2))])
 def test_gemm_two_group_kernel(ops, monkeypatch, M, N, K, plan):
-    """The tiled kernel whose waves take turns at the matrix cores (direct-to-LDS loads, a ring of stages) with its tile of 256
+    """The large tiles' kernel (loads straight to LDS, a ring of half stages) with its tile of 256
     rows, whatever the choice between tiles makes of these sizes: every epilogue, with a bias, partial tiles in both directions, K from four stages to many, inputs and
     outputs whose rows are not contiguous, K cut in two or four with partial sums (also an odd number of stages per half);
     against float64."""
@@ -241,10 +245,12 @@ def test_gemm_two_group_kernel_with_wide_last_rows(ops, monkeypatch, M, N, K, cu
     assert bool(((got[1].double() - ref).abs() <= K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
 
 
-@pytest.mark.parametrize("M,N,K,cut", [(65, 68, 64, 1), (129, 131, 128, 1), (255, 260, 320, 2), (257, 516, 448, 3), (300, 1028, 1088, 5)])
+@pytest.mark.parametrize("M,N,K,cut", [(65, 68, 64, 1), (129, 131, 128, 1), (255, 260, 320, 2), (257, 516, 448, 3), (300, 1028, 1088, 5),
+                                       (300, 260, 1088, 1), (129, 131, 1024, 1), (257, 516, 2176, 3), (200, 324, 704, 1), (70, 200, 960, 2)])
 def test_gemm_small_tiles(ops, monkeypatch, M, N, K, cut):
-    """Every tile of the small kernel against every other, bit for bit, and float64: one row beyond a tile and one short of it, K of one
-    stage, shorter than the rings and longer, an odd number of stages, whole and in parts of unequal length, every epilogue. (Gated:
+    """Every tile of the small kernel against every other and against the tile of 256 x 256, bit for bit, and float64: one row beyond a tile
+    and one short of it, odd numbers of column tiles, K of one stage, shorter than the rings (of three to five stages), and so long that
+    every slot of every ring is filled again, an even and an odd number of stages, whole and in parts of unequal length, every epilogue. (Gated:
     tiles that lie inside the output take the hardware's exponential and reciprocal, others the library's, some 2^-22 of the value.)"""
     gen = torch.Generator(device=DEV)
     gen.manual_seed(M + K)
@@ -260,6 +266,13 @@ def test_gemm_small_tiles(ops, monkeypatch, M, N, K, cut):
         ops.gemm(a, w, bias=bias, out=res, epilogue=ops.EPI_ADD)
         got.append([res, ops.gemm(a, w, out_dtype=torch.float32), ops.gemm(a, w, bias=bias), ops.gemm(a, w, w2=w2, epilogue=ops.EPI_GATED)])
         assert ops.stats()["ran"] == {"jllm_gemm_mfma_bf16": 4}
+    if K // cut >= 128:
+        monkeypatch.setattr(ops, "_tiled_choice", lambda m, n, k, gated, normed: (256, 1 if gated else cut))
+        ops.reset_stats()
+        res = torch.ones(M, N, device=DEV)
+        ops.gemm(a, w, bias=bias, out=res, epilogue=ops.EPI_ADD)
+        got.append([res, ops.gemm(a, w, out_dtype=torch.float32), ops.gemm(a, w, bias=bias), ops.gemm(a, w, w2=w2, epilogue=ops.EPI_GATED)])
+        assert ops.stats()["ran"] == {"jllm_gemm_pingpong_bf16": 4}
     for other in got[1:]:
         assert all(torch.equal(x, y) for x, y in zip(got[0][:3], other[:3]))
         x, y = got[0][3].double(), other[3].double()
@@ -315,7 +328,7 @@ def test_gemm_of_very_long_rows(ops, M, N, K, stride):
 
 @pytest.mark.parametrize("M,N,K", [(65, 520, 128), (130, 516, 192), (256, 1024, 256), (385, 131, 576)])
 def test_the_small_tile_gives_the_bits_of_the_two_group_kernel(ops, monkeypatch, M, N, K):
-    """The small tile's accumulators lie otherwise over the lanes (32 x 32) than the two-group kernel's (16 x 16): every
+    """Tiles of 128 x 128 (fragments of a whole stage in registers) against tiles of 256 x 256 (of half a stage): every
     epilogue at whole tiles, at edges and at rows that cannot be stored eight at a time, bit for bit."""
     gen = torch.Generator(device=DEV)
     gen.manual_seed(M + N)

@@ -110,7 +110,7 @@ def test_plan_of_the_two_group_kernel():
 
 def test_plan_of_the_tiled_products():
     """The plan that the dispatch asks for: a tile that a kernel has (192 or 256 rows, or none), K cut only where every
-    workgroup keeps a long range of whole stages and never for the gated product, few rows and shapes that the two-group
+    workgroup keeps a long range of whole stages and never for the gated product, few rows and shapes that the large tiles'
     kernel cannot take with the small tile, whose cuts are the small tile's own, tiles of 192 rows with K cut only where they
     leave fewer empty rows than 256, never for a near tie of the gated product, nor in one round over a short K where they
     have no empty rows to save; for the models' products and for odd sizes."""
