@@ -16,6 +16,8 @@
 // What stood here before (128 x 128 through registers and two LDS buffers, 32 x 32 x 16; below a thousand rows mostly gemm_stream.hip,
 // with LDS reads of 144 KB a stage) / this, us inside a graph, products alone: 0.6B shape at 487 rows qkv 12.2 / 8.9, gate/up 16.8 /
 // 14.6, 8B qkv at 128 rows 25.7 / 20.5, at 631 50.9 / 41.4, o at 128 20.1 / 15.
+// A ring of two stages (64 KB, four waves) lets two workgroups of 128 x 128 share a compute unit, each stage's loads landing within the stage
+// before: the grouped form's, and the per-head form's where it takes many.
 //
 // Epilogues as in gemm_epilogue.h; K cut over gridDim.z leaves fp32 partial tiles that the reduction below adds up. Two further
 // forms: grouped (a workgroup's rows belong to one group, with weights of its own, gathered by an index list) and per head.

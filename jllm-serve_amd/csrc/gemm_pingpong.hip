@@ -236,10 +236,10 @@ __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_kernel(
 // Tiles of 256 x 256 and, for the last rows where those are at most 128, of 128 x 512 (64 x 512 where they are at most 64): `wide`
 // of the latter, which come first because they take longer, then rows of `cols` of the former. A tile of 256 rows of which a few
 // are there takes as long as a full one, and so does the round of workgroups that it begins. A wide tile takes half as many
-// workgroups; its stage moves a quarter (an eighth) more bytes into LDS and takes 1.25 (1.17) times as long. us, what was chosen
-// among whole tiles / this: gate/up of the 8B shape at 560 rows (288 tiles / 240) 167 / 122, at 631 171 / 131, of the 14B shape at 300 223 / 153,
-// at 1,320 522 / 457, at 4,614 (10.1 rounds / 9.8) 1,558 / 1,498, of the 32B shape at 600 412 / 345; 14B down at 3,111 620 / 501, 4B
-// qkv at 2,600 106 / 75. Last rows of 129 to 192 in a tile of either kind gained nothing (8B gate/up at 700 rows 169 / 196).
+// workgroups; its stage moves a quarter (an eighth) more bytes into LDS and takes 1.13 (1.03) times as long. us, the best of whole tiles of
+// any size / this: gate/up of the 8B shape at 560 rows (288 tiles / 240) 125.7 / 98.7, at 631 131.4 / 104.4, of the 14B shape at 300 182.7 / 138.9,
+// at 1,320 392.8 / 370.4, at 4,614 (10.1 rounds / 9.8) 1,285 / 1,189, of the 32B shape at 600 351.6 / 305.9; 14B down at 3,111 484.1 / 406.8, 4B
+// qkv at 2,600 79.8 / 64.9. Last rows of 129 to 192 in a tile of either kind gained nothing.
 template <bool GATED>
 __global__ __launch_bounds__(PP_WAVES * 64) void gemm_pingpong_mixed_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,

@@ -666,17 +666,13 @@ def check_attention_shape(heads: int, kv_heads: int, head_dim: int, rotary_dim: 
 
 SKINNY_MAX_ROWS = 16   # up to here the weight-streaming kernel; its activation traffic grows with the rows
 TILE_COLS = 128
-# first a workgroup for every compute unit; then two of the small tile's workgroups share a compute unit ...
-SPLIT_LONG_STEPS = 16     # ... where each still has this many 64-wide K steps
+SPLIT_LONG_STEPS = 16     # 64-wide K steps that each of two workgroups a compute unit still has
 
 
 def _k_splits(M: int, N: int, K: int, gated: bool) -> int:
-    """How many ways the tiled kernel cuts K so that a product with few output tiles still fills the GPU. Splits are
-    doubled until every compute unit has a workgroup, and further, up to two per compute unit, only while the K range
-    of a workgroup stays long (short ranges are mostly prologue, and every split writes and reads a partial
-    result). Measured on the products of the 8B shape at 96 to 1,024 rows against every power of two: this choice
-    is the fastest or within 3 % of it; the four products together at 384 rows 324 -> 283 us, at 512 rows
-    332 -> 304, at 1,024 rows 559 -> 534 against filling the compute units once."""
+    """How many ways `_pingpong_plan` takes the tiles of 128 x 128 to cut K, which it weighs the large tile against: doubled until every
+    compute unit has a workgroup, and further, up to two per compute unit, only while the K range of a workgroup stays long. What such a
+    product is cut into is `_small_bests`' choice."""
     if gated:
         return 1
     tiles = -(-N // TILE_COLS) * -(-M // 128)
@@ -696,50 +692,36 @@ def _k_splits(M: int, N: int, K: int, gated: bool) -> int:
 
 PINGPONG_SPLIT_MIN_K = 1024    # a K range this long per workgroup pays for the partial sums of a cut in two or four
 PINGPONG_MIN_ROWS = 257        # below, the 256-row tile is mostly empty rows
-# Estimated times, in microseconds, fitted to the sweep that `_pingpong_plan` describes:
+# Its prices, in microseconds (`_pingpong_plan` says what is left to them):
 PINGPONG_STEP_US = 0.69        # 32 of K on a 256 x 256 tile, one workgroup a compute unit
-TILED_STEP_US = 0.54           # 32 of K on the other kernel's 128 x 128 tiles, two workgroups a compute unit
-TILED_ROUND_US = 4.4           # what a round of the other kernel's workgroups costs beside its K steps
+TILED_STEP_US = 0.54           # 32 of K on tiles of 128 x 128, two workgroups a compute unit
+TILED_ROUND_US = 4.4           # what a round of those costs beside its K steps
 PINGPONG_SUM_US = 2.3e-6       # per element of a partial result: written in 32-bit, read back and summed
 TILED_SUM_US = 1.9e-6
 
 
 def _pingpong_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int]:
-    """(rows of the output tile, ways K is cut) with which the two-group kernel takes a product, or (0, 1) when the
-    other tiled kernel is the better choice. The 256 x 256 tile moves the fewest bytes per multiply (a compute unit
-    fills its LDS at 32 bytes a clock at most, which is what this tile needs at the matrix cores' full rate) but
-    needs enough tiles to fill the compute units; since the kernel's loads cost no vector instructions, K ranges
-    down to 1,024 pay as well (ranges of 512 and cuts in eight were slower). A 128-row form of the same kernel was
-    measured (86 / 88 us and 222 / 235 alone, 90 / 88 and 254 / 234 inside the model) and not kept.
+    """(256, ways K is cut) where tiles of 256 x 256 are the first choice for a product, or (0, 1) where tiles of 128 x 128 are. Where the
+    dispatch begins: the prices are of earlier forms of both kernels, `_tiled_plan` weighs tiles of 192 rows beside the outcome,
+    `_finer_tiles` all large tiles and cuts and `_choice_of` the smaller ones, each by `_tile_us`, so that a plan stays only where nothing is
+    estimated at less than `FINER_AT_MOST` or `SMALL_AT_MOST` of its time.
 
-    Plain products: the choice with the smallest estimated time. Workgroups run in rounds (one per compute unit here,
-    two of the other kernel's); a round takes its K steps, and a cut of K adds the partial sums' traffic. The five
-    constants were fitted to a sweep of the plain products of the 8B, 14B and 32B shapes at 25 row counts from 320 to
-    4,096 (225 cases) with every choice measured (the other kernel, K whole, in two, in four), the other kernel's step
-    a little above its least-squares value because near a tie this kernel wins more often: the estimate's choice is
-    0.2 % behind the best on average, within 5 % in 222 cases and 8 % behind at worst (8B qkv at 1,152 rows). The
-    conditions that stood here before (a fill of 0.6 of the compute units for K whole, cuts only within one round)
-    were 3.7 % behind on average and 30 to 54 % where 0.5 to 0.6 of the compute units had a tile and no cut fitted
-    (8B qkv at 1,536 rows 126 us against 93; 32B down at 1,792 rows 832 against 539) and 15 to 22 % where a second
-    round was a quarter full (14B and 32B down at 4,096 rows)."""
+    The large tile moves the fewest bytes per multiply (a compute unit fills its LDS at 32 bytes a clock at most, which is what this tile
+    needs at the matrix cores' full rate) but needs enough tiles to fill the compute units. Workgroups run in rounds (one per compute unit
+    here, two of the smaller tiles'); a round takes its K steps, and a cut of K, into ranges of 1,024 at least, adds the partial sums'
+    traffic."""
     if K % 32 or K < 128:
         return 0, 1
     cus = compute_units()
     if gated:
-        # The gated product cannot cut K, so what decides is how the two kernels' workgroups fall into rounds: this
-        # kernel's one per compute unit, the other's (tiles of 128 rows by 64 outputs) two. A round of this kernel takes
-        # about 1.25 of the other's. Swept on the 8B, 14B and 32B shapes at 160 to 1,024 rows: within 3 % of the better
-        # kernel everywhere (before: 19 % behind at 640 rows of the 8B shape, where 288 tiles are a full round and an
-        # eighth of one, and 26 to 32 % at 160 to 256 rows of the 14B shape, where 136 tiles in one round beat 544 small
-        # ones in two).
+        # The gated product cannot cut K, so what decides is how the two kernels' workgroups fall into rounds: a round of the large
+        # tile takes about 1.25 of one of tiles of 128 rows by 64 outputs, two to a compute unit.
         big = -(-N // 128) * -(-M // 256)
         rounds = -(-big // cus)
         rounds_other = -(-(-(-N // 64) * -(-M // 128)) // (2 * cus))
         if rounds_other > 1:
             return (256, 1) if 1.25 * rounds <= rounds_other else (0, 1)
-        # both in one round (65 to 128 rows): the large tile where it gives most compute units a workgroup (gate/up of
-        # the 32B shape at 96 and 128 rows, 200 tiles: 143 and 145 us against 160 and 161; the 14B shape's 136 tiles
-        # are a tie, the 8B shape's 96 lose, 87 us against 57)
+        # both in one round (65 to 128 rows): the large tile where it gives most compute units a workgroup
         return (256, 1) if big >= 0.7 * cus else (0, 1)
     if M < PINGPONG_MIN_ROWS:
         return 0, 1
@@ -831,25 +813,16 @@ def _small_us(M: int, N: int, K: int, gated: bool, normed: bool = False) -> floa
 
 
 def _tiled_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int]:
-    """(rows of the two-group kernel's tile or 0 for the small tile, ways K is cut): what `_pingpong_plan` and `_k_splits`
-    choose between 256 rows and the small tile, or tiles of 192 rows where these are estimated to be faster. A tile of
-    192 rows moves a sixth more bytes per multiply, but its rounds and its empty rows fall differently.
+    """(256 or 192 rows of a large tile, or 0, ways K is cut): what `_pingpong_plan` chooses, or tiles of 192 rows where these are estimated
+    to be faster. A tile of 192 rows moves a sixth more bytes per multiply, but its rounds and its empty rows fall differently. Cuts of K
+    are taken only where 192 leaves fewer empty rows than 256.
 
-    The constants were fitted to the times, inside a graph, of every choice for 252 products (ten row counts from 100 to
-    4,614 on the products of six shapes). On 216 products at nine other row counts (150 to 3,500) the choice is 0.2 % behind
-    the best on average, within 5 % in 213 and 14 % behind at worst (14B gate/up at 350 rows); without tiles of 192 rows 4.2 %
-    on average, within 5 % in 155. Inside whole prompt passes, which run hotter: 900 rows of the 8B shape 17.3 -> 16.5 ms,
-    1,300 23.8 -> 22.1, 3,000 of the 4B shape 27.6 -> 27.0, prompts of 4,614 rows of the 14B shape 131.5 -> 125.6. Not
-    taken: cuts of K where 192 leaves no fewer empty rows than 256 (631 rows of the 8B shape: the o and
-    down products 6 % faster alone, the pass 1 % slower: what binds there is the chip's power), and the small tile's count
-    of cuts by the same estimate (up to a third faster alone, nothing or 1 % slower inside a pass).
-
-    Two places where whole passes disagree with the estimate, so that 256 rows stay. A near tie of the gated product, over many
-    rounds: 1,800 rows of the 32B shape 138.4 ms with tiles of 192 rows there, 132.3 with 256, 2,850 of the 14B shape 82.3 /
-    80.3. And one round over a short K where the last tile of 256 rows is nearly empty (what it repeats costs it little) and
-    that of 192 is not: qkv at 1,300 rows of the 4B shape 14.76 / 14.53 ms, at 2,080 of the 0.6B 5.58 / 5.48, at 2,850 6.92 /
-    6.82; a step of 32 rows through all others up to 3,000 found 192 up to 8 % of the pass ahead, as they are at such row
-    counts too from K = 4,096 on (1,318 rows of the 8B shape 23.6 / 23.7)."""
+    One round over a short K where the last tile of 256 rows is nearly empty (what it repeats costs it little) and that of 192 is not keeps
+    256 rows against the estimate, since whole passes disagree with it there (ms, 256 rows / 192): qkv at 2,080 rows of the 0.6B shape 4.74 /
+    4.80, at 2,850 6.10 / 6.16, of the 1.7B at 2,846 10.61 / 10.66, at 1,300 of the 4B, a near tie, 12.57 / 12.47 with gate/up's last rows in
+    wide tiles. From K = 4,096 on 192 rows are ahead at such counts too. A near tie of the gated product keeps 256 rows as well
+    (`GATED_192_AT_MOST`): seldom, and within what passes differ by (8B at 3,361 rows 44.9 / 44.9, 14B at 2,081 49.5 / 49.3, 4B at 4,289 36.1 /
+    35.8)."""
     rows, cut = _pingpong_plan(M, N, K, gated)
     if K % 64 == 0:
         cut = cut if rows else _k_splits(M, N, K, gated)
@@ -879,18 +852,17 @@ FINER_AT_MOST = 0.96                # of the plan's estimate
 
 
 def _tiles(M: int, N: int, K: int, gated: bool, normed: bool, rows: int, cut: int) -> Tuple[int, int]:
-    """(rows of the two-group kernel's tile, `WIDE_LAST`, or 0 for the small tile, ways K is cut): the plan (``rows``, ``cut``) of
+    """(256, 192, `WIDE_LAST`, or 0 for the smaller tiles, ways K is cut): the plan (``rows``, ``cut``) of
     `_tiled_plan`, or what is estimated to take at most `FINER_AT_MOST` of its time among tiles of 256, 192 and wide last rows
     with K in any number of parts up to `FINER_CUTS`; ``normed``: the product adds into the residual and the RMSNorm of the new
     rows follows, which the reduction of a cut product makes on its way. A plan that is not `_tiled_plan`'s own stands.
 
-    Against the times, inside a graph, of every choice for 142 products (six shapes at 280 to 4,614 rows): 1.7 % behind the best
-    on average, where the plan is 4.7 % behind. With 0.95 for 0.96 8B o at 1,200 rows stays with two parts for three (68.4 / 64.3 us, the
-    pass 17.65 / 17.46 ms) and 2,500 rows of 2,048 x 4,096 likewise (68.7 / 65.4); with 1.0 and no exception 4B down at 900 goes to 192
-    rows in five parts (the pass 10.02 / 10.14). Whole passes, plan /
-    now: 560 rows of the 8B shape 12.7 / 11.2 ms, 280 to 340 of the 14B 16.7 to 17.6 / 13.9 to 14.5, 2,600 of the 8B 40.7 / 37.5, of
-    the 0.6B 3.5 % less. us, plan / now: 8B down at 1,100 rows 139.8 (192 rows, two parts) / 120.5 (256, three), at 280 64.1 (small tile, four) / 54.0 (192, eight), 14B qkv at 631 77.0 (256,
-    two) / 67.1 (three), down at 900 195.6 (192, two) / 174.9 (256, three); wide last rows: csrc/gemm_pingpong.hip."""
+    Whole passes, plan / so, the smaller tiles in either: 560 rows of the 8B shape 11.10 / 9.95 ms, 1,200 18.03 / 17.31, 2,600 35.57 / 33.25, 280 and
+    320 of the 14B 14.81 / 12.42 and 15.33 / 12.75, 1,800 46.1 / 44.3, of the 32B 106.8 / 104.1, 2,600 of the 0.6B 5.63 / 5.32. us with the norm: 8B down
+    at 1,100 rows 123.5 (192 rows, two parts) / 114.6 (256, three), 14B at 900 167.3 (192, two) / 157.7 (256, three), 14B qkv at 631 74.0 (256,
+    two) / 64.3 (three); wide last rows: csrc/gemm_pingpong.hip. With 0.95 for 0.96 8B o at 1,200 rows stays with two parts for three (68.4 /
+    64.3 us, the pass 17.65 / 17.46 ms) and 2,500 rows of 2,048 x 4,096 likewise (68.7 / 65.4); with 1.0 and no exception 4B down at 900 goes
+    to 192 rows in five parts (the pass 9.81 / 9.95)."""
     return _finer_tiles(M, N, K, gated, normed, rows, cut)[:2] if (rows, cut) == _own_tiled_plan(M, N, K, gated) else (rows, cut)
 
 
@@ -1133,17 +1105,15 @@ def _wide_best(tiles64: int, most: int, N: int, K: int, gated: bool) -> Tuple[fl
 @functools.lru_cache(maxsize=8192)
 def _wide_plan(M: int, N: int, K: int, gated: bool, adds: int = 0) -> Optional[Tuple[int, int, int]]:
     """(weight rows, activation rows, parts of K) with which the second weight-streaming kernel takes a product of more than
-    64 rows, or None where the tiled kernels are estimated to be faster: they move fewer bytes per multiply through a compute
-    unit, but their tiles of 128 x 128 and larger leave compute units without work where a product is small, and cutting K
-    costs them a second launch. ``adds``: into the residual (`ADDS`), or there with the norm behind it prepared, which is then no
-    launch of its own (`ADDS_AND_NORM`, see `_ride_plan`). Here tiles of 64 or 128 rows by 32 to 128 fill the chip with K whole.
+    64 rows, or None where the tiled kernels are estimated to be faster. ``adds``: into the residual (`ADDS`), or there with the norm behind
+    it prepared, which is then no launch of its own (`ADDS_AND_NORM`, see `_ride_plan`). Tiles of 64 or 128 rows by 32 to 128 fill the chip
+    with K whole, and parts of K need no second launch.
 
-    The constants were fitted to a sweep of every choice for the products of the 0.6B, 1.7B, 4B and 8B shapes at 100, 200, 320, 487 and
-    631 rows against what the tiled kernels take, when a last tile of few rows still made a launch slower than a full one; of the
-    480 choices between 65 and 1,024 rows of nine shapes one is now behind the tiled kernels (gated 8,960 x 1,536 at 128 rows,
-    25.9 / 26.6). us, tiled / here: 0.6B shape at 487 rows qkv 22.4 / 12.6, o 18.3 / 10.6, gate/up 18.7 / 15.7 (and the norm
-    behind o, 4.0, costs no launch of its own); 4B qkv at 640 rows 41.5 / 33.8, 8B qkv at 320 39.4 / 34.1. Beyond, the tiled
-    kernels win: 8B gate/up at 200 rows 79.9 / 101, down 44.8 / 54.9."""
+    Its constants were fitted to a sweep of the products of the 0.6B, 1.7B, 4B and 8B shapes at 100, 200, 320, 487 and 631 rows. What
+    is left to it since the tiled kernels have tiles of 64 x 64 up are mostly gated products of up to some 250 rows, which cannot cut K. us,
+    tiled / here: gate/up of the 0.6B shape at 100 rows 9.8 / 9.4, of the 1.7B 22.2 / 20.1, of the 8B at 128 61.4 / 58.9. Elsewhere the tiles are ahead:
+    0.6B at 487 rows qkv 10.3 / 12.6, o with its norm 11.5 / 14.2, gate/up 13.1 / 15.1, 4B qkv at 640 29.8 / 34.0, 8B qkv at 320 31.5 / 35.1, gate/up at
+    200 71.7 / 99.5, down 42.2 / 58.1. It misses: gate/up of the 32B shape at 100 rows 123.9 / 147.0, which the estimate gives it."""
     if not STREAM_MAX_ROWS < M <= WIDE_MOST_ROWS or K % 128 or N % 16 or K < WIDE_LEAST_K or (adds and N > WIDE_ADD_COLUMNS):
         return None
     t, plan = _wide_best(-(-M // 64), min(M, 128), N, K, gated)
@@ -1170,7 +1140,12 @@ def _own_choice(M: int, N: int, K: int, gated: bool, normed: bool) -> Tuple[int,
 @functools.lru_cache(maxsize=8192)
 def _choice_of(rows32: int, N: int, K: int, gated: bool, normed: bool) -> Tuple[int, int, float]:
     """A large tile (256, 192 or `WIDE_LAST`: `_tiles`), or one of `SMALL_TILES` where its estimate is below `SMALL_AT_MOST` of the large
-    one's or no large one fits."""
+    one's or no large one fits.
+
+    Of 43 products (six sizes of Qwen3, two of either other family) at 46 row counts from 65 to 3,000 the choice, `_wide_plan`'s included, is
+    1.7 % behind the fastest of all tiles and cuts on average, 14 % of them by more than 5 %, 4 % by more than 10. The plain minimum of the
+    estimates (no plan, no exceptions, no margins) is 1.6 % behind; in whole passes it is 2 % faster at some row counts (8B at 1,400 and 1,480
+    rows, down in 192 rows) and 1 to 1.5 % slower at others (0.6B at 2,080 and 2,600, 4B at 900)."""
     M = 32 * rows32
     tile, cut, large = _finer_tiles(M, N, K, gated, normed, *_own_tiled_plan(M, N, K, gated))
     if K % 64:
